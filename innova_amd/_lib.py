@@ -141,6 +141,15 @@ def probe() -> dict:
     return {"gfx": gfx.value, "hbm_bytes": hbm.value, "compute_units": cus.value, "name": name.value.decode()}
 
 
+_stream_of = _device_of = None
+
+
 def current_stream() -> int:
-    import torch
-    return torch.cuda.current_stream().cuda_stream
+    """The hipStream_t of torch's current stream.  Asked of torch's C layer: torch.cuda.current_stream() builds a Python
+    stream object on every call (2.85 us against 0.2 us, of a GEMV call's 10 us)."""
+    global _stream_of, _device_of
+    if _stream_of is None:
+        import torch
+        torch.cuda.init()
+        _stream_of, _device_of = torch._C._cuda_getCurrentRawStream, torch._C._cuda_getDevice
+    return _stream_of(_device_of())

@@ -32,7 +32,7 @@ def oil8_gemm(indices, codebook, activations, M: int, N: int, K: int):
     i, d1 = _dev(indices, np.uint8)
     c, _ = _dev(codebook, np.float32)
     a, d2 = _dev(activations, np.float32)
-    out = torch.empty((M, N), dtype=torch.float32, device="cuda")
+    out = a.new_empty((M, N), dtype=torch.float32)
     _lib.check(_lib.lib().oilhip_flat_oil8_gemm(i.data_ptr(), c.data_ptr(), a.data_ptr(), out.data_ptr(),
                                                 M, N, K, _lib.current_stream()))
     return _ret(out, d1 and d2)
@@ -44,7 +44,7 @@ def oil4_gemm(packed_indices, codebook, activations, M: int, N: int, K: int):
     i, d1 = _dev(packed_indices, np.uint8)
     c, _ = _dev(codebook, np.uint16)
     a, d2 = _dev(activations, np.float32)
-    out = torch.empty((M, N), dtype=torch.float32, device="cuda")
+    out = a.new_empty((M, N), dtype=torch.float32)
     _lib.check(_lib.lib().oilhip_flat_oil4_gemm(i.data_ptr(), c.data_ptr(), a.data_ptr(), out.data_ptr(),
                                                 M, N, K, _lib.current_stream()))
     return _ret(out, d1 and d2)
@@ -54,7 +54,7 @@ def _prod(fn, w, cb, cb_dtype, scale, X, M, N, K):
     import torch
     wd, d1 = _dev(w, np.uint8)
     xd, d2 = _dev(X, np.float32)
-    Y = torch.empty((N, M), dtype=torch.float32, device="cuda")
+    Y = xd.new_empty((N, M), dtype=torch.float32)
     if cb is None:
         _lib.check(fn(wd.data_ptr(), float(scale), xd.data_ptr(), Y.data_ptr(), M, K, N, _lib.current_stream()))
     else:
@@ -99,7 +99,7 @@ def engine_quant_gemm(bits: int, a, b_idx, codebook, M: int, N: int, K: int):
     cd, _ = _dev(codebook, np.float32)
     if cd.numel() < (1 << bits):
         raise _lib.OilHipError("engine_quant_gemm: codebook has fewer than 2^bits entries")
-    out = torch.empty((M, N), dtype=torch.float32, device="cuda")
+    out = ad.new_empty((M, N), dtype=torch.float32)
     _lib.check(_lib.lib().oilhip_engine_quant_gemm(bits, ad.data_ptr(), bd.data_ptr(), cd.data_ptr(), out.data_ptr(),
                                                    M, N, K, _lib.current_stream()))
     return _ret(out, d1 and d2)
@@ -124,7 +124,7 @@ def engine_dense_gemm(kind: int, a, b, M: int, N: int, K: int, scales=None, bloc
         if scales is None:
             raise _lib.OilHipError("engine_dense_gemm: the SPARK engine needs scales")
         sd, _ = _dev(scales, np.float32)
-    out = torch.empty((M, N), dtype=torch.float32, device="cuda")
+    out = ad.new_empty((M, N), dtype=torch.float32)
     _lib.check(_lib.lib().oilhip_engine_dense_gemm(kind, ad.data_ptr(), bd.data_ptr(), sd.data_ptr() if sd is not None else None,
                                                    int(block_size), out.data_ptr(), M, N, K, _lib.current_stream()))
     return _ret(out, d1 and d2)
@@ -149,7 +149,7 @@ def _tl(kind, weights, activations, M, N, K):
     import torch
     w, d1 = _dev(weights, np.uint8)
     a, d2 = _dev(activations, np.float32)
-    out = torch.empty((M, N), dtype=torch.float32, device="cuda")
+    out = a.new_empty((M, N), dtype=torch.float32)
     _lib.check(_lib.lib().oilhip_tl_gemm(kind, w.data_ptr(), a.data_ptr(), out.data_ptr(), M, N, K, _lib.current_stream()))
     return _ret(out, d1 and d2)
 

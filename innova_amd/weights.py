@@ -98,38 +98,46 @@ class DeviceWeights:
         _lib.check(_lib.lib().oilhip_dequant_f32(self.handle, out.data_ptr(), _lib.current_stream()))
         return out
 
-    def _xy(self, x, dtype, out):
-        import torch
+    def _rows(self, x, dtype):
+        """Activation rows of x, which may have any shape whose values are whole rows of `cols`."""
         assert x.is_cuda and x.dtype == dtype and x.is_contiguous()
-        x2 = x.reshape(-1, self.cols)
-        M = x2.shape[0]
+        M, rest = divmod(x.numel(), self.cols)
+        if rest:
+            raise _lib.OilHipError(f"activations of shape {tuple(x.shape)} are not rows of {self.cols}")
+        return M
+
+    def _out(self, x, M, out):
+        import torch
         if out is None:
-            out = torch.empty((M, self.rows), dtype=torch.float32, device=x.device)
+            return x.new_empty((M, self.rows), dtype=torch.float32)
         assert out.is_cuda and out.dtype == torch.float32 and out.is_contiguous() and out.numel() == M * self.rows
-        return x2, M, out
+        return out
 
     def gemv(self, x, out=None, general: bool = False, noalloc: bool = False):
         """Y[M][rows] = X[M][cols] . W^T, FP32 (decode path).  general=True forces the
         all-format kernel (used by tests to cross-check the specialised kernels); noalloc=True takes the entry
         point that allocates no device memory (uniform OIL4 only, scratch in a fixed device array)."""
         import torch
-        x2, M, out = self._xy(x, torch.float32, out)
+        M = self._rows(x, torch.float32)
+        out = self._out(x, M, out)
         L = _lib.lib()
         fn = L.oilhip_gemv_f32_general if general else L.oilhip_gemv_oil4_f32_noalloc if noalloc else L.oilhip_gemv_f32
-        _lib.check(fn(self.handle, x2.data_ptr(), out.data_ptr(), M, _lib.current_stream()))
+        _lib.check(fn(self.handle, x.data_ptr(), out.data_ptr(), M, _lib.current_stream()))
         return out
 
     def gemm_bf16(self, x, out=None):
         """Y[M][rows] = X[M][cols] . W^T with bf16 operands on MFMA, FP32 accumulate (prefill path)."""
         import torch
-        x2, M, out = self._xy(x, torch.bfloat16, out)
-        _lib.check(_lib.lib().oilhip_gemm_bf16(self.handle, x2.data_ptr(), out.data_ptr(), M, _lib.current_stream()))
+        M = self._rows(x, torch.bfloat16)
+        out = self._out(x, M, out)
+        _lib.check(_lib.lib().oilhip_gemm_bf16(self.handle, x.data_ptr(), out.data_ptr(), M, _lib.current_stream()))
         return out
 
     def gemm_f32(self, x, out=None):
         """The prefill GEMM for FP32 activations (the reference's own gemm() arguments, qwen35_engine.cpp:47-85):
         X is rounded once to bf16 inside the kernel's pre-pass; bf16 tolerance (rel-L2 <= 2e-3)."""
         import torch
-        x2, M, out = self._xy(x, torch.float32, out)
-        _lib.check(_lib.lib().oilhip_gemm_f32(self.handle, x2.data_ptr(), out.data_ptr(), M, _lib.current_stream()))
+        M = self._rows(x, torch.float32)
+        out = self._out(x, M, out)
+        _lib.check(_lib.lib().oilhip_gemm_f32(self.handle, x.data_ptr(), out.data_ptr(), M, _lib.current_stream()))
         return out
