@@ -22,14 +22,14 @@ def gemv_rmsnorm(w: DeviceWeights, x, norm_w, out=None):
     """y = W . rmsnorm(x; norm_w): the norm in front of a projection, formed inside the GEMV for one OIL4 row."""
     import torch
     assert x.is_cuda and x.dtype == torch.float32 and x.is_contiguous() and norm_w.is_cuda and norm_w.dtype == torch.float32
-    x2 = x.reshape(-1, w.cols)
-    M = x2.shape[0]
+    M = w._rows(x, torch.float32)
     if out is None:
-        out = torch.empty((M, w.rows), dtype=torch.float32, device=x.device)
-    xn = torch.empty_like(x2)
-    _lib.check(_lib.lib().oilhip_gemv_rmsnorm_f32(w.handle, x2.data_ptr(), norm_w.data_ptr(), out.data_ptr(), M, xn.data_ptr(),
+        out = x.new_empty((M, w.rows))
+    # xn and the scratch of mlp_step go back to torch's allocator when these return, while the launches may still be queued:
+    # the allocator hands a block out again in the order of the stream it came from, which is the stream they run on
+    xn = torch.empty_like(x)
+    _lib.check(_lib.lib().oilhip_gemv_rmsnorm_f32(w.handle, x.data_ptr(), norm_w.data_ptr(), out.data_ptr(), M, xn.data_ptr(),
                                                   _lib.current_stream()))
-    torch.cuda.current_stream().synchronize()      # xn is released when this returns
     return out
 
 
@@ -38,15 +38,13 @@ def mlp_step(gate_up: DeviceWeights, down: DeviceWeights, x, out=None, norm_w=No
     (DeviceWeights.stack_rows)."""
     import torch
     assert x.is_cuda and x.dtype == torch.float32 and x.is_contiguous()
-    x2 = x.reshape(-1, gate_up.cols)
-    M, F = x2.shape[0], down.cols
+    M, F = gate_up._rows(x, torch.float32), down.cols
     if out is None:
-        out = torch.empty((M, down.rows), dtype=torch.float32, device=x.device)
-    scratch = torch.empty((3 * F + gate_up.cols) * M, dtype=torch.float32, device=x.device)
-    _lib.check(_lib.lib().oilhip_mlp_step_f32(gate_up.handle, down.handle, x2.data_ptr(),
+        out = x.new_empty((M, down.rows))
+    scratch = x.new_empty((3 * F + gate_up.cols) * M)
+    _lib.check(_lib.lib().oilhip_mlp_step_f32(gate_up.handle, down.handle, x.data_ptr(),
                                               norm_w.data_ptr() if norm_w is not None else None, out.data_ptr(), M,
                                               scratch.data_ptr(), _lib.current_stream()))
-    torch.cuda.current_stream().synchronize()      # scratch is released when this returns
     return out
 
 

@@ -56,8 +56,8 @@ def moe_dispatch_batched(x, experts, indices, weights, want_z_loss: bool = True,
     g, u, d = arr([e.gate_proj for e in experts]), arr([e.up_proj for e in experts]), arr([e.down_proj for e in experts])
     L = _lib.lib()
     nbytes = L.oilhip_moe_workspace_bytes(T, K, D, F)
-    own_ws = workspace is None
-    ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device) if own_ws else workspace
+    # a workspace of our own goes back to torch's allocator on return, which hands it out again in stream order
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device) if workspace is None else workspace
     assert ws.is_cuda and ws.dtype == torch.uint8 and ws.numel() >= nbytes
     if out is None:
         out = torch.empty((T, D), dtype=torch.float32, device=x.device)
@@ -66,6 +66,4 @@ def moe_dispatch_batched(x, experts, indices, weights, want_z_loss: bool = True,
     _lib.check(L.oilhip_moe_forward(g, u, d, E, x.data_ptr(), idx.ctypes.data, w.ctypes.data, T, K, out.data_ptr(),
                                     ws.data_ptr(), nbytes, C.byref(z) if want_z_loss else None, C.byref(dropped),
                                     _lib.current_stream()))
-    if own_ws:
-        torch.cuda.current_stream().synchronize()   # ws is released when this returns
     return out, (z.value if want_z_loss else None), dropped.value
