@@ -4,6 +4,8 @@
 // accelerated decode path.  The reference build fuses a*b+c (its -mfma flag
 // with the compiler's default contraction), so sums of products below use
 // std::fma explicitly and this file is compiled with -ffp-contract=off.
+#include <sched.h>
+
 #include <algorithm>
 #include <array>
 #include <cmath>
@@ -20,6 +22,11 @@ int fail(int code, const std::string& msg);
 }
 
 namespace {
+
+// quantize_tensor: at least this many weights per thread (0.2 ms of work; starting one costs 0.02 ms), at most this many
+// threads (67 MB of weights take 3.0 ms on 16 and on 32 of them)
+constexpr uint64_t kWeightsPerThread = 262144;
+constexpr int kMaxThreads = 32;
 
 constexpr std::array<float, 4> kL2 = {-1.5104f, -0.4528f, 0.4528f, 1.5104f};
 constexpr std::array<float, 16> kL4 = {-2.7178f, -2.0522f, -1.5995f, -1.2392f, -0.9275f, -0.6508f,
@@ -296,6 +303,226 @@ bool encode_block(int fmt, std::span<const float> w, uint8_t* idx, size_t& il, u
     }
 }
 
+// ---- full 256-weight blocks ------------------------------------------------------------------------------------
+// What a model's tensors consist of, so the encoders below are written for the vector units: the same rounded
+// operations as above in the same order per result, laid out so that independent results run side by side.
+//   * sums of squares and means are sequential chains in double: one chain per block, group or run as above, but
+//     several of them interleaved (a single chain waits four cycles per weight).  A float's square is exact in
+//     double, so adding it rounds as the fused form does.
+//   * nearest() over a sorted table is a step function of v: the code is the number of thresholds that v reaches.
+//     The thresholds are found once with nearest() itself (threshold_table), ties and rounding included.  Only values
+//     of bounded magnitude come here (|v| <= 16: a weight over the RMS of its 256), where distances to distant levels
+//     never round to the same float.
+//   * codes are laid out one per byte and packed a dword at a time instead of bit by bit.
+// Blocks with a non-finite or enormous weight go through encode_block.  Each function is compiled for AVX-512, AVX2 and
+// the baseline and chosen at run time.  One thread, 4 M weights (Xeon 2.7 GHz, AVX-512), before -> after: OIL4 54 -> 1.8 ns
+// per weight, OIL8 53 -> 1.2, OIL4_GRP 62 -> 3.0, SPARK_Q0 11.9 -> 2.0; about half of what is left is the first touch of
+// the output pages.
+#define OIL_INLINE inline __attribute__((always_inline))
+
+template <size_t N>
+std::array<float, N - 1> threshold_table(const std::array<float, N>& lv) {
+    std::array<float, N - 1> t;
+    for (uint32_t i = 1; i < N; ++i) {
+        // the smallest float between two levels at which nearest() answers i; bit patterns of floats of one sign are
+        // ordered, so the search runs over integers that order floats of both signs
+        auto key = [](float f) { int32_t b; std::memcpy(&b, &f, 4); return b < 0 ? int32_t(0x80000000u - uint32_t(b)) : b; };
+        auto val = [](int32_t k) { const int32_t b = k < 0 ? int32_t(0x80000000u - uint32_t(k)) : k; float f; std::memcpy(&f, &b, 4); return f; };
+        int64_t lo = key(lv[i - 1]), hi = key(lv[i]);                  // nearest(lo) = i - 1, nearest(hi) = i
+        while (hi - lo > 1) {
+            const int64_t mid = lo + (hi - lo) / 2;
+            (nearest(val(int32_t(mid)), lv) >= i ? hi : lo) = mid;
+        }
+        t[i - 1] = val(int32_t(hi));
+    }
+    return t;
+}
+const std::array<float, 3> kT2 = threshold_table(kL2);
+const std::array<float, 15> kT4 = threshold_table(kL4);
+
+OIL_INLINE void put16(uint8_t* p, uint16_t v) { std::memcpy(p, &v, 2); }
+
+// sum of squares of `runs` consecutive runs of `len` floats each, every run a chain of its own
+template <int RUNS, int LEN>
+OIL_INLINE void square_sums(const float* w, double* s) {
+    for (int r = 0; r < RUNS; ++r) s[r] = 0.0;
+    for (int i = 0; i < LEN; ++i)
+        for (int r = 0; r < RUNS; ++r) { const double x = w[r * LEN + i]; s[r] += x * x; }
+}
+
+template <int BITS>
+OIL_INLINE uint32_t level_code(float v) {
+    if constexpr (BITS == 8) {
+        const float lo = v < 8.0f ? v : 8.0f, c = -8.0f < lo ? lo : -8.0f;
+        const float r = (c + 8.0f) * 255.0f / 16.0f;                   // lround: halves away from zero, r >= 0
+        const int k = int(r);
+        return uint32_t(k + (r - float(k) >= 0.5f ? 1 : 0));
+    } else {
+        uint32_t q = 0;
+        if constexpr (BITS == 4) for (float t : kT4) q += v >= t ? 1u : 0u;
+        else for (float t : kT2) q += v >= t ? 1u : 0u;
+        return q;
+    }
+}
+
+// codes (one per byte, `n` of them, n * BITS a multiple of 8) -> bytes, first code in the low bits
+template <int BITS>
+OIL_INLINE void pack_codes(const uint8_t* c, int n, uint8_t* out) {
+    if constexpr (BITS == 8) std::memcpy(out, c, size_t(n));
+    else if constexpr (BITS == 4) for (int i = 0; i < n / 2; ++i) out[i] = uint8_t(c[2 * i] | c[2 * i + 1] << 4);
+    else for (int i = 0; i < n / 4; ++i) out[i] = uint8_t(c[4 * i] | c[4 * i + 1] << 2 | c[4 * i + 2] << 4 | c[4 * i + 3] << 6);
+}
+
+template <int BITS>
+OIL_INLINE void full_lattice(const float* w, double sum_sq, uint8_t* out) {
+    const float scale = float(std::sqrt(sum_sq / 256.0));
+    put16(out, to_half(scale));
+    alignas(64) uint8_t code[256], dense[256];
+    if (scale <= 1e-12f) {
+        const uint32_t q = level_code<BITS>(0.0f);
+        for (int i = 0; i < 256; ++i) code[i] = uint8_t(q);
+    } else {
+        for (int i = 0; i < 256; ++i) code[i] = uint8_t(level_code<BITS>(w[i] / scale));
+    }
+    // 16 / BITS weights, the last of every 16 * BITS, have no code: their bits hold the scale
+    constexpr int RUN = 16 * BITS;
+    for (int r = 0; r < 256 / RUN; ++r) std::memcpy(dense + r * (RUN - 1), code + r * RUN, RUN - 1);
+    pack_codes<BITS>(dense, 256 - 256 / RUN, out + 2);
+}
+
+template <int BITS>
+OIL_INLINE bool full_grouped(const float* w, uint8_t* out) {
+    float zp[4], sc[4];
+    if constexpr (BITS == 8) {
+        for (int g = 0; g < 4; ++g) {
+            float lo = w[g * 64], hi = lo;
+            for (int i = 1; i < 64; ++i) { const float x = w[g * 64 + i]; lo = x < lo ? x : lo; hi = x > hi ? x : hi; }
+            if (lo == 0.0f) return false;                              // which of several zeros is the first: encode_block finds it
+            zp[g] = lo;
+            sc[g] = hi - lo;
+        }
+    } else {
+        double mu[4] = {0, 0, 0, 0}, ss[4] = {0, 0, 0, 0};
+        for (int i = 0; i < 64; ++i)
+            for (int g = 0; g < 4; ++g) mu[g] += w[g * 64 + i];
+        for (int g = 0; g < 4; ++g) mu[g] /= 64.0;
+        for (int i = 0; i < 64; ++i)
+            for (int g = 0; g < 4; ++g) { const double d = double(w[g * 64 + i]) - mu[g]; ss[g] = std::fma(d, d, ss[g]); }
+        for (int g = 0; g < 4; ++g) { zp[g] = float(mu[g]); sc[g] = ss[g] > 0.0 ? float(std::sqrt(ss[g] / 64.0)) : 0.0f; }
+    }
+    constexpr int GROUP = 4 + 8 * BITS;
+    for (int g = 0; g < 4; ++g) {
+        uint8_t* o = out + g * GROUP;
+        put16(o, to_half(zp[g]));
+        put16(o + 2, to_half(sc[g]));
+        alignas(64) uint8_t code[64];
+        if (sc[g] == 0.0f) {
+            std::memset(code, 0, sizeof code);
+        } else if constexpr (BITS == 8) {
+            for (int i = 0; i < 64; ++i) {
+                const float r = (w[g * 64 + i] - zp[g]) / sc[g] * 255.0f;
+                const int k = int(r), q = k + (r - float(k) >= 0.5f ? 1 : 0);
+                code[i] = uint8_t(q > 255 ? 255 : q);
+            }
+        } else {
+            for (int i = 0; i < 64; ++i) code[i] = uint8_t(level_code<BITS>(float((double(w[g * 64 + i]) - zp[g]) / double(sc[g]))));
+        }
+        pack_codes<BITS>(code, 64, o + 4);
+    }
+    return true;
+}
+
+OIL_INLINE uint32_t sign_bits(const float* w, int n) {                 // n <= 32
+    uint32_t m = 0;
+    for (int i = 0; i < n; ++i) m |= (w[i] >= 0.0f ? 1u : 0u) << i;
+    return m;
+}
+
+// One full block; `sum_sq` is its sum of squares where the format is scaled by the block's RMS.  False: not covered
+// here, encode_block takes it.
+OIL_INLINE bool encode_full(int fmt, const float* w, double sum_sq, uint8_t* out) {
+    uint32_t top = 0;
+    for (int i = 0; i < 256; ++i) { uint32_t b; std::memcpy(&b, w + i, 4); b &= 0x7FFFFFFFu; top = b > top ? b : top; }
+    if (top > 0x70000000u) return false;                               // 1.6e29 and beyond, infinities, NaN
+    switch (fmt) {
+        case OILHIP_OIL2: full_lattice<2>(w, sum_sq, out); return true;
+        case OILHIP_OIL4: full_lattice<4>(w, sum_sq, out); return true;
+        case OILHIP_OIL8: full_lattice<8>(w, sum_sq, out); return true;
+        case OILHIP_OIL2_GRP: return full_grouped<2>(w, out);
+        case OILHIP_OIL4_GRP: return full_grouped<4>(w, out);
+        case OILHIP_OIL8_GRP: return full_grouped<8>(w, out);
+        case OILHIP_OIL1: {
+            double s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+            for (int i = 0; i < 32; ++i)
+                for (int r = 0; r < 8; ++r) s[r] += w[r * 32 + i];
+            for (int r = 0; r < 8; ++r) put16(out + 2 * r, to_half(float(s[r] / 32.0)));
+            return true;
+        }
+        case OILHIP_SPARK_Q0: {
+            double s[8];
+            square_sums<8, 32>(w, s);
+            for (int r = 0; r < 8; ++r) {
+                const uint32_t m = sign_bits(w + 32 * r, 32);
+                put16(out + 6 * r, to_half(float(std::sqrt(s[r] / 32.0))));
+                std::memcpy(out + 6 * r + 2, &m, 4);
+            }
+            return true;
+        }
+        case OILHIP_OIL1_GRP: {                                        // a scale, then 15 signs of every 16 weights
+            uint64_t word = to_half(float(std::sqrt(sum_sq / 256.0)));
+            int held = 16;
+            for (int r = 0; r < 16; ++r) {
+                word |= uint64_t(sign_bits(w + 16 * r, 15)) << held;
+                held += 15;
+                if (held >= 32) { const uint32_t lo = uint32_t(word); std::memcpy(out, &lo, 4); out += 4; word >>= 32; held -= 32; }
+            }
+            return true;
+        }
+        default: return false;
+    }
+}
+
+// Blocks [b0, b1) into payload + blocks[b].cb_off; only the last block of a tensor can be shorter than 256.
+OIL_INLINE void encode_range(const uint8_t* fmts, const float* w, uint64_t numel, const oilhip_block_t* blocks, uint8_t* payload,
+                             uint32_t b0, uint32_t b1) {
+    constexpr uint32_t SIDE = 8;                                       // RMS chains side by side
+    for (uint32_t b = b0; b < b1; b += SIDE) {
+        const uint32_t nb = std::min(SIDE, b1 - b);
+        const bool full = uint64_t(b + nb) * 256 <= numel;
+        double s[SIDE] = {};
+        if (full && nb == SIDE) square_sums<SIDE, 256>(w + uint64_t(b) * 256, s);
+        else if (full) for (uint32_t j = 0; j < nb; ++j) square_sums<1, 256>(w + uint64_t(b + j) * 256, s + j);
+        for (uint32_t j = 0; j < nb; ++j) {
+            const uint64_t at = uint64_t(b + j) * 256;
+            uint8_t* out = payload + blocks[b + j].cb_off;
+            if (full && encode_full(fmts[b + j], w + at, s[j], out)) continue;
+            size_t il = 0, cl = 0;                                     // one channel is empty in every format: both may point at `out`
+            encode_block(fmts[b + j], {w + at, size_t(std::min<uint64_t>(256, numel - at))}, out, il, out, cl);
+        }
+    }
+}
+
+using RangeFn = void (*)(const uint8_t*, const float*, uint64_t, const oilhip_block_t*, uint8_t*, uint32_t, uint32_t);
+__attribute__((target("avx512f,avx512bw,avx512dq,avx512vl,avx2,fma")))
+void encode_range_avx512(const uint8_t* f, const float* w, uint64_t n, const oilhip_block_t* b, uint8_t* p, uint32_t b0, uint32_t b1) { encode_range(f, w, n, b, p, b0, b1); }
+__attribute__((target("avx2,fma")))
+void encode_range_avx2(const uint8_t* f, const float* w, uint64_t n, const oilhip_block_t* b, uint8_t* p, uint32_t b0, uint32_t b1) { encode_range(f, w, n, b, p, b0, b1); }
+void encode_range_base(const uint8_t* f, const float* w, uint64_t n, const oilhip_block_t* b, uint8_t* p, uint32_t b0, uint32_t b1) { encode_range(f, w, n, b, p, b0, b1); }
+
+RangeFn range_fn() {
+    if (__builtin_cpu_supports("avx512f") && __builtin_cpu_supports("avx512bw") && __builtin_cpu_supports("avx512dq") && __builtin_cpu_supports("avx512vl"))
+        return encode_range_avx512;
+    return __builtin_cpu_supports("avx2") && __builtin_cpu_supports("fma") ? encode_range_avx2 : encode_range_base;
+}
+
+// Threads for a tensor when the caller names no number: those this process may run on, each with enough work to pay for
+// being started.
+int auto_threads(uint64_t numel) {
+    cpu_set_t set;
+    const int cpus = sched_getaffinity(0, sizeof set, &set) == 0 ? CPU_COUNT(&set) : int(std::max(1u, std::thread::hardware_concurrency()));
+    return int(std::clamp<uint64_t>(numel / kWeightsPerThread, 1, uint64_t(std::min(cpus, kMaxThreads))));
+}
+
 }  // namespace
 
 extern "C" {
@@ -319,49 +546,67 @@ int oilhip_quantize_tensor(const uint8_t* fmts, uint32_t nblocks, const float* w
     if (uint64_t(nblocks) * 256 < numel || uint64_t(nblocks - 1) * 256 >= numel)
         return oilhip::fail(OILHIP_E_ARG, "quantize_tensor: nblocks does not match numel");
     size_t widest = 0;
+    bool sparse = false;
     uint64_t bound = 0;
     for (uint32_t b = 0; b < nblocks; ++b) {
         if (fmts[b] >= OILHIP_NUM_FORMATS) return oilhip::fail(OILHIP_E_ARG, "quantize_tensor: unknown format");
         const size_t m = payload_bound(fmts[b], 256);
         widest = std::max(widest, m);
+        sparse |= fmts[b] == OILHIP_SPARK_SPARSE || fmts[b] == OILHIP_SPARK_SPARSE_GRP;   // an all-zero block is shorter there
         bound += (m + 15) & ~size_t(15);
     }
     if (!payload) { *total = bound; return OILHIP_OK; }
     if (!blocks) return oilhip::fail(OILHIP_E_ARG, "quantize_tensor: blocks is null");
+    if (threads <= 0) threads = auto_threads(numel);
+    threads = int(std::min<uint32_t>(uint32_t(std::min(threads, 64)), nblocks));
+    const uint32_t chunk = (nblocks + uint32_t(threads) - 1) / uint32_t(threads);
+    auto in_chunks = [&](auto&& work) {
+        std::vector<std::thread> pool;
+        for (int t = 1; t < threads; ++t) {
+            const uint32_t b0 = uint32_t(t) * chunk, b1 = std::min(nblocks, b0 + chunk);
+            if (b0 < b1) pool.emplace_back(work, b0, b1);
+        }
+        work(0u, std::min(nblocks, chunk));
+        for (auto& th : pool) th.join();
+    };
+    auto weights_of = [&](uint32_t b) { return uint32_t(std::min<uint64_t>(256, numel - uint64_t(b) * 256)); };
+    uint64_t off = 0;
+    if (!sparse) {
+        // every block's size follows from its format and length, so the blocks are encoded where they belong
+        size_t full[OILHIP_NUM_FORMATS];
+        for (int f = 0; f < OILHIP_NUM_FORMATS; ++f) full[f] = payload_bound(f, 256);
+        for (uint32_t b = 0; b < nblocks; ++b) {
+            const uint32_t n = weights_of(b), bytes = uint32_t(n == 256 ? full[fmts[b]] : payload_bound(fmts[b], int(n)));
+            const uint32_t cl = fmts[b] == OILHIP_OIL1 ? bytes : 0u;
+            off = (off + 15) & ~uint64_t(15);
+            blocks[b] = oilhip_block_t{off, off + cl, cl, bytes - cl, n, fmts[b], {0, 0, 0}};
+            off += bytes;
+        }
+        if (off > cap) return oilhip::fail(OILHIP_E_ARG, "quantize_tensor: payload buffer too small");
+        const RangeFn encode = range_fn();
+        in_chunks([&](uint32_t b0, uint32_t b1) { encode(fmts, w, numel, blocks, payload, b0, b1); });
+        *total = off;
+        return OILHIP_OK;
+    }
     struct Enc { uint32_t il, cl; };
     const size_t stride = widest + 32;             // [32 bytes codebook channel][index channel]
     std::vector<uint8_t> tmp(size_t(nblocks) * stride);
     std::vector<Enc> len(nblocks);
-    if (threads <= 0) threads = int(std::max(1u, std::thread::hardware_concurrency()));
-    threads = int(std::min<uint32_t>(uint32_t(std::min(threads, 64)), nblocks));
-    auto work = [&](uint32_t b0, uint32_t b1) {
+    in_chunks([&](uint32_t b0, uint32_t b1) {
         for (uint32_t b = b0; b < b1; ++b) {
-            const uint64_t at = uint64_t(b) * 256;
-            const size_t n = size_t(std::min<uint64_t>(256, numel - at));
             size_t il = 0, cl = 0;
             uint8_t* slot = tmp.data() + size_t(b) * stride;
-            encode_block(fmts[b], {w + at, n}, slot + 32, il, slot, cl);
+            encode_block(fmts[b], {w + uint64_t(b) * 256, weights_of(b)}, slot + 32, il, slot, cl);
             len[b] = {uint32_t(il), uint32_t(cl)};
         }
-    };
-    std::vector<std::thread> pool;
-    const uint32_t chunk = (nblocks + uint32_t(threads) - 1) / uint32_t(threads);
-    for (int t = 1; t < threads; ++t) {
-        const uint32_t b0 = uint32_t(t) * chunk, b1 = std::min(nblocks, b0 + chunk);
-        if (b0 < b1) pool.emplace_back(work, b0, b1);
-    }
-    work(0, std::min(nblocks, chunk));
-    for (auto& th : pool) th.join();
-    uint64_t off = 0;
+    });
     for (uint32_t b = 0; b < nblocks; ++b) {
         off = (off + 15) & ~uint64_t(15);
         if (off + len[b].cl + len[b].il > cap) return oilhip::fail(OILHIP_E_ARG, "quantize_tensor: payload buffer too small");
         const uint8_t* slot = tmp.data() + size_t(b) * stride;
         std::memcpy(payload + off, slot, len[b].cl);
         std::memcpy(payload + off + len[b].cl, slot + 32, len[b].il);
-        const uint64_t at = uint64_t(b) * 256;
-        blocks[b] = oilhip_block_t{off, off + len[b].cl, len[b].cl, len[b].il,
-                                   uint32_t(std::min<uint64_t>(256, numel - at)), fmts[b], {0, 0, 0}};
+        blocks[b] = oilhip_block_t{off, off + len[b].cl, len[b].cl, len[b].il, weights_of(b), fmts[b], {0, 0, 0}};
         off += len[b].cl + len[b].il;
     }
     *total = off;
