@@ -116,162 +116,160 @@ prod_packed_kernel(const uint8_t* __restrict__ wq, const uint16_t* __restrict__ 
     }
 }
 
-// Engine layout: codes packed along the flat [K][N] index; thread per output column
-// n, sequential in k like the reference loop (terms with A == 0 are skipped).
-template <int BITS>
-__global__ void __launch_bounds__(64)
-engine_kernel(const float* __restrict__ A, const uint8_t* __restrict__ bq, const float* __restrict__ cb,
-              float* __restrict__ C, long long M, long long N, long long K) {
-    // One wavefront per 64 outputs of a row of C: the chain of every output stays one thread's k-ordered FMA
-    // sequence (bit-identical to the reference loop), so the only parallelism is across outputs; what can be taken
-    // off the chain is taken off: the codes of 32 steps are fetched together, A[m][k] is wave-uniform and read
-    // through the scalar cache, and the codebook sits in LDS in 8 copies.
-    __shared__ float c[(1 << BITS) * 8];
-    for (int i = threadIdx.x; i < (1 << BITS) * 8; i += 64) c[i] = cb[i >> 3];
-    __syncthreads();
-    const long long n = (long long)blockIdx.x * 64 + threadIdx.x;
-    const long long m = blockIdx.y;
-    const bool live = n < N;
-    const long long nn = live ? n : N - 1;                // idle lanes follow the last column and store nothing
-    constexpr int PER = 8 / BITS;
-    constexpr int UN = 32;
-    const float* a_row = A + m * K;
-    const uint32_t copy = threadIdx.x & 7u;
-    float acc = 0.0f;
-    long long k = 0;
-    uint8_t raw[UN], nxt[UN];
-    auto fetch = [&](uint8_t (&dst)[UN], long long k0) {
-#pragma unroll
-        for (int j = 0; j < UN; ++j) dst[j] = bq[((unsigned long long)(k0 + j) * (unsigned long long)N + (unsigned long long)nn) / PER];
-    };
-    if (K >= UN) fetch(raw, 0);
-    for (; k + UN <= K; k += UN) {
-        const bool more = k + 2 * UN <= K;
-        if (more) fetch(nxt, k + UN);                     // the next 32 steps fly while these are folded in
-        float lv[UN];
-#pragma unroll
-        for (int j = 0; j < UN; ++j) {                    // look-ups off the chain: none of them depends on acc
-            const uint32_t sub = (uint32_t)((unsigned long long)(k + j) * (unsigned long long)N + (unsigned long long)nn) & (uint32_t)(PER - 1);
-            const uint32_t code = ((uint32_t)raw[j] >> (sub * BITS)) & ((1u << BITS) - 1u);
-            lv[j] = c[code * 8u + copy];
-        }
-#pragma unroll
-        for (int j = 0; j < UN; ++j) {
-            const float a = a_row[k + j];
-            const float t = __fmaf_rn(a, lv[j], acc);
-            acc = a != 0.0f ? t : acc;                    // the reference skips the term, 0 * inf must not reach acc
-        }
-        if (more) {
-#pragma unroll
-            for (int j = 0; j < UN; ++j) raw[j] = nxt[j];
-        }
-    }
-    for (; k < K; ++k) {
-        const float a = a_row[k];
-        if (a == 0.0f) continue;
-        const long long flat = k * N + nn;
-        const uint32_t code = (bq[flat / PER] >> ((flat % PER) * BITS)) & ((1u << BITS) - 1u);
-        acc = __fmaf_rn(a, c[code * 8u + copy], acc);
-    }
-    if (live) C[m * N + n] = acc;
-}
+// OIL{8,4,2}Engine::quant_gemm: codes packed along the flat [K][N] index, every output one k-ordered chain of fused
+// multiply-adds, terms with A == 0 skipped, bit for bit as in the reference loop.
+// The chain bounds it: K dependent FMAs of one wavefront, which issues an instruction every four to five cycles, so the
+// time is the number of instructions on the wavefront that carries the chain.  A workgroup therefore splits the work by
+// role: four or eight producer wavefronts fetch, unpack and look up the levels of COLS columns and kEngTile steps into LDS while one
+// wavefront per row of A walks the previous tile with 1.25 instructions per step (an FMA, a quarter of a 16-byte LDS
+// read; A[m][k] sits in a register of 16 lanes and the broadcast is part of the FMA).  16 columns per workgroup, three quarters of the chain's
+// lanes idle: the chain costs the same for any number of lanes, and 256 workgroups at N = 4096 share the unpacking and
+// the fetches.  A producer lane takes one k step: its 16 columns' codes are 2 to 5 neighbouring dwords at any bit
+// offset, its 16 levels go to 16 rows of the tile (lanes side by side, no bank conflicts), and four tiles of codes are in
+// flight.  N = K = 4096, M = 1: 8-bit 59.6 -> 27 us, 4-bit 176 -> 21, 2-bit 176 -> 19.
+constexpr int kEngTile = 256, kEngPitch = kEngTile + 4, kEngMaxRows = 4;
+constexpr int eng_producers(int cols) { return cols == 16 ? 4 : 8; }
+constexpr int eng_copies(int bits) { return bits == 8 ? 16 : 64; }          // lane-private copies of the codebook
+constexpr size_t eng_lds(int bits, int cols) { return 4u * ((size_t)eng_copies(bits) << bits) + 8u * (size_t)cols * kEngPitch; }
 
-// engine_kernel<8> for N a multiple of 4: the same k-ordered chain per output, fed differently.  A wavefront per 64
-// outputs leaves most of the chip idle and a single wavefront issues one instruction at a time, so the time is the
-// instruction count per k step.  The four lanes of a quad own four neighbouring columns, whose codes of one k step
-// share a dword: lane q of the quad loads the dword of step 4i + q and the quad passes the dwords round with DPP
-// (8 loads per lane and 32 steps instead of 32 byte loads, three batches of 32 steps in flight); the look-up address
-// is one v_perm_b32 (entry v of lane l at byte v*256 + l*4 of a 64 KB table); the levels of batch b+1 are looked up
-// before the chain of batch b runs.  A batch without a zero in A (the usual case) is 32 bare FMAs; one with a zero
-// keeps the reference's skip as a select behind every FMA, so the result is the reference's bit for bit either way.
-__global__ void __launch_bounds__(64)
-engine8_quad_kernel(const float* __restrict__ A, const uint8_t* __restrict__ bq, const float* __restrict__ cb,
-                    float* __restrict__ C, long long M, long long N, long long K) {
-    __shared__ float c[256 * 64];
-    {
-        const float mine[4] = {cb[threadIdx.x], cb[64 + threadIdx.x], cb[128 + threadIdx.x], cb[192 + threadIdx.x]};
-#pragma unroll
-        for (int part = 0; part < 4; ++part)
-            for (int v = 0; v < 64; ++v)
-                c[(part * 64 + v) * 64 + threadIdx.x] = __shfl(mine[part], v);
-    }
+template <int BITS, int COLS>
+__global__ void __launch_bounds__(64 * (eng_producers(COLS) + kEngMaxRows))
+engine_kernel(const float* __restrict__ A, const uint8_t* __restrict__ bq, const float* __restrict__ cb, float* __restrict__ C,
+              long long M, long long N, long long K) {
+    constexpr int PRODUCERS = eng_producers(COLS), OWN = COLS * 4 / PRODUCERS;   // 4 wavefronts' lanes cover a tile's steps, each OWN columns
+    constexpr int W = OWN * BITS / 32;                     // dwords of one step's codes
+    constexpr uint32_t COPIES = eng_copies(BITS);
+    constexpr int AHEAD = 4;                               // tiles of codes in flight
+    extern __shared__ __align__(16) float eng_mem[];
+    float* lev0 = eng_mem;                                 // two tiles: [column][step]
+    float* tab = eng_mem + 2 * COLS * kEngPitch;
+    const uint32_t lane = threadIdx.x & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    for (uint32_t i = threadIdx.x; i < (1u << BITS) * COPIES; i += blockDim.x) tab[i] = cb[i / COPIES];
+    // workgroups are dealt to the eight XCDs in turn: each takes a run of neighbouring columns, whose codes share lines
+    const uint32_t q8 = gridDim.x >> 3, r8 = gridDim.x & 7u, xcd = blockIdx.x & 7u;
+    const long long n0 = (long long)(xcd * q8 + (xcd < r8 ? xcd : r8) + (blockIdx.x >> 3)) * COLS;
+    const long long tiles = (K + kEngTile - 1) / kEngTile;
     __syncthreads();
-    const long long n = (long long)blockIdx.x * 64 + threadIdx.x;
-    const long long m = blockIdx.y;
-    const bool live = n < N;                               // N % 4 == 0: a quad is live or idle as a whole
-    const uint32_t sub = threadIdx.x & 3u, lane = threadIdx.x;
-    const unsigned long long n4 = (unsigned long long)(live ? n - sub : N - 4);
-    const float* a_row = A + m * K;
-    constexpr int UN = 32, NB = 4;
-    const long long nb = K / UN;                           // full batches
-    const uint32_t lanebase = lane * 4u, sel = 0x0C0C0000u | ((4u + sub) << 8);
-    uint32_t dw[NB][8];
-    float av[NB];                                          // lane j < 32: A[m][32 b + j], for the zero test
-    auto clampb = [&](long long b) { return b < nb ? b : nb - 1; };
-    // a lane's byte offset inside a k step's row pair: uniform 64-bit bases, 32-bit lane offsets (N < 2^29)
-    const uint32_t lane_off = sub * (uint32_t)N + (uint32_t)n4;
-    auto fetch = [&](int slot, long long b) {              // batch b, clamped to the last one: issued unconditionally
-        const unsigned long long k0 = (unsigned long long)clampb(b) * UN;
-        const uint8_t* ub = bq + k0 * (unsigned long long)N;                 // uniform
+    if (wave < (uint32_t)PRODUCERS) {
+        const uint32_t step0 = (wave & 3u) * 64u + lane, col0 = (wave >> 2) * OWN;
+        uint32_t raw[AHEAD][W + 1], sh[AHEAD];
+        const uintptr_t base = reinterpret_cast<uintptr_t>(bq);
+        const uintptr_t last = (base + ((unsigned long long)K * (unsigned long long)N * BITS + 7) / 8 - 1) & ~(uintptr_t)3;
+        auto fetch = [&](int slot, long long t) {          // this lane's step of tile t; past the end: the last step again
+            long long k = t * kEngTile + step0;
+            k = k < K ? k : K - 1;
+            const unsigned long long bit = ((unsigned long long)k * (unsigned long long)N + (unsigned long long)n0 + col0) * BITS;
+            const uintptr_t at = base + (bit >> 3), word = at & ~(uintptr_t)3;
+            sh[slot] = (uint32_t)(at & 3) * 8u + (uint32_t)(bit & 7);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) dw[slot][i] = *reinterpret_cast<const uint32_t*>(ub + 4ull * i * (unsigned long long)N + lane_off);
-        av[slot] = a_row[k0 + (lane & 31u)];
-    };
-    float lv[2][UN];
-    auto lookup = [&](int slot, int set) {
+            for (int i = 0; i <= W; ++i) raw[slot][i] = *reinterpret_cast<const uint32_t*>(word + 4 * i < last ? word + 4 * i : last);
+        };
+        auto decode = [&](int slot, float* dst, bool live) {   // steps past K: zeros
+            float lv[OWN];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int v = (int)dw[slot][i];
-            const uint32_t qs[4] = {(uint32_t)__builtin_amdgcn_mov_dpp(v, 0x00, 0xF, 0xF, true),     // quad_perm [0,0,0,0]
-                                    (uint32_t)__builtin_amdgcn_mov_dpp(v, 0x55, 0xF, 0xF, true),     // [1,1,1,1]
-                                    (uint32_t)__builtin_amdgcn_mov_dpp(v, 0xAA, 0xF, 0xF, true),     // [2,2,2,2]
-                                    (uint32_t)__builtin_amdgcn_mov_dpp(v, 0xFF, 0xF, 0xF, true)};    // [3,3,3,3]
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const uint32_t addr = __builtin_amdgcn_perm(qs[q], lanebase, sel);
-                lv[set][4 * i + q] = *reinterpret_cast<const float*>(reinterpret_cast<const uint8_t*>(c) + addr);
+            for (int c = 0; c < OWN; ++c) {
+                const uint32_t d = __builtin_amdgcn_alignbit(raw[slot][c * BITS / 32 + 1], raw[slot][c * BITS / 32], sh[slot]);
+                const uint32_t code = (d >> (c * BITS % 32)) & ((1u << BITS) - 1u);
+                lv[c] = tab[code * COPIES + (lane & (COPIES - 1))];
             }
-        }
-    };
-    float acc = 0.0f;
-    auto chain = [&](const float (&a)[UN], int slot, int set) {
-        const bool any_zero = __ballot(av[slot] == 0.0f) != 0ull;         // uniform
-        if (!any_zero) {
 #pragma unroll
-            for (int j = 0; j < UN; ++j) acc = __fmaf_rn(a[j], lv[set][j], acc);
+            for (int c = 0; c < OWN; ++c) dst[(col0 + c) * kEngPitch + step0] = live ? lv[c] : 0.0f;
+        };
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) fetch(u, u);
+        for (long long t = 0; t < tiles; t += AHEAD)
+#pragma unroll
+            for (int u = 0; u < AHEAD; ++u)
+                if (t + u < tiles) {                       // uniform over the workgroup, as in the other role
+                    decode(u, lev0 + (u & 1) * (COLS * kEngPitch), (t + u) * kEngTile + step0 < K);                 // tile t + u: the chain has left this buffer (AHEAD is even)
+                    fetch(u, t + u + AHEAD);
+                    __syncthreads();
+                }
+        return;
+    }
+    __builtin_amdgcn_s_setprio(3);                         // the chain goes first where it shares a SIMD with producers
+    const uint32_t row = wave - PRODUCERS, rows = (blockDim.x >> 6) - PRODUCERS;
+    const long long m = (long long)blockIdx.y * rows + row;
+    const bool live = m < M;
+    const float* a_row = A + (live ? m : M - 1) * K;
+    const float* mine = lev0 + (lane & (COLS - 1)) * kEngPitch;
+    constexpr int GA = kEngTile / 16;                      // A of a tile: lane j of every 16 holds steps 16 g + j
+    auto fetch_a = [&](float (&dst)[GA], long long t) {
+        const long long k0 = t * kEngTile;
+        if (k0 + kEngTile <= K) {
+            const float* p = a_row + k0 + (lane & 15u);
+#pragma unroll
+            for (int g = 0; g < GA; ++g) dst[g] = p[16 * g];
         } else {
 #pragma unroll
-            for (int j = 0; j < UN; ++j) {
-                const float t = __fmaf_rn(a[j], lv[set][j], acc);
-                acc = a[j] != 0.0f ? t : acc;              // the reference skips the term
+            for (int g = 0; g < GA; ++g) {
+                const long long k = k0 + 16 * g + (lane & 15u);
+                // past K: -0 meets a zero level, and adding their product, -0, changes no sum, not even a zero's sign
+                dst[g] = k < K ? a_row[k] : -0.0f;
             }
         }
     };
-    if (nb > 0) {
+    float acc = 0.0f;
+    auto walk = [&](const float (&a)[GA], const float* src, int steps) {
+        uint32_t low = 0x7FFFFFFFu;                        // smallest magnitude of the tile's A: is there a zero?
 #pragma unroll
-        for (int u = 0; u < NB - 1; ++u) fetch(u, u);
-        lookup(0, 0);
-        for (long long b = 0; b < nb; b += NB) {
+        for (int g = 0; g < GA; ++g)
+            if (16 * g + (int)(lane & 15u) < steps) low = min(low, __float_as_uint(a[g]) & 0x7FFFFFFFu);
+        if (__ballot(low == 0u) == 0ull) {
+            float4 lv[2][8];                               // 32 steps' levels, read while the 32 before are walked
+            auto read = [&](float4 (&dst)[8], int b) {
 #pragma unroll
-            for (int u = 0; u < NB; ++u) {
-                if (b + u < nb) {
-                    float a[UN];                           // A[m][32 (b+u) ..], uniform: requested before the look-ups
+                for (int j = 0; j < 8; ++j) dst[j] = *reinterpret_cast<const float4*>(src + 32 * b + 4 * j);
+            };
+            read(lv[0], 0);
 #pragma unroll
-                    for (int j = 0; j < UN; ++j) a[j] = a_row[(b + u) * UN + j];
-                    fetch((u + NB - 1) % NB, b + u + NB - 1);
-                    lookup((u + 1) % NB, (u + 1) & 1);     // batch b+u+1 (past the end: the clamped copy, never folded in)
-                    chain(a, u, u & 1);
+            for (int b = 0; b < kEngTile / 32; ++b) {
+                if (b + 1 < kEngTile / 32) read(lv[(b + 1) & 1], b + 1);
+                __builtin_amdgcn_sched_barrier(0);
+                const float4* l = lv[b & 1];
+                // acc += a[step] * level: the broadcast of lane `step` of each row of 16 rides on the FMA (the compiler
+                // keeps it as a move of its own, which doubles the chain's instructions).  A register that a VALU
+                // instruction has just written must not be read this way: a[] is written by memory loads only.
+#define ENG_STEP(J, LV) "v_fmac_f32_dpp %0, %1, %" #LV " row_newbcast:" #J " row_mask:0xf bank_mask:0xf\n\t"
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {              // one statement per 16 steps: the compiler puts a wait state between two
+                    const float4* q = l + 4 * h;
+                    asm(ENG_STEP(0, 2) ENG_STEP(1, 3) ENG_STEP(2, 4) ENG_STEP(3, 5) ENG_STEP(4, 6) ENG_STEP(5, 7) ENG_STEP(6, 8) ENG_STEP(7, 9)
+                        ENG_STEP(8, 10) ENG_STEP(9, 11) ENG_STEP(10, 12) ENG_STEP(11, 13) ENG_STEP(12, 14) ENG_STEP(13, 15) ENG_STEP(14, 16) ENG_STEP(15, 17)
+                        : "+v"(acc) : "v"(a[2 * b + h]), "v"(q[0].x), "v"(q[0].y), "v"(q[0].z), "v"(q[0].w), "v"(q[1].x), "v"(q[1].y), "v"(q[1].z),
+                          "v"(q[1].w), "v"(q[2].x), "v"(q[2].y), "v"(q[2].z), "v"(q[2].w), "v"(q[3].x), "v"(q[3].y), "v"(q[3].z), "v"(q[3].w));
                 }
+#undef ENG_STEP
+                __builtin_amdgcn_sched_barrier(0);
             }
+        } else {                                           // a zero: the reference skips the term, 0 * inf must not reach the sum
+#pragma unroll
+            for (int g = 0; g < GA; ++g)
+_Pragma("unroll 1")
+                for (int j = 0; j < 16 && 16 * g + j < steps; ++j) {
+                    const float x = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(a[g]), j));
+                    const float r = __fmaf_rn(x, src[16 * g + j], acc);
+                    acc = x != 0.0f ? r : acc;
+                }
+        }
+    };
+    float a0[GA], a1[GA];
+    fetch_a(a0, 0);
+    for (long long t = 0; t < tiles; t += 2) {
+        fetch_a(a1, t + 1);
+        __syncthreads();                                   // tile t is in lev[0]
+        walk(a0, mine, K - t * kEngTile < kEngTile ? (int)(K - t * kEngTile) : kEngTile);
+        if (t + 1 < tiles) {
+            fetch_a(a0, t + 2);
+            __syncthreads();
+            walk(a1, mine + COLS * kEngPitch, K - (t + 1) * kEngTile < kEngTile ? (int)(K - (t + 1) * kEngTile) : kEngTile);
         }
     }
-    const unsigned long long nn = n4 + sub;
-    for (long long k = nb * UN; k < K; ++k) {
-        const float a = a_row[k];
-        if (a == 0.0f) continue;
-        acc = __fmaf_rn(a, c[(uint32_t)bq[(unsigned long long)k * (unsigned long long)N + nn] * 64u + lane], acc);
-    }
-    if (live) C[m * N + n] = acc;
+    if (live && lane < (uint32_t)COLS && n0 + lane < N) C[m * N + n0 + lane] = acc;
+}
+
+__global__ void __launch_bounds__(256) engine_empty_kernel(float* __restrict__ C, long long n) {
+    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256) C[i] = 0.0f;
 }
 
 // The engines whose B operand is not a codebook index: kind 1 = Oil1Engine (one float per 32 flat positions,
@@ -384,6 +382,25 @@ engine_dequant_kernel(int bits, const uint8_t* __restrict__ idx, const float* __
             out[i] = __fmaf_rn(cb[idx[i] & 15u], scales[2 * b + 1], scales[2 * b]);
         }
     }
+}
+
+template <int BITS, int COLS>
+int launch_engine(const float* a, const uint8_t* b, const float* cb, float* c, int64_t M, int64_t N, int64_t K, hipStream_t s) {
+    static std::atomic<uint64_t> raised{0};
+    constexpr size_t lds = eng_lds(BITS, COLS);
+    if (int rc = ensure_max_lds(raised, (const void*)engine_kernel<BITS, COLS>, (int)lds)) return rc;
+    const int64_t rows = std::min<int64_t>(M, kEngMaxRows), groups = (N + COLS - 1) / COLS;   // rows of A of one workgroup share the levels
+    if (groups > 0x7FFFFFFFll) return fail(OILHIP_E_ARG, "N exceeds the grid limit");
+    hipLaunchKernelGGL((engine_kernel<BITS, COLS>), dim3((uint32_t)groups, (uint32_t)((M + rows - 1) / rows)),
+                       dim3((uint32_t)(64 * (eng_producers(COLS) + rows))), lds, s, a, b, cb, c, (long long)M, (long long)N, (long long)K);
+    OILHIP_HIP(hipGetLastError());
+    return OILHIP_OK;
+}
+
+template <int BITS>
+int launch_engine_bits(int cols, const float* a, const uint8_t* b, const float* cb, float* c, int64_t M, int64_t N, int64_t K, hipStream_t s) {
+    return cols == 16 ? launch_engine<BITS, 16>(a, b, cb, c, M, N, K, s)
+         : cols == 32 ? launch_engine<BITS, 32>(a, b, cb, c, M, N, K, s) : launch_engine<BITS, 64>(a, b, cb, c, M, N, K, s);
 }
 
 // Negative sizes are errors; an empty output (M or N zero) needs no pointers at all.
@@ -514,15 +531,17 @@ int oilhip_engine_quant_gemm(int bits, const float* d_a, const uint8_t* d_b, con
     if (bits != 2 && bits != 4 && bits != 8) return fail(OILHIP_E_ARG, "bits must be 2, 4 or 8");
     if (M == 0 || N == 0) return OILHIP_OK;
     if (M > 65535) return fail(OILHIP_E_ARG, "M exceeds the grid limit");
-    const dim3 grid((uint32_t)((N + 63) / 64), (uint32_t)M);
+    if (K == 0) {                                          // empty sums
+        hipLaunchKernelGGL(engine_empty_kernel, dim3((uint32_t)std::min<int64_t>((M * N + 255) / 256, 65535)), dim3(256), 0, (hipStream_t)stream, d_c, (long long)(M * N));
+        OILHIP_HIP(hipGetLastError());
+        return OILHIP_OK;
+    }
+    // as few columns per workgroup as keeps the launch at one workgroup per CU: two chains on one SIMD take turns
+    const int cus = device_cu_count(), cols = N <= 16ll * cus ? 16 : N <= 32ll * cus ? 32 : 64;
     hipStream_t s = (hipStream_t)stream;
-    if (bits == 8 && (N & 3) == 0 && N < (1ll << 29) && (reinterpret_cast<uintptr_t>(d_b) & 3u) == 0)
-        hipLaunchKernelGGL(engine8_quad_kernel, grid, dim3(64), 0, s, d_a, d_b, d_cb, d_c, M, N, K);
-    else if (bits == 8) hipLaunchKernelGGL(engine_kernel<8>, grid, dim3(64), 0, s, d_a, d_b, d_cb, d_c, M, N, K);
-    else if (bits == 4) hipLaunchKernelGGL(engine_kernel<4>, grid, dim3(64), 0, s, d_a, d_b, d_cb, d_c, M, N, K);
-    else hipLaunchKernelGGL(engine_kernel<2>, grid, dim3(64), 0, s, d_a, d_b, d_cb, d_c, M, N, K);
-    OILHIP_HIP(hipGetLastError());
-    return OILHIP_OK;
+    return bits == 8 ? launch_engine_bits<8>(cols, d_a, d_b, d_cb, d_c, M, N, K, s)
+         : bits == 4 ? launch_engine_bits<4>(cols, d_a, d_b, d_cb, d_c, M, N, K, s)
+                     : launch_engine_bits<2>(cols, d_a, d_b, d_cb, d_c, M, N, K, s);
 }
 
 int oilhip_engine_dequant(int bits, const uint8_t* d_idx, const float* d_cb, int64_t n, const float* d_scales,

@@ -142,3 +142,22 @@ def test_engine_dequant_bit_exact():
         assert np.array_equal(np.asarray(got).view(np.uint32), gold[f"pb{bits}"]), bits
     with pytest.raises(ia.OilHipError):
         ia.kernel.engine_dequant(2, np.zeros(4, np.uint8), np.zeros(4, np.float32), 4, scales=np.zeros(1, np.float32), block_size=4)
+
+
+@pytest.mark.parametrize("bits,M,N,K", [(8, 1, 16, 255), (8, 5, 33, 257), (8, 2, 9001, 300), (4, 1, 17, 512), (4, 3, 4097, 511), (4, 4, 8193, 30),
+                                        (2, 1, 1, 1), (2, 9, 63, 769), (2, 1, 8200, 513)])
+def test_engine_quant_gemm_tiles_and_remainders(bits, M, N, K):
+    """Edges of the engine kernel's tiles (256 steps; 16, 32 or 64 columns; 4 rows), codes at every bit offset (odd N), and the
+    skipped terms: zeros of A in some tiles meet an infinite level, whole tiles without a zero take the unchecked chain."""
+    rng = np.random.default_rng(bits * 1000 + N)
+    A = rng.standard_normal((M, K)).astype(np.float32)
+    A[:, : K // 2][rng.random((M, K // 2)) < 0.1] = 0.0
+    A[0, K // 3] = -0.0
+    b = rng.integers(0, 256, (K * N * bits + 7) // 8, dtype=np.uint8)
+    cb = rng.standard_normal(1 << bits).astype(np.float32)
+    if K > 256:
+        cb[0] = np.inf
+    got = ia.kernel.engine_quant_gemm(bits, A, b, cb, M, N, K)
+    want = O.engine_quant_gemm(bits, A, b, cb, M, N, K)
+    assert np.array_equal(got.view(np.uint32)[~np.isnan(want)], want.view(np.uint32)[~np.isnan(want)])
+    assert np.array_equal(np.isnan(got), np.isnan(want))
