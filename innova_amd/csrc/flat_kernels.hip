@@ -3,36 +3,26 @@
 //   oil::kernel::oil8_gemm / oil4_gemm          src/kernel_oil8.cpp, src/kernel_oil4.cpp
 //   oil::adapters::prod::gemv_{spark,oil4,oil8} src/kernel_production.cpp:79-128,345-364
 //   oil::engines::OIL{8,4,2}Engine::quant_gemm  src/oil_engines_oil{8,4,2}.cpp
-// One workgroup of 256 threads per output row; the codebook sits in LDS; thread t
-// walks k = t, t+256, ... so index bytes are read coalesced.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
+#include "oil4_lds.h"
 
 namespace oilhip {
 namespace {
 
-constexpr int MBF = 4;   // activation rows per pass
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 
+// sum over the wavefront, in lane 63
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    v += oil4::dpp_quad_xor1(v);
+    v += oil4::dpp_quad_xor2(v);
+    v += oil4::dpp_half_mirror(v);
+    v += oil4::dpp_row_mirror(v);
+    v += oil4::dpp_row_bcast15(v);
+    v += oil4::dpp_row_bcast31(v);
     return v;
-}
-
-// Sum acc[0..MBF) over the 256 threads; thread b < MBF returns the total of acc[b].
-__device__ __forceinline__ float block_sums(const float (&acc)[MBF], float (*part)[4]) {
-    const uint32_t t = threadIdx.x;
-#pragma unroll
-    for (int b = 0; b < MBF; ++b) {
-        const float s = wave_sum(acc[b]);
-        if ((t & 63) == 0) part[b][t >> 6] = s;
-    }
-    __syncthreads();
-    float r = 0.0f;
-    if (t < MBF) r = (part[t][0] + part[t][1]) + (part[t][2] + part[t][3]);
-    __syncthreads();
-    return r;
 }
 
 // FP16 codebook entry exactly as fp16_to_float (src/kernel_oil4.cpp:15-29).
@@ -42,78 +32,218 @@ __device__ __forceinline__ float flat_half(uint16_t h) {
     return half_bits_to_float(h);
 }
 
-// mode 0: oil8_gemm  -- weights row n (K bytes),        activations row m, out[m*N+n]
-// mode 1: prod oil8  -- weights row n (K bytes),        activations row m, out[m*N+n] * scale
-__global__ void __launch_bounds__(256)
-flat8_kernel(const uint8_t* __restrict__ idx, const float* __restrict__ cb, const float* __restrict__ act,
-             float* __restrict__ out, int M, int N, int K, float scale) {
-    __shared__ float c[256];
-    __shared__ float part[MBF][4];
-    const uint32_t t = threadIdx.x, n = blockIdx.x;
-    c[t] = cb[t];
-    __syncthreads();
-    const uint8_t* w = idx + (size_t)n * K;
-    for (int m0 = 0; m0 < M; m0 += MBF) {
-        float acc[MBF] = {0.0f, 0.0f, 0.0f, 0.0f};
-        for (int k = t; k < K; k += 256) {
-            const float v = c[w[k]];
-#pragma unroll
-            for (int b = 0; b < MBF; ++b)
-                if (m0 + b < M) acc[b] = __fmaf_rn(v, act[(size_t)(m0 + b) * K + k], acc[b]);
-        }
-        const float r = block_sums(acc, part);
-        if (t < MBF && m0 + (int)t < M) out[(size_t)(m0 + t) * N + n] = r * scale;
-    }
-}
+// One row (or R rows) of codes against activations: kernel::oil4_gemm, the production GEMVs and the index-byte forms that
+// gemv_oil8.hip does not take.  BITS = 8: a byte per weight, codebook of 256 floats; 4: a nibble, FP16 codebook of 16; 2:
+// SPARK ternary (0 -> -1, 1 -> 0, 2 and 3 -> +1).
+// What bounds it: bytes from memory at the large sizes, the launch at the small ones; the form this replaces (a workgroup
+// per row, a byte load, a shift and a table read in LDS per weight and thread) was bound by its instructions.  A lane takes
+// UNIT consecutive weights of every row with one load, at any alignment, and the activations of those weights once for
+// the R rows; nibbles and ternary codes become FP16 pairs by byte permutes of a codebook held in registers (16 entries are
+// two 8-byte tables for each half of an FP16 value; the code's top bit selects between them) and enter the FP32 sum
+// through v_fma_mix.  The four wavefronts of a workgroup take every fourth 64 * UNIT weights of the same rows, so that a
+// short row still occupies them all.  4096 x 4096, M = 1, before -> after: SPARK 10.9 -> 6.7 us (the host's launch rate); M = 4:
+// SPARK 19.9 -> 7.6, production OIL4 22.1 -> 9.0, M = 8: OIL8 63 -> 16; oil4_gemm M = 6, 3000 x 2044: 42.6 -> 20.8.
+struct FlatRows {
+    const uint8_t* w;            // row r starts at byte r * row_bytes; PAIR: row (m, n) at byte ((m * rows + n) * K) / 2
+    const void* cb;
+    const float* x;              // activation row b at x + b * K; PAIR: row n
+    float* y;                    // y[b * rows + r]; PAIR: y[m * rows + n]
+    float scale;
+    uint32_t rows, K, batch;     // PAIR: batch = M
+    uint64_t row_bytes;
+    const uint8_t* last = nullptr;   // the codes' last dword, when a lane's codes can start off a dword; else nullptr
+};
 
-// oil4_gemm: one workgroup per (m, n) pair; the pair's K nibbles start at nibble
-// (m*N+n)*K rounded down to a byte, activations are row n (src/kernel_oil4.cpp:38-56).
-__global__ void __launch_bounds__(256)
-flat4_pair_kernel(const uint8_t* __restrict__ packed, const uint16_t* __restrict__ cb16,
-                  const float* __restrict__ act, float* __restrict__ out, int N, int K) {
-    __shared__ float c[16];
-    __shared__ float part[MBF][4];
-    const uint32_t t = threadIdx.x;
-    const uint64_t pair = blockIdx.x;
-    if (t < 16) c[t] = flat_half(cb16[t]);
-    __syncthreads();
-    const uint8_t* w = packed + (pair * (uint64_t)K) / 2;
-    const float* a = act + (pair % (uint64_t)N) * (uint64_t)K;
-    float acc[MBF] = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int k = t; k < K; k += 256) {
-        const uint32_t byte = w[k >> 1];
-        acc[0] = __fmaf_rn(c[(k & 1) ? (byte >> 4) : (byte & 15u)], a[k], acc[0]);
-    }
-    const float r = block_sums(acc, part);
-    if (t == 0) out[pair] = r;
+// 32 bits that start at bit `bit` behind p, from the one or two dwords they lie in; `last` keeps the second inside the array.
+__device__ __forceinline__ uint32_t load_bits32(const uint8_t* p, uint32_t bit, const uint8_t* last) {
+    const uintptr_t at = reinterpret_cast<uintptr_t>(p) + (bit >> 3), q = at & ~(uintptr_t)3, l = reinterpret_cast<uintptr_t>(last);
+    const uint32_t a = *reinterpret_cast<const uint32_t*>(q), b = *reinterpret_cast<const uint32_t*>(q < l ? q + 4 : l);
+    return __builtin_amdgcn_alignbit(b, a, (uint32_t)(at & 3) * 8u + (bit & 7u));
 }
+__device__ __forceinline__ float4 load_f4(const float* p) { float4 v; __builtin_memcpy(&v, p, 16); return v; }
 
-// prod gemv over packed rows: BITS = 4 (two codes per byte, FP16 codebook) or
-// BITS = 2 (SPARK ternary: 0 -> -1, 1 -> 0, 2 and 3 -> +1).  Row m of W against
-// activation row b; Y[b*M + m] = scale * dot.
 template <int BITS>
-__global__ void __launch_bounds__(256)
-prod_packed_kernel(const uint8_t* __restrict__ wq, const uint16_t* __restrict__ cb16, float scale,
-                   const float* __restrict__ x, float* __restrict__ y, int M, int K, int batch) {
-    __shared__ float c[16];
-    __shared__ float part[MBF][4];
-    const uint32_t t = threadIdx.x, m = blockIdx.x;
-    if (BITS == 4 && t < 16) c[t] = flat_half(cb16[t]);
-    __syncthreads();
-    constexpr int PER = 8 / BITS;
-    const uint8_t* row = wq + (size_t)m * ((K + PER - 1) / PER);
-    for (int b0 = 0; b0 < batch; b0 += MBF) {
-        float acc[MBF] = {0.0f, 0.0f, 0.0f, 0.0f};
-        for (int k = t; k < K; k += 256) {
-            const uint32_t code = (row[k / PER] >> ((k % PER) * BITS)) & ((1u << BITS) - 1u);
-            const float v = BITS == 4 ? c[code] : (code == 0 ? -1.0f : (code == 1 ? 0.0f : 1.0f));
+struct FlatBook;
+
+template <>
+struct FlatBook<4> {                                       // low bytes of entries 0-3, 4-7, 8-11, 12-15, then high bytes
+    uint32_t lo[4], hi[4];
+    __device__ __forceinline__ void init(const void* cb, const float*) {
+        const uint16_t* c = reinterpret_cast<const uint16_t*>(cb);
 #pragma unroll
-            for (int b = 0; b < MBF; ++b)
-                if (b0 + b < batch) acc[b] = __fmaf_rn(v, x[(size_t)(b0 + b) * K + k], acc[b]);
+        for (int g = 0; g < 4; ++g) {
+            lo[g] = hi[g] = 0u;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) { const uint32_t h = c[4 * g + j]; lo[g] |= (h & 255u) << (8 * j); hi[g] |= (h >> 8) << (8 * j); }
         }
-        const float r = block_sums(acc, part);
-        if (t < MBF && b0 + (int)t < batch) y[(size_t)(b0 + t) * M + m] = r * scale;
     }
+    // eight nibbles of d -> f(i, value), i = 0 .. 7
+    template <class F>
+    __device__ __forceinline__ void each(uint32_t d, F&& f) const {
+#pragma unroll
+        for (int odd = 0; odd < 2; ++odd) {
+            const uint32_t n = odd ? d >> 4 : d, at = n & 0x07070707u;
+            const uint32_t top = __builtin_amdgcn_perm(0u, 0u, (n & 0x08080808u) | 0x05050505u);   // 0xFF in bytes whose code is 8 or more (selector 13), else 0
+            const uint32_t l = (__builtin_amdgcn_perm(lo[1], lo[0], at) & ~top) | (__builtin_amdgcn_perm(lo[3], lo[2], at) & top);
+            const uint32_t h = (__builtin_amdgcn_perm(hi[1], hi[0], at) & ~top) | (__builtin_amdgcn_perm(hi[3], hi[2], at) & top);
+            const auto p0 = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(h, l, 0x05010400u));
+            const auto p1 = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(h, l, 0x07030602u));
+            f(odd, (float)p0[0]); f(odd + 2, (float)p0[1]); f(odd + 4, (float)p1[0]); f(odd + 6, (float)p1[1]);
+        }
+    }
+    __device__ __forceinline__ float one(uint32_t code) const {
+        const uint32_t g = code >> 2, sh = 8u * (code & 3u);
+        const uint32_t l = g == 0u ? lo[0] : g == 1u ? lo[1] : g == 2u ? lo[2] : lo[3], h = g == 0u ? hi[0] : g == 1u ? hi[1] : g == 2u ? hi[2] : hi[3];
+        return flat_half((uint16_t)(((l >> sh) & 255u) | (((h >> sh) & 255u) << 8)));
+    }
+};
+
+template <>
+struct FlatBook<2> {
+    __device__ __forceinline__ void init(const void*, const float*) {}
+    // sixteen codes of d; codes i and i + 8 become one FP16 pair (only the high bytes differ: 0xBC, 0x00, 0x3C, 0x3C)
+    template <class F>
+    __device__ __forceinline__ void each(uint32_t d, F&& f) const {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const uint32_t at = ((i < 4 ? d << (8 - 2 * i) : d >> (2 * i - 8)) & 0x03000300u) | 0x000C000Cu;
+            const auto p = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0u, 0x3C3C00BCu, at));
+            f(i, (float)p[0]); f(i + 8, (float)p[1]);
+        }
+    }
+    __device__ __forceinline__ float one(uint32_t code) const { return code == 0u ? -1.0f : code == 1u ? 0.0f : 1.0f; }
+};
+
+template <>
+struct FlatBook<8> {
+    const float* tab;                                      // LDS: entry v of copy c at v * 16 + c
+    uint32_t copy;
+    __device__ __forceinline__ void init(const void*, const float* lds) { tab = lds; copy = threadIdx.x & 15u; }
+    template <class F>
+    __device__ __forceinline__ void each(uint32_t d, F&& f) const {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) f(i, tab[((d >> (8 * i)) & 255u) * 16u + copy]);
+    }
+    __device__ __forceinline__ float one(uint32_t code) const { return tab[code * 16u + copy]; }
+};
+
+// R rows (PAIR: the rows of R values of m for one n) against B activation rows (PAIR: one).
+template <int BITS, int R, int B, bool PAIR>
+__global__ void __launch_bounds__(256)
+flat_rows_kernel(const FlatRows a) {
+    constexpr uint32_t PER = 32 / BITS, WORDS = BITS == 2 ? 1 : 8 / PER, UNIT = PER * WORDS;   // weights of a lane per step: 16 or 8
+    __shared__ float tab[BITS == 8 ? 256 * 16 : 1];
+    __shared__ float part[4][R * B];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    if (BITS == 8) {
+        for (uint32_t i = tid; i < 256u * 16u; i += 256u) tab[i] = reinterpret_cast<const float*>(a.cb)[i >> 4];
+        __syncthreads();
+    }
+    FlatBook<BITS> book;
+    book.init(a.cb, tab);
+    const uint32_t groups = PAIR ? a.rows : (a.rows + R - 1) / R, bg = blockIdx.x / groups, rg = blockIdx.x - bg * groups;
+    const uint32_t r0 = PAIR ? rg : rg * R, b0 = bg * (PAIR ? R : B);
+    const uint8_t* w[R];
+    const float* x[B];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {                          // rows past the end repeat the last one
+        if (PAIR) {
+            const uint64_t pair = (uint64_t)min(b0 + r, a.batch - 1u) * a.rows + r0;
+            w[r] = a.w + pair * a.K / 2;
+        } else {
+            w[r] = a.w + (uint64_t)min(r0 + r, a.rows - 1u) * a.row_bytes;
+        }
+    }
+#pragma unroll
+    for (int b = 0; b < B; ++b) x[b] = a.x + (uint64_t)(PAIR ? r0 : min(b0 + b, a.batch - 1u)) * a.K;
+    float acc[R][B] = {};
+    if (a.K >= UNIT) {
+        for (uint32_t k0 = (wave * 64u + lane) * UNIT; k0 < a.K; k0 += 256u * UNIT) {
+            // the lane that would run past the row's end takes the row's last UNIT weights and leaves out what its
+            // neighbour has: a remainder walked weight by weight is a chain of loads (K = 4092: 12.3 us with it, 7.1 without)
+            const uint32_t k = k0 + UNIT <= a.K ? k0 : a.K - UNIT, skip = k0 - k;
+            uint32_t d[R][WORDS];
+            if (a.last) {
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+#pragma unroll
+                    for (uint32_t q = 0; q < WORDS; ++q) d[r][q] = load_bits32(w[r], (k + q * PER) * BITS, a.last);
+            } else {
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+#pragma unroll
+                    for (uint32_t q = 0; q < WORDS; ++q) d[r][q] = reinterpret_cast<const uint32_t*>(w[r] + k * BITS / 8)[q];
+            }
+            float xv[B][UNIT];
+#pragma unroll
+            for (int b = 0; b < B; ++b)
+#pragma unroll
+                for (uint32_t q = 0; q < UNIT / 4; ++q) {
+                    const float4 v = load_f4(x[b] + k + 4 * q);
+                    xv[b][4 * q] = v.x; xv[b][4 * q + 1] = v.y; xv[b][4 * q + 2] = v.z; xv[b][4 * q + 3] = v.w;
+                }
+            auto products = [&](auto masked) {
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+#pragma unroll
+                    for (uint32_t q = 0; q < WORDS; ++q)
+                        book.each(d[r][q], [&](int i, float v) {
+                            if (masked.value) v = q * PER + i >= skip ? v : 0.0f;       // both factors: the other may be infinite
+#pragma unroll
+                            for (int b = 0; b < B; ++b) acc[r][b] = __builtin_fmaf(v, xv[b][q * PER + i], acc[r][b]);
+                        });
+            };
+            if (__ballot(skip != 0u) == 0ull) {
+                products(std::false_type{});
+            } else {
+#pragma unroll
+                for (int b = 0; b < B; ++b)
+#pragma unroll
+                    for (uint32_t i = 0; i < UNIT; ++i) xv[b][i] = i >= skip ? xv[b][i] : 0.0f;
+                products(std::true_type{});
+            }
+        }
+    } else if (tid < a.K) {                                // rows shorter than a lane's share
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const float v = book.one((w[r][tid * BITS / 8] >> (tid * BITS % 8)) & ((1u << BITS) - 1u));
+#pragma unroll
+            for (int b = 0; b < B; ++b) acc[r][b] = v * x[b][tid];
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int b = 0; b < B; ++b) {
+            const float v = wave_sum(acc[r][b]);
+            if (lane == 63u) part[wave][r * B + b] = v;
+        }
+    __syncthreads();
+    if (tid < R * B) {
+        const uint32_t r = tid / B, b = tid % B;
+        const float v = ((part[0][tid] + part[1][tid]) + (part[2][tid] + part[3][tid])) * a.scale;
+        if (PAIR) { if (b0 + r < a.batch) a.y[(uint64_t)(b0 + r) * a.rows + r0] = v; }
+        else if (r0 + r < a.rows && b0 + b < a.batch) a.y[(uint64_t)(b0 + b) * a.rows + r0 + r] = v;
+    }
+}
+
+template <int BITS, int R, int B, bool PAIR>
+int launch_flat_rows(FlatRows a, hipStream_t s) {
+    const uint64_t bytes = PAIR ? ((uint64_t)a.batch * a.rows * a.K + 1) / 2 : a.rows * a.row_bytes;
+    if (bytes && ((reinterpret_cast<uintptr_t>(a.w) & 3u) || (a.K & (32u / BITS - 1u)) || (!PAIR && (a.row_bytes & 3u))))
+        a.last = reinterpret_cast<const uint8_t*>((reinterpret_cast<uintptr_t>(a.w) + bytes - 1) & ~(uintptr_t)3);
+    const uint64_t gx = PAIR ? a.rows : (a.rows + R - 1) / R, gy = (a.batch + (PAIR ? R : B) - 1) / (PAIR ? R : B);
+    if (gx * gy > 0x7FFFFFFFull) return fail(OILHIP_E_ARG, "outputs exceed the grid limit");
+    hipLaunchKernelGGL((flat_rows_kernel<BITS, R, B, PAIR>), dim3((uint32_t)(gx * gy)), dim3(256), 0, s, a);
+    OILHIP_HIP(hipGetLastError());
+    return OILHIP_OK;
+}
+
+// Rows per workgroup: four share the activations' loads; few rows go one per workgroup so that every CU has some.
+template <int BITS>
+int launch_flat_rows(const FlatRows& a, hipStream_t s) {
+    if (a.rows < 2048u) return a.batch == 1 ? launch_flat_rows<BITS, 1, 1, false>(a, s) : a.batch == 2 ? launch_flat_rows<BITS, 1, 2, false>(a, s) : launch_flat_rows<BITS, 1, 4, false>(a, s);
+    return a.batch == 1 ? launch_flat_rows<BITS, 4, 1, false>(a, s) : a.batch == 2 ? launch_flat_rows<BITS, 4, 2, false>(a, s) : launch_flat_rows<BITS, 4, 4, false>(a, s);
 }
 
 // OIL{8,4,2}Engine::quant_gemm: codes packed along the flat [K][N] index, every output one k-ordered chain of fused
@@ -426,9 +556,7 @@ int oilhip_flat_oil8_gemm(const uint8_t* d_idx, const float* d_cb, const float* 
         const int rc = launch_gemv_flat8(d_idx, d_cb, d_act, d_out, M, N, K, 1.0f, (hipStream_t)stream);
         if (rc <= 0) return rc;
     }
-    hipLaunchKernelGGL(flat8_kernel, dim3(N), dim3(256), 0, (hipStream_t)stream, d_idx, d_cb, d_act, d_out, M, N, K, 1.0f);
-    OILHIP_HIP(hipGetLastError());
-    return OILHIP_OK;
+    return launch_flat_rows<8>(FlatRows{d_idx, d_cb, d_act, d_out, 1.0f, (uint32_t)N, (uint32_t)K, (uint32_t)M, (uint64_t)K}, (hipStream_t)stream);
 }
 
 int oilhip_flat_oil4_gemm(const uint8_t* d_packed, const uint16_t* d_cb16, const float* d_act, float* d_out,
@@ -436,36 +564,27 @@ int oilhip_flat_oil4_gemm(const uint8_t* d_packed, const uint16_t* d_cb16, const
     if (int rc = check(d_packed, d_cb16, d_act, d_out, M, N, K)) return rc;
     if (M == 0 || N == 0) return OILHIP_OK;
     if ((long long)M * N > 0x7FFFFFFFll) return fail(OILHIP_E_ARG, "M*N exceeds the grid limit");
-    hipLaunchKernelGGL(flat4_pair_kernel, dim3((uint32_t)((long long)M * N)), dim3(256), 0, (hipStream_t)stream,
-                       d_packed, d_cb16, d_act, d_out, N, K);
-    OILHIP_HIP(hipGetLastError());
-    return OILHIP_OK;
+    const FlatRows a{d_packed, d_cb16, d_act, d_out, 1.0f, (uint32_t)N, (uint32_t)K, (uint32_t)M, 0};
+    return M == 1 ? launch_flat_rows<4, 1, 1, true>(a, (hipStream_t)stream) : M == 2 ? launch_flat_rows<4, 2, 1, true>(a, (hipStream_t)stream)
+                  : launch_flat_rows<4, 4, 1, true>(a, (hipStream_t)stream);
 }
 
 int oilhip_prod_gemv_spark(const uint8_t* d_w, float scale, const float* d_x, float* d_y,
                            int M, int K, int batch, void* stream) {
     if (int rc = check(d_w, d_x, d_y, d_y, M, batch, K)) return rc;
     if (M == 0 || batch == 0) return OILHIP_OK;
-    hipLaunchKernelGGL(prod_packed_kernel<2>, dim3(M), dim3(256), 0, (hipStream_t)stream, d_w,
-                       (const uint16_t*)nullptr, scale, d_x, d_y, M, K, batch);
-    OILHIP_HIP(hipGetLastError());
-    return OILHIP_OK;
+    return launch_flat_rows<2>(FlatRows{d_w, nullptr, d_x, d_y, scale, (uint32_t)M, (uint32_t)K, (uint32_t)batch, ((uint64_t)K + 3) / 4}, (hipStream_t)stream);
 }
 
 int oilhip_prod_gemv_oil4(const uint8_t* d_w, const uint16_t* d_cb16, float scale, const float* d_x,
                           float* d_y, int M, int K, int batch, void* stream) {
     if (int rc = check(d_w, d_cb16, d_x, d_y, M, batch, K)) return rc;
     if (M == 0 || batch == 0) return OILHIP_OK;
-    if (batch <= 2) {                                 // decode: the register-resident kernel, one activation row per launch
-        int rc = 0;
-        for (int b = 0; b < batch && rc == 0; ++b)
-            rc = launch_gemv_flat4(d_w, d_cb16, scale, d_x + (size_t)b * K, d_y + (size_t)b * M, M, K, (hipStream_t)stream);
+    if (batch == 1) {                                 // decode: the register-resident kernel (11008 x 4096: 7.6 us against 11.4)
+        const int rc = launch_gemv_flat4(d_w, d_cb16, scale, d_x, d_y, M, K, (hipStream_t)stream);
         if (rc <= 0) return rc;
     }
-    hipLaunchKernelGGL(prod_packed_kernel<4>, dim3(M), dim3(256), 0, (hipStream_t)stream, d_w, d_cb16, scale,
-                       d_x, d_y, M, K, batch);
-    OILHIP_HIP(hipGetLastError());
-    return OILHIP_OK;
+    return launch_flat_rows<4>(FlatRows{d_w, d_cb16, d_x, d_y, scale, (uint32_t)M, (uint32_t)K, (uint32_t)batch, ((uint64_t)K + 1) / 2}, (hipStream_t)stream);
 }
 
 // Y[b*M + m]: the flat OIL8 kernel with (rows = M weight rows, batch = activation rows).
@@ -477,9 +596,7 @@ int oilhip_prod_gemv_oil8(const uint8_t* d_w, const float* d_cb, float scale, co
         const int rc = launch_gemv_flat8(d_w, d_cb, d_x, d_y, batch, M, K, scale, (hipStream_t)stream);
         if (rc <= 0) return rc;
     }
-    hipLaunchKernelGGL(flat8_kernel, dim3(M), dim3(256), 0, (hipStream_t)stream, d_w, d_cb, d_x, d_y, batch, M, K, scale);
-    OILHIP_HIP(hipGetLastError());
-    return OILHIP_OK;
+    return launch_flat_rows<8>(FlatRows{d_w, d_cb, d_x, d_y, scale, (uint32_t)M, (uint32_t)K, (uint32_t)batch, (uint64_t)K}, (hipStream_t)stream);
 }
 
 // profile_gemv_{spark,oil4,oil8} (src/kernel_production.cpp:433-485): `repeats` launches of the tiled GEMV between two

@@ -161,3 +161,25 @@ def test_engine_quant_gemm_tiles_and_remainders(bits, M, N, K):
     want = O.engine_quant_gemm(bits, A, b, cb, M, N, K)
     assert np.array_equal(got.view(np.uint32)[~np.isnan(want)], want.view(np.uint32)[~np.isnan(want)])
     assert np.array_equal(np.isnan(got), np.isnan(want))
+
+
+@pytest.mark.parametrize("rows,K,batch", [(1, 1, 1), (3, 15, 2), (5, 17, 3), (257, 1024, 1), (2047, 513, 5), (2049, 260, 1), (2050, 4097, 2), (2053, 2048, 9)])
+def test_flat_rows_remainders(rows, K, batch):
+    """Rows, activation rows and row lengths around the tiles of the flat-codebook kernel (4 rows, 4 activation rows, 8 or 16
+    weights per lane, 256 lanes), rows that start at any byte."""
+    rng = np.random.default_rng(rows + K)
+    X = rng.standard_normal((batch, K)).astype(np.float32)
+    cb16 = rng.standard_normal(16).astype(np.float16).view(np.uint16)
+    cb8 = rng.standard_normal(256).astype(np.float32)
+    ws = rng.integers(0, 256, rows * ((K + 3) // 4), dtype=np.uint8)
+    w4 = rng.integers(0, 256, rows * ((K + 1) // 2), dtype=np.uint8)
+    w8 = rng.integers(0, 256, rows * K, dtype=np.uint8)
+    assert rel_l2(ia.kernel.gemv_spark_batch(ws, 1.7, X, rows, batch, K), np.stack([O.gemv_spark(ws, 1.7, x, rows, K, 1) for x in X])) <= TOL
+    assert rel_l2(ia.kernel.gemv_oil4_batch(w4, cb16, 1.7, X, rows, batch, K), np.stack([O.gemv_oil4(w4, cb16, 1.7, x, rows, K, 1) for x in X])) <= TOL
+    y8 = np.stack([O.gemv_oil8(w8, cb8, 1.7, x, rows, K, 1) for x in X])
+    assert rel_l2(ia.kernel.gemv_oil8_batch(w8, cb8, 1.7, X, rows, batch, K), y8) <= TOL
+    assert rel_l2(ia.kernel.oil8_gemm(w8, cb8, X, batch, rows, K), y8 / np.float32(1.7)) <= TOL
+    n = min(rows, 300)                                     # the pair form: a packed row per (m, n), activations by n
+    packed = rng.integers(0, 256, (batch * n * K + 1) // 2, dtype=np.uint8)
+    act = rng.standard_normal((n, K)).astype(np.float32)
+    assert rel_l2(ia.kernel.oil4_gemm(packed, cb16, act, batch, n, K), O.oil4_gemm(packed, cb16, act, batch, n, K)) <= TOL
