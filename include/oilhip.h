@@ -172,20 +172,17 @@ int oilhip_gemv_f32(const oilhip_weights* w, const float* d_x, float* d_y, int M
 
 /* The same product for uniform OIL4 tensors, for callers that cannot allocate device memory (code under HIP graph
  * capture, serving loops and harnesses that forbid hipMalloc).  No counterpart in the reference.  It calls no
- * hipMalloc/hipFree: the scratch its multi-row kernel needs (packed activations and their exponents, 8 MB) is a fixed array in the
- * library's code object, one per GPU.  Limits: uniform OIL4 in the plain block layout, cols <= 32768; and, where
- * the rows are cut into three or more parts along K whose sums meet in the scratch (M >= 3 with cols > 8192, or
- * M > 16 with cols > 4096, ordered sums on), parts * tokens_per_pass * rows <= 1,043,456 floats (parts =
+ * hipMalloc/hipFree: the scratch its multi-row kernel needs (packed activations and their powers of two, 8 MB) is a fixed array in the
+ * library's code object, one per GPU.  Limits: uniform OIL4 in the plain block layout, cols <= 32768; and, for
+ * wide rows (M >= 3 with cols > 8192, or M > 16 with cols > 4096), parts * tokens_per_pass * rows <= 1,043,456 (parts =
  * ceil(cols / 4096) for passes of up to 16 tokens, ceil(cols / 2048) for passes of 32; e.g. cols = 11008, M <= 16:
- * rows <= 21,738).  Anything else returns OILHIP_E_ARG.  All calls on one GPU share that array: calls that overlap on one GPU (two streams, two
+ * rows <= 21,738), whatever the kernel would need.  Anything else returns OILHIP_E_ARG.  All calls on one GPU share that array: calls that overlap on one GPU (two streams, two
  * threads) race on it and must be serialized by the caller. */
 int oilhip_gemv_oil4_f32_noalloc(const oilhip_weights* w, const float* d_x, float* d_y, int M, void* stream);
 
-/* Rows too wide for one workgroup pass of the multi-row OIL4 kernel (more than 16 blocks, 8 for batches beyond 16 rows)
- * are cut into parts whose partial sums have to meet.  ordered = 1 (the default): three or more parts are added in a
- * fixed order through a workspace, so a call returns the same bits every time, like the reference's sequential loop
- * (src/adapters/tools/qwen35_engine.cpp:71-78).  ordered = 0: float atomics, a few microseconds faster, last bits may
- * differ from run to run (within the 1e-5 bound).  Process-wide. */
+/* The multi-row OIL4 kernel adds everything in a fixed order inside a workgroup, so a call returns the same bits every
+ * time, like the reference's sequential loop (src/adapters/tools/qwen35_engine.cpp:71-78).  The call is accepted for
+ * either argument and changes nothing. */
 int oilhip_set_ordered_sums(int ordered);
 
 

@@ -101,7 +101,8 @@ int stream_scratch(hipStream_t s, int slot, size_t bytes, void** out) {
             (void)hipGetLastError();
             return fail(OILHIP_E_NOMEM, "hipMalloc of " + std::to_string(want) + " bytes of scratch failed");
         }
-        if (hipMemset(p, 0, want) != hipSuccess) {
+        // on the stream that will use it: a clear on the null stream is not ordered before launches on a non-blocking stream
+        if (hipMemsetAsync(p, 0, want, s) != hipSuccess) {
             (void)hipGetLastError();
             (void)hipFree(p);
             return fail(OILHIP_E_DEVICE, "hipMemset of the new scratch failed");

@@ -115,29 +115,25 @@ int launch_gemv_oil8(const oilhip_weights& w, const float* d_x, float* d_y, int 
 // kernel::oil8_gemm form: rows of K index bytes, any 256-entry codebook; out[m*N + n] = scale * dot
 int launch_gemv_flat8(const uint8_t* d_idx, const float* d_cb, const float* d_act, float* d_out, int M, int N, int K, float scale,
                       hipStream_t s);
-// several activation rows at once (FP32 MFMA); x row tok[m] (or m) of an [xrows][ldx] matrix, y row stride ldy
-int launch_gemv_oil4_multi(const oilhip_weights& w, const float* d_x, const int* d_tok, float* d_y, int M,
-                           uint32_t ldx, uint32_t ldy, uint32_t xrows, hipStream_t s, const oilhip_weights* w2 = nullptr,
-                           float* d_y2 = nullptr, uint32_t ldy2 = 0, const float* d_x2 = nullptr, uint32_t* d_pack = nullptr,
-                           size_t pack_cap = 0);
-void g_ordered_sums_set(int v);
-// several batches of one tensor shape in one launch (gemv_oil4_multi.hip); kinds[b] = 0 / 1 / 2: batch b holds up to 8 / 16 / 32 rows
-size_t gemv_oil4_multi_batches_bytes(int nb, uint64_t rows, uint64_t cols, bool two_tensors);   // two_tensors: every batch goes through wa[b] and wb[b]
-int launch_gemv_oil4_multi_batches(int nb, const int* kinds, const oilhip_weights* const* wa, float* const* ya,
-                                   const oilhip_weights* const* wb, float* const* yb, const int* M, const int* row0,
-                                   const int* list, int nlist, const float* d_x, const float* d_x2, uint32_t ldx, uint32_t xrows,
-                                   uint32_t ldy, void* d_ws, size_t ws_bytes, hipStream_t s, bool counters_clean = false,
-                                   float* d_parts = nullptr, uint32_t parts_rows = 0);
-uint32_t gemv_oil4_multi_parts(int kind, uint64_t cols);
-bool gemv_oil4_multi_ordered();
-// clears the slab counters at the start of a batch workspace; launches over it may then be told that they are clean
-constexpr size_t kGemvBatchCounterBytes = 32u * 4096u;   // slab counters at the start of a batch workspace: a 4 KB page per job
-int zero_gemv_oil4_multi_batch_counters(void* d_ws, hipStream_t s);
-bool gemv_oil4_multi_batches_accumulate(int kind, uint64_t cols);
-// widest row that kernel takes and the bytes of packed activations one pass of it needs (d_pack, or stream scratch)
+// several activation rows at once (INT8 MFMA, gemv_oil4_multi.hip); x row tok[m] (or m) of an [xrows][ldx] matrix, y row
+// stride ldy.  What a row is multiplied as: itself, silu(x) * x2, or x * (1 + norm_w) / rms(x)
+struct MultiInput {
+    const float* x2 = nullptr;      // same layout as x
+    const float* norm_w = nullptr;  // cols floats
+    bool inv_form = false;          // silu as x * (1 / (1 + exp(-x))) instead of x / (1 + exp(-x))
+};
+int launch_gemv_oil4_multi(const oilhip_weights& w, const float* d_x, const int* d_tok, float* d_y, int M, uint32_t ldx, uint32_t ldy,
+                           uint32_t xrows, hipStream_t s, const MultiInput& in = {}, const oilhip_weights* w2 = nullptr, float* d_y2 = nullptr,
+                           uint32_t ldy2 = 0, uint8_t* d_pack = nullptr);
+// several batches of one tensor shape in one launch, at most 32 rows each
+size_t gemv_oil4_multi_batches_bytes(int nb, uint64_t cols);
+int launch_gemv_oil4_multi_batches(int nb, const oilhip_weights* const* wa, float* const* ya, const oilhip_weights* const* wb, float* const* yb,
+                                   const int* M, const int* row0, const int* list, int nlist, const float* d_x, const float* d_x2,
+                                   uint32_t ldx, uint32_t xrows, uint32_t ldy, void* d_ws, size_t ws_bytes, hipStream_t s);
+// widest row that kernel takes and the bytes of packed activations one pass of it needs (d_pack, or stream scratch): per
+// block 32 floats (powers of two) and three digits of 256 activations for 32 tokens
 constexpr uint32_t kGemvPackMaxCols = 32768;
-constexpr size_t kGemvPackExpBytes = (size_t)(kGemvPackMaxCols >> 8) * 2u * 16u * 4u;    // one scale exponent per (token tile, block, column)
-constexpr size_t kGemvPackBytes = (size_t)(kGemvPackMaxCols >> 8) * 128u * 128u * 2u + kGemvPackExpBytes;   // two token tiles, then the exponents
+constexpr size_t kGemvPackBytes = (size_t)(kGemvPackMaxCols >> 8) * (128u + 24576u);
 // rows that mix formats, stored tile by tile and format by format
 int launch_gemv_seg(const oilhip_weights& w, const float* d_x, float* d_y, int M, hipStream_t s);
 // every format, a lane per run of 32 weights

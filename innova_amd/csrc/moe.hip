@@ -17,16 +17,6 @@ __global__ void __launch_bounds__(256) fill_zero_kernel(float* __restrict__ p, s
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) p[i] = 0.0f;
 }
 
-// three ranges in one launch (what a grouped step needs cleared before its first kernel)
-__global__ void __launch_bounds__(256) fill_zero3_kernel(float* __restrict__ a, size_t na, float* __restrict__ b, size_t nb,
-                                                         float* __restrict__ c, size_t nc) {
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < na + nb + nc; i += (size_t)gridDim.x * 256) {
-        if (i < na) a[i] = 0.0f;
-        else if (i < na + nb) b[i - na] = 0.0f;
-        else c[i - na - nb] = 0.0f;
-    }
-}
-
 // h = silu(g) * u, silu(v) = v / (1 + exp(-v))  (src/math.cpp:117-126)
 __global__ void __launch_bounds__(256) swiglu_kernel(float* __restrict__ g, const float* __restrict__ u, size_t n) {
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
@@ -92,18 +82,14 @@ constexpr int kMaxPairs = 448;
 struct CombineLists {
     int K;
     int16_t pair[kMaxPairs];    // pair[t * K + k]: row of o behind the k-th contribution of token t, or -1
-    uint8_t nparts[kMaxPairs];  // nparts[row of o]: K parts of that row left in `parts` by the down projection (0: the row is in o)
     float wgt[kMaxPairs];       // its weight (<= 0: dropped)
 };
 
 static_assert(sizeof(CombineLists) <= 3584, "the lists travel in the kernel arguments (4 KB with the other arguments)");
 
 // zacc == nullptr: the caller does not want the z-loss, and the workgroups skip their atomic on its one address.
-// Rows whose down projection was cut into three or more K parts arrive as those parts (parts[p * pstride + row * D + d])
-// and are summed here in ascending part order: the sum does not depend on the order in which workgroups ran.
-__global__ void __launch_bounds__(256) combine_grouped_kernel(const float* __restrict__ o, const float* __restrict__ parts, uint32_t pstride,
-                                                              uint32_t D, float* __restrict__ out, double* __restrict__ zacc,
-                                                              const CombineLists L) {
+__global__ void __launch_bounds__(256) combine_grouped_kernel(const float* __restrict__ o, uint32_t D, float* __restrict__ out,
+                                                              double* __restrict__ zacc, const CombineLists L) {
     __shared__ double part[4];
     const uint32_t d = blockIdx.x * 256 + threadIdx.x, t = blockIdx.y;
     double z = 0.0;
@@ -113,11 +99,7 @@ __global__ void __launch_bounds__(256) combine_grouped_kernel(const float* __res
             const int i = L.pair[t * L.K + k];
             const float w = L.wgt[t * L.K + k];
             if (i < 0 || !(w > 0.0f)) continue;
-            float y = 0.0f;
-            const uint32_t np = L.nparts[i];
-            if (np == 0u) y = o[(size_t)i * D + d];
-            for (uint32_t p = 0; p < np; ++p) y += parts[(size_t)p * pstride + (size_t)i * D + d];
-            const float v = w * y;
+            const float v = w * o[(size_t)i * D + d];
             sum += v;
             z += (double)v * (double)v;
         }
@@ -133,23 +115,14 @@ __global__ void __launch_bounds__(256) combine_grouped_kernel(const float* __res
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 struct Workspace {
-    int* tok; float* wgt; float* g; float* u; float* o; float* xg; float* parts; double* z; uint8_t* batch;
+    int* tok; float* wgt; float* g; float* u; float* o; float* xg; double* z; uint8_t* batch;
     size_t bytes, batch_bytes;
 };
 
 constexpr int kChunk = 16;      // expert batches per grouped launch (gate and up together are 32 tensors)
 
-// scratch of one grouped launch: the larger of the gate/up side (rows F, cols D) and the down side (rows D, cols F)
-size_t batch_scratch_bytes(int64_t D, int64_t F) {
-    return std::max(gemv_oil4_multi_batches_bytes(kChunk, (uint64_t)F, (uint64_t)D, true), gemv_oil4_multi_batches_bytes(kChunk, (uint64_t)D, (uint64_t)F, false));
-}
-
-// the most K parts a row of F weights is cut into, over the pass sizes; 0 when no pass size cuts it in three or more
-uint32_t down_parts_max(int64_t F) {
-    uint32_t m = 0;
-    for (int kind = 0; kind < 3; ++kind) m = std::max(m, gemv_oil4_multi_parts(kind, (uint64_t)F));
-    return m > 2u ? m : 0u;
-}
+// scratch of one grouped launch: the wider of the gate/up side (rows of D weights) and the down side (rows of F)
+size_t batch_scratch_bytes(int64_t D, int64_t F) { return gemv_oil4_multi_batches_bytes(kChunk, (uint64_t)std::max(D, F)); }
 
 Workspace carve(void* base, int64_t pairs, int64_t D, int64_t F) {
     Workspace w{};
@@ -165,8 +138,6 @@ Workspace carve(void* base, int64_t pairs, int64_t D, int64_t F) {
     w.xg = (float*)take((size_t)pairs * D * 4);
     w.batch_bytes = (D % 256 == 0 && F % 256 == 0 && D <= 32768 && F <= 32768) ? batch_scratch_bytes(D, F) : 0;
     w.batch = take(w.batch_bytes);
-    // K parts of the down projections' outputs (rows of F weights cut into three or more parts), summed by the combine
-    w.parts = (float*)take(w.batch_bytes ? (size_t)down_parts_max(F) * pairs * D * 4 : 0);
     w.bytes = off;
     return w;
 }
@@ -275,33 +246,17 @@ int oilhip_moe_forward(const oilhip_weights* const* gate, const oilhip_weights* 
     for (int e = 0; e < E && grouped; ++e) grouped = plain_oil4(*gate[e]) && plain_oil4(*up[e]) && plain_oil4(*down[e]);
     if (grouped) {
         const int64_t pairs = (int64_t)tok.size();
-        // the z-loss accumulator and the slab counters at the start of the batch workspace start at zero (every launch
-        // leaves the counters at zero again); outputs that row parts add into are cleared by the launch that splits
-        // the activations
-        // (the launch is skipped when nothing needs it: no z-loss asked for, and no launch of the step counts arrivals --
-        // the gate/up rows are cut in at most two parts and the down projections leave their parts to the combine)
-        const bool parts_mode = gemv_oil4_multi_ordered() && down_parts_max(F) > 0u;
-        const bool counters = gemv_oil4_multi_ordered() && (down_parts_max(D) > 0u || (down_parts_max(F) > 0u && !parts_mode));
-        if (z_loss || counters) {
-            hipLaunchKernelGGL(fill_zero3_kernel, dim3(64), dim3(256), 0, s, ws.g, (size_t)0, (float*)ws.z, (size_t)2, (float*)ws.batch,
-                               kGemvBatchCounterBytes / 4);
+        if (z_loss) {
+            hipLaunchKernelGGL(fill_zero_kernel, dim3(1), dim3(256), 0, s, (float*)ws.z, (size_t)2);
             OILHIP_HIP(hipGetLastError());
         }
-        // down projections cut into three or more K parts leave the parts to the combine (parts_mode: ordered sums; with
-        // the atomic sums switched on they add into their outputs instead)
-        struct Batch { int e, pair0, m, kind; };
+        struct Batch { int e, pair0, m; };
         std::vector<Batch> batches;
-        for (int pass = 2; pass >= 0; --pass)                     // the longest passes first: they end last
-            for (int e = 0; e < E; ++e) {
-                int n = begin[(size_t)e + 1] - begin[(size_t)e], pos = begin[(size_t)e];
-                while (n > 0) {
-                    // more than 16 tokens: a pass of 32 (its table reads serve two token tiles: 1.36 times the cost of a
-                    // pass of 16); then what is left as a pass of 16 or of 8
-                    const int take = n > 32 ? 32 : n, kind = take <= 8 ? 0 : take <= 16 ? 1 : 2;
-                    if (kind == pass) batches.push_back(Batch{e, pos, take, kind});
-                    pos += take; n -= take;
-                }
-            }
+        for (int e = 0; e < E; ++e)                               // passes of 32 tokens, then what is left
+            for (int n = begin[(size_t)e + 1] - begin[(size_t)e], pos = begin[(size_t)e]; n > 0; n -= 32, pos += 32)
+                batches.push_back(Batch{e, pos, std::min(n, 32)});
+        // the longest passes first: they end last
+        std::stable_sort(batches.begin(), batches.end(), [](const Batch& x, const Batch& y) { return x.m > y.m; });
         // all pass sizes of a chunk of batches share one launch per side: one launch that splits the gathered
         // activations, one over the gate and up projections, one that forms silu(gate) * up while splitting it, one
         // over the down projections
@@ -309,29 +264,24 @@ int oilhip_moe_forward(const oilhip_weights* const* gate, const oilhip_weights* 
             const int nb = (int)std::min<size_t>(kChunk, batches.size() - c0);
             const oilhip_weights *wg[kChunk], *wu[kChunk], *wd[kChunk];
             float *yg[kChunk], *yu[kChunk], *yo[kChunk];
-            int Mb[kChunk], r0[kChunk], kd[kChunk];
+            int Mb[kChunk], r0[kChunk];
             for (int b = 0; b < nb; ++b) {
                 const Batch& B = batches[c0 + b];
                 wg[b] = gate[B.e]; wu[b] = up[B.e]; wd[b] = down[B.e];
                 yg[b] = ws.g + (size_t)B.pair0 * F; yu[b] = ws.u + (size_t)B.pair0 * F; yo[b] = ws.o + (size_t)B.pair0 * D;
-                Mb[b] = B.m; r0[b] = B.pair0; kd[b] = B.kind;
+                Mb[b] = B.m; r0[b] = B.pair0;
             }
-            int rc = launch_gemv_oil4_multi_batches(nb, kd, wg, yg, wu, yu, Mb, r0, tok.data(), (int)tok.size(), d_x, nullptr,
-                                                    (uint32_t)D, (uint32_t)T, (uint32_t)F, ws.batch, ws.batch_bytes, s, true);
+            int rc = launch_gemv_oil4_multi_batches(nb, wg, yg, wu, yu, Mb, r0, tok.data(), (int)tok.size(), d_x, nullptr,
+                                                    (uint32_t)D, (uint32_t)T, (uint32_t)F, ws.batch, ws.batch_bytes, s);
             if (rc == 0)
-                rc = launch_gemv_oil4_multi_batches(nb, kd, wd, yo, nullptr, nullptr, Mb, r0, nullptr, 0, ws.g, ws.u,
-                                                    (uint32_t)F, (uint32_t)pairs, (uint32_t)D, ws.batch, ws.batch_bytes, s, true,
-                                                    parts_mode ? ws.parts : nullptr, (uint32_t)pairs);
+                rc = launch_gemv_oil4_multi_batches(nb, wd, yo, nullptr, nullptr, Mb, r0, nullptr, 0, ws.g, ws.u, (uint32_t)F,
+                                                    (uint32_t)pairs, (uint32_t)D, ws.batch, ws.batch_bytes, s);
             if (rc < 0) return rc;
             if (rc == 1) return fail(OILHIP_E_ARG, "moe_forward: the grouped launch refused a shape it was planned for");
         }
         CombineLists L{};
         L.K = (int)K;
         for (int64_t i = 0; i < T * K; ++i) { L.pair[i] = -1; L.wgt[i] = 0.0f; }
-        for (const Batch& B : batches) {
-            const uint32_t np = parts_mode ? gemv_oil4_multi_parts(B.kind, (uint64_t)F) : 0u;
-            for (int m = 0; m < B.m; ++m) L.nparts[B.pair0 + m] = (uint8_t)(np > 2u ? np : 0u);
-        }
         std::vector<int> filled((size_t)T, 0);
         for (int e = 0; e < E; ++e)                      // ascending expert, list order: the order of the reference's additions
             for (int i = begin[(size_t)e]; i < begin[(size_t)e + 1]; ++i) {
@@ -340,8 +290,8 @@ int oilhip_moe_forward(const oilhip_weights* const* gate, const oilhip_weights* 
                 L.wgt[t * K + filled[(size_t)t]] = wgt[(size_t)i];
                 filled[(size_t)t]++;
             }
-        hipLaunchKernelGGL(combine_grouped_kernel, dim3((uint32_t)((D + 255) / 256), (uint32_t)T), dim3(256), 0, s, ws.o, ws.parts,
-                           (uint32_t)(pairs * D), (uint32_t)D, d_out, z_loss ? ws.z : (double*)nullptr, L);
+        hipLaunchKernelGGL(combine_grouped_kernel, dim3((uint32_t)((D + 255) / 256), (uint32_t)T), dim3(256), 0, s, ws.o, (uint32_t)D, d_out,
+                           z_loss ? ws.z : (double*)nullptr, L);
         OILHIP_HIP(hipGetLastError());
         if (z_loss) {
             double z = 0.0;
@@ -365,7 +315,7 @@ int oilhip_moe_forward(const oilhip_weights* const* gate, const oilhip_weights* 
         // gate and up read the same gathered activations: uniform OIL4 experts split them once per pass for both
         int both = 1;
         if (plain_oil4(*gate[e]))
-            both = launch_gemv_oil4_multi(*gate[e], d_x, ws.tok + b, ws.g, nt, (uint32_t)D, (uint32_t)F, (uint32_t)T, s, up[e], ws.u,
+            both = launch_gemv_oil4_multi(*gate[e], d_x, ws.tok + b, ws.g, nt, (uint32_t)D, (uint32_t)F, (uint32_t)T, s, {}, up[e], ws.u,
                                           (uint32_t)F);
         if (both < 0) return both;
         if (both == 1) {
@@ -375,8 +325,7 @@ int oilhip_moe_forward(const oilhip_weights* const* gate, const oilhip_weights* 
         // silu(gate) * up: formed while the down projection's activations are split (uniform OIL4), or by a kernel of its own
         int fused = 1;
         if (plain_oil4(*down[e]))
-            fused = launch_gemv_oil4_multi(*down[e], ws.g, nullptr, ws.o, nt, (uint32_t)F, (uint32_t)D, (uint32_t)nt, s, nullptr, nullptr, 0,
-                                           ws.u);
+            fused = launch_gemv_oil4_multi(*down[e], ws.g, nullptr, ws.o, nt, (uint32_t)F, (uint32_t)D, (uint32_t)nt, s, MultiInput{ws.u});
         if (fused < 0) return fused;
         if (fused == 1) {
             const size_t n = (size_t)nt * (size_t)F;

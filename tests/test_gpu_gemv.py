@@ -257,6 +257,32 @@ def test_oil4_multi_token_activation_ranges(rows, cols, M):
         assert rel_l2(got[m], want[m]) <= TOL, m
 
 
+# The multi-token kernel's launch shapes: row groups per workgroup around the lengths of its runs (1, 2, 3, 4, 5, 7 groups of 16
+# rows on 256 CUs), rows that fit one part of the wavefronts' registers and rows of several parts whose sums wait in LDS, past
+# the number of groups that wait together (24 for passes of 32 tokens, 48 for 16), pass sizes at their edges.  The rows repeat
+# with a period that meets every position in a group, so the oracle computes one period.
+@pytest.mark.parametrize("bpr,rows,tokens", [
+    (1, 17, (3, 4, 5, 8, 9, 16, 17, 32, 33)), (5, 4096, (4, 8, 16, 32)), (5, 4097, (3, 5, 9, 17)), (8, 8191, (4, 8, 16, 32)),
+    (5, 4096 * 3 + 1, (4, 8, 16, 32)), (7, 4096 * 5, (3, 7, 15, 31)), (5, 4096 * 7 - 15, (4, 8, 16, 32)),
+    (9, 4096 * 25 + 1, (24,)), (17, 4096 * 49 + 5, (12,)), (33, 500, (4, 8, 16, 32)), (57, 130, (4, 8, 16, 32)), (128, 33, (4, 32))])
+def test_oil4_multi_token_launch_shapes(bpr, rows, tokens):
+    cols, period = 256 * bpr, min(rows, 131)
+    payload, blocks = ia.block_codec.quantize_tensor(gaussian_weights(period * cols, rows), ia.Format.OIL4)
+    size, copies = period * bpr * 128, -(-rows // period)
+    big = np.tile(blocks, copies)[:rows * bpr]
+    shift = (np.arange(rows * bpr) // (period * bpr) * size).astype(np.uint64)
+    big["cb_off"] += shift
+    big["idx_off"] += shift
+    with ia.DeviceWeights.from_blocks(np.tile(payload[:size], copies)[:rows * bpr * 128], big, rows, cols) as dw:
+        for M in tokens:
+            X = np.random.default_rng(M).standard_normal((M, cols)).astype(np.float32)
+            want = O.block_gemm(payload, to_orc_blocks(blocks), period, cols, X, wide=True)
+            got = dw.gemv(torch.from_numpy(X).cuda()).cpu().numpy()
+            for r in range(0, rows, period):
+                n = min(period, rows - r)
+                assert rel_l2(got[:, r:r + n], want[:, :n]) <= TOL, (M, r)
+
+
 def test_two_streams_run_multi_token_gemvs_concurrently():
     """Calls on different streams keep separate activation scratch: M = 16 GEMVs of two tensors issued back and forth
     on two streams, all in flight together, the first and last round checked against the oracle, one in between
