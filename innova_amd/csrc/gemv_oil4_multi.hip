@@ -111,10 +111,13 @@ __device__ __forceinline__ void load_activations(const Activations& a, uint32_t 
         for (int e = 0; e < 4; ++e) v[e] = (a.inv_form ? v[e] * (1.0f / (1.0f + expf(-v[e]))) : v[e] / (1.0f + expf(-v[e]))) * u[e];
     } else if (a.norm_w) {
         float s = 0.0f;
-        for (uint32_t c = 4u * lane; c < 256u * bpr; c += 256u) {
-            float f[4];
-            load(row + c, f);
-            s += (f[0] * f[0] + f[1] * f[1]) + (f[2] * f[2] + f[3] * f[3]);
+        for (uint32_t b = 0; b < bpr; b += 8u) {                           // eight loads in flight; past the end: the last block, counted as 0
+            float f[8][4];
+#pragma unroll
+            for (uint32_t i = 0; i < 8u; ++i) load(row + 256u * (b + i < bpr ? b + i : bpr - 1u) + 4u * lane, f[i]);
+#pragma unroll
+            for (uint32_t i = 0; i < 8u; ++i)
+                s += b + i < bpr ? (f[i][0] * f[i][0] + f[i][1] * f[i][1]) + (f[i][2] * f[i][2] + f[i][3] * f[i][3]) : 0.0f;
         }
         for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
         rms = 1.0f / sqrtf(s / (float)(256u * bpr) + 1e-6f);

@@ -112,6 +112,28 @@ def test_mlp_step_with_norm(fmt):
         d.close()
 
 
+# several rows of an OIL4 tensor: norm and SwiGLU are formed while the activations are packed (the norm up to 8192 columns), eight
+# blocks of the row at a time; passes of 32 rows
+@pytest.mark.parametrize("M,D,F", [(2, 256, 512), (5, 2304, 768), (16, 1792, 2816), (33, 2048, 256), (4, 8192, 512), (3, 8448, 256)])
+def test_norm_and_swiglu_of_several_rows(M, D, F):
+    rng = np.random.default_rng(M + D)
+    mats = [(r, c) + tuple(ia.block_codec.quantize_tensor(gaussian_weights(r * c, seed=r) * np.float32(50.0 / np.sqrt(c)), ia.Format.OIL4))
+            for r, c in ((2 * F, D), (D, F))]
+    x = (rng.standard_normal((M, D)) * np.logspace(-3, 3, M)[:, None]).astype(np.float32)
+    nw = (rng.standard_normal(D) * 0.2).astype(np.float32)
+    gu, down = (ia.DeviceWeights.from_blocks(m[2], m[3], m[0], m[1]) for m in mats)
+    xd, nd = torch.from_numpy(x).cuda(), torch.from_numpy(nw).cuda()
+    g = O.block_gemm(mats[0][2], to_orc_blocks(mats[0][3]), 2 * F, D, O.rmsnorm(x, nw), wide=True)
+    assert rel_l2(layers.gemv_rmsnorm(gu, xd, nd).cpu().numpy(), g) <= TOL
+    h = O.swiglu(g[:, :F].astype(np.float32), g[:, F:].astype(np.float32))
+    want = O.block_gemm(mats[1][2], to_orc_blocks(mats[1][3]), D, F, h, wide=True)
+    got = layers.mlp_step(gu, down, xd, norm_w=nd).cpu().numpy()
+    for m in range(M):
+        assert rel_l2(got[m], want[m]) <= TOL, m
+    gu.close()
+    down.close()
+
+
 def test_embed_rows():
     vocab, cols = 40, 1024
     w = gaussian_weights(vocab * cols, 5)
