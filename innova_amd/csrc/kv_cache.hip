@@ -2,8 +2,8 @@
 // src/kv_cache_oil4.cpp) held in HBM: 4-bit codes, two per byte (low nibble first), and 16 FP16 centroids per block of
 // 32 / 64 / 128 consecutive values of a layer's [token][heads * dim] stream.
 //
-//   append    : every chunk (a token's values cut at block boundaries, :207-291) is quantized by one wavefront with
-//               the reference's 16-level Lloyd-Max (:75-153) step for step -- same initial centroids, same 20
+//   append    : every chunk (a token's values cut at block boundaries, :207-291) is quantized by 16 lanes, one per
+//               cluster, with the reference's 16-level Lloyd-Max (:75-153) step for step -- same initial centroids, same 20
 //               iterations over the sorted values, same sequential sums -- so codes and centroids are identical.
 //   get_range : codes -> centroids -> FP32 [len][heads * dim] through the cache's own half decode
 //               (CodebookOIL4::half_to_float, src/codebook.cpp:36-64, which is not IEEE for subnormals).
@@ -15,6 +15,7 @@
 // byte to the later chunk.
 #include <algorithm>
 #include <new>
+#include <type_traits>
 #include <vector>
 
 #include "common.h"
@@ -72,13 +73,14 @@ __device__ __forceinline__ float kv_half_to_float(uint32_t h) {
     return __uint_as_float(f);
 }
 
-__device__ __forceinline__ uint32_t kv_nearest(const float (&cen)[16], float x) {
+// the first of the nearest centroids (a loop over LDS: this path is for rare chunks and should cost the common one no registers)
+__device__ __forceinline__ uint32_t kv_nearest(const float* cen, float x) {
     float best = fabsf(__fsub_rn(x, cen[0]));
     uint32_t bi = 0;
-#pragma unroll
-    for (int c = 1; c < 16; ++c) {
+#pragma unroll 1
+    for (uint32_t c = 1; c < 16; ++c) {
         const float d = fabsf(__fsub_rn(x, cen[c]));
-        if (d < best) { best = d; bi = (uint32_t)c; }
+        if (d < best) { best = d; bi = c; }
     }
     return bi;
 }
@@ -106,36 +108,15 @@ __device__ __forceinline__ void kv_min_max(float x0, float x1, uint32_t n, uint3
     }
 }
 
-// lloyd_max_16 (src/kv_cache_oil4.cpp:75-153) for n <= 128 values by one wavefront.  Leaves the n codes in L.code and
+// lloyd_max_16 (src/kv_cache_oil4.cpp:75-153) for n <= 128 values by one wavefront, for any values.  Leaves the n codes in L.code and
 // the 16 centroids (FP32) in L.cen.
-__device__ void kv_quantize_chunk(const float* __restrict__ src, uint32_t n, uint32_t lane, KvLds& L) {
+__device__ __forceinline__ void kv_quantize_chunk(const float* __restrict__ src, uint32_t n, uint32_t lane, KvLds& L) {
     const float x0 = lane < n ? src[lane] : 0.f;
     const float x1 = lane + 64 < n ? src[lane + 64] : 0.f;
-    // Ascending sort of the n values, padded with +inf: a bitonic network, in registers with one value per lane for
-    // chunks of up to 64 values (both lanes of a pair evaluate the same comparison, so equal values are never
-    // duplicated), over 128 LDS slots otherwise.  The sorted ends are the minimum and the maximum.
-    float s0, s1, lo, hi;
-    if (n <= 64) {
-        s0 = lane < n ? x0 : __builtin_inff();
-        s1 = __builtin_inff();
-#pragma unroll
-        for (uint32_t k = 2; k <= 64; k <<= 1) {
-#pragma unroll
-            for (uint32_t j = k >> 1; j > 0; j >>= 1) {
-                const float other = __shfl_xor(s0, (int)j, 64);
-                const bool keep_small = ((lane & j) == 0) == ((lane & k) == 0);
-                const bool take = keep_small ? other < s0 : other > s0;
-                s0 = take ? other : s0;
-            }
-        }
-        lo = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s0), 0));
-        hi = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s0), (int)n - 1));
-    } else {
-        kv_min_max(x0, x1, n, lane, lo, hi);
-    }
+    float lo, hi;
+    kv_min_max(x0, x1, n, lane, lo, hi);
     const float range = __fsub_rn(hi, lo);
     if (range < 1e-10f) {
-        if (n <= 64) kv_min_max(x0, x1, n, lane, lo, hi);       // which of several equal zeros comes first
         if (lane < n) L.code[lane] = 8;
         if (lane + 64 < n) L.code[lane + 64] = 8;
         if (lane < 16) L.cen[lane] = lo;
@@ -143,148 +124,359 @@ __device__ void kv_quantize_chunk(const float* __restrict__ src, uint32_t n, uin
         return;
     }
     if (lane < 16) L.cen[lane] = __fadd_rn(lo, __fdiv_rn(__fmul_rn(range, (float)lane + 0.5f), 16.0f));
-    if (n <= 64) {
-        L.srt[lane] = s0;
-        __syncthreads();
-    } else {
-        L.srt[lane] = x0;
-        L.srt[lane + 64] = lane + 64 < n ? x1 : __builtin_inff();
-        __syncthreads();
-        for (uint32_t k = 2; k <= 128; k <<= 1) {
-            for (uint32_t j = k >> 1; j > 0; j >>= 1) {
-                const uint32_t i = ((lane & ~(j - 1)) << 1) | (lane & (j - 1));
-                const uint32_t p = i | j;
-                const bool up = (i & k) == 0;
-                const float a = L.srt[i], b = L.srt[p];
-                if ((a > b) == up) { L.srt[i] = b; L.srt[p] = a; }
-                __syncthreads();
-            }
+    // ascending bitonic sort over 128 slots, +inf behind the values
+    L.srt[lane] = lane < n ? x0 : __builtin_inff();
+    L.srt[lane + 64] = lane + 64 < n ? x1 : __builtin_inff();
+    __syncthreads();
+    for (uint32_t k = 2; k <= 128; k <<= 1) {
+        for (uint32_t j = k >> 1; j > 0; j >>= 1) {
+            const uint32_t i = ((lane & ~(j - 1)) << 1) | (lane & (j - 1));
+            const uint32_t p = i | j;
+            const bool up = (i & k) == 0;
+            const float a = L.srt[i], b = L.srt[p];
+            if ((a > b) == up) { L.srt[i] = b; L.srt[p] = a; }
+            __syncthreads();
         }
-        s0 = L.srt[lane];
-        s1 = L.srt[lane + 64];
     }
-    float cen[16];
-#pragma unroll
-    for (int c = 0; c < 16; ++c) cen[c] = L.cen[c];
     for (int it = 0; it < 20; ++it) {
-        const uint32_t b0 = lane < n ? kv_nearest(cen, s0) : 16u;
-        bool moved = false;
-        // the cluster of the value to the left (wave_shr:1; lane 0 reads 0)
-        const uint32_t prev = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)b0, 0x138, 0xF, 0xF, true);
-        if (n <= 64 && __ballot(lane > 0 && b0 < prev) == 0) {
-            // Cluster numbers do not fall along the sorted values (the usual case), so every cluster is one run of
-            // lanes.  Each lane folds its run from the left, one neighbour step at a time: after step t the lanes at
-            // depth <= t of their run hold 0 + x_first + ... + x_self in exactly the reference's order.  The last lane
-            // of a run owns the cluster's sum and count.
-            const uint64_t heads = __ballot(lane == 0 || b0 != prev);
-            const uint32_t first = 63u - (uint32_t)__builtin_clzll(heads & (~0ull >> (63u - lane)));
-            const uint32_t depth = lane - first;
-            float fold = __fadd_rn(0.f, s0);
-            for (uint32_t t = 1; __ballot(depth >= t) != 0; ++t) {
-                const float left = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(fold), 0x138, 0xF, 0xF, true));
-                const float next = __fadd_rn(left, s0);
-                fold = depth >= t ? next : fold;
-            }
-            const bool tail = lane == 63 || ((heads >> ((lane + 1) & 63u)) & 1ull) != 0;
-            if (tail && b0 < 16) {
-                const float nv = __fdiv_rn(fold, (float)(depth + 1));
-                moved = __float_as_uint(nv) != __float_as_uint(L.cen[b0]);
-                L.cen[b0] = nv;
-            }
-        } else {
-            // lane c < 16 collects the members of cluster c as bit masks over the sorted order and adds them up in that
-            // order, as the reference's loop over the sorted values does (four LDS reads in flight per round)
-            const uint32_t b1 = lane + 64 < n ? kv_nearest(cen, s1) : 16u;
-            uint64_t m0 = 0, m1 = 0;
-#pragma unroll
-            for (uint32_t c = 0; c < 16; ++c) {
-                const uint64_t w0 = __ballot(b0 == c);
-                const uint64_t w1 = n > 64 ? __ballot(b1 == c) : 0ull;
-                if (lane == c) { m0 = w0; m1 = w1; }
-            }
-            float sum = 0.f;
-            const int cnt = __popcll(m0) + __popcll(m1);
-            for (int half = 0; half < 2; ++half) {
-                uint64_t m = half ? m1 : m0;
-                const float* base = L.srt + 64 * half;
-                while (m) {
-                    uint32_t i[4];
-                    bool h[4];
-                    float val[4];
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-                        h[u] = m != 0;
-                        i[u] = h[u] ? (uint32_t)__builtin_ctzll(m) : 0u;
-                        m &= m - 1;
-                    }
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) val[u] = base[i[u]];
-#pragma unroll
-                    for (int u = 0; u < 4; ++u)
-                        if (h[u]) sum = __fadd_rn(sum, val[u]);
-                }
-            }
-            if (lane < 16 && cnt > 0) {                                              // an empty cluster keeps its centroid
-                const float nv = __fdiv_rn(sum, (float)cnt);
-                moved = __float_as_uint(nv) != __float_as_uint(L.cen[lane]);
-                L.cen[lane] = nv;
-            }
+        // lane c < 16 collects the members of cluster c as bit masks over the sorted order and adds them up in that
+        // order, as the reference's loop over the sorted values does
+        const uint32_t b0 = lane < n ? kv_nearest(L.cen, L.srt[lane]) : 16u;
+        const uint32_t b1 = lane + 64 < n ? kv_nearest(L.cen, L.srt[lane + 64]) : 16u;
+        uint64_t m0 = 0, m1 = 0;
+#pragma unroll 1
+        for (uint32_t c = 0; c < 16; ++c) {
+            const uint64_t w0 = __ballot(b0 == c), w1 = __ballot(b1 == c);
+            if (lane == c) { m0 = w0; m1 = w1; }
         }
-        const bool any_moved = __ballot(moved) != 0;
+        float sum = 0.f;
+        const int cnt = __popcll(m0) + __popcll(m1);
+        for (; m0; m0 &= m0 - 1) sum = __fadd_rn(sum, L.srt[__builtin_ctzll(m0)]);
+        for (; m1; m1 &= m1 - 1) sum = __fadd_rn(sum, L.srt[64 + __builtin_ctzll(m1)]);
+        bool moved = false;
+        if (lane < 16 && cnt > 0) {                                                  // an empty cluster keeps its centroid
+            const float nv = __fdiv_rn(sum, (float)cnt);
+            moved = __float_as_uint(nv) != __float_as_uint(L.cen[lane]);
+            L.cen[lane] = nv;
+        }
         __syncthreads();
-        if (!any_moved) break;           // a fixed point: the remaining iterations would reproduce these centroids bit for bit
-#pragma unroll
-        for (int c = 0; c < 16; ++c) cen[c] = L.cen[c];
-        __syncthreads();
+        if (__ballot(moved) == 0) break;     // a fixed point: the remaining iterations would reproduce these centroids bit for bit
     }
-    if (lane < n) L.code[lane] = (uint8_t)kv_nearest(cen, x0);
-    if (lane + 64 < n) L.code[lane + 64] = (uint8_t)kv_nearest(cen, x1);
+    if (lane < n) L.code[lane] = (uint8_t)kv_nearest(L.cen, x0);
+    if (lane + 64 < n) L.code[lane + 64] = (uint8_t)kv_nearest(L.cen, x1);
     __syncthreads();
 }
 
-// One wavefront per (token, chunk of the token, K or V).  pos = tokens the layer held before this call, ntok = tokens
-// of this call that fit.  K centroids are stored by the chunk that opens a block, or -- while the layer is empty, and
+// ---- the same quantizer, 16 lanes per chunk ----------------------------------------------------------------------------
+// A wavefront takes up to four chunks of at most 16 V values, one per row of 16 lanes; lane c of a row holds values c V ..
+// c V + V - 1 and is cluster c.  The values are sorted across the row in registers and kept in LDS.  Sorted values
+// that belong to one cluster are neighbours, so an iteration is: every cluster moves its first member's position (from where it
+// was) until |x - cen[c]| < |x - cen[c - 1]| holds at it and not before it, and adds its members up in sorted order, as the
+// reference's loop does.  A cluster whose range stays has the same sum as before, and when all ranges stay the centroids are a fixed
+// point.
+// That the comparison of neighbours is monotone over the sorted values and equals the reference's scan over all 16 needs
+// centroids that rise by more than the rounding of the distances (at most range * 2^-22); this is checked in every iteration, and
+// chunks that fail it, hold infinities or NaN, or are constant, go through kv_quantize_chunk.
+// What bounds it: vector issue of the iterations (about 60 instructions for four chunks each, of which a long append takes about a
+// dozen); the chain of dependent instructions and LDS round trips when a decode step appends one token, where each wavefront
+// takes one chunk.  One wavefront per chunk before (every value compared with all 16 centroids in each iteration, sums passed
+// from lane to lane) -> now, 4096 values per token, K and V: 2048 tokens 490 -> 93 us with blocks of 64, 1024 tokens of 2048
+// values with blocks of 32 300 -> 37 us and of 128 268 -> 40 us (clearing included), one token 13 -> 6 us.
+// Windows of four positions per move and sums of eight values per round need fewer steps, and were slower by 12 %.
+constexpr int kSrtPad = 8;                 // floats before a row's values
+
+template <int CTRL>
+__device__ __forceinline__ int row_dpp(int v) { return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, true); }
+
+// the key order of floats (finite: no NaN reaches this)
+__device__ __forceinline__ int kv_key(float f) { const int i = __float_as_int(f); return i ^ ((i >> 31) & 0x7FFFFFFF); }
+__device__ __forceinline__ float kv_unkey(int i) { return __int_as_float(i ^ ((i >> 31) & 0x7FFFFFFF)); }
+
+__device__ __forceinline__ int med3(int a, int b, int c) {                 // v_med3_i32: the smaller of a and b for c = INT_MIN, the larger for INT_MAX
+    return max(min(a, b), min(max(a, b), c));
+}
+
+template <int V>
+__device__ __forceinline__ void in_lane_merge(int (&k)[V]) {
+#pragma unroll
+    for (int j = V / 2; j > 0; j >>= 1)
+#pragma unroll
+        for (int e = 0; e < V; ++e)
+            if (!(e & j)) { const int a = k[e], b = k[e | j]; k[e] = min(a, b); k[e | j] = max(a, b); }
+}
+
+// Ascending bitonic sort of 16 V keys, element c V + e in lane c.  A merge begins with the mirrored partner, so that all
+// comparisons point the same way; `bound[i]` is INT_MIN in lanes whose bit i is clear (they keep the smaller key), else INT_MAX.
+template <int V>
+__device__ __forceinline__ void row_sort(int (&k)[V], uint32_t c) {
+    int bound[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) bound[i] = (c >> i) & 1u ? 0x7FFFFFFF : (int)0x80000000;
+    // inside a lane
+#pragma unroll
+    for (int m = 2; m <= V; m <<= 1) {
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
+            const int o = e ^ (m - 1);
+            if (e < o) { const int a = k[e], b = k[o]; k[e] = min(a, b); k[o] = max(a, b); }
+        }
+#pragma unroll
+        for (int j = m / 4; j > 0; j >>= 1)
+#pragma unroll
+            for (int e = 0; e < V; ++e)
+                if (!(e & j)) { const int a = k[e], b = k[e | j]; k[e] = min(a, b); k[e | j] = max(a, b); }
+    }
+    auto flip = [&](auto ctrl, int bit) {
+        int o[V];
+#pragma unroll
+        for (int e = 0; e < V; ++e) o[e] = row_dpp<decltype(ctrl)::value>(k[V - 1 - e]);
+#pragma unroll
+        for (int e = 0; e < V; ++e) k[e] = med3(k[e], o[e], bound[bit]);
+    };
+    auto step = [&](auto ctrl, int bit) {
+#pragma unroll
+        for (int e = 0; e < V; ++e) k[e] = med3(k[e], row_dpp<decltype(ctrl)::value>(k[e]), bound[bit]);
+    };
+    using std::integral_constant;
+    flip(integral_constant<int, 0xB1>{}, 0);                               // lane ^ 1
+    in_lane_merge<V>(k);
+    flip(integral_constant<int, 0x1B>{}, 1);                               // ^ 3
+    step(integral_constant<int, 0xB1>{}, 0);
+    in_lane_merge<V>(k);
+    flip(integral_constant<int, 0x141>{}, 2);                              // ^ 7
+    step(integral_constant<int, 0x4E>{}, 1);                               // ^ 2
+    step(integral_constant<int, 0xB1>{}, 0);
+    in_lane_merge<V>(k);
+    flip(integral_constant<int, 0x140>{}, 3);                              // ^ 15
+#pragma unroll
+    for (int e = 0; e < V; ++e) k[e] = med3(k[e], row_dpp<0x141>(row_dpp<0x1B>(k[e])), bound[2]);   // ^ 4
+    step(integral_constant<int, 0x4E>{}, 1);
+    step(integral_constant<int, 0xB1>{}, 0);
+    in_lane_merge<V>(k);
+}
+
+// sum / count, correctly rounded, for a count of at most 128: sum * (1 / count) in two floats has an error of about 2^-46 of it, and a
+// quotient with so small a divisor is never closer than 2^-32 to the middle between two floats.
+__device__ __forceinline__ float kv_mean(float sum, float count) {
+#pragma clang fp contract(off)
+    const float r = __builtin_amdgcn_rcpf(count), r2 = __builtin_fmaf(-count, r, 1.0f) * r;
+    const float q = sum * r;
+    float d = q + __builtin_fmaf(sum, r2, __builtin_fmaf(sum, r, -q));
+    const bool tiny = fabsf(sum) < 0x1p-90f;                               // the remainders may not be floats
+    if (__ballot(tiny)) {
+        asm volatile("" : "+v"(sum));                                      // keeps the division inside the branch
+        d = tiny ? __fdiv_rn(sum, count) : d;
+    }
+    return d;
+}
+
+// `n` values (x[e] = value c V + e of the row's chunk; anything past n).  Returns false where the chunk has to take the other path;
+// n = 0: nothing to do.  Uniform over a row of lanes; all 64 lanes take part.  srt: room for kSrtPad + 32 V floats, from
+// -kSrtPad on.
+template <int V>
+__device__ __forceinline__ bool kv_lloyd_rows(const float (&x)[V], uint32_t n, uint32_t lane, float* srt, uint32_t (&code)[V], float& cen_out) {
+    const uint32_t c = lane & 15u;
+    const int nan = 0x7FC00000;
+    int k[V];
+    bool finite = true;
+#pragma unroll
+    for (int e = 0; e < V; ++e) {
+        const bool in = c * V + (uint32_t)e < n;
+        finite &= !in || (__float_as_uint(x[e]) & 0x7FFFFFFFu) < 0x7F800000u;
+        k[e] = in ? kv_key(x[e]) : 0x7F800000;                             // +infinity behind the values
+    }
+    row_sort<V>(k, c);
+#pragma unroll
+    for (int e = 0; e < V; ++e) srt[c * V + (uint32_t)e] = kv_unkey(k[e]);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const float lo = srt[0], hi = srt[n ? n - 1u : 0u];
+    const float range = __fsub_rn(hi, lo);
+    bool ok = range >= 1e-10f && range < __builtin_inff();
+    ok &= ((__ballot(!finite) >> (lane & 48u)) & 0xFFFFull) == 0;
+    float cen = __fadd_rn(lo, __fdiv_rn(__fmul_rn(range, (float)c + 0.5f), 16.0f));
+    const float least_gap = range * 0x1p-20f;
+    // NaN before the first value and behind the last one: no comparison holds there.  Likewise the centroid before the first one, and
+    // all centroids of a row that takes the other path: its boundaries stay where they are.
+    if (c < 2u) srt[c ? (int)n : -1] = __int_as_float(nan);
+    cen = ok ? cen : __int_as_float(nan);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    auto lane_below = [&](float v) { return __int_as_float(__builtin_amdgcn_update_dpp(nan, __float_as_int(v), 0x111, 0xF, 0xF, false)); };
+    float below = lane_below(cen);
+    // p: the first sorted value of this cluster, the end of the one before
+    uint32_t p = 0;
+#pragma unroll
+    for (uint32_t h = 8u * V; h > 0; h >>= 1) {
+        const float v = srt[p + h - 1u];
+        p += (p + h <= n) & (fabsf(__fsub_rn(v, below)) <= fabsf(__fsub_rn(v, cen))) ? h : 0u;
+    }
+    uint32_t p_was = 0xFFFFFFFFu, end = 0, end_was = 0;
+    for (int it = 0;; ++it) {
+        for (int moves = 0; moves <= 16 * V; ++moves) {                    // towards the boundary; a direction never turns
+            const float left = srt[(int)p - 1], right = srt[p];
+            const bool up = fabsf(__fsub_rn(right, below)) <= fabsf(__fsub_rn(right, cen));
+            const bool down = fabsf(__fsub_rn(left, cen)) < fabsf(__fsub_rn(left, below));
+            p += up ? 1u : down ? 0xFFFFFFFFu : 0u;
+            if ((__ballot(up) | __ballot(down)) == 0) break;
+        }
+        end = (uint32_t)__builtin_amdgcn_update_dpp((int)n, (int)p, 0x101, 0xF, 0xF, false);   // p of cluster c + 1
+        const bool changed = (p != p_was) | (end != end_was);
+        if (it == 20 || __ballot(changed) == 0) break;
+        const int cnt = changed ? (int)(end - p) : 0;                      // an empty cluster keeps its centroid
+        float sum = 0.f;
+        const float* at = srt + p;                                         // up to 16 V + 16 V floats on, in lanes that are done
+        int left = cnt;
+        do {
+            float v[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[u] = at[u];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) sum = __fadd_rn(sum, left > u ? v[u] : 0.f);   // sum is never -0: + 0 changes nothing
+            at += 4;
+            left -= 4;
+        } while (__ballot(left > 0));
+        const float mean = kv_mean(cnt > 0 ? sum : 1.0f, (float)(cnt > 0 ? cnt : 1));
+        cen = cnt > 0 ? mean : cen;
+        below = lane_below(cen);
+        const bool tight = __fsub_rn(cen, below) <= least_gap;             // false for the first one
+        ok &= !tight;
+        p_was = p;
+        end_was = end;
+    }
+    ok = ((__ballot(!ok) >> (lane & 48u)) & 0xFFFFull) == 0;
+    // a value's cluster is the last one whose first member is not larger
+    const float first = p < n ? srt[p] : __builtin_inff();
+#pragma unroll
+    for (int e = 0; e < V; ++e) {
+        uint32_t q = 0;
+#pragma unroll
+        for (uint32_t h = 8; h > 0; h >>= 1) {
+            const float t = __int_as_float(__builtin_amdgcn_ds_bpermute((int)(4u * ((lane & 48u) + q + h)), __float_as_int(first)));
+            q = x[e] >= t ? q + h : q;
+        }
+        code[e] = q;
+    }
+    cen_out = cen;
+    return ok || n == 0;
+}
+
+// Up to four chunks of a wavefront: chunk(g, src, n) says where row g's chunk is (n = 0: none).  Leaves the codes of values c V + e in
+// code[e] and centroid c in cen.
+template <int V>
+struct KvRows {
+    float srt[4 * (16 * V + kSrtPad) + 16 * V];
+    KvLds slow;
+};
+template <int V>
+__device__ __forceinline__ void kv_quantize_rows(const float* src, uint32_t n, uint32_t lane, KvRows<V>& L, uint32_t (&code)[V], float& cen) {
+    const uint32_t c = lane & 15u;
+    float x[V];
+    if (n == 16u * V && (reinterpret_cast<uintptr_t>(src) & (V == 2 ? 7u : 15u)) == 0) {
+        if constexpr (V == 2) {
+            const float2 f = reinterpret_cast<const float2*>(src)[c];
+            x[0] = f.x; x[1] = f.y;
+        } else {
+#pragma unroll
+            for (int h = 0; h < V / 4; ++h) {
+                const float4 f = reinterpret_cast<const float4*>(src)[c * (V / 4) + (uint32_t)h];
+                x[4 * h] = f.x; x[4 * h + 1] = f.y; x[4 * h + 2] = f.z; x[4 * h + 3] = f.w;
+            }
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < V; ++e) x[e] = c * V + (uint32_t)e < n ? src[c * V + (uint32_t)e] : 0.f;
+    }
+    const bool ok = kv_lloyd_rows<V>(x, n, lane, L.srt + (lane >> 4) * (16 * V + kSrtPad) + kSrtPad, code, cen);
+    uint64_t left = __ballot(!ok);
+    while (left) {                                                         // chunk by chunk, by all 64 lanes
+        const uint32_t at = (uint32_t)__builtin_ctzll(left);
+        left &= ~(0xFFFFull << (at & 48u));
+        const uint64_t p = reinterpret_cast<uint64_t>(src);
+        const uint64_t q = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)p, (int)at) |
+                           (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(p >> 32), (int)at) << 32;
+        kv_quantize_chunk(reinterpret_cast<const float*>(q), (uint32_t)__builtin_amdgcn_readlane((int)n, (int)at), lane, L.slow);
+        if ((lane & 48u) == (at & 48u)) {
+#pragma unroll
+            for (int e = 0; e < V; ++e) code[e] = L.slow.code[(c * V + (uint32_t)e) & 127u];
+            cen = L.slow.cen[c];
+        }
+        __syncthreads();
+    }
+}
+
+// One row of 16 lanes per (token, chunk of the token, K or V), `per_wave` rows of a wavefront in use.  pos = tokens the layer
+// held before this call, ntok = tokens of this call that fit.  K centroids are stored by the chunk that opens a block, or -- while the layer is empty, and
 // for V always -- by the last chunk of the call that touches the block (:256-261, :277-279: later writes win).
+template <int V>
 __global__ void __launch_bounds__(64)
 kv_append_kernel(uint8_t* __restrict__ k_idx, uint8_t* __restrict__ v_idx, uint16_t* __restrict__ k_cb,
                  uint16_t* __restrict__ v_cb, const float* __restrict__ k, const float* __restrict__ v, int64_t pos,
-                 int64_t ntok, int64_t per_token, uint32_t block, uint32_t chunks_per_token, int64_t idx_bytes) {
-    __shared__ KvLds L;
-    const uint32_t lane = threadIdx.x;
-    const int64_t s = blockIdx.x / chunks_per_token;
-    const uint32_t c = blockIdx.x % chunks_per_token;
+                 int64_t ntok, int64_t per_token, uint32_t chunks_per_token, uint32_t items, uint32_t per_wave, int64_t idx_bytes) {
+    __shared__ KvRows<V> L;
+    constexpr int64_t block = 16 * V;
+    const uint32_t lane = threadIdx.x, row = lane >> 4, c = lane & 15u;
     const bool is_v = blockIdx.y != 0;
+    const uint32_t item = blockIdx.x * per_wave + row;
+    const bool in = row < per_wave && item < items;
+    const int64_t s = in ? item / chunks_per_token : 0;
+    const uint32_t ch = in ? item % chunks_per_token : 0u;
     const int64_t tok_lo = (pos + s) * per_token, tok_hi = tok_lo + per_token;
-    const int64_t blk = tok_lo / block + c;
-    const int64_t a = c == 0 ? tok_lo : blk * block;
-    if (a >= tok_hi) return;
+    const int64_t blk = tok_lo / block + ch;
+    const int64_t a = ch == 0 ? tok_lo : blk * block;
     const int64_t b = (blk + 1) * block < tok_hi ? (blk + 1) * block : tok_hi;
-    const uint32_t n = (uint32_t)(b - a);
-    const float* src = (is_v ? v : k) + (a - pos * per_token);
-    kv_quantize_chunk(src, n, lane, L);
-    const bool last_on_block = (b % block) == 0 || b == (pos + ntok) * per_token;
-    const uint32_t off = (uint32_t)(a % block);
-    const int64_t at = blk * (int64_t)(block >> 1) + (off >> 1);
+    const uint32_t n = in && a < tok_hi ? (uint32_t)(b - a) : 0u;
+    const float* src = (is_v ? v : k) + (n ? a - pos * per_token : 0);
+    uint32_t code[V];
+    float cen;
+    kv_quantize_rows<V>(src, n, lane, L, code, cen);
+    if (n == 0) return;
+    const bool last_on_block = (b & (block - 1)) == 0 || b == (pos + ntok) * per_token;
+    const uint32_t off = (uint32_t)(a & (block - 1));
+    const int64_t at = blk * (block >> 1) + (off >> 1);
     uint32_t nbytes = (n + 1) >> 1;
     if (!(off & 1u) && (n & 1u) && !last_on_block) --nbytes;        // that byte belongs to the next chunk of this call
     if (at + nbytes > idx_bytes) nbytes = at < idx_bytes ? (uint32_t)(idx_bytes - at) : 0u;   // :248-249
     uint8_t* idx = (is_v ? v_idx : k_idx) + at;
-    if (lane < nbytes) idx[lane] = (uint8_t)(L.code[2 * lane] | (2 * lane + 1 < n ? L.code[2 * lane + 1] << 4 : 0));
-    const bool store_cb = (is_v || pos == 0) ? last_on_block : (a % block) == 0;
-    if (store_cb && lane < 16) (is_v ? v_cb : k_cb)[blk * 16 + lane] = (uint16_t)kv_float_to_half(L.cen[lane]);
+    uint32_t bytes = 0;
+#pragma unroll
+    for (int e = 0; e < V; ++e) bytes |= (c * V + (uint32_t)e < n ? code[e] : 0u) << (4 * e);
+    if (nbytes == (uint32_t)block / 2u) {                            // whole block: aligned
+        if constexpr (V == 2) idx[c] = (uint8_t)bytes;
+        if constexpr (V == 4) reinterpret_cast<uint16_t*>(idx)[c] = (uint16_t)bytes;
+        if constexpr (V == 8) reinterpret_cast<uint32_t*>(idx)[c] = bytes;
+    } else {
+#pragma unroll
+        for (int i = 0; i < V / 2; ++i)
+            if (c * (V / 2) + (uint32_t)i < nbytes) idx[c * (V / 2) + (uint32_t)i] = (uint8_t)(bytes >> (8 * i));
+    }
+    const bool store_cb = (is_v || pos == 0) ? last_on_block : off == 0;
+    if (store_cb) (is_v ? v_cb : k_cb)[blk * 16 + c] = (uint16_t)kv_float_to_half(cen);
 }
 
-// OIL4KVCache::quantize_block_oil4 over nblocks independent runs of n <= 128 values: one code per byte, 16 centroids.
+// OIL4KVCache::quantize_block_oil4 over nblocks independent runs of n <= 16 V values: one code per byte, 16 centroids.
+template <int V>
 __global__ void __launch_bounds__(64)
-kv_quantize_blocks_kernel(const float* __restrict__ src, uint32_t n, uint8_t* __restrict__ codes, uint16_t* __restrict__ cb) {
-    __shared__ KvLds L;
-    const uint32_t lane = threadIdx.x;
-    const size_t at = (size_t)blockIdx.x * n;
-    kv_quantize_chunk(src + at, n, lane, L);
-    if (lane < n) codes[at + lane] = L.code[lane];
-    if (lane + 64 < n) codes[at + lane + 64] = L.code[lane + 64];
-    if (lane < 16) cb[(size_t)blockIdx.x * 16 + lane] = (uint16_t)kv_float_to_half(L.cen[lane]);
+kv_quantize_blocks_kernel(const float* __restrict__ src, uint32_t n, uint32_t nblocks, uint32_t per_wave, uint8_t* __restrict__ codes,
+                          uint16_t* __restrict__ cb) {
+    __shared__ KvRows<V> L;
+    const uint32_t lane = threadIdx.x, row = lane >> 4, c = lane & 15u;
+    const uint32_t item = blockIdx.x * per_wave + row;
+    const bool in = row < per_wave && item < nblocks;
+    const size_t at = in ? (size_t)item * n : 0;
+    uint32_t code[V];
+    float cen;
+    kv_quantize_rows<V>(src + at, in ? n : 0u, lane, L, code, cen);
+    if (!in) return;
+#pragma unroll
+    for (int e = 0; e < V; ++e)
+        if (c * V + (uint32_t)e < n) codes[at + c * V + (uint32_t)e] = (uint8_t)code[e];
+    cb[(size_t)item * 16 + c] = (uint16_t)kv_float_to_half(cen);
 }
+
+// Chunks per wavefront: four fill its lanes; with fewer chunks than keep two wavefronts on every SIMD, one each, so that a chunk waits
+// for its own iterations only.
+uint32_t kv_per_wave(uint64_t chunks) { return chunks >= 8ull * (uint64_t)device_cu_count() ? 4u : 1u; }
 
 // dequantize_block_oil4 (:155-161): dst[b][i] = half_to_float(cb[b][codes[b][i] & 15])
 __global__ void __launch_bounds__(256)
@@ -297,8 +489,11 @@ kv_dequantize_blocks_kernel(const uint8_t* __restrict__ codes, const uint16_t* _
 
 // get_range for tokens whose value count is a multiple of 4 (value e is then nibble e & 1 of byte e / 2).  A workgroup decodes kTile consecutive elements of K
 // (blockIdx.y = 0) or V (1): the centroids of the blocks under the tile go to LDS as FP32 once, then each thread
-// turns 2 bytes of codes into one 16-byte store, four times.
+// turns 2 bytes of codes into one 16-byte store, four times.  Bound by the stores, which bypass the caches: 2056 tokens of
+// 4096 (67 MB out) take 13.9 us, with ordinary stores 16.9.
 constexpr uint32_t kTile = 4096;
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 __global__ void __launch_bounds__(256)
 kv_get_range_kernel(const uint8_t* __restrict__ k_idx, const uint8_t* __restrict__ v_idx, const uint16_t* __restrict__ k_cb,
                     const uint16_t* __restrict__ v_cb, float* __restrict__ k_out, float* __restrict__ v_out, uint64_t first,
@@ -323,8 +518,9 @@ kv_get_range_kernel(const uint8_t* __restrict__ k_idx, const uint8_t* __restrict
             const uint64_t e = first + j0 + j;
             const uint32_t codes = *reinterpret_cast<const uint16_t*>(idx + (e >> 1));
             const float* t = cen + (uint32_t)((e >> block_shift) - blk0) * 16;
-            *reinterpret_cast<float4*>(out + j0 + j) =
-                make_float4(t[codes & 15u], t[(codes >> 4) & 15u], t[(codes >> 8) & 15u], t[(codes >> 12) & 15u]);
+            f32x4 o;
+            o.x = t[codes & 15u]; o.y = t[(codes >> 4) & 15u]; o.z = t[(codes >> 8) & 15u]; o.w = t[(codes >> 12) & 15u];
+            __builtin_nontemporal_store(o, reinterpret_cast<f32x4*>(out + j0 + j));
         }
     }
 }
@@ -350,9 +546,10 @@ kv_get_range_scalar_kernel(const uint8_t* __restrict__ k_idx, const uint8_t* __r
     (blockIdx.y ? v_out : k_out)[j] = kv_half_to_float(cb[blk * 16 + code]);
 }
 
-__global__ void __launch_bounds__(256) kv_zero_kernel(uint4* p, uint64_t n16) {
-    for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n16; i += (uint64_t)gridDim.x * 256)
-        p[i] = make_uint4(0, 0, 0, 0);
+// codes and centroids in one launch
+__global__ void __launch_bounds__(256) kv_zero_kernel(uint4* p, uint64_t np, uint4* q, uint64_t nq) {
+    for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < np + nq; i += (uint64_t)gridDim.x * 256)
+        __builtin_nontemporal_store(u32x4{0, 0, 0, 0}, reinterpret_cast<u32x4*>((i < np ? p : q - np) + i));
 }
 
 int kv_alloc(oilhip_kv* c) {
@@ -426,11 +623,14 @@ int oilhip_kv_append(oilhip_kv* c, int layer, const float* d_k, const float* d_v
     if (ntok > seq_len) ntok = seq_len;
     if (ntok > 0 && c->per_token > 0) {
         if (!d_k || !d_v) return fail(OILHIP_E_ARG, "kv_append: null input");
-        const uint32_t cpt = (uint32_t)((c->per_token + c->block - 1) / c->block + 1);
-        if (ntok * (int64_t)cpt > 0x7FFFFFFF) return fail(OILHIP_E_ARG, "kv_append: too many tokens for one call");
-        hipLaunchKernelGGL(kv_append_kernel, dim3((uint32_t)(ntok * cpt), 2), dim3(64), 0, (hipStream_t)stream,
-                           kv_idx(c, layer, 0), kv_idx(c, layer, 1), kv_cb(c, layer, 0), kv_cb(c, layer, 1), d_k, d_v, pos, ntok,
-                           c->per_token, (uint32_t)c->block, cpt, c->idx_bytes);
+        // chunks of a token: one more where its ends may lie inside blocks
+        const int64_t cpt = (c->per_token + c->block - 1) / c->block + (c->per_token % c->block ? 1 : 0);
+        if (ntok * cpt > 0x7FFFFFFF) return fail(OILHIP_E_ARG, "kv_append: too many tokens for one call");
+        const uint32_t items = (uint32_t)(ntok * cpt), per_wave = kv_per_wave(2ull * items);
+        auto kern = c->block == 32 ? kv_append_kernel<2> : c->block == 64 ? kv_append_kernel<4> : kv_append_kernel<8>;
+        hipLaunchKernelGGL(kern, dim3((items + per_wave - 1u) / per_wave, 2), dim3(64), 0, (hipStream_t)stream, kv_idx(c, layer, 0),
+                           kv_idx(c, layer, 1), kv_cb(c, layer, 0), kv_cb(c, layer, 1), d_k, d_v, pos, ntok, c->per_token, (uint32_t)cpt,
+                           items, per_wave, c->idx_bytes);
         OILHIP_HIP(hipGetLastError());
     }
     c->pos[(size_t)layer] = pos + seq_len;                                          // :290, dropped tokens counted as well
@@ -483,8 +683,9 @@ int oilhip_kv_info(const oilhip_kv* c, int* context_len, int64_t* block_size, ui
 int oilhip_kv_clear(oilhip_kv* c, void* stream) {
     if (!c) return fail(OILHIP_E_ARG, "kv_clear: cache is null");
     const uint64_t n_idx = (uint64_t)c->layers * 2 * (uint64_t)c->idx_stride / 16, n_cb = (uint64_t)c->layers * 2 * (uint64_t)c->nblocks * 32 / 16;
-    if (n_idx) hipLaunchKernelGGL(kv_zero_kernel, dim3((uint32_t)std::min<uint64_t>((n_idx + 255) / 256, 4096)), dim3(256), 0, (hipStream_t)stream, reinterpret_cast<uint4*>(c->d_idx), n_idx);
-    if (n_cb) hipLaunchKernelGGL(kv_zero_kernel, dim3((uint32_t)std::min<uint64_t>((n_cb + 255) / 256, 4096)), dim3(256), 0, (hipStream_t)stream, reinterpret_cast<uint4*>(c->d_cb), n_cb);
+    if (n_idx + n_cb)
+        hipLaunchKernelGGL(kv_zero_kernel, dim3((uint32_t)std::min<uint64_t>((n_idx + n_cb + 255) / 256, 4096)), dim3(256), 0, (hipStream_t)stream,
+                           reinterpret_cast<uint4*>(c->d_idx), n_idx, reinterpret_cast<uint4*>(c->d_cb), n_cb);
     OILHIP_HIP(hipGetLastError());
     for (auto& p : c->pos) p = 0;
     return OILHIP_OK;
@@ -519,7 +720,10 @@ int oilhip_kv_quantize_blocks(const float* d_src, int64_t n, int64_t nblocks, ui
     if (n == 0 || nblocks == 0) return OILHIP_OK;                                   // :78
     if (!d_src || !d_codes || !d_cb16) return fail(OILHIP_E_ARG, "kv_quantize_blocks: null pointer");
     if (nblocks > 0x7FFFFFFF) return fail(OILHIP_E_ARG, "kv_quantize_blocks: too many blocks for one call");
-    hipLaunchKernelGGL(kv_quantize_blocks_kernel, dim3((uint32_t)nblocks), dim3(64), 0, (hipStream_t)stream, d_src, (uint32_t)n, d_codes, d_cb16);
+    const uint32_t per_wave = kv_per_wave((uint64_t)nblocks);
+    auto kern = n <= 32 ? kv_quantize_blocks_kernel<2> : n <= 64 ? kv_quantize_blocks_kernel<4> : kv_quantize_blocks_kernel<8>;
+    hipLaunchKernelGGL(kern, dim3(((uint32_t)nblocks + per_wave - 1u) / per_wave), dim3(64), 0, (hipStream_t)stream, d_src, (uint32_t)n,
+                       (uint32_t)nblocks, per_wave, d_codes, d_cb16);
     OILHIP_HIP(hipGetLastError());
     return OILHIP_OK;
 }

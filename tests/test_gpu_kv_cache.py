@@ -62,6 +62,26 @@ def test_quantize_blocks_fixture_and_oracle():
         assert np.array_equal(back[0].view(np.uint32), want.view(np.uint32))
 
 
+# sixteen lanes per block: rows of 2, 4 and 8 values per lane, full and partial; one block per wavefront (few blocks) and four (from
+# 2048 on, the last wavefront not full); blocks whose centroids come too close together for the boundary search, tiny sums,
+# clusters that stay empty, and constant blocks between ordinary ones
+@pytest.mark.parametrize("n", [1, 3, 16, 31, 32, 33, 50, 64, 65, 127, 128])
+@pytest.mark.parametrize("blocks", [5, 2053])
+def test_quantize_blocks_rows_of_lanes(n, blocks):
+    rng = np.random.default_rng(n + blocks)
+    x = rng.standard_normal((blocks, n)).astype(np.float32)
+    x[1::7] = np.float32(1.0) + rng.integers(0, 40, x[1::7].shape).astype(np.float32) * np.float32(2.0 ** -23)   # range below and near the constant limit
+    x[2::7, 0] = 3e7                                          # everything else within a few steps of the distances' rounding
+    x[3::7] = rng.integers(-3, 4, x[3::7].shape)              # ties, fewer values than clusters, zeros
+    x[4::7] *= np.float32(1e-30)
+    x[4::7, :1] += np.float32(1.0)                            # sums far below the range
+    codes, cb = ia.OIL4KVCache.quantize_block_oil4(dev(x))
+    codes, cb = codes.cpu().numpy(), cb.cpu().numpy().view(np.uint16)
+    for b in range(blocks):
+        wcb, wcodes = O.kv_quantize_block(x[b])
+        assert np.array_equal(cb[b], wcb) and np.array_equal(codes[b], wcodes), b
+
+
 @pytest.mark.parametrize("i", range(len(MF.KV_CASES)))
 def test_cache_fixture(i):
     ms, h, d, block, lens = MF.KV_CASES[i]
