@@ -586,23 +586,20 @@ int oilhip_gemv_f32_general(const oilhip_weights* w, const float* d_x, float* d_
     return launch_gemv_generic(*w, d_x, d_y, M, (hipStream_t)stream);
 }
 
-int oilhip_gemm_bf16(const oilhip_weights* w, const uint16_t* d_x, float* d_y, int M, void* stream) {
+static int prefill(const oilhip_weights* w, const void* d_x, bool x_is_f32, float* d_y, int M, hipStream_t s) {
     if (int rc = check_matmul_shape(w, d_x, d_y, M)) return rc;
-    if (plain_oil4(*w)) return launch_gemm_oil4_bf16(*w, d_x, d_y, M, (hipStream_t)stream);
-    // any other tensor of full blocks: decoded to bf16 slab by slab, then the same kernel over a dense operand
-    const int rc = launch_gemm_any_bf16(*w, d_x, d_y, M, (hipStream_t)stream);
+    if (plain_oil4(*w)) return launch_gemm_oil4_frag(*w, d_x, x_is_f32, d_y, M, s);
+    const int rc = launch_gemm_any(*w, d_x, x_is_f32, d_y, M, s);
     if (rc == 1) return fail(OILHIP_E_ARG, "bf16 prefill GEMM needs full blocks with the channel sizes the quantizer writes");
     return rc;
 }
 
+int oilhip_gemm_bf16(const oilhip_weights* w, const uint16_t* d_x, float* d_y, int M, void* stream) {
+    return prefill(w, d_x, false, d_y, M, (hipStream_t)stream);
+}
+
 int oilhip_gemm_f32(const oilhip_weights* w, const float* d_x, float* d_y, int M, void* stream) {
-    if (int rc = check_matmul_shape(w, d_x, d_y, M)) return rc;
-    hipStream_t s = (hipStream_t)stream;
-    // plain OIL4: the pre-pass of the prefill kernel rounds X on its way into fragment order
-    if (plain_oil4(*w) && (reinterpret_cast<uintptr_t>(d_x) & 15u) == 0u) return launch_gemm_oil4_frag(*w, d_x, true, d_y, M, s);
-    uint16_t* xb = nullptr;
-    if (int rc = launch_x_to_bf16(d_x, (uint64_t)M * w->cols, &xb, s)) return rc;
-    return oilhip_gemm_bf16(w, xb, d_y, M, stream);
+    return prefill(w, d_x, true, d_y, M, (hipStream_t)stream);
 }
 
 int oilhip_release_stream_scratch(void* stream) {

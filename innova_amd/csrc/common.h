@@ -46,7 +46,7 @@ int ensure_max_lds(std::atomic<uint64_t>& done, const void* kernel, int bytes);
 // one and the old one stays allocated.  No allocation can happen while the stream is being captured, so the first
 // call of a given size on a stream has to be made outside capture; otherwise the call fails with OILHIP_E_ARG.
 // New buffers are zero-filled.
-enum ScratchSlot { kScratchGemvPack = 0, kScratchGemmX = 1, kScratchTl = 2, kScratchGemmW = 3, kScratchGemmXb = 4 };
+enum ScratchSlot { kScratchGemvPack = 0, kScratchGemmX = 1, kScratchTl = 2, kScratchGemmW = 3, kScratchGemmP = 4 };
 int stream_scratch(hipStream_t s, int slot, size_t bytes, void** out);
 
 // Tensors whose rows mix formats are stored as `nstreams` streams of windows of at most 4 KB, one wavefront per stream
@@ -103,8 +103,10 @@ inline bool plain_oil8(const oilhip_weights& w) {
 
 // kernels (each returns an OILHIP_* code and sets the error text)
 int launch_dequant(const oilhip_weights& w, float* d_out, hipStream_t s);
-int launch_dequant_bf16_blocks(const oilhip_weights& w, uint32_t b0, uint32_t nb, uint16_t* d_out, hipStream_t s);
-bool dequant_bf16_blocks_covers(const oilhip_weights& w);   // whether launch_dequant_bf16_blocks takes this tensor's layout
+// operands of the prefill GEMM in fragment order (generic_kernels.hip)
+int launch_dense_prepare(const oilhip_weights& w, uint32_t row0, uint32_t rows, uint16_t* wf, const void* x, bool x_is_f32, uint32_t M,
+                         uint16_t* xf, uint32_t* arrived, uint32_t ncount, hipStream_t s);
+bool dense_prepare_covers(const oilhip_weights& w);   // whether launch_dense_prepare takes this tensor's layout
 int launch_gemv_generic(const oilhip_weights& w, const float* d_x, float* d_y, int M, hipStream_t s);
 // fast paths return 1 when they do not cover the case (caller falls through to the general kernel)
 int launch_gemv_oil4(const oilhip_weights& w, const float* d_x, float* d_y, int M, hipStream_t s);
@@ -138,10 +140,8 @@ constexpr size_t kGemvPackBytes = (size_t)(kGemvPackMaxCols >> 8) * (128u + 2457
 int launch_gemv_seg(const oilhip_weights& w, const float* d_x, float* d_y, int M, hipStream_t s);
 // every format, a lane per run of 32 weights
 int launch_gemv_runs(const oilhip_weights& w, const float* d_x, float* d_y, int M, hipStream_t s);
-int launch_gemm_oil4_bf16(const oilhip_weights& w, const uint16_t* d_x, float* d_y, int M, hipStream_t s);
-int launch_gemm_any_bf16(const oilhip_weights& w, const uint16_t* d_x, float* d_y, int M, hipStream_t s);
-// FP32 activations [M][K] rounded once to bf16 bit patterns (a scratch buffer of the stream)
-int launch_x_to_bf16(const float* d_x, uint64_t n, uint16_t** out, hipStream_t s);
-// plain uniform OIL4, more than 256 tokens: activations in fragment order straight from memory (gemm_oil4_frag.hip)
+// prefill: x is bf16 bit patterns, or FP32 (rounded once to bf16) when x_is_f32; any tensor of full blocks (gemm_dense.hip) ...
+int launch_gemm_any(const oilhip_weights& w, const void* d_x, bool x_is_f32, float* d_y, int M, hipStream_t s);
+// ... and plain uniform OIL4, decoded inside the kernel (gemm_oil4_frag.hip)
 int launch_gemm_oil4_frag(const oilhip_weights& w, const void* d_x, bool x_is_f32, float* d_y, int M, hipStream_t s);
 }  // namespace oilhip

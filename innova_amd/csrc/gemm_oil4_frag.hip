@@ -1,4 +1,4 @@
-// gemm_oil4_frag.hip -- prefill GEMM over uniform OIL4 tensors (any batch size; 16-byte aligned activations):
+// gemm_oil4_frag.hip -- prefill GEMM over uniform OIL4 tensors (any batch size):
 // Y[M][N] = X[M][K] . W^T, X in bf16 (or FP32, rounded once to bf16), W dequantized to bf16 on the fly,
 // v_mfma_f32_32x32x16_bf16 with FP32 accumulation, FP32 output.  Same contraction as the reference's FP32
 // prefill (Qwen35Engine::gemm with B up to 512, src/adapters/tools/qwen35_engine.cpp:47-85,630-753) over
@@ -37,6 +37,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "gemm_tiles.h"
 #include "oil4_lds.h"
 
 namespace oilhip {
@@ -51,23 +52,6 @@ using oil4::u32x4;
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-// Tile order: token blocks in groups of four; inside a group weight-row blocks ascending, the group's token blocks
-// innermost.  A run of consecutive tiles therefore covers few token blocks and neighbouring weight rows.
-__host__ __device__ inline void frag_tile_of(uint32_t T, uint32_t MT, uint32_t NT, uint32_t& mt, uint32_t& nt) {
-    const uint32_t per = 4u * NT, lastg = (MT - 1u) / 4u;
-    uint32_t mg = T / per;
-    if (mg > lastg) mg = lastg;
-    const uint32_t rem = T - mg * per, left = MT - 4u * mg, gm = left < 4u ? left : 4u;
-    nt = rem / gm;
-    mt = 4u * mg + rem % gm;
-}
-
-// Workgroups are dealt to the eight XCDs in turn; XCD x takes the x-th run of n / 8 consecutive items.
-__device__ inline uint32_t xcd_chunk(uint32_t b, uint32_t n) {
-    const uint32_t x = b & 7u, q = b >> 3, c = n >> 3, r = n & 7u;
-    return (x < r ? x * (c + 1u) : r * (c + 1u) + (x - r) * c) + q;
-}
 
 struct FragGrid {
     uint32_t MT, NT;        // tiles along tokens and weight rows
@@ -109,20 +93,24 @@ pack_x_frag_kernel(const void* __restrict__ xin, uint16_t* __restrict__ xf, uint
 #pragma unroll
         for (int j = 0; j < 4; ++j) v[j] = make_uint4(0u, 0u, 0u, 0u);
         if (m < M) {
+            // 16-byte loads wherever the rows start
             if constexpr (F32) {
-                const float4* xr = reinterpret_cast<const float4*>(reinterpret_cast<const float*>(xin) + (size_t)m * K + blk * 256u);
+                typedef float f32x4 __attribute__((ext_vector_type(4)));
+                typedef f32x4 f32x4_4 __attribute__((aligned(4)));
+                const f32x4_4* xr = reinterpret_cast<const f32x4_4*>(reinterpret_cast<const float*>(xin) + (size_t)m * K + blk * 256u);
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    const float4 f0 = xr[2u * (q + 8u * j)], f1 = xr[2u * (q + 8u * j) + 1u];
+                    const f32x4 f0 = xr[2u * (q + 8u * j)], f1 = xr[2u * (q + 8u * j) + 1u];
                     const bf16x2 p0 = bf16x2{(__bf16)f0.x, (__bf16)f0.y}, p1 = bf16x2{(__bf16)f0.z, (__bf16)f0.w};
                     const bf16x2 p2 = bf16x2{(__bf16)f1.x, (__bf16)f1.y}, p3 = bf16x2{(__bf16)f1.z, (__bf16)f1.w};
                     v[j] = make_uint4(*reinterpret_cast<const uint32_t*>(&p0), *reinterpret_cast<const uint32_t*>(&p1),
                                       *reinterpret_cast<const uint32_t*>(&p2), *reinterpret_cast<const uint32_t*>(&p3));
                 }
             } else {
-                const uint4* xr = reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(xin) + (size_t)m * K + blk * 256u);
+                typedef u32x4 u32x4_2 __attribute__((aligned(2)));
+                const u32x4_2* xr = reinterpret_cast<const u32x4_2*>(reinterpret_cast<const uint16_t*>(xin) + (size_t)m * K + blk * 256u);
 #pragma unroll
-                for (int j = 0; j < 4; ++j) v[j] = xr[q + 8u * j];
+                for (int j = 0; j < 4; ++j) { const u32x4 t = xr[q + 8u * j]; v[j] = make_uint4(t.x, t.y, t.z, t.w); }
             }
         }
 #pragma unroll

@@ -309,7 +309,7 @@ __device__ __forceinline__ bool kv_lloyd_rows(const float (&x)[V], uint32_t n, u
 #pragma unroll
     for (uint32_t h = 8u * V; h > 0; h >>= 1) {
         const float v = srt[p + h - 1u];
-        p += (p + h <= n) & (fabsf(__fsub_rn(v, below)) <= fabsf(__fsub_rn(v, cen))) ? h : 0u;
+        p += ((p + h <= n) & (fabsf(__fsub_rn(v, below)) <= fabsf(__fsub_rn(v, cen)))) ? h : 0u;
     }
     uint32_t p_was = 0xFFFFFFFFu, end = 0, end_was = 0;
     for (int it = 0;; ++it) {

@@ -140,6 +140,25 @@ def test_planner_routed_matrix_prefill():
     _check_any_format(np.asarray(pl.allocate(rows * cols // 256).formats, dtype=np.uint8), rows, cols, M, 5)
 
 
+# the dense-operand kernel: token and row counts around its tiles of 64 and 128, K from one block (no parts) to several parts, a launch of
+# 128-tiles, tensors with more and with fewer workgroups in the pre-pass than the chip holds, both kinds of activations
+@pytest.mark.parametrize("fmt", [ia.Format.OIL8_GRP, (0, 1), (7, 9, 10, 11), (0, 3, 13, 14)])
+@pytest.mark.parametrize("rows,cols,M", [(1, 256, 1), (63, 256, 65), (65, 512, 64), (129, 1536, 127), (200, 2048, 129), (31, 7936, 33),
+                                          (4100, 1024, 600)])
+def test_dense_operand_tiles(fmt, rows, cols, M):
+    nb = rows * cols // 256
+    ids = np.full(nb, int(fmt)) if isinstance(fmt, ia.Format) else np.random.default_rng(nb).choice(fmt, nb)
+    payload, blocks = ia.block_codec.quantize_tensor(gaussian_weights(rows * cols, nb), ids.astype(np.uint8))
+    x = torch.randn(M, cols, generator=torch.Generator().manual_seed(M))
+    sel = np.unique(np.r_[np.arange(0, rows, max(1, rows // 40)), rows - 1])
+    want = O.block_gemm(payload, to_orc_blocks(blocks).reshape(rows, -1)[sel].reshape(-1), sel.size, cols, x.to(torch.bfloat16).float().numpy(), wide=True)
+    with ia.DeviceWeights.from_blocks(payload, blocks, rows, cols) as dw:
+        yb, yf = dw.gemm_bf16(x.to(torch.bfloat16).cuda()), dw.gemm_f32(x.cuda())
+        assert torch.equal(yb, yf)
+        assert rel_l2(yb.cpu().numpy()[:, sel], want) <= TOL
+        assert torch.equal(dw.gemm_f32(x.cuda()), yf)          # parts are added in one order
+
+
 def test_slabs_of_a_tall_tensor():
     """More rows than one 64 MB slab of bf16 holds (8192 at 4096 columns): two slabs, the second partial."""
     _check_any_format(ia.Format.SPARK_Q0, 8192 + 384, 4096, 260, 77)
