@@ -115,6 +115,18 @@ int stream_scratch(hipStream_t s, int slot, size_t bytes, void** out) {
     return OILHIP_OK;
 }
 
+// whether stream_scratch would succeed without an allocation that stream capture forbids
+bool stream_scratch_ready(hipStream_t s, int slot, size_t bytes) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) == hipSuccess && st == hipStreamCaptureStatusNone) return true;
+    (void)hipGetLastError();
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return false;
+    std::lock_guard<std::mutex> lk(g_scratch_mu);
+    const auto e = g_scratch.find(std::make_tuple(dev, (void*)s, slot));
+    return e != g_scratch.end() && e->second.second >= bytes;
+}
+
 int check_matmul_shape(const oilhip_weights* w, const void* x, const void* y, int M) {
     if (!w || !x || !y) return fail(OILHIP_E_ARG, "null argument");
     if (M < 1) return fail(OILHIP_E_ARG, "M must be >= 1");
@@ -558,6 +570,10 @@ int oilhip_gemv_f32(const oilhip_weights* w, const float* d_x, float* d_y, int M
             rc = launch_gemv_oil4_multi(*w, d_x, nullptr, d_y, M, (uint32_t)w->cols, (uint32_t)w->rows, (uint32_t)M,
                                         (hipStream_t)stream);
         if (rc == 1 && M > 2 && M <= 4) rc = launch_gemv_oil4(*w, d_x, d_y, M, (hipStream_t)stream);
+        if (rc <= 0) return rc;
+    }
+    if (M >= 2) {
+        const int rc = launch_gemv_any_multi(*w, d_x, d_y, M, (hipStream_t)stream);
         if (rc <= 0) return rc;
     }
     if (plain_oil8(*w)) {

@@ -48,6 +48,7 @@ int ensure_max_lds(std::atomic<uint64_t>& done, const void* kernel, int bytes);
 // New buffers are zero-filled.
 enum ScratchSlot { kScratchGemvPack = 0, kScratchGemmX = 1, kScratchTl = 2, kScratchGemmW = 3, kScratchGemmP = 4 };
 int stream_scratch(hipStream_t s, int slot, size_t bytes, void** out);
+bool stream_scratch_ready(hipStream_t s, int slot, size_t bytes);   // false: this call would fail, the stream is being captured
 
 // Tensors whose rows mix formats are stored as `nstreams` streams of windows of at most 4 KB, one wavefront per stream
 // (gemv_seg.hip).  The first window of stream s sits at byte s * stream_bytes of the payload buffer, the later ones
@@ -132,10 +133,12 @@ size_t gemv_oil4_multi_batches_bytes(int nb, uint64_t cols);
 int launch_gemv_oil4_multi_batches(int nb, const oilhip_weights* const* wa, float* const* ya, const oilhip_weights* const* wb, float* const* yb,
                                    const int* M, const int* row0, const int* list, int nlist, const float* d_x, const float* d_x2,
                                    uint32_t ldx, uint32_t xrows, uint32_t ldy, void* d_ws, size_t ws_bytes, hipStream_t s);
-// widest row that kernel takes and the bytes of packed activations one pass of it needs (d_pack, or stream scratch): per
-// block 32 floats (powers of two) and three digits of 256 activations for 32 tokens
+// other formats, 3 to 16 rows per pass (FP16 MFMA, gemv_any_multi.hip)
+int launch_gemv_any_multi(const oilhip_weights& w, const float* d_x, float* d_y, int M, hipStream_t s);
+// widest row that these kernels take and the bytes of packed activations one pass needs (d_pack, or stream scratch): per
+// block 32 floats (powers of two) and three digits of 256 activations for 32 tokens, or 48 floats and 27 KB of FP16 pieces
 constexpr uint32_t kGemvPackMaxCols = 32768;
-constexpr size_t kGemvPackBytes = (size_t)(kGemvPackMaxCols >> 8) * (128u + 24576u);
+constexpr size_t kGemvPackBytes = (size_t)(kGemvPackMaxCols >> 8) * (192u + 27648u);
 // rows that mix formats, stored tile by tile and format by format
 int launch_gemv_seg(const oilhip_weights& w, const float* d_x, float* d_y, int M, hipStream_t s);
 // every format, a lane per run of 32 weights

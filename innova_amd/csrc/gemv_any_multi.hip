@@ -1,0 +1,662 @@
+// gemv_any_multi.hip -- decode GEMV for 3 to 16 activation rows per pass over tensors of other formats than plain OIL4
+// (Qwen35Engine::gemm with small B, src/adapters/tools/qwen35_engine.cpp:47-85, over dequantize_block_all,
+// src/block_codec.cpp:576-720): uniform SPARK_Q0, OIL2, OIL8 and grouped lattices, and the mixes of the planner (OIL1, SPARK_Q0) and
+// of the registry (OIL1_GRP, OIL2_GRP, OIL4_GRP, OIL8_GRP).
+//
+// The products run on v_mfma_f32_16x16x32_f16 and are exact: an activation is scaled by a power of two per (token, block) and cut
+// into three FP16 pieces (33 bits), which are three rows of the matrix instruction's A operand; a weight is an exact FP16 number
+// times a factor that its block, or its group of 64, shares:
+//   SPARK_Q0, OIL1, OIL1_GRP   the weight itself (+- an FP16 scale, an FP16 mean)
+//   OIL2, OIL2_GRP             10^4 times the level (15104, 4528)
+//   OIL4_GRP                   10^4 / 256 times the level as a sum of two (signed bytes a and b / 256 of 256 a + b)
+//   OIL8, OIL8_GRP             2 q - 255, q
+// Sums are FP32; the factor and the power of two meet a block's or group's sum.  The zero points of grouped formats are
+// one more matrix instruction (group sums of the activations, in three pieces, times the FP16 zero points).
+// A wavefront takes every n-th block of the row for a run of 16-row groups, keeps the activations of its block in registers, and
+// the wavefronts' sums meet in LDS once per run; every sum has a fixed order.  All but OIL8 are stored as
+// window streams; a block is found through its descriptor, two steps ahead.
+//
+// What bounds it: the activations' way into each compute unit (8 KB per block and five rows, about 30 bytes per clock), once per
+// workgroup, on wide rows; latency and the two launches on small tensors.  Tried: shares of K for several workgroups of a range
+// of rows, added by the last one, 10 to 20 % faster on the widest rows only and two to three times slower on others.
+// Before (window-stream kernel in passes of up to four rows, OIL8 kernel likewise) -> now, pre-pass included:
+//   16795 x 12032 SPARK_Q0, 15 rows 507 -> 53 us;  11008 x 4096 planner mix, 16 rows 73 -> 20 us;  11008 x 4096 OIL2, 8 rows 49 -> 19 us
+//   6613 x 8192, registry mix, 9 rows 103 -> 43 us;  4096 x 4096 OIL8, 32 rows 90 -> 28 us;  649 x 768 planner mix, 5 rows 12.3 -> 6.9 us
+#include <hip/hip_fp16.h>
+
+#include <algorithm>
+#include <type_traits>
+
+#include "common.h"
+#include "oil4_lds.h"
+
+namespace oilhip {
+namespace {
+
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned int u32x3 __attribute__((ext_vector_type(3)));
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kMaxWaves = 8;
+// tiles of 16 operand rows for M tokens of three pieces each
+constexpr int tiles_for(int M) { return (3 * M + 15) / 16; }
+constexpr int kMaxTiles = 3, kPassTokens = 16;
+
+// What the weights are: kOrderA formats have one factor per block at most, kOrderC formats one per group of 64 columns.
+// Operand columns: step s of a block, lane group kq, element e is column 64 kq + 8 s + e (A), or 64 (s / 2) + 16 kq + 8 (s % 2) + e (C).
+enum Source { kSpark = 0, kPlanner, kOil2, kOil8, kOil2Grp, kOil4Grp, kOil8Grp, kSparkMix };
+constexpr bool grouped(int S) { return S >= kOil2Grp; }
+constexpr bool by_descriptor(int S) { return S != kOil8; }                 // stored as window streams (common.h)
+constexpr int steps_of(int S) { return grouped(S) ? 9 : 8; }               // the ninth: group sums
+__host__ __device__ constexpr uint32_t tile_bytes(bool grp) { return (grp ? 9u : 8u) * 1024u; }
+
+// ---- pre-pass --------------------------------------------------------------------------------------------------------
+struct PackArgs {
+    const float* x;
+    uint8_t* xp;            // powers of two [block][16 NT] floats, then the operands [block][tile][step][lane][8 halves]
+    uint32_t ldx, bpr, tiles, grp, aligned;
+    int M;
+};
+
+__global__ void __launch_bounds__(256)
+pack_pieces_kernel(const PackArgs a) {
+    const uint32_t lane = threadIdx.x & 63u, blk = blockIdx.x % a.bpr, t = blockIdx.x / a.bpr * 4u + (threadIdx.x >> 6);
+    const uint32_t rows = 16u * a.tiles;
+    if (3u * t >= rows) return;
+    float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    if ((int)t < a.M) {
+        const float* p = a.x + (size_t)t * a.ldx + 256u * blk + 4u * lane;
+        if (a.aligned) { const float4 f = *reinterpret_cast<const float4*>(p); v[0] = f.x; v[1] = f.y; v[2] = f.z; v[3] = f.w; }
+        else { for (int e = 0; e < 4; ++e) v[e] = p[e]; }
+    }
+    // the largest magnitude as a bit pattern: infinities and NaN are the largest of all
+    uint32_t top = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) top = max(top, __float_as_uint(v[e]) & 0x7FFFFFFFu);
+    for (int o = 32; o > 0; o >>= 1) top = max(top, (uint32_t)__shfl_xor((int)top, o, 64));
+    const bool bad = top >= 0x7F800000u;
+    int ex = top == 0u || bad ? 0 : 14 - ((int)(top >> 23) - 127);         // to [2^14, 2^15)
+    ex = ex > 140 ? 140 : ex;
+    _Float16 h[3][4];
+    float sum = 0.0f;
+    auto cut = [](float f, _Float16& h0, _Float16& h1, _Float16& h2) {
+        h0 = (_Float16)f;
+        const float r = f - (float)h0;
+        h1 = (_Float16)r;
+        h2 = (_Float16)(r - (float)h1);
+    };
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const float f = bad ? 0.0f : ldexpf(v[e], ex);
+        sum += f;
+        cut(f, h[0][e], h[1][e], h[2][e]);
+    }
+    const float undo = bad ? __uint_as_float(0x7FC00000u) : ldexpf(1.0f, -ex);
+    uint32_t step, kq;
+    if (a.grp) { step = 2u * (lane >> 4) + ((lane & 3u) >> 1); kq = (lane & 15u) >> 2; }
+    else { step = (lane & 15u) >> 1; kq = lane >> 4; }
+    uint8_t* base = a.xp + a.bpr * rows * 4u + (size_t)blk * a.tiles * tile_bytes(a.grp);
+    sum += oil4::dpp_quad_xor1(sum);
+    sum += oil4::dpp_quad_xor2(sum);
+    sum += oil4::dpp_half_mirror(sum);
+    sum += oil4::dpp_row_mirror(sum);                                       // of the lane's group of 64 columns: below 2^21
+    _Float16 g[3];
+    cut(sum * 0x1p-6f, g[0], g[1], g[2]);
+#pragma unroll
+    for (uint32_t d = 0; d < 3u; ++d) {
+        const uint32_t r = 3u * t + d;
+        if (r >= rows) break;
+        uint8_t* tile = base + (r >> 4) * tile_bytes(a.grp);
+        const f16x2 lo = f16x2{h[d][0], h[d][1]}, hi = f16x2{h[d][2], h[d][3]};
+        *reinterpret_cast<uint2*>(tile + (step * 64u + kq * 16u + (r & 15u)) * 16u + (lane & 1u) * 8u) =
+            make_uint2(__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi));
+        if (a.grp && (lane & 15u) == 0u) {                                  // group lane / 16 at lane group lane / 16, element 0
+            const f16x2 s = f16x2{g[d], (_Float16)0.0f};
+            *reinterpret_cast<uint4*>(tile + (8u * 64u + (lane >> 4) * 16u + (r & 15u)) * 16u) = make_uint4(__builtin_bit_cast(uint32_t, s), 0u, 0u, 0u);
+        }
+        if (lane == 0) reinterpret_cast<float*>(a.xp)[blk * rows + r] = undo;
+    }
+}
+
+// ---- weights ---------------------------------------------------------------------------------------------------------
+__device__ __forceinline__ uint32_t pair16(uint32_t h) { return __builtin_amdgcn_perm(h, h, 0x01000100u); }   // the low half twice
+__device__ __forceinline__ uint32_t pk_add(uint32_t a, _Float16 b) {
+    const f16x2 r = __builtin_bit_cast(f16x2, a) + f16x2{b, b};
+    return __builtin_bit_cast(uint32_t, r);
+}
+__device__ __forceinline__ uint32_t pk_fma(uint32_t a, _Float16 b, _Float16 c) {
+    const f16x2 r = __builtin_elementwise_fma(__builtin_bit_cast(f16x2, a), f16x2{b, b}, f16x2{c, c});
+    return __builtin_bit_cast(uint32_t, r);
+}
+__device__ __forceinline__ f16x8 eight(uint32_t a, uint32_t b, uint32_t c, uint32_t d) { return __builtin_bit_cast(f16x8, u32x4{a, b, c, d}); }
+
+// bits 0..7 of b: set -> +scale, clear -> -scale; minus = the scale's halves with their signs flipped
+__device__ __forceinline__ f16x8 signs(uint32_t b, uint32_t minus) {
+    uint32_t t = b | (b << 15);                                             // bit 2 d at 2 d, bit 2 d + 1 at 2 d + 16
+    asm("" : "+v"(t));                                                     // shifts below, not 32-bit multiplications of b
+    return eight(((t << 15) & 0x80008000u) ^ minus, ((t << 13) & 0x80008000u) ^ minus, ((t << 11) & 0x80008000u) ^ minus,
+                 ((t << 9) & 0x80008000u) ^ minus);
+}
+// eight 2-bit codes -> 10^4 times their levels (-15104, -4528, 4528, 15104)
+__device__ __forceinline__ f16x8 levels2(uint32_t c) {
+    uint32_t d[4];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        uint32_t t = (c >> (8 * i)) & 0xFFu;
+        t |= t << 6;
+        t = (t | (t << 12)) & 0x03030303u;
+        const uint32_t hi = __builtin_amdgcn_perm(0u, 0x736CECF3u, t), lo = __builtin_amdgcn_perm(0u, 0x606C6C60u, t);
+        d[2 * i] = __builtin_amdgcn_perm(hi, lo, 0x05010400u);
+        d[2 * i + 1] = __builtin_amdgcn_perm(hi, lo, 0x07030602u);
+    }
+    return eight(d[0], d[1], d[2], d[3]);
+}
+// four bytes -> 1024 + byte as FP16, two per dword
+__device__ __forceinline__ void widen(uint32_t b, uint32_t& d0, uint32_t& d1) {
+    d0 = __builtin_amdgcn_perm(0x64646464u, b, 0x04010400u);
+    d1 = __builtin_amdgcn_perm(0x64646464u, b, 0x04030402u);
+}
+// eight bytes q -> 2 q - 255 (centred) or q
+template <bool CENTRED>
+__device__ __forceinline__ f16x8 bytes8(uint32_t b0, uint32_t b1) {
+    uint32_t d[4];
+    widen(b0, d[0], d[1]);
+    widen(b1, d[2], d[3]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        if constexpr (CENTRED) d[i] = pk_fma(pk_add(d[i], (_Float16)-1151.0f), (_Float16)2.0f, (_Float16)-1.0f);
+        else d[i] = pk_add(d[i], (_Float16)-1024.0f);
+    }
+    return eight(d[0], d[1], d[2], d[3]);
+}
+
+// bytes of a format's digit tables: magnitude m = 0..7 of 10^4 times the upper levels as 256 a + b
+constexpr int kLevelTimes1e4[8] = {1260, 3976, 6508, 9275, 12392, 15995, 20522, 27178};
+constexpr int low_digit(int n) { return (n & 255) > 127 ? (n & 255) - 256 : n & 255; }
+constexpr uint32_t digits(bool high, int first) {
+    uint32_t t = 0;
+    for (int i = 0; i < 4; ++i) {
+        const int n = kLevelTimes1e4[first + i], b = low_digit(n), a = (n - b) / 256;
+        t |= (uint32_t)((high ? a : b) & 255) << (8 * i);
+    }
+    return t;
+}
+// four 4-bit codes (low nibbles) -> digits a and b as signed bytes (no digit is 0 or -128, so the byte-wise negation carries nowhere)
+__device__ __forceinline__ void digits4(uint32_t w, uint32_t& a, uint32_t& b) {
+    const uint32_t m = __builtin_amdgcn_perm(0u, 0u, (~w & 0x08080808u) | 0x05050505u);   // 0xFF where the code is below 8
+    const uint32_t at = (w ^ m) & 0x07070707u, one = m & 0x01010101u;
+    a = (__builtin_amdgcn_perm(digits(true, 4), digits(true, 0), at) ^ m) + one;
+    b = (__builtin_amdgcn_perm(digits(false, 4), digits(false, 0), at) ^ m) + one;
+}
+// eight 4-bit codes of c -> the two summands
+__device__ __forceinline__ void levels4(uint32_t c, f16x8& va, f16x8& vb) {
+    uint32_t ae, be, ao, bo, d[8];
+    digits4(c, ae, be);                                                     // codes 0, 2, 4, 6
+    digits4(c >> 4, ao, bo);                                                // codes 1, 3, 5, 7
+    // bytes to code order, then to FP16: 1024 + (digit + 128)
+    const uint32_t a0 = __builtin_amdgcn_perm(ao, ae, 0x05010400u) ^ 0x80808080u, a1 = __builtin_amdgcn_perm(ao, ae, 0x07030602u) ^ 0x80808080u;
+    const uint32_t b0 = __builtin_amdgcn_perm(bo, be, 0x05010400u) ^ 0x80808080u, b1 = __builtin_amdgcn_perm(bo, be, 0x07030602u) ^ 0x80808080u;
+    widen(a0, d[0], d[1]);
+    widen(a1, d[2], d[3]);
+    widen(b0, d[4], d[5]);
+    widen(b1, d[6], d[7]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        d[i] = pk_add(d[i], (_Float16)-1152.0f);
+        d[4 + i] = pk_fma(d[4 + i], (_Float16)0x1p-8f, (_Float16)-4.5f);
+    }
+    va = eight(d[0], d[1], d[2], d[3]);
+    vb = eight(d[4], d[5], d[6], d[7]);
+}
+
+// dwords of a block that a lane holds
+constexpr int raw_dwords(int S) {
+    return S == kSpark || S == kPlanner ? 3 : S == kOil2 ? 6 : S == kOil8 ? 18 : S == kOil2Grp ? 5 : S == kOil4Grp ? 9 : 17;
+}
+__host__ __device__ constexpr uint32_t block_bytes(int S) { return S == kSpark ? 48u : S == kOil2 ? 64u : S == kOil8 ? 256u : S == kOil2Grp ? 80u : S == kOil4Grp ? 144u : 272u; }
+// row groups of a run: as many as registers and LDS take
+constexpr int run_groups(int S, int NT) { return NT == 3 && grouped(S) ? 1 : NT > 1 || raw_dwords(S) > 6 ? 2 : 4; }
+// blocks of activations that a wavefront holds
+constexpr int x_slots(int S, int NT) { return NT == 1 ? (grouped(S) || raw_dwords(S) > 9 ? 2 : 3) : 1; }
+
+struct BodyArgs {
+    const uint8_t* W;
+    const DevBlock* blocks;        // by_descriptor
+    const uint8_t* xp;
+    float* y;
+    uint32_t wbytes;               // size of the payload (by_descriptor)
+    uint32_t rows, bpr, ldy, parts, part_blocks, chunk, g_base, g_rem;
+    int M;
+};
+
+template <int S, int NT, int G>
+__global__ void __launch_bounds__(64 * kMaxWaves) __attribute__((amdgpu_waves_per_eu(2, 2)))
+gemv_any_multi_kernel(const BodyArgs a) {
+    constexpr int XD = x_slots(S, NT), ST = steps_of(S), N = raw_dwords(S), ROWS = 16 * NT;
+    extern __shared__ __align__(16) float red[];
+    const uint32_t wgid = blockIdx.x, g_begin = wgid * a.g_base + (wgid < a.g_rem ? wgid : a.g_rem), g_end = g_begin + a.g_base + (wgid < a.g_rem ? 1u : 0u);
+    const uint32_t lane = threadIdx.x & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), waves = blockDim.x >> 6;
+    const uint32_t li = lane & 15u, kq = lane >> 4, bpr = a.bpr;
+    const uint32_t iters = (a.part_blocks + waves - 1u) / waves;
+    const uint32_t stride = block_bytes(S), row_bytes = bpr * stride;
+    const uint32_t last = a.rows - 1u - 16u * g_begin, ngroups = g_end - g_begin;      // rows past the end repeat the last one
+    const auto wrs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(by_descriptor(S) ? a.W : a.W + (size_t)g_begin * 16u * row_bytes), (short)0,
+                                                       (int)(by_descriptor(S) ? a.wbytes : 0xFFFFFFFFu), 0x00020000);
+    const auto drs = __builtin_amdgcn_make_buffer_rsrc(const_cast<DevBlock*>(by_descriptor(S) ? a.blocks + (size_t)g_begin * 16u * bpr : nullptr), (short)0,
+                                                       (int)0xFFFFFFFFu, 0x00020000);
+    const float* undo = reinterpret_cast<const float*>(a.xp);
+    const uint8_t* xblocks = a.xp + bpr * ROWS * 4u;
+    auto place = [&](uint32_t part, uint32_t i) { const uint32_t b = wave + i * waves; return b < a.part_blocks ? part * a.part_blocks + b : 0xFFFFFFFFu; };
+    auto block_at = [&](uint32_t part, uint32_t i) { const uint32_t b = place(part, i); return b < bpr ? b : bpr - 1u; };
+
+    uint32_t w[G][N];
+    uint32_t fmt[G], dnext[G], fnext[G];                                   // by_descriptor: format of w; place and format of the step after
+    auto load_desc = [&](int g, uint32_t part, uint32_t run, uint32_t i) {
+        if constexpr (by_descriptor(S)) {
+            uint32_t r = (run + (uint32_t)g) * 16u + li;
+            r = r < last ? r : last;
+            const u32x4 d = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(drs, r * bpr * 16u, block_at(part, i) * 16u, 0));
+            dnext[g] = d.x * 16u;
+            fnext[g] = (d.w >> 16) & 0xFFu;
+        }
+    };
+    auto b32 = [&](uint32_t off, uint32_t so) { return (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(wrs, off, so, 0); };
+    auto load_w = [&](int g, uint32_t part, uint32_t run, uint32_t i) {
+        uint32_t (&o)[N] = w[g];
+        uint32_t r = (run + (uint32_t)g) * 16u + li;
+        r = r < last ? r : last;
+        const uint32_t off = by_descriptor(S) ? dnext[g] : r * row_bytes, so = by_descriptor(S) ? 0u : block_at(part, i) * stride;
+        if constexpr (by_descriptor(S)) fmt[g] = fnext[g];
+        auto group_loads = [&](auto bits) {
+            constexpr uint32_t B = decltype(bits)::value, GB = 4u + 8u * B, Q = B / 2u;
+            o[0] = b32(off + kq * GB, so);                                 // zero point and scale of group kq
+#pragma unroll
+            for (uint32_t j = 0; j < 4u; ++j) {
+                const uint32_t at = off + j * GB + 4u + 2u * B * kq;
+                if constexpr (B == 2u) o[1 + Q * j] = b32(at, so);
+                if constexpr (B == 4u) { const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(wrs, at, so, 0)); o[1 + Q * j] = v.x; o[2 + Q * j] = v.y; }
+                if constexpr (B == 8u) { const u32x4 v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wrs, at, so, 0)); o[1 + Q * j] = v.x; o[2 + Q * j] = v.y; o[3 + Q * j] = v.z; o[4 + Q * j] = v.w; }
+            }
+        };
+        if constexpr (S == kSpark || S == kPlanner) {                      // runs 2 kq and 2 kq + 1: 12 bytes, or (OIL1) 4
+            const uint32_t at = S == kPlanner && fmt[g] != 1u ? 4u : 12u;
+            const u32x3 v = __builtin_bit_cast(u32x3, __builtin_amdgcn_raw_buffer_load_b96(wrs, off + at * kq, so, 0));
+            o[0] = v.x; o[1] = v.y; o[2] = v.z;
+        } else if constexpr (S == kOil2) {                                 // 124 bits from bit 16 + 124 kq; the scale
+            const uint32_t at = off + ((16u + 124u * kq) >> 5) * 4u;
+            const u32x4 v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wrs, at, so, 0));
+            o[0] = v.x; o[1] = v.y; o[2] = v.z; o[3] = v.w;
+            o[4] = kq < 3u ? b32(at + 16u, so) : 0u;
+            o[5] = b32(off, so);
+        } else if constexpr (S == kOil8) {                                 // bytes 64 kq .. 64 kq + 67; the scale
+#pragma unroll
+            for (uint32_t j = 0; j < 4u; ++j) {
+                const u32x4 v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wrs, off + 64u * kq + 16u * j, so, 0));
+                o[4 * j] = v.x; o[4 * j + 1] = v.y; o[4 * j + 2] = v.z; o[4 * j + 3] = v.w;
+            }
+            o[16] = kq < 3u ? b32(off + 64u * kq + 64u, so) : 0u;
+            o[17] = b32(off, so);
+        } else if constexpr (S == kOil2Grp) {
+            group_loads(std::integral_constant<uint32_t, 2u>{});
+        } else if constexpr (S == kOil4Grp) {
+            group_loads(std::integral_constant<uint32_t, 4u>{});
+        } else if constexpr (S == kOil8Grp) {
+            group_loads(std::integral_constant<uint32_t, 8u>{});
+        } else {
+            // four 16-byte places of which a format fills what it has
+            auto b64 = [&](uint32_t at) { const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(wrs, at, so, 0)); return u32x4{v.x, v.y, 0u, 0u}; };
+            auto b128 = [&](uint32_t at) { return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wrs, at, so, 0)); };
+            u32x4 q0 = {0u, 0u, 0u, 0u}, q1 = q0, q2 = q0, q3 = q0;
+            const uint32_t f = fmt[g];
+            const uint32_t header = f == 7u ? 0u : (f == 9u ? 20u : f == 10u ? 36u : 68u) * kq;
+            const uint32_t hdr = b32(off + header, so);
+            if (f == 9u) {
+                const uint32_t at = off + 4u + 4u * kq;
+                q0.x = b32(at, so); q1.x = b32(at + 20u, so); q2.x = b32(at + 40u, so); q3.x = b32(at + 60u, so);
+            } else if (f == 7u) {                                          // all 32 bytes
+                q0 = b128(off); q1 = b128(off + 16u);
+            } else if (f == 10u) {
+                const uint32_t at = off + 4u + 8u * kq;
+                q0 = b64(at); q1 = b64(at + 36u); q2 = b64(at + 72u); q3 = b64(at + 108u);
+            } else {
+                const uint32_t at = off + 4u + 16u * kq;
+                q0 = b128(at); q1 = b128(at + 68u); q2 = b128(at + 136u); q3 = b128(at + 204u);
+            }
+            o[0] = hdr;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) { o[1 + k] = q0[k]; o[5 + k] = q1[k]; o[9 + k] = q2[k]; o[13 + k] = q3[k]; }
+        }
+    };
+    f16x8 x[XD][NT][ST];
+    f32x4 un[XD][NT];
+    auto load_part = [&](uint32_t part) {
+#pragma unroll
+        for (int s = 0; s < XD; ++s)
+            if (s == 0 || (uint32_t)s < iters) {
+                const uint32_t blk = block_at(part, (uint32_t)s);
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
+                    const f16x8* p = reinterpret_cast<const f16x8*>(xblocks + ((size_t)blk * NT + (uint32_t)t) * tile_bytes(grouped(S))) + lane;
+#pragma unroll
+                    for (int k = 0; k < ST; ++k) x[s][t][k] = p[64 * k];
+                    un[s][t] = *reinterpret_cast<const f32x4*>(undo + blk * ROWS + 16u * (uint32_t)t + 4u * kq);
+                }
+            }
+    };
+    float acc[G][NT][4];
+    // The sums of a chain of matrix instructions, before anything reads them.  With a branch right behind the last instruction of a
+    // chain the sums were seen to lack its products, although the instructions in between outlast its passes; so no branch follows
+    // one here, and every chain ends with independent cycles.
+    auto settle = [](f32x4& v) { asm volatile("s_nop 7" : "+v"(v)); };
+    // one block of 16 rows into acc[g]; spare: a wavefront that has a block less than the others
+    auto multiply = [&](int xs, int g, bool spare) {
+        const uint32_t (&o)[N] = w[g];
+        f32x4 sum[NT];
+        if constexpr (!grouped(S)) {
+            const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+            float factor = 1.0f;
+            uint32_t minus[2], bits[2], c[16];
+            if constexpr (S == kSpark || S == kPlanner) {
+                const bool spark = S == kSpark || fmt[g] == 1u;
+                minus[0] = pair16(o[0]) ^ 0x80008000u;
+                minus[1] = pair16((spark ? o[1] : o[0]) >> 16) ^ 0x80008000u;
+                bits[0] = spark ? __builtin_amdgcn_alignbit(o[1], o[0], 16) : 0xFFFFFFFFu;
+                bits[1] = spark ? o[2] : 0xFFFFFFFFu;
+            } else if constexpr (S == kOil2) {
+                factor = __half2float(__ushort_as_half((unsigned short)o[5])) * 1e-4f;
+                const uint32_t sh = 16u - 4u * kq;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) c[j] = __builtin_amdgcn_alignbit(o[j + 1], o[j], sh);
+            } else {
+                factor = __half2float(__ushort_as_half((unsigned short)o[17])) * (8.0f / 255.0f);
+                const uint32_t sh = kq < 2u ? 2u : 1u;
+#pragma unroll
+                for (int j = 0; j < 16; ++j) c[j] = __builtin_amdgcn_alignbyte(o[j + 1], o[j], sh);
+            }
+#pragma unroll
+            for (int s = 0; s < 8; ++s) {
+                f16x8 v;
+                if constexpr (S == kSpark || S == kPlanner) {
+                    v = signs((bits[s >> 2] >> (8 * (s & 3))) & 0xFFu, minus[s >> 2]);
+                } else if constexpr (S == kOil2) {                         // columns 31 and 63 of the lane are slots: 31 codes a run
+                    const int at = 62 * (s >> 2) + 16 * (s & 3);
+                    uint32_t q = at % 32 == 0 ? c[at / 32] : __builtin_amdgcn_alignbit(at / 32 + 1 < 4 ? c[at / 32 + 1] : 0u, c[at / 32], at % 32);
+                    v = levels2(q & 0xFFFFu);
+                    if ((s & 3) == 3) v[7] = (_Float16)0.0f;
+                } else {
+                    v = bytes8<true>(c[2 * s], c[2 * s + 1]);
+                    if (s == 7) v[7] = (kq & 1u) ? (_Float16)0.0f : v[7];  // columns 127 and 255 are slots
+                }
+#pragma unroll
+                for (int t = 0; t < NT; ++t) sum[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x[xs][t][s], v, s ? sum[t] : zero, 0, 0, 0);
+            }
+            factor = spare ? 0.0f : factor;
+#pragma unroll
+            for (int t = 0; t < NT; ++t) settle(sum[t]);
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[g][t][e] = fmaf(sum[t][e] * un[xs][t][e], factor, acc[g][t][e]);
+        } else {
+            // zero point (a 64th of it would do: the group sums are packed divided by 64) and scale of group kq, this lane's row
+            const bool own = S != kSparkMix || fmt[g] != 7u;
+            float zp = __half2float(__ushort_as_half((unsigned short)o[0])), sc = __half2float(__ushort_as_half((unsigned short)(o[0] >> 16)));
+            const float unit = S == kOil2Grp ? 1e-4f : S == kOil4Grp ? 256e-4f : S == kOil8Grp ? 1.0f / 255.0f
+                             : fmt[g] == 9u ? 1e-4f : fmt[g] == 10u ? 256e-4f : 1.0f / 255.0f;
+            sc = own ? sc * unit : 1.0f;
+            const uint32_t zbits = own ? o[0] & 0xFFFFu : 0u;
+            (void)zp;
+            const f16x8 zv = eight(zbits, 0u, 0u, 0u);
+            float factor[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) factor[j] = __int_as_float(__builtin_amdgcn_ds_bpermute((int)((li + 16u * (uint32_t)j) * 4u), __float_as_int(sc)));
+            const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                sum[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x[xs][t][8], zv, zero, 0, 0, 0);
+                settle(sum[t]);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) sum[t][e] *= 64.0f;
+            }
+            const uint32_t minus = S == kSparkMix ? pair16(o[1]) ^ 0x80008000u : 0u;      // OIL1_GRP: the scale
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                f32x4 part[NT];
+                f16x8 vs[2], vs2[2];                                       // both halves first: their decoding may branch
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    f16x8 v, v2 = eight(0u, 0u, 0u, 0u);
+                    if constexpr (S == kOil2Grp) {
+                        v = levels2((o[1 + j] >> (16 * h)) & 0xFFFFu);
+                    } else if constexpr (S == kOil4Grp) {
+                        levels4(o[1 + 2 * j + h], v, v2);
+                    } else if constexpr (S == kOil8Grp) {
+                        v = bytes8<false>(o[1 + 4 * j + 2 * h], o[2 + 4 * j + 2 * h]);
+                    } else {
+                        v = levels2((o[1 + 4 * j] >> (16 * h)) & 0xFFFFu);
+                        if (fmt[g] == 7u) {                                // 15 bits from 16 + 15 (4 j + kq)
+                            const int d = (16 + 60 * j) / 32, r = (16 + 60 * j) % 32;
+                            const uint64_t lo = o[1 + d] | (uint64_t)o[2 + d] << 32;
+                            const uint64_t win = (lo >> r) | (r ? (uint64_t)(d + 2 < 8 ? o[3 + d] : 0u) << (64 - r) : 0ull);
+                            const uint32_t b = (uint32_t)(win >> (15u * kq)) & 0x7FFFu;
+                            v = signs((b >> (8 * h)) & 0xFFu, minus);
+                            if (h == 1) v[7] = (_Float16)0.0f;
+                        } else if (fmt[g] == 10u) {
+                            levels4(o[1 + 4 * j + h], v, v2);
+                        } else if (fmt[g] == 11u) {
+                            v = bytes8<false>(o[1 + 4 * j + 2 * h], o[2 + 4 * j + 2 * h]);
+                        }
+                    }
+                    vs[h] = v;
+                    vs2[h] = v2;
+                }
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) {
+                        part[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x[xs][t][2 * j + h], vs[h], h ? part[t] : zero, 0, 0, 0);
+                        if constexpr (S == kOil4Grp || S == kSparkMix) part[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x[xs][t][2 * j + h], vs2[h], part[t], 0, 0, 0);
+                    }
+#pragma unroll
+                for (int t = 0; t < NT; ++t) settle(part[t]);
+#pragma unroll
+                for (int t = 0; t < NT; ++t)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) sum[t][e] = fmaf(part[t][e], factor[j], sum[t][e]);
+                __builtin_amdgcn_sched_barrier(0);                         // one group's weights in registers at a time
+            }
+            const float on = spare ? 0.0f : 1.0f;
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[g][t][e] = fmaf(sum[t][e] * on, un[xs][t][e], acc[g][t][e]);
+        }
+    };
+    auto lds_barrier = [&]() {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    };
+    constexpr uint32_t OUT = (uint32_t)(G * NT * 4) * 64u, AREA = (uint32_t)kMaxWaves * OUT;
+    float* keep = red + 2u * AREA;
+    if (waves < (uint32_t)kMaxWaves)
+        for (uint32_t o = waves * OUT + threadIdx.x; o < AREA; o += blockDim.x) { red[o] = 0.0f; red[AREA + o] = 0.0f; }
+    // outputs of a run: the eight wavefronts' sums of a token's three pieces
+    auto finish = [&](uint32_t part, uint32_t run, const float* area) {
+        for (uint32_t o = threadIdx.x; o < (uint32_t)(G * 16) * (uint32_t)a.M; o += blockDim.x) {
+            const uint32_t l = o & 15u, g = (o >> 4) % G, token = (o >> 4) / G;
+            float s = 0.0f;
+#pragma unroll
+            for (uint32_t d = 0; d < 3u; ++d) {
+                const uint32_t q = 3u * token + d;
+                const float* p = area + ((g * NT + (q >> 4)) * 4u + (q & 3u)) * 64u + ((q >> 2) & 3u) * 16u + l;
+                s += ((p[0] + p[OUT]) + (p[2u * OUT] + p[3u * OUT])) + ((p[4u * OUT] + p[5u * OUT]) + (p[6u * OUT] + p[7u * OUT]));
+            }
+            float* k = keep + ((run % a.chunk) / G) * (uint32_t)(G * 16 * kPassTokens) + o;
+            if (part) s += *k;
+            if (part + 1u < a.parts) { *k = s; continue; }
+            const uint32_t r = (g_begin + run + g) * 16u + l;
+            if (run + g < ngroups && r < a.rows) a.y[(size_t)token * a.ldy + r] = s;
+        }
+    };
+    // the step after (part, run, i)
+    uint32_t chunk_begin = 0, chunk_end = a.chunk < ngroups ? a.chunk : ngroups;
+    struct At { uint32_t part, run, i, cb, ce; };
+    auto after = [&](At p) {                                               // selects only: see settle
+        const bool turn = p.i + 1u >= iters, done = turn & (p.run + G >= p.ce), over = done & (p.part + 1u >= a.parts);
+        const uint32_t cb = over ? (p.ce < ngroups ? p.ce : 0u) : p.cb, far = cb + a.chunk < ngroups ? cb + a.chunk : ngroups;
+        return At{over ? 0u : done ? p.part + 1u : p.part, done ? cb : turn ? p.run + G : p.run, turn ? 0u : p.i + 1u, cb, over ? far : p.ce};
+    };
+    load_part(0u);
+    At here{0u, 0u, 0u, chunk_begin, chunk_end}, next = after(here), then = after(next);
+#pragma unroll
+    for (int g = 0; g < G; ++g) load_desc(g, 0u, 0u, 0u);
+#pragma unroll
+    for (int g = 0; g < G; ++g) { load_w(g, 0u, 0u, 0u); load_desc(g, next.part, next.run, next.i); }
+    uint32_t odd = 0, done_part = 0, done_run = 0xFFFFFFFFu;
+    for (; chunk_begin < ngroups; chunk_begin = chunk_end, chunk_end = chunk_end + a.chunk < ngroups ? chunk_end + a.chunk : ngroups)
+    for (uint32_t part = 0; part < a.parts; ++part) {
+        if (a.parts > 1u && (part || chunk_begin)) load_part(part);
+        for (uint32_t run = chunk_begin; run < chunk_end; run += G) {
+            if (done_run != 0xFFFFFFFFu) finish(done_part, done_run, red + (odd ^ 1u) * AREA);
+#pragma unroll
+            for (int g = 0; g < G; ++g)
+#pragma unroll
+                for (int t = 0; t < NT; ++t)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[g][t][e] = 0.0f;
+#pragma unroll
+            for (int i = 0; i < XD; ++i)
+                if (i == 0 || (uint32_t)i < iters) {
+                    const bool spare = place(part, (uint32_t)i) >= bpr;
+#pragma unroll
+                    for (int g = 0; g < G; ++g) {
+                        multiply(i, g, spare);
+                        load_w(g, next.part, next.run, next.i);
+                        load_desc(g, then.part, then.run, then.i);
+                    }
+                    next = then;
+                    then = after(then);
+                }
+            float* area = red + odd * AREA + wave * OUT;
+#pragma unroll
+            for (int g = 0; g < G; ++g)
+#pragma unroll
+                for (int t = 0; t < NT; ++t)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) area[(uint32_t)((g * NT + t) * 4 + e) * 64u + lane] = acc[g][t][e];
+            lds_barrier();
+            odd ^= 1u;
+            done_part = part; done_run = run;
+        }
+    }
+    finish(done_part, done_run, red + (odd ^ 1u) * AREA);
+}
+
+constexpr uint32_t kKeepGroups = 48;                                       // groups whose sums wait in LDS between parts: a multiple of every run length
+
+template <int S, int NT, int G>
+int launch_run(const BodyArgs& a, uint32_t wgs, uint32_t waves, hipStream_t s) {
+    const size_t lds = (size_t)2u * kMaxWaves * G * NT * 1024u + (a.parts > 1u ? (size_t)kKeepGroups * 16u * kPassTokens * 4u : 0u);
+    static std::atomic<uint64_t> raised{0};
+    auto kern = gemv_any_multi_kernel<S, NT, G>;
+    if (int rc = ensure_max_lds(raised, (const void*)kern, 160 * 1024)) return rc;
+    hipLaunchKernelGGL(kern, dim3(wgs), dim3(64u * waves), lds, s, a);
+    OILHIP_HIP(hipGetLastError());
+    return OILHIP_OK;
+}
+
+template <int S, int NT>
+int launch_one(BodyArgs a, hipStream_t s) {
+    constexpr int G = run_groups(S, NT), XD = x_slots(S, NT);
+    const uint32_t most = (uint32_t)(kMaxWaves * XD);
+    a.parts = (a.bpr + most - 1u) / most;
+    a.part_blocks = (a.bpr + a.parts - 1u) / a.parts;
+    a.parts = (a.bpr + a.part_blocks - 1u) / a.part_blocks;
+    const uint32_t each = (a.part_blocks + kMaxWaves - 1u) / kMaxWaves, waves = (a.part_blocks + each - 1u) / each;
+    a.chunk = a.parts > 1u ? kKeepGroups : 0x7FFFFFFFu;
+    const uint32_t groups = (a.rows + 15u) / 16u, slots = (uint32_t)device_cu_count() * std::max(1u, (uint32_t)kMaxWaves / waves);
+    const uint32_t wgs = std::min(groups, slots);
+    a.g_base = groups / wgs;
+    a.g_rem = groups % wgs;
+    // runs of one group while the chip has room for every group in a workgroup of its own
+    if (G == 1 || a.g_base + (a.g_rem ? 1u : 0u) == 1u) return launch_run<S, NT, 1>(a, wgs, waves, s);
+    return launch_run<S, NT, G>(a, wgs, waves, s);
+}
+
+template <int S>
+int launch_tiles(int tiles, const BodyArgs& a, hipStream_t s) {
+    return tiles == 1 ? launch_one<S, 1>(a, s) : tiles == 2 ? launch_one<S, 2>(a, s) : launch_one<S, 3>(a, s);
+}
+
+int source_of(const oilhip_weights& w) {
+    if (w.seg.nstreams && w.seg.nf > 0) {
+        uint32_t formats = 0;
+        for (uint32_t i = 0; i < w.seg.nf; ++i) {
+            if (w.seg.cb_bytes[i] != full_block_cb_bytes((int)w.seg.fmt[i]) || w.seg.cb_bytes[i] + w.seg.idx_bytes[i] != full_block_bytes((int)w.seg.fmt[i])) return -1;
+            formats |= 1u << w.seg.fmt[i];
+        }
+        if (w.alloc_bytes >= 0xFFFFFFF0ull) return -1;                     // 32-bit offsets
+        switch (formats) {
+            case 1u << OILHIP_SPARK_Q0: return kSpark;
+            case 1u << OILHIP_OIL2: return kOil2;
+            case 1u << OILHIP_OIL2_GRP: return kOil2Grp;
+            case 1u << OILHIP_OIL4_GRP: return kOil4Grp;
+            case 1u << OILHIP_OIL8_GRP: return kOil8Grp;
+        }
+        if ((formats & ~(1u << OILHIP_OIL1 | 1u << OILHIP_SPARK_Q0)) == 0) return kPlanner;
+        if ((formats & ~(1u << OILHIP_OIL1_GRP | 1u << OILHIP_OIL2_GRP | 1u << OILHIP_OIL4_GRP | 1u << OILHIP_OIL8_GRP)) == 0) return kSparkMix;
+        return -1;
+    }
+    return w.uniform_fmt == OILHIP_OIL8 && w.uniform_stride == 256u && w.uniform_cb == 0 && w.uniform_idx == 256u && (w.uniform_base & 3u) == 0 ? kOil8 : -1;
+}
+
+}  // namespace
+
+// Returns 1 when the tensor, the shape or the stream (one that is being captured and has no scratch yet) is outside what this
+// kernel covers, or another one is faster.
+int launch_gemv_any_multi(const oilhip_weights& w, const float* d_x, float* d_y, int M, hipStream_t s) {
+    const int src = source_of(w);
+    if (src < 0 || M < 2 || !w.all_full || (w.cols & 255u) || w.cols == 0 || w.cols > kGemvPackMaxCols || w.rows == 0 || w.rows > 0x7FFFFFFFull) return 1;
+    // The kernels of up to four rows per pass stay for two rows, and for three and four (window streams: while four rows of
+    // activations fit their LDS) on tensors of less than 12 M weights: 2000 x 2048, 3 rows 8.5 against 8.9 us; 4096 x 4096 14.2
+    // against 12.8 us.  The OIL8 kernel stays up to two passes on small tensors: 1000 x 1024, 6 rows 7.6 against 8.0 us.
+    const uint64_t weights = w.rows * w.cols;
+    if (M == 2 || (M <= 4 && weights < 12000000u && !(by_descriptor(src) && w.cols > 5120u))) return 1;
+    if (src == kOil8 && M <= 8 && weights < 2000000u) return 1;
+    const uint32_t bpr = (uint32_t)(w.cols >> 8);
+    // 32-bit byte offsets inside a workgroup's rows (blocks, or descriptors)
+    const uint64_t per_row = std::max<uint64_t>(16u, by_descriptor(src) ? 16u : block_bytes(src)) * bpr;
+    if ((w.rows / (16u * (uint64_t)device_cu_count()) + 8u) * 16u * per_row >= 0x80000000ull) return 1;
+    uint8_t* xp = nullptr;
+    if (!stream_scratch_ready(s, kScratchGemvPack, kGemvPackBytes)) return 1;
+    if (int rc = stream_scratch(s, kScratchGemvPack, kGemvPackBytes, reinterpret_cast<void**>(&xp))) return rc;
+    for (int m0 = 0; m0 < M; m0 += kPassTokens) {
+        const int m = std::min(M - m0, kPassTokens), tiles = tiles_for(m);
+        const float* x = d_x + (size_t)m0 * w.cols;
+        const PackArgs p{x, xp, (uint32_t)w.cols, bpr, (uint32_t)tiles, grouped(src) ? 1u : 0u, (reinterpret_cast<uintptr_t>(x) & 15u) == 0 ? 1u : 0u, m};
+        const uint32_t tokens = (16u * (uint32_t)tiles + 2u) / 3u;
+        hipLaunchKernelGGL(pack_pieces_kernel, dim3(bpr * ((tokens + 3u) / 4u)), dim3(256), 0, s, p);
+        OILHIP_HIP(hipGetLastError());
+        const BodyArgs a{w.d_payload + (by_descriptor(src) ? 0u : w.uniform_base), w.d_blocks, xp, d_y + (size_t)m0 * w.rows, (uint32_t)w.alloc_bytes,
+                         (uint32_t)w.rows, bpr, (uint32_t)w.rows, 0u, 0u, 0u, 0u, 0u, m};
+        int rc = 1;
+        switch (src) {
+            case kSpark: rc = launch_tiles<kSpark>(tiles, a, s); break;
+            case kPlanner: rc = launch_tiles<kPlanner>(tiles, a, s); break;
+            case kOil2: rc = launch_tiles<kOil2>(tiles, a, s); break;
+            case kOil8: rc = launch_tiles<kOil8>(tiles, a, s); break;
+            case kOil2Grp: rc = launch_tiles<kOil2Grp>(tiles, a, s); break;
+            case kOil4Grp: rc = launch_tiles<kOil4Grp>(tiles, a, s); break;
+            case kOil8Grp: rc = launch_tiles<kOil8Grp>(tiles, a, s); break;
+            case kSparkMix: rc = launch_tiles<kSparkMix>(tiles, a, s); break;
+        }
+        if (rc) return rc;
+    }
+    return OILHIP_OK;
+}
+
+}  // namespace oilhip

@@ -283,6 +283,41 @@ def test_oil4_multi_token_launch_shapes(bpr, rows, tokens):
                 assert rel_l2(got[:, r:r + n], want[:, :n]) <= TOL, (M, r)
 
 
+# Several rows through the other formats: operand tiles of 1 to 5, 6 to 10 and 11 to 16 rows, two passes beyond; rows of one block, of fewer
+# blocks than wavefronts, of several parts whose sums wait in LDS (one part holds 8 to 24 blocks); row groups around the lengths of a
+# run; uniform tensors and the two mixes whose blocks are found through their descriptors, which may also hold one of their formats
+# only in places.
+@pytest.mark.parametrize("fmt", [(1,), (2,), (4,), (9,), (10,), (11,), (0, 1), (7, 9, 10, 11), (7, 9)])
+@pytest.mark.parametrize("rows,cols,tokens", [(1, 256, (2, 16)), (17, 768, (3, 5, 6, 17)), (33, 4096, (2, 5, 10, 11, 16, 33)), (50, 7936, (4, 9, 13)),
+                                               (4096 + 40, 512, (2, 7, 12)), (3 * 4096 + 1, 2304, (3, 4, 5)), (100, 32768, (16,))])
+def test_other_formats_several_rows(fmt, rows, cols, tokens):
+    nb, period = rows * cols // 256, min(rows, 131)
+    ids = np.random.default_rng(nb).choice(fmt, period * cols // 256).astype(np.uint8)
+    payload, blocks = ia.block_codec.quantize_tensor(gaussian_weights(period * cols, rows, outlier_every=7), ids)
+    big = np.tile(blocks, -(-rows // period))[:nb]             # the rows repeat, their blocks share bytes
+    if len(fmt) == 1:                                          # uniform tensors: back to back
+        size = payload.size
+        shift = (np.arange(nb) // blocks.size * size).astype(np.uint64)
+        big["cb_off"] += shift
+        big["idx_off"] += shift
+        flat = np.tile(payload, -(-rows // period))
+    else:
+        flat = payload
+    rms = np.sqrt(np.mean(np.square(O.dequant_blocks(payload, to_orc_blocks(blocks)).astype(np.float64))))
+    with ia.DeviceWeights.from_blocks(flat, big, rows, cols) as dw:
+        for M in tokens:
+            X = np.random.default_rng(M).standard_normal((M, cols)).astype(np.float32) * np.logspace(-6, 6, M, dtype=np.float32)[:, None]
+            X[0, :7] = 0.0
+            want = O.block_gemm(payload, to_orc_blocks(blocks), period, cols, X, wide=True)
+            got = dw.gemv(torch.from_numpy(X).cuda()).cpu().numpy()
+            for m in range(M):
+                for r in range(0, rows, period):
+                    n = min(period, rows - r)
+                    size = np.linalg.norm(X[m].astype(np.float64)) * rms * np.sqrt(n)       # of outputs without cancellation
+                    err = np.linalg.norm(got[m, r:r + n].astype(np.float64) - want[m, :n])
+                    assert err <= TOL * max(np.linalg.norm(want[m, :n]), size), (M, m, r)
+
+
 def test_two_streams_run_multi_token_gemvs_concurrently():
     """Calls on different streams keep separate activation scratch: M = 16 GEMVs of two tensors issued back and forth
     on two streams, all in flight together, the first and last round checked against the oracle, one in between
