@@ -142,8 +142,8 @@ __device__ __forceinline__ float block_to_digits(float (&v)[4], float rms, uint3
               max((uint32_t)__builtin_amdgcn_readlane((int)top, 32), (uint32_t)__builtin_amdgcn_readlane((int)top, 48)));
     const bool bad = top >= 0x7F800000u;
     // the power of two that brings the largest magnitude to [2^22, 2^23), one less where its top digit would pass 127 (a
-    // mantissa above 8355711 / 2^22); subnormal magnitudes count as 2^-127
-    int ex = 22 - ((int)(top >> 23) - 127) - ((top & 0x7FFFFFu) > 0x7EFFFEu ? 1 : 0);
+    // mantissa above 8355711 / 2^22 = 1 + 0x7EFEFE / 2^23); subnormal magnitudes count as 2^-127
+    int ex = 22 - ((int)(top >> 23) - 127) - ((top & 0x7FFFFFu) > 0x7EFEFEu ? 1 : 0);
     ex = top == 0u || bad ? 0 : ex > 149 ? 149 : ex;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {

@@ -318,6 +318,22 @@ def test_other_formats_several_rows(fmt, rows, cols, tokens):
                     assert err <= TOL * max(np.linalg.norm(want[m, :n]), size), (M, m, r)
 
 
+# The digits of a block's largest magnitude: mantissas on both sides of the one above which the block takes a power of two less (its
+# top digit would not fit a signed byte), and the largest of all; both signs
+@pytest.mark.parametrize("M", [4, 16])
+def test_oil4_multi_token_largest_mantissas(M):
+    rows, mant = 40, np.array([0, 0x7EFEFD, 0x7EFEFE, 0x7EFEFF, 0x7EFF00, 0x7EFFFE, 0x7EFFFF, 0x7FFFFF], np.uint32)
+    cols = 256 * 2 * mant.size
+    payload, blocks = ia.block_codec.quantize_tensor(gaussian_weights(rows * cols, M), ia.Format.OIL4)
+    X = np.random.default_rng(M).standard_normal((M, cols)).astype(np.float32) * np.float32(0.3)
+    big = (mant | np.uint32(128 << 23)).view(np.float32)          # 2 to 4
+    X[:, 17:256 * mant.size:256] = big
+    X[:, 256 * mant.size + 200::256] = -big
+    want = O.block_gemm(payload, to_orc_blocks(blocks), rows, cols, X, wide=True)
+    with ia.DeviceWeights.from_blocks(payload, blocks, rows, cols) as dw:
+        assert rel_l2(dw.gemv(torch.from_numpy(X).cuda()).cpu().numpy(), want) <= TOL
+
+
 def test_two_streams_run_multi_token_gemvs_concurrently():
     """Calls on different streams keep separate activation scratch: M = 16 GEMVs of two tensors issued back and forth
     on two streams, all in flight together, the first and last round checked against the oracle, one in between
