@@ -201,9 +201,15 @@ static void pack_window_streams(std::vector<uint8_t>& pay, std::vector<DevBlock>
             return;
         }
     }
-    // streams: at most two per SIMD, and as many as give every stream the same number of rows (or one less): streams of
+    uint32_t widest = 0;
+    for (uint32_t i = 0; i < nf; ++i) widest = std::max(widest, g.stride[i]);
+    // Sixteen streams per CU for tensors of more than sixteen rows per CU, else eight: a stream with fewer than two rows fills
+    // too little of the decoding steps (4096 x 4096 of the planner's mix: 5.9 us with eight, 6.7 with sixteen; 11008 x 4096: 9.3 and 8.8),
+    // and of the stored floats' blocks (512 bytes and more) the smaller windows would hold three at most
+    const uint32_t cus = (uint32_t)device_cu_count(), waves = rows > (uint64_t)cus * 32 && widest < 512 ? 16u : 8u, window = waves == 16u ? kSegWindow / 2 : kSegWindow;
+    // streams: at most `waves` per CU, and as many as give every stream the same number of rows (or one less): streams of
     // five and six rows side by side would leave the fixed-size first windows a sixth empty
-    const uint64_t max_streams = (uint64_t)device_cu_count() * 8, rows_each = (rows + max_streams - 1) / max_streams;
+    const uint64_t max_streams = (uint64_t)cus * waves, rows_each = (rows + max_streams - 1) / max_streams;
     const uint32_t ns = (uint32_t)((rows + rows_each - 1) / rows_each);
     // a block's tag is its row of the tile and its column block: one byte while a row has at most 64 blocks
     const uint32_t tagw = bpr <= 64 ? 1u : 2u, tag_shift = bpr <= 64 ? 6u : 12u;
@@ -216,12 +222,10 @@ static void pack_window_streams(std::vector<uint8_t>& pay, std::vector<DevBlock>
     // nearly the same number of bytes, so the first windows (fetched blind, all at the size of the fullest) carry
     // little slack and the wavefronts finish together.  A stream's rows need not be neighbours.
     std::vector<uint32_t> row_bytes(rows, 0);
-    uint64_t widest = 0;
     for (uint64_t r = 0; r < rows; ++r)
         for (uint64_t c = 0; c < bpr; ++c) {
             const uint32_t st = g.stride[slot_of[db[r * bpr + c].fmt]];
             row_bytes[r] += st + tagw;
-            widest = std::max<uint64_t>(widest, st);
         }
     std::vector<uint32_t> order(rows);
     for (uint32_t r = 0; r < rows; ++r) order[r] = r;
@@ -256,7 +260,7 @@ static void pack_window_streams(std::vector<uint8_t>& pay, std::vector<DevBlock>
                         if (slot_of[db[b].fmt] != (int)s) continue;
                         Window* w = &ws.back();
                         // room for the block, its tag, its entry if a new one opens, and the row record of a closing entry
-                        if (bytes_of(w->rec + (open ? 0 : 1) + 2, w->tags.size() + 1, w->data + g.stride[s]) > kSegWindow) {
+                        if (bytes_of(w->rec + (open ? 0 : 1) + 2, w->tags.size() + 1, w->data + g.stride[s]) > window) {
                             ws.emplace_back();
                             w = &ws.back();
                             open = false;
@@ -331,6 +335,7 @@ static void pack_window_streams(std::vector<uint8_t>& pay, std::vector<DevBlock>
     pay.swap(out);
     g.nf = nf;
     g.nstreams = ns;
+    g.waves = waves;
     g.blind16 = (uint32_t)((first_used + 15) >> 4);
     g.stream_bytes = stride;
 }

@@ -50,8 +50,8 @@ enum ScratchSlot { kScratchGemvPack = 0, kScratchGemmX = 1, kScratchTl = 2, kScr
 int stream_scratch(hipStream_t s, int slot, size_t bytes, void** out);
 bool stream_scratch_ready(hipStream_t s, int slot, size_t bytes);   // false: this call would fail, the stream is being captured
 
-// Tensors whose rows mix formats are stored as `nstreams` streams of windows of at most 4 KB, one wavefront per stream
-// (gemv_seg.hip).  The first window of stream s sits at byte s * stream_bytes of the payload buffer, the later ones
+// Tensors whose rows mix formats are stored as `nstreams` streams of windows of at most 4 KB, made for one wavefront each,
+// `waves` (8, or 16 with windows of at most 2 KB) wavefronts per CU (gemv_seg.hip).  The first window of stream s sits at byte s * stream_bytes of the payload buffer, the later ones
 // behind all first windows, each found through its predecessor.  A stream covers a set of rows (chosen so that all
 // streams weigh about the same) in tiles of at most kSegTileRows; inside a tile the blocks are ordered by format (in the
 // order of `fmt`), inside a format by row and column.  Window: 2 dwords {8-byte units of records | 1 << 12 if another
@@ -65,7 +65,7 @@ constexpr int kSegMaxFormats = 15;
 constexpr uint32_t kSegWindow = 4096;
 constexpr int kSegTileRows = 4;
 struct SegLayout {
-    uint32_t nf = 0, nstreams = 0, blind16 = 0, tag_bytes = 2;
+    uint32_t nf = 0, nstreams = 0, waves = 8, blind16 = 0, tag_bytes = 2;
     uint64_t stream_bytes = 0;
     uint32_t fmt[kSegMaxFormats] = {}, cb_bytes[kSegMaxFormats] = {}, idx_bytes[kSegMaxFormats] = {}, stride[kSegMaxFormats] = {};
 };

@@ -625,7 +625,7 @@ int launch_gemv_any_multi(const oilhip_weights& w, const float* d_x, float* d_y,
     // activations fit their LDS) on tensors of less than 12 M weights: 2000 x 2048, 3 rows 8.5 against 8.9 us; 4096 x 4096 14.2
     // against 12.8 us.  The OIL8 kernel stays up to two passes on small tensors: 1000 x 1024, 6 rows 7.6 against 8.0 us.
     const uint64_t weights = w.rows * w.cols;
-    if (M == 2 || (M <= 4 && weights < 12000000u && !(by_descriptor(src) && w.cols > 5120u))) return 1;
+    if (M == 2 || (M <= 4 && w.seg.waves != 16 && weights < 12000000u && !(by_descriptor(src) && w.cols > 5120u))) return 1;
     if (src == kOil8 && M <= 8 && weights < 2000000u) return 1;
     const uint32_t bpr = (uint32_t)(w.cols >> 8);
     // 32-bit byte offsets inside a workgroup's rows (blocks, or descriptors)

@@ -25,7 +25,13 @@ namespace {
 
 constexpr int kRunPad = 36;                // floats per run of 32 activations in LDS: 16-byte reads of neighbouring lanes
                                            // fall into different banks
-constexpr int kWaves = 8;                  // wavefronts (streams) per workgroup
+// Wavefronts per workgroup, one workgroup per CU: 16 (four per SIMD, windows of at most 2 KB) for one or two activation rows
+// of a tensor that was packed for them, else 8 (two per SIMD, windows of at most 4 KB).  The decoding is bound by instruction
+// issue with waits on LDS in between (a step of 8 SPARK_Q0 blocks is 91 vector and 10 LDS instructions), so more wavefronts
+// side by side fill the waits: 11008 x 4096 at the registry's SPARK mix went from 15.7 to 13.1 us, at the planner's mix from 9.3 to
+// 8.8.  Three and four activation rows need more registers than four wavefronts per SIMD leave (128): there a workgroup has 8,
+// and each takes two streams, one after the other.
+constexpr uint32_t window_of(int waves) { return waves == 16 ? kSegWindow / 2 : kSegWindow; }
 constexpr int TR = kSegTileRows;           // accumulators per lane and activation row: a tile has at most this many rows
 typedef _Float16 h2v __attribute__((ext_vector_type(2)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
@@ -183,12 +189,14 @@ __device__ __forceinline__ void run_entry(const uint8_t* data, const uint8_t* ta
 // multiplies with siluf(h[k]) * h[cols + k] (the SwiGLU product of Qwen35Engine::mlp_step,
 // src/adapters/tools/qwen35_engine.cpp:611-621); 2 = x * (1 + xw[k]) is staged and every output is scaled by
 // 1 / sqrt(mean(x^2) + 1e-6), which each workgroup forms from the row it loads anyway (Qwen35Engine::rmsnorm, :39-44).
-template <int MB, int XF>
-__global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 2)))
+template <int MB, int XF, int kWaves>
+__global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kWaves / 4, kWaves / 4)))
 gemv_seg_kernel(const uint8_t* __restrict__ streams, const DecodeTables* __restrict__ T, const float* __restrict__ x,
                 const float* __restrict__ xw, float* __restrict__ y, uint32_t rows, uint32_t cols, int m0, int M,
                 const SegArgs A) {
     static_assert(XF == 0 || MB == 1, "the fused input transforms serve one activation row");
+    constexpr uint32_t WIN = window_of(kWaves);
+    constexpr int NW = WIN / 1024;                     // 16-byte pieces of a window per lane
     extern __shared__ __align__(16) float smem[];
     const uint32_t nruns = cols >> 5, xpad = nruns * kRunPad;
     float* ssq_part = smem + kLevelTabBytes / 4;       // XF = 2: sum(x^2) per wavefront
@@ -196,18 +204,18 @@ gemv_seg_kernel(const uint8_t* __restrict__ streams, const DecodeTables* __restr
     float* rs = xs + (size_t)MB * xpad;                // [MB][nruns] run sums
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = uniform(tid >> 6);
-    uint8_t* win = reinterpret_cast<uint8_t*>(rs + (size_t)MB * nruns) + (size_t)wave * 2u * kSegWindow;
+    uint8_t* win = reinterpret_cast<uint8_t*>(rs + (size_t)MB * nruns) + (size_t)wave * 2u * WIN;
     const LdsTables L{nullptr, nullptr, nullptr, nullptr};      // the formats that expand weight by weight here use no level table
 
-    const uint32_t sid = blockIdx.x * kWaves + wave;
+    uint32_t sid = blockIdx.x * kWaves + wave;
     const bool active = sid < A.nstreams;
     const uint8_t* sp = streams + (active ? (size_t)sid * A.stream_bytes : 0);
-    u32x4 wreg[4];                                     // a window in flight: 4 x 16 bytes per lane
+    u32x4 wreg[NW];                                    // a window in flight
     // the first window is fetched before anything is known about it: as many 16-byte pieces as the fullest first
     // window of the tensor has
     // (pieces past that size repeat the last one: every lane loads, unconditionally, so that nothing waits here)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < NW; ++j) {
         const uint32_t piece = j * 64u + lane < A.blind16 ? j * 64u + lane : A.blind16 - 1u;
         wreg[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(sp + (size_t)piece * 16u));
     }
@@ -265,12 +273,14 @@ gemv_seg_kernel(const uint8_t* __restrict__ streams, const DecodeTables* __restr
         if (lane == 63) ssq_part[wave] = v;
     }
 #pragma unroll
-    for (int j = 0; j < 4; ++j) *reinterpret_cast<u32x4*>(win + ((size_t)j * 64u + lane) * 16u) = wreg[j];
+    for (int j = 0; j < NW; ++j) *reinterpret_cast<u32x4*>(win + ((size_t)j * 64u + lane) * 16u) = wreg[j];
     __syncthreads();
     if (!active) return;
     float yscale = 1.0f;
     if constexpr (XF == 2) {
-        const float tot = ((ssq_part[0] + ssq_part[1]) + (ssq_part[2] + ssq_part[3])) + ((ssq_part[4] + ssq_part[5]) + (ssq_part[6] + ssq_part[7]));
+        float tot = 0.f;
+#pragma unroll
+        for (int j = 0; j < kWaves; j += 4) tot += (ssq_part[j] + ssq_part[j + 1]) + (ssq_part[j + 2] + ssq_part[j + 3]);
         yscale = 1.0f / sqrtf(tot / (float)cols + 1e-6f);
     }
 
@@ -280,15 +290,20 @@ gemv_seg_kernel(const uint8_t* __restrict__ streams, const DecodeTables* __restr
 #pragma unroll
         for (int j = 0; j < TR; ++j) acc[m][j] = 0.f;
     for (uint32_t wi = 0;; ++wi) {
-        const uint8_t* cur = win + (wi & 1u) * kSegWindow;
+        const uint8_t* cur = win + (wi & 1u) * WIN;
         const uint32_t* hdr = reinterpret_cast<const uint32_t*>(cur);
         const uint32_t h0 = uniform(hdr[0]);           // 8-byte units of records | another window follows << 12 | its 16-byte pieces << 16
-        const bool more = (h0 >> 12) & 1u;
-        if (more) {                                    // the next window: its size and place are in this one's header
-            const uint32_t used16 = h0 >> 16;
-            const uint8_t* np = streams + (size_t)uniform(hdr[1]) * 16u;
+        bool more = (h0 >> 12) & 1u;
+        uint32_t used16 = h0 >> 16;                    // the next window: its size and place are in this one's header, ...
+        const uint8_t* np = streams + (size_t)uniform(hdr[1]) * 16u;
+        if (MB > 1 && !more && (sid += gridDim.x * kWaves) < A.nstreams) {         // ... or it is the first one of this wavefront's next stream
+            more = true;
+            used16 = A.blind16;
+            np = streams + (size_t)sid * A.stream_bytes;
+        }
+        if (more) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
+            for (int j = 0; j < NW; ++j) {
                 const uint32_t piece = j * 64u + lane < used16 ? j * 64u + lane : used16 - 1u;
                 wreg[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(np + (size_t)piece * 16u));
             }
@@ -327,9 +342,9 @@ gemv_seg_kernel(const uint8_t* __restrict__ streams, const DecodeTables* __restr
             }
         }
         if (more) {
-            uint8_t* nxt = win + ((wi + 1u) & 1u) * kSegWindow;
+            uint8_t* nxt = win + ((wi + 1u) & 1u) * WIN;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) *reinterpret_cast<u32x4*>(nxt + ((size_t)j * 64u + lane) * 16u) = wreg[j];
+            for (int j = 0; j < NW; ++j) *reinterpret_cast<u32x4*>(nxt + ((size_t)j * 64u + lane) * 16u) = wreg[j];
             __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");       // other lanes read what this lane wrote
         } else {
             break;
@@ -338,15 +353,15 @@ gemv_seg_kernel(const uint8_t* __restrict__ streams, const DecodeTables* __restr
 }
 
 template <int MB>
-size_t seg_lds_bytes(const oilhip_weights& w) {
-    return kLevelTabBytes + 64 + (size_t)MB * ((w.cols >> 5) * (kRunPad + 1)) * 4 + (size_t)kWaves * 2 * kSegWindow;
+size_t seg_lds_bytes(const oilhip_weights& w) {        // the windows take 64 KB with 8 wavefronts and with 16
+    return kLevelTabBytes + 64 + (size_t)MB * ((w.cols >> 5) * (kRunPad + 1)) * 4 + 16 * (size_t)kSegWindow;
 }
 
-template <int MB, int XF = 0>
-int launch_seg(const oilhip_weights& w, const DecodeTables* T, const float* d_x, float* d_y, int m0, int M, hipStream_t s,
-               const float* d_xw = nullptr) {
+template <int MB, int XF, int kWaves>
+int launch_waves(const oilhip_weights& w, const DecodeTables* T, const float* d_x, float* d_y, int m0, int M, hipStream_t s,
+                 const float* d_xw) {
     static std::atomic<uint64_t> attr_done{0};
-    auto kern = gemv_seg_kernel<MB, XF>;
+    auto kern = gemv_seg_kernel<MB, XF, kWaves>;
     const SegLayout& g = w.seg;
     const size_t lds = seg_lds_bytes<MB>(w);
     if (lds > 160 * 1024) return 1;
@@ -354,10 +369,19 @@ int launch_seg(const oilhip_weights& w, const DecodeTables* T, const float* d_x,
     SegArgs A{};
     A.nstreams = g.nstreams; A.blind16 = g.blind16; A.tag_bytes = g.tag_bytes; A.stream_bytes = g.stream_bytes;
     for (uint32_t i = 0; i < g.nf; ++i) { A.cb_bytes[i] = g.cb_bytes[i]; A.idx_bytes[i] = g.idx_bytes[i]; A.stride[i] = g.stride[i]; }
-    hipLaunchKernelGGL(kern, dim3((g.nstreams + kWaves - 1) / kWaves), dim3(64 * kWaves), lds, s, w.d_payload, T, d_x, d_xw,
+    const uint32_t per = (g.waves + kWaves - 1) / kWaves;              // streams per wavefront
+    hipLaunchKernelGGL(kern, dim3((g.nstreams + kWaves * per - 1) / (kWaves * per)), dim3(64 * kWaves), lds, s, w.d_payload, T, d_x, d_xw,
                        d_y, (uint32_t)w.rows, (uint32_t)w.cols, m0, M, A);
     OILHIP_HIP(hipGetLastError());
     return OILHIP_OK;
+}
+
+template <int MB, int XF = 0>
+int launch_seg(const oilhip_weights& w, const DecodeTables* T, const float* d_x, float* d_y, int m0, int M, hipStream_t s,
+               const float* d_xw = nullptr) {
+    if constexpr (MB <= 2)
+        if (w.seg.waves == 16) return launch_waves<MB, XF, 16>(w, T, d_x, d_y, m0, M, s, d_xw);
+    return launch_waves<MB, XF, 8>(w, T, d_x, d_y, m0, M, s, d_xw);
 }
 
 }  // namespace

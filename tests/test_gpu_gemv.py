@@ -85,6 +85,18 @@ def test_mixed_format_tiles(fmt_ids, rows, cols, M):
     assert np.array_equal(got.view(np.uint32).ravel(), ref.view(np.uint32).ravel())
 
 
+# tensors of more than 32 rows per CU are packed in smaller windows, for sixteen wavefronts per CU: either side of that
+# line, streams of unequal row counts, and formats whose blocks are too large for it
+@pytest.mark.parametrize("fmt_ids", [(0, 1), (6, 9, 11, 7), (0, 13, 14)])
+@pytest.mark.parametrize("rows,cols", [(8192, 256), (8193, 512), (12305, 768)])
+@pytest.mark.parametrize("M", [1, 2, 3])
+def test_mixed_format_tall(fmt_ids, rows, cols, M):
+    rng = np.random.default_rng(rows + cols + M)
+    fmts = rng.choice(np.array(fmt_ids, dtype=np.uint8), size=rows * cols // 256)
+    err, *_ = run_case(fmts, rows, cols, M=M, seed=rows)
+    assert err <= TOL
+
+
 def test_mixed_format_skewed_tiles():
     """Tiles in which a format is absent, or holds a single block, or fills every block."""
     rows, cols = 24, 2048
