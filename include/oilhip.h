@@ -306,7 +306,7 @@ int oilhip_dense_map_f32(int op, const float* d_a, const float* d_b, float s, fl
  * oilhip_gemv_rmsnorm_f32   : y[M][rows] = W . rmsnorm(x; normw), the rmsnorm + gemm pair in front of every projection
  *                             (:484-486 attention input, :611-614 MLP input).  With M = 1 and an OIL4 or window-stream
  *                             tensor the norm is formed while the GEMV stages x (one launch, d_xn unused and may be NULL);
- *                             otherwise d_xn[M][cols] receives the normalised rows and the GEMV reads them.
+ *                             otherwise d_xn[M][cols] receives the normalised rows, whichever launch forms them.
  * oilhip_mlp_step_f32       : Qwen35Engine::mlp_step (:611-621): y[M][D] = down(siluf(gate x) * up x), gate_up = the
  *                             gate and up projections stacked (2F x D, gate rows first), down = D x F.  A non-NULL
  *                             d_normw applies rmsnorm(x; d_normw) first, as the caller of mlp_step does.

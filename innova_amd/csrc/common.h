@@ -124,6 +124,7 @@ struct MultiInput {
     const float* x2 = nullptr;      // same layout as x
     const float* norm_w = nullptr;  // cols floats
     bool inv_form = false;          // silu as x * (1 / (1 + exp(-x))) instead of x / (1 + exp(-x))
+    float* xn = nullptr;            // with norm_w: receives the normalised rows, same layout as x, no overlap with it
 };
 int launch_gemv_oil4_multi(const oilhip_weights& w, const float* d_x, const int* d_tok, float* d_y, int M, uint32_t ldx, uint32_t ldy,
                            uint32_t xrows, hipStream_t s, const MultiInput& in = {}, const oilhip_weights* w2 = nullptr, float* d_y2 = nullptr,

@@ -83,6 +83,7 @@ __host__ __device__ constexpr uint32_t undo_bytes(uint32_t bpr) { return bpr * (
 // undone on the sums).
 struct Activations {
     const float *x, *x2, *norm_w;
+    float* xn;                  // with norm_w: the normalised rows go here as well (optional, laid out like x)
     uint32_t ldx, aligned, inv_form;
 };
 
@@ -122,6 +123,10 @@ __device__ __forceinline__ void load_activations(const Activations& a, uint32_t 
         for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
         rms = 1.0f / sqrtf(s / (float)(256u * bpr) + 1e-6f);
         for (int e = 0; e < 4; ++e) v[e] *= 1.0f + a.norm_w[256u * blk + 4u * lane + e];
+        if (a.xn) {
+            float* o = a.xn + (size_t)src * a.ldx + 256u * blk + 4u * lane;
+            for (int e = 0; e < 4; ++e) o[e] = v[e] * rms;
+        }
     }
 }
 
@@ -578,7 +583,7 @@ int launch_gemv_oil4_multi(const oilhip_weights& w, const float* d_x, const int*
     for (int m0 = 0; m0 < M; m0 += kMaxTokens) {
         const int m = std::min(M - m0, kMaxTokens), kind = kind_of(m);
         const size_t skip = d_tok ? 0 : (size_t)m0 * ldx;
-        const Activations act{d_x + skip, in.x2 ? in.x2 + skip : nullptr, in.norm_w, ldx, aligned, in.inv_form ? 1u : 0u};
+        const Activations act{d_x + skip, in.x2 ? in.x2 + skip : nullptr, in.norm_w, in.xn ? in.xn + skip : nullptr, ldx, aligned, in.inv_form ? 1u : 0u};
         hipLaunchKernelGGL(pack_digits_kernel, dim3(bpr * kind_tokens(kind) / 4u), dim3(256), 0, s,
                            PackArgs{act, d_tok ? d_tok + m0 : nullptr, xp, bpr, d_tok ? xrows : xrows - (uint32_t)m0, m, kind}, PackJobs{});
         OILHIP_HIP(hipGetLastError());
@@ -655,7 +660,7 @@ int launch_gemv_oil4_multi_batches(int nb, const oilhip_weights* const* wa, floa
             mj.wg_begin[j + 1] = mj.wg_begin[j] + wgs;
         }
     const uint32_t aligned = ((reinterpret_cast<uintptr_t>(d_x) | reinterpret_cast<uintptr_t>(d_x2)) & 15u) == 0 && (ldx & 3u) == 0;
-    const PackArgs a{{d_x, d_x2, nullptr, ldx, aligned, 0u}, nullptr, static_cast<uint8_t*>(d_ws), bpr, xrows, 0, 0};
+    const PackArgs a{{d_x, d_x2, nullptr, nullptr, ldx, aligned, 0u}, nullptr, static_cast<uint8_t*>(d_ws), bpr, xrows, 0, 0};
     hipLaunchKernelGGL(pack_digits_kernel, dim3(pj.begin[nb]), dim3(256), 0, s, a, pj);
     OILHIP_HIP(hipGetLastError());
     static std::atomic<uint64_t> raised{0};

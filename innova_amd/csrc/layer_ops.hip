@@ -116,9 +116,11 @@ int oilhip_gemv_rmsnorm_f32(const oilhip_weights* w, const float* d_x, const flo
         if (rc <= 0) return rc;
     }
     if (!d_xn) return fail(OILHIP_E_ARG, "gemv_rmsnorm: this shape needs the d_xn workspace");
-    if (M > 1 && plain_oil4(*w) && w->cols <= kPackNormMaxCols) {          // the norm rides on the packing of the activations
+    const uintptr_t x0 = reinterpret_cast<uintptr_t>(d_x), xn0 = reinterpret_cast<uintptr_t>(d_xn), size = (uintptr_t)M * w->cols * 4u;
+    const bool apart = x0 + size <= xn0 || xn0 + size <= x0;               // packing wavefronts read whole rows while others store theirs
+    if (M > 1 && plain_oil4(*w) && w->cols <= kPackNormMaxCols && apart) { // the norm rides on the packing of the activations
         const int rc = launch_gemv_oil4_multi(*w, d_x, nullptr, d_y, M, (uint32_t)w->cols, (uint32_t)w->rows, (uint32_t)M, (hipStream_t)stream,
-                                              MultiInput{nullptr, d_normw, false});
+                                              MultiInput{nullptr, d_normw, false, d_xn});
         if (rc <= 0) return rc;
     }
     if (int rc = oilhip_rmsnorm_f32(d_x, d_normw, (int)w->cols, M, d_xn, stream)) return rc;

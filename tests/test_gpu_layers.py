@@ -134,6 +134,31 @@ def test_norm_and_swiglu_of_several_rows(M, D, F):
     down.close()
 
 
+# the normalised rows themselves, which a C caller may feed to its own projections: every path that serves more than one row, up to and
+# beyond the width at which the norm is formed while the activations are packed, passes of 32 rows, rows at a misaligned address, and
+# rows normalised in place
+@pytest.mark.parametrize("fmt", [ia.Format.OIL4, (0, 1)])
+@pytest.mark.parametrize("M,cols,where", [(2, 256, "apart"), (5, 2816, "apart"), (33, 768, "apart"), (3, 8448, "apart"), (4, 1024, "odd"), (3, 1024, "in place")])
+def test_gemv_rmsnorm_returns_the_normalised_rows(fmt, M, cols, where):
+    rows, rng = 200, np.random.default_rng(M + cols)
+    payload, blocks = ia.block_codec.quantize_tensor(gaussian_weights(rows * cols, 3), block_formats(fmt, rows * cols // 256, cols))
+    x = (rng.standard_normal((M, cols)) * np.logspace(-2, 2, M)[:, None]).astype(np.float32)
+    nw = (rng.standard_normal(cols) * 0.2).astype(np.float32)
+    xd, nd, y = torch.from_numpy(x).cuda(), torch.from_numpy(nw).cuda(), torch.empty(M, rows, device="cuda")
+    buf = torch.full((M * cols + 1,), float("nan"), device="cuda")
+    xn = xd if where == "in place" else buf[where == "odd":][:M * cols].view(M, cols)
+    with ia.DeviceWeights.from_blocks(payload, blocks, rows, cols) as dw:
+        ia._lib.check(ia._lib.lib().oilhip_gemv_rmsnorm_f32(dw.handle, xd.data_ptr(), nd.data_ptr(), y.data_ptr(), M, xn.data_ptr(),
+                                                            ia._lib.current_stream()))
+        got, y = xn.cpu().numpy(), y.cpu().numpy()
+    x64 = x.astype(np.float64)
+    closed = x64 / np.sqrt((x64 ** 2).mean(1, keepdims=True) + 1e-6) * (1.0 + nw.astype(np.float64))
+    want = O.block_gemm(payload, to_orc_blocks(blocks), rows, cols, closed.astype(np.float32), wide=True)
+    for m in range(M):
+        assert rel_l2(got[m], closed[m]) <= 1e-6, m
+        assert rel_l2(y[m], want[m]) <= TOL, m
+
+
 def test_embed_rows():
     vocab, cols = 40, 1024
     w = gaussian_weights(vocab * cols, 5)
