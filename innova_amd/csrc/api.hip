@@ -83,7 +83,15 @@ struct ScratchBuffers {
 };
 static std::map<std::tuple<int, void*, int>, ScratchBuffers> g_scratch;
 
-int stream_scratch(hipStream_t s, int slot, size_t bytes, void** out) {
+// A fixed set of locks, so that none has to outlive its stream: streams that share one wait for each other's launches to be
+// queued.  No call takes two of them.
+std::mutex& stream_mutex(hipStream_t s) {
+    static std::mutex locks[64];
+    return locks[(reinterpret_cast<uintptr_t>(s) * 0x9E3779B97F4A7C15ull) >> 58];
+}
+
+int stream_scratch(const StreamLock& lock, int slot, size_t bytes, void** out) {
+    const hipStream_t s = lock.stream;
     int dev = 0;
     OILHIP_HIP(hipGetDevice(&dev));
     std::lock_guard<std::mutex> lk(g_scratch_mu);
@@ -626,6 +634,7 @@ int oilhip_gemm_f32(const oilhip_weights* w, const float* d_x, float* d_y, int M
 int oilhip_release_stream_scratch(void* stream) {
     int dev = 0;
     OILHIP_HIP(hipGetDevice(&dev));
+    const StreamLock lock((hipStream_t)stream);
     OILHIP_HIP(hipStreamSynchronize((hipStream_t)stream));
     std::lock_guard<std::mutex> lk(g_scratch_mu);
     for (auto it = g_scratch.begin(); it != g_scratch.end();) {

@@ -4,6 +4,7 @@
 #include <stdint.h>
 
 #include <atomic>
+#include <mutex>
 #include <string>
 
 #include "../../include/oilhip.h"
@@ -46,8 +47,19 @@ int ensure_max_lds(std::atomic<uint64_t>& done, const void* kernel, int bytes);
 // one and the old one stays allocated.  No allocation can happen while the stream is being captured, so the first
 // call of a given size on a stream has to be made outside capture; otherwise the call fails with OILHIP_E_ARG.
 // New buffers are zero-filled.
+// One call's launches write and read the scratch one after the other; a second thread's launches on the same stream must
+// not come between them.  So the scratch is asked for under the stream's lock, which the caller holds until the last launch
+// that uses it is queued.
 enum ScratchSlot { kScratchGemvPack = 0, kScratchGemmX = 1, kScratchTl = 2, kScratchGemmW = 3, kScratchGemmP = 4 };
-int stream_scratch(hipStream_t s, int slot, size_t bytes, void** out);
+std::mutex& stream_mutex(hipStream_t s);
+class StreamLock {
+public:
+    explicit StreamLock(hipStream_t s) : stream(s), held_(stream_mutex(s)) {}
+    const hipStream_t stream;
+private:
+    std::lock_guard<std::mutex> held_;
+};
+int stream_scratch(const StreamLock& lock, int slot, size_t bytes, void** out);
 bool stream_scratch_ready(hipStream_t s, int slot, size_t bytes);   // false: this call would fail, the stream is being captured
 
 // Tensors whose rows mix formats are stored as `nstreams` streams of windows of at most 4 KB, made for one wavefront each,

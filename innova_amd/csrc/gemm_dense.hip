@@ -214,10 +214,11 @@ int launch_gemm_any(const oilhip_weights& w, const void* d_x, bool x_is_f32, flo
     // slab: at most 128 MB of bf16, a multiple of 256 rows
     const uint32_t slab = (uint32_t)std::min<uint64_t>((N + 255u) & ~255u, std::max<uint64_t>(256, ((128ull << 20) / ((uint64_t)K * 2u)) & ~255ull));
     if ((uint64_t)K * 512u >= 0x80000000ull) return fail(OILHIP_E_ARG, "rows too wide for the prefill kernel");
+    const StreamLock lock(s);
     uint16_t *wf = nullptr, *xf = nullptr;
-    if (int rc = stream_scratch(s, kScratchGemmW, (size_t)slab * K * 2, reinterpret_cast<void**>(&wf))) return rc;
+    if (int rc = stream_scratch(lock, kScratchGemmW, (size_t)slab * K * 2, reinterpret_cast<void**>(&wf))) return rc;
     const uint32_t mpad = (M + 255u) & ~255u;
-    if (int rc = stream_scratch(s, kScratchGemmX, (size_t)mpad * K * 2, reinterpret_cast<void**>(&xf))) return rc;
+    if (int rc = stream_scratch(lock, kScratchGemmX, (size_t)mpad * K * 2, reinterpret_cast<void**>(&xf))) return rc;
     for (uint32_t n0 = 0; n0 < N; n0 += slab) {
         const uint32_t nc = std::min(slab, N - n0);
         const DensePlan pl = dense_plan(M, nc, K);
@@ -226,7 +227,7 @@ int launch_gemm_any(const oilhip_weights& w, const void* d_x, bool x_is_f32, flo
         if (a.parts > 1u) {
             void* p = nullptr;
             const size_t counters = ((size_t)a.MT * a.NT * 4u + 255u) & ~(size_t)255u;
-            if (int rc = stream_scratch(s, kScratchGemmP, counters + (size_t)a.MT * a.NT * a.parts * t * t * 4u, &p)) return rc;
+            if (int rc = stream_scratch(lock, kScratchGemmP, counters + (size_t)a.MT * a.NT * a.parts * t * t * 4u, &p)) return rc;
             a.arrived = static_cast<uint32_t*>(p);
             a.partial = reinterpret_cast<float*>(static_cast<uint8_t*>(p) + counters);
         }

@@ -454,8 +454,9 @@ int launch_frag(const oilhip_weights& w, const void* d_x, float* d_y, uint32_t M
     gr.halves = split && FN == 4 ? 2u : 1u;
     gr.ksplit = split && FN != 4 ? 2u : 1u;
     const uint32_t Mpad = gr.MT * TM;
+    const StreamLock lock(s);
     uint16_t* xf = nullptr;
-    if (int rc = stream_scratch(s, kScratchGemmX, (size_t)Mpad * K * 2, reinterpret_cast<void**>(&xf))) return rc;
+    if (int rc = stream_scratch(lock, kScratchGemmX, (size_t)Mpad * K * 2, reinterpret_cast<void**>(&xf))) return rc;
     const uint32_t npack = (Mpad / 32u) * (K >> 8), nzero = gr.ksplit > 1u ? tiles - gr.nfull : 0u;
     hipLaunchKernelGGL((pack_x_frag_kernel<F32, TM, TN>), dim3(npack + nzero), dim3(256), 0, s, d_x, xf, M, K, npack, d_y, N, N, gr);
     OILHIP_HIP(hipGetLastError());

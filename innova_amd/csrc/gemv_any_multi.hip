@@ -631,9 +631,10 @@ int launch_gemv_any_multi(const oilhip_weights& w, const float* d_x, float* d_y,
     // 32-bit byte offsets inside a workgroup's rows (blocks, or descriptors)
     const uint64_t per_row = std::max<uint64_t>(16u, by_descriptor(src) ? 16u : block_bytes(src)) * bpr;
     if ((w.rows / (16u * (uint64_t)device_cu_count()) + 8u) * 16u * per_row >= 0x80000000ull) return 1;
+    const StreamLock lock(s);
     uint8_t* xp = nullptr;
     if (!stream_scratch_ready(s, kScratchGemvPack, kGemvPackBytes)) return 1;
-    if (int rc = stream_scratch(s, kScratchGemvPack, kGemvPackBytes, reinterpret_cast<void**>(&xp))) return rc;
+    if (int rc = stream_scratch(lock, kScratchGemvPack, kGemvPackBytes, reinterpret_cast<void**>(&xp))) return rc;
     for (int m0 = 0; m0 < M; m0 += kPassTokens) {
         const int m = std::min(M - m0, kPassTokens), tiles = tiles_for(m);
         const float* x = d_x + (size_t)m0 * w.cols;

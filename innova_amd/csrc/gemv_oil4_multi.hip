@@ -574,10 +574,11 @@ int launch_gemv_oil4_multi(const oilhip_weights& w, const float* d_x, const int*
     if (!shape_covered(w, xrows, ldx)) return 1;
     if (w2 && (w2->cols != w.cols || !shape_covered(*w2, xrows, ldx) || !plain_oil4(*w2) || !d_y2)) return 1;
     const uint32_t bpr = (uint32_t)(w.cols >> 8);
+    const StreamLock lock(s);
     uint8_t* xp = d_pack;
     if (!xp)
         // a stream's scratch comes in two sizes: one pass, and from rows of more than 4096 weights on the static scratch's
-        if (int rc = stream_scratch(s, kScratchGemvPack, bpr > 16u ? kStaticScratchBytes : kGemvPackBytes, reinterpret_cast<void**>(&xp))) return rc;
+        if (int rc = stream_scratch(lock, kScratchGemvPack, bpr > 16u ? kStaticScratchBytes : kGemvPackBytes, reinterpret_cast<void**>(&xp))) return rc;
     const uintptr_t at = reinterpret_cast<uintptr_t>(d_x) | reinterpret_cast<uintptr_t>(in.x2);
     const uint32_t aligned = (at & 15u) == 0 && (ldx & 3u) == 0;
     for (int m0 = 0; m0 < M; m0 += kMaxTokens) {

@@ -76,8 +76,9 @@ extern "C" int oilhip_tl_gemm(int kind, const uint8_t* d_w, const float* d_act, 
     if (!d_out || (K > 0 && (!d_w || !d_act))) return fail(OILHIP_E_ARG, "tl_gemm: null pointer");
     auto s = static_cast<hipStream_t>(stream);
     const size_t qbytes = ((size_t)N * (size_t)K + 255) & ~(size_t)255;
+    const StreamLock lock(s);
     void* ws = nullptr;
-    if (int rc = stream_scratch(s, kScratchTl, qbytes + sizeof(float) * (size_t)N, &ws)) return rc;
+    if (int rc = stream_scratch(lock, kScratchTl, qbytes + sizeof(float) * (size_t)N, &ws)) return rc;
     int8_t* q = static_cast<int8_t*>(ws);
     float* scales = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + qbytes);
     hipLaunchKernelGGL(tl_quantize_kernel, dim3((unsigned)N), dim3(256), 0, s, d_act, K, q, scales);

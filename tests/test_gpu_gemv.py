@@ -4,6 +4,7 @@ Tolerance (north star): relative L2 error <= 1e-5 against the double-precision
 dot of the bit-exact decoded weights.  The reference's own FP32 summation order
 is measured against the same yardstick for comparison."""
 import os
+import threading
 
 import numpy as np
 import pytest
@@ -380,6 +381,36 @@ def test_two_streams_run_multi_token_gemvs_concurrently():
         assert np.array_equal(mid, again.cpu().numpy()), i
     for h in handles:
         h.close()
+
+
+# Packing and product share a scratch of the stream: two threads that call on one stream must not get between each other's launches.
+# Every output of both threads equals, bit for bit, what a quiet call returns.
+@pytest.mark.parametrize("fmt,M", [(ia.Format.OIL4, 5), (ia.Format.SPARK_Q0, 5), (ia.Format.OIL8, 9)])
+def test_two_threads_on_one_stream(fmt, M):
+    rows, cols, calls = 256, 2048, 400
+    payload, blocks = ia.block_codec.quantize_tensor(gaussian_weights(rows * cols, 8), fmt)
+    gen, L = torch.Generator().manual_seed(M), ia._lib.lib()
+    xs = [torch.randn(M, cols, generator=gen).cuda() for _ in range(2)]
+    ys = [torch.empty(calls, M, rows, device="cuda") for _ in range(2)]
+    with ia.DeviceWeights.from_blocks(payload, blocks, rows, cols) as dw:
+        want = [dw.gemv(x).clone() for x in xs]
+        stream = ia._lib.current_stream()
+        torch.cuda.synchronize()
+        gate, rcs = threading.Barrier(2), [[], []]
+
+        def work(i):
+            gate.wait()
+            for c in range(calls):
+                rcs[i].append(L.oilhip_gemv_f32(dw.handle, xs[i].data_ptr(), ys[i][c].data_ptr(), M, stream))
+        threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        torch.cuda.synchronize()
+    for i in range(2):
+        assert rcs[i] == [0] * calls
+        assert int((ys[i] != want[i]).any(-1).any(-1).sum()) == 0, i
 
 
 def test_release_stream_scratch_frees_every_buffer_of_the_stream():
