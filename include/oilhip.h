@@ -170,6 +170,15 @@ int oilhip_dequant_f32(const oilhip_weights* w, float* d_out, void* stream);
  * FP32 accumulation, 1 <= M (the reference caps a call at 512). */
 int oilhip_gemv_f32(const oilhip_weights* w, const float* d_x, float* d_y, int M, void* stream);
 
+/* The same product over a workspace of the caller's, where oilhip_gemv_f32 packs several activation rows in a scratch that
+ * belongs to the stream.  For calls that are captured: a graph keeps the address of what it packs into, so two graphs captured
+ * on one stream may be replayed side by side only if their calls had workspaces of their own (without one, calls on
+ * uniform OIL4 tensors with M >= 3 share the stream's, and calls on other tensors take slower kernels that pack nothing).
+ * d_ws: 16-byte aligned, at least oilhip_gemv_workspace_bytes(w, M), which may be 0; it has to live as long as the graph, and calls
+ * that follow one another on the stream may share it.  No counterpart in the reference. */
+size_t oilhip_gemv_workspace_bytes(const oilhip_weights* w, int M);
+int oilhip_gemv_f32_ws(const oilhip_weights* w, const float* d_x, float* d_y, int M, void* d_ws, size_t ws_bytes, void* stream);
+
 /* The same product for uniform OIL4 tensors, for callers that cannot allocate device memory (code under HIP graph
  * capture, serving loops and harnesses that forbid hipMalloc).  No counterpart in the reference.  It calls no
  * hipMalloc/hipFree: the scratch its multi-row kernel needs (packed activations and their powers of two, 8 MB) is a fixed array in the
@@ -322,6 +331,11 @@ int oilhip_gemv_rmsnorm_f32(const oilhip_weights* w, const float* d_x, const flo
                             void* stream);
 int oilhip_mlp_step_f32(const oilhip_weights* gate_up, const oilhip_weights* down, const float* d_x, const float* d_normw,
                         float* d_y, int M, float* d_scratch, void* stream);
+/* the two with a workspace as in oilhip_gemv_f32_ws (for the step: the larger of its tensors' needs) */
+int oilhip_gemv_rmsnorm_f32_ws(const oilhip_weights* w, const float* d_x, const float* d_normw, float* d_y, int M, float* d_xn,
+                               void* d_ws, size_t ws_bytes, void* stream);
+int oilhip_mlp_step_f32_ws(const oilhip_weights* gate_up, const oilhip_weights* down, const float* d_x, const float* d_normw,
+                           float* d_y, int M, float* d_scratch, void* d_ws, size_t ws_bytes, void* stream);
 int oilhip_embed_rows_f32(const oilhip_weights* w, const int32_t* d_ids, int n, float* d_out, void* stream);
 
 /* ------------------------------------------------------------ mixture of experts

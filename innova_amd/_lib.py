@@ -64,6 +64,8 @@ _SIGNATURES = {
     "oilhip_rmsnorm_f32": (C.c_int, [vp, vp, C.c_int, C.c_int, vp, vp]),
     "oilhip_gemv_rmsnorm_f32": (C.c_int, [vp, vp, vp, vp, C.c_int, vp, vp]),
     "oilhip_mlp_step_f32": (C.c_int, [vp, vp, vp, vp, vp, C.c_int, vp, vp]),
+    "oilhip_gemv_rmsnorm_f32_ws": (C.c_int, [vp, vp, vp, vp, C.c_int, vp, vp, C.c_size_t, vp]),
+    "oilhip_mlp_step_f32_ws": (C.c_int, [vp, vp, vp, vp, vp, C.c_int, vp, vp, C.c_size_t, vp]),
     "oilhip_embed_rows_f32": (C.c_int, [vp, vp, C.c_int, vp, vp]),
     "oilhip_moe_route": (C.c_int, [vp, C.c_int64, C.c_int64, C.c_int64, vp, vp, vp]),
     "oilhip_moe_workspace_bytes": (C.c_size_t, [C.c_int64, C.c_int64, C.c_int64, C.c_int64]),
@@ -71,6 +73,8 @@ _SIGNATURES = {
                                      C.POINTER(C.c_float), C.POINTER(C.c_int64), vp]),
     "oilhip_dequant_f32": (C.c_int, [vp, vp, vp]),
     "oilhip_gemv_f32": (C.c_int, [vp, vp, vp, C.c_int, vp]),
+    "oilhip_gemv_workspace_bytes": (C.c_size_t, [vp, C.c_int]),
+    "oilhip_gemv_f32_ws": (C.c_int, [vp, vp, vp, C.c_int, vp, C.c_size_t, vp]),
     "oilhip_gemv_f32_general": (C.c_int, [vp, vp, vp, C.c_int, vp]),
     "oilhip_gemv_oil4_f32_noalloc": (C.c_int, [vp, vp, vp, C.c_int, vp]),
     "oilhip_set_ordered_sums": (C.c_int, [C.c_int]),
@@ -153,3 +157,13 @@ def current_stream() -> int:
         torch.cuda.init()
         _stream_of, _device_of = torch._C._cuda_getCurrentRawStream, torch._C._cuda_getDevice
     return _stream_of(_device_of())
+
+
+def graph_workspace(M, *weights):
+    """While torch captures a graph: a workspace for calls of M rows over these tensors, as (tensor, bytes).  It comes from the
+    graph's own memory pool, so that two graphs captured on one stream share nothing.  None otherwise."""
+    import torch
+    if M < 2 or not torch._C._cuda_isCurrentStreamCapturing():
+        return None
+    need = max(lib().oilhip_gemv_workspace_bytes(w.handle, M) for w in weights)
+    return torch.empty(max(need, 1), dtype=torch.uint8, device="cuda"), need

@@ -123,16 +123,18 @@ int stream_scratch(const StreamLock& lock, int slot, size_t bytes, void** out) {
     return OILHIP_OK;
 }
 
-// whether stream_scratch would succeed without an allocation that stream capture forbids
-bool stream_scratch_ready(hipStream_t s, int slot, size_t bytes) {
+bool stream_capturing(hipStream_t s) {
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &st) == hipSuccess && st == hipStreamCaptureStatusNone) return true;
+    if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
     (void)hipGetLastError();
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return false;
-    std::lock_guard<std::mutex> lk(g_scratch_mu);
-    const auto e = g_scratch.find(std::make_tuple(dev, (void*)s, slot));
-    return e != g_scratch.end() && e->second.second >= bytes;
+    return true;
+}
+
+int check_workspace(const oilhip_weights& w, int M, const void* d_ws, size_t ws_bytes) {
+    const size_t need = oilhip_gemv_workspace_bytes(&w, M);
+    if (need && (!d_ws || ws_bytes < need || (reinterpret_cast<uintptr_t>(d_ws) & 15u)))
+        return fail(OILHIP_E_ARG, "this call needs a 16-byte aligned workspace of " + std::to_string(need) + " bytes");
+    return OILHIP_OK;
 }
 
 int check_matmul_shape(const oilhip_weights* w, const void* x, const void* y, int M) {
@@ -145,6 +147,38 @@ int check_matmul_shape(const oilhip_weights* w, const void* x, const void* y, in
     if (w->rows > 0xFFFFFFFFull || w->cols > 0xFFFFFFFFull)
         return fail(OILHIP_E_ARG, "rows/cols exceed 32 bits");
     return OILHIP_OK;
+}
+
+int gemv_f32(const oilhip_weights& w, const float* d_x, float* d_y, int M, hipStream_t s, uint8_t* d_pack) {
+    if (plain_oil4(w)) {
+        // one or two rows: the register-resident kernel; from three on the matrix-core kernel (16 rows per pass) is faster
+        int rc = 1;                                                                          // 1: shape not covered
+        if (M <= 2) rc = launch_gemv_oil4(w, d_x, d_y, M, s);
+        if (rc == 1 && M >= 2)
+            rc = launch_gemv_oil4_multi(w, d_x, nullptr, d_y, M, (uint32_t)w.cols, (uint32_t)w.rows, (uint32_t)M, s, {}, nullptr, nullptr, 0, d_pack);
+        if (rc == 1 && M > 2 && M <= 4) rc = launch_gemv_oil4(w, d_x, d_y, M, s);
+        if (rc <= 0) return rc;
+    }
+    if (M >= 2) {
+        const int rc = launch_gemv_any_multi(w, d_x, d_y, M, s, d_pack);
+        if (rc <= 0) return rc;
+    }
+    if (plain_oil8(w)) {
+        // the register-resident kernel takes up to four activation rows per launch
+        int rc = 1;
+        for (int m0 = 0; m0 < M; m0 += 4) {
+            rc = launch_gemv_oil8(w, d_x + (size_t)m0 * w.cols, d_y + (size_t)m0 * w.rows, M - m0 < 4 ? M - m0 : 4, s);
+            if (rc != 0) break;
+        }
+        if (rc <= 0) return rc;
+    }
+    if (w.seg.nstreams) {
+        const int rc = launch_gemv_seg(w, d_x, d_y, M, s);
+        if (rc <= 0) return rc;
+    }
+    const int rc = launch_gemv_runs(w, d_x, d_y, M, s);
+    if (rc <= 0) return rc;
+    return launch_gemv_generic(w, d_x, d_y, M, s);
 }
 
 }  // namespace oilhip
@@ -575,37 +609,19 @@ int oilhip_dequant_f32(const oilhip_weights* w, float* d_out, void* stream) {
 
 int oilhip_gemv_f32(const oilhip_weights* w, const float* d_x, float* d_y, int M, void* stream) {
     if (int rc = check_matmul_shape(w, d_x, d_y, M)) return rc;
-    if (plain_oil4(*w)) {
-        // one or two rows: the register-resident kernel; from three on the matrix-core kernel (16 rows per pass) is faster
-        int rc = 1;                                                                          // 1: shape not covered
-        if (M <= 2) rc = launch_gemv_oil4(*w, d_x, d_y, M, (hipStream_t)stream);
-        if (rc == 1 && M >= 2)
-            rc = launch_gemv_oil4_multi(*w, d_x, nullptr, d_y, M, (uint32_t)w->cols, (uint32_t)w->rows, (uint32_t)M,
-                                        (hipStream_t)stream);
-        if (rc == 1 && M > 2 && M <= 4) rc = launch_gemv_oil4(*w, d_x, d_y, M, (hipStream_t)stream);
-        if (rc <= 0) return rc;
-    }
-    if (M >= 2) {
-        const int rc = launch_gemv_any_multi(*w, d_x, d_y, M, (hipStream_t)stream);
-        if (rc <= 0) return rc;
-    }
-    if (plain_oil8(*w)) {
-        // the register-resident kernel takes up to four activation rows per launch
-        int rc = 1;
-        for (int m0 = 0; m0 < M; m0 += 4) {
-            rc = launch_gemv_oil8(*w, d_x + (size_t)m0 * w->cols, d_y + (size_t)m0 * w->rows, M - m0 < 4 ? M - m0 : 4,
-                                  (hipStream_t)stream);
-            if (rc != 0) break;
-        }
-        if (rc <= 0) return rc;
-    }
-    if (w->seg.nstreams) {
-        const int rc = launch_gemv_seg(*w, d_x, d_y, M, (hipStream_t)stream);
-        if (rc <= 0) return rc;
-    }
-    const int rc = launch_gemv_runs(*w, d_x, d_y, M, (hipStream_t)stream);
-    if (rc <= 0) return rc;
-    return launch_gemv_generic(*w, d_x, d_y, M, (hipStream_t)stream);
+    return gemv_f32(*w, d_x, d_y, M, (hipStream_t)stream, nullptr);
+}
+
+size_t oilhip_gemv_workspace_bytes(const oilhip_weights* w, int M) {
+    if (!w || M < 2) return 0;
+    const size_t n = plain_oil4(*w) ? gemv_oil4_multi_bytes(*w, M) : gemv_any_multi_bytes(*w, M);
+    return (n + 255u) & ~(size_t)255u;
+}
+
+int oilhip_gemv_f32_ws(const oilhip_weights* w, const float* d_x, float* d_y, int M, void* d_ws, size_t ws_bytes, void* stream) {
+    if (int rc = check_matmul_shape(w, d_x, d_y, M)) return rc;
+    if (int rc = check_workspace(*w, M, d_ws, ws_bytes)) return rc;
+    return gemv_f32(*w, d_x, d_y, M, (hipStream_t)stream, static_cast<uint8_t*>(d_ws));
 }
 
 // Test hook: the all-format kernel regardless of shape (the specialised kernels

@@ -60,7 +60,7 @@ private:
     std::lock_guard<std::mutex> held_;
 };
 int stream_scratch(const StreamLock& lock, int slot, size_t bytes, void** out);
-bool stream_scratch_ready(hipStream_t s, int slot, size_t bytes);   // false: this call would fail, the stream is being captured
+bool stream_capturing(hipStream_t s);
 
 // Tensors whose rows mix formats are stored as `nstreams` streams of windows of at most 4 KB, made for one wavefront each,
 // `waves` (8, or 16 with windows of at most 2 KB) wavefronts per CU (gemv_seg.hip).  The first window of stream s sits at byte s * stream_bytes of the payload buffer, the later ones
@@ -147,8 +147,14 @@ int launch_gemv_oil4_multi_batches(int nb, const oilhip_weights* const* wa, floa
                                    const int* M, const int* row0, const int* list, int nlist, const float* d_x, const float* d_x2,
                                    uint32_t ldx, uint32_t xrows, uint32_t ldy, void* d_ws, size_t ws_bytes, hipStream_t s);
 // other formats, 3 to 16 rows per pass (FP16 MFMA, gemv_any_multi.hip)
-int launch_gemv_any_multi(const oilhip_weights& w, const float* d_x, float* d_y, int M, hipStream_t s);
-// widest row that these kernels take and the bytes of packed activations one pass needs (d_pack, or stream scratch): per
+int launch_gemv_any_multi(const oilhip_weights& w, const float* d_x, float* d_y, int M, hipStream_t s, uint8_t* d_pack = nullptr);
+// bytes of d_pack that these two kernels need (0: they do not serve the tensor)
+size_t gemv_oil4_multi_bytes(const oilhip_weights& w, int M);
+size_t gemv_any_multi_bytes(const oilhip_weights& w, int M);
+// oilhip_gemv_f32 after its checks; d_pack as in oilhip_gemv_f32_ws
+int gemv_f32(const oilhip_weights& w, const float* d_x, float* d_y, int M, hipStream_t s, uint8_t* d_pack);
+int check_workspace(const oilhip_weights& w, int M, const void* d_ws, size_t ws_bytes);
+// widest row that these kernels take and the bytes of packed activations that any pass needs (d_pack, or stream scratch): per
 // block 32 floats (powers of two) and three digits of 256 activations for 32 tokens, or 48 floats and 27 KB of FP16 pieces
 constexpr uint32_t kGemvPackMaxCols = 32768;
 constexpr size_t kGemvPackBytes = (size_t)(kGemvPackMaxCols >> 8) * (192u + 27648u);

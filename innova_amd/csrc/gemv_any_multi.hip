@@ -614,27 +614,42 @@ int source_of(const oilhip_weights& w) {
     return w.uniform_fmt == OILHIP_OIL8 && w.uniform_stride == 256u && w.uniform_cb == 0 && w.uniform_idx == 256u && (w.uniform_base & 3u) == 0 ? kOil8 : -1;
 }
 
-}  // namespace
-
-// Returns 1 when the tensor, the shape or the stream (one that is being captured and has no scratch yet) is outside what this
-// kernel covers, or another one is faster.
-int launch_gemv_any_multi(const oilhip_weights& w, const float* d_x, float* d_y, int M, hipStream_t s) {
+// what the tensor's weights are, or -1 where these kernels do not cover the tensor and the batch, or another one is faster
+int source_for(const oilhip_weights& w, int M) {
     const int src = source_of(w);
-    if (src < 0 || M < 2 || !w.all_full || (w.cols & 255u) || w.cols == 0 || w.cols > kGemvPackMaxCols || w.rows == 0 || w.rows > 0x7FFFFFFFull) return 1;
+    if (src < 0 || M < 2 || !w.all_full || (w.cols & 255u) || w.cols == 0 || w.cols > kGemvPackMaxCols || w.rows == 0 || w.rows > 0x7FFFFFFFull) return -1;
     // The kernels of up to four rows per pass stay for two rows, and for three and four (window streams: while four rows of
     // activations fit their LDS) on tensors of less than 12 M weights: 2000 x 2048, 3 rows 8.5 against 8.9 us; 4096 x 4096 14.2
     // against 12.8 us.  The OIL8 kernel stays up to two passes on small tensors: 1000 x 1024, 6 rows 7.6 against 8.0 us.
     const uint64_t weights = w.rows * w.cols;
-    if (M == 2 || (M <= 4 && w.seg.waves != 16 && weights < 12000000u && !(by_descriptor(src) && w.cols > 5120u))) return 1;
-    if (src == kOil8 && M <= 8 && weights < 2000000u) return 1;
+    if (M == 2 || (M <= 4 && w.seg.waves != 16 && weights < 12000000u && !(by_descriptor(src) && w.cols > 5120u))) return -1;
+    if (src == kOil8 && M <= 8 && weights < 2000000u) return -1;
     const uint32_t bpr = (uint32_t)(w.cols >> 8);
     // 32-bit byte offsets inside a workgroup's rows (blocks, or descriptors)
     const uint64_t per_row = std::max<uint64_t>(16u, by_descriptor(src) ? 16u : block_bytes(src)) * bpr;
-    if ((w.rows / (16u * (uint64_t)device_cu_count()) + 8u) * 16u * per_row >= 0x80000000ull) return 1;
+    if ((w.rows / (16u * (uint64_t)device_cu_count()) + 8u) * 16u * per_row >= 0x80000000ull) return -1;
+    return src;
+}
+
+}  // namespace
+
+size_t gemv_any_multi_bytes(const oilhip_weights& w, int M) {
+    const int src = source_for(w, M);
+    if (src < 0) return 0;
+    const size_t tiles = (size_t)tiles_for(std::min(M, kPassTokens));
+    return (size_t)(w.cols >> 8) * tiles * (64u + tile_bytes(grouped(src)));
+}
+
+// Returns 1 where these kernels do not serve the call.  Without d_pack, a call that is being captured is left to the kernels that
+// use no scratch: two graphs captured on one stream would share the stream's, and they may be replayed side by side.
+int launch_gemv_any_multi(const oilhip_weights& w, const float* d_x, float* d_y, int M, hipStream_t s, uint8_t* d_pack) {
+    const int src = source_for(w, M);
+    if (src < 0 || (!d_pack && stream_capturing(s))) return 1;
+    const uint32_t bpr = (uint32_t)(w.cols >> 8);
     const StreamLock lock(s);
-    uint8_t* xp = nullptr;
-    if (!stream_scratch_ready(s, kScratchGemvPack, kGemvPackBytes)) return 1;
-    if (int rc = stream_scratch(lock, kScratchGemvPack, kGemvPackBytes, reinterpret_cast<void**>(&xp))) return rc;
+    uint8_t* xp = d_pack;
+    if (!xp)
+        if (int rc = stream_scratch(lock, kScratchGemvPack, kGemvPackBytes, reinterpret_cast<void**>(&xp))) return rc;
     for (int m0 = 0; m0 < M; m0 += kPassTokens) {
         const int m = std::min(M - m0, kPassTokens), tiles = tiles_for(m);
         const float* x = d_x + (size_t)m0 * w.cols;

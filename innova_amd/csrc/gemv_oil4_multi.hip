@@ -564,6 +564,12 @@ int static_pack_buffer(uint8_t** out) {
 
 }  // namespace
 
+size_t gemv_oil4_multi_bytes(const oilhip_weights& w, int M) {
+    if (!plain_oil4(w) || !shape_covered(w, 1, (uint32_t)w.cols)) return 0;
+    const uint32_t bpr = (uint32_t)(w.cols >> 8);
+    return undo_bytes(bpr) + (size_t)bpr * kind_block_bytes(kind_of(std::min(M, kMaxTokens)));
+}
+
 // Y[m][r] for m < M: x row tok[m] (or m when tok is null) of an [xrows][ldx] activation matrix; with w2 the same activations
 // also go through a second tensor of the same width into d_y2 (the gate and up projections of an expert): they are packed
 // once per pass for both.  `in` says what the activations are (common.h).  Returns 1 when the shape is outside what this

@@ -87,6 +87,60 @@ embed_rows_kernel(const uint8_t* __restrict__ payload, const DevBlock* __restric
     o[threadIdx.x] = decode_weight(d.fmt, cb, d.cb_bytes, cb + d.cb_bytes, d.idx_bytes, d.nw, threadIdx.x, T);
 }
 
+// oilhip_gemv_rmsnorm_f32 and oilhip_mlp_step_f32; d_pack as in oilhip_gemv_f32_ws
+int gemv_rmsnorm(const oilhip_weights& w, const float* d_x, const float* d_normw, float* d_y, int M, float* d_xn, hipStream_t s, uint8_t* d_pack) {
+    if (int rc = check_matmul_shape(&w, d_x, d_y, M)) return rc;
+    if (M == 1 && plain_oil4(w)) {
+        const int rc = launch_gemv_oil4_rmsnorm(w, d_x, d_normw, d_y, s);  // the norm rides on the staging of x
+        if (rc <= 0) return rc;
+    }
+    if (M == 1 && w.seg.nstreams) {
+        const int rc = launch_gemv_seg_rmsnorm(w, d_x, d_normw, d_y, s);   // likewise for window-stream tensors
+        if (rc <= 0) return rc;
+    }
+    if (!d_xn) return fail(OILHIP_E_ARG, "gemv_rmsnorm: this shape needs the d_xn workspace");
+    const uintptr_t x0 = reinterpret_cast<uintptr_t>(d_x), xn0 = reinterpret_cast<uintptr_t>(d_xn), size = (uintptr_t)M * w.cols * 4u;
+    const bool apart = x0 + size <= xn0 || xn0 + size <= x0;               // packing wavefronts read whole rows while others store theirs
+    if (M > 1 && plain_oil4(w) && w.cols <= kPackNormMaxCols && apart) {   // the norm rides on the packing of the activations
+        const int rc = launch_gemv_oil4_multi(w, d_x, nullptr, d_y, M, (uint32_t)w.cols, (uint32_t)w.rows, (uint32_t)M, s,
+                                              MultiInput{nullptr, d_normw, false, d_xn}, nullptr, nullptr, 0, d_pack);
+        if (rc <= 0) return rc;
+    }
+    if (int rc = oilhip_rmsnorm_f32(d_x, d_normw, (int)w.cols, M, d_xn, s)) return rc;
+    return gemv_f32(w, d_xn, d_y, M, s, d_pack);
+}
+
+int mlp_step(const oilhip_weights& gate_up, const oilhip_weights& down, const float* d_x, const float* d_normw, float* d_y, int M,
+             float* d_scratch, hipStream_t s, uint8_t* d_pack) {
+    const uint64_t F = down.cols;
+    if (gate_up.rows != 2 * F || gate_up.cols != down.rows)
+        return fail(OILHIP_E_ARG, "mlp_step: gate_up must be 2F x D (gate rows first) and down D x F");
+    if (int rc = check_matmul_shape(&gate_up, d_x, d_y, M)) return rc;
+    if (int rc = check_matmul_shape(&down, d_x, d_y, M)) return rc;
+    float* h2 = d_scratch;                                   // [M][2F]
+    float* h = d_scratch + (size_t)M * 2 * F;                // [M][F]
+    float* xn = h + (size_t)M * F;                           // [M][D], only with d_normw
+    if (int rc = d_normw ? gemv_rmsnorm(gate_up, d_x, d_normw, h2, M, xn, s, d_pack) : gemv_f32(gate_up, d_x, h2, M, s, d_pack)) return rc;
+    if (M == 1 && plain_oil4(down)) {
+        const int rc = launch_gemv_oil4_swiglu(down, h2, d_y, s);          // SwiGLU formed while the activations are staged
+        if (rc <= 0) return rc;
+    }
+    if (M == 1 && down.seg.nstreams) {
+        const int rc = launch_gemv_seg_swiglu(down, h2, d_y, s);
+        if (rc <= 0) return rc;
+    }
+    if (M > 1 && plain_oil4(down)) {                         // SwiGLU formed while the activations are packed
+        const int rc = launch_gemv_oil4_multi(down, h2, nullptr, d_y, M, (uint32_t)(2 * F), (uint32_t)down.rows, (uint32_t)M, s,
+                                              MultiInput{h2 + F, nullptr, true}, nullptr, nullptr, 0, d_pack);
+        if (rc <= 0) return rc;
+    }
+    const size_t n = (size_t)F * (size_t)M;
+    hipLaunchKernelGGL(swiglu_rows_kernel, dim3((uint32_t)((n + 255) / 256 < 4096 ? (n + 255) / 256 : 4096)), dim3(256), 0, s,
+                       h2, h, (uint32_t)F, (uint32_t)M);
+    OILHIP_HIP(hipGetLastError());
+    return gemv_f32(down, h, d_y, M, s, d_pack);
+}
+
 }  // namespace
 }  // namespace oilhip
 
@@ -106,59 +160,28 @@ int oilhip_rmsnorm_f32(const float* d_x, const float* d_w, int n, int rows, floa
 int oilhip_gemv_rmsnorm_f32(const oilhip_weights* w, const float* d_x, const float* d_normw, float* d_y, int M, float* d_xn,
                             void* stream) {
     if (!w || !d_x || !d_normw || !d_y || M <= 0) return fail(OILHIP_E_ARG, "gemv_rmsnorm: bad arguments");
-    if (int rc = check_matmul_shape(w, d_x, d_y, M)) return rc;
-    if (M == 1 && plain_oil4(*w)) {
-        const int rc = launch_gemv_oil4_rmsnorm(*w, d_x, d_normw, d_y, (hipStream_t)stream);   // the norm rides on the staging of x
-        if (rc <= 0) return rc;
-    }
-    if (M == 1 && w->seg.nstreams) {
-        const int rc = launch_gemv_seg_rmsnorm(*w, d_x, d_normw, d_y, (hipStream_t)stream);    // likewise for window-stream tensors
-        if (rc <= 0) return rc;
-    }
-    if (!d_xn) return fail(OILHIP_E_ARG, "gemv_rmsnorm: this shape needs the d_xn workspace");
-    const uintptr_t x0 = reinterpret_cast<uintptr_t>(d_x), xn0 = reinterpret_cast<uintptr_t>(d_xn), size = (uintptr_t)M * w->cols * 4u;
-    const bool apart = x0 + size <= xn0 || xn0 + size <= x0;               // packing wavefronts read whole rows while others store theirs
-    if (M > 1 && plain_oil4(*w) && w->cols <= kPackNormMaxCols && apart) { // the norm rides on the packing of the activations
-        const int rc = launch_gemv_oil4_multi(*w, d_x, nullptr, d_y, M, (uint32_t)w->cols, (uint32_t)w->rows, (uint32_t)M, (hipStream_t)stream,
-                                              MultiInput{nullptr, d_normw, false, d_xn});
-        if (rc <= 0) return rc;
-    }
-    if (int rc = oilhip_rmsnorm_f32(d_x, d_normw, (int)w->cols, M, d_xn, stream)) return rc;
-    return oilhip_gemv_f32(w, d_xn, d_y, M, stream);
+    return gemv_rmsnorm(*w, d_x, d_normw, d_y, M, d_xn, (hipStream_t)stream, nullptr);
+}
+
+int oilhip_gemv_rmsnorm_f32_ws(const oilhip_weights* w, const float* d_x, const float* d_normw, float* d_y, int M, float* d_xn,
+                               void* d_ws, size_t ws_bytes, void* stream) {
+    if (!w || !d_x || !d_normw || !d_y || M <= 0) return fail(OILHIP_E_ARG, "gemv_rmsnorm: bad arguments");
+    if (int rc = check_workspace(*w, M, d_ws, ws_bytes)) return rc;
+    return gemv_rmsnorm(*w, d_x, d_normw, d_y, M, d_xn, (hipStream_t)stream, static_cast<uint8_t*>(d_ws));
 }
 
 int oilhip_mlp_step_f32(const oilhip_weights* gate_up, const oilhip_weights* down, const float* d_x, const float* d_normw,
                         float* d_y, int M, float* d_scratch, void* stream) {
     if (!gate_up || !down || !d_x || !d_y || !d_scratch || M <= 0) return fail(OILHIP_E_ARG, "mlp_step: bad arguments");
-    const uint64_t F = down->cols;
-    if (gate_up->rows != 2 * F || gate_up->cols != down->rows)
-        return fail(OILHIP_E_ARG, "mlp_step: gate_up must be 2F x D (gate rows first) and down D x F");
-    if (int rc = check_matmul_shape(gate_up, d_x, d_y, M)) return rc;
-    if (int rc = check_matmul_shape(down, d_x, d_y, M)) return rc;
-    hipStream_t s = (hipStream_t)stream;
-    float* h2 = d_scratch;                                   // [M][2F]
-    float* h = d_scratch + (size_t)M * 2 * F;                // [M][F]
-    float* xn = h + (size_t)M * F;                           // [M][D], only with d_normw
-    if (int rc = d_normw ? oilhip_gemv_rmsnorm_f32(gate_up, d_x, d_normw, h2, M, xn, stream)
-                         : oilhip_gemv_f32(gate_up, d_x, h2, M, stream)) return rc;
-    if (M == 1 && plain_oil4(*down)) {
-        const int rc = launch_gemv_oil4_swiglu(*down, h2, d_y, s);      // SwiGLU formed while the activations are staged
-        if (rc <= 0) return rc;
-    }
-    if (M == 1 && down->seg.nstreams) {
-        const int rc = launch_gemv_seg_swiglu(*down, h2, d_y, s);
-        if (rc <= 0) return rc;
-    }
-    if (M > 1 && plain_oil4(*down)) {                        // SwiGLU formed while the activations are packed
-        const int rc = launch_gemv_oil4_multi(*down, h2, nullptr, d_y, M, (uint32_t)(2 * F), (uint32_t)down->rows, (uint32_t)M, s,
-                                              MultiInput{h2 + F, nullptr, true});
-        if (rc <= 0) return rc;
-    }
-    const size_t n = (size_t)F * (size_t)M;
-    hipLaunchKernelGGL(swiglu_rows_kernel, dim3((uint32_t)((n + 255) / 256 < 4096 ? (n + 255) / 256 : 4096)), dim3(256), 0, s,
-                       h2, h, (uint32_t)F, (uint32_t)M);
-    OILHIP_HIP(hipGetLastError());
-    return oilhip_gemv_f32(down, h, d_y, M, stream);
+    return mlp_step(*gate_up, *down, d_x, d_normw, d_y, M, d_scratch, (hipStream_t)stream, nullptr);
+}
+
+int oilhip_mlp_step_f32_ws(const oilhip_weights* gate_up, const oilhip_weights* down, const float* d_x, const float* d_normw,
+                           float* d_y, int M, float* d_scratch, void* d_ws, size_t ws_bytes, void* stream) {
+    if (!gate_up || !down || !d_x || !d_y || !d_scratch || M <= 0) return fail(OILHIP_E_ARG, "mlp_step: bad arguments");
+    if (int rc = check_workspace(*gate_up, M, d_ws, ws_bytes)) return rc;
+    if (int rc = check_workspace(*down, M, d_ws, ws_bytes)) return rc;
+    return mlp_step(*gate_up, *down, d_x, d_normw, d_y, M, d_scratch, (hipStream_t)stream, static_cast<uint8_t*>(d_ws));
 }
 
 int oilhip_embed_rows_f32(const oilhip_weights* w, const int32_t* d_ids, int n, float* d_out, void* stream) {

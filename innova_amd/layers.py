@@ -28,8 +28,12 @@ def gemv_rmsnorm(w: DeviceWeights, x, norm_w, out=None):
     # xn and the scratch of mlp_step go back to torch's allocator when these return, while the launches may still be queued:
     # the allocator hands a block out again in the order of the stream it came from, which is the stream they run on
     xn = torch.empty_like(x)
-    _lib.check(_lib.lib().oilhip_gemv_rmsnorm_f32(w.handle, x.data_ptr(), norm_w.data_ptr(), out.data_ptr(), M, xn.data_ptr(),
-                                                  _lib.current_stream()))
+    args = w.handle, x.data_ptr(), norm_w.data_ptr(), out.data_ptr(), M, xn.data_ptr()
+    ws = _lib.graph_workspace(M, w)
+    if ws is not None:
+        _lib.check(_lib.lib().oilhip_gemv_rmsnorm_f32_ws(*args, ws[0].data_ptr(), ws[1], _lib.current_stream()))
+    else:
+        _lib.check(_lib.lib().oilhip_gemv_rmsnorm_f32(*args, _lib.current_stream()))
     return out
 
 
@@ -42,9 +46,13 @@ def mlp_step(gate_up: DeviceWeights, down: DeviceWeights, x, out=None, norm_w=No
     if out is None:
         out = x.new_empty((M, down.rows))
     scratch = x.new_empty((3 * F + gate_up.cols) * M)
-    _lib.check(_lib.lib().oilhip_mlp_step_f32(gate_up.handle, down.handle, x.data_ptr(),
-                                              norm_w.data_ptr() if norm_w is not None else None, out.data_ptr(), M,
-                                              scratch.data_ptr(), _lib.current_stream()))
+    args = (gate_up.handle, down.handle, x.data_ptr(), norm_w.data_ptr() if norm_w is not None else None, out.data_ptr(), M,
+            scratch.data_ptr())
+    ws = _lib.graph_workspace(M, gate_up, down)
+    if ws is not None:
+        _lib.check(_lib.lib().oilhip_mlp_step_f32_ws(*args, ws[0].data_ptr(), ws[1], _lib.current_stream()))
+    else:
+        _lib.check(_lib.lib().oilhip_mlp_step_f32(*args, _lib.current_stream()))
     return out
 
 

@@ -121,6 +121,10 @@ class DeviceWeights:
         M = self._rows(x, torch.float32)
         out = self._out(x, M, out)
         L = _lib.lib()
+        ws = None if general or noalloc else _lib.graph_workspace(M, self)
+        if ws is not None:
+            _lib.check(L.oilhip_gemv_f32_ws(self.handle, x.data_ptr(), out.data_ptr(), M, ws[0].data_ptr(), ws[1], _lib.current_stream()))
+            return out
         fn = L.oilhip_gemv_f32_general if general else L.oilhip_gemv_oil4_f32_noalloc if noalloc else L.oilhip_gemv_f32
         _lib.check(fn(self.handle, x.data_ptr(), out.data_ptr(), M, _lib.current_stream()))
         return out

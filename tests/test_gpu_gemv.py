@@ -13,6 +13,7 @@ import torch
 import innova_amd as ia
 import oracle as O
 from gpu_util import gaussian_weights, rel_l2, to_orc_blocks
+from innova_amd import layers
 
 pytestmark = pytest.mark.gpu
 TOL = 1e-5
@@ -411,6 +412,79 @@ def test_two_threads_on_one_stream(fmt, M):
     for i in range(2):
         assert rcs[i] == [0] * calls
         assert int((ys[i] != want[i]).any(-1).any(-1).sum()) == 0, i
+
+
+# Two graphs captured on one stream (torch's default) and replayed side by side on two: their calls must not share what they pack into.
+# "c": the entry point without a workspace, which takes kernels that pack nothing while a call is captured.
+@pytest.mark.parametrize("fmt,M,how", [(ia.Format.OIL4, 5, "gemv"), (ia.Format.SPARK_Q0, 5, "gemv"), (ia.Format.OIL8, 12, "gemv"),
+                                       (ia.Format.SPARK_Q0, 5, "c"), (ia.Format.OIL4, 2, "layer"), (ia.Format.OIL4, 5, "layer"),
+                                       (ia.Format.OIL2, 5, "layer")])
+def test_two_graphs_of_one_capture_stream(fmt, M, how):
+    rows, cols, calls = 512, 512, 24
+    payload, blocks = ia.block_codec.quantize_tensor(gaussian_weights(rows * cols, 8) * np.float32(2.0), fmt)
+    gen, L = torch.Generator().manual_seed(M), ia._lib.lib()
+    dw = ia.DeviceWeights.from_blocks(payload, blocks, rows, cols)
+    half = ia.DeviceWeights.quantize(gaussian_weights(cols * 256, 9), fmt, cols, 256)
+    norm = torch.zeros(cols, device="cuda")
+    ins = [[torch.randn(M, cols, generator=gen).cuda() for _ in range(calls)] for _ in range(2)]
+    outs = [[torch.empty(M, rows, device="cuda") for _ in range(calls)] for _ in range(2)]
+
+    def call(x, y):
+        if how == "gemv":
+            dw.gemv(x, out=y)
+        elif how == "c":
+            ia._lib.check(L.oilhip_gemv_f32(dw.handle, x.data_ptr(), y.data_ptr(), M, ia._lib.current_stream()))
+        else:
+            layers.gemv_rmsnorm(dw, x, norm, out=y)
+            layers.mlp_step(dw, half, y, out=y, norm_w=norm)
+    side = torch.cuda.Stream()                            # warm-up and capture
+    with torch.cuda.stream(side):
+        for i in range(2):
+            for x, y in zip(ins[i], outs[i]):
+                call(x, y)
+    torch.cuda.synchronize()
+    want = [[y.clone() for y in ys] for ys in outs]
+    graphs = []
+    for i in range(2):
+        graphs.append(torch.cuda.CUDAGraph())
+        with torch.cuda.graph(graphs[i], stream=side):
+            for x, y in zip(ins[i], outs[i]):
+                call(x, y)
+    streams, bad = [torch.cuda.Stream(), torch.cuda.Stream()], 0
+    for _ in range(40):
+        for ys in outs:
+            for y in ys:
+                y.fill_(float("nan"))
+        torch.cuda.synchronize()
+        for g, s in zip(graphs, streams):
+            with torch.cuda.stream(s):
+                g.replay()
+        torch.cuda.synchronize()
+        for i in range(2):
+            for y, ref in zip(outs[i], want[i]):          # "c" adds in another order than the eager call
+                bad += int((y - ref).norm() > 1e-5 * ref.norm()) if how == "c" else int(not torch.equal(y, ref))
+                bad += int(not bool(torch.isfinite(y).all()))
+    assert bad == 0
+    dw.close()
+    half.close()
+
+
+def test_workspace_of_the_caller():
+    """oilhip_gemv_f32_ws: the size that is asked for, the results of oilhip_gemv_f32, what is refused, and nothing beyond the size
+    written."""
+    L, rows, cols = ia._lib.lib(), 300, 1024
+    for fmt in (ia.Format.OIL4, ia.Format.OIL8, ia.Format.SPARK_Q0, ia.Format.OIL4_GRP, ia.Format.OIL16):
+        with ia.DeviceWeights.quantize(gaussian_weights(rows * cols, 4), fmt, rows, cols) as dw:
+            for M in (1, 2, 4, 5, 8, 16, 17, 33):
+                need = L.oilhip_gemv_workspace_bytes(dw.handle, M)
+                assert (need == 0) == (M == 1 or fmt == ia.Format.OIL16 or (fmt != ia.Format.OIL4 and M <= 4) or (fmt == ia.Format.OIL8 and M <= 8))
+                x = torch.randn(M, cols, generator=torch.Generator().manual_seed(M)).cuda()
+                y, ws = torch.empty(M, rows, device="cuda"), torch.full((need + 256,), 0x5A, dtype=torch.uint8, device="cuda")
+                ia._lib.check(L.oilhip_gemv_f32_ws(dw.handle, x.data_ptr(), y.data_ptr(), M, ws.data_ptr(), need, ia._lib.current_stream()))
+                assert torch.equal(y, dw.gemv(x)) and bool((ws[need:] == 0x5A).all())
+                if need:
+                    for at, size in ((ws.data_ptr(), need - 1), (ws.data_ptr() + 4, need), (None, need)):
+                        assert L.oilhip_gemv_f32_ws(dw.handle, x.data_ptr(), y.data_ptr(), M, at, size, ia._lib.current_stream()) != 0
 
 
 def test_release_stream_scratch_frees_every_buffer_of_the_stream():
