@@ -175,8 +175,9 @@ __device__ __forceinline__ void kv_quantize_chunk(const float* __restrict__ src,
 // reference's loop does.  A cluster whose range stays has the same sum as before, and when all ranges stay the centroids are a fixed
 // point.
 // That the comparison of neighbours is monotone over the sorted values and equals the reference's scan over all 16 needs
-// centroids that rise by more than the rounding of the distances (at most range * 2^-22); this is checked in every iteration, and
-// chunks that fail it, hold infinities or NaN, or are constant, go through kv_quantize_chunk.
+// centroids that are finite and rise by more than the rounding of the distances (at most range * 2^-22); this is checked in every
+// iteration, and chunks that fail it (large values: a cluster's sum overflows although its members are finite), hold infinities or
+// NaN, or are constant, go through kv_quantize_chunk.
 // What bounds it: vector issue of the iterations (about 60 instructions for four chunks each, of which a long append takes about a
 // dozen); the chain of dependent instructions and LDS round trips when a decode step appends one token, where each wavefront
 // takes one chunk.  One wavefront per chunk before (every value compared with all 16 centroids in each iteration, sums passed
@@ -295,6 +296,7 @@ __device__ __forceinline__ bool kv_lloyd_rows(const float (&x)[V], uint32_t n, u
     bool ok = range >= 1e-10f && range < __builtin_inff();
     ok &= ((__ballot(!finite) >> (lane & 48u)) & 0xFFFFull) == 0;
     float cen = __fadd_rn(lo, __fdiv_rn(__fmul_rn(range, (float)c + 0.5f), 16.0f));
+    ok &= ((__ballot(!(fabsf(cen) < __builtin_inff())) >> (lane & 48u)) & 0xFFFFull) == 0;
     const float least_gap = range * 0x1p-20f;
     // NaN before the first value and behind the last one: no comparison holds there.  Likewise the centroid before the first one, and
     // all centroids of a row that takes the other path: its boundaries stay where they are.
@@ -340,7 +342,7 @@ __device__ __forceinline__ bool kv_lloyd_rows(const float (&x)[V], uint32_t n, u
         cen = cnt > 0 ? mean : cen;
         below = lane_below(cen);
         const bool tight = __fsub_rn(cen, below) <= least_gap;             // false for the first one
-        ok &= !tight;
+        ok &= !tight & (fabsf(cen) < __builtin_inff());                    // of an infinite sum kv_mean makes NaN
         p_was = p;
         end_was = end;
     }

@@ -82,6 +82,24 @@ def test_quantize_blocks_rows_of_lanes(n, blocks):
         assert np.array_equal(cb[b], wcb) and np.array_equal(codes[b], wcodes), b
 
 
+# finite values so large that a cluster's sum overflows, that the first centroids do, or that the range does, beside ordinary blocks
+@pytest.mark.parametrize("n", [1, 16, 32, 50, 64, 128])
+@pytest.mark.parametrize("blocks", [5, 2053])
+def test_quantize_blocks_whose_sums_overflow(n, blocks):
+    rng = np.random.default_rng(n + blocks)
+    x = rng.standard_normal((blocks, n)).astype(np.float32)
+    x[1::5] = np.float32(1e38) * (1.0 + 0.01 * rng.standard_normal(x[1::5].shape)).astype(np.float32)
+    x[2::5] = np.float32(3e37) * rng.uniform(-1.0, 1.0, x[2::5].shape).astype(np.float32)
+    x[3::5] = np.float32(3.4e38) * np.sign(rng.standard_normal(x[3::5].shape)).astype(np.float32)
+    x[4::5] *= (10.0 ** rng.uniform(35.0, 37.8, (x[4::5].shape[0], 1))).astype(np.float32)
+    assert np.isfinite(x).all()
+    codes, cb = ia.OIL4KVCache.quantize_block_oil4(dev(x))
+    codes, cb = codes.cpu().numpy(), cb.cpu().numpy().view(np.uint16)
+    for b in range(blocks):
+        wcb, wcodes = O.kv_quantize_block(x[b])
+        assert np.array_equal(cb[b], wcb) and np.array_equal(codes[b], wcodes), b
+
+
 @pytest.mark.parametrize("i", range(len(MF.KV_CASES)))
 def test_cache_fixture(i):
     ms, h, d, block, lens = MF.KV_CASES[i]
