@@ -123,6 +123,11 @@ gemm_dense_kernel(const DenseArgs a) {
         }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // nothing may write LDS after the end
+    // 12 wait states between the last matrix instruction and a read of its sums, which the compiler does not count along a branch
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) asm volatile("s_nop 11" : "+v"(acc[i][j]));
 
     // lane l holds column l % 32; register v holds row 8 * (v / 4) + 4 * (l / 32) + v % 4
     if (a.parts > 1u) {

@@ -347,9 +347,10 @@ gemv_any_multi_kernel(const BodyArgs a) {
             }
     };
     float acc[G][NT][4];
-    // The sums of a chain of matrix instructions, before anything reads them.  With a branch right behind the last instruction of a
-    // chain the sums were seen to lack its products, although the instructions in between outlast its passes; so no branch follows
-    // one here, and every chain ends with independent cycles.
+    // The sums of a chain of matrix instructions, before anything reads them.  A result must not be read for 8 wait states, which the
+    // hardware does not enforce and the compiler leaves; but where a branch follows the last instruction of a chain, the
+    // compiler counts the wait states of the code that falls through, and a read at the branch's target came one wait state behind
+    // the instruction: the sums lacked its products.  So a chain ends with its wait states, in front of any branch.
     auto settle = [](f32x4& v) { asm volatile("s_nop 7" : "+v"(v)); };
     // one block of 16 rows into acc[g]; spare: a wavefront that has a block less than the others
     auto multiply = [&](int xs, int g, bool spare) {
@@ -505,7 +506,7 @@ gemv_any_multi_kernel(const BodyArgs a) {
     // the step after (part, run, i)
     uint32_t chunk_begin = 0, chunk_end = a.chunk < ngroups ? a.chunk : ngroups;
     struct At { uint32_t part, run, i, cb, ce; };
-    auto after = [&](At p) {                                               // selects only: see settle
+    auto after = [&](At p) {                                               // selects: the walk is on the way of every step
         const bool turn = p.i + 1u >= iters, done = turn & (p.run + G >= p.ce), over = done & (p.part + 1u >= a.parts);
         const uint32_t cb = over ? (p.ce < ngroups ? p.ce : 0u) : p.cb, far = cb + a.chunk < ngroups ? cb + a.chunk : ngroups;
         return At{over ? 0u : done ? p.part + 1u : p.part, done ? cb : turn ? p.run + G : p.run, turn ? 0u : p.i + 1u, cb, over ? far : p.ce};
