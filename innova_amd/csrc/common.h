@@ -155,9 +155,9 @@ size_t gemv_any_multi_bytes(const oilhip_weights& w, int M);
 int gemv_f32(const oilhip_weights& w, const float* d_x, float* d_y, int M, hipStream_t s, uint8_t* d_pack);
 int check_workspace(const oilhip_weights& w, int M, const void* d_ws, size_t ws_bytes);
 // widest row that these kernels take and the bytes of packed activations that any pass needs (d_pack, or stream scratch): per
-// block 32 floats (powers of two) and three digits of 256 activations for 32 tokens, or 48 floats and 27 KB of FP16 pieces
+// block 32 floats (powers of two) and four digits of 256 activations for 32 tokens, or 48 floats and 27 KB of FP16 pieces
 constexpr uint32_t kGemvPackMaxCols = 32768;
-constexpr size_t kGemvPackBytes = (size_t)(kGemvPackMaxCols >> 8) * (192u + 27648u);
+constexpr size_t kGemvPackBytes = (size_t)(kGemvPackMaxCols >> 8) * (192u + 32768u);
 // rows that mix formats, stored tile by tile and format by format
 int launch_gemv_seg(const oilhip_weights& w, const float* d_x, float* d_y, int M, hipStream_t s);
 // every format, a lane per run of 32 weights

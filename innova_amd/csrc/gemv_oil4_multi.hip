@@ -7,21 +7,26 @@
 // -128, and level q < 8 is minus level 15 - q.  So a code becomes its two digits without a table in memory: three bits
 // of four codes at a time select bytes of an 8-byte table held in two registers (v_perm_b32), and the sign is applied to
 // the four bytes at once (x ^ m) + (m & 1) (v_xad_u32; no carry crosses bytes because no digit is 0): 17 vector instructions
-// per dword of eight codes.  An activation is scaled by a power of two per (token, block of 256) and rounded to three
-// signed bytes (|X| < 127.5 * 2^16, so the rounding is 2^-23 to 2^-24 of the block's largest magnitude); sums over a block
-// are exact in INT32, then scaled in FP32 by the block's FP16 scale and the power of two.  v_mfma_i32_16x16x64_i8 takes the
+// per dword of eight codes.  An activation is scaled by a power of two per (token, block of 256) and rounded to four
+// signed bytes (|X| < 127.5 * 2^24: the rounding is 2^-31 to 2^-32 of the block's largest magnitude, and values from a 128th of it on are
+// exact); sums over a block are exact in INT32, then scaled in FP32 by the block's FP16 scale and the power of two.
+// Three bytes would leave 23 bits of the largest value to all of them: with one activation of 1000 among ordinary ones in every block,
+// an error of 6e-7 instead of 1e-7 with FP16 pairs or four bytes.  v_mfma_i32_16x16x64_i8 takes the
 // activations as its rows and 16 weight rows as its columns, so a lane's outputs belong to one weight row and meet one scale.
 //
 // A wavefront takes every n-th block of the row for a run of 16-row groups; the activations of its block sit in registers
 // and serve every group of the run, and the wavefronts' sums meet in LDS once per run.  There is no table to build, nothing
 // is summed across workgroups, and the order of every sum is fixed.
-// What bounds it: vector issue (about 170 instructions per block of 16 rows, beside 16 to 20 matrix instructions that other
-// wavefronts overlap) on the tall shapes, launch and round trips on the small ones.
-// Before (FP16 halves of levels from a 64 KB LDS table, K cut between workgroups) -> now, pre-pass included:
-//   11008 x 4096, 4 / 8 / 16 / 32 tokens: 13.4 / 13.9 / 16.0 / 21.1 us -> 12.1 / 13.5 / 14.8 / 19.0 us
-//   4096 x 11008, 4 / 16 tokens: 18.0 / 20.6 us -> 14.0 / 18.6 us
-//   131072 x 4096, 4 / 16 tokens: 67 / 82 us -> 60 / 76 us;  30000 x 14336, 16 / 32 tokens: 80 / 121 us -> 74 / 114 us
-//   2838 x 512, 5 tokens: 9.0 -> 6.8 us
+// What bounds it: up to 8 tokens vector issue (about 170 instructions per block of 16 rows, beside 8 to 16 matrix instructions that
+// other wavefronts overlap) on the tall shapes, launch and round trips on the small ones; above, the activations' way into the compute
+// unit: 16 KB per block and 16 tokens at about 30 bytes per clock, once per workgroup (at three digits, 12 KB, 4096 x 11008 took
+// 17.6 us with 16 tokens and 24.8 with 32).
+// Before (FP16 halves of levels from a 64 KB LDS table, K cut between workgroups) -> now, pre-pass included, weights from memory:
+//   11008 x 4096, 4 / 8 / 16 / 32 tokens: 12.8 / 12.5 / 14.3 / 19.7 us -> 11.6 / 12.8 / 14.8 / 20.0 us
+//   4096 x 11008: 17.0 / 17.5 / 19.8 / 25.1 us -> 13.2 / 15.7 / 20.4 / 30.6 us
+//   131072 x 4096, 4 / 16 / 32 tokens: 81 / 86 / 127 us -> 72 / 90 / 134 us;  30000 x 14336: 77 / 81 / 120 us -> 68 / 83 / 130 us
+//   2838 x 512, 5 / 16 / 32 tokens: 7.5 / 8.7 / 9.3 -> 5.1 / 5.7 / 7.0 us
+// Error against 64 bits (2-norm): 1.8e-7 -> 0.9e-7, whatever the distribution of the activations.
 #include <hip/hip_fp16.h>
 
 #include <algorithm>
@@ -39,15 +44,15 @@ using namespace oil4;
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 
 // Passes by token count.  The activation operand of one matrix instruction has 16 rows.  Few: up to four tokens, their
-// three digits side by side (row 4 t + d is digit d of token t), so two instructions (digits a and b of the weights) give all six
-// products.  Digits: 16 tokens per tile and a tile of rows per digit; five instructions, the product of the two lowest
-// digits is left out (it is below 2^-22 of the result's scale).  NT tiles of tokens share the decoded weights.
+// four digits side by side (row 4 t + d is digit d of token t), so two instructions (digits a and b of the weights) give all eight
+// products.  Digits: 16 tokens per tile and a tile of rows per digit; seven instructions, the product of the two lowest
+// digits is left out (2^-31 of the result's scale).  NT tiles of tokens share the decoded weights.
 enum PassKind { kFew4 = 0, kFew8 = 1, kDigits16 = 2, kDigits32 = 3, kPassKinds = 4 };
 __host__ __device__ constexpr bool kind_few(int k) { return k < 2; }
 __host__ __device__ constexpr int kind_tiles(int k) { return (k & 1) + 1; }
 __host__ __device__ constexpr uint32_t kind_tokens(int k) { return k == 0 ? 4u : k == 1 ? 8u : k == 2 ? 16u : 32u; }
 // packed bytes of one block: 1 KB pieces (64 lanes x 16 bytes), four per tile and operand (half of the block x even / odd nibbles)
-__host__ __device__ constexpr uint32_t kind_block_bytes(int k) { return (kind_few(k) ? 4096u : 12288u) * (uint32_t)kind_tiles(k); }
+__host__ __device__ constexpr uint32_t kind_block_bytes(int k) { return (kind_few(k) ? 4096u : 16384u) * (uint32_t)kind_tiles(k); }
 inline int kind_of(int tokens) { return tokens <= 4 ? kFew4 : tokens <= 8 ? kFew8 : tokens <= 16 ? kDigits16 : kDigits32; }
 
 // blocks of activations that a wavefront holds: as many as the registers take
@@ -60,8 +65,7 @@ constexpr uint32_t kMaxKeep = 48u * 1024u;                                 // by
 
 // ---- pre-pass: activations to digits in operand order -----------------------------------------------------------------
 // A wavefront takes one (token, block): 256 columns as one 16-byte load per lane, optionally silu(x) * x2 or the RMSNorm's
-// x * (1 + w) (whose 1 / rms joins the power of two that the main kernel undoes), the largest magnitude, the digits by
-// nibble position in LDS, and 48 16-byte pieces out.  Column i of a block sits at nibble p = 4 + i - i / 64 (columns 63,
+// x / rms * (1 + w), the largest magnitude, the digits by nibble position in LDS, and 64 16-byte pieces out.  Column i of a block sits at nibble p = 4 + i - i / 64 (columns 63,
 // 127, 191, 255 meet empty slots and nibbles 0..3 the block's scale: both see activation 0).
 // Several batches in one launch (the experts of a mixture-of-experts step): batch j packs M[j] rows of x into
 // xp + xp_off[j]; its rows are list[row0[j] + m] when use_list is set, else row0[j] + m.  The list travels by value with
@@ -79,8 +83,7 @@ struct PackJobs {
 // where a batch's powers of two start (floats [block][kMaxTokens]) and its packed blocks after them
 __host__ __device__ constexpr uint32_t undo_bytes(uint32_t bpr) { return bpr * (uint32_t)kMaxTokens * 4u; }
 
-// What the rows are multiplied as: x, silu(x) * x2, or x * (1 + norm_w) / rms(x) (the 1 / rms joins the power of two that is
-// undone on the sums).
+// What the rows are multiplied as: x, silu(x) * x2, or x * (1 + norm_w) / rms(x).
 struct Activations {
     const float *x, *x2, *norm_w;
     float* xn;                  // with norm_w: the normalised rows go here as well (optional, laid out like x)
@@ -95,8 +98,8 @@ struct PackArgs {
     int M, kind;
 };
 
-// this lane's four columns of block `blk` of row `src`, and 1 / rms (1 without a norm)
-__device__ __forceinline__ void load_activations(const Activations& a, uint32_t src, uint32_t blk, uint32_t bpr, uint32_t lane, float (&v)[4], float& rms) {
+// this lane's four columns of block `blk` of row `src`
+__device__ __forceinline__ void load_activations(const Activations& a, uint32_t src, uint32_t blk, uint32_t bpr, uint32_t lane, float (&v)[4]) {
     const float* row = a.x + (size_t)src * a.ldx;
     const float* p = row + 256u * blk + 4u * lane;
     auto load = [&](const float* q, float (&o)[4]) {
@@ -104,7 +107,6 @@ __device__ __forceinline__ void load_activations(const Activations& a, uint32_t 
         else { for (int e = 0; e < 4; ++e) o[e] = q[e]; }
     };
     load(p, v);
-    rms = 1.0f;
     if (a.x2) {
         float u[4];
         load(a.x2 + (p - a.x), u);
@@ -121,19 +123,19 @@ __device__ __forceinline__ void load_activations(const Activations& a, uint32_t 
                 s += b + i < bpr ? (f[i][0] * f[i][0] + f[i][1] * f[i][1]) + (f[i][2] * f[i][2] + f[i][3] * f[i][3]) : 0.0f;
         }
         for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-        rms = 1.0f / sqrtf(s / (float)(256u * bpr) + 1e-6f);
-        for (int e = 0; e < 4; ++e) v[e] *= 1.0f + a.norm_w[256u * blk + 4u * lane + e];
+        const float r = 1.0f / sqrtf(s / (float)(256u * bpr) + 1e-6f);
+        for (int e = 0; e < 4; ++e) v[e] = v[e] * r * (1.0f + a.norm_w[256u * blk + 4u * lane + e]);
         if (a.xn) {
             float* o = a.xn + (size_t)src * a.ldx + 256u * blk + 4u * lane;
-            for (int e = 0; e < 4; ++e) o[e] = v[e] * rms;
+            for (int e = 0; e < 4; ++e) o[e] = v[e];
         }
     }
 }
 
 // A block's 256 columns (four per lane) to digits: put(e, p, bytes) receives for column e of the lane its nibble p and the digits
-// as bytes 0 (low), 1, 2 (high).  Returns what undoes the scaling.  Uniform over the wavefront.
+// as bytes 0 (low) to 3.  Returns what undoes the scaling.  Uniform over the wavefront.
 template <class Put>
-__device__ __forceinline__ float block_to_digits(float (&v)[4], float rms, uint32_t lane, Put&& put) {
+__device__ __forceinline__ float block_to_digits(float (&v)[4], uint32_t lane, Put&& put) {
     if ((lane & 15u) == 15u) v[3] = 0.0f;                                  // column 64 n + 63: no weight there
     // the largest magnitude as a bit pattern: infinities and NaN are the largest of all
     uint32_t top = 0;
@@ -146,17 +148,17 @@ __device__ __forceinline__ float block_to_digits(float (&v)[4], float rms, uint3
     top = max(max((uint32_t)__builtin_amdgcn_readlane((int)top, 0), (uint32_t)__builtin_amdgcn_readlane((int)top, 16)),
               max((uint32_t)__builtin_amdgcn_readlane((int)top, 32), (uint32_t)__builtin_amdgcn_readlane((int)top, 48)));
     const bool bad = top >= 0x7F800000u;
-    // the power of two that brings the largest magnitude to [2^22, 2^23), one less where its top digit would pass 127 (a
-    // mantissa above 8355711 / 2^22 = 1 + 0x7EFEFE / 2^23); subnormal magnitudes count as 2^-127
-    int ex = 22 - ((int)(top >> 23) - 127) - ((top & 0x7FFFFFu) > 0x7EFEFEu ? 1 : 0);
+    // the power of two that brings the largest magnitude to [2^30, 2^31), one less where its top digit would pass 127 (above
+    // 0x7F7F7F7F, a mantissa above 0x7EFEFE); magnitudes below 2^-119 go lower, so that the power that undoes it stays a float
+    int ex = 30 - ((int)(top >> 23) - 127) - ((top & 0x7FFFFFu) > 0x7EFEFEu ? 1 : 0);
     ex = top == 0u || bad ? 0 : ex > 149 ? 149 : ex;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         const uint32_t i = 4u * lane + (uint32_t)e, p = 4u + i - (i >> 6);
         const int X = bad ? 0 : (int)rintf(ldexpf(v[e], ex));
-        if ((i & 63u) != 63u) put(e, p, (uint32_t)(X + 0x808080) ^ 0x808080u);   // signed digits: the bytes of X + 128 (1 + 2^8 + 2^16), less 128 each
+        if ((i & 63u) != 63u) put(e, p, ((uint32_t)X + 0x80808080u) ^ 0x80808080u);   // signed digits: the bytes of X + 128 (1 + 2^8 + 2^16 + 2^24), less 128 each
     }
-    return bad ? __uint_as_float(0x7FC00000u) : ldexpf(rms, -ex);
+    return bad ? __uint_as_float(0x7FC00000u) : ldexpf(1.0f, -ex);
 }
 
 __global__ void __launch_bounds__(256)
@@ -176,18 +178,17 @@ pack_digits_kernel(PackArgs a, const PackJobs jobs) {
     const uint32_t blk = bid % a.bpr, t = (bid / a.bpr) * 4u + wave;
     uint32_t src = 0xFFFFFFFFu;
     if ((int)t < a.M) src = jobs.n ? (jobs.use_list ? (uint32_t)jobs.list[row0 + t] : (uint32_t)row0 + t) : a.tok ? (uint32_t)a.tok[t] : t;
-    float v[4] = {0.0f, 0.0f, 0.0f, 0.0f}, rms = 1.0f;
-    if (src < a.xrows) load_activations(a.in, src, blk, a.bpr, lane, v, rms);
+    float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (src < a.xrows) load_activations(a.in, src, blk, a.bpr, lane, v);
     // digit d of nibble p at byte d * 256 + ((2 (p / 128) + p % 2) * 4 + (p / 32) % 4) * 16 + (p % 32) / 2: 16-byte pieces by (operand, lane group)
     uint8_t* mine = lds[wave];
     if (lane < 4u) {
         const uint32_t at = (lane & 1u) * 64u + (lane >> 1);
-        mine[at] = 0; mine[256u + at] = 0; mine[512u + at] = 0;
+        mine[at] = 0; mine[256u + at] = 0; mine[512u + at] = 0; mine[768u + at] = 0;
     }
-    reinterpret_cast<uint32_t*>(mine + 768)[lane] = 0u;                    // the fourth row of a Few tile's token
-    const float undo = block_to_digits(v, rms, lane, [&](int, uint32_t p, uint32_t bytes) {
+    const float undo = block_to_digits(v, lane, [&](int, uint32_t p, uint32_t bytes) {
         const uint32_t at = (((p >> 7) * 2u + (p & 1u)) * 4u + ((p >> 5) & 3u)) * 16u + ((p & 31u) >> 1);
-        mine[at] = (uint8_t)bytes; mine[256u + at] = (uint8_t)(bytes >> 8); mine[512u + at] = (uint8_t)(bytes >> 16);
+        mine[at] = (uint8_t)bytes; mine[256u + at] = (uint8_t)(bytes >> 8); mine[512u + at] = (uint8_t)(bytes >> 16); mine[768u + at] = (uint8_t)(bytes >> 24);
     });
     const uint32_t tokens = kind_few(a.kind) ? 4u : 16u, tile = t / tokens, tt = t - tile * tokens;
     if (lane == 0) reinterpret_cast<float*>(a.xp)[blk * (uint32_t)kMaxTokens + t] = undo;
@@ -199,7 +200,7 @@ pack_digits_kernel(PackArgs a, const PackJobs jobs) {
     const uint4 piece = *reinterpret_cast<const uint4*>(mine + 16u * lane);
     uint8_t* o = a.xp + undo_bytes(a.bpr) + (size_t)blk * kind_block_bytes(a.kind);
     if (kind_few(a.kind)) *reinterpret_cast<uint4*>(o + tile * 4096u + op * 1024u + (kq * 16u + tt * 4u + d) * 16u) = piece;
-    else if (d < 3u) *reinterpret_cast<uint4*>(o + tile * 12288u + (d * 4u + op) * 1024u + (kq * 16u + tt) * 16u) = piece;
+    else *reinterpret_cast<uint4*>(o + tile * 16384u + (d * 4u + op) * 1024u + (kq * 16u + tt) * 16u) = piece;
 }
 
 // ---- main kernel --------------------------------------------------------------------------------------------------
@@ -247,7 +248,7 @@ __device__ __forceinline__ void decode_four(uint32_t w, int& a, int& b) {
 
 template <int KIND>
 struct Sums {                                                              // one block's integer sums of one token tile
-    static constexpr int N = kind_few(KIND) ? 2 : 3;
+    static constexpr int N = kind_few(KIND) ? 2 : 4;
     i32x4 s[N];
     __device__ __forceinline__ void clear() {
 #pragma unroll
@@ -273,7 +274,7 @@ template <int KIND, int G>
 __device__ __forceinline__ void
 multi_body(const BodyArgs& a, uint32_t g_begin, uint32_t g_end, float* red) {
     constexpr bool FEW = kind_few(KIND);
-    constexpr int NT = kind_tiles(KIND), PER = FEW ? 1 : 4, DIG = FEW ? 1 : 3;   // outputs of a lane per tile, operand pieces per half and parity
+    constexpr int NT = kind_tiles(KIND), PER = FEW ? 1 : 4, DIG = FEW ? 1 : 4;   // outputs of a lane per tile, operand pieces per half and parity
     constexpr int XD = x_slots(KIND);
     constexpr int WD = G < 3 ? XD : 1;                                     // weights in flight: the run's, for short runs of all blocks of the part
     const uint32_t lane = threadIdx.x & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), waves = blockDim.x >> 6;
@@ -382,27 +383,30 @@ multi_body(const BodyArgs& a, uint32_t g_begin, uint32_t g_end, float* red) {
                     if constexpr (FEW) {
                         sum[t].s[0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[XS][t][0][o], da, sum[t].s[0], 0, 0, 0);
                         sum[t].s[1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[XS][t][0][o], db, sum[t].s[1], 0, 0, 0);
-                    } else {                                               // digits of the activations: [0] low, [1] middle, [2] high
+                    } else {                                               // digits of the activations: [0] low to [3] high
                         // (an order in which no instruction waits for the one before the last)
-                        sum[t].s[1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[XS][t][2][o], db, sum[t].s[1], 0, 0, 0);     // 2^16
-                        sum[t].s[2] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[XS][t][0][o], da, sum[t].s[2], 0, 0, 0);     // 2^8
-                        sum[t].s[0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[XS][t][2][o], da, sum[t].s[0], 0, 0, 0);     // 2^24
-                        sum[t].s[1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[XS][t][1][o], da, sum[t].s[1], 0, 0, 0);
-                        sum[t].s[2] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[XS][t][1][o], db, sum[t].s[2], 0, 0, 0);
+                        sum[t].s[1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[XS][t][3][o], db, sum[t].s[1], 0, 0, 0);     // 2^24
+                        sum[t].s[2] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[XS][t][2][o], db, sum[t].s[2], 0, 0, 0);     // 2^16
+                        sum[t].s[3] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[XS][t][1][o], db, sum[t].s[3], 0, 0, 0);     // 2^8
+                        sum[t].s[0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[XS][t][3][o], da, sum[t].s[0], 0, 0, 0);     // 2^32
+                        sum[t].s[1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[XS][t][2][o], da, sum[t].s[1], 0, 0, 0);
+                        sum[t].s[2] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[XS][t][1][o], da, sum[t].s[2], 0, 0, 0);
+                        sum[t].s[3] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[XS][t][0][o], da, sum[t].s[3], 0, 0, 0);
                     }
                 }
             }
             load_w(WS, g, npart, nrun, ni);
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
-                if constexpr (FEW) {                                       // element d is digit d of this lane's token: at most 252 * 127 * 27178 < 2^30
-                    const float f = fmaf((float)(sum[t].s[0][2] * 256 + sum[t].s[1][2]), 65536.0f,
-                                         fmaf((float)(sum[t].s[0][1] * 256 + sum[t].s[1][1]), 256.0f, (float)(sum[t].s[0][0] * 256 + sum[t].s[1][0])));
+                if constexpr (FEW) {                                       // element d is digit d of this lane's token: at most 252 * 128 * 27178 < 2^30
+                    const float f = fmaf((float)(sum[t].s[0][3] * 256 + sum[t].s[1][3]), 16777216.0f, fmaf((float)(sum[t].s[0][2] * 256 + sum[t].s[1][2]), 65536.0f,
+                                         fmaf((float)(sum[t].s[0][1] * 256 + sum[t].s[1][1]), 256.0f, (float)(sum[t].s[0][0] * 256 + sum[t].s[1][0]))));
                     acc[g][t][0] = fmaf(f * un[XS][t][0], scale, acc[g][t][0]);
                 } else {
 #pragma unroll
                     for (int v = 0; v < PER; ++v) {
-                        const float f = fmaf((float)(sum[t].s[0][v] * 256 + sum[t].s[1][v]), 256.0f, (float)sum[t].s[2][v]);
+                        // below 252 (128 * 128 + 128 * 106) (256 + 1) < 2^31
+                        const float f = fmaf((float)(sum[t].s[0][v] * 256 + sum[t].s[1][v]), 65536.0f, (float)(sum[t].s[2][v] * 256 + sum[t].s[3][v]));
                         acc[g][t][v] = fmaf(f * un[XS][t][v], scale, acc[g][t][v]);
                     }
                 }

@@ -13,7 +13,7 @@ int launch_gemv_seg_rmsnorm(const oilhip_weights& w, const float* d_x, const flo
 
 namespace {
 
-// Several rows of an OIL4 tensor: the norm is formed while the activations are packed, where every wavefront (one token, one
+// Three rows and more of an OIL4 tensor: the norm is formed while the activations are packed, where every wavefront (one token, one
 // block) reads its whole row from L2, and saves a launch of 3 us.  The reading grows with the square of the width: a layer
 // with 5 rows of 2816 takes 48.0 us instead of 52.7 (SwiGLU formed there as well), 32 rows of 8192 144.8 instead of 146.8, 32
 // rows of 16384 322 instead of 315.
@@ -101,7 +101,8 @@ int gemv_rmsnorm(const oilhip_weights& w, const float* d_x, const float* d_normw
     if (!d_xn) return fail(OILHIP_E_ARG, "gemv_rmsnorm: this shape needs the d_xn workspace");
     const uintptr_t x0 = reinterpret_cast<uintptr_t>(d_x), xn0 = reinterpret_cast<uintptr_t>(d_xn), size = (uintptr_t)M * w.cols * 4u;
     const bool apart = x0 + size <= xn0 || xn0 + size <= x0;               // packing wavefronts read whole rows while others store theirs
-    if (M > 1 && plain_oil4(w) && w.cols <= kPackNormMaxCols && apart) {   // the norm rides on the packing of the activations
+    // (two rows go through the register kernel below, which multiplies in FP32 and lets infinities through)
+    if (M > 2 && plain_oil4(w) && w.cols <= kPackNormMaxCols && apart) {   // the norm rides on the packing of the activations
         const int rc = launch_gemv_oil4_multi(w, d_x, nullptr, d_y, M, (uint32_t)w.cols, (uint32_t)w.rows, (uint32_t)M, s,
                                               MultiInput{nullptr, d_normw, false, d_xn}, nullptr, nullptr, 0, d_pack);
         if (rc <= 0) return rc;
@@ -129,7 +130,7 @@ int mlp_step(const oilhip_weights& gate_up, const oilhip_weights& down, const fl
         const int rc = launch_gemv_seg_swiglu(down, h2, d_y, s);
         if (rc <= 0) return rc;
     }
-    if (M > 1 && plain_oil4(down)) {                         // SwiGLU formed while the activations are packed
+    if (M > 2 && plain_oil4(down)) {                         // SwiGLU formed while the activations are packed
         const int rc = launch_gemv_oil4_multi(down, h2, nullptr, d_y, M, (uint32_t)(2 * F), (uint32_t)down.rows, (uint32_t)M, s,
                                               MultiInput{h2 + F, nullptr, true}, nullptr, nullptr, 0, d_pack);
         if (rc <= 0) return rc;

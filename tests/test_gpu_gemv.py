@@ -247,7 +247,7 @@ def test_shape_errors():
             dw.gemv(torch.zeros(1, w.size, device="cuda"))        # ragged block: matmul refuses
 
 
-# The multi-row kernel splits activations into two FP16 parts after scaling each token row by a power of two, so its
+# The multi-row kernel cuts activations into four digits after scaling each block of a row by a power of two, so its
 # accuracy must not depend on the magnitude of the activations: tiny rows, huge rows (beyond the FP16 range), rows that
 # mix magnitudes, a zero row, and tokens of very different scale in one batch.
 @pytest.mark.parametrize("rows,cols,M", [(130, 4096, 5), (61, 11008, 16), (300, 2048, 24)])
@@ -330,6 +330,29 @@ def test_other_formats_several_rows(fmt, rows, cols, tokens):
                     size = np.linalg.norm(X[m].astype(np.float64)) * rms * np.sqrt(n)       # of outputs without cancellation
                     err = np.linalg.norm(got[m, r:r + n].astype(np.float64) - want[m, :n])
                     assert err <= TOL * max(np.linalg.norm(want[m, :n]), size), (M, m, r)
+
+
+# The error of an output is that of FP32 sums whatever the activations look like: the operands must not cost more than the sums.
+# Activations of one large value among ordinary ones (every block of 256), of heavy tails, and Gaussian ones; per token the error
+# against 64 bits in the 2-norm.  Bound: an output adds at most 43 block sums with three roundings each, at most
+# 2^-24 of partial sums that grow to the output's size: sqrt(3 * 43 / 3) * 2^-24 / sqrt(3) = 2.3e-7 if all were that large.
+@pytest.mark.parametrize("rows,cols", [(512, 4096), (300, 11008)])
+@pytest.mark.parametrize("M", [3, 8, 16, 32])
+def test_oil4_multi_token_error_of_uneven_activations(rows, cols, M):
+    payload, blocks = ia.block_codec.quantize_tensor(gaussian_weights(rows * cols, M), ia.Format.OIL4)
+    rng = np.random.default_rng(M)
+    with ia.DeviceWeights.from_blocks(payload, blocks, rows, cols) as dw:
+        W = dw.dequant().view(rows, cols).double()
+        for kind in ("gauss", 30.0, 100.0, 1000.0, 10000.0, "tails"):
+            x = rng.standard_normal((M, cols)).astype(np.float32)
+            if kind == "tails":
+                x = (np.sign(x) * np.exp(1.5 * rng.standard_normal((M, cols)))).astype(np.float32)
+            elif kind != "gauss":
+                x.reshape(M, -1, 256)[:, :, 17] = kind * np.where(rng.random((M, cols // 256)) < 0.5, -1.0, 1.0)
+            xd = torch.from_numpy(x).cuda()
+            want = xd.double() @ W.T
+            err = (dw.gemv(xd).double() - want).norm(dim=1) / want.norm(dim=1)
+            assert float(err.max()) <= 2.3e-7, (kind, err.max())
 
 
 # The digits of a block's largest magnitude: mantissas on both sides of the one above which the block takes a power of two less (its
