@@ -633,7 +633,11 @@ int oilhip_gemv_f32_general(const oilhip_weights* w, const float* d_x, float* d_
 
 static int prefill(const oilhip_weights* w, const void* d_x, bool x_is_f32, float* d_y, int M, hipStream_t s) {
     if (int rc = check_matmul_shape(w, d_x, d_y, M)) return rc;
-    if (plain_oil4(*w)) return launch_gemm_oil4_frag(*w, d_x, x_is_f32, d_y, M, s);
+    // The fragment-order kernel rounds an OIL4 level to FP16 before it multiplies and rounds to bf16.  Activations that are not 16-byte
+    // aligned never took it and keep weights that are rounded once, as far as the other kernel's 32-bit offsets reach.
+    const bool aligned = (reinterpret_cast<uintptr_t>(d_x) & 15u) == 0u;
+    if (plain_oil4(*w) && (aligned || (uint64_t)M * w->cols * 2u >= 0x80000000ull || w->cols * 512u >= 0x80000000ull))
+        return launch_gemm_oil4_frag(*w, d_x, x_is_f32, d_y, M, s);
     const int rc = launch_gemm_any(*w, d_x, x_is_f32, d_y, M, s);
     if (rc == 1) return fail(OILHIP_E_ARG, "bf16 prefill GEMM needs full blocks with the channel sizes the quantizer writes");
     return rc;

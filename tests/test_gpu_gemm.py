@@ -54,8 +54,9 @@ def test_fragment_kernel_edges(rows, cols, M):
 
 @pytest.mark.parametrize("M", [300, 64])
 def test_fragment_kernel_takes_misaligned_activations_another_way(M):
-    """An activation pointer that is not 16-byte aligned cannot use the kernel's 16-byte loads: same result through
-    the older paths (the pipelined kernel above 256 tokens, the 128 x 128 tiles below)."""
+    """Activations that are not 16-byte aligned go through the dense-operand kernel, bf16 and FP32 alike: its weights are the
+    dequantized values rounded once to bf16 (the fragment-order kernel holds levels as FP16), so only the FP32 sums differ from the
+    product in 64 bits."""
     rows, cols = 256, 512
     w = gaussian_weights(rows * cols, 21)
     payload, blocks = ia.block_codec.quantize_tensor(w, ia.Format.OIL4)
@@ -68,10 +69,16 @@ def test_fragment_kernel_takes_misaligned_activations_another_way(M):
         ya = dw.gemm_bf16(xa)
         ym = torch.empty(M, rows, device="cuda")
         ia._lib.check(L.oilhip_gemm_bf16(dw.handle, xm.data_ptr(), ym.data_ptr(), M, ia._lib.current_stream()))
+        yf, base32 = torch.empty(M, rows, device="cuda"), torch.empty(M * cols + 1, device="cuda")
+        xf = base32[1:].view(M, cols)
+        xf.copy_(xm)
+        ia._lib.check(L.oilhip_gemm_f32(dw.handle, xf.data_ptr(), yf.data_ptr(), M, ia._lib.current_stream()))
+        once = xm.double() @ dw.dequant().view(rows, cols).to(torch.bfloat16).double().T
+    assert torch.equal(ym, yf)
+    assert rel_l2(ym.cpu().numpy(), once.cpu().numpy()) <= 1e-6
     X = xm.float().cpu().numpy()
     want = O.block_gemm(payload, to_orc_blocks(blocks), rows, cols, X, wide=True)
     assert rel_l2(ym.cpu().numpy(), want) <= TOL
-    # the two kernels round the same products (levels held as FP32 there, as FP16 here): they agree far inside the bound
     ya2 = O.block_gemm(payload, to_orc_blocks(blocks), rows, cols, xa.float().cpu().numpy(), wide=True)
     assert rel_l2(ya.cpu().numpy(), ya2) <= TOL
 
