@@ -56,7 +56,7 @@ __host__ __device__ constexpr uint32_t tile_bytes(bool grp) { return (grp ? 9u :
 // ---- pre-pass --------------------------------------------------------------------------------------------------------
 struct PackArgs {
     const float* x;
-    uint8_t* xp;            // powers of two [block][16 NT] floats, then the operands [block][tile][step][lane][8 halves]
+    uint8_t* xp;            // powers of two [block][16 NT] floats, one block of zeros, then the operands [block][tile][step][lane][8 halves]
     uint32_t ldx, bpr, tiles, grp, aligned;
     int M;
 };
@@ -94,17 +94,42 @@ pack_pieces_kernel(const PackArgs a) {
         sum += f;
         cut(f, h[0][e], h[1][e], h[2][e]);
     }
-    const float undo = bad ? __uint_as_float(0x7FC00000u) : ldexpf(1.0f, -ex);
+    float undo[3];
+    undo[0] = undo[1] = undo[2] = bad ? __uint_as_float(0x7FC00000u) : ldexpf(1.0f, -ex);
     uint32_t step, kq;
     if (a.grp) { step = 2u * (lane >> 4) + ((lane & 3u) >> 1); kq = (lane & 15u) >> 2; }
     else { step = (lane & 15u) >> 1; kq = lane >> 4; }
-    uint8_t* base = a.xp + a.bpr * rows * 4u + (size_t)blk * a.tiles * tile_bytes(a.grp);
+    uint8_t* base = a.xp + (a.bpr + 1u) * rows * 4u + (size_t)blk * a.tiles * tile_bytes(a.grp);
     sum += oil4::dpp_quad_xor1(sum);
     sum += oil4::dpp_quad_xor2(sum);
     sum += oil4::dpp_half_mirror(sum);
     sum += oil4::dpp_row_mirror(sum);                                       // of the lane's group of 64 columns: below 2^21
     _Float16 g[3];
     cut(sum * 0x1p-6f, g[0], g[1], g[2]);
+    if (top == 0x7F800000u) {                                              // infinities, no NaN (uniform)
+        // Up to three of them: each is +-1 in a piece of its own, the rest of the block 0, and the piece's power of two is
+        // infinity, so that an output gets the infinity with its weight's sign (NaN of a zero weight), as in FP32.  More: NaN.
+        uint32_t before = 0;
+#pragma unroll
+        for (uint32_t e = 0; e < 4u; ++e) {
+            const bool here = (__float_as_uint(v[e]) & 0x7FFFFFFFu) == 0x7F800000u;
+            const uint64_t m = __ballot(here);
+            const uint32_t rank = before + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+#pragma unroll
+            for (uint32_t d = 0; d < 3u; ++d) h[d][e] = here && rank == d ? (_Float16)(v[e] > 0.0f ? 1.0f : -1.0f) : (_Float16)0.0f;
+            before += (uint32_t)__popcll(m);
+        }
+#pragma unroll
+        for (uint32_t d = 0; d < 3u; ++d) {
+            if (before <= 3u) undo[d] = d < before ? __builtin_inff() : 1.0f;
+            float s = ((float)h[d][0] + (float)h[d][1]) + ((float)h[d][2] + (float)h[d][3]);
+            s += oil4::dpp_quad_xor1(s);
+            s += oil4::dpp_quad_xor2(s);
+            s += oil4::dpp_half_mirror(s);
+            s += oil4::dpp_row_mirror(s);
+            g[d] = (_Float16)(s * 0x1p-6f);
+        }
+    }
 #pragma unroll
     for (uint32_t d = 0; d < 3u; ++d) {
         const uint32_t r = 3u * t + d;
@@ -117,7 +142,10 @@ pack_pieces_kernel(const PackArgs a) {
             const f16x2 s = f16x2{g[d], (_Float16)0.0f};
             *reinterpret_cast<uint4*>(tile + (8u * 64u + (lane >> 4) * 16u + (r & 15u)) * 16u) = make_uint4(__builtin_bit_cast(uint32_t, s), 0u, 0u, 0u);
         }
-        if (lane == 0) reinterpret_cast<float*>(a.xp)[blk * rows + r] = undo;
+        if (lane == 0) {
+            reinterpret_cast<float*>(a.xp)[blk * rows + r] = undo[d];
+            if (blk == 0) reinterpret_cast<float*>(a.xp)[a.bpr * rows + r] = 0.0f;
+        }
     }
 }
 
@@ -248,7 +276,7 @@ gemv_any_multi_kernel(const BodyArgs a) {
     const auto drs = __builtin_amdgcn_make_buffer_rsrc(const_cast<DevBlock*>(by_descriptor(S) ? a.blocks + (size_t)g_begin * 16u * bpr : nullptr), (short)0,
                                                        (int)0xFFFFFFFFu, 0x00020000);
     const float* undo = reinterpret_cast<const float*>(a.xp);
-    const uint8_t* xblocks = a.xp + bpr * ROWS * 4u;
+    const uint8_t* xblocks = a.xp + (bpr + 1u) * ROWS * 4u;
     auto place = [&](uint32_t part, uint32_t i) { const uint32_t b = wave + i * waves; return b < a.part_blocks ? part * a.part_blocks + b : 0xFFFFFFFFu; };
     auto block_at = [&](uint32_t part, uint32_t i) { const uint32_t b = place(part, i); return b < bpr ? b : bpr - 1u; };
 
@@ -336,13 +364,14 @@ gemv_any_multi_kernel(const BodyArgs a) {
 #pragma unroll
         for (int s = 0; s < XD; ++s)
             if (s == 0 || (uint32_t)s < iters) {
-                const uint32_t blk = block_at(part, (uint32_t)s);
+                // a wavefront that has a block less than the others takes the last one again, times 0
+                const uint32_t blk = block_at(part, (uint32_t)s), scale_of = place(part, (uint32_t)s) < bpr ? blk : bpr;
 #pragma unroll
                 for (int t = 0; t < NT; ++t) {
                     const f16x8* p = reinterpret_cast<const f16x8*>(xblocks + ((size_t)blk * NT + (uint32_t)t) * tile_bytes(grouped(S))) + lane;
 #pragma unroll
                     for (int k = 0; k < ST; ++k) x[s][t][k] = p[64 * k];
-                    un[s][t] = *reinterpret_cast<const f32x4*>(undo + blk * ROWS + 16u * (uint32_t)t + 4u * kq);
+                    un[s][t] = *reinterpret_cast<const f32x4*>(undo + scale_of * ROWS + 16u * (uint32_t)t + 4u * kq);
                 }
             }
     };
@@ -352,8 +381,9 @@ gemv_any_multi_kernel(const BodyArgs a) {
     // compiler counts the wait states of the code that falls through, and a read at the branch's target came one wait state behind
     // the instruction: the sums lacked its products.  So a chain ends with its wait states, in front of any branch.
     auto settle = [](f32x4& v) { asm volatile("s_nop 7" : "+v"(v)); };
-    // one block of 16 rows into acc[g]; spare: a wavefront that has a block less than the others
-    auto multiply = [&](int xs, int g, bool spare) {
+    // One block of 16 rows into acc[g].  The weights' factor meets the sum before the power of two does, so that no partial sum is
+    // larger than it would be in FP32.
+    auto multiply = [&](int xs, int g) {
         const uint32_t (&o)[N] = w[g];
         f32x4 sum[NT];
         if constexpr (!grouped(S)) {
@@ -394,13 +424,12 @@ gemv_any_multi_kernel(const BodyArgs a) {
 #pragma unroll
                 for (int t = 0; t < NT; ++t) sum[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x[xs][t][s], v, s ? sum[t] : zero, 0, 0, 0);
             }
-            factor = spare ? 0.0f : factor;
 #pragma unroll
             for (int t = 0; t < NT; ++t) settle(sum[t]);
 #pragma unroll
             for (int t = 0; t < NT; ++t)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) acc[g][t][e] = fmaf(sum[t][e] * un[xs][t][e], factor, acc[g][t][e]);
+                for (int e = 0; e < 4; ++e) acc[g][t][e] = fmaf(sum[t][e] * factor, un[xs][t][e], acc[g][t][e]);
         } else {
             // zero point (a 64th of it would do: the group sums are packed divided by 64) and scale of group kq, this lane's row
             const bool own = S != kSparkMix || fmt[g] != 7u;
@@ -469,11 +498,10 @@ gemv_any_multi_kernel(const BodyArgs a) {
                     for (int e = 0; e < 4; ++e) sum[t][e] = fmaf(part[t][e], factor[j], sum[t][e]);
                 __builtin_amdgcn_sched_barrier(0);                         // one group's weights in registers at a time
             }
-            const float on = spare ? 0.0f : 1.0f;
 #pragma unroll
             for (int t = 0; t < NT; ++t)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) acc[g][t][e] = fmaf(sum[t][e] * on, un[xs][t][e], acc[g][t][e]);
+                for (int e = 0; e < 4; ++e) acc[g][t][e] = fmaf(sum[t][e], un[xs][t][e], acc[g][t][e]);
         }
     };
     auto lds_barrier = [&]() {
@@ -532,10 +560,9 @@ gemv_any_multi_kernel(const BodyArgs a) {
 #pragma unroll
             for (int i = 0; i < XD; ++i)
                 if (i == 0 || (uint32_t)i < iters) {
-                    const bool spare = place(part, (uint32_t)i) >= bpr;
 #pragma unroll
                     for (int g = 0; g < G; ++g) {
-                        multiply(i, g, spare);
+                        multiply(i, g);
                         load_w(g, next.part, next.run, next.i);
                         load_desc(g, then.part, then.run, then.i);
                     }
@@ -638,7 +665,7 @@ size_t gemv_any_multi_bytes(const oilhip_weights& w, int M) {
     const int src = source_for(w, M);
     if (src < 0) return 0;
     const size_t tiles = (size_t)tiles_for(std::min(M, kPassTokens));
-    return (size_t)(w.cols >> 8) * tiles * (64u + tile_bytes(grouped(src)));
+    return tiles * (64u + (size_t)(w.cols >> 8) * (64u + tile_bytes(grouped(src))));
 }
 
 // Returns 1 where these kernels do not serve the call.  Without d_pack, a call that is being captured is left to the kernels that

@@ -45,7 +45,7 @@ typedef int i32x4 __attribute__((ext_vector_type(4)));
 
 // Passes by token count.  The activation operand of one matrix instruction has 16 rows.  Few: up to four tokens, their
 // four digits side by side (row 4 t + d is digit d of token t), so two instructions (digits a and b of the weights) give all eight
-// products.  Digits: 16 tokens per tile and a tile of rows per digit; seven instructions, the product of the two lowest
+// products.  Digits: 16 tokens per tile and a tile of rows per digit, seven instructions.  The product of the two lowest
 // digits is left out (2^-31 of the result's scale).  NT tiles of tokens share the decoded weights.
 enum PassKind { kFew4 = 0, kFew8 = 1, kDigits16 = 2, kDigits32 = 3, kPassKinds = 4 };
 __host__ __device__ constexpr bool kind_few(int k) { return k < 2; }
@@ -291,6 +291,8 @@ multi_body(const BodyArgs& a, uint32_t g_begin, uint32_t g_end, float* red) {
     auto place = [&](uint32_t part, uint32_t i) { const uint32_t b = wave + i * waves; return b < a.part_blocks ? part * a.part_blocks + b : 0xFFFFFFFFu; };
     auto block_at = [&](uint32_t part, uint32_t i) { const uint32_t b = place(part, i); return b < bpr ? b : bpr - 1u; };
 
+    // the levels' integer form (10^-4), and the 2^8 of the lowest digit product kept: a power of two with the scale, exactly, the rest at the end
+    constexpr float kScaleUnit = 0x1p-6f, kAccUnit = 1.6384f;
     u32x4 w[WD][G][2];
     auto load_w = [&](int slot, int g, uint32_t part, uint32_t run, uint32_t i) {
         uint32_t r = (run + (uint32_t)g) * 16u + li;
@@ -366,9 +368,10 @@ multi_body(const BodyArgs& a, uint32_t g_begin, uint32_t g_end, float* red) {
             Sums<KIND> sum[NT];
 #pragma unroll
             for (int t = 0; t < NT; ++t) sum[t].clear();
-            // the block's FP16 scale: the low half of the first dword of lane li
+            // the block's FP16 scale: the low half of the first dword of lane li.  It meets the integer sum before the power of two does: a
+            // partial sum is below the output's own size then and overflows where the output would (kAccUnit).  A spare block adds 0, or the NaN that its output has anyway.
             float scale = __half2float(__ushort_as_half((unsigned short)__builtin_amdgcn_ds_bpermute((int)scale_lane, (int)w[WS][g][0].x)));
-            scale = spare ? 0.0f : scale;
+            scale = spare ? 0.0f : scale * kScaleUnit;
 #pragma unroll
             for (int o = 0; o < 4; ++o) {                                  // operand: half o / 2 of the block, even or odd nibbles
                 i32x4 da, db;
@@ -398,16 +401,17 @@ multi_body(const BodyArgs& a, uint32_t g_begin, uint32_t g_end, float* red) {
             load_w(WS, g, npart, nrun, ni);
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
-                if constexpr (FEW) {                                       // element d is digit d of this lane's token: at most 252 * 128 * 27178 < 2^30
-                    const float f = fmaf((float)(sum[t].s[0][3] * 256 + sum[t].s[1][3]), 16777216.0f, fmaf((float)(sum[t].s[0][2] * 256 + sum[t].s[1][2]), 65536.0f,
-                                         fmaf((float)(sum[t].s[0][1] * 256 + sum[t].s[1][1]), 256.0f, (float)(sum[t].s[0][0] * 256 + sum[t].s[1][0]))));
-                    acc[g][t][0] = fmaf(f * un[XS][t][0], scale, acc[g][t][0]);
+                if constexpr (FEW) {                                       // element d is digit d of this lane's token
+                    // below 252 (128 * 27178 + 128 * 106) < 2^30; the product of the two lowest digits is left out here as well
+                    const float f = fmaf((float)(sum[t].s[0][3] * 256 + sum[t].s[1][3]), 65536.0f,
+                                         fmaf((float)(sum[t].s[0][2] * 256 + sum[t].s[1][2]), 256.0f, (float)(sum[t].s[0][1] * 256 + (sum[t].s[1][1] + sum[t].s[0][0]))));
+                    acc[g][t][0] = fmaf(f * scale, un[XS][t][0], acc[g][t][0]);
                 } else {
 #pragma unroll
                     for (int v = 0; v < PER; ++v) {
                         // below 252 (128 * 128 + 128 * 106) (256 + 1) < 2^31
                         const float f = fmaf((float)(sum[t].s[0][v] * 256 + sum[t].s[1][v]), 65536.0f, (float)(sum[t].s[2][v] * 256 + sum[t].s[3][v]));
-                        acc[g][t][v] = fmaf(f * un[XS][t][v], scale, acc[g][t][v]);
+                        acc[g][t][v] = fmaf(f * scale, un[XS][t][v], acc[g][t][v]);
                     }
                 }
             }
@@ -415,7 +419,6 @@ multi_body(const BodyArgs& a, uint32_t g_begin, uint32_t g_end, float* red) {
     };
     // the sums of a run, out of the area that all wavefronts have written
     auto finish = [&](uint32_t part, uint32_t run, const float* area) {
-        constexpr float unit = FEW ? 1e-4f : 256.0f * 1e-4f;               // the levels' integer form, and the 2^8 of the lowest digit product kept
         for (uint32_t o = threadIdx.x; o < OUT; o += blockDim.x) {
             float p[kMaxWaves];
 #pragma unroll
@@ -427,7 +430,7 @@ multi_body(const BodyArgs& a, uint32_t g_begin, uint32_t g_end, float* red) {
             const uint32_t l = o & 63u, e = o >> 6, v = e % PER, t = (e / PER) % NT, g = e / (PER * NT);
             const uint32_t token = FEW ? 4u * t + (l >> 4) : 16u * t + 4u * (l >> 4) + v;
             const uint32_t r = (g_begin + run + g) * 16u + (l & 15u);
-            if (run + g < ngroups && r < a.rows && (int)token < a.M) a.y[(size_t)token * a.ldy + r] = s * unit;
+            if (run + g < ngroups && r < a.rows && (int)token < a.M) a.y[(size_t)token * a.ldy + r] = s * kAccUnit;
         }
     };
     uint32_t odd = 0, done_part = 0, done_run = 0xFFFFFFFFu;

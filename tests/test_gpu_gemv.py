@@ -355,6 +355,53 @@ def test_oil4_multi_token_error_of_uneven_activations(rows, cols, M):
             assert float(err.max()) <= 2.3e-7, (kind, err.max())
 
 
+# Outputs near the end of the FP32 range: no partial sum may overflow before the output does (levels enter the products as 10^4 times
+# themselves), and a block that a wavefront takes again must not add anything (11 blocks on 6 wavefronts)
+@pytest.mark.parametrize("fmt", [(3,), (1,), (0, 1), (2,), (4,), (9,), (10,), (11,), (7, 9, 10, 11)])
+@pytest.mark.parametrize("M", [5, 12, 20])
+def test_several_rows_of_large_activations(fmt, M):
+    rows, cols = 40, 256 * 11
+    rng = np.random.default_rng(M)
+    payload, blocks = ia.block_codec.quantize_tensor(gaussian_weights(rows * cols, M), rng.choice(fmt, rows * cols // 256).astype(np.uint8))
+    x = torch.from_numpy((rng.standard_normal((M, cols)) * 1e36).astype(np.float32)).cuda()
+    with ia.DeviceWeights.from_blocks(payload, blocks, rows, cols) as dw:
+        W = dw.dequant().view(rows, cols).double()
+        x *= float(1e36 / (x.double() @ W.T).abs().max())        # the largest output is 1e36
+        want, got = x.double() @ W.T, dw.gemv(x).double()
+    assert rel_l2((got / 1e30).cpu().numpy(), (want / 1e30).cpu().numpy()) <= TOL
+
+
+# Infinite and NaN activations give what FP32 sums over the dequantized weights give: an infinity with its weight's sign, NaN where
+# opposite ones meet, and nothing in the other rows.  Up to three infinities per block of 256 in tensors of other formats than OIL4
+# (beyond, and in OIL4 tensors of three rows and more, the whole row is NaN).
+@pytest.mark.parametrize("fmt", [(1,), (0, 1), (2,), (9,), (10,), (11,), (7, 9), (7, 9, 10, 11), (4,)])
+@pytest.mark.parametrize("M", [9, 16, 20])
+def test_other_formats_infinite_activations(fmt, M):
+    rows, bpr = 40, 11
+    cols, inf = 256 * bpr, float("inf")
+    rng = np.random.default_rng(M)
+    payload, blocks = ia.block_codec.quantize_tensor(gaussian_weights(rows * cols, M), rng.choice(fmt, rows * cols // 256).astype(np.uint8))
+    x = rng.standard_normal((M, cols)).astype(np.float32)
+    last = 256 * (bpr - 1)                                       # columns that no format leaves without a weight
+    x[0, 5] = inf
+    x[1, last + 70] = -inf
+    x[2, [33, 200]] = inf
+    x[3, [33, last + 4, 300]] = [inf, -inf, inf]
+    x[4, [last, last + 64, last + 254]] = [-inf, inf, -inf]
+    x[5, 18] = float("nan")
+    with ia.DeviceWeights.from_blocks(payload, blocks, rows, cols) as dw:
+        xd = torch.from_numpy(x).cuda()
+        W = dw.dequant().view(rows, cols).cpu().numpy().astype(np.float64)
+        got = dw.gemv(xd).cpu().numpy()
+    with np.errstate(invalid="ignore"):
+        want = np.stack([(W * x[m].astype(np.float64)).sum(1) for m in range(M)])
+    assert np.isinf(want[[0, 1]]).all() and np.isnan(want[2:5]).any() and np.isinf(want[2:5]).any() and np.isnan(want[5]).all()
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(np.where(np.isinf(got), np.sign(got), 0), np.where(np.isinf(want), np.sign(want), 0))
+    for m in range(6, M):
+        assert rel_l2(got[m], want[m]) <= TOL, m
+
+
 # The digits of a block's largest magnitude: mantissas on both sides of the one above which the block takes a power of two less (its
 # top digit would not fit a signed byte), and the largest of all; both signs
 @pytest.mark.parametrize("M", [4, 16])
