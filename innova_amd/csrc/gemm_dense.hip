@@ -12,11 +12,12 @@
 // What bounds it: the operands' way into the compute unit.  A lone workgroup and a full chip both move about 30 bytes per clock
 // and compute unit, through LDS or straight into registers, whatever is in flight; the matrix cores would take 64 for tiles of
 // 128 x 128.  Tried and slower (11008 x 4096, 1024 tokens; this: 95 us): loads through registers into LDS 105 us, no LDS and K cut
-// among the wavefronts 105 us, tiles of 256 x 256 105 to 110 us, 256 x 128 105 us.
+// among the wavefronts 105 us, tiles of 256 x 256 105 to 110 us, 256 x 128 105 us (whole call at 2048 / 4096 tokens: 128 x 128 203 / 363 us,
+// 256 x 128 with three stages 202 / 376, 256 x 256 236 / 365).
 // Before (pipelined tiles of 256 x 128 and 128 x 128, operands in row order, activations rounded and weights decoded by launches of
 // their own) -> now, whole call: 5000 x 2816 planner mix, 437 tokens 55.2 -> 36.7 us; 719 x 3840, four formats, 81 tokens 47.9 ->
 // 20.3 us; 4096 x 11008 planner mix, 64 tokens 252 -> 42.5 us; 7532 x 4864 OIL8, 602 tokens 151 -> 113 us; 11008 x 4096 OIL8, 1024
-// tokens 154 -> 145 us.
+// tokens 154 -> 145 us; 11008 x 4096 SPARK_Q0, 512 / 1024 / 2048 / 4096 tokens 111 / 144 / 237 / 441 -> 79 / 120 / 204 / 363 us.
 #include <hip/hip_fp16.h>
 
 #include <algorithm>
@@ -189,10 +190,15 @@ int launch_tiles(const DenseArgs& a, hipStream_t s) {
 
 }  // namespace
 
-// Workgroup tile (64 f x 64 f) and parts along K for M tokens and N weight rows, by an estimate of the clocks: a workgroup's stage
-// (16 KB) takes 540; the stages of the workgroups of a compute unit add up, and the last of them leave others without work; parts
-// cost their meeting and one pass over each partial tile.  Measured against it: 719 x 3840, 81 tokens: 128-tiles 30 us, 64-tiles in
-// 1 / 4 parts 16 / 9.5 us; 5000 x 2816, 437 tokens: 128-tiles in 1 / 2 parts 26 / 28 us, 64-tiles 29 us.
+// Workgroup tile (64 f x 64 f) and parts along K for M tokens and N weight rows, by an estimate of the clocks.  A workgroup's stage
+// (16 KB) takes 480 (f = 1) or 540; the stages of the workgroups of a compute unit add up, and the last of them leave others without
+// work.  A workgroup that has a part of K stores its whole tile, 2500 f^2 clocks that add up in the same way, and one of a tile's
+// workgroups reads all of its parts.  (Counted once instead of for every workgroup, the stores let large products be cut in two:
+// 11008 x 4096, 2048 tokens 276 us instead of 201, 512 tokens 97 instead of 78.)
+// Over 30 measured pairs of shape and batch (500 to 11008 rows, 1024 to 11008 columns, 33 to 2048 tokens) the choice is 0.4 % slower
+// than the best of f = 1, 2 and 1, 2, 4, 8 parts on average, 3.5 % at most; over 20 others that the numbers were not taken from (35 to
+// 3000 tokens) 1.4 %, 12 % at most.  719 x 3840, 81 tokens: f = 1 in 1 / 4 parts 23.5 / 17.1 us,
+// f = 2 in 1 / 4 39.1 / 24.6; 4096 x 11008, 700 tokens: f = 2 in 1 / 2 / 4 parts 114 / 111 / 134 us.
 struct DensePlan { uint32_t f, parts; };
 static DensePlan dense_plan(uint32_t M, uint32_t N, uint32_t K) {
     const double cus = (double)device_cu_count();
@@ -201,8 +207,9 @@ static DensePlan dense_plan(uint32_t M, uint32_t N, uint32_t K) {
     for (uint32_t f = 1; f <= 2u; ++f)
         for (uint32_t parts = 1; parts <= 8u && parts * 4u <= K / 64u; parts *= 2u) {
             const uint32_t t = 64u * f;
-            const double wgs = (double)((M + t - 1u) / t) * (double)((N + t - 1u) / t) * parts, stages = (double)K * f / 64.0 / parts;
-            const double clocks = (wgs <= cus ? 1.0 : wgs / cus + 0.4) * stages * 540.0 + (parts > 1u ? 4000.0 + 1000.0 * f * f * parts : 0.0);
+            const double wgs = (double)((M + t - 1u) / t) * (double)((N + t - 1u) / t) * parts, each = std::max(wgs / cus, 1.0);
+            const double stages = (double)K * f / 64.0 / parts * (f == 1u ? 480.0 : 540.0);
+            const double clocks = (wgs <= cus ? 1.0 : each + 0.2) * stages + (parts > 1u ? (2500.0 * each + 1000.0 * parts) * f * f : 0.0);
             if (clocks < least) { least = clocks; best = {f, parts}; }
         }
     return best;

@@ -171,6 +171,30 @@ def test_slabs_of_a_tall_tensor():
     _check_any_format(ia.Format.SPARK_Q0, 8192 + 384, 4096, 260, 77)
 
 
+def test_large_product_is_not_cut_along_k():
+    """2048 tokens through 11008 x 4096 SPARK_Q0: 1376 tiles fill the chip several times over, and K parts would only add their
+    meeting in memory.  About 204 us; with two parts 276 us."""
+    rows, cols, M = 11008, 4096, 2048
+    payload, blocks = ia.block_codec.quantize_tensor(gaussian_weights(256 * cols, 9), ia.Format.SPARK_Q0)
+    big = np.tile(blocks, rows // 256)                    # the rows repeat
+    x = torch.randn(M, cols, generator=torch.Generator().manual_seed(3)).to(torch.bfloat16).cuda()
+    with ia.DeviceWeights.from_blocks(payload, big, rows, cols) as dw:
+        out = dw.gemm_bf16(x)
+        assert torch.equal(out[:, :256], out[:, -256:])
+        for _ in range(5):
+            dw.gemm_bf16(x, out=out)
+        e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        best = 1e9
+        for _ in range(5):
+            e0.record()
+            for _ in range(10):
+                dw.gemm_bf16(x, out=out)
+            e1.record()
+            torch.cuda.synchronize()
+            best = min(best, e0.elapsed_time(e1) * 100.0)
+    assert best < 245.0, f"{best:.1f} us per call"
+
+
 def test_fp32_activation_entry_matches_bf16_entry_and_meets_its_time():
     """oilhip_gemm_f32 (the reference's own gemm() arguments: FP32 X, B up to 512, qwen35_engine.cpp:47-85,630-753)
     rounds X to bf16 inside the pre-pass: same result as handing over bf16(X), bit for bit; at B = 512 on the
