@@ -166,9 +166,31 @@ def test_dense_operand_tiles(fmt, rows, cols, M):
         assert torch.equal(dw.gemm_f32(x.cuda()), yf)          # parts are added in one order
 
 
-def test_slabs_of_a_tall_tensor():
-    """More rows than one 64 MB slab of bf16 holds (8192 at 4096 columns): two slabs, the second partial."""
-    _check_any_format(ia.Format.SPARK_Q0, 8192 + 384, 4096, 260, 77)
+@pytest.mark.parametrize("fmt", [(1,), (4,), (0, 1)])
+def test_slabs_of_a_tall_tensor(fmt):
+    """More rows than one slab of decoded weights holds (128 MB of bf16: 16384 rows of 4096): two slabs, the second partial.  The rows
+    repeat with a period that does not divide the slab, so the oracle computes one period."""
+    rows, cols, M, period = 16384 + 389, 4096, 260, 131
+    assert rows * cols * 2 > 128 << 20 and 16384 % period
+    nb, per = rows * cols // 256, period * cols // 256
+    payload, blocks = ia.block_codec.quantize_tensor(gaussian_weights(period * cols, 77, outlier_every=97),
+                                                     np.random.default_rng(7).choice(fmt, per).astype(np.uint8))
+    big = np.tile(blocks, -(-rows // period))[:nb]
+    flat = payload
+    if len(fmt) == 1:                                     # uniform tensors: back to back
+        shift = (np.arange(nb) // per * payload.size).astype(np.uint64)
+        big["cb_off"] += shift
+        big["idx_off"] += shift
+        flat = np.tile(payload, -(-rows // period))
+    x = torch.randn(M, cols, generator=torch.Generator().manual_seed(7)).to(torch.bfloat16)
+    wd = O.dequant_blocks(payload, to_orc_blocks(blocks)).reshape(period, cols).astype(np.float64)
+    want = x.float().numpy().astype(np.float64) @ wd.T
+    with ia.DeviceWeights.from_blocks(flat, big, rows, cols) as dw:
+        y = dw.gemm_bf16(x.cuda()).cpu().numpy()
+    assert rel_l2(y[:, :period], want) <= TOL
+    for r in range(period, rows, period):                 # the same products, whose K parts may be added in another order
+        n = min(period, rows - r)
+        assert rel_l2(y[:, r:r + n], y[:, :n]) <= 1e-6, r
 
 
 def test_large_product_is_not_cut_along_k():
