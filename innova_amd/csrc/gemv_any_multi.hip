@@ -28,6 +28,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "level_digits.h"
 #include "oil4_lds.h"
 
 namespace oilhip {
@@ -43,7 +44,7 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 constexpr int kMaxWaves = 8;
 // tiles of 16 operand rows for M tokens of three pieces each
 constexpr int tiles_for(int M) { return (3 * M + 15) / 16; }
-constexpr int kMaxTiles = 3, kPassTokens = 16;
+constexpr int kPassTokens = 16;
 
 // What the weights are: kOrderA formats have one factor per block at most, kOrderC formats one per group of 64 columns.
 // Operand columns: step s of a block, lane group kq, element e is column 64 kq + 8 s + e (A), or 64 (s / 2) + 16 kq + 8 (s % 2) + e (C).
@@ -201,29 +202,11 @@ __device__ __forceinline__ f16x8 bytes8(uint32_t b0, uint32_t b1) {
     return eight(d[0], d[1], d[2], d[3]);
 }
 
-// bytes of a format's digit tables: magnitude m = 0..7 of 10^4 times the upper levels as 256 a + b
-constexpr int kLevelTimes1e4[8] = {1260, 3976, 6508, 9275, 12392, 15995, 20522, 27178};
-constexpr int low_digit(int n) { return (n & 255) > 127 ? (n & 255) - 256 : n & 255; }
-constexpr uint32_t digits(bool high, int first) {
-    uint32_t t = 0;
-    for (int i = 0; i < 4; ++i) {
-        const int n = kLevelTimes1e4[first + i], b = low_digit(n), a = (n - b) / 256;
-        t |= (uint32_t)((high ? a : b) & 255) << (8 * i);
-    }
-    return t;
-}
-// four 4-bit codes (low nibbles) -> digits a and b as signed bytes (no digit is 0 or -128, so the byte-wise negation carries nowhere)
-__device__ __forceinline__ void digits4(uint32_t w, uint32_t& a, uint32_t& b) {
-    const uint32_t m = __builtin_amdgcn_perm(0u, 0u, (~w & 0x08080808u) | 0x05050505u);   // 0xFF where the code is below 8
-    const uint32_t at = (w ^ m) & 0x07070707u, one = m & 0x01010101u;
-    a = (__builtin_amdgcn_perm(digits(true, 4), digits(true, 0), at) ^ m) + one;
-    b = (__builtin_amdgcn_perm(digits(false, 4), digits(false, 0), at) ^ m) + one;
-}
 // eight 4-bit codes of c -> the two summands
 __device__ __forceinline__ void levels4(uint32_t c, f16x8& va, f16x8& vb) {
     uint32_t ae, be, ao, bo, d[8];
-    digits4(c, ae, be);                                                     // codes 0, 2, 4, 6
-    digits4(c >> 4, ao, bo);                                                // codes 1, 3, 5, 7
+    level_digits(c, ae, be);                                                    // codes 0, 2, 4, 6
+    level_digits(c >> 4, ao, bo);                                              // codes 1, 3, 5, 7
     // bytes to code order, then to FP16: 1024 + (digit + 128)
     const uint32_t a0 = __builtin_amdgcn_perm(ao, ae, 0x05010400u) ^ 0x80808080u, a1 = __builtin_amdgcn_perm(ao, ae, 0x07030602u) ^ 0x80808080u;
     const uint32_t b0 = __builtin_amdgcn_perm(bo, be, 0x05010400u) ^ 0x80808080u, b1 = __builtin_amdgcn_perm(bo, be, 0x07030602u) ^ 0x80808080u;
@@ -431,14 +414,13 @@ gemv_any_multi_kernel(const BodyArgs a) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) acc[g][t][e] = fmaf(sum[t][e] * factor, un[xs][t][e], acc[g][t][e]);
         } else {
-            // zero point (a 64th of it would do: the group sums are packed divided by 64) and scale of group kq, this lane's row
+            // zero point and scale of group kq, this lane's row (the group sums are packed divided by 64)
             const bool own = S != kSparkMix || fmt[g] != 7u;
-            float zp = __half2float(__ushort_as_half((unsigned short)o[0])), sc = __half2float(__ushort_as_half((unsigned short)(o[0] >> 16)));
+            float sc = __half2float(__ushort_as_half((unsigned short)(o[0] >> 16)));
             const float unit = S == kOil2Grp ? 1e-4f : S == kOil4Grp ? 256e-4f : S == kOil8Grp ? 1.0f / 255.0f
                              : fmt[g] == 9u ? 1e-4f : fmt[g] == 10u ? 256e-4f : 1.0f / 255.0f;
             sc = own ? sc * unit : 1.0f;
             const uint32_t zbits = own ? o[0] & 0xFFFFu : 0u;
-            (void)zp;
             const f16x8 zv = eight(zbits, 0u, 0u, 0u);
             float factor[4];
 #pragma unroll

@@ -34,6 +34,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "level_digits.h"
 #include "oil4_lds.h"
 
 namespace oilhip {
@@ -218,34 +219,6 @@ struct MultiJobs {
 
 struct PartsOf { uint32_t n[kPassKinds], blocks[kPassKinds], chunk[kPassKinds]; };
 
-// the digits a and b of eight magnitudes: 10000 times the levels 0.1260, 0.3976, 0.6508, 0.9275, 1.2392, 1.5995, 2.0522, 2.7178
-constexpr int kLevelTimes1e4[8] = {1260, 3976, 6508, 9275, 12392, 15995, 20522, 27178};
-constexpr int low_digit(int n) { return ((n + 128) & 255) - 128; }
-constexpr uint32_t digit_table(bool high, int first) {
-    uint32_t t = 0;
-    for (int i = 0; i < 4; ++i) {
-        const int n = kLevelTimes1e4[first + i], b = low_digit(n), a = (n - b) / 256;
-        t |= (uint32_t)((high ? a : b) & 255) << (8 * i);
-    }
-    return t;
-}
-constexpr bool digits_fit() {
-    for (int n : kLevelTimes1e4) {
-        const int b = low_digit(n), a = (n - b) / 256;
-        if (a <= 0 || a > 127 || b == 0 || b == -128) return false;
-    }
-    return true;
-}
-static_assert(digits_fit(), "the byte-wise negation needs digits other than 0 and -128");
-
-// four codes (low nibbles of the bytes of w) -> their digits
-__device__ __forceinline__ void decode_four(uint32_t w, int& a, int& b) {
-    const uint32_t m = __builtin_amdgcn_perm(0u, 0u, (~w & 0x08080808u) | 0x05050505u);   // 0xFF where the code is below 8 (selector 13), else 0
-    const uint32_t at = (w ^ m) & 0x07070707u, one = m & 0x01010101u;                     // magnitude: code - 8, or 7 - code
-    a = (int)((__builtin_amdgcn_perm(digit_table(true, 4), digit_table(true, 0), at) ^ m) + one);
-    b = (int)((__builtin_amdgcn_perm(digit_table(false, 4), digit_table(false, 0), at) ^ m) + one);
-}
-
 template <int KIND>
 struct Sums {                                                              // one block's integer sums of one token tile
     static constexpr int N = kind_few(KIND) ? 2 : 4;
@@ -377,9 +350,9 @@ multi_body(const BodyArgs& a, uint32_t g_begin, uint32_t g_end, float* red) {
                 i32x4 da, db;
 #pragma unroll
                 for (int d = 0; d < 4; ++d) {
-                    int ad, bd;
-                    decode_four((o & 1) ? w[WS][g][o >> 1][d] >> 4 : w[WS][g][o >> 1][d], ad, bd);
-                    da[d] = ad; db[d] = bd;
+                    uint32_t ad, bd;
+                    level_digits((o & 1) ? w[WS][g][o >> 1][d] >> 4 : w[WS][g][o >> 1][d], ad, bd);
+                    da[d] = (int)ad; db[d] = (int)bd;
                 }
 #pragma unroll
                 for (int t = 0; t < NT; ++t) {
