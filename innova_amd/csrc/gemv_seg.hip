@@ -25,12 +25,13 @@ namespace {
 
 constexpr int kRunPad = 36;                // floats per run of 32 activations in LDS: 16-byte reads of neighbouring lanes
                                            // fall into different banks
-// Wavefronts per workgroup, one workgroup per CU: 16 (four per SIMD, windows of at most 2 KB) for one or two activation rows
+// Wavefronts per workgroup, one workgroup per CU: 16 (four per SIMD, windows of at most 2 KB) for one activation row
 // of a tensor that was packed for them, else 8 (two per SIMD, windows of at most 4 KB).  The decoding is bound by instruction
 // issue with waits on LDS in between (a step of 8 SPARK_Q0 blocks is 91 vector and 10 LDS instructions), so more wavefronts
-// side by side fill the waits: 11008 x 4096 at the registry's SPARK mix went from 15.7 to 13.1 us, at the planner's mix from 9.3 to
-// 8.8.  Three and four activation rows need more registers than four wavefronts per SIMD leave (128): there a workgroup has 8,
-// and each takes two streams, one after the other.
+// side by side fill the waits: 11008 x 4096 at the registry's SPARK mix went from 15.7 to 13.5 us, at the planner's mix from 9.2 to
+// 8.8.  More rows need more registers than four wavefronts per SIMD leave (128): there a workgroup has 8,
+// and each takes two streams, one after the other (two rows with 16 wavefronts spill 31 registers to memory: 11008 x 4096 at the
+// planner's mix 15.1 us, OIL8_GRP 35 us; with 8 wavefronts 12.0 and 21.6; packed for 8 wavefronts they took 11.7 and 17.9).
 constexpr uint32_t window_of(int waves) { return waves == 16 ? kSegWindow / 2 : kSegWindow; }
 constexpr int TR = kSegTileRows;           // accumulators per lane and activation row: a tile has at most this many rows
 typedef _Float16 h2v __attribute__((ext_vector_type(2)));
@@ -379,7 +380,7 @@ int launch_waves(const oilhip_weights& w, const DecodeTables* T, const float* d_
 template <int MB, int XF = 0>
 int launch_seg(const oilhip_weights& w, const DecodeTables* T, const float* d_x, float* d_y, int m0, int M, hipStream_t s,
                const float* d_xw = nullptr) {
-    if constexpr (MB <= 2)
+    if constexpr (MB == 1)
         if (w.seg.waves == 16) return launch_waves<MB, XF, 16>(w, T, d_x, d_y, m0, M, s, d_xw);
     return launch_waves<MB, XF, 8>(w, T, d_x, d_y, m0, M, s, d_xw);
 }
