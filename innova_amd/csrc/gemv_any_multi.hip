@@ -228,7 +228,7 @@ constexpr int raw_dwords(int S) {
     return S == kSpark || S == kPlanner ? 3 : S == kOil2 ? 6 : S == kOil8 ? 18 : S == kOil2Grp ? 5 : S == kOil4Grp ? 9 : 17;
 }
 __host__ __device__ constexpr uint32_t block_bytes(int S) { return S == kSpark ? 48u : S == kOil2 ? 64u : S == kOil8 ? 256u : S == kOil2Grp ? 80u : S == kOil4Grp ? 144u : 272u; }
-// row groups of a run: as many as registers and LDS take
+// row groups of a run, at most: as many as registers and LDS take
 constexpr int run_groups(int S, int NT) { return NT == 3 && grouped(S) ? 1 : NT > 1 || raw_dwords(S) > 6 ? 2 : 4; }
 // blocks of activations that a wavefront holds
 constexpr int x_slots(int S, int NT) { return NT == 1 ? (grouped(S) || raw_dwords(S) > 9 ? 2 : 3) : 1; }
@@ -592,9 +592,15 @@ int launch_one(BodyArgs a, hipStream_t s) {
     const uint32_t wgs = std::min(groups, slots);
     a.g_base = groups / wgs;
     a.g_rem = groups % wgs;
-    // runs of one group while the chip has room for every group in a workgroup of its own
-    if (G == 1 || a.g_base + (a.g_rem ? 1u : 0u) == 1u) return launch_run<S, NT, 1>(a, wgs, waves, s);
-    return launch_run<S, NT, G>(a, wgs, waves, s);
+    // The longest run that divides the fullest workgroup's groups: a run that is not full costs as much as a full one (5120 x 4096,
+    // 4 rows, runs of 1 / 2 / 4 for 2 groups: SPARK_Q0 9.9 / 9.7 / 12.7 us, OIL2_GRP 12.4 / 12.7 / 18.7; 11008 x 4096, 3 groups: OIL2 14.9 / 16.8 /
+    // 18.5, the registry's mix 28.2 / 34.0; 16384 x 4096, 4 groups: SPARK_Q0 14.5 / 13.2 / 13.4).
+    const uint32_t most_groups = a.g_base + (a.g_rem ? 1u : 0u);
+    if constexpr (G > 2)
+        if (most_groups % (uint32_t)G == 0u) return launch_run<S, NT, G>(a, wgs, waves, s);
+    if constexpr (G > 1)
+        if (most_groups % 2u == 0u) return launch_run<S, NT, 2>(a, wgs, waves, s);
+    return launch_run<S, NT, 1>(a, wgs, waves, s);
 }
 
 template <int S>
