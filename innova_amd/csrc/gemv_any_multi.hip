@@ -372,6 +372,11 @@ gemv_any_multi_kernel(const BodyArgs a) {
         if constexpr (!grouped(S)) {
             const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
             float factor = 1.0f;
+            // Several chains, whose sums meet afterwards: an instruction rounds its sums four times, one after the other (eight products of a
+            // lane group at a time), so one chain of eight rounds 32 times.  SPARK_Q0, 4096 columns, 16 rows, error against 64 bits with 1 / 2 / 4
+            // chains: 12.2e-8 / 10.1e-8 / 9.3e-8 (one row at a time in FP32: 10.7e-8).
+            constexpr int CH = NT == 3 && S == kOil8 ? 2 : 4;              // (as many as the registers take)
+            f32x4 chain[NT][CH];
             uint32_t minus[2], bits[2], c[16];
             if constexpr (S == kSpark || S == kPlanner) {
                 const bool spark = S == kSpark || fmt[g] == 1u;
@@ -405,10 +410,18 @@ gemv_any_multi_kernel(const BodyArgs a) {
                     if (s == 7) v[7] = (kq & 1u) ? (_Float16)0.0f : v[7];  // columns 127 and 255 are slots
                 }
 #pragma unroll
-                for (int t = 0; t < NT; ++t) sum[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x[xs][t][s], v, s ? sum[t] : zero, 0, 0, 0);
+                for (int t = 0; t < NT; ++t) chain[t][s * CH / 8] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x[xs][t][s], v, s % (8 / CH) ? chain[t][s * CH / 8] : zero, 0, 0, 0);
             }
 #pragma unroll
-            for (int t = 0; t < NT; ++t) settle(sum[t]);
+            for (int t = 0; t < NT; ++t) {
+#pragma unroll
+                for (int c = 0; c < CH; ++c) settle(chain[t][c]);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    sum[t][e] = chain[t][0][e] + chain[t][1][e];
+                    if constexpr (CH == 4) sum[t][e] += chain[t][2][e] + chain[t][3][e];
+                }
+            }
 #pragma unroll
             for (int t = 0; t < NT; ++t)
 #pragma unroll

@@ -402,6 +402,20 @@ def test_other_formats_infinite_activations(fmt, M):
         assert rel_l2(got[m], want[m]) <= TOL, m
 
 
+# Several rows at once are no less accurate than one row at a time in FP32: error against 64 bits over all outputs.  5 % for the
+# spread of the two figures (each over 16 x 2048 outputs and more).
+@pytest.mark.parametrize("fmt", [(1,), (0, 1)])
+def test_other_formats_error_of_several_rows(fmt):
+    rows, cols, M = 2048, 4096, 16
+    ids = np.random.default_rng(5).choice(fmt, rows * cols // 256).astype(np.uint8)
+    payload, blocks = ia.block_codec.quantize_tensor(gaussian_weights(rows * cols, 6), ids)
+    x = torch.randn(M, cols, generator=torch.Generator().manual_seed(3)).cuda()
+    with ia.DeviceWeights.from_blocks(payload, blocks, rows, cols) as dw:
+        want = x.double() @ dw.dequant().view(rows, cols).double().T
+        one = torch.cat([dw.gemv(x[m:m + 1]) for m in range(M)]).double()
+        assert float((dw.gemv(x).double() - want).norm()) <= 1.05 * float((one - want).norm())
+
+
 # The digits of a block's largest magnitude: mantissas on both sides of the one above which the block takes a power of two less (its
 # top digit would not fit a signed byte), and the largest of all; both signs
 @pytest.mark.parametrize("M", [4, 16])
