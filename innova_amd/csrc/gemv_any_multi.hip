@@ -643,16 +643,36 @@ int source_of(const oilhip_weights& w) {
     return w.uniform_fmt == OILHIP_OIL8 && w.uniform_stride == 256u && w.uniform_cb == 0 && w.uniform_idx == 256u && (w.uniform_base & 3u) == 0 ? kOil8 : -1;
 }
 
+// Whether two to four rows (OIL8: to eight) are faster here than through the kernels of up to four rows per pass (window streams: two where
+// four rows of activations do not fit their LDS).  From 36 shapes of 0.26 to 123 M weights per format, all timed both ways; "M weights" are
+// millions.
+bool faster_than_row_kernels(int src, const oilhip_weights& w, int M) {
+    const uint64_t weights = w.rows * w.cols;
+    const bool light = src == kSpark || src == kPlanner;
+    if (src == kOil8) return M <= 4 ? weights >= 12000000u : M > 2 && weights >= 2000000u;
+    // Two rows: tall tensors, which are packed for one row at a time, and of these the formats whose error is no larger here (11008 x 4096
+    // SPARK_Q0 16.5 against 12.3 us, planner's mix 12.0 against 12.4; 22016 x 4096 24 against 13, 19 against 15).
+    if (M == 2) return light && w.seg.waves == 16;
+    // Three and four: SPARK_Q0 and the planner's mix always (1000 x 2048, 3 rows 7.2 against 6.1 us, 4096 x 11008, 4 rows 43 against 14).
+    if (light || w.seg.waves == 16) return true;
+    // Heavier decoding needs a full chip.  Workgroups of which few have a second group: 5120 x 4096, 3 rows OIL4_GRP 15.8 against 16.7 us,
+    // registry's mix 18.9 against 20.8; 6144 x 2048 OIL2_GRP 10.1 against 11.2; 7000 x 3072 14.0 against 11.4.
+    const uint64_t groups = (w.rows + 15u) / 16u, cus = (uint64_t)device_cu_count();
+    if (grouped(src) && w.cols <= 5120u && groups > cus && groups * 5u < cus * 8u) return false;
+    // Rows of more than 16 blocks are two parts or more of at most 16, with little work each where rows are few: 2048 x 6144, 3 rows
+    // OIL4_GRP 13.3 against 15.2, registry's mix 16.8 against 20.7; 4096 x 5120 mix 18.3 against 20.6; 1024 x 8192 OIL4_GRP 17.2 against
+    // 16.0, mix 17.8 against 21.5; 4096 x 8192 mix 25.5 against 22.3.
+    if ((src == kOil4Grp || src == kSparkMix) && w.cols > 4096u && weights < 30000000u) return src == kOil4Grp ? w.cols >= 8192u : M == 4 && w.cols > 8192u;
+    // 12 M weights: 2048 x 2048, 3 rows OIL4_GRP 7.8 against 8.1; 1500 x 4096 OIL2_GRP 8.9 against 9.6; 4096 x 4096 OIL2 11.5 against 9.2.
+    // Wider than 5120 columns four rows take two passes there: 1000 x 11008 OIL2 22.3 against 14.6.
+    return weights >= 12000000u || w.cols > 5120u;
+}
+
 // what the tensor's weights are, or -1 where these kernels do not cover the tensor and the batch, or another one is faster
 int source_for(const oilhip_weights& w, int M) {
     const int src = source_of(w);
     if (src < 0 || M < 2 || !w.all_full || (w.cols & 255u) || w.cols == 0 || w.cols > kGemvPackMaxCols || w.rows == 0 || w.rows > 0x7FFFFFFFull) return -1;
-    // The kernels of up to four rows per pass stay for two rows, and for three and four (window streams: while four rows of
-    // activations fit their LDS) on tensors of less than 12 M weights: 2000 x 2048, 3 rows 8.5 against 8.9 us; 4096 x 4096 14.2
-    // against 12.8 us.  The OIL8 kernel stays up to two passes on small tensors: 1000 x 1024, 6 rows 7.6 against 8.0 us.
-    const uint64_t weights = w.rows * w.cols;
-    if (M == 2 || (M <= 4 && w.seg.waves != 16 && weights < 12000000u && !(by_descriptor(src) && w.cols > 5120u))) return -1;
-    if (src == kOil8 && M <= 8 && weights < 2000000u) return -1;
+    if (M <= (src == kOil8 ? 8 : 4) && !faster_than_row_kernels(src, w, M)) return -1;
     const uint32_t bpr = (uint32_t)(w.cols >> 8);
     // 32-bit byte offsets inside a workgroup's rows (blocks, or descriptors)
     const uint64_t per_row = std::max<uint64_t>(16u, by_descriptor(src) ? 16u : block_bytes(src)) * bpr;

@@ -561,7 +561,8 @@ def test_workspace_of_the_caller():
         with ia.DeviceWeights.quantize(gaussian_weights(rows * cols, 4), fmt, rows, cols) as dw:
             for M in (1, 2, 4, 5, 8, 16, 17, 33):
                 need = L.oilhip_gemv_workspace_bytes(dw.handle, M)
-                assert (need == 0) == (M == 1 or fmt == ia.Format.OIL16 or (fmt != ia.Format.OIL4 and M <= 4) or (fmt == ia.Format.OIL8 and M <= 8))
+                packs_from = {ia.Format.OIL4: 2, ia.Format.SPARK_Q0: 3, ia.Format.OIL4_GRP: 5, ia.Format.OIL8: 9}.get(fmt, 99)
+                assert (need == 0) == (M < packs_from)
                 x = torch.randn(M, cols, generator=torch.Generator().manual_seed(M)).cuda()
                 y, ws = torch.empty(M, rows, device="cuda"), torch.full((need + 256,), 0x5A, dtype=torch.uint8, device="cuda")
                 ia._lib.check(L.oilhip_gemv_f32_ws(dw.handle, x.data_ptr(), y.data_ptr(), M, ws.data_ptr(), need, ia._lib.current_stream()))
