@@ -245,9 +245,11 @@ static void pack_window_streams(std::vector<uint8_t>& pay, std::vector<DevBlock>
     }
     uint32_t widest = 0;
     for (uint32_t i = 0; i < nf; ++i) widest = std::max(widest, g.stride[i]);
-    // Sixteen streams per CU for tensors of more than sixteen rows per CU, else eight: a stream with fewer than two rows fills
-    // too little of the decoding steps (4096 x 4096 of the planner's mix: 5.9 us with eight, 6.7 with sixteen; 11008 x 4096: 9.3 and 8.8),
-    // and of the stored floats' blocks (512 bytes and more) the smaller windows would hold three at most
+    // Sixteen streams per CU for tensors of more than 32 rows per CU, else eight: a stream with fewer than two rows fills
+    // too little of the decoding steps (4096 x 4096 of the planner's mix: 5.9 us with eight, 6.7 with sixteen).  With more, one row, eight -> sixteen:
+    // planner's mix 9000 x 2048 7.2 -> 6.5 us, 11008 x 4096 9.3 -> 9.0, 22016 x 4096 13.6 -> 13.6, 32768 x 4096 18.6 -> 16.5; SPARK_Q0, OIL2,
+    // registry's mix 11008 x 4096 11.7 -> 11.2, 13.3 -> 12.5, 15.7 -> 13.4.  Of the stored floats' blocks (512 bytes and more) the smaller
+    // windows would hold three at most.
     const uint32_t cus = (uint32_t)device_cu_count(), waves = rows > (uint64_t)cus * 32 && widest < 512 ? 16u : 8u, window = waves == 16u ? kSegWindow / 2 : kSegWindow;
     // streams: at most `waves` per CU, and as many as give every stream the same number of rows (or one less): streams of
     // five and six rows side by side would leave the fixed-size first windows a sixth empty

@@ -248,15 +248,15 @@ int launch_flat_rows(const FlatRows& a, hipStream_t s) {
 
 // OIL{8,4,2}Engine::quant_gemm: codes packed along the flat [K][N] index, every output one k-ordered chain of fused
 // multiply-adds, terms with A == 0 skipped, bit for bit as in the reference loop.
-// The chain bounds it: K dependent FMAs of one wavefront, which issues an instruction every four to five cycles, so the
-// time is the number of instructions on the wavefront that carries the chain.  A workgroup therefore splits the work by
-// role: four or eight producer wavefronts fetch, unpack and look up the levels of COLS columns and kEngTile steps into LDS while one
+// The chain bounds it: K dependent FMAs of one wavefront.  Instructions on the wavefront that carries it cost the most, so a workgroup
+// splits the work by role: four or eight producer wavefronts fetch, unpack and look up the levels of COLS columns and kEngTile steps into LDS while one
 // wavefront per row of A walks the previous tile with 1.25 instructions per step (an FMA, a quarter of a 16-byte LDS
 // read; A[m][k] sits in a register of 16 lanes and the broadcast is part of the FMA).  16 columns per workgroup, three quarters of the chain's
 // lanes idle: the chain costs the same for any number of lanes, and 256 workgroups at N = 4096 share the unpacking and
 // the fetches.  A producer lane takes one k step: its 16 columns' codes are 2 to 5 neighbouring dwords at any bit
 // offset, its 16 levels go to 16 rows of the tile (lanes side by side, no bank conflicts), and four tiles of codes are in
-// flight.  N = K = 4096, M = 1: 8-bit 59.6 -> 27 us, 4-bit 176 -> 21, 2-bit 176 -> 19.
+// flight.  N = K = 4096, M = 1: 8-bit 59.6 -> 27 us, 4-bit 176 -> 21, 2-bit 176 -> 19.  That is 13 cycles per step with 1.25
+// instructions issued and vector issue at 22 %: latency on the chain (FMA with a broadcast operand, LDS reads, a barrier per tile).
 constexpr int kEngTile = 256, kEngPitch = kEngTile + 4, kEngMaxRows = 4;
 constexpr int eng_producers(int cols) { return cols == 16 ? 4 : 8; }
 constexpr int eng_copies(int bits) { return bits == 8 ? 16 : 64; }          // lane-private copies of the codebook

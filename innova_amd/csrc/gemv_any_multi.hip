@@ -1,4 +1,4 @@
-// gemv_any_multi.hip -- decode GEMV for 3 to 16 activation rows per pass over tensors of other formats than plain OIL4
+// gemv_any_multi.hip -- decode GEMV for several activation rows (up to 16 per pass) over tensors of other formats than plain OIL4
 // (Qwen35Engine::gemm with small B, src/adapters/tools/qwen35_engine.cpp:47-85, over dequantize_block_all,
 // src/block_codec.cpp:576-720): uniform SPARK_Q0, OIL2, OIL8 and grouped lattices, and the mixes of the planner (OIL1, SPARK_Q0) and
 // of the registry (OIL1_GRP, OIL2_GRP, OIL4_GRP, OIL8_GRP).
@@ -14,14 +14,17 @@
 // one more matrix instruction (group sums of the activations, in three pieces, times the FP16 zero points).
 // A wavefront takes every n-th block of the row for a run of 16-row groups, keeps the activations of its block in registers, and
 // the wavefronts' sums meet in LDS once per run; every sum has a fixed order.  All but OIL8 are stored as
-// window streams; a block is found through its descriptor, two steps ahead.
+// window streams; a block is found through its descriptor, two steps ahead.  The pieces lie in a workspace of the caller's or in scratch of the
+// stream; a call that is being captured without a workspace is left to the kernels that pack nothing.
 //
-// What bounds it: the activations' way into each compute unit (8 KB per block and five rows, about 30 bytes per clock), once per
-// workgroup, on wide rows; latency and the two launches on small tensors.  Tried: shares of K for several workgroups of a range
+// What bounds it: latency at two wavefronts per SIMD and the two launches where rows are short or few (planner's mix, 11008 x 4096, five rows: vector
+// issue 27 %, matrix cores 7 %, memory 1.3 TB/s); the decode's vector instructions in the grouped formats (registry's mix 42 %); towards
+// 16 rows and wide rows the activations' way into each compute unit (8 KB per block and five rows, once per workgroup).  Tried: shares of K for several workgroups of a range
 // of rows, added by the last one, 10 to 20 % faster on the widest rows only and two to three times slower on others.
 // Before (window-stream kernel in passes of up to four rows, OIL8 kernel likewise) -> now, pre-pass included:
-//   16795 x 12032 SPARK_Q0, 15 rows 507 -> 53 us;  11008 x 4096 planner mix, 16 rows 73 -> 20 us;  11008 x 4096 OIL2, 8 rows 49 -> 19 us
-//   6613 x 8192, registry mix, 9 rows 103 -> 43 us;  4096 x 4096 OIL8, 32 rows 90 -> 28 us;  649 x 768 planner mix, 5 rows 12.3 -> 6.9 us
+//   16795 x 12032 SPARK_Q0, 15 rows 498 -> 53 us;  11008 x 4096 planner mix, 5 / 16 rows 26.7 / 70 -> 11.8 / 16.3 us;  OIL2, 8 rows 46.6 -> 15.8 us
+//   6613 x 8192, registry mix, 9 rows 99.6 -> 40.6 us;  4096 x 4096 OIL8, 32 rows 87 -> 27.4 us;  649 x 768 planner mix, 5 rows 11.3 -> 5.5 us
+// Other mixes of formats stay with the window-stream kernel, four rows at a time (11008 x 4096, 75 % OIL2 and 25 % OIL4, 8 rows 58 us).
 #include <hip/hip_fp16.h>
 
 #include <algorithm>

@@ -18,14 +18,16 @@
 // and serve every group of the run, and the wavefronts' sums meet in LDS once per run.  There is no table to build, nothing
 // is summed across workgroups, and the order of every sum is fixed.
 // What bounds it: up to 8 tokens vector issue (about 170 instructions per block of 16 rows, beside 8 to 16 matrix instructions that
-// other wavefronts overlap) on the tall shapes, launch and round trips on the small ones; above, the activations' way into the compute
-// unit: 16 KB per block and 16 tokens at about 30 bytes per clock, once per workgroup (at three digits, 12 KB, 4096 x 11008 took
-// 17.6 us with 16 tokens and 24.8 with 32).
+// other wavefronts overlap; 35 to 38 % of the cycles) on the tall shapes, launch and round trips on the small ones; above, on wide rows,
+// the activations' way into the compute unit: 16 KB per block and 16 tokens, once per workgroup, at about 30 bytes per clock.  4096 x 11008
+// from 4 to 16 to 32 tokens: L2 read requests 0.96, 2.01, 3.37 M, vector instructions 1.97, 2.32, 2.95 M, 10.2, 17.9, 27.8 us (with three
+// digits, 12 KB, 17.6 us at 16 tokens and 24.8 at 32).  In batches of several tensors matrix (35 %) and vector instructions (55 %) bound it.
 // Before (FP16 halves of levels from a 64 KB LDS table, K cut between workgroups) -> now, pre-pass included, weights from memory:
-//   11008 x 4096, 4 / 8 / 16 / 32 tokens: 12.8 / 12.5 / 14.3 / 19.7 us -> 11.6 / 12.8 / 14.8 / 20.0 us
-//   4096 x 11008: 17.0 / 17.5 / 19.8 / 25.1 us -> 13.2 / 15.7 / 20.4 / 30.6 us
-//   131072 x 4096, 4 / 16 / 32 tokens: 81 / 86 / 127 us -> 72 / 90 / 134 us;  30000 x 14336: 77 / 81 / 120 us -> 68 / 83 / 130 us
+//   11008 x 4096, 4 / 8 / 16 / 32 tokens: 12.9 / 12.9 / 15.0 / 19.9 us -> 11.6 / 12.7 / 15.3 / 21.1 us
+//   4096 x 11008: 17.4 / 18.0 / 20.5 / 25.8 us -> 13.5 / 15.8 / 20.4 / 30.7 us
+//   131072 x 4096, 4 / 16 / 32 tokens: 81 / 86 / 127 us -> 72 / 90 / 133 us;  30000 x 14336: 77 / 81 / 120 us -> 68 / 83 / 130 us
 //   2838 x 512, 5 / 16 / 32 tokens: 7.5 / 8.7 / 9.3 -> 5.1 / 5.7 / 7.0 us
+// (slower with more than 16 tokens, where four digits cost more than the table did)
 // Error against 64 bits (2-norm): 1.8e-7 -> 0.9e-7, whatever the distribution of the activations.
 #include <hip/hip_fp16.h>
 
