@@ -135,8 +135,8 @@ def test_oil4_multi_token_counts(rows, cols, M):
     assert err <= TOL
 
 
-# rows wider than 16 blocks are cut along K between workgroups whose sums meet in a workspace and are added in a fixed
-# order (the output buffer holds NaNs before the call), several row tiles per workgroup, parts of unequal length, both
+# rows of more blocks than the wavefronts hold at once are walked in parts, one after the other in one workgroup, whose sums are
+# carried in LDS (the output buffer holds NaNs before the call), several row groups per workgroup, parts of unequal length, both
 # pass widths
 @pytest.mark.parametrize("rows,cols,M", [(9000, 8192, 5), (9000, 8192, 17), (5000, 11008, 16), (700, 8448, 24)])
 def test_oil4_multi_token_rows_cut_along_k(rows, cols, M):
@@ -578,7 +578,7 @@ def test_release_stream_scratch_frees_every_buffer_of_the_stream():
     st = torch.cuda.Stream()
     rng = np.random.default_rng(31)
     cases = []
-    for rows, cols, M in ((256, 4096, 5), (8192, 11008, 16)):       # packed activations (4 MB), then partial sums on top
+    for rows, cols, M in ((256, 4096, 5), (8192, 11008, 16)):       # packed activations: 4 MB, and 8 MB for rows of more than 4096 weights
         w = gaussian_weights(rows * cols, rows + M)
         payload, blocks = ia.block_codec.quantize_tensor(w, ia.Format.OIL4)
         cases.append((ia.DeviceWeights.from_blocks(payload, blocks, rows, cols),

@@ -41,8 +41,7 @@ def test_noalloc_matches_gemv(first, second):
 
 
 def test_noalloc_allocates_nothing_and_runs_under_capture_on_a_fresh_stream():
-    """A shape whose kernel needs scratch (five rows, 11008 columns: packed activations, three K parts that meet in
-    the scratch): the call leaves the device's free memory as it found it on a stream the library has never seen, and
+    """A shape whose kernel needs scratch (five rows, 11008 columns: packed activations): the call leaves the device's free memory as it found it on a stream the library has never seen, and
     the same call is captured into a graph on another fresh stream (where a scratch allocation would be refused) and
     replayed."""
     rows, cols, M = 200, 11008, 5
