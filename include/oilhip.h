@@ -199,23 +199,23 @@ int oilhip_set_ordered_sums(int ordered);
  * weights dequantized to bf16 (each value rounded once), MFMA with FP32 accumulation, FP32 out.
  * (The reference has no bf16 path; its FP32 prefill loop is
  * qwen35_engine.cpp:630-753 over the same gemm.)  Uniform OIL4 tensors are decoded tile by tile in LDS inside the
- * GEMM kernel.  Tensors of any other format, or that mix formats, are decoded to bf16 in slabs of weight rows (at
- * most 64 MB, a scratch buffer of the stream: the first call of a size on a stream allocates, so make it outside
- * graph capture) and multiplied by the same kernel reading a dense operand; they need full 256-weight blocks with
- * the channel sizes the quantizer writes (OILHIP_E_ARG otherwise). */
+ * GEMM kernel, which takes 16-byte aligned X.  Tensors of any other format, or that mix formats, and OIL4 with X at another alignment are
+ * decoded to bf16 in slabs of weight rows (at most 128 MB) by one launch that writes the activations in operand order
+ * as well, and multiplied by a kernel of their own; small products are cut along K, with partial sums that one
+ * workgroup adds in order.  All of it is scratch of the stream: the first call of a size on a stream allocates, so make it outside
+ * graph capture.  These tensors need full 256-weight blocks with the channel sizes the quantizer writes (OILHIP_E_ARG otherwise). */
 int oilhip_gemm_bf16(const oilhip_weights* w, const uint16_t* d_x_bf16, float* d_y, int M, void* stream);
 
 /* The same prefill GEMM for the reference's own call: FP32 activations X[M][cols], as Qwen35Engine::prefill hands
  * them to gemm() in chunks of up to 512 tokens (src/adapters/tools/qwen35_engine.cpp:47-85,630-753).  X is rounded
- * once to bf16 on its way into the kernel's operand order (no extra pass for plain OIL4 and 16-byte aligned X;
- * otherwise one conversion launch into a scratch buffer of the stream).  The result is bit for bit what oilhip_gemm_bf16
+ * once to bf16 on its way into the kernel's operand order, by the launch that writes that order.  The result is bit for bit what oilhip_gemm_bf16
  * returns for bf16(X): relative L2 <= 2e-3 against the FP32 contraction over the rounded activations, about 2.4e-3
  * against the one over the FP32 activations themselves (both operands' roundings, Gaussian data), where
  * oilhip_gemv_f32 keeps 1e-5: a caller chooses it per call. */
 int oilhip_gemm_f32(const oilhip_weights* w, const float* d_x, float* d_y, int M, void* stream);
 
 /* Frees the scratch buffers the library holds for `stream` on the current device (packed activations of the
- * multi-token GEMV, X' and decoded slabs of the prefill GEMM, the lookup kernels' codes; buffers that a larger request
+ * multi-token GEMV, X', decoded slabs and partial sums of the prefill GEMM, the lookup kernels' codes; buffers that a larger request
  * has replaced included): before a stream is destroyed, or to trim after a large batch.  Synchronizes the stream
  * first, so the stream must still exist; no captured graph may still replay launches that were recorded on it.  (No counterpart in the reference, which owns no device memory.) */
 int oilhip_release_stream_scratch(void* stream);
