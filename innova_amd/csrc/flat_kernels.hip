@@ -5,6 +5,7 @@
 //   oil::engines::OIL{8,4,2}Engine::quant_gemm  src/oil_engines_oil{8,4,2}.cpp
 #include <algorithm>
 #include <type_traits>
+#include <utility>
 
 #include "common.h"
 #include "oil4_lds.h"
@@ -54,10 +55,25 @@ struct FlatRows {
     const uint8_t* last = nullptr;   // the codes' last dword, when a lane's codes can start off a dword; else nullptr
 };
 
+// The dword at an address that was computed as a number.  The address space is said because a pointer made from an integer is generic to
+// the compiler: a flat load counts as an LDS access too and returns out of order, so the next wait on LDS waits for memory.
+__device__ __forceinline__ uint32_t load_dword(uintptr_t at) { return *(const __attribute__((address_space(1))) uint32_t*)at; }
+typedef uint32_t u32x4_at4 __attribute__((ext_vector_type(4), aligned(4)));
+// N neighbouring dwords, dword-aligned, four to a load
+template <int N>
+__device__ __forceinline__ void load_dwords(uint32_t (&d)[N], uintptr_t at) {
+#pragma unroll
+    for (int i = 0; i + 4 <= N; i += 4) {
+        const u32x4_at4 v = *(const __attribute__((address_space(1))) u32x4_at4*)(at + 4 * i);
+        d[i] = v.x; d[i + 1] = v.y; d[i + 2] = v.z; d[i + 3] = v.w;
+    }
+#pragma unroll
+    for (int i = N / 4 * 4; i < N; ++i) d[i] = load_dword(at + 4 * i);
+}
 // 32 bits that start at bit `bit` behind p, from the one or two dwords they lie in; `last` keeps the second inside the array.
 __device__ __forceinline__ uint32_t load_bits32(const uint8_t* p, uint32_t bit, const uint8_t* last) {
     const uintptr_t at = reinterpret_cast<uintptr_t>(p) + (bit >> 3), q = at & ~(uintptr_t)3, l = reinterpret_cast<uintptr_t>(last);
-    const uint32_t a = *reinterpret_cast<const uint32_t*>(q), b = *reinterpret_cast<const uint32_t*>(q < l ? q + 4 : l);
+    const uint32_t a = load_dword(q), b = load_dword(q < l ? q + 4 : l);
     return __builtin_amdgcn_alignbit(b, a, (uint32_t)(at & 3) * 8u + (bit & 7u));
 }
 __device__ __forceinline__ float4 load_f4(const float* p) { float4 v; __builtin_memcpy(&v, p, 16); return v; }
@@ -248,152 +264,236 @@ int launch_flat_rows(const FlatRows& a, hipStream_t s) {
 
 // OIL{8,4,2}Engine::quant_gemm: codes packed along the flat [K][N] index, every output one k-ordered chain of fused
 // multiply-adds, terms with A == 0 skipped, bit for bit as in the reference loop.
-// The chain bounds it: K dependent FMAs of one wavefront.  Instructions on the wavefront that carries it cost the most, so a workgroup
-// splits the work by role: four or eight producer wavefronts fetch, unpack and look up the levels of COLS columns and kEngTile steps into LDS while one
-// wavefront per row of A walks the previous tile with 1.25 instructions per step (an FMA, a quarter of a 16-byte LDS
-// read; A[m][k] sits in a register of 16 lanes and the broadcast is part of the FMA).  16 columns per workgroup, three quarters of the chain's
+// The chain bounds it: K dependent FMAs of one wavefront, at least 4 cycles each.  Instructions on the wavefront that carries it cost the
+// most, so a workgroup splits the work by role: producer wavefronts fetch, unpack and look up the levels of COLS columns and a tile of
+// steps into LDS while one wavefront per row of A walks an earlier tile with 1.25 instructions per step (an FMA, a quarter of a 16-byte LDS
+// read; A sits in a register of 16 lanes and the broadcast is part of the FMA).  16 columns per workgroup, three quarters of the chain's
 // lanes idle: the chain costs the same for any number of lanes, and 256 workgroups at N = 4096 share the unpacking and
-// the fetches.  A producer lane takes one k step: its 16 columns' codes are 2 to 5 neighbouring dwords at any bit
-// offset, its 16 levels go to 16 rows of the tile (lanes side by side, no bank conflicts), and four tiles of codes are in
-// flight.  N = K = 4096, M = 1: 8-bit 59.6 -> 27 us, 4-bit 176 -> 21, 2-bit 176 -> 19.  That is 13 cycles per step with 1.25
-// instructions issued and vector issue at 22 %: latency on the chain (FMA with a broadcast operand, LDS reads, a barrier per tile).
-constexpr int kEngTile = 256, kEngPitch = kEngTile + 4, kEngMaxRows = 4;
-constexpr int eng_producers(int cols) { return cols == 16 ? 4 : 8; }
-constexpr int eng_copies(int bits) { return bits == 8 ? 16 : 64; }          // lane-private copies of the codebook
-constexpr size_t eng_lds(int bits, int cols) { return 4u * ((size_t)eng_copies(bits) << bits) + 8u * (size_t)cols * kEngPitch; }
+// the fetches.  A producer lane takes one k step: its columns' codes are neighbouring dwords at any bit
+// offset, its levels go to as many rows of the tile (lanes side by side, no bank conflicts), and four tiles of codes are in
+// flight.  For that the loops over whole tiles have no branch between a fetch and its use, or the compiler waits for all loads, and
+// the loads say that they are global (load_dword): with either missing, every tile waited out a trip to memory, 13 cycles per step.
+// Three buffers let the chain pass the next tile's barrier and start its reads before it ends a tile.  ONE (one row of A, COLS < 64): the
+// chain has a SIMD to itself; with 64 columns the producers need all four (N = 11008, 4-bit: 28.5 us on three, 26.5).
+// K = 4096, M = 1, 4-bit, N = 300 / 4096 / 8192 / 11008: 20.5 / 22.6 / 27.0 / 36.5 -> 17.0 / 18.7 / 21.6 / 26.5 us; 8-bit 21.5 / 23.8 / 35.6 / 49.5 ->
+// 18.2 / 19.8 / 24.6 / 31; M = 8, N = 4096, 4-bit 48 -> 41.  Now 8 cycles per step: 4.6 for the FMA with its broadcast, 1.2 for the LDS
+// reads' issue (both measured alone), the rest around a tile's barrier, its test for zeros and its loads of A.
+constexpr int kEngMaxRows = 4, kEngTile = 192, kEngPitch = kEngTile + 4, kEngBuffers = 3;
+constexpr int eng_parts(int cols) { return cols > 16 ? 2 : 1; }             // producers that share a tile's step
+constexpr int eng_producers(int cols) { return kEngTile / 64 * eng_parts(cols); }
+constexpr int eng_copies(int bits, int cols) { return bits != 8 ? 64 : cols == 64 ? 8 : 16; }   // lane-private copies of the codebook
+constexpr size_t eng_lds(int bits, int cols) { return 4u * ((size_t)eng_copies(bits, cols) << bits) + 4u * (size_t)(kEngBuffers * cols * kEngPitch); }
 
-template <int BITS, int COLS>
-__global__ void __launch_bounds__(64 * (eng_producers(COLS) + kEngMaxRows))
+// Sixteen steps of a chain: acc += a * level, step 4 i + e with A from a[e] of lane J + i of every 16.  The broadcast rides on the FMA
+// (the compiler keeps it as a move of its own, which doubles the chain's instructions).  A register that a VALU instruction has just
+// written must not be read this way: a[] is written by memory loads only.
+template <int J>
+__device__ __forceinline__ void eng_steps(float& acc, const float4& a, const float4* q) {
+#define ENG_FOUR(I, L0, L1, L2, L3)                                                                                                          \
+    "v_fmac_f32_dpp %0, %1, %" #L0 " row_newbcast:%" #I " row_mask:0xf bank_mask:0xf\n\tv_fmac_f32_dpp %0, %2, %" #L1 " row_newbcast:%" #I   \
+    " row_mask:0xf bank_mask:0xf\n\tv_fmac_f32_dpp %0, %3, %" #L2 " row_newbcast:%" #I " row_mask:0xf bank_mask:0xf\n\tv_fmac_f32_dpp %0, %4, %" #L3 \
+    " row_newbcast:%" #I " row_mask:0xf bank_mask:0xf\n\t"
+    asm(ENG_FOUR(21, 5, 6, 7, 8) ENG_FOUR(22, 9, 10, 11, 12) ENG_FOUR(23, 13, 14, 15, 16) ENG_FOUR(24, 17, 18, 19, 20)
+        : "+v"(acc) : "v"(a.x), "v"(a.y), "v"(a.z), "v"(a.w), "v"(q[0].x), "v"(q[0].y), "v"(q[0].z), "v"(q[0].w), "v"(q[1].x), "v"(q[1].y),
+          "v"(q[1].z), "v"(q[1].w), "v"(q[2].x), "v"(q[2].y), "v"(q[2].z), "v"(q[2].w), "v"(q[3].x), "v"(q[3].y), "v"(q[3].z), "v"(q[3].w),
+          "n"(J), "n"(J + 1), "n"(J + 2), "n"(J + 3));
+#undef ENG_FOUR
+}
+
+template <int BITS, int COLS, bool ONE>
+__global__ void __launch_bounds__(ONE ? 256 * eng_parts(COLS) : 64 * (eng_producers(COLS) + kEngMaxRows))
 engine_kernel(const float* __restrict__ A, const uint8_t* __restrict__ bq, const float* __restrict__ cb, float* __restrict__ C,
               long long M, long long N, long long K) {
-    constexpr int PRODUCERS = eng_producers(COLS), OWN = COLS * 4 / PRODUCERS;   // 4 wavefronts' lanes cover a tile's steps, each OWN columns
+    constexpr int TILE = kEngTile, PITCH = kEngPitch, PRODUCERS = eng_producers(COLS);
+    constexpr int OWN = COLS / eng_parts(COLS);       // a producer's lanes take a step each, OWN columns of it
     constexpr int W = OWN * BITS / 32;                     // dwords of one step's codes
-    constexpr uint32_t COPIES = eng_copies(BITS);
+    constexpr uint32_t COPIES = eng_copies(BITS, COLS), SHIFT = COPIES == 64 ? 8 : COPIES == 16 ? 6 : 5;   // an entry's copies take 1 << SHIFT bytes
     constexpr int AHEAD = 4;                               // tiles of codes in flight
     extern __shared__ __align__(16) float eng_mem[];
-    float* lev0 = eng_mem;                                 // two tiles: [column][step]
-    float* tab = eng_mem + 2 * COLS * kEngPitch;
+    float* tab = eng_mem;
+    float* lev0 = eng_mem + (COPIES << BITS);              // three tiles: [column][step]
     const uint32_t lane = threadIdx.x & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     for (uint32_t i = threadIdx.x; i < (1u << BITS) * COPIES; i += blockDim.x) tab[i] = cb[i / COPIES];
     // workgroups are dealt to the eight XCDs in turn: each takes a run of neighbouring columns, whose codes share lines
     const uint32_t q8 = gridDim.x >> 3, r8 = gridDim.x & 7u, xcd = blockIdx.x & 7u;
     const long long n0 = (long long)(xcd * q8 + (xcd < r8 ? xcd : r8) + (blockIdx.x >> 3)) * COLS;
-    const long long tiles = (K + kEngTile - 1) / kEngTile;
+    const long long full = K / TILE, tiles = (K + TILE - 1) / TILE;
     __syncthreads();
-    if (wave < (uint32_t)PRODUCERS) {
-        const uint32_t step0 = (wave & 3u) * 64u + lane, col0 = (wave >> 2) * OWN;
+    // ONE: wavefront 0 is the chain, and wavefront 4, which would share its SIMD, ends here
+    if (ONE && wave == 4u) return;
+    if (ONE ? wave != 0u : wave < (uint32_t)PRODUCERS) {
+        const uint32_t step0 = (ONE ? (wave & 3u) - 1u : wave % 3u) * 64u + lane, col0 = (ONE ? wave >> 2 : wave / 3u) * OWN;
         uint32_t raw[AHEAD][W + 1], sh[AHEAD];
         const uintptr_t base = reinterpret_cast<uintptr_t>(bq);
         const uintptr_t last = (base + ((unsigned long long)K * (unsigned long long)N * BITS + 7) / 8 - 1) & ~(uintptr_t)3;
-        auto fetch = [&](int slot, long long t) {          // this lane's step of tile t; past the end: the last step again
-            long long k = t * kEngTile + step0;
-            k = k < K ? k : K - 1;
-            const unsigned long long bit = ((unsigned long long)k * (unsigned long long)N + (unsigned long long)n0 + col0) * BITS;
+        // This lane's step of the next tile, as wide loads where no lane's dwords can reach past the codes' end (the first `safe`
+        // tiles), else dword by dword; past the end: the last step again.
+        const unsigned long long first = (unsigned long long)n0 + col0, end_bit = ((unsigned long long)(K - 1) * N + first) * BITS;
+        unsigned long long next_bit = ((unsigned long long)step0 * N + first) * BITS;
+        const long long safe = (K - (COLS * BITS + 95) / (N * BITS) - 1) / TILE;
+        auto fetch = [&](int slot, auto wide) {
+            const unsigned long long bit = next_bit < end_bit ? next_bit : end_bit;
+            next_bit += (unsigned long long)TILE * N * BITS;
             const uintptr_t at = base + (bit >> 3), word = at & ~(uintptr_t)3;
             sh[slot] = (uint32_t)(at & 3) * 8u + (uint32_t)(bit & 7);
+            if (wide.value) {
+                load_dwords<W + 1>(raw[slot], word);
+                return;
+            }
 #pragma unroll
-            for (int i = 0; i <= W; ++i) raw[slot][i] = *reinterpret_cast<const uint32_t*>(word + 4 * i < last ? word + 4 * i : last);
+            for (int i = 0; i <= W; ++i) raw[slot][i] = load_dword(word + 4 * i < last ? word + 4 * i : last);
         };
-        auto decode = [&](int slot, float* dst, bool live) {   // steps past K: zeros
+        uint32_t buffer = 0;
+        auto decode = [&](int slot, auto partial, bool live) {   // a tile that K ends in: zeros past K
             float lv[OWN];
 #pragma unroll
             for (int c = 0; c < OWN; ++c) {
                 const uint32_t d = __builtin_amdgcn_alignbit(raw[slot][c * BITS / 32 + 1], raw[slot][c * BITS / 32], sh[slot]);
-                const uint32_t code = (d >> (c * BITS % 32)) & ((1u << BITS) - 1u);
-                lv[c] = tab[code * COPIES + (lane & (COPIES - 1))];
+                constexpr uint32_t MASK = ((1u << BITS) - 1u) << SHIFT;
+                const int right = c * BITS % 32 - (int)SHIFT;
+                const uint32_t at = ((right > 0 ? d >> right : d << -right) & MASK) | ((lane & (COPIES - 1)) * 4u);   // byte offset of the entry's copy
+                lv[c] = *reinterpret_cast<const float*>(reinterpret_cast<const uint8_t*>(tab) + at);
             }
+            float* dst = lev0 + buffer * (COLS * PITCH) + col0 * PITCH + step0;
 #pragma unroll
-            for (int c = 0; c < OWN; ++c) dst[(col0 + c) * kEngPitch + step0] = live ? lv[c] : 0.0f;
+            for (int c = 0; c < OWN; ++c) dst[c * PITCH] = partial.value && !live ? 0.0f : lv[c];
+            buffer = buffer == kEngBuffers - 1 ? 0u : buffer + 1u;
         };
 #pragma unroll
-        for (int u = 0; u < AHEAD; ++u) fetch(u, u);
-        for (long long t = 0; t < tiles; t += AHEAD)
+        for (int u = 0; u < AHEAD; ++u) fetch(u, std::false_type{});
+        long long t = 0;
+        for (; t + 2 * AHEAD <= safe; t += AHEAD)          // no branch inside, so that a wait counts exactly the loads before it
+#pragma unroll
+            for (int u = 0; u < AHEAD; ++u) {
+                decode(u, std::false_type{}, true);        // tile t + u: the chain has left tile t + u - 3
+                fetch(u, std::true_type{});
+                __syncthreads();
+                __builtin_amdgcn_sched_barrier(0);         // the next tile's waits stay behind this tile
+            }
+        for (; t < tiles; t += AHEAD)
 #pragma unroll
             for (int u = 0; u < AHEAD; ++u)
                 if (t + u < tiles) {                       // uniform over the workgroup, as in the other role
-                    decode(u, lev0 + (u & 1) * (COLS * kEngPitch), (t + u) * kEngTile + step0 < K);                 // tile t + u: the chain has left this buffer (AHEAD is even)
-                    fetch(u, t + u + AHEAD);
+                    decode(u, std::true_type{}, (t + u) * TILE + step0 < K);
+                    fetch(u, std::false_type{});
                     __syncthreads();
                 }
         return;
     }
     __builtin_amdgcn_s_setprio(3);                         // the chain goes first where it shares a SIMD with producers
-    const uint32_t row = wave - PRODUCERS, rows = (blockDim.x >> 6) - PRODUCERS;
+    const uint32_t row = ONE ? 0u : wave - PRODUCERS, rows = ONE ? 1u : (blockDim.x >> 6) - PRODUCERS;
     const long long m = (long long)blockIdx.y * rows + row;
     const bool live = m < M;
     const float* a_row = A + (live ? m : M - 1) * K;
-    const float* mine = lev0 + (lane & (COLS - 1)) * kEngPitch;
-    constexpr int GA = kEngTile / 16;                      // A of a tile: lane j of every 16 holds steps 16 g + j
-    auto fetch_a = [&](float (&dst)[GA], long long t) {
-        const long long k0 = t * kEngTile;
-        if (k0 + kEngTile <= K) {
-            const float* p = a_row + k0 + (lane & 15u);
+    const float* mine = lev0 + (lane & (COLS - 1)) * PITCH;
+    constexpr int GA = TILE / 64;                          // A of a tile: lane j of every 16 holds steps 64 g + 4 j to 64 g + 4 j + 3
+    auto fetch_a = [&](float4 (&dst)[GA], long long t) {
+        const float* p = a_row + t * TILE + 4u * (lane & 15u);
 #pragma unroll
-            for (int g = 0; g < GA; ++g) dst[g] = p[16 * g];
-        } else {
+        for (int g = 0; g < GA; ++g) dst[g] = load_f4(p + 64 * g);
+    };
+    auto fetch_last = [&](float4 (&dst)[GA]) {             // the tile that K ends in
 #pragma unroll
-            for (int g = 0; g < GA; ++g) {
-                const long long k = k0 + 16 * g + (lane & 15u);
-                // past K: -0 meets a zero level, and adding their product, -0, changes no sum, not even a zero's sign
-                dst[g] = k < K ? a_row[k] : -0.0f;
-            }
+        for (int g = 0; g < GA; ++g) {
+            const long long k = full * TILE + 64 * g + 4u * (lane & 15u);
+            // past K: -0 meets a zero level, and adding their product, -0, changes no sum, not even a zero's sign
+            dst[g].x = k < K ? a_row[k] : -0.0f; dst[g].y = k + 1 < K ? a_row[k + 1] : -0.0f;
+            dst[g].z = k + 2 < K ? a_row[k + 2] : -0.0f; dst[g].w = k + 3 < K ? a_row[k + 3] : -0.0f;
         }
     };
     float acc = 0.0f;
-    auto walk = [&](const float (&a)[GA], const float* src, int steps) {
-        uint32_t low = 0x7FFFFFFFu;                        // smallest magnitude of the tile's A: is there a zero?
+    constexpr int BATCHES = TILE / 32, RING = ONE ? 3 : 2; // batches of 32 steps; the levels of one, and of those that are read ahead
+    static_assert(BATCHES % RING == 0);
+    float4 lv[RING][8];
+    const float* src = mine;
+    auto read = [&](float4 (&dst)[8], const float* tile, int b) {
 #pragma unroll
-        for (int g = 0; g < GA; ++g)
-            if (16 * g + (int)(lane & 15u) < steps) low = min(low, __float_as_uint(a[g]) & 0x7FFFFFFFu);
-        if (__ballot(low == 0u) == 0ull) {
-            float4 lv[2][8];                               // 32 steps' levels, read while the 32 before are walked
-            auto read = [&](float4 (&dst)[8], int b) {
+        for (int j = 0; j < 8; ++j) dst[j] = *reinterpret_cast<const float4*>(tile + 32 * b + 4 * j);
+    };
+    auto after = [&](const float* tile) { return tile == mine + (kEngBuffers - 1) * (COLS * PITCH) ? mine : tile + COLS * PITCH; };
+    // A tile's steps.  The next tile's barrier and first reads come before this one's end.
+    // for LDS alone, whose writers wait for their writes: reads stay in flight across it
+    auto barrier = [&]() {
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_barrier" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto walk = [&](const float4 (&a)[GA], auto partial, int steps, bool more) {
+        float low = INFINITY;                              // smallest magnitude of the tile's A: is there a zero?
+        if (!partial.value) {
 #pragma unroll
-                for (int j = 0; j < 8; ++j) dst[j] = *reinterpret_cast<const float4*>(src + 32 * b + 4 * j);
-            };
-            read(lv[0], 0);
-#pragma unroll
-            for (int b = 0; b < kEngTile / 32; ++b) {
-                if (b + 1 < kEngTile / 32) read(lv[(b + 1) & 1], b + 1);
-                __builtin_amdgcn_sched_barrier(0);
-                const float4* l = lv[b & 1];
-                // acc += a[step] * level: the broadcast of lane `step` of each row of 16 rides on the FMA (the compiler
-                // keeps it as a move of its own, which doubles the chain's instructions).  A register that a VALU
-                // instruction has just written must not be read this way: a[] is written by memory loads only.
-#define ENG_STEP(J, LV) "v_fmac_f32_dpp %0, %1, %" #LV " row_newbcast:" #J " row_mask:0xf bank_mask:0xf\n\t"
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {              // one statement per 16 steps: the compiler puts a wait state between two
-                    const float4* q = l + 4 * h;
-                    asm(ENG_STEP(0, 2) ENG_STEP(1, 3) ENG_STEP(2, 4) ENG_STEP(3, 5) ENG_STEP(4, 6) ENG_STEP(5, 7) ENG_STEP(6, 8) ENG_STEP(7, 9)
-                        ENG_STEP(8, 10) ENG_STEP(9, 11) ENG_STEP(10, 12) ENG_STEP(11, 13) ENG_STEP(12, 14) ENG_STEP(13, 15) ENG_STEP(14, 16) ENG_STEP(15, 17)
-                        : "+v"(acc) : "v"(a[2 * b + h]), "v"(q[0].x), "v"(q[0].y), "v"(q[0].z), "v"(q[0].w), "v"(q[1].x), "v"(q[1].y), "v"(q[1].z),
-                          "v"(q[1].w), "v"(q[2].x), "v"(q[2].y), "v"(q[2].z), "v"(q[2].w), "v"(q[3].x), "v"(q[3].y), "v"(q[3].z), "v"(q[3].w));
-                }
-#undef ENG_STEP
-                __builtin_amdgcn_sched_barrier(0);
+            for (int g = 0; g < GA; ++g) {
+                asm("v_min3_f32 %0, %0, |%1|, |%2|" : "+v"(low) : "v"(a[g].x), "v"(a[g].y));
+                asm("v_min3_f32 %0, %0, |%1|, |%2|" : "+v"(low) : "v"(a[g].z), "v"(a[g].w));
             }
+        } else {
+#pragma unroll
+            for (int g = 0; g < GA; ++g) {
+                const int k = 64 * g + 4 * (int)(lane & 15u);
+                if (k < steps) low = fminf(low, fabsf(a[g].x));
+                if (k + 1 < steps) low = fminf(low, fabsf(a[g].y));
+                if (k + 2 < steps) low = fminf(low, fabsf(a[g].z));
+                if (k + 3 < steps) low = fminf(low, fabsf(a[g].w));
+            }
+        }
+        const float* next = after(src);
+        if (__builtin_expect(__ballot(low == 0.0f) == 0ull, 1)) {
+            auto batch = [&](auto number) {
+                constexpr int b = decltype(number)::value, FAR = RING - 1;
+                if constexpr (b + FAR < BATCHES) {
+                    read(lv[(b + FAR) % RING], src, b + FAR);
+                } else if (more) {
+                    if (b + FAR == BATCHES) barrier();
+                    read(lv[(b + FAR) % RING], next, b + FAR - BATCHES);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                const float4* l = lv[b % RING];
+                eng_steps<8 * (b & 1)>(acc, a[b / 2], l);  // one statement per 16 steps: the compiler puts a wait state between two
+                eng_steps<8 * (b & 1) + 4>(acc, a[b / 2], l + 4);
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            [&]<int... B>(std::integer_sequence<int, B...>) { (batch(std::integral_constant<int, B>{}), ...); }(std::make_integer_sequence<int, BATCHES>{});
         } else {                                           // a zero: the reference skips the term, 0 * inf must not reach the sum
 #pragma unroll
             for (int g = 0; g < GA; ++g)
 _Pragma("unroll 1")
-                for (int j = 0; j < 16 && 16 * g + j < steps; ++j) {
-                    const float x = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(a[g]), j));
-                    const float r = __fmaf_rn(x, src[16 * g + j], acc);
-                    acc = x != 0.0f ? r : acc;
+                for (int j = 0; j < 16; ++j) {
+                    const float v[4] = {a[g].x, a[g].y, a[g].z, a[g].w};
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {          // steps past K: -0, whose terms change nothing
+                        const float x = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v[e]), j));
+                        const float r = __fmaf_rn(x, src[64 * g + 4 * j + e], acc);
+                        acc = x != 0.0f ? r : acc;
+                    }
                 }
+            if (more) {
+                barrier();
+#pragma unroll
+                for (int b = 0; b < RING - 1; ++b) read(lv[b], next, b);
+            }
         }
+        src = next;
     };
-    float a0[GA], a1[GA];
-    fetch_a(a0, 0);
-    for (long long t = 0; t < tiles; t += 2) {
+    float4 a0[GA], a1[GA];
+    auto fetch_any = [&](float4 (&dst)[GA], long long t) { if (t < full) fetch_a(dst, t); else if (t < tiles) fetch_last(dst); };
+    auto walk_any = [&](const float4 (&a)[GA], long long t) { walk(a, std::true_type{}, t < full ? TILE : (int)(K - full * TILE), t + 1 < tiles); };
+    fetch_any(a0, 0);
+    __syncthreads();
+#pragma unroll
+    for (int b = 0; b < RING - 1; ++b) read(lv[b], src, b);
+    long long t = 0;
+    for (; t + 2 < full; t += 2) {                         // no branch but walk's own: A of the next tile stays in flight
         fetch_a(a1, t + 1);
-        __syncthreads();                                   // tile t is in lev[0]
-        walk(a0, mine, K - t * kEngTile < kEngTile ? (int)(K - t * kEngTile) : kEngTile);
-        if (t + 1 < tiles) {
-            fetch_a(a0, t + 2);
-            __syncthreads();
-            walk(a1, mine + COLS * kEngPitch, K - (t + 1) * kEngTile < kEngTile ? (int)(K - (t + 1) * kEngTile) : kEngTile);
-        }
+        walk(a0, std::false_type{}, TILE, true);
+        fetch_a(a0, t + 2);
+        walk(a1, std::false_type{}, TILE, true);
+    }
+    for (; t < tiles; t += 2) {                            // at most three tiles
+        fetch_any(a1, t + 1);
+        walk_any(a0, t);
+        if (t + 1 == tiles) break;
+        fetch_any(a0, t + 2);
+        walk_any(a1, t + 1);
     }
     if (live && lane < (uint32_t)COLS && n0 + lane < N) C[m * N + n0 + lane] = acc;
 }
@@ -514,23 +614,24 @@ engine_dequant_kernel(int bits, const uint8_t* __restrict__ idx, const float* __
     }
 }
 
-template <int BITS, int COLS>
+template <int BITS, int COLS, bool ONE>
 int launch_engine(const float* a, const uint8_t* b, const float* cb, float* c, int64_t M, int64_t N, int64_t K, hipStream_t s) {
     static std::atomic<uint64_t> raised{0};
     constexpr size_t lds = eng_lds(BITS, COLS);
-    if (int rc = ensure_max_lds(raised, (const void*)engine_kernel<BITS, COLS>, (int)lds)) return rc;
+    if (int rc = ensure_max_lds(raised, (const void*)engine_kernel<BITS, COLS, ONE>, (int)lds)) return rc;
     const int64_t rows = std::min<int64_t>(M, kEngMaxRows), groups = (N + COLS - 1) / COLS;   // rows of A of one workgroup share the levels
     if (groups > 0x7FFFFFFFll) return fail(OILHIP_E_ARG, "N exceeds the grid limit");
-    hipLaunchKernelGGL((engine_kernel<BITS, COLS>), dim3((uint32_t)groups, (uint32_t)((M + rows - 1) / rows)),
-                       dim3((uint32_t)(64 * (eng_producers(COLS) + rows))), lds, s, a, b, cb, c, (long long)M, (long long)N, (long long)K);
+    hipLaunchKernelGGL((engine_kernel<BITS, COLS, ONE>), dim3((uint32_t)groups, (uint32_t)((M + rows - 1) / rows)),
+                       dim3((uint32_t)(ONE ? 256 * eng_parts(COLS) : 64 * (eng_producers(COLS) + rows))), lds, s, a, b, cb, c, (long long)M, (long long)N, (long long)K);
     OILHIP_HIP(hipGetLastError());
     return OILHIP_OK;
 }
 
 template <int BITS>
 int launch_engine_bits(int cols, const float* a, const uint8_t* b, const float* cb, float* c, int64_t M, int64_t N, int64_t K, hipStream_t s) {
-    return cols == 16 ? launch_engine<BITS, 16>(a, b, cb, c, M, N, K, s)
-         : cols == 32 ? launch_engine<BITS, 32>(a, b, cb, c, M, N, K, s) : launch_engine<BITS, 64>(a, b, cb, c, M, N, K, s);
+    if (M == 1 && cols < 64) return cols == 16 ? launch_engine<BITS, 16, true>(a, b, cb, c, M, N, K, s) : launch_engine<BITS, 32, true>(a, b, cb, c, M, N, K, s);
+    return cols == 16 ? launch_engine<BITS, 16, false>(a, b, cb, c, M, N, K, s)
+         : cols == 32 ? launch_engine<BITS, 32, false>(a, b, cb, c, M, N, K, s) : launch_engine<BITS, 64, false>(a, b, cb, c, M, N, K, s);
 }
 
 // Negative sizes are errors; an empty output (M or N zero) needs no pointers at all.

@@ -163,6 +163,21 @@ def test_engine_quant_gemm_tiles_and_remainders(bits, M, N, K):
     assert np.array_equal(np.isnan(got), np.isnan(want))
 
 
+@pytest.mark.parametrize("bits,M,N,K", [(8, 1, 1, 192), (8, 1, 4097, 1537), (8, 1, 8193, 1700), (4, 1, 5, 191), (4, 1, 16, 193), (4, 1, 4095, 2304),
+                                        (4, 1, 8192, 1729), (2, 1, 3, 3000), (2, 1, 4097, 575), (2, 1, 8195, 2113), (8, 4, 40, 2305), (4, 2, 8193, 1730), (2, 5, 4100, 1920)])
+def test_engine_quant_gemm_long_rows(bits, M, N, K):
+    """Around the engine kernel's tiles of 192 steps with its pipeline full: the last tiles, which are fetched dword by dword, narrow and
+    odd N whose lanes' codes reach over several steps, one row (its own wavefront layout up to 32 columns) and several, and a zero of A
+    in one tile only."""
+    rng = np.random.default_rng(bits * 7000 + N + K)
+    A = rng.standard_normal((M, K)).astype(np.float32)
+    A[:, K // 2] = 0.0
+    b = rng.integers(0, 256, (K * N * bits + 7) // 8, dtype=np.uint8)
+    cb = rng.standard_normal(1 << bits).astype(np.float32)
+    got = ia.kernel.engine_quant_gemm(bits, A, b, cb, M, N, K)
+    assert np.array_equal(got.view(np.uint32), O.engine_quant_gemm(bits, A, b, cb, M, N, K).view(np.uint32))
+
+
 @pytest.mark.parametrize("rows,K,batch", [(1, 1, 1), (3, 15, 2), (5, 17, 3), (257, 1024, 1), (2047, 513, 5), (2049, 260, 1), (2050, 4097, 2), (2053, 2048, 9)])
 def test_flat_rows_remainders(rows, K, batch):
     """Rows, activation rows and row lengths around the tiles of the flat-codebook kernel (4 rows, 4 activation rows, 8 or 16
