@@ -128,6 +128,27 @@ def lib():
     return _lib
 
 
+_native = None
+
+
+def native():
+    """The module with the ordinary calls as C functions (csrc/native_calls.cpp): they return None for what they do not take.  Loaded
+    after torch and liboilhip, whose libraries it uses."""
+    global _native
+    if _native is None:
+        lib()
+        try:
+            from . import _native as module
+        except ImportError as e:
+            raise OilHipError(f"innova_amd/_native.so cannot be loaded ({e}): build it first (make -C innova_amd/csrc, or "
+                              "python -c 'import __graft_entry__ as g; g.build()')") from e
+        import torch
+        if torch.cuda.is_available():
+            torch.cuda.init()
+        _native = module
+    return _native
+
+
 def exported_symbols():
     return list(_SIGNATURES)
 

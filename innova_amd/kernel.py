@@ -28,6 +28,9 @@ def _ret(out, on_device):
 
 def oil8_gemm(indices, codebook, activations, M: int, N: int, K: int):
     """out[m*N+n] = sum_k codebook[indices[n*K+k]] * activations[m*K+k]  (kernel.h:24-26)."""
+    y = (_lib._native or _lib.native()).oil8_gemm(indices, codebook, activations, M, N, K)
+    if y is not None:
+        return y
     import torch
     i, d1 = _dev(indices, np.uint8)
     c, _ = _dev(codebook, np.float32)
@@ -40,6 +43,9 @@ def oil8_gemm(indices, codebook, activations, M: int, N: int, K: int):
 
 def oil4_gemm(packed_indices, codebook, activations, M: int, N: int, K: int):
     """out[m*N+n] = sum_k f16(codebook[nib((m*N+n)*K+k)]) * activations[n*K+k]  (kernel.h:30-32)."""
+    y = (_lib._native or _lib.native()).oil4_gemm(packed_indices, codebook, activations, M, N, K)
+    if y is not None:
+        return y
     import torch
     i, d1 = _dev(packed_indices, np.uint8)
     c, _ = _dev(codebook, np.uint16)
@@ -50,8 +56,13 @@ def oil4_gemm(packed_indices, codebook, activations, M: int, N: int, K: int):
     return _ret(out, d1 and d2)
 
 
-def _prod(fn, w, cb, cb_dtype, scale, X, M, N, K):
+def _prod(bits, w, cb, cb_dtype, scale, X, M, N, K):
+    y = (_lib._native or _lib.native()).prod(bits, w, cb, scale, X, M, N, K)
+    if y is not None:
+        return y
     import torch
+    L = _lib.lib()
+    fn = L.oilhip_prod_gemv_spark if bits == 2 else L.oilhip_prod_gemv_oil4 if bits == 4 else L.oilhip_prod_gemv_oil8
     wd, d1 = _dev(w, np.uint8)
     xd, d2 = _dev(X, np.float32)
     Y = xd.new_empty((N, M), dtype=torch.float32)
@@ -66,15 +77,15 @@ def _prod(fn, w, cb, cb_dtype, scale, X, M, N, K):
 
 def gemv_spark_batch(packed_w, scale, X, M: int, N: int, K: int):
     """Y[n*M+m] = scale * sum_k tern(W[m][k]) * X[n*K+k]  (kernel_production.h:40-42)."""
-    return _prod(_lib.lib().oilhip_prod_gemv_spark, packed_w, None, None, scale, X, M, N, K)
+    return _prod(2, packed_w, None, None, scale, X, M, N, K)
 
 
 def gemv_oil4_batch(packed_indices, codebook, scale, X, M: int, N: int, K: int):
-    return _prod(_lib.lib().oilhip_prod_gemv_oil4, packed_indices, codebook, np.uint16, scale, X, M, N, K)
+    return _prod(4, packed_indices, codebook, np.uint16, scale, X, M, N, K)
 
 
 def gemv_oil8_batch(indices, codebook, scale, X, M: int, N: int, K: int):
-    return _prod(_lib.lib().oilhip_prod_gemv_oil8, indices, codebook, np.float32, scale, X, M, N, K)
+    return _prod(8, indices, codebook, np.float32, scale, X, M, N, K)
 
 
 def gemv_spark_tiled(packed_w, scale, x, M: int, K: int, tile_m: int = 32):
@@ -93,6 +104,9 @@ def gemv_oil8_tiled(indices, codebook, scale, x, M: int, K: int, tile_m: int = 3
 def engine_quant_gemm(bits: int, a, b_idx, codebook, M: int, N: int, K: int):
     """C[m*N+n] = sum_k A[m*K+k] * codebook[code(k*N+n)]: OIL{8,4,2}Engine::quant_gemm
     (include/oil/oil_engines.h:49,78,151)."""
+    y = (_lib._native or _lib.native()).engine_quant_gemm(bits, a, b_idx, codebook, M, N, K)
+    if y is not None:
+        return y
     import torch
     ad, d1 = _dev(a, np.float32)
     bd, d2 = _dev(b_idx, np.uint8)

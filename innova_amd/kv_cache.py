@@ -51,6 +51,8 @@ class OIL4KVCache:
 
     # ---- core operations
     def append(self, layer, k, v):
+        if (_lib._native or _lib.native()).kv_append(self._h.value, layer, k, v, self._heads * self._dim):
+            return
         import torch
         for t in (k, v):
             assert t.is_cuda and t.dtype == torch.float32 and t.is_contiguous() and t.dim() == 4
@@ -59,6 +61,9 @@ class OIL4KVCache:
         _lib.check(_lib.lib().oilhip_kv_append(self._h, layer, k.data_ptr(), v.data_ptr(), seq, _lib.current_stream()))
 
     def get_range(self, layer, start, end):
+        both = (_lib._native or _lib.native()).kv_get_range(self._h.value, layer, start, end, self._max_seq, self._heads, self._dim)
+        if both is not None:
+            return both
         import torch
         n = max(0, min(end, self._max_seq) - start)
         k = torch.empty((1, self._heads, n, self._dim), dtype=torch.float32, device="cuda")

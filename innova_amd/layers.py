@@ -20,6 +20,9 @@ def rmsnorm(x, w, out=None):
 
 def gemv_rmsnorm(w: DeviceWeights, x, norm_w, out=None):
     """y = W . rmsnorm(x; norm_w): the norm in front of a projection, formed inside the GEMV for one OIL4 row."""
+    y = (_lib._native or _lib.native()).gemv_rmsnorm(w._h, x, norm_w, out, w.rows, w.cols)
+    if y is not None:
+        return y
     import torch
     assert x.is_cuda and x.dtype == torch.float32 and x.is_contiguous() and norm_w.is_cuda and norm_w.dtype == torch.float32
     M = w._rows(x, torch.float32)
@@ -40,6 +43,9 @@ def gemv_rmsnorm(w: DeviceWeights, x, norm_w, out=None):
 def mlp_step(gate_up: DeviceWeights, down: DeviceWeights, x, out=None, norm_w=None):
     """y = down(siluf(gate x') * up x'), x' = rmsnorm(x; norm_w) or x; gate_up = the gate and up projections stacked
     (DeviceWeights.stack_rows)."""
+    y = (_lib._native or _lib.native()).mlp_step(gate_up._h, down._h, x, norm_w, out, down.rows, gate_up.cols, down.cols)
+    if y is not None:
+        return y
     import torch
     assert x.is_cuda and x.dtype == torch.float32 and x.is_contiguous()
     M, F = gate_up._rows(x, torch.float32), down.cols
@@ -58,6 +64,10 @@ def mlp_step(gate_up: DeviceWeights, down: DeviceWeights, x, out=None, norm_w=No
 
 def embed_rows(w: DeviceWeights, ids, out=None):
     """Rows ids[i] of a quantized [vocab][cols] tensor decoded to float32 [n][cols]; ids: int32 cuda tensor."""
+    if out is None:
+        y = (_lib._native or _lib.native()).embed_rows(w._h, ids, w.cols)
+        if y is not None:
+            return y
     import torch
     assert ids.is_cuda and ids.dtype == torch.int32 and ids.is_contiguous()
     n = ids.numel()

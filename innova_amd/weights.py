@@ -91,6 +91,10 @@ class DeviceWeights:
     # ---- compute ----------------------------------------------------------------
     def dequant(self, out=None):
         """All blocks decoded back to back -> float32 cuda tensor [rows*cols]."""
+        if out is None:
+            y = (_lib._native or _lib.native()).dequant(self._h, self.rows, self.cols)
+            if y is not None:
+                return y
         import torch
         if out is None:
             out = torch.empty(self.rows * self.cols, dtype=torch.float32, device="cuda")
@@ -117,6 +121,10 @@ class DeviceWeights:
         """Y[M][rows] = X[M][cols] . W^T, FP32 (decode path).  general=True forces the
         all-format kernel (used by tests to cross-check the specialised kernels); noalloc=True takes the entry
         point that allocates no device memory (uniform OIL4 only, scratch in a fixed device array)."""
+        if not general and not noalloc:
+            y = (_lib._native or _lib.native()).gemv(self._h, x, out, self.rows, self.cols)
+            if y is not None:
+                return y
         import torch
         M = self._rows(x, torch.float32)
         out = self._out(x, M, out)
@@ -131,6 +139,9 @@ class DeviceWeights:
 
     def gemm_bf16(self, x, out=None):
         """Y[M][rows] = X[M][cols] . W^T with bf16 operands on MFMA, FP32 accumulate (prefill path)."""
+        y = (_lib._native or _lib.native()).gemm(self._h, x, out, self.rows, self.cols, 1)
+        if y is not None:
+            return y
         import torch
         M = self._rows(x, torch.bfloat16)
         out = self._out(x, M, out)
@@ -140,6 +151,9 @@ class DeviceWeights:
     def gemm_f32(self, x, out=None):
         """The prefill GEMM for FP32 activations (the reference's own gemm() arguments, qwen35_engine.cpp:47-85):
         X is rounded once to bf16 inside the kernel's pre-pass; bf16 tolerance (rel-L2 <= 2e-3)."""
+        y = (_lib._native or _lib.native()).gemm(self._h, x, out, self.rows, self.cols, 0)
+        if y is not None:
+            return y
         import torch
         M = self._rows(x, torch.float32)
         out = self._out(x, M, out)
