@@ -140,7 +140,7 @@ struct MultiInput {
 };
 int launch_gemv_oil4_multi(const oilhip_weights& w, const float* d_x, const int* d_tok, float* d_y, int M, uint32_t ldx, uint32_t ldy,
                            uint32_t xrows, hipStream_t s, const MultiInput& in = {}, const oilhip_weights* w2 = nullptr, float* d_y2 = nullptr,
-                           uint32_t ldy2 = 0, uint8_t* d_pack = nullptr);
+                           uint32_t ldy2 = 0, uint8_t* d_pack = nullptr, size_t pack_room = 0);
 // several batches of one tensor shape in one launch, at most 32 rows each
 size_t gemv_oil4_multi_batches_bytes(int nb, uint64_t cols);
 int launch_gemv_oil4_multi_batches(int nb, const oilhip_weights* const* wa, float* const* ya, const oilhip_weights* const* wb, float* const* yb,

@@ -15,13 +15,16 @@
 // activations as its rows and 16 weight rows as its columns, so a lane's outputs belong to one weight row and meet one scale.
 //
 // A wavefront takes every n-th block of the row for a run of 16-row groups; the activations of its block sit in registers
-// and serve every group of the run, and the wavefronts' sums meet in LDS once per run.  There is no table to build, nothing
-// is summed across workgroups, and the order of every sum is fixed.
-// What bounds it: up to 8 tokens vector issue (about 170 instructions per block of 16 rows, beside 8 to 16 matrix instructions that
-// other wavefronts overlap; 35 to 38 % of the cycles) on the tall shapes, launch and round trips on the small ones; above, on wide rows,
-// the activations' way into the compute unit: 16 KB per block and 16 tokens, once per workgroup, at about 30 bytes per clock.  4096 x 11008
-// from 4 to 16 to 32 tokens: L2 read requests 0.96, 2.01, 3.37 M, vector instructions 1.97, 2.32, 2.95 M, 10.2, 17.9, 27.8 us (with three
-// digits, 12 KB, 17.6 us at 16 tokens and 24.8 at 32).  In batches of several tensors matrix (35 %) and vector instructions (55 %) bound it.
+// and serve every group of the run, and the wavefronts' sums meet in LDS once per run.  Where a workgroup would have few row groups,
+// several share them and cut K (best_cut): their sums meet in memory and the last to arrive adds them up in order, so the order of every sum is fixed.
+// Long launches read a byte's digits from a 64 KB table in LDS (whole_cut) instead of forming them: 8 vector instructions and 4 LDS reads
+// for eight codes.
+// What bounds it: the intake of activations, then the work on them, one after the other.  A compute unit takes in about 30 bytes per clock;
+// activations are 4 to 32 KB per block and workgroup, weights 2 KB per block and row group.  Clocks inside a workgroup (4096 x 11008, 16 tokens,
+// K whole, one row group): loads issued at 3200, the first wavefront's data at 5000 and its sums at 7900, the last one's sums at
+// 14200; the next third of K the same, the end at 33600.  On tall tensors vector issue (about 170 instructions per block of 16 rows, of which
+// 4.6 to 5 clocks each; 100 with the table) beside 8 to 56 matrix instructions (16 clocks each, 6.5 of which hold the issue back), and memory:
+// 131072 x 4096, 4 tokens 5.2 TB/s.
 // Before (FP16 halves of levels from a 64 KB LDS table, K cut between workgroups) -> now, pre-pass included, weights from memory:
 //   11008 x 4096, 4 / 8 / 16 / 32 tokens: 12.9 / 12.9 / 15.0 / 19.9 us -> 11.6 / 12.7 / 15.3 / 21.1 us
 //   4096 x 11008: 17.4 / 18.0 / 20.5 / 25.8 us -> 13.5 / 15.8 / 20.4 / 30.7 us
@@ -45,6 +48,7 @@ namespace {
 using namespace oil4;
 
 typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // Passes by token count.  The activation operand of one matrix instruction has 16 rows.  Few: up to four tokens, their
 // four digits side by side (row 4 t + d is digit d of token t), so two instructions (digits a and b of the weights) give all eight
@@ -54,17 +58,19 @@ enum PassKind { kFew4 = 0, kFew8 = 1, kDigits16 = 2, kDigits32 = 3, kPassKinds =
 __host__ __device__ constexpr bool kind_few(int k) { return k < 2; }
 __host__ __device__ constexpr int kind_tiles(int k) { return (k & 1) + 1; }
 __host__ __device__ constexpr uint32_t kind_tokens(int k) { return k == 0 ? 4u : k == 1 ? 8u : k == 2 ? 16u : 32u; }
-// packed bytes of one block: 1 KB pieces (64 lanes x 16 bytes), four per tile and operand (half of the block x even / odd nibbles)
+// packed bytes of one block: 1 KB pieces (64 lanes x 16 bytes), four per tile and operand (half of the block x half of its nibbles)
 __host__ __device__ constexpr uint32_t kind_block_bytes(int k) { return (kind_few(k) ? 4096u : 16384u) * (uint32_t)kind_tiles(k); }
 inline int kind_of(int tokens) { return tokens <= 4 ? kFew4 : tokens <= 8 ? kFew8 : tokens <= 16 ? kDigits16 : kDigits32; }
 
 // blocks of activations that a wavefront holds: as many as the registers take
-constexpr int x_slots(int kind) { return kind == kFew4 ? 4 : kind == kFew8 ? 3 : kind == kDigits16 ? 2 : 1; }
-constexpr int kMaxTokens = 32, kMaxWaves = 8;
+// (8 wavefronts per CU, 256 registers each, or 16 with 128)
+constexpr int x_slots(int kind, int waves) { return kind == kFew4 ? 4 : kind == kFew8 ? 3 : kind == kDigits16 && waves == 8 ? 2 : 1; }
+constexpr int kMaxTokens = 32;
+constexpr uint32_t kMaxSplit = 8;
 // row groups of a run
-constexpr int longest_run(int kind) { return kind == kDigits32 ? 3 : 4; }
+constexpr int longest_run(int kind, int waves) { return kind == kDigits32 ? 3 : waves == 16 ? 2 : 4; }
 constexpr int lane_outputs(int kind) { return kind_tiles(kind) * (kind_few(kind) ? 1 : 4); }
-constexpr uint32_t kMaxKeep = 48u * 1024u;                                 // bytes of LDS for sums that are carried from part to part
+constexpr uint32_t kMaxKeep = 24u * 1024u, kMaxKeepNoTable = 48u * 1024u;  // bytes of LDS for sums that are carried from part to part
 
 // ---- pre-pass: activations to digits in operand order -----------------------------------------------------------------
 // A wavefront takes one (token, block): 256 columns as one 16-byte load per lane, optionally silu(x) * x2 or the RMSNorm's
@@ -99,6 +105,8 @@ struct PackArgs {
     uint8_t* xp;                // undo floats at the start, then the blocks
     uint32_t bpr, xrows;
     int M, kind;
+    uint32_t* arrived;          // counters that the main launch wants zero
+    uint32_t ncount;
 };
 
 // this lane's four columns of block `blk` of row `src`
@@ -164,33 +172,47 @@ __device__ __forceinline__ float block_to_digits(float (&v)[4], uint32_t lane, P
     return bad ? __uint_as_float(0x7FC00000u) : ldexpf(1.0f, -ex);
 }
 
+// BY_TABLE: in the order of multi_body's TABLE.  (One batch, without the jobs: 1.4 KB of arguments cost the host 1.2 us of a launch.)
+template <bool BY_TABLE>
+__device__ __forceinline__ void pack_body(PackArgs a, uint32_t bid, uint32_t jobs, bool use_list, uint32_t row0, const int16_t* list);
+
+template <bool BY_TABLE>
 __global__ void __launch_bounds__(256)
-pack_digits_kernel(PackArgs a, const PackJobs jobs) {
+pack_digits_kernel(const PackArgs a) {
+    if (blockIdx.x == 0) for (uint32_t i = threadIdx.x; i < a.ncount; i += 256u) a.arrived[i] = 0u;
+    pack_body<BY_TABLE>(a, blockIdx.x, 0u, false, 0u, nullptr);
+}
+__global__ void __launch_bounds__(256)
+pack_digits_jobs_kernel(PackArgs a, const PackJobs jobs) {
+    uint32_t j = 0, bid = blockIdx.x;
+    while (j + 1u < jobs.n && bid >= jobs.begin[j + 1u]) ++j;              // uniform
+    a.M = jobs.M[j]; a.kind = jobs.kind[j]; a.xp += jobs.xp_off[j];
+    pack_body<false>(a, bid - jobs.begin[j], jobs.n, jobs.use_list, jobs.row0[j], jobs.list);
+}
+
+template <bool BY_TABLE>
+__device__ __forceinline__ void pack_body(PackArgs a, uint32_t bid, uint32_t jobs, bool use_list, uint32_t row0, const int16_t* list) {
     __shared__ __align__(16) uint8_t lds[4][1024];
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    uint32_t bid = blockIdx.x;
-    int row0 = 0;
-    if (jobs.n) {
-        uint32_t j = 0;
-        while (j + 1u < jobs.n && bid >= jobs.begin[j + 1u]) ++j;          // uniform
-        bid -= jobs.begin[j];
-        a.M = jobs.M[j]; a.kind = jobs.kind[j]; a.xp += jobs.xp_off[j];
-        row0 = jobs.row0[j];
-    }
     // workgroup = four tokens of one block
     const uint32_t blk = bid % a.bpr, t = (bid / a.bpr) * 4u + wave;
     uint32_t src = 0xFFFFFFFFu;
-    if ((int)t < a.M) src = jobs.n ? (jobs.use_list ? (uint32_t)jobs.list[row0 + t] : (uint32_t)row0 + t) : a.tok ? (uint32_t)a.tok[t] : t;
+    if ((int)t < a.M) src = jobs ? (use_list ? (uint32_t)list[row0 + t] : row0 + t) : a.tok ? (uint32_t)a.tok[t] : t;
     float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     if (src < a.xrows) load_activations(a.in, src, blk, a.bpr, lane, v);
-    // digit d of nibble p at byte d * 256 + ((2 (p / 128) + p % 2) * 4 + (p / 32) % 4) * 16 + (p % 32) / 2: 16-byte pieces by (operand, lane group)
+    // digit d of nibble p at byte d * 256 + ((2 (p / 128) + s) * 4 + (p / 32) % 4) * 16 + i: 16-byte pieces by (operand, lane group); the
+    // operands of a half are its even and odd nibbles, s = p % 2 and i = (p % 32) / 2, or by table the halves of a lane's 32
+    auto place = [&](uint32_t p) {
+        const uint32_t sub = BY_TABLE ? (p >> 4) & 1u : p & 1u, i = BY_TABLE ? p & 15u : (p & 31u) >> 1;
+        return (((p >> 7) * 2u + sub) * 4u + ((p >> 5) & 3u)) * 16u + i;
+    };
     uint8_t* mine = lds[wave];
     if (lane < 4u) {
-        const uint32_t at = (lane & 1u) * 64u + (lane >> 1);
+        const uint32_t at = place(lane);
         mine[at] = 0; mine[256u + at] = 0; mine[512u + at] = 0; mine[768u + at] = 0;
     }
     const float undo = block_to_digits(v, lane, [&](int, uint32_t p, uint32_t bytes) {
-        const uint32_t at = (((p >> 7) * 2u + (p & 1u)) * 4u + ((p >> 5) & 3u)) * 16u + ((p & 31u) >> 1);
+        const uint32_t at = place(p);
         mine[at] = (uint8_t)bytes; mine[256u + at] = (uint8_t)(bytes >> 8); mine[512u + at] = (uint8_t)(bytes >> 16); mine[768u + at] = (uint8_t)(bytes >> 24);
     });
     const uint32_t tokens = kind_few(a.kind) ? 4u : 16u, tile = t / tokens, tt = t - tile * tokens;
@@ -231,6 +253,26 @@ struct Sums {                                                              // on
     }
 };
 
+// Digits of a packed byte, 64 KB at LDS offset 0: entry of byte value v at byte 256 v + 4 lane (a copy per lane: no bank conflicts),
+// {a, b} of its low nibble, {a, b} of its high one.
+constexpr uint32_t kDigitTab = 65536u;
+__device__ __forceinline__ void build_digit_table(uint8_t* lds) {
+    const uint32_t lane = threadIdx.x & 63u;
+    for (uint32_t q = threadIdx.x >> 6; q < 64u; q += blockDim.x >> 6) {   // four entries at a time: byte values 4 q + lane / 16
+        uint32_t a, b;
+        level_digits(((q & 3u) * 4u + (lane >> 4)) | (q >> 2) << 8, a, b);
+        const uint32_t e = __builtin_amdgcn_perm(b, a, 0x05010400u);
+        reinterpret_cast<uint4*>(lds)[q * 64u + lane] = make_uint4(e, e, e, e);
+    }
+}
+// the entries of a dword's four bytes; `lane4`: 4 * lane
+__device__ __forceinline__ void digit_entries(uint32_t w, uint32_t lane4, uint32_t* e) {
+    e[0] = *(lds_cuint*)(uintptr_t)__builtin_amdgcn_perm(w, lane4, 0x0C0C0400u);
+    e[1] = *(lds_cuint*)(uintptr_t)__builtin_amdgcn_perm(w, lane4, 0x0C0C0500u);
+    e[2] = *(lds_cuint*)(uintptr_t)__builtin_amdgcn_perm(w, lane4, 0x0C0C0600u);
+    e[3] = *(lds_cuint*)(uintptr_t)__builtin_amdgcn_perm(w, lane4, 0x0C0C0700u);
+}
+
 struct BodyArgs {
     const uint8_t* W;
     const uint8_t* xp;             // packed activations
@@ -239,22 +281,31 @@ struct BodyArgs {
     uint32_t parts, part_blocks;   // the row's blocks, cut so that the wavefronts hold the activations of a part
     uint32_t chunk;                // groups that go through all parts together: their sums wait in LDS
     int M;
+    uint32_t part0 = 0;            // this workgroup walks parts part0 to parts - 1
+};
+
+// K cut between workgroups: `n` workgroups (1: no cut) share the rows and take each parts / n parts (rounded up).  Their sums meet
+// in memory, [workgroup][token][row], and the last of them to arrive adds them up in order.
+struct Split {
+    uint32_t n = 1, each = 0, ld = 0;
+    float* partial = nullptr;
+    uint32_t* arrived = nullptr;
 };
 
 // G: row groups of a run.  Workgroups of a runtime number of at most kMaxWaves wavefronts, so that a part's blocks divide
 // evenly among them; one that has a block less than the others takes the last one again, scaled by 0.  A workgroup walks the
 // runs of a chunk of its groups for one part of the rows after the other: activations that are fetched once per part cost nothing, fetched
 // once per run they cost as much as the products (37449 x 14336, 16 tokens: 98 us against 73).  The sums wait in LDS.
-template <int KIND, int G>
+template <int KIND, int G, int kMaxWaves, bool TABLE, bool SPLIT>
 __device__ __forceinline__ void
-multi_body(const BodyArgs& a, uint32_t g_begin, uint32_t g_end, float* red) {
+multi_body(const BodyArgs& a, uint32_t g_begin, uint32_t g_end, float* lds, float* partial = nullptr, uint32_t ldp = 0) {
     constexpr bool FEW = kind_few(KIND);
     constexpr int NT = kind_tiles(KIND), PER = FEW ? 1 : 4, DIG = FEW ? 1 : 4;   // outputs of a lane per tile, operand pieces per half and parity
-    constexpr int XD = x_slots(KIND);
+    constexpr int XD = x_slots(KIND, kMaxWaves);
     constexpr int WD = G < 3 ? XD : 1;                                     // weights in flight: the run's, for short runs of all blocks of the part
     const uint32_t lane = threadIdx.x & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), waves = blockDim.x >> 6;
     const uint32_t li = lane & 15u, kq = lane >> 4;
-    const uint32_t row_bytes = a.bpr * 128u, bpr = a.bpr;
+    const uint32_t row_bytes = a.bpr * 128u, bpr = a.bpr, part0 = SPLIT ? a.part0 : 0u;
     const uint32_t iters = (a.part_blocks + waves - 1u) / waves;           // blocks per wavefront and part, at most XD
     // this workgroup's rows: 32-bit offsets from its first group
     const uint8_t* base = a.W + (size_t)g_begin * 16u * row_bytes;
@@ -262,6 +313,11 @@ multi_body(const BodyArgs& a, uint32_t g_begin, uint32_t g_end, float* red) {
     const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(base), (short)0, (int)0xFFFFFFFFu, 0x00020000);
     const float* undo = reinterpret_cast<const float*>(a.xp);
     const uint8_t* xblocks = a.xp + undo_bytes(bpr);
+    // five to eight tokens: rows of absent ones in the second tile repeat a present one, and nothing more is fetched (5 tokens, 4096 x 4096
+    // 8.95 -> 8.40 us; for the other sizes level)
+    uint32_t xlane[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) xlane[t] = KIND == kFew8 && t == 1 ? kq * 16u + min(li >> 2, (uint32_t)a.M - 5u) * 4u + (li & 3u) : lane;
     const uint32_t scale_lane = li * 4u;                                   // ds_bpermute address of lane li: it holds the block's scale
     auto place = [&](uint32_t part, uint32_t i) { const uint32_t b = wave + i * waves; return b < a.part_blocks ? part * a.part_blocks + b : 0xFFFFFFFFu; };
     auto block_at = [&](uint32_t part, uint32_t i) { const uint32_t b = place(part, i); return b < bpr ? b : bpr - 1u; };
@@ -283,7 +339,7 @@ multi_body(const BodyArgs& a, uint32_t g_begin, uint32_t g_end, float* red) {
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
-            for (int d = 0; d < DIG; ++d) x[slot][t][d][o] = p[((t * DIG + d) * 4 + o) * 64 + (int)lane];
+            for (int d = 0; d < DIG; ++d) x[slot][t][d][o] = p[((t * DIG + d) * 4 + o) * 64 + (int)xlane[t]];
     };
     auto load_undo = [&](int slot, uint32_t blk) {
         const float* u = undo + blk * (uint32_t)kMaxTokens;
@@ -307,21 +363,28 @@ multi_body(const BodyArgs& a, uint32_t g_begin, uint32_t g_end, float* red) {
                 load_undo(s, blk);
             }
     };
-    load_part(0u);                                                         // activations first: loads return in order
+    load_part(part0);                                                      // activations first: loads return in order
 #pragma unroll
     for (int s = 0; s < WD; ++s)
         if (s == 0 || (uint32_t)s < iters)
 #pragma unroll
-            for (int g = 0; g < G; ++g) load_w(s, g, 0u, 0u, (uint32_t)s);
+            for (int g = 0; g < G; ++g) load_w(s, g, part0, 0u, (uint32_t)s);
     // a barrier for LDS alone: __syncthreads() would also wait for the weights that are in flight
     auto lds_barrier = [&]() {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
     };
-    constexpr uint32_t OUT = (uint32_t)(G * NT * PER) * 64u, AREA = (uint32_t)kMaxWaves * OUT;
+    if constexpr (TABLE) {
+        build_digit_table(reinterpret_cast<uint8_t*>(lds));
+        lds_barrier();
+    }
+    const uint32_t lane4 = 4u * lane;
+    float* red = lds + (TABLE ? kDigitTab / 4u : 0u);
+    constexpr uint32_t OUT = (uint32_t)(G * NT * PER) * 64u;
+    const uint32_t held = kMaxWaves == 8 ? 8u : (waves + 3u) & ~3u, AREA = held * OUT;   // wavefronts that sums are held for
     float* keep = red + 2u * AREA;                                         // sums of the parts before, by run
-    if (waves < (uint32_t)kMaxWaves) {                                     // the sums of absent wavefronts read as zero
+    if (waves < held) {                                                  // the sums of absent wavefronts read as zero
         for (uint32_t o = waves * OUT + threadIdx.x; o < AREA; o += blockDim.x) { red[o] = 0.0f; red[AREA + o] = 0.0f; }
     }
 
@@ -336,7 +399,7 @@ multi_body(const BodyArgs& a, uint32_t g_begin, uint32_t g_end, float* red) {
         if (WD > 1 || ni >= iters) { ni = WD > 1 ? i : 0u; nrun += G; }
         if (nrun >= chunk_end) {
             if (npart + 1u < a.parts) { ++npart; nrun = chunk_begin; }
-            else { npart = 0u; nrun = chunk_end < ngroups ? chunk_end : 0u; }
+            else { npart = part0; nrun = chunk_end < ngroups ? chunk_end : 0u; }
         }
 #pragma unroll
         for (int g = 0; g < G; ++g) {
@@ -348,13 +411,24 @@ multi_body(const BodyArgs& a, uint32_t g_begin, uint32_t g_end, float* red) {
             float scale = __half2float(__ushort_as_half((unsigned short)__builtin_amdgcn_ds_bpermute((int)scale_lane, (int)w[WS][g][0].x)));
             scale = spare ? 0.0f : scale * kScaleUnit;
 #pragma unroll
-            for (int o = 0; o < 4; ++o) {                                  // operand: half o / 2 of the block, even or odd nibbles
+            for (int o = 0; o < 4; ++o) {                                  // operand: half o / 2 of the block, half of its nibbles
                 i32x4 da, db;
 #pragma unroll
                 for (int d = 0; d < 4; ++d) {
-                    uint32_t ad, bd;
-                    level_digits((o & 1) ? w[WS][g][o >> 1][d] >> 4 : w[WS][g][o >> 1][d], ad, bd);
-                    da[d] = (int)ad; db[d] = (int)bd;
+                    if constexpr (!TABLE) {
+                        uint32_t ad, bd;
+                        level_digits((o & 1) ? w[WS][g][o >> 1][d] >> 4 : w[WS][g][o >> 1][d], ad, bd);
+                        da[d] = (int)ad; db[d] = (int)bd;
+                    } else if (d == 0) {
+                        uint32_t e[8];
+                        digit_entries(w[WS][g][o >> 1][(o & 1) * 2], lane4, e);
+                        digit_entries(w[WS][g][o >> 1][(o & 1) * 2 + 1], lane4, e + 4);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            da[i] = (int)__builtin_amdgcn_perm(e[2 * i + 1], e[2 * i], 0x06040200u);
+                            db[i] = (int)__builtin_amdgcn_perm(e[2 * i + 1], e[2 * i], 0x07050301u);
+                        }
+                    }
                 }
 #pragma unroll
                 for (int t = 0; t < NT; ++t) {
@@ -397,21 +471,30 @@ multi_body(const BodyArgs& a, uint32_t g_begin, uint32_t g_end, float* red) {
         for (uint32_t o = threadIdx.x; o < OUT; o += blockDim.x) {
             float p[kMaxWaves];
 #pragma unroll
-            for (int wv = 0; wv < kMaxWaves; ++wv) p[wv] = area[(uint32_t)wv * OUT + o];
+            for (uint32_t wv = 0; wv < (uint32_t)kMaxWaves; ++wv) p[wv] = area[(kMaxWaves == 8 || wv < 4u || (wv & ~3u) < held ? wv : 0u) * OUT + o];   // all in flight
             float s = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+            if constexpr (kMaxWaves == 16) {
+                s = held > 4u ? s : (p[0] + p[1]) + (p[2] + p[3]);
+                s = held > 8u ? s + ((p[8] + p[9]) + (p[10] + p[11])) : s;
+                s = held > 12u ? s + ((p[12] + p[13]) + (p[14] + p[15])) : s;
+            }
             float* k = keep + ((run % a.chunk) / G) * OUT + o;             // this thread's own from part to part
-            if (part) s += *k;
+            if (part > part0) s += *k;
             if (part + 1u < a.parts) { *k = s; continue; }
             const uint32_t l = o & 63u, e = o >> 6, v = e % PER, t = (e / PER) % NT, g = e / (PER * NT);
             const uint32_t token = FEW ? 4u * t + (l >> 4) : 16u * t + 4u * (l >> 4) + v;
             const uint32_t r = (g_begin + run + g) * 16u + (l & 15u);
-            if (run + g < ngroups && r < a.rows && (int)token < a.M) a.y[(size_t)token * a.ldy + r] = s * kAccUnit;
+            if (run + g < ngroups && r < a.rows && (int)token < a.M) {
+                // (stores that are coherent across the device by themselves: a release fence would write a whole L2 back)
+                if (SPLIT) __hip_atomic_store(partial + (size_t)token * ldp + r, s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                else a.y[(size_t)token * a.ldy + r] = s * kAccUnit;
+            }
         }
     };
     uint32_t odd = 0, done_part = 0, done_run = 0xFFFFFFFFu;
     for (; chunk_begin < ngroups; chunk_begin = chunk_end, chunk_end = chunk_end + a.chunk < ngroups ? chunk_end + a.chunk : ngroups)
-    for (uint32_t part = 0; part < a.parts; ++part) {
-        if (a.parts > 1u && (part || chunk_begin)) load_part(part);
+    for (uint32_t part = part0; part < a.parts; ++part) {
+        if (a.parts > part0 + 1u && (part > part0 || chunk_begin)) load_part(part);
         for (uint32_t run = chunk_begin; run < chunk_end; run += G) {
             // the run before: its sums are complete since the barrier; the area is written again after the next barrier
             if (done_run != 0xFFFFFFFFu) finish(done_part, done_run, red + (odd ^ 1u) * AREA);
@@ -440,81 +523,201 @@ multi_body(const BodyArgs& a, uint32_t g_begin, uint32_t g_end, float* red) {
     finish(done_part, done_run, red + (odd ^ 1u) * AREA);
 }
 
-template <int KIND, int G>
-__global__ void __launch_bounds__(64 * kMaxWaves) __attribute__((amdgpu_waves_per_eu(2, 2)))
+template <int KIND, int G, int W, bool TABLE>
+__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W / 4, W / 4)))
 gemv_oil4_multi_kernel(const BodyArgs a, uint32_t g_base, uint32_t g_rem) {
-    extern __shared__ __align__(16) float red[];
+    extern __shared__ __align__(16) float lds[];
     const uint32_t b = blockIdx.x, g0 = b * g_base + (b < g_rem ? b : g_rem);
-    multi_body<KIND, G>(a, g0, g0 + g_base + (b < g_rem ? 1u : 0u), red);
+    multi_body<KIND, G, W, TABLE, false>(a, g0, g0 + g_base + (b < g_rem ? 1u : 0u), lds);
+}
+
+// K cut between workgroups.  Workgroups are dealt to the eight XCDs in turn, so neighbours in blockIdx take different parts: with two,
+// four or eight parts an XCD's L2 holds one part of the activations.
+template <int KIND, int G, int W, bool TABLE>
+__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W / 4, W / 4)))
+gemv_oil4_multi_split_kernel(BodyArgs a, uint32_t g_base, uint32_t g_rem, const Split sp) {
+    extern __shared__ __align__(16) float lds[];
+    const uint32_t b = blockIdx.x / sp.n, mine = blockIdx.x - b * sp.n, g0 = b * g_base + (b < g_rem ? b : g_rem), g1 = g0 + g_base + (b < g_rem ? 1u : 0u);
+    const uint32_t all = a.parts;
+    a.part0 = mine * sp.each;
+    a.parts = a.part0 + sp.each < all ? a.part0 + sp.each : all;
+    multi_body<KIND, G, W, TABLE, true>(a, g0, g1, lds, sp.partial + (size_t)mine * a.M * sp.ld, sp.ld);
+    uint32_t* order = reinterpret_cast<uint32_t*>(lds);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // this thread's sums are in place before the barrier, the others' before theirs
+    __syncthreads();
+    if (threadIdx.x == 0) *order = __hip_atomic_fetch_add(sp.arrived + b, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (*order + 1u != sp.n) return;
+    // four rows of a token at a time, all parts' loads in flight together (rows are padded to sixteen)
+    const uint32_t r0 = 16u * g0, quads = 4u * (g1 - g0);
+    const auto sums = __builtin_amdgcn_make_buffer_rsrc(sp.partial, (short)0, 0x7FFFFFFF, 0x00020000);
+    for (uint32_t o = threadIdx.x; o < quads * (uint32_t)a.M; o += blockDim.x) {
+        const uint32_t token = o / quads, r = r0 + 4u * (o - token * quads);
+        f32x4 p[kMaxSplit];
+        const uint32_t at = (token * sp.ld + r) * 4u, step = (uint32_t)a.M * sp.ld * 4u;
+#pragma unroll
+        for (uint32_t i = 0; i < kMaxSplit; ++i)           // 16: sc1, past the XCD's own cache; beyond the parts: out of range, zeros
+            p[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(sums, i < sp.n ? at + i * step : 0x80000000u, 0, 16));
+        f32x4 s = p[0];
+#pragma unroll
+        for (uint32_t i = 1; i < kMaxSplit; ++i) s += p[i];
+        float* y = a.y + (size_t)token * a.ldy + r;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (r + e < a.rows) y[e] = s[e] * 1.6384f;
+    }
+    if (threadIdx.x == 0) __hip_atomic_store(sp.arrived + b, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // for the next launch on these activations
 }
 
 // Batches of different pass sizes side by side: the job's pass size selects the body.
-__global__ void __launch_bounds__(64 * kMaxWaves) __attribute__((amdgpu_waves_per_eu(2, 2)))
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 gemv_oil4_multi_jobs_kernel(const uint8_t* __restrict__ xp, uint32_t rows, uint32_t bpr, uint32_t ldy, const PartsOf parts, const MultiJobs jobs) {
-    extern __shared__ __align__(16) float red[];
+    extern __shared__ __align__(16) float lds[];
     uint32_t j = 0;
     while (j + 1u < jobs.n && blockIdx.x >= jobs.wg_begin[j + 1u]) ++j;    // uniform
     const uint32_t b = blockIdx.x - jobs.wg_begin[j], gb = jobs.g_base[j], gr = jobs.g_rem[j], kind = jobs.kind[j];
     const uint32_t g0 = b * gb + (b < gr ? b : gr), g1 = g0 + gb + (b < gr ? 1u : 0u);
     const BodyArgs a{jobs.W[j], xp + jobs.xp_off[j], jobs.y[j], rows, bpr, ldy, parts.n[kind], parts.blocks[kind], parts.chunk[kind], jobs.M[j]};
     switch (kind) {
-        case kFew4: multi_body<kFew4, longest_run(kFew4)>(a, g0, g1, red); break;
-        case kFew8: multi_body<kFew8, longest_run(kFew8)>(a, g0, g1, red); break;
-        case kDigits16: multi_body<kDigits16, longest_run(kDigits16)>(a, g0, g1, red); break;
-        default: multi_body<kDigits32, longest_run(kDigits32)>(a, g0, g1, red); break;
+        case kFew4: multi_body<kFew4, longest_run(kFew4, 8), 8, false, false>(a, g0, g1, lds); break;
+        case kFew8: multi_body<kFew8, longest_run(kFew8, 8), 8, false, false>(a, g0, g1, lds); break;
+        case kDigits16: multi_body<kDigits16, longest_run(kDigits16, 8), 8, false, false>(a, g0, g1, lds); break;
+        default: multi_body<kDigits32, longest_run(kDigits32, 8), 8, false, false>(a, g0, g1, lds); break;
     }
 }
 
 // How a row's blocks are cut into parts of at most x_slots blocks per wavefront, and the wavefronts of a workgroup: as many as
 // divide a part with the least left over.
-void cut_row(int kind, uint32_t bpr, uint32_t& parts, uint32_t& part_blocks) {
-    const uint32_t most = (uint32_t)(kMaxWaves * x_slots(kind));
+void cut_row(int kind, int max_waves, uint32_t bpr, uint32_t& parts, uint32_t& part_blocks) {
+    const uint32_t most = (uint32_t)(max_waves * x_slots(kind, max_waves));
     parts = (bpr + most - 1u) / most;
     part_blocks = (bpr + parts - 1u) / parts;
     parts = (bpr + part_blocks - 1u) / part_blocks;
 }
-uint32_t waves_of(uint32_t blocks) { const uint32_t each = (blocks + kMaxWaves - 1u) / kMaxWaves; return (blocks + each - 1u) / each; }
+uint32_t waves_of(int max_waves, uint32_t blocks) { const uint32_t each = (blocks + (uint32_t)max_waves - 1u) / (uint32_t)max_waves; return (blocks + each - 1u) / each; }
 // groups whose sums may wait in LDS between parts (a multiple of every run length), and the LDS of a workgroup with `most` groups
-constexpr uint32_t chunk_of(int kind) { return kMaxKeep / ((uint32_t)lane_outputs(kind) * 256u) / 12u * 12u; }
-size_t lds_of(int kind, int g, uint32_t parts, uint32_t most) {
-    const size_t unit = (size_t)lane_outputs(kind) * 256u, waiting = std::min((most + g - 1u) / g * g, chunk_of(kind));
-    return unit * (2u * kMaxWaves * g + (parts > 1u ? waiting : 0u));
+constexpr uint32_t chunk_of(int kind, bool table) { return (table ? kMaxKeep : kMaxKeepNoTable) / ((uint32_t)lane_outputs(kind) * 256u) / 12u * 12u; }
+size_t lds_of(int kind, int max_waves, uint32_t waves, bool table, int g, uint32_t parts, uint32_t most) {
+    const size_t unit = (size_t)lane_outputs(kind) * 256u, waiting = std::min((most + g - 1u) / g * g, chunk_of(kind, table));
+    return (table ? kDigitTab : 0u) + unit * (2u * (max_waves == 8 ? 8u : (waves + 3u) & ~3u) * g + (parts > 1u ? waiting : 0u));
 }
 
-template <int KIND, int G>
-int launch_one(const BodyArgs& a, uint32_t wgs, uint32_t most, hipStream_t s) {
-    static std::atomic<uint64_t> raised{0};
-    if (int rc = ensure_max_lds(raised, (const void*)gemv_oil4_multi_kernel<KIND, G>, kMaxLds)) return rc;
-    const uint32_t groups = (a.rows + 15u) / 16u;
-    hipLaunchKernelGGL((gemv_oil4_multi_kernel<KIND, G>), dim3(wgs), dim3(64u * waves_of(a.part_blocks)), lds_of(KIND, G, a.parts, most), s, a,
-                       groups / wgs, groups % wgs);
-    OILHIP_HIP(hipGetLastError());
-    return OILHIP_OK;
-}
-
-template <int KIND>
-int launch_kind(BodyArgs a, hipStream_t s) {
-    cut_row(KIND, a.bpr, a.parts, a.part_blocks);
-    a.chunk = a.parts > 1u ? chunk_of(KIND) : 0x7FFFFFFFu;
-    // eight wavefronts per CU (the registers of two per SIMD)
-    const uint32_t groups = (a.rows + 15u) / 16u, slots = (uint32_t)device_cu_count() * std::max(1u, (uint32_t)kMaxWaves / waves_of(a.part_blocks));
-    const uint32_t wgs = std::min(groups, slots), most = (groups + wgs - 1u) / wgs;
+// How a launch cuts the tensor.
+struct Cut {
+    uint32_t parts, part_blocks, wgs, most;                                // parts of a row, workgroups along the rows, row groups of the fullest
+    uint32_t split, each;                                                  // workgroups along K, parts of each
+    int waves, run;                                                        // most wavefronts of a workgroup, row groups of a run
+    bool table;                                                            // digits from the table in LDS
+};
+Cut cut_for(int kind, int waves, bool table, uint32_t rows, uint32_t bpr, uint32_t split) {
+    Cut c{};
+    c.waves = waves; c.table = table;
+    cut_row(kind, waves, (bpr + split - 1u) / split, c.each, c.part_blocks);
+    c.parts = (bpr + c.part_blocks - 1u) / c.part_blocks;
+    c.split = (c.parts + c.each - 1u) / c.each;
+    // eight or sixteen wavefronts per CU, as far as LDS goes
+    const uint32_t groups = (rows + 15u) / 16u, w = waves_of(waves, c.part_blocks), cus = (uint32_t)device_cu_count();
+    const uint32_t fit = (uint32_t)(kMaxLds / lds_of(kind, waves, w, table, longest_run(kind, waves), c.each, 1u << 20));
+    c.wgs = std::max(1u, std::min(groups, cus * std::max(1u, std::min((uint32_t)waves / w, fit)) / c.split));
+    c.most = (groups + c.wgs - 1u) / c.wgs;
     // The longest run that divides the fullest workgroup's groups: a run that is not full costs as much as a full one.  Over 136
     // measured shapes (256 to 3000 groups, 2048 to 11008 columns, 4 to 32 tokens) 2.2 % behind the best run length on average, 16 % at most;
     // 16384 x 11008, 32 tokens: runs of 2 / 3 for 4 groups 55 / 78 us; 20480 x 4096, 8 tokens: 1 / 3 / 4 for 5 groups 17.0 / 18.6 / 23.6 us.
-    if constexpr (longest_run(KIND) == 4)
-        if (most % 4u == 0u) return launch_one<KIND, 4>(a, wgs, most, s);
-    if (most % 3u == 0u) return launch_one<KIND, 3>(a, wgs, most, s);
-    if (most % 2u == 0u) return launch_one<KIND, 2>(a, wgs, most, s);
-    return launch_one<KIND, 1>(a, wgs, most, s);
+    c.run = longest_run(kind, waves);
+    while (c.most % (uint32_t)c.run) --c.run;
+    return c;
+}
+// Without a cut along K.  Sixteen wavefronts and the table for 9 to 16 tokens where eight would not fill the SIMDs evenly, or walk many runs
+// of one group (8448 x 2816, 16 tokens 13.1 -> 12.3 us, 20000 x 8192 34.1 -> 32.0; 12288 x 4096 stays, 14.7 against 15.2); up to 8 tokens the
+// table alone where a wavefront has enough to do to earn its 0.5 us (131072 x 4096, 4 / 8 tokens 60.6 / 66.5 -> 57.1 / 63.1).
+Cut whole_cut(int kind, uint32_t rows, uint32_t bpr) {
+    Cut c = cut_for(kind, 8, false, rows, bpr, 1u);
+    const uint32_t w = waves_of(8, c.part_blocks);
+    if (kind == kDigits16 && (w < 8u ? bpr > 8u : c.most >= 16u || (c.run == 1 && c.most >= 5u))) return cut_for(kind, 16, true, rows, bpr, 1u);
+    if (kind_few(kind) && c.most * c.each * ((c.part_blocks + w - 1u) / w) >= 16u) return cut_for(kind, 8, true, rows, bpr, 1u);
+    return c;
+}
+// Where a workgroup has few row groups, what it takes in is mostly activations: K is cut between workgroups then.  The line is an estimate in
+// us that counts a workgroup's bytes of activations, its work and what the meeting of the sums costs; it was fitted to 1 to 8 parts on
+// 25 shapes (300 to 131072 rows, 1024 to 14336 columns), and on them its choice is 1.5 % slower than the best on average, 15 % at most, and never slower than no
+// cut by more than 3 %.  5 tokens, 1 / best: 600 x 14336 16.7 / 10.2 us, 5120 x 13824 25.3 / 18.3; 16 tokens 4096 x 11008 20.7 / 17.2;
+// 32 tokens 32.5 / 24.4; 4096 x 4096 stays whole up to 16 tokens (10.7 / 11.9 for 16).
+Cut best_cut(int kind, uint32_t rows, uint32_t bpr) {
+    static const struct { double x, weights, unit, run, meet, meet_part, sums; } kCost[kPassKinds] = {
+        {1.59e-5, 0.0, 0.517, 0.131, 1.95, 0.19, 0.43}, {0.92e-5, 0.0, 0.574, 0.103, 2.01, 0.19, 0.0},
+        {0.99e-5, 7.0e-5, 0.0, 0.0, 2.65, 0.27, 0.0}, {0.96e-5, 11.3e-5, 0.0, 0.039, 1.91, 0.37, 0.0}};
+    const auto& k = kCost[kind];
+    Cut best = whole_cut(kind, rows, bpr);
+    const double x_block = (double)kind_block_bytes(kind);
+    if (x_block * bpr < 96e3) return best;
+    auto cost = [&](const Cut& c) {
+        const uint32_t w = waves_of(c.waves, c.part_blocks), blocks = c.part_blocks * c.each, cus = (uint32_t)device_cu_count();
+        const double turns = (double)((c.wgs * c.split + cus - 1u) / cus), side = std::max(1.0, w * turns / 4.0);
+        const double units = (double)(c.most * c.each * ((c.part_blocks + w - 1u) / w)) * side;
+        double t = turns * blocks * (k.x * x_block + k.weights * 2048.0 * c.most) + k.unit * units + k.run * (double)(c.each * (c.most / (uint32_t)c.run));
+        if (c.split > 1u) t += k.meet + k.meet_part * c.split + k.sums * c.split * c.most * kind_tokens(kind) / 256.0;
+        return t;
+    };
+    // the estimate of the whole row is for the forms that it was fitted on; 4.6 us are in all of them
+    double least = (4.6 + cost(cut_for(kind, 8, false, rows, bpr, 1u))) * (kind == kDigits32 ? 0.92 : 0.97) - 4.6;
+    for (uint32_t n : {2u, 3u, 4u, 5u, 6u, 8u}) {
+        const Cut c = kind == kDigits16 ? cut_for(kind, 16, true, rows, bpr, n) : cut_for(kind, 8, false, rows, bpr, n);
+        if (c.split != n) continue;
+        const double t = cost(c);
+        if (t < least) { least = t; best = c; }
+    }
+    return best;
+}
+// bytes of a split launch's counters and sums
+size_t split_bytes(const Cut& c, uint32_t rows, int M) {
+    return c.split < 2u ? 0u : (((size_t)c.wgs * 4u + 255u) & ~(size_t)255u) + (size_t)c.split * (size_t)M * ((rows + 15u) & ~15u) * 4u;
 }
 
-int launch_main(int kind, const BodyArgs& a, hipStream_t s) {
+template <int KIND, int G, int W, bool TABLE, bool SPLIT>
+int launch_one(const BodyArgs& a, const Cut& c, const Split& sp, hipStream_t s) {
+    static std::atomic<uint64_t> raised{0};
+    const uint32_t groups = (a.rows + 15u) / 16u, waves = waves_of(W, a.part_blocks);
+    const size_t lds = lds_of(KIND, W, waves, TABLE, G, c.each, c.most);
+    if constexpr (SPLIT) {
+        if (int rc = ensure_max_lds(raised, (const void*)gemv_oil4_multi_split_kernel<KIND, G, W, TABLE>, kMaxLds)) return rc;
+        hipLaunchKernelGGL((gemv_oil4_multi_split_kernel<KIND, G, W, TABLE>), dim3(c.wgs * c.split), dim3(64u * waves), lds, s, a, groups / c.wgs, groups % c.wgs, sp);
+    } else {
+        if (int rc = ensure_max_lds(raised, (const void*)gemv_oil4_multi_kernel<KIND, G, W, TABLE>, kMaxLds)) return rc;
+        hipLaunchKernelGGL((gemv_oil4_multi_kernel<KIND, G, W, TABLE>), dim3(c.wgs), dim3(64u * waves), lds, s, a, groups / c.wgs, groups % c.wgs);
+    }
+    OILHIP_HIP(hipGetLastError());
+    return OILHIP_OK;
+}
+template <int KIND, int W, bool TABLE, bool SPLIT>
+int launch_run(const BodyArgs& a, const Cut& c, const Split& sp, hipStream_t s) {
+    constexpr int LONGEST = longest_run(KIND, W);
+    if constexpr (LONGEST >= 4) if (c.run == 4) return launch_one<KIND, 4, W, TABLE, SPLIT>(a, c, sp, s);
+    if constexpr (LONGEST >= 3) if (c.run == 3) return launch_one<KIND, 3, W, TABLE, SPLIT>(a, c, sp, s);
+    if (c.run == 2) return launch_one<KIND, 2, W, TABLE, SPLIT>(a, c, sp, s);
+    return launch_one<KIND, 1, W, TABLE, SPLIT>(a, c, sp, s);
+}
+template <int KIND>
+int launch_kind(BodyArgs a, const Cut& c, const Split& sp, hipStream_t s) {
+    a.parts = c.parts;
+    a.part_blocks = c.part_blocks;
+    a.chunk = c.each > 1u ? chunk_of(KIND, c.table) : 0x7FFFFFFFu;
+    if constexpr (KIND == kDigits16) {
+        if (c.split > 1u) return launch_run<KIND, 16, true, true>(a, c, sp, s);
+        return c.table ? launch_run<KIND, 16, true, false>(a, c, sp, s) : launch_run<KIND, 8, false, false>(a, c, sp, s);
+    } else {
+        if (c.split > 1u) return launch_run<KIND, 8, false, true>(a, c, sp, s);
+        if constexpr (KIND != kDigits32)
+            if (c.table) return launch_run<KIND, 8, true, false>(a, c, sp, s);
+        return launch_run<KIND, 8, false, false>(a, c, sp, s);
+    }
+}
+
+int launch_main(int kind, const BodyArgs& a, const Cut& c, const Split& sp, hipStream_t s) {
     switch (kind) {
-        case kFew4: return launch_kind<kFew4>(a, s);
-        case kFew8: return launch_kind<kFew8>(a, s);
-        case kDigits16: return launch_kind<kDigits16>(a, s);
-        default: return launch_kind<kDigits32>(a, s);
+        case kFew4: return launch_kind<kFew4>(a, c, sp, s);
+        case kFew8: return launch_kind<kFew8>(a, c, sp, s);
+        case kDigits16: return launch_kind<kDigits16>(a, c, sp, s);
+        default: return launch_kind<kDigits32>(a, c, sp, s);
     }
 }
 
@@ -550,10 +753,13 @@ int static_pack_buffer(uint8_t** out) {
 
 }  // namespace
 
+static size_t pack_bytes(uint32_t bpr, int kind) { return undo_bytes(bpr) + (size_t)bpr * kind_block_bytes(kind); }
+
 size_t gemv_oil4_multi_bytes(const oilhip_weights& w, int M) {
     if (!plain_oil4(w) || !shape_covered(w, 1, (uint32_t)w.cols)) return 0;
     const uint32_t bpr = (uint32_t)(w.cols >> 8);
-    return undo_bytes(bpr) + (size_t)bpr * kind_block_bytes(kind_of(std::min(M, kMaxTokens)));
+    const int m = std::min(M, kMaxTokens), kind = kind_of(m);
+    return pack_bytes(bpr, kind) + split_bytes(best_cut(kind, (uint32_t)w.rows, bpr), (uint32_t)w.rows, m);
 }
 
 // Y[m][r] for m < M: x row tok[m] (or m when tok is null) of an [xrows][ldx] activation matrix; with w2 the same activations
@@ -562,27 +768,48 @@ size_t gemv_oil4_multi_bytes(const oilhip_weights& w, int M) {
 // kernel covers.
 int launch_gemv_oil4_multi(const oilhip_weights& w, const float* d_x, const int* d_tok, float* d_y, int M, uint32_t ldx, uint32_t ldy,
                            uint32_t xrows, hipStream_t s, const MultiInput& in, const oilhip_weights* w2, float* d_y2, uint32_t ldy2,
-                           uint8_t* d_pack) {
+                           uint8_t* d_pack, size_t pack_room) {
     if (!shape_covered(w, xrows, ldx)) return 1;
     if (w2 && (w2->cols != w.cols || !shape_covered(*w2, xrows, ldx) || !plain_oil4(*w2) || !d_y2)) return 1;
     const uint32_t bpr = (uint32_t)(w.cols >> 8);
     const StreamLock lock(s);
     uint8_t* xp = d_pack;
-    if (!xp)
-        // a stream's scratch comes in two sizes: one pass, and from rows of more than 4096 weights on the static scratch's
-        if (int rc = stream_scratch(lock, kScratchGemvPack, bpr > 16u ? kStaticScratchBytes : kGemvPackBytes, reinterpret_cast<void**>(&xp))) return rc;
+    // a stream's scratch comes in two sizes: one pass, and from rows of more than 4096 weights on the static scratch's
+    size_t room = bpr > 16u ? kStaticScratchBytes : kGemvPackBytes;
+    if (!xp) {
+        if (int rc = stream_scratch(lock, kScratchGemvPack, room, reinterpret_cast<void**>(&xp))) return rc;
+    } else {
+        room = pack_room ? pack_room : gemv_oil4_multi_bytes(w, M);
+    }
+    // how a tensor is cut; K only as far as the sums fit behind the activations
+    auto cut = [&](const oilhip_weights& t, int kind, int m, uint8_t* behind, Split& sp) {
+        const uint32_t rows = (uint32_t)t.rows;
+        Cut c = best_cut(kind, rows, bpr);
+        if (c.split > 1u && pack_bytes(bpr, kind) + split_bytes(c, rows, m) > room) c = whole_cut(kind, rows, bpr);
+        if (c.split > 1u) sp = {c.split, c.each, (rows + 15u) & ~15u, reinterpret_cast<float*>(behind + (((size_t)c.wgs * 4u + 255u) & ~(size_t)255u)), reinterpret_cast<uint32_t*>(behind)};
+        return c;
+    };
     const uintptr_t at = reinterpret_cast<uintptr_t>(d_x) | reinterpret_cast<uintptr_t>(in.x2);
     const uint32_t aligned = (at & 15u) == 0 && (ldx & 3u) == 0;
     for (int m0 = 0; m0 < M; m0 += kMaxTokens) {
         const int m = std::min(M - m0, kMaxTokens), kind = kind_of(m);
         const size_t skip = d_tok ? 0 : (size_t)m0 * ldx;
         const Activations act{d_x + skip, in.x2 ? in.x2 + skip : nullptr, in.norm_w, in.xn ? in.xn + skip : nullptr, ldx, aligned, in.inv_form ? 1u : 0u};
-        hipLaunchKernelGGL(pack_digits_kernel, dim3(bpr * kind_tokens(kind) / 4u), dim3(256), 0, s,
-                           PackArgs{act, d_tok ? d_tok + m0 : nullptr, xp, bpr, d_tok ? xrows : xrows - (uint32_t)m0, m, kind}, PackJobs{});
+        uint8_t* behind = xp + pack_bytes(bpr, kind);
+        Split sp{}, sp2{};
+        Cut c = cut(w, kind, m, behind, sp), c2 = w2 ? cut(*w2, kind, m, behind, sp2) : Cut{};
+        if (w2 && c.table != c2.table) {                                   // the activations are packed in one order
+            c = cut_for(kind, 8, false, (uint32_t)w.rows, bpr, 1u);
+            c2 = cut_for(kind, 8, false, (uint32_t)w2->rows, bpr, 1u);
+            sp = sp2 = Split{};
+        }
+        const uint32_t counters = std::max(sp.n > 1u ? c.wgs : 0u, sp2.n > 1u ? c2.wgs : 0u);
+        hipLaunchKernelGGL(c.table ? pack_digits_kernel<true> : pack_digits_kernel<false>, dim3(bpr * kind_tokens(kind) / 4u), dim3(256), 0, s,
+                           PackArgs{act, d_tok ? d_tok + m0 : nullptr, xp, bpr, d_tok ? xrows : xrows - (uint32_t)m0, m, kind, reinterpret_cast<uint32_t*>(behind), counters});
         OILHIP_HIP(hipGetLastError());
-        if (int rc = launch_main(kind, BodyArgs{w.d_payload, xp, d_y + (size_t)m0 * ldy, (uint32_t)w.rows, bpr, ldy, 0u, 0u, 0u, m}, s)) return rc;
+        if (int rc = launch_main(kind, BodyArgs{w.d_payload, xp, d_y + (size_t)m0 * ldy, (uint32_t)w.rows, bpr, ldy, 0u, 0u, 0u, m}, c, sp, s)) return rc;
         if (w2)
-            if (int rc = launch_main(kind, BodyArgs{w2->d_payload, xp, d_y2 + (size_t)m0 * ldy2, (uint32_t)w2->rows, bpr, ldy2, 0u, 0u, 0u, m}, s)) return rc;
+            if (int rc = launch_main(kind, BodyArgs{w2->d_payload, xp, d_y2 + (size_t)m0 * ldy2, (uint32_t)w2->rows, bpr, ldy2, 0u, 0u, 0u, m}, c2, sp2, s)) return rc;
     }
     return OILHIP_OK;
 }
@@ -632,11 +859,11 @@ int launch_gemv_oil4_multi_batches(int nb, const oilhip_weights* const* wa, floa
     PartsOf parts{};
     uint32_t waves = 1;
     for (int k = 0; k < kPassKinds; ++k) {
-        cut_row(k, bpr, parts.n[k], parts.blocks[k]);
-        parts.chunk[k] = parts.n[k] > 1u ? chunk_of(k) : 0x7FFFFFFFu;
-        if (present[k]) waves = std::max(waves, waves_of(parts.blocks[k]));
+        cut_row(k, 8, bpr, parts.n[k], parts.blocks[k]);
+        parts.chunk[k] = parts.n[k] > 1u ? chunk_of(k, false) : 0x7FFFFFFFu;
+        if (present[k]) waves = std::max(waves, waves_of(8, parts.blocks[k]));
     }
-    const double total = (double)device_cu_count() * (double)std::max(1u, (uint32_t)kMaxWaves / waves);
+    const double total = (double)device_cu_count() * (double)std::max(1u, 8u / waves);
     for (int b = 0; b < nb; ++b)
         for (int t = 0; t < per; ++t) {
             const int j = b * per + t;
@@ -649,12 +876,12 @@ int launch_gemv_oil4_multi_batches(int nb, const oilhip_weights* const* wa, floa
             const uint32_t wgs = std::min(std::max((uint32_t)(total * kCost[kind] / cost_sum), 1u), groups);
             if ((groups / wgs + 6ull) * 16u * (w0.cols / 2u) >= 0x80000000ull) return 1;
             mj.g_base[j] = groups / wgs; mj.g_rem[j] = groups % wgs;
-            lds = std::max(lds, lds_of(kind, longest_run(kind), parts.n[kind], (groups + wgs - 1u) / wgs));
+            lds = std::max(lds, lds_of(kind, 8, waves, false, longest_run(kind, 8), parts.n[kind], (groups + wgs - 1u) / wgs));
             mj.wg_begin[j + 1] = mj.wg_begin[j] + wgs;
         }
     const uint32_t aligned = ((reinterpret_cast<uintptr_t>(d_x) | reinterpret_cast<uintptr_t>(d_x2)) & 15u) == 0 && (ldx & 3u) == 0;
-    const PackArgs a{{d_x, d_x2, nullptr, nullptr, ldx, aligned, 0u}, nullptr, static_cast<uint8_t*>(d_ws), bpr, xrows, 0, 0};
-    hipLaunchKernelGGL(pack_digits_kernel, dim3(pj.begin[nb]), dim3(256), 0, s, a, pj);
+    const PackArgs a{{d_x, d_x2, nullptr, nullptr, ldx, aligned, 0u}, nullptr, static_cast<uint8_t*>(d_ws), bpr, xrows, 0, 0, nullptr, 0u};
+    hipLaunchKernelGGL(pack_digits_jobs_kernel, dim3(pj.begin[nb]), dim3(256), 0, s, a, pj);
     OILHIP_HIP(hipGetLastError());
     static std::atomic<uint64_t> raised{0};
     if (int rc = ensure_max_lds(raised, (const void*)gemv_oil4_multi_jobs_kernel, kMaxLds)) return rc;
@@ -683,7 +910,7 @@ extern "C" int oilhip_gemv_oil4_f32_noalloc(const oilhip_weights* w, const float
             return fail(OILHIP_E_ARG, "gemv_oil4_f32_noalloc: this shape needs a kernel that allocates; use oilhip_gemv_f32");
         uint8_t* pack = nullptr;
         if (int e = static_pack_buffer(&pack)) return e;
-        rc = launch_gemv_oil4_multi(*w, d_x, nullptr, d_y, M, (uint32_t)w->cols, (uint32_t)w->rows, (uint32_t)M, s, {}, nullptr, nullptr, 0, pack);
+        rc = launch_gemv_oil4_multi(*w, d_x, nullptr, d_y, M, (uint32_t)w->cols, (uint32_t)w->rows, (uint32_t)M, s, {}, nullptr, nullptr, 0, pack, kStaticScratchBytes);
     }
     if (rc == 1 && M > 2 && M <= 4) rc = launch_gemv_oil4(*w, d_x, d_y, M, s);
     if (rc == 1) return fail(OILHIP_E_ARG, "gemv_oil4_f32_noalloc: this shape needs a kernel that allocates; use oilhip_gemv_f32");

@@ -553,6 +553,42 @@ def test_two_graphs_of_one_capture_stream(fmt, M, how):
     half.close()
 
 
+# K cut between workgroups in 2 to 8 parts, the last part shorter, rows that end inside a group of sixteen, passes of every size with
+# absent tokens, and 33 tokens (two passes over one set of counters).  A sum's order does not depend on who arrives last.
+@pytest.mark.parametrize("rows,cols", [(600, 14336), (37, 11264), (1000, 8192), (1500, 11264)])
+@pytest.mark.parametrize("tokens", [3, 5, 8, 9, 16, 17, 32, 33])
+def test_oil4_several_rows_with_k_cut_between_workgroups(rows, cols, tokens):
+    if tokens in (3, 8, 16, 32) and rows > 600:
+        pytest.skip("the other sizes cover these rows")
+    w = gaussian_weights(rows * cols, rows + tokens, outlier_every=13)
+    payload, blocks = ia.block_codec.quantize_tensor(w, ia.Format.OIL4)
+    X = np.random.default_rng(tokens).standard_normal((tokens, cols)).astype(np.float32)
+    x = torch.from_numpy(X).cuda()
+    with ia.DeviceWeights.from_blocks(payload, blocks, rows, cols) as dw:
+        got = dw.gemv(x)
+        assert all(torch.equal(got, dw.gemv(x)) for _ in range(3))
+        assert torch.equal(got, dw.gemv(x, noalloc=True)) or tokens > 16     # (its scratch is shared by fewer sums)
+    want = O.block_gemm(payload, to_orc_blocks(blocks), rows, cols, X, wide=True)
+    assert rel_l2(got.cpu().numpy(), want) <= 3e-7                # the digits' own error is 1e-7
+
+
+# Tall tensors, whose digits come from a table in LDS, against one row at a time through the FP32 kernel (its error is 1e-7 to 2e-7)
+@pytest.mark.parametrize("rows,cols,tokens", [(66001, 2048, 3), (66001, 2048, 8), (69633, 2048, 13), (20001, 8192, 5), (20001, 8192, 16), (8500, 2816, 11)])
+def test_oil4_several_rows_of_tall_tensors(rows, cols, tokens):
+    bpr, pool = cols // 256, 4096
+    payload, blocks = ia.block_codec.quantize_tensor(gaussian_weights(pool * 256, 7, outlier_every=13), ia.Format.OIL4)
+    pick = np.random.default_rng(rows).integers(0, pool, rows * bpr)
+    desc = np.zeros(rows * bpr, dtype=blocks.dtype)
+    for name in ("nw", "fmt", "cb_bytes", "idx_bytes"):
+        desc[name] = blocks[name][0]
+    desc["cb_off"] = desc["idx_off"] = 128 * np.arange(rows * bpr, dtype=np.uint64)
+    with ia.DeviceWeights.from_blocks(payload.reshape(pool, 128)[pick].reshape(-1), desc, rows, cols) as dw:
+        x = torch.randn(tokens, cols, generator=torch.Generator().manual_seed(cols)).cuda()
+        got = dw.gemv(x).double()
+        one = torch.cat([dw.gemv(x[t:t + 1]) for t in range(tokens)]).double()
+    assert float((got - one).norm() / one.norm()) <= 6e-7
+
+
 def test_workspace_of_the_caller():
     """oilhip_gemv_f32_ws: the size that is asked for, the results of oilhip_gemv_f32, what is refused, and nothing beyond the size
     written."""
