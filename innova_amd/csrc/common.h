@@ -141,11 +141,17 @@ struct MultiInput {
 int launch_gemv_oil4_multi(const oilhip_weights& w, const float* d_x, const int* d_tok, float* d_y, int M, uint32_t ldx, uint32_t ldy,
                            uint32_t xrows, hipStream_t s, const MultiInput& in = {}, const oilhip_weights* w2 = nullptr, float* d_y2 = nullptr,
                            uint32_t ldy2 = 0, uint8_t* d_pack = nullptr, size_t pack_room = 0);
-// several batches of one tensor shape in one launch, at most 32 rows each
+// several batches of one tensor shape in one launch, at most 32 rows each; BatchSums: where parts of K may leave their sums
+constexpr int kMaxBatchParts = 4;
+struct BatchSums {
+    int most, n;                                    // parts that may be used, and that were
+    float* to[kMaxBatchParts - 1];                  // part p > 0: row i of all activation rows at to[p - 1] + i * ld[p - 1]
+    uint32_t ld[kMaxBatchParts - 1];
+};
 size_t gemv_oil4_multi_batches_bytes(int nb, uint64_t cols);
 int launch_gemv_oil4_multi_batches(int nb, const oilhip_weights* const* wa, float* const* ya, const oilhip_weights* const* wb, float* const* yb,
                                    const int* M, const int* row0, const int* list, int nlist, const float* d_x, const float* d_x2,
-                                   uint32_t ldx, uint32_t xrows, uint32_t ldy, void* d_ws, size_t ws_bytes, hipStream_t s);
+                                   uint32_t ldx, uint32_t xrows, uint32_t ldy, void* d_ws, size_t ws_bytes, hipStream_t s, BatchSums* sums = nullptr);
 // other formats, up to 16 rows per pass (FP16 MFMA, gemv_any_multi.hip)
 int launch_gemv_any_multi(const oilhip_weights& w, const float* d_x, float* d_y, int M, hipStream_t s, uint8_t* d_pack = nullptr);
 // bytes of d_pack that these two kernels need (0: they do not serve the tensor)

@@ -79,6 +79,8 @@ constexpr uint32_t kMaxKeep = 24u * 1024u, kMaxKeepNoTable = 48u * 1024u;  // by
 // Several batches in one launch (the experts of a mixture-of-experts step): batch j packs M[j] rows of x into
 // xp + xp_off[j]; its rows are list[row0[j] + m] when use_list is set, else row0[j] + m.  The list travels by value with
 // the launch, so the host needs no copy and no synchronisation.
+// (32 tokens: the table leaves room for runs of two groups only, 3.6 -> 3.7 us per group of 16 blocks)
+__host__ __device__ constexpr bool jobs_table(int kind) { return kind != kDigits32; }
 constexpr int kMaxJobs = 32, kMaxListed = 448;
 struct PackJobs {
     uint32_t n;                 // 0: one batch, described by PackArgs alone
@@ -87,6 +89,7 @@ struct PackJobs {
     uint32_t xp_off[kMaxJobs];
     uint8_t kind[kMaxJobs];
     int use_list;
+    bool table;                 // pack in the order of multi_body's TABLE, where jobs_table allows it
     int16_t list[kMaxListed];
 };
 // where a batch's powers of two start (floats [block][kMaxTokens]) and its packed blocks after them
@@ -187,7 +190,8 @@ pack_digits_jobs_kernel(PackArgs a, const PackJobs jobs) {
     uint32_t j = 0, bid = blockIdx.x;
     while (j + 1u < jobs.n && bid >= jobs.begin[j + 1u]) ++j;              // uniform
     a.M = jobs.M[j]; a.kind = jobs.kind[j]; a.xp += jobs.xp_off[j];
-    pack_body<false>(a, bid - jobs.begin[j], jobs.n, jobs.use_list, jobs.row0[j], jobs.list);
+    if (jobs.table && jobs_table(a.kind)) pack_body<true>(a, bid - jobs.begin[j], jobs.n, jobs.use_list, jobs.row0[j], jobs.list);
+    else pack_body<false>(a, bid - jobs.begin[j], jobs.n, jobs.use_list, jobs.row0[j], jobs.list);
 }
 
 template <bool BY_TABLE>
@@ -229,19 +233,26 @@ __device__ __forceinline__ void pack_body(PackArgs a, uint32_t bid, uint32_t job
 }
 
 // ---- main kernel --------------------------------------------------------------------------------------------------
-// Several tensors of one shape in one launch (the experts of a mixture-of-experts step): each tensor (job) owns a range of
-// the launch's workgroups and brings its packed activations, batch size and output.
+// Several tensors of one shape in one launch (the experts of a mixture-of-experts step).  A tensor brings its packed activations,
+// batch size and output; with K cut, the products of part p > 0 go to rows row0 + m of sums[p - 1].  A job is one tensor's row groups for one part of K; the jobs
+// lie one behind the other (tensor by tensor, part by part) and the launch's workgroups take pieces of that line: of job j workgroup wg[j]
+// takes the first `first` groups, the ones behind it `each` each, and one that has room left goes on with the job after it.
+constexpr uint32_t kMaxLines = 64;
 struct MultiJobs {
-    uint32_t n;
-    uint32_t wg_begin[kMaxJobs + 1];
-    uint32_t g_base[kMaxJobs], g_rem[kMaxJobs];   // row groups per workgroup of the job: g_base, and one more for the first g_rem
+    uint32_t n, split;
+    uint32_t first[kMaxLines], each[kMaxLines];
+    uint16_t wg[kMaxLines];
     const uint8_t* W[kMaxJobs];
     float* y[kMaxJobs];
+    float* sums[kMaxBatchParts - 1];
+    uint32_t ld[kMaxBatchParts];
     uint32_t xp_off[kMaxJobs];
+    uint16_t row0[kMaxJobs];
     uint8_t M[kMaxJobs], kind[kMaxJobs];
 };
 
-struct PartsOf { uint32_t n[kPassKinds], blocks[kPassKinds], chunk[kPassKinds]; };
+// how a pass size walks a job's blocks: steps begin[k][p] to end[k][p] - 1 of blocks[k][p] blocks each
+struct PartsOf { uint16_t begin[kPassKinds][kMaxBatchParts], end[kPassKinds][kMaxBatchParts], blocks[kPassKinds][kMaxBatchParts]; uint32_t chunk[kPassKinds]; };
 
 template <int KIND>
 struct Sums {                                                              // one block's integer sums of one token tile
@@ -296,7 +307,8 @@ struct Split {
 // evenly among them; one that has a block less than the others takes the last one again, scaled by 0.  A workgroup walks the
 // runs of a chunk of its groups for one part of the rows after the other: activations that are fetched once per part cost nothing, fetched
 // once per run they cost as much as the products (37449 x 14336, 16 tokens: 98 us against 73).  The sums wait in LDS.
-template <int KIND, int G, int kMaxWaves, bool TABLE, bool SPLIT>
+// FROM: a workgroup may begin with a later part than the first.  SPLIT: its sums go to `partial`.
+template <int KIND, int G, int kMaxWaves, bool TABLE, bool SPLIT, bool FROM = SPLIT>
 __device__ __forceinline__ void
 multi_body(const BodyArgs& a, uint32_t g_begin, uint32_t g_end, float* lds, float* partial = nullptr, uint32_t ldp = 0) {
     constexpr bool FEW = kind_few(KIND);
@@ -305,7 +317,7 @@ multi_body(const BodyArgs& a, uint32_t g_begin, uint32_t g_end, float* lds, floa
     constexpr int WD = G < 3 ? XD : 1;                                     // weights in flight: the run's, for short runs of all blocks of the part
     const uint32_t lane = threadIdx.x & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), waves = blockDim.x >> 6;
     const uint32_t li = lane & 15u, kq = lane >> 4;
-    const uint32_t row_bytes = a.bpr * 128u, bpr = a.bpr, part0 = SPLIT ? a.part0 : 0u;
+    const uint32_t row_bytes = a.bpr * 128u, bpr = a.bpr, part0 = FROM ? a.part0 : 0u;
     const uint32_t iters = (a.part_blocks + waves - 1u) / waves;           // blocks per wavefront and part, at most XD
     // this workgroup's rows: 32-bit offsets from its first group
     const uint8_t* base = a.W + (size_t)g_begin * 16u * row_bytes;
@@ -570,19 +582,33 @@ gemv_oil4_multi_split_kernel(BodyArgs a, uint32_t g_base, uint32_t g_rem, const 
 }
 
 // Batches of different pass sizes side by side: the job's pass size selects the body.
+// What bounds it: 4 and 8 tokens memory (a CU's pace of 23 KB per us is 6 TB/s), more tokens vector and matrix issue, one after the other.  A launch
+// lasts as long as its longest workgroup, so the line is cut by an estimate that was fitted to the workgroups themselves, and the down projections cut K
+// (with all of K their workgroups had 7 to 13 row groups each and four to seven intakes of activations).  Eight experts 4096 <-> 14336,
+// 64 tokens, top-2, whole workgroups per job and K whole -> now: gate / up ends at 157 to 196 us -> 143 to 150, down 105 to 135 -> 76 to 83.
+template <bool TABLE>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
-gemv_oil4_multi_jobs_kernel(const uint8_t* __restrict__ xp, uint32_t rows, uint32_t bpr, uint32_t ldy, const PartsOf parts, const MultiJobs jobs) {
+gemv_oil4_multi_jobs_kernel(const uint8_t* __restrict__ xp, uint32_t rows, uint32_t bpr, const PartsOf parts, const MultiJobs jobs) {
     extern __shared__ __align__(16) float lds[];
-    uint32_t j = 0;
-    while (j + 1u < jobs.n && blockIdx.x >= jobs.wg_begin[j + 1u]) ++j;    // uniform
-    const uint32_t b = blockIdx.x - jobs.wg_begin[j], gb = jobs.g_base[j], gr = jobs.g_rem[j], kind = jobs.kind[j];
-    const uint32_t g0 = b * gb + (b < gr ? b : gr), g1 = g0 + gb + (b < gr ? 1u : 0u);
-    const BodyArgs a{jobs.W[j], xp + jobs.xp_off[j], jobs.y[j], rows, bpr, ldy, parts.n[kind], parts.blocks[kind], parts.chunk[kind], jobs.M[j]};
-    switch (kind) {
-        case kFew4: multi_body<kFew4, longest_run(kFew4, 8), 8, false, false>(a, g0, g1, lds); break;
-        case kFew8: multi_body<kFew8, longest_run(kFew8, 8), 8, false, false>(a, g0, g1, lds); break;
-        case kDigits16: multi_body<kDigits16, longest_run(kDigits16, 8), 8, false, false>(a, g0, g1, lds); break;
-        default: multi_body<kDigits32, longest_run(kDigits32, 8), 8, false, false>(a, g0, g1, lds); break;
+    const uint32_t lane = threadIdx.x & 63u, lines = jobs.n * jobs.split, groups = (rows + 15u) / 16u;
+    // Workgroups are dealt to the eight XCDs in turn: an XCD takes neighbouring pieces of the line, so that its L2 holds one or two jobs' activations.
+    const uint32_t wg = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    // the last job that begins before this workgroup (it may reach into it), or the first one
+    const uint64_t before = __ballot(lane < lines && (uint32_t)jobs.wg[lane] < wg);
+    for (uint32_t line = before ? 63u - (uint32_t)__builtin_clzll(before) : 0u; line < lines && jobs.wg[line] <= wg; ++line) {
+        const uint32_t at = wg - jobs.wg[line], f = jobs.first[line], e = jobs.each[line];
+        const uint32_t g0 = at ? f + (at - 1u) * e : 0u, to = at ? g0 + e : f, g1 = to < groups ? to : groups;
+        if (g0 >= groups) continue;
+        const uint32_t j = line / jobs.split, part = line - j * jobs.split, kind = jobs.kind[j];
+        float* y = part ? jobs.sums[part - 1u] + (size_t)jobs.row0[j] * jobs.ld[part] : jobs.y[j];
+        const BodyArgs a{jobs.W[j], xp + jobs.xp_off[j], y, rows, bpr, jobs.ld[part], parts.end[kind][part], parts.blocks[kind][part], parts.chunk[kind], jobs.M[j], parts.begin[kind][part]};
+        switch (kind) {
+            case kFew4: multi_body<kFew4, longest_run(kFew4, 8), 8, TABLE, false, true>(a, g0, g1, lds); break;
+            case kFew8: multi_body<kFew8, longest_run(kFew8, 8), 8, TABLE, false, true>(a, g0, g1, lds); break;
+            case kDigits16: multi_body<kDigits16, longest_run(kDigits16, 8), 8, TABLE, false, true>(a, g0, g1, lds); break;
+            default: multi_body<kDigits32, longest_run(kDigits32, 8), 8, false, false, true>(a, g0, g1, lds); break;
+        }
+        __syncthreads();                                                   // the next job's sums go to the same places in LDS
     }
 }
 
@@ -819,33 +845,40 @@ int launch_gemv_oil4_multi(const oilhip_weights& w, const float* d_x, const int*
 // an expert's gate and up projections share their activations).  All tensors have one shape; the batches may differ in pass
 // size.  The activation rows of batch b are rows list[row0[b] + m] of x when `list` is given (the list is passed by value
 // with the launch), else rows row0[b] + m; with x2 they are silu(x) * x2.  Outputs: ya[b][m * ldy + r].
+// With `sums` K may be cut into up to kMaxBatchParts parts: part p > 0 goes to rows row0[b] + m of sums->to[p - 1], sums->n says how many there
+// are, and the caller adds them up.
 size_t gemv_oil4_multi_batches_bytes(int nb, uint64_t cols) {
     const uint32_t bpr = (uint32_t)(cols >> 8);
     return (size_t)nb * (undo_bytes(bpr) + (size_t)bpr * kind_block_bytes(kDigits32));
 }
 
+namespace {
+// Estimated us of a workgroup's piece of a job: a start per step (its activations, the table), then its runs of row groups at the pace of a
+// wavefront's blocks.  Fitted to the workgroups of seven steps of four to eight experts (1024 <-> 3584 to 4096 <-> 14336, 1 to 32 tokens
+// each) without and with the table, 2 us off on average in pieces of 5 to 170 us.
+struct PieceCost { double start, run; };                                   // run: of longest_run groups
+PieceCost piece_cost(int kind, bool table, uint32_t steps, uint32_t blocks, uint32_t waves) {
+    static const double kStart[2][kPassKinds] = {{3.6, 3.2, 3.9, 1.8}, {4.5, 4.3, 4.7, 1.8}}, kRun[2][kPassKinds] = {{0.083, 0.296, 0.533, 0.01}, {0.211, 0.419, 0.747, 0.01}},
+                        kGroupBlock[2][kPassKinds] = {{0.0936, 0.1081, 0.1267, 0.2225}, {0.0865, 0.0941, 0.1131, 0.2225}};
+    return {kStart[table][kind] * steps, steps * (kRun[table][kind] + 8.0 * ((blocks + waves - 1u) / waves) * kGroupBlock[table][kind] * longest_run(kind, 8))};
+}
+}  // namespace
+
 int launch_gemv_oil4_multi_batches(int nb, const oilhip_weights* const* wa, float* const* ya, const oilhip_weights* const* wb, float* const* yb,
                                    const int* M, const int* row0, const int* list, int nlist, const float* d_x, const float* d_x2,
-                                   uint32_t ldx, uint32_t xrows, uint32_t ldy, void* d_ws, size_t ws_bytes, hipStream_t s) {
+                                   uint32_t ldx, uint32_t xrows, uint32_t ldy, void* d_ws, size_t ws_bytes, hipStream_t s, BatchSums* sums) {
     const int per = wb ? 2 : 1, njobs = per * nb;
     if (nb < 1 || njobs > kMaxJobs || nlist > kMaxListed) return 1;
     const oilhip_weights& w0 = *wa[0];
     if (!shape_covered(w0, xrows, ldx) || xrows > 32767u) return 1;
     if (ws_bytes < gemv_oil4_multi_batches_bytes(nb, w0.cols)) return 1;
-    const uint32_t bpr = (uint32_t)(w0.cols >> 8);
+    const uint32_t bpr = (uint32_t)(w0.cols >> 8), groups = ((uint32_t)w0.rows + 15u) / 16u;
     PackJobs pj{};
     pj.n = (uint32_t)nb;
     pj.use_list = list ? 1 : 0;
     for (int i = 0; i < nlist; ++i) pj.list[i] = (int16_t)list[i];
     MultiJobs mj{};
-    mj.n = (uint32_t)njobs;
-    // The launch fills the device once; a job's share of the workgroups follows its cost, so that all run
-    // about equally long: vector instructions per block of 16 rows (decode 136, then 10 to 35 per token tile).
-    static const double kCost[kPassKinds] = {1.0, 1.12, 1.27, 1.84};
-    const uint32_t groups = ((uint32_t)w0.rows + 15u) / 16u;
-    double cost_sum = 0.0;
-    size_t lds = 0;
-    bool present[kPassKinds] = {};
+    int of_kind[kPassKinds] = {};
     uint32_t xp_at = 0;
     for (int b = 0; b < nb; ++b) {
         if (M[b] < 1 || M[b] > kMaxTokens) return fail(OILHIP_E_ARG, "multi-row batches: a batch exceeds the pass size");
@@ -853,40 +886,113 @@ int launch_gemv_oil4_multi_batches(int nb, const oilhip_weights* const* wa, floa
         pj.M[b] = (uint16_t)M[b]; pj.row0[b] = (uint16_t)row0[b]; pj.kind[b] = (uint8_t)kind; pj.xp_off[b] = xp_at;
         pj.begin[b + 1] = pj.begin[b] + bpr * kind_tokens(kind) / 4u;
         xp_at += undo_bytes(bpr) + bpr * kind_block_bytes(kind);
-        cost_sum += kCost[kind] * per;
-        present[kind] = true;
-    }
-    PartsOf parts{};
-    uint32_t waves = 1;
-    for (int k = 0; k < kPassKinds; ++k) {
-        cut_row(k, 8, bpr, parts.n[k], parts.blocks[k]);
-        parts.chunk[k] = parts.n[k] > 1u ? chunk_of(k, false) : 0x7FFFFFFFu;
-        if (present[k]) waves = std::max(waves, waves_of(8, parts.blocks[k]));
-    }
-    const double total = (double)device_cu_count() * (double)std::max(1u, 8u / waves);
-    for (int b = 0; b < nb; ++b)
+        of_kind[kind] += per;
         for (int t = 0; t < per; ++t) {
             const int j = b * per + t;
             const oilhip_weights* w = t ? wb[b] : wa[b];
             if (!plain_oil4(*w) || w->rows != w0.rows || w->cols != w0.cols) return 1;
-            mj.W[j] = w->d_payload; mj.y[j] = t ? yb[b] : ya[b];
-            mj.M[j] = (uint8_t)M[b]; mj.kind[j] = pj.kind[b]; mj.xp_off[j] = pj.xp_off[b];
-            // rounded down: one workgroup past the last full round costs a round
-            const int kind = pj.kind[b];
-            const uint32_t wgs = std::min(std::max((uint32_t)(total * kCost[kind] / cost_sum), 1u), groups);
-            if ((groups / wgs + 6ull) * 16u * (w0.cols / 2u) >= 0x80000000ull) return 1;
-            mj.g_base[j] = groups / wgs; mj.g_rem[j] = groups % wgs;
-            lds = std::max(lds, lds_of(kind, 8, waves, false, longest_run(kind, 8), parts.n[kind], (groups + wgs - 1u) / wgs));
-            mj.wg_begin[j + 1] = mj.wg_begin[j] + wgs;
+            mj.W[j] = w->d_payload; mj.y[j] = t ? yb[b] : ya[b]; mj.row0[j] = (uint16_t)row0[b];
+            mj.M[j] = (uint8_t)M[b]; mj.kind[j] = (uint8_t)kind; mj.xp_off[j] = pj.xp_off[b];
         }
+    }
+    // How K is cut: parts of whole steps of eight blocks (the last one takes what is left), walked in the longest steps that the
+    // wavefronts hold the activations of; without a cut, steps of one size.
+    struct Plan { PartsOf parts; uint32_t split, waves, wgs; bool table; double us; PieceCost cost[kPassKinds][kMaxBatchParts]; };
+    auto plan_for = [&](uint32_t split, bool table, Plan& p) {
+        p = Plan{};
+        p.table = table; p.split = split; p.waves = split > 1u ? 8u : 1u;
+        const uint32_t eights = (bpr + 7u) / 8u, q = (eights + split - 1u) / split;
+        if (split > 1u && (eights + q - 1u) / q != split) return false;
+        for (int k = 0; k < kPassKinds; ++k) {
+            if (!of_kind[k]) continue;
+            bool steps = false;
+            if (split == 1u) {
+                uint32_t n, blocks;
+                cut_row(k, 8, bpr, n, blocks);
+                p.parts.end[k][0] = (uint16_t)n; p.parts.blocks[k][0] = (uint16_t)blocks;
+                p.waves = std::max(p.waves, waves_of(8, blocks));
+                steps = n > 1u;
+            }
+            for (uint32_t i = 0; split > 1u && i < split; ++i) {
+                const uint32_t at = i * q, mine = std::min(q, eights - at);
+                uint32_t step = (uint32_t)x_slots(k, 8);
+                while (mine % step || at % step) --step;
+                p.parts.begin[k][i] = (uint16_t)(at / step); p.parts.end[k][i] = (uint16_t)((at + mine) / step); p.parts.blocks[k][i] = (uint16_t)(8u * step);
+                steps |= mine > step;
+            }
+            p.parts.chunk[k] = steps ? chunk_of(k, table && jobs_table(k)) : 0x7FFFFFFFu;
+        }
+        double work = 0.0, start = 0.0, grain = 0.0;
+        for (int k = 0; k < kPassKinds; ++k)
+            for (uint32_t i = 0; of_kind[k] && i < split; ++i) {
+                const uint32_t run = (uint32_t)longest_run(k, 8);
+                const PieceCost c = p.cost[k][i] = piece_cost(k, table, p.parts.end[k][i] - p.parts.begin[k][i], p.parts.blocks[k][i], p.waves);
+                const double w = (double)of_kind[k] * ((groups + run - 1u) / run) * c.run;
+                work += w; start += w * c.start; grain += w * c.run;
+            }
+        const uint32_t side = std::max(1u, 8u / p.waves);
+        if (table && side > 1u) return false;                              // no room for two tables
+        p.wgs = (uint32_t)device_cu_count() * side;
+        p.us = work / p.wgs + (start + 0.5 * grain) / work + 0.7 * (split - 1u);
+        return true;
+    };
+    Plan plan, other;
+    if (!plan_for(1u, false, plan)) return 1;
+    for (uint32_t n = 1; n <= (sums ? (uint32_t)sums->most : 1u) && (uint32_t)njobs * n <= kMaxLines; ++n)
+        for (bool table : {false, true})
+            if ((n > 1u || table) && plan_for(n, table, other) && other.us < plan.us) plan = other;
+    pj.table = plan.table;
+    // The line of jobs, cut into pieces of at most `most` us each: the least `most`, to 1 %, that the workgroups suffice for.
+    mj.n = (uint32_t)njobs; mj.split = plan.split;
+    uint32_t wgs = 0, fullest = 0;
+    auto cut_line = [&](double most, MultiJobs& o) {
+        uint32_t wg = 0, longest = 0;
+        double used = 0.0;
+        for (uint32_t line = 0; line < mj.n * mj.split; ++line) {
+            const int kind = mj.kind[line / mj.split];
+            const uint32_t run = (uint32_t)longest_run(kind, 8);
+            const PieceCost& c = plan.cost[kind][line % mj.split];
+            auto fits = [&](double room) { return room > c.run + c.start ? (uint32_t)((room - c.start) / c.run) * run : 0u; };
+            const uint32_t e = std::max(fits(most), run);
+            uint32_t f = used > 0.0 ? fits(most - used) : e;
+            if (f == 0u) { ++wg; used = 0.0; f = e; }
+            f = std::min(f, groups);
+            const uint32_t more = (groups - f + e - 1u) / e, last = more ? groups - f - (more - 1u) * e : f;
+            o.wg[line] = (uint16_t)std::min(wg, 65535u); o.first[line] = f; o.each[line] = e;
+            wg += more;
+            used = (more ? 0.0 : used) + c.start + (last + run - 1u) / run * c.run;
+            longest = std::max({longest, f, more ? e : 0u});
+        }
+        if (wg >= plan.wgs) return false;
+        wgs = wg + 1u; fullest = longest;
+        return true;
+    };
+    double most = plan.us;
+    while (!cut_line(most, mj)) most *= 1.01;
+    if (most == plan.us)
+        for (int i = 0; i < 16; ++i) {                                     // (pieces of one run each never stop fitting)
+            MultiJobs less = mj;
+            if (!cut_line(most *= 0.99, less)) break;
+            mj = less;
+        }
+    if ((fullest + 6ull) * 16u * (w0.cols / 2u) >= 0x80000000ull) return 1;
+    size_t lds = 0;
+    for (int k = 0; k < kPassKinds; ++k)
+        if (of_kind[k]) lds = std::max(lds, lds_of(k, 8, plan.waves, plan.table && jobs_table(k), longest_run(k, 8), plan.parts.chunk[k] != 0x7FFFFFFFu ? 2u : 1u, fullest));
+    mj.ld[0] = ldy;
+    if (sums) {
+        sums->n = (int)plan.split;
+        for (uint32_t p = 1; p < plan.split; ++p) { mj.sums[p - 1] = sums->to[p - 1]; mj.ld[p] = sums->ld[p - 1]; }
+    }
     const uint32_t aligned = ((reinterpret_cast<uintptr_t>(d_x) | reinterpret_cast<uintptr_t>(d_x2)) & 15u) == 0 && (ldx & 3u) == 0;
     const PackArgs a{{d_x, d_x2, nullptr, nullptr, ldx, aligned, 0u}, nullptr, static_cast<uint8_t*>(d_ws), bpr, xrows, 0, 0, nullptr, 0u};
     hipLaunchKernelGGL(pack_digits_jobs_kernel, dim3(pj.begin[nb]), dim3(256), 0, s, a, pj);
     OILHIP_HIP(hipGetLastError());
-    static std::atomic<uint64_t> raised{0};
-    if (int rc = ensure_max_lds(raised, (const void*)gemv_oil4_multi_jobs_kernel, kMaxLds)) return rc;
-    hipLaunchKernelGGL(gemv_oil4_multi_jobs_kernel, dim3(mj.wg_begin[njobs]), dim3(64u * waves), lds, s, static_cast<const uint8_t*>(d_ws),
-                       (uint32_t)w0.rows, bpr, ldy, parts, mj);
+    static std::atomic<uint64_t> raised[2]{};
+    auto kern = plan.table ? gemv_oil4_multi_jobs_kernel<true> : gemv_oil4_multi_jobs_kernel<false>;
+    if (int rc = ensure_max_lds(raised[plan.table], (const void*)kern, kMaxLds)) return rc;
+    hipLaunchKernelGGL(kern, dim3((wgs + 7u) & ~7u), dim3(64u * plan.waves), lds, s, static_cast<const uint8_t*>(d_ws),
+                       (uint32_t)w0.rows, bpr, plan.parts, mj);
     OILHIP_HIP(hipGetLastError());
     return OILHIP_OK;
 }

@@ -89,7 +89,7 @@ static_assert(sizeof(CombineLists) <= 3584, "the lists travel in the kernel argu
 
 // zacc == nullptr: the caller does not want the z-loss, and the workgroups skip their atomic on its one address.
 __global__ void __launch_bounds__(256) combine_grouped_kernel(const float* __restrict__ o, uint32_t D, float* __restrict__ out,
-                                                              double* __restrict__ zacc, const CombineLists L) {
+                                                              double* __restrict__ zacc, const BatchSums more, const CombineLists L) {
     __shared__ double part[4];
     const uint32_t d = blockIdx.x * 256 + threadIdx.x, t = blockIdx.y;
     double z = 0.0;
@@ -99,7 +99,13 @@ __global__ void __launch_bounds__(256) combine_grouped_kernel(const float* __res
             const int i = L.pair[t * L.K + k];
             const float w = L.wgt[t * L.K + k];
             if (i < 0 || !(w > 0.0f)) continue;
-            const float v = w * o[(size_t)i * D + d];
+            float p[kMaxBatchParts] = {o[(size_t)i * D + d]};
+#pragma unroll
+            for (int q = 1; q < kMaxBatchParts; ++q) p[q] = q < more.n ? more.to[q - 1][(size_t)i * more.ld[q - 1] + d] : 0.0f;
+            float s = p[0];
+#pragma unroll
+            for (int q = 1; q < kMaxBatchParts; ++q) s = q < more.n ? s + p[q] : s;
+            const float v = w * s;
             sum += v;
             z += (double)v * (double)v;
         }
@@ -260,6 +266,9 @@ int oilhip_moe_forward(const oilhip_weights* const* gate, const oilhip_weights* 
         // all pass sizes of a chunk of batches share one launch per side: one launch that splits the gathered
         // activations, one over the gate and up projections, one that forms silu(gate) * up while splitting it, one
         // over the down projections
+        // Parts of the down projections' sums go where nothing is needed any more: the copies of gathered rows (not made here) and, once
+        // the down projections' activations are packed, the same rows of gate and up.  (Launches could differ in how they cut K: one only.)
+        BatchSums sums{batches.size() > (size_t)kChunk ? 1 : F >= D ? 4 : 2, 1, {ws.xg, ws.g, ws.u}, {(uint32_t)D, (uint32_t)F, (uint32_t)F}};
         for (size_t c0 = 0; c0 < batches.size(); c0 += kChunk) {
             const int nb = (int)std::min<size_t>(kChunk, batches.size() - c0);
             const oilhip_weights *wg[kChunk], *wu[kChunk], *wd[kChunk];
@@ -275,7 +284,7 @@ int oilhip_moe_forward(const oilhip_weights* const* gate, const oilhip_weights* 
                                                     (uint32_t)D, (uint32_t)T, (uint32_t)F, ws.batch, ws.batch_bytes, s);
             if (rc == 0)
                 rc = launch_gemv_oil4_multi_batches(nb, wd, yo, nullptr, nullptr, Mb, r0, nullptr, 0, ws.g, ws.u, (uint32_t)F,
-                                                    (uint32_t)pairs, (uint32_t)D, ws.batch, ws.batch_bytes, s);
+                                                    (uint32_t)pairs, (uint32_t)D, ws.batch, ws.batch_bytes, s, &sums);
             if (rc < 0) return rc;
             if (rc == 1) return fail(OILHIP_E_ARG, "moe_forward: the grouped launch refused a shape it was planned for");
         }
@@ -291,7 +300,7 @@ int oilhip_moe_forward(const oilhip_weights* const* gate, const oilhip_weights* 
                 filled[(size_t)t]++;
             }
         hipLaunchKernelGGL(combine_grouped_kernel, dim3((uint32_t)((D + 255) / 256), (uint32_t)T), dim3(256), 0, s, ws.o, (uint32_t)D, d_out,
-                           z_loss ? ws.z : (double*)nullptr, L);
+                           z_loss ? ws.z : (double*)nullptr, sums, L);
         OILHIP_HIP(hipGetLastError());
         if (z_loss) {
             double z = 0.0;

@@ -72,6 +72,30 @@ def test_dispatch_against_oracle(T, E, K, D, F, fmts):
     assert abs(z - zw) <= 1e-4 * zw
 
 
+@pytest.mark.parametrize("T,E,K,D,F", [(60, 4, 2, 512, 4096),     # workgroups that go from one expert's rows to the next one's
+                                       (44, 5, 2, 768, 4352),     # down rows of 17 blocks: a last part that is shorter and half empty
+                                       (64, 2, 1, 256, 14336),    # 56 blocks, one tile of rows: four parts of K
+                                       (33, 3, 2, 2048, 512),     # d_ff < d: room for two parts only
+                                       (3, 2, 1, 512, 8192),      # few tokens
+                                       (17, 1, 1, 272 * 16, 16640)])   # 65 blocks, one expert
+def test_grouped_pieces_and_parts(T, E, K, D, F):
+    """Sums of the two projections have at most a rounding per block of 256 weights, part and token tile between them; the digits of an
+    activation and the products are exact to 2^-31."""
+    packs, dense = MF.moe_experts(7 + F, E, D, F, (3, 3, 3))
+    ex = upload(packs, D, F)
+    rng = np.random.default_rng(F)
+    x = rng.standard_normal((T, D)).astype(np.float32)
+    logits = rng.standard_normal((T, E)).astype(np.float32)
+    logits[:, 0] += 1.0
+    _, idx, w = moe.softmax_with_topk(logits, K)
+    out, _, _ = moe.moe_dispatch_batched(torch.from_numpy(x).cuda(), ex, idx, w, want_z_loss=False)
+    again, _, _ = moe.moe_dispatch_batched(torch.from_numpy(x).cuda(), ex, idx, w, want_z_loss=False)
+    assert torch.equal(out, again)
+    g, u, d = ([e[j] for e in dense] for j in range(3))
+    want, _, _ = O.moe_dispatch(x, g, u, d, idx, w, wide=True)
+    assert rel(out.cpu().numpy(), want) <= (D / 256 + F / 256 + 16) * 2.0 ** -24
+
+
 def test_step_with_caller_workspace_is_captured_and_replays_bit_for_bit():
     """With the caller's workspace and without the z-loss a step only queues launches: captured into a graph, every
     replay returns the bits of the eager step (passes of 32, 16 and 8 tokens; rows cut along K with ordered sums)."""
