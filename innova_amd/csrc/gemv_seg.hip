@@ -40,12 +40,16 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 struct SegArgs {
     uint32_t nstreams, blind16, tag_bytes;
     uint64_t stream_bytes;
-    uint32_t cb_bytes[kSegMaxFormats], idx_bytes[kSegMaxFormats], stride[kSegMaxFormats];
 };
 
+static_assert(TR == 4, "a closed tile's rows are summed in the four lanes of a quad");
+__device__ __forceinline__ float dpp_row_ror4(float v) {                  // lane i: lane i - 4 of its sixteen
+    return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), 0x124, 0xF, 0xF, true));
+}
 __device__ __forceinline__ uint32_t uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
 
-// One entry of a window: nblk blocks of format FMT, `stride` bytes apart from `data`, their tags from `tags` (both in LDS).
+// One entry of a window: nblk blocks of format FMT (of the size the quantizer writes: no other is packed into windows) from `data`, their tags from `tags`
+// (both in LDS).
 // adds a run's dot products to the accumulators of its row of the tile
 template <int MB>
 __device__ __forceinline__ void add_to_row(float (&acc)[MB][TR], uint32_t rowl, const float (&part)[MB]) {
@@ -58,11 +62,11 @@ __device__ __forceinline__ void add_to_row(float (&acc)[MB][TR], uint32_t rowl, 
 }
 
 template <int FMT, int MB>
-__device__ __forceinline__ void run_entry(const uint8_t* data, const uint8_t* tags, uint32_t tagw, uint32_t nblk, uint32_t stride,
-                                          uint32_t cb_bytes, uint32_t idx_bytes, const DecodeTables* __restrict__ T,
-                                          const LdsTables& L, const float* xs, const float* rs, float (&acc)[MB][TR],
-                                          uint32_t xpad, uint32_t nruns, uint32_t lane) {
+__device__ __forceinline__ void run_entry(const uint8_t* data, const uint8_t* tags, uint32_t tagw, uint32_t nblk,
+                                          const DecodeTables* __restrict__ T, const LdsTables& L, const float* xs, const float* rs,
+                                          float (&acc)[MB][TR], uint32_t xpad, uint32_t nruns, uint32_t lane) {
     constexpr int N = run_raw_dwords(FMT);
+    constexpr uint32_t stride = (full_block_bytes(FMT) + 15u) & ~15u, cb_bytes = full_block_cb_bytes(FMT), idx_bytes = full_block_bytes(FMT) - cb_bytes;
     const uint32_t steps = (nblk + 7u) >> 3, r = lane & 7u, g = lane >> 3;
     // a block's tag: row of the tile and column block, one byte (row << 6 | column) or two (row << 12 | column)
     const uint32_t tshift = tagw == 1u ? 6u : 12u, tmask = tagw == 1u ? 0x3Fu : 0xFFFu;
@@ -292,11 +296,19 @@ gemv_seg_kernel(const uint8_t* __restrict__ streams, const DecodeTables* __restr
         for (int j = 0; j < TR; ++j) acc[m][j] = 0.f;
     for (uint32_t wi = 0;; ++wi) {
         const uint8_t* cur = win + (wi & 1u) * WIN;
-        const uint32_t* hdr = reinterpret_cast<const uint32_t*>(cur);
-        const uint32_t h0 = uniform(hdr[0]);           // 8-byte units of records | another window follows << 12 | its 16-byte pieces << 16
+        // the header and the records, 8 bytes each: a lane holds one of 64 in a row, and an entry costs no LDS round trip of its own
+        const uint2* units = reinterpret_cast<const uint2*>(cur);
+        uint2 held = units[lane];
+        uint32_t held0 = 0;
+        auto unit = [&](uint32_t u) -> uint2 {
+            if (u - held0 >= 64u) { held0 = u; held = units[u + lane < WIN / 8u ? u + lane : u]; }
+            return make_uint2((uint32_t)__builtin_amdgcn_readlane((int)held.x, (int)(u - held0)), (uint32_t)__builtin_amdgcn_readlane((int)held.y, (int)(u - held0)));
+        };
+        const uint2 hdr = unit(0u);
+        const uint32_t h0 = hdr.x;                     // 8-byte units of records | another window follows << 12 | its 16-byte pieces << 16
         bool more = (h0 >> 12) & 1u;
         uint32_t used16 = h0 >> 16;                    // the next window: its size and place are in this one's header, ...
-        const uint8_t* np = streams + (size_t)uniform(hdr[1]) * 16u;
+        const uint8_t* np = streams + (size_t)hdr.y * 16u;
         if (MB > 1 && !more && (sid += gridDim.x * kWaves) < A.nstreams) {         // ... or it is the first one of this wavefront's next stream
             more = true;
             used16 = A.blind16;
@@ -310,36 +322,37 @@ gemv_seg_kernel(const uint8_t* __restrict__ streams, const DecodeTables* __restr
             }
         }
         const uint32_t ne = h0 & 0xFFFu;               // an entry is one unit, the row numbers behind a closing entry two
-        for (uint32_t i = 0; i < ne; ++i) {
-            const uint32_t* rec = reinterpret_cast<const uint32_t*>(cur) + 2u + 2u * i;
-            const uint32_t r0 = uniform(rec[0]), r1 = uniform(rec[1]);
-            const uint32_t sl = r0 & 15u, nblk = r0 >> 16, nrows = (r0 >> 9) & 7u;
+        for (uint32_t i = 1; i <= ne; ++i) {
+            const uint2 rec = unit(i);
+            const uint32_t r0 = rec.x, r1 = rec.y, nblk = r0 >> 16, nrows = (r0 >> 9) & 7u;
             const uint8_t* data = cur + (r1 & 0xFFFFu);
             const uint8_t* tags = cur + (r1 >> 16);
 #define OILHIP_SEG_CASE(F)                                                                                              \
     case F:                                                                                                             \
-        run_entry<F, MB>(data, tags, A.tag_bytes, nblk, A.stride[sl], A.cb_bytes[sl], A.idx_bytes[sl], T, L, xs, rs, acc, xpad,  \
-                         nruns, lane);                                                                                  \
+        run_entry<F, MB>(data, tags, A.tag_bytes, nblk, T, L, xs, rs, acc, xpad, nruns, lane);                                                                                  \
         break;
             switch ((r0 >> 4) & 15u) { OILHIP_SEG_FORMATS(OILHIP_SEG_CASE) default: break; }
 #undef OILHIP_SEG_CASE
-            if ((r0 >> 8) & 1u) {                      // the tile is complete: sum each row across the wavefront
-                i += 2;                                // the two units behind a closing entry: the tile's row numbers
-                const uint32_t trow[TR] = {uniform(rec[2]), uniform(rec[3]), uniform(rec[4]), uniform(rec[5])};
+            if ((r0 >> 8) & 1u) {                      // the tile is complete: sum its rows across the wavefront, row q in every lane with lane % 4 = q
+                // (two units with the row numbers follow a closing entry)
+                const uint32_t trow = reinterpret_cast<const uint32_t*>(cur + 8u * (i + 1u))[lane & 3u];
+                const bool b0 = lane & 1u, b1 = lane & 2u;
+                i += 2;
 #pragma unroll
-                for (int m = 0; m < MB; ++m)
+                for (int m = 0; m < MB; ++m) {
+                    const float r01 = (b0 ? acc[m][1] : acc[m][0]) + oil4::dpp_quad_xor1(b0 ? acc[m][0] : acc[m][1]);
+                    const float r23 = (b0 ? acc[m][3] : acc[m][2]) + oil4::dpp_quad_xor1(b0 ? acc[m][2] : acc[m][3]);
+                    float v = (b1 ? r23 : r01) + oil4::dpp_quad_xor2(b1 ? r01 : r23);
+                    v += dpp_row_ror4(v);                                  // lanes 4 to 7 and 12 to 15: with the quad before
+                    v += oil4::dpp_row_ror8(v);                            // ... and the other two
+                    const auto rows2 = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+                    v = __uint_as_float(rows2[0]) + __uint_as_float(rows2[1]);
+                    const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+                    v = __uint_as_float(halves[0]) + __uint_as_float(halves[1]);
+                    if ((lane & ~3u) == 4u && (lane & 3u) < nrows && m0 + m < M) y[(size_t)(m0 + m) * rows + trow] = v * yscale;
 #pragma unroll
-                    for (int j = 0; j < TR; ++j) {
-                        float v = acc[m][j];
-                        acc[m][j] = 0.f;
-                        v += oil4::dpp_quad_xor1(v);
-                        v += oil4::dpp_quad_xor2(v);
-                        v += oil4::dpp_half_mirror(v);
-                        v += oil4::dpp_row_mirror(v);
-                        v += oil4::dpp_row_bcast15(v);
-                        v += oil4::dpp_row_bcast31(v);
-                        if (lane == 63 && (uint32_t)j < nrows && m0 + m < M) y[(size_t)(m0 + m) * rows + trow[j]] = v * yscale;
-                    }
+                    for (int j = 0; j < TR; ++j) acc[m][j] = 0.f;
+                }
             }
         }
         if (more) {
@@ -369,7 +382,6 @@ int launch_waves(const oilhip_weights& w, const DecodeTables* T, const float* d_
     if (int rc = ensure_max_lds(attr_done, reinterpret_cast<const void*>(kern), 160 * 1024)) return rc;
     SegArgs A{};
     A.nstreams = g.nstreams; A.blind16 = g.blind16; A.tag_bytes = g.tag_bytes; A.stream_bytes = g.stream_bytes;
-    for (uint32_t i = 0; i < g.nf; ++i) { A.cb_bytes[i] = g.cb_bytes[i]; A.idx_bytes[i] = g.idx_bytes[i]; A.stride[i] = g.stride[i]; }
     const uint32_t per = (g.waves + kWaves - 1) / kWaves;              // streams per wavefront
     hipLaunchKernelGGL(kern, dim3((g.nstreams + kWaves * per - 1) / (kWaves * per)), dim3(64 * kWaves), lds, s, w.d_payload, T, d_x, d_xw,
                        d_y, (uint32_t)w.rows, (uint32_t)w.cols, m0, M, A);
