@@ -37,8 +37,40 @@ constexpr int TR = kSegTileRows;           // accumulators per lane and activati
 typedef _Float16 h2v __attribute__((ext_vector_type(2)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
+// Sign table of one activation row: for every four columns all sixteen sums +-x0 +-x1 +-x2 +-x3, entry n the one in which bit j of n makes x[j]
+// positive.  A SPARK_Q0 run is then eight reads instead of 32 products of unpacked signs: 30 vector instructions fewer per step, and
+// about 10 clocks of LDS for each read (16 for 16 bytes per lane of plain activations).  Where another format of the tensor works on few instructions per weight
+// beside it that pays: planner's mix, 12288 x 4096 7.53 -> 7.28 us, 22016 x 4096 12.3 -> 11.5, 30000 x 2048 10.4 -> 9.6.  SPARK_Q0 alone is bound by LDS
+// then (11008 x 4096 10.2 -> 10.4), and with eight wavefronts building the table costs more than it saves (4096 x 4096 5.03 -> 5.22): both stay.  Error
+// against 64 bits (2-norm, planner's mix) 1.0e-7 -> 0.94e-7.
+constexpr uint32_t kSignRunBytes = 8u * 64u + 64u;        // a run's eight tables; the gap spreads runs over the LDS banks
+constexpr uint32_t kSignTab = kLevelTabBytes + 64;        // where the table starts in LDS
+typedef __attribute__((address_space(3))) f32x4_t lds_f4;
+
+// the entries of columns 4 * c4 .. 4 * c4 + 3
+__device__ __forceinline__ void put_signs(uint32_t c4, float4 t) {
+    // neighbouring lanes write their four 16-byte pieces in different orders, so that eight of them hit all banks: piece j ^ sw holds the
+    // sums with the signs of j and those that sw flips
+    const uint32_t g = c4 & 7u, sw = g >> 1, at = kSignTab + (c4 >> 3) * kSignRunBytes + g * 64u + sw * 16u;
+    const float p = t.x + t.y, q = t.x - t.y;
+    const float x2 = __uint_as_float(__float_as_uint(t.z) ^ (sw << 31)), x3 = __uint_as_float(__float_as_uint(t.w) ^ ((sw >> 1) << 31));
+#pragma unroll
+    for (uint32_t j = 0; j < 4u; ++j) {
+        const float b = (j & 1u ? x2 : -x2) + (j & 2u ? x3 : -x3);
+        *(lds_f4*)(uintptr_t)(at ^ (j * 16u)) = f32x4_t{b - p, b + q, b - q, b + p};
+    }
+}
+
+// sum of +-x over the run whose table is at `base`: bit k of u set -> +x[k], else -x[k]
+__device__ __forceinline__ float signed_sum(uint32_t u, uint32_t base) {
+    float v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = *(lds_cf*)(uintptr_t)((((i == 0 ? u << 2 : u >> (4 * i - 2)) & 0x3Cu) | base) + 64u * i);
+    return ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+}
+
 struct SegArgs {
-    uint32_t nstreams, blind16, tag_bytes;
+    uint32_t nstreams, blind16, tag_bytes, keep_x;
     uint64_t stream_bytes;
 };
 
@@ -61,7 +93,7 @@ __device__ __forceinline__ void add_to_row(float (&acc)[MB][TR], uint32_t rowl, 
     }
 }
 
-template <int FMT, int MB>
+template <int FMT, int MB, bool SIGNS>
 __device__ __forceinline__ void run_entry(const uint8_t* data, const uint8_t* tags, uint32_t tagw, uint32_t nblk,
                                           const DecodeTables* __restrict__ T, const LdsTables& L, const float* xs, const float* rs,
                                           float (&acc)[MB][TR], uint32_t xpad, uint32_t nruns, uint32_t lane) {
@@ -110,7 +142,9 @@ __device__ __forceinline__ void run_entry(const uint8_t* data, const uint8_t* ta
         fetch_run<FMT>(cb, cb_bytes, r, raw);
         const uint32_t rowl = tag >> tshift, run = (tag & tmask) * 8u + r;
         float part[MB];
-        if constexpr (FMT == 1) {
+        if constexpr (FMT == 1 && SIGNS) {
+            part[0] = f16_bits(raw[0]) * signed_sum(raw[1], kSignTab + run * kSignRunBytes);
+        } else if constexpr (FMT == 1) {
             // weight k = bit k ? +scale : -scale; as FP16: |scale| with the sign bit from the (inverted) sign word.
             // Pair k holds weights k (low half) and k + 16 (high half).
             const uint32_t s16 = raw[0] & 0xFFFFu;
@@ -194,22 +228,24 @@ __device__ __forceinline__ void run_entry(const uint8_t* data, const uint8_t* ta
 // multiplies with siluf(h[k]) * h[cols + k] (the SwiGLU product of Qwen35Engine::mlp_step,
 // src/adapters/tools/qwen35_engine.cpp:611-621); 2 = x * (1 + xw[k]) is staged and every output is scaled by
 // 1 / sqrt(mean(x^2) + 1e-6), which each workgroup forms from the row it loads anyway (Qwen35Engine::rmsnorm, :39-44).
-template <int MB, int XF, int kWaves>
+template <int MB, int XF, int kWaves, bool SIGNS>
 __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kWaves / 4, kWaves / 4)))
 gemv_seg_kernel(const uint8_t* __restrict__ streams, const DecodeTables* __restrict__ T, const float* __restrict__ x,
                 const float* __restrict__ xw, float* __restrict__ y, uint32_t rows, uint32_t cols, int m0, int M,
                 const SegArgs A) {
-    static_assert(XF == 0 || MB == 1, "the fused input transforms serve one activation row");
+    static_assert((XF == 0 && !SIGNS) || MB == 1, "the fused input transforms and the sign table serve one activation row");
     constexpr uint32_t WIN = window_of(kWaves);
     constexpr int NW = WIN / 1024;                     // 16-byte pieces of a window per lane
     extern __shared__ __align__(16) float smem[];
     const uint32_t nruns = cols >> 5, xpad = nruns * kRunPad;
     float* ssq_part = smem + kLevelTabBytes / 4;       // XF = 2: sum(x^2) per wavefront
-    float* xs = ssq_part + 16;                         // [MB][nruns][36], behind the level tables of dot_run
-    float* rs = xs + (size_t)MB * xpad;                // [MB][nruns] run sums
+    float* xs = ssq_part + 16;                         // [MB][nruns][36], behind the level tables of dot_run (and the sign table)
+    if constexpr (SIGNS) xs += nruns * (kSignRunBytes / 4u);
+    float* rs = xs + (!SIGNS || A.keep_x ? (size_t)MB * xpad : 0);                // [MB][nruns] run sums
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = uniform(tid >> 6);
-    uint8_t* win = reinterpret_cast<uint8_t*>(rs + (size_t)MB * nruns) + (size_t)wave * 2u * WIN;
+    constexpr uint32_t NBUF = SIGNS ? 1u : 2u;         // windows in LDS (the next one waits in registers: it may overwrite the one that is worked off)
+    uint8_t* win = reinterpret_cast<uint8_t*>(rs + (size_t)MB * nruns) + (size_t)wave * NBUF * WIN;
     const LdsTables L{nullptr, nullptr, nullptr, nullptr};      // the formats that expand weight by weight here use no level table
 
     uint32_t sid = blockIdx.x * kWaves + wave;
@@ -257,7 +293,8 @@ gemv_seg_kernel(const uint8_t* __restrict__ streams, const DecodeTables* __restr
                         ssq = __fmaf_rn(t.x, t.x, __fmaf_rn(t.y, t.y, __fmaf_rn(t.z, t.z, __fmaf_rn(t.w, t.w, ssq))));
                         t.x *= 1.0f + b[j].x; t.y *= 1.0f + b[j].y; t.z *= 1.0f + b[j].z; t.w *= 1.0f + b[j].w;
                     }
-                    *reinterpret_cast<float4*>(xs + (size_t)m * xpad + (c4 >> 3) * kRunPad + (c4 & 7u) * 4) = t;
+                    if constexpr (SIGNS) put_signs(c4, t);
+                    if (!SIGNS || A.keep_x) *reinterpret_cast<float4*>(xs + (size_t)m * xpad + (c4 >> 3) * kRunPad + (c4 & 7u) * 4) = t;
                     float s = (t.x + t.y) + (t.z + t.w);
                     s += oil4::dpp_quad_xor1(s);
                     s += oil4::dpp_quad_xor2(s);
@@ -295,7 +332,7 @@ gemv_seg_kernel(const uint8_t* __restrict__ streams, const DecodeTables* __restr
 #pragma unroll
         for (int j = 0; j < TR; ++j) acc[m][j] = 0.f;
     for (uint32_t wi = 0;; ++wi) {
-        const uint8_t* cur = win + (wi & 1u) * WIN;
+        const uint8_t* cur = win + (NBUF == 2u ? (wi & 1u) * WIN : 0u);
         // the header and the records, 8 bytes each: a lane holds one of 64 in a row, and an entry costs no LDS round trip of its own
         const uint2* units = reinterpret_cast<const uint2*>(cur);
         uint2 held = units[lane];
@@ -329,7 +366,7 @@ gemv_seg_kernel(const uint8_t* __restrict__ streams, const DecodeTables* __restr
             const uint8_t* tags = cur + (r1 >> 16);
 #define OILHIP_SEG_CASE(F)                                                                                              \
     case F:                                                                                                             \
-        run_entry<F, MB>(data, tags, A.tag_bytes, nblk, T, L, xs, rs, acc, xpad, nruns, lane);                                                                                  \
+        run_entry<F, MB, SIGNS>(data, tags, A.tag_bytes, nblk, T, L, xs, rs, acc, xpad, nruns, lane);                                                                                  \
         break;
             switch ((r0 >> 4) & 15u) { OILHIP_SEG_FORMATS(OILHIP_SEG_CASE) default: break; }
 #undef OILHIP_SEG_CASE
@@ -356,7 +393,7 @@ gemv_seg_kernel(const uint8_t* __restrict__ streams, const DecodeTables* __restr
             }
         }
         if (more) {
-            uint8_t* nxt = win + ((wi + 1u) & 1u) * WIN;
+            uint8_t* nxt = win + (NBUF == 2u ? ((wi + 1u) & 1u) * WIN : 0u);
 #pragma unroll
             for (int j = 0; j < NW; ++j) *reinterpret_cast<u32x4*>(nxt + ((size_t)j * 64u + lane) * 16u) = wreg[j];
             __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");       // other lanes read what this lane wrote
@@ -371,17 +408,36 @@ size_t seg_lds_bytes(const oilhip_weights& w) {        // the windows take 64 KB
     return kLevelTabBytes + 64 + (size_t)MB * ((w.cols >> 5) * (kRunPad + 1)) * 4 + 16 * (size_t)kSegWindow;
 }
 
-template <int MB, int XF, int kWaves>
+// whether a format of the tensor reads the activations themselves (OIL1 takes their sums, SPARK_Q0 the sign table)
+bool keeps_x(const SegLayout& g) {
+    for (uint32_t i = 0; i < g.nf; ++i)
+        if (g.fmt[i] > 1u) return true;
+    return false;
+}
+
+size_t signs_lds_bytes(const oilhip_weights& w) {
+    const size_t nruns = w.cols >> 5;
+    return kSignTab + nruns * (kSignRunBytes + (keeps_x(w.seg) ? kRunPad * 4 : 0) + 4) + 8 * (size_t)kSegWindow;
+}
+
+// The sign table: SPARK_Q0 beside other formats, sixteen wavefronts, and a row short enough for it (7168 columns of the planner's mix).
+bool takes_signs(const oilhip_weights& w) {
+    bool spark = false;
+    for (uint32_t i = 0; i < w.seg.nf; ++i) spark |= w.seg.fmt[i] == OILHIP_SPARK_Q0;
+    return spark && w.seg.nf > 1 && w.seg.waves == 16 && signs_lds_bytes(w) <= 160 * 1024;
+}
+
+template <int MB, int XF, int kWaves, bool SIGNS>
 int launch_waves(const oilhip_weights& w, const DecodeTables* T, const float* d_x, float* d_y, int m0, int M, hipStream_t s,
                  const float* d_xw) {
     static std::atomic<uint64_t> attr_done{0};
-    auto kern = gemv_seg_kernel<MB, XF, kWaves>;
+    auto kern = gemv_seg_kernel<MB, XF, kWaves, SIGNS>;
     const SegLayout& g = w.seg;
-    const size_t lds = seg_lds_bytes<MB>(w);
+    const size_t lds = SIGNS ? signs_lds_bytes(w) : seg_lds_bytes<MB>(w);
     if (lds > 160 * 1024) return 1;
     if (int rc = ensure_max_lds(attr_done, reinterpret_cast<const void*>(kern), 160 * 1024)) return rc;
     SegArgs A{};
-    A.nstreams = g.nstreams; A.blind16 = g.blind16; A.tag_bytes = g.tag_bytes; A.stream_bytes = g.stream_bytes;
+    A.nstreams = g.nstreams; A.blind16 = g.blind16; A.tag_bytes = g.tag_bytes; A.keep_x = keeps_x(g); A.stream_bytes = g.stream_bytes;
     const uint32_t per = (g.waves + kWaves - 1) / kWaves;              // streams per wavefront
     hipLaunchKernelGGL(kern, dim3((g.nstreams + kWaves * per - 1) / (kWaves * per)), dim3(64 * kWaves), lds, s, w.d_payload, T, d_x, d_xw,
                        d_y, (uint32_t)w.rows, (uint32_t)w.cols, m0, M, A);
@@ -392,9 +448,11 @@ int launch_waves(const oilhip_weights& w, const DecodeTables* T, const float* d_
 template <int MB, int XF = 0>
 int launch_seg(const oilhip_weights& w, const DecodeTables* T, const float* d_x, float* d_y, int m0, int M, hipStream_t s,
                const float* d_xw = nullptr) {
-    if constexpr (MB == 1)
-        if (w.seg.waves == 16) return launch_waves<MB, XF, 16>(w, T, d_x, d_y, m0, M, s, d_xw);
-    return launch_waves<MB, XF, 8>(w, T, d_x, d_y, m0, M, s, d_xw);
+    if constexpr (MB == 1) {
+        if (takes_signs(w)) return launch_waves<MB, XF, 16, true>(w, T, d_x, d_y, m0, M, s, d_xw);
+        if (w.seg.waves == 16) return launch_waves<MB, XF, 16, false>(w, T, d_x, d_y, m0, M, s, d_xw);
+    }
+    return launch_waves<MB, XF, 8, false>(w, T, d_x, d_y, m0, M, s, d_xw);
 }
 
 }  // namespace

@@ -99,6 +99,30 @@ def test_mixed_format_tall(fmt_ids, rows, cols, M):
     assert err <= TOL
 
 
+# SPARK_Q0 beside other formats with sixteen wavefronts: signs looked up in a table of sums (alone with OIL1, and with a format that needs the
+# activations as well), its widest row and the next one, and behind the fused norm; a lane adds at most a block's runs, its share of the row's blocks
+# and six partners
+@pytest.mark.parametrize("rows,cols,fmt_ids", [(8193, 512, (0, 1)), (9000, 1280, (0, 1, 10)), (8193, 7168, (0, 1)), (8193, 7424, (0, 1))])
+def test_mixed_format_sign_table(rows, cols, fmt_ids):
+    rng = np.random.default_rng(rows + cols)
+    fmts = rng.choice(np.array(fmt_ids, dtype=np.uint8), size=rows * cols // 256)
+    bound = (cols / 256 + 32 + 6) * 2.0 ** -24
+    err, payload, blocks, X, want = run_case(fmts, rows, cols, M=1, seed=cols)
+    assert err <= bound
+    norm_w = (rng.standard_normal(cols) * 0.1).astype(np.float32)
+    x64 = X.astype(np.float64)
+    normed = x64 / np.sqrt((x64 ** 2).mean() + 1e-6) * (1.0 + norm_w.astype(np.float64))
+    want = O.block_gemm(payload, to_orc_blocks(blocks), rows, cols, normed.astype(np.float32), wide=True)
+    with ia.DeviceWeights.from_blocks(payload, blocks, rows, cols) as dw:
+        got = layers.gemv_rmsnorm(dw, torch.from_numpy(X).cuda(), torch.from_numpy(norm_w).cuda()).cpu().numpy()
+        X[:, cols // 2] = np.inf                          # reaches every row whose weight there is not zero
+        inf = dw.gemv(torch.from_numpy(X).cuda()).cpu().numpy()
+        plain = dw.gemv(torch.from_numpy(X).cuda(), general=True).cpu().numpy()
+    assert rel_l2(got, want) <= bound
+    if 10 not in fmt_ids:                                 # (OIL4_GRP: scale * sum + zero point * sum, which may be inf - inf, with or without the table)
+        assert np.array_equal(np.isnan(inf), np.isnan(plain)) and np.array_equal(np.isinf(inf), np.isinf(plain))
+
+
 def test_mixed_format_skewed_tiles():
     """Tiles in which a format is absent, or holds a single block, or fills every block."""
     rows, cols = 24, 2048
