@@ -183,52 +183,55 @@ __device__ __forceinline__ void kv_quantize_chunk(const float* __restrict__ src,
 // takes one chunk.  One wavefront per chunk before (every value compared with all 16 centroids in each iteration, sums passed
 // from lane to lane) -> now, 4096 values per token, K and V: 2048 tokens 490 -> 93 us with blocks of 64, 1024 tokens of 2048
 // values with blocks of 32 300 -> 37 us and of 128 268 -> 40 us (clearing included), one token 13 -> 6 us.
+// Sorting floats instead of keys, tokens of whole blocks without index arithmetic, and sums by lane masks (BUSY) -> kernel alone, 2048 tokens of 4096
+// values 85 -> 72 us, 1024 tokens of 2048 values with blocks of 32 29.5 -> 23.6 us and of 128 33.4 -> 32.4 us, one token of 4096 7.0 -> 6.6 us.
 // Windows of four positions per move and sums of eight values per round need fewer steps, and were slower by 12 %.
 constexpr int kSrtPad = 8;                 // floats before a row's values
 
 template <int CTRL>
 __device__ __forceinline__ int row_dpp(int v) { return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, true); }
 
-// the key order of floats (finite: no NaN reaches this)
-__device__ __forceinline__ int kv_key(float f) { const int i = __float_as_int(f); return i ^ ((i >> 31) & 0x7FFFFFFF); }
-__device__ __forceinline__ float kv_unkey(int i) { return __int_as_float(i ^ ((i >> 31) & 0x7FFFFFFF)); }
+template <int CTRL>
+__device__ __forceinline__ float row_dpp(float v) { return __int_as_float(row_dpp<CTRL>(__float_as_int(v))); }
 
-__device__ __forceinline__ int med3(int a, int b, int c) {                 // v_med3_i32: the smaller of a and b for c = INT_MIN, the larger for INT_MAX
-    return max(min(a, b), min(max(a, b), c));
-}
+// Finite values and +inf (a chunk with a NaN or an infinity in it takes the other path, whatever becomes of it here).  A zero may
+// change its sign where zeros of both signs meet: no sum, distance or comparison notices.
+__device__ __forceinline__ float lesser(float a, float b) { float r; asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b)); return r; }
+__device__ __forceinline__ float greater(float a, float b) { float r; asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b)); return r; }
 
 template <int V>
-__device__ __forceinline__ void in_lane_merge(int (&k)[V]) {
+__device__ __forceinline__ void in_lane_merge(float (&k)[V]) {
 #pragma unroll
     for (int j = V / 2; j > 0; j >>= 1)
 #pragma unroll
         for (int e = 0; e < V; ++e)
-            if (!(e & j)) { const int a = k[e], b = k[e | j]; k[e] = min(a, b); k[e | j] = max(a, b); }
+            if (!(e & j)) { const float a = k[e], b = k[e | j]; k[e] = lesser(a, b); k[e | j] = greater(a, b); }
 }
 
-// Ascending bitonic sort of 16 V keys, element c V + e in lane c.  A merge begins with the mirrored partner, so that all
-// comparisons point the same way; `bound[i]` is INT_MIN in lanes whose bit i is clear (they keep the smaller key), else INT_MAX.
+// Ascending bitonic sort of 16 V values, element c V + e in lane c.  A merge begins with the mirrored partner, so that all
+// comparisons point the same way; `bound[i]` is -inf in lanes whose bit i is clear (they keep the smaller value), else +inf.
 template <int V>
-__device__ __forceinline__ void row_sort(int (&k)[V], uint32_t c) {
-    int bound[4];
+__device__ __forceinline__ void row_sort(float (&k)[V], uint32_t c) {
+    auto med3 = [](float a, float b, float m) { return __builtin_amdgcn_fmed3f(a, b, m); };
+    float bound[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) bound[i] = (c >> i) & 1u ? 0x7FFFFFFF : (int)0x80000000;
+    for (int i = 0; i < 4; ++i) bound[i] = (c >> i) & 1u ? __builtin_inff() : -__builtin_inff();
     // inside a lane
 #pragma unroll
     for (int m = 2; m <= V; m <<= 1) {
 #pragma unroll
         for (int e = 0; e < V; ++e) {
             const int o = e ^ (m - 1);
-            if (e < o) { const int a = k[e], b = k[o]; k[e] = min(a, b); k[o] = max(a, b); }
+            if (e < o) { const float a = k[e], b = k[o]; k[e] = lesser(a, b); k[o] = greater(a, b); }
         }
 #pragma unroll
         for (int j = m / 4; j > 0; j >>= 1)
 #pragma unroll
             for (int e = 0; e < V; ++e)
-                if (!(e & j)) { const int a = k[e], b = k[e | j]; k[e] = min(a, b); k[e | j] = max(a, b); }
+                if (!(e & j)) { const float a = k[e], b = k[e | j]; k[e] = lesser(a, b); k[e | j] = greater(a, b); }
     }
     auto flip = [&](auto ctrl, int bit) {
-        int o[V];
+        float o[V];
 #pragma unroll
         for (int e = 0; e < V; ++e) o[e] = row_dpp<decltype(ctrl)::value>(k[V - 1 - e]);
 #pragma unroll
@@ -274,21 +277,23 @@ __device__ __forceinline__ float kv_mean(float sum, float count) {
 // `n` values (x[e] = value c V + e of the row's chunk; anything past n).  Returns false where the chunk has to take the other path;
 // n = 0: nothing to do.  Uniform over a row of lanes; all 64 lanes take part.  srt: room for kSrtPad + 32 V floats, from
 // -kSrtPad on.
-template <int V>
+// BUSY: with wavefronts enough to wait for each other a member costs one vector instruction and a comparison for all lanes, instead of a comparison,
+// a selection and an addition of zero; a wavefront by itself waits longer for that.
+template <int V, bool BUSY>
 __device__ __forceinline__ bool kv_lloyd_rows(const float (&x)[V], uint32_t n, uint32_t lane, float* srt, uint32_t (&code)[V], float& cen_out) {
     const uint32_t c = lane & 15u;
     const int nan = 0x7FC00000;
-    int k[V];
+    float k[V];
     bool finite = true;
 #pragma unroll
     for (int e = 0; e < V; ++e) {
         const bool in = c * V + (uint32_t)e < n;
-        finite &= !in || (__float_as_uint(x[e]) & 0x7FFFFFFFu) < 0x7F800000u;
-        k[e] = in ? kv_key(x[e]) : 0x7F800000;                             // +infinity behind the values
+        finite &= !in || fabsf(x[e]) < __builtin_inff();
+        k[e] = in ? x[e] : __builtin_inff();                               // +infinity behind the values
     }
     row_sort<V>(k, c);
 #pragma unroll
-    for (int e = 0; e < V; ++e) srt[c * V + (uint32_t)e] = kv_unkey(k[e]);
+    for (int e = 0; e < V; ++e) srt[c * V + (uint32_t)e] = k[e];
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
     const float lo = srt[0], hi = srt[n ? n - 1u : 0u];
@@ -333,8 +338,16 @@ __device__ __forceinline__ bool kv_lloyd_rows(const float (&x)[V], uint32_t n, u
             float v[4];
 #pragma unroll
             for (int u = 0; u < 4; ++u) v[u] = at[u];
+            if constexpr (BUSY) {                                          // lanes drop out as their members end
+                const uint64_t first = __ballot(left > 0), second = __ballot(left > 1), third = __ballot(left > 2), fourth = __ballot(left > 3);
+                uint64_t all;
+                asm volatile("s_mov_b64 %1, exec\n\ts_mov_b64 exec, %6\n\tv_add_f32_e32 %0, %0, %2\n\ts_mov_b64 exec, %7\n\tv_add_f32_e32 %0, %0, %3\n\t"
+                             "s_mov_b64 exec, %8\n\tv_add_f32_e32 %0, %0, %4\n\ts_mov_b64 exec, %9\n\tv_add_f32_e32 %0, %0, %5\n\ts_mov_b64 exec, %1"
+                             : "+v"(sum), "=&s"(all) : "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "s"(first), "s"(second), "s"(third), "s"(fourth));
+            } else {
 #pragma unroll
-            for (int u = 0; u < 4; ++u) sum = __fadd_rn(sum, left > u ? v[u] : 0.f);   // sum is never -0: + 0 changes nothing
+                for (int u = 0; u < 4; ++u) sum = __fadd_rn(sum, left > u ? v[u] : 0.f);   // sum is never -0: + 0 changes nothing
+            }
             at += 4;
             left -= 4;
         } while (__ballot(left > 0));
@@ -370,11 +383,13 @@ struct KvRows {
     float srt[4 * (16 * V + kSrtPad) + 16 * V];
     KvLds slow;
 };
-template <int V>
+// WHOLE: all chunks have 16 V values and begin at a multiple of their loads' size.
+template <int V, bool BUSY, bool WHOLE>
 __device__ __forceinline__ void kv_quantize_rows(const float* src, uint32_t n, uint32_t lane, KvRows<V>& L, uint32_t (&code)[V], float& cen) {
     const uint32_t c = lane & 15u;
     float x[V];
-    if (n == 16u * V && (reinterpret_cast<uintptr_t>(src) & (V == 2 ? 7u : 15u)) == 0) {
+    if (WHOLE) n = 16u * V;
+    if (WHOLE || (n == 16u * V && (reinterpret_cast<uintptr_t>(src) & (V == 2 ? 7u : 15u)) == 0)) {
         if constexpr (V == 2) {
             const float2 f = reinterpret_cast<const float2*>(src)[c];
             x[0] = f.x; x[1] = f.y;
@@ -389,7 +404,7 @@ __device__ __forceinline__ void kv_quantize_rows(const float* src, uint32_t n, u
 #pragma unroll
         for (int e = 0; e < V; ++e) x[e] = c * V + (uint32_t)e < n ? src[c * V + (uint32_t)e] : 0.f;
     }
-    const bool ok = kv_lloyd_rows<V>(x, n, lane, L.srt + (lane >> 4) * (16 * V + kSrtPad) + kSrtPad, code, cen);
+    const bool ok = kv_lloyd_rows<V, BUSY>(x, n, lane, L.srt + (lane >> 4) * (16 * V + kSrtPad) + kSrtPad, code, cen);
     uint64_t left = __ballot(!ok);
     while (left) {                                                         // chunk by chunk, by all 64 lanes
         const uint32_t at = (uint32_t)__builtin_ctzll(left);
@@ -410,7 +425,7 @@ __device__ __forceinline__ void kv_quantize_rows(const float* src, uint32_t n, u
 // One row of 16 lanes per (token, chunk of the token, K or V), `per_wave` rows of a wavefront in use.  pos = tokens the layer
 // held before this call, ntok = tokens of this call that fit.  K centroids are stored by the chunk that opens a block, or -- while the layer is empty, and
 // for V always -- by the last chunk of the call that touches the block (:256-261, :277-279: later writes win).
-template <int V>
+template <int V, bool BUSY>
 __global__ void __launch_bounds__(64)
 kv_append_kernel(uint8_t* __restrict__ k_idx, uint8_t* __restrict__ v_idx, uint16_t* __restrict__ k_cb,
                  uint16_t* __restrict__ v_cb, const float* __restrict__ k, const float* __restrict__ v, int64_t pos,
@@ -431,7 +446,7 @@ kv_append_kernel(uint8_t* __restrict__ k_idx, uint8_t* __restrict__ v_idx, uint1
     const float* src = (is_v ? v : k) + (n ? a - pos * per_token : 0);
     uint32_t code[V];
     float cen;
-    kv_quantize_rows<V>(src, n, lane, L, code, cen);
+    kv_quantize_rows<V, BUSY, false>(src, n, lane, L, code, cen);
     if (n == 0) return;
     const bool last_on_block = (b & (block - 1)) == 0 || b == (pos + ntok) * per_token;
     const uint32_t off = (uint32_t)(a & (block - 1));
@@ -456,6 +471,31 @@ kv_append_kernel(uint8_t* __restrict__ k_idx, uint8_t* __restrict__ v_idx, uint1
     if (store_cb) (is_v ? v_cb : k_cb)[blk * 16 + c] = (uint16_t)kv_float_to_half(cen);
 }
 
+// The same where a token is whole blocks and the inputs are aligned: the call's chunks lie one behind the other, in memory and in the cache, and
+// every one writes its block's codes and centroids.  Rows without a chunk repeat the last one.
+template <int V, bool BUSY>
+__global__ void __launch_bounds__(64)
+kv_append_whole_kernel(uint8_t* __restrict__ k_idx, uint8_t* __restrict__ v_idx, uint16_t* __restrict__ k_cb, uint16_t* __restrict__ v_cb,
+                       const float* __restrict__ k, const float* __restrict__ v, int64_t first_block, uint32_t items, uint32_t per_wave) {
+    __shared__ KvRows<V> L;
+    const uint32_t lane = threadIdx.x, row = lane >> 4, c = lane & 15u;
+    const bool is_v = blockIdx.y != 0;
+    const uint32_t item = min(blockIdx.x * per_wave + row, items - 1u);
+    uint32_t code[V];
+    float cen;
+    kv_quantize_rows<V, BUSY, true>((is_v ? v : k) + (size_t)item * (16u * V), 16u * V, lane, L, code, cen);
+    if (row >= per_wave || blockIdx.x * per_wave + row >= items) return;
+    const size_t blk = (size_t)first_block + item;
+    uint8_t* idx = (is_v ? v_idx : k_idx) + blk * (8u * V);
+    uint32_t bytes = code[0];
+#pragma unroll
+    for (int e = 1; e < V; ++e) bytes |= code[e] << (4 * e);
+    if constexpr (V == 2) idx[c] = (uint8_t)bytes;
+    if constexpr (V == 4) reinterpret_cast<uint16_t*>(idx)[c] = (uint16_t)bytes;
+    if constexpr (V == 8) reinterpret_cast<uint32_t*>(idx)[c] = bytes;
+    (is_v ? v_cb : k_cb)[blk * 16 + c] = (uint16_t)kv_float_to_half(cen);
+}
+
 // OIL4KVCache::quantize_block_oil4 over nblocks independent runs of n <= 16 V values: one code per byte, 16 centroids.
 template <int V>
 __global__ void __launch_bounds__(64)
@@ -468,7 +508,7 @@ kv_quantize_blocks_kernel(const float* __restrict__ src, uint32_t n, uint32_t nb
     const size_t at = in ? (size_t)item * n : 0;
     uint32_t code[V];
     float cen;
-    kv_quantize_rows<V>(src + at, in ? n : 0u, lane, L, code, cen);
+    kv_quantize_rows<V, false, false>(src + at, in ? n : 0u, lane, L, code, cen);
     if (!in) return;
 #pragma unroll
     for (int e = 0; e < V; ++e)
@@ -479,6 +519,10 @@ kv_quantize_blocks_kernel(const float* __restrict__ src, uint32_t n, uint32_t nb
 // Chunks per wavefront: four fill its lanes; with fewer chunks than keep two wavefronts on every SIMD, one each, so that a chunk waits
 // for its own iterations only.
 uint32_t kv_per_wave(uint64_t chunks) { return chunks >= 8ull * (uint64_t)device_cu_count() ? 4u : 1u; }
+
+// Eight wavefronts for every SIMD (that many: 16 x 128 values, blocks of 128, 1024 tokens 32.9 -> 32.4 us with masks; two for every SIMD, 400 values,
+// blocks of 64, 500 tokens 9.8 -> 10.3; one token of 4096 6.6 -> 7.0).
+bool kv_busy(uint64_t wavefronts) { return wavefronts >= 32ull * (uint64_t)device_cu_count(); }
 
 // dequantize_block_oil4 (:155-161): dst[b][i] = half_to_float(cb[b][codes[b][i] & 15])
 __global__ void __launch_bounds__(256)
@@ -629,10 +673,19 @@ int oilhip_kv_append(oilhip_kv* c, int layer, const float* d_k, const float* d_v
         const int64_t cpt = (c->per_token + c->block - 1) / c->block + (c->per_token % c->block ? 1 : 0);
         if (ntok * cpt > 0x7FFFFFFF) return fail(OILHIP_E_ARG, "kv_append: too many tokens for one call");
         const uint32_t items = (uint32_t)(ntok * cpt), per_wave = kv_per_wave(2ull * items);
-        auto kern = c->block == 32 ? kv_append_kernel<2> : c->block == 64 ? kv_append_kernel<4> : kv_append_kernel<8>;
-        hipLaunchKernelGGL(kern, dim3((items + per_wave - 1u) / per_wave, 2), dim3(64), 0, (hipStream_t)stream, kv_idx(c, layer, 0),
-                           kv_idx(c, layer, 1), kv_cb(c, layer, 0), kv_cb(c, layer, 1), d_k, d_v, pos, ntok, c->per_token, (uint32_t)cpt,
-                           items, per_wave, c->idx_bytes);
+        const dim3 grid((items + per_wave - 1u) / per_wave, 2);
+        const bool busy = kv_busy(2ull * grid.x);
+        if (c->per_token % c->block == 0 && (((uintptr_t)d_k | (uintptr_t)d_v) & 15) == 0) {
+            auto kern = busy ? (c->block == 32 ? kv_append_whole_kernel<2, true> : c->block == 64 ? kv_append_whole_kernel<4, true> : kv_append_whole_kernel<8, true>)
+                             : (c->block == 32 ? kv_append_whole_kernel<2, false> : c->block == 64 ? kv_append_whole_kernel<4, false> : kv_append_whole_kernel<8, false>);
+            hipLaunchKernelGGL(kern, grid, dim3(64), 0, (hipStream_t)stream, kv_idx(c, layer, 0), kv_idx(c, layer, 1), kv_cb(c, layer, 0),
+                               kv_cb(c, layer, 1), d_k, d_v, pos * cpt, items, per_wave);
+        } else {
+            auto kern = busy ? (c->block == 32 ? kv_append_kernel<2, true> : c->block == 64 ? kv_append_kernel<4, true> : kv_append_kernel<8, true>)
+                             : (c->block == 32 ? kv_append_kernel<2, false> : c->block == 64 ? kv_append_kernel<4, false> : kv_append_kernel<8, false>);
+            hipLaunchKernelGGL(kern, grid, dim3(64), 0, (hipStream_t)stream, kv_idx(c, layer, 0), kv_idx(c, layer, 1), kv_cb(c, layer, 0),
+                               kv_cb(c, layer, 1), d_k, d_v, pos, ntok, c->per_token, (uint32_t)cpt, items, per_wave, c->idx_bytes);
+        }
         OILHIP_HIP(hipGetLastError());
     }
     c->pos[(size_t)layer] = pos + seq_len;                                          // :290, dropped tokens counted as well

@@ -170,6 +170,31 @@ def test_prefill_then_decode_against_oracle(heads, dim, block, prefill, steps):
     assert np.array_equal(c.get_all(0)[0].cpu().numpy().reshape(-1, heads * dim).view(np.uint32), o2.get_range(0, 3)[0].view(np.uint32))
 
 
+# appends long enough for the form that serves many wavefronts: tokens of whole blocks of each size, tokens that end inside blocks, inputs that are
+# not aligned, and a short one; ties, zeros of both signs, constant chunks, values whose sums overflow and tiny ones between ordinary values
+@pytest.mark.parametrize("heads,dim,block,tokens,shift", [(64, 128, 32, 70, 0), (64, 128, 64, 141, 0), (64, 128, 128, 281, 0), (25, 80, 64, 560, 0),
+                                                         (64, 128, 64, 140, 1), (3, 64, 64, 2, 0)])
+def test_long_appends_against_oracle(heads, dim, block, tokens, shift):
+    pt = heads * dim
+    rng = np.random.default_rng(block + tokens + shift)
+    kv = rng.standard_normal((2, tokens, pt)).astype(np.float32)
+    rows = kv.reshape(-1, 16)
+    rows[3::37] = rng.integers(-2, 3, rows[3::37].shape)
+    rows[5::41] = np.where(rng.random(rows[5::41].shape) < 0.5, np.float32(0.0), np.float32(-0.0))
+    rows[7::43] *= np.float32(1e-39)
+    kv[:, ::5, :block] = np.float32(0.25)
+    kv[:, 1::7, -block:] *= np.float32(3e37)
+    c, o = ia.OIL4KVCache(1, tokens + 3, heads, dim, block), O.KVCache(tokens + 3, heads, dim, block)
+    for a, b in ((0, tokens - 1), (tokens - 1, tokens)):
+        part = [torch.zeros(shift + (b - a) * pt, device="cuda")[shift:] for _ in range(2)]
+        for t, src in zip(part, kv):
+            t.copy_(dev(src[a:b]).reshape(-1))
+        c.append(0, *(t.view(1, heads, b - a, dim) for t in part))
+        o.append(kv[0, a:b], kv[1, a:b])
+    for got, want in zip(c.state(0), (o.k_idx, o.v_idx, o.k_cb, o.v_cb)):
+        assert np.array_equal(got, want)
+
+
 def test_full_size_layer():
     """A Llama-7B layer (32 heads x 128) with a 2048-token prefill: sampled chunks against the oracle's quantizer,
     ranges against slices of the whole, decoded values against the stored centroids."""
