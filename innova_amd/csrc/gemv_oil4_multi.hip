@@ -54,22 +54,30 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // four digits side by side (row 4 t + d is digit d of token t), so two instructions (digits a and b of the weights) give all eight
 // products.  Digits: 16 tokens per tile and a tile of rows per digit, seven instructions.  The product of the two lowest
 // digits is left out (2^-31 of the result's scale).  NT tiles of tokens share the decoded weights.
-enum PassKind { kFew4 = 0, kFew8 = 1, kDigits16 = 2, kDigits32 = 3, kPassKinds = 4 };
-__host__ __device__ constexpr bool kind_few(int k) { return k < 2; }
-__host__ __device__ constexpr int kind_tiles(int k) { return (k & 1) + 1; }
-__host__ __device__ constexpr uint32_t kind_tokens(int k) { return k == 0 ? 4u : k == 1 ? 8u : k == 2 ? 16u : 32u; }
-// packed bytes of one block: 1 KB pieces (64 lanes x 16 bytes), four per tile and operand (half of the block x half of its nibbles)
-__host__ __device__ constexpr uint32_t kind_block_bytes(int k) { return (kind_few(k) ? 4096u : 16384u) * (uint32_t)kind_tiles(k); }
-inline int kind_of(int tokens) { return tokens <= 4 ? kFew4 : tokens <= 8 ? kFew8 : tokens <= 16 ? kDigits16 : kDigits32; }
+// 9 to 12 tokens: three tiles of few (24 matrix instructions for a block of 16 rows instead of 28, and 3 sums of a lane instead of 28).  17 to 24: a
+// tile by digits and one or two of few (36 or 44 instead of 56).  With tiles by digits alone -> now, 12 / 20 / 24 tokens: 11008 x 4096 14.3 / 18.9 / 18.7 ->
+// 13.8 / 15.2 / 16.4 us, 2816 x 7424 14.3 / 20.4 / 20.4 -> 13.1 / 15.0 / 15.2, 20000 x 8192 33.0 / 47.0 / 47.0 -> 30.7 / 38.3 / 42.9.
+enum PassKind { kFew4 = 0, kFew8 = 1, kFew12 = 2, kDigits16 = 3, kMixed20 = 4, kMixed24 = 5, kDigits32 = 6, kPassKinds = 7 };
+__host__ __device__ constexpr bool kind_few(int k) { return k < kDigits16; }
+__host__ __device__ constexpr bool tile_few(int k, int t) { return kind_few(k) || ((k == kMixed20 || k == kMixed24) && t > 0); }
+__host__ __device__ constexpr int kind_tiles(int k) { return k == kFew4 || k == kDigits16 ? 1 : k == kFew12 || k == kMixed24 ? 3 : 2; }
+__host__ __device__ constexpr int tile_outputs(int k, int t) { return tile_few(k, t) ? 1 : 4; }             // of a lane
+__host__ __device__ constexpr int outputs_before(int k, int t) { return t == 0 ? 0 : outputs_before(k, t - 1) + tile_outputs(k, t - 1); }
+__host__ __device__ constexpr int lane_outputs(int k) { return outputs_before(k, kind_tiles(k)); }
+__host__ __device__ constexpr uint32_t tokens_before(int k, int t) { return t == 0 ? 0u : tokens_before(k, t - 1) + (tile_few(k, t - 1) ? 4u : 16u); }
+__host__ __device__ constexpr uint32_t kind_tokens(int k) { return tokens_before(k, kind_tiles(k)); }
+// packed bytes of one block: 1 KB pieces (64 lanes x 16 bytes), four per operand (half of the block x half of its nibbles) for a
+// tile of few, sixteen for one by digits: 1 KB per token
+__host__ __device__ constexpr uint32_t kind_block_bytes(int k) { return kind_tokens(k) * 1024u; }
+inline int kind_of(int tokens) { return tokens <= 4 ? kFew4 : tokens <= 8 ? kFew8 : tokens <= 12 ? kFew12 : tokens <= 16 ? kDigits16 : tokens <= 20 ? kMixed20 : tokens <= 24 ? kMixed24 : kDigits32; }
 
 // blocks of activations that a wavefront holds: as many as the registers take
 // (8 wavefronts per CU, 256 registers each, or 16 with 128)
-constexpr int x_slots(int kind, int waves) { return kind == kFew4 ? 4 : kind == kFew8 ? 3 : kind == kDigits16 && waves == 8 ? 2 : 1; }
+constexpr int x_slots(int kind, int waves) { return kind == kFew4 ? 4 : kind == kFew8 ? 3 : (kind == kFew12 || kind == kDigits16) && waves == 8 ? 2 : 1; }
 constexpr int kMaxTokens = 32;
 constexpr uint32_t kMaxSplit = 8;
 // row groups of a run
-constexpr int longest_run(int kind, int waves) { return kind == kDigits32 ? 3 : waves == 16 ? 2 : 4; }
-constexpr int lane_outputs(int kind) { return kind_tiles(kind) * (kind_few(kind) ? 1 : 4); }
+constexpr int longest_run(int kind, int waves) { return kind >= kMixed24 ? 3 : waves == 16 ? 2 : 4; }
 constexpr uint32_t kMaxKeep = 24u * 1024u, kMaxKeepNoTable = 48u * 1024u;  // bytes of LDS for sums that are carried from part to part
 
 // ---- pre-pass: activations to digits in operand order -----------------------------------------------------------------
@@ -79,8 +87,10 @@ constexpr uint32_t kMaxKeep = 24u * 1024u, kMaxKeepNoTable = 48u * 1024u;  // by
 // Several batches in one launch (the experts of a mixture-of-experts step): batch j packs M[j] rows of x into
 // xp + xp_off[j]; its rows are list[row0[j] + m] when use_list is set, else row0[j] + m.  The list travels by value with
 // the launch, so the host needs no copy and no synchronisation.
-// (32 tokens: the table leaves room for runs of two groups only, 3.6 -> 3.7 us per group of 16 blocks)
-__host__ __device__ constexpr bool jobs_table(int kind) { return kind != kDigits32; }
+// (more than 16 tokens: the table leaves room for runs of two groups only, 3.6 -> 3.7 us per group of 16 blocks)
+__host__ __device__ constexpr bool jobs_table(int kind) { return kind <= kDigits16; }
+// row groups of a run beside the other bodies, without spilling registers
+constexpr int jobs_run(int kind) { return kind == kDigits32 ? 2 : kind == kMixed24 ? 3 : 4; }
 constexpr int kMaxJobs = 32, kMaxListed = 448;
 struct PackJobs {
     uint32_t n;                 // 0: one batch, described by PackArgs alone
@@ -177,29 +187,33 @@ __device__ __forceinline__ float block_to_digits(float (&v)[4], uint32_t lane, P
 
 // BY_TABLE: in the order of multi_body's TABLE.  (One batch, without the jobs: 1.4 KB of arguments cost the host 1.2 us of a launch.)
 template <bool BY_TABLE>
-__device__ __forceinline__ void pack_body(PackArgs a, uint32_t bid, uint32_t jobs, bool use_list, uint32_t row0, const int16_t* list);
+__device__ __forceinline__ void pack_body(const PackArgs& a, uint32_t blk, uint32_t four, uint32_t jobs, bool use_list, uint32_t row0, const int16_t* list);
 
 template <bool BY_TABLE>
 __global__ void __launch_bounds__(256)
 pack_digits_kernel(const PackArgs a) {
-    if (blockIdx.x == 0) for (uint32_t i = threadIdx.x; i < a.ncount; i += 256u) a.arrived[i] = 0u;
-    pack_body<BY_TABLE>(a, blockIdx.x, 0u, false, 0u, nullptr);
+    // all arguments at once: read where they are needed, each adds a scalar load's latency (3.04 -> 2.85 us for a few blocks)
+    asm volatile("" :: "s"(a.in.x), "s"(a.in.x2), "s"(a.in.norm_w), "s"(a.in.ldx), "s"(a.in.aligned), "s"(a.tok), "s"(a.xp), "s"(a.xrows), "s"(a.M), "s"(a.kind));
+    pack_body<BY_TABLE>(a, blockIdx.x, blockIdx.y, 0u, false, 0u, nullptr);
+    if (a.ncount && blockIdx.x + blockIdx.y == 0) for (uint32_t i = threadIdx.x; i < a.ncount; i += 256u) a.arrived[i] = 0u;
 }
 __global__ void __launch_bounds__(256)
 pack_digits_jobs_kernel(PackArgs a, const PackJobs jobs) {
     uint32_t j = 0, bid = blockIdx.x;
     while (j + 1u < jobs.n && bid >= jobs.begin[j + 1u]) ++j;              // uniform
     a.M = jobs.M[j]; a.kind = jobs.kind[j]; a.xp += jobs.xp_off[j];
-    if (jobs.table && jobs_table(a.kind)) pack_body<true>(a, bid - jobs.begin[j], jobs.n, jobs.use_list, jobs.row0[j], jobs.list);
-    else pack_body<false>(a, bid - jobs.begin[j], jobs.n, jobs.use_list, jobs.row0[j], jobs.list);
+    bid -= jobs.begin[j];
+    const uint32_t four = bid / a.bpr, blk = bid - four * a.bpr;
+    if (jobs.table && jobs_table(a.kind)) pack_body<true>(a, blk, four, jobs.n, jobs.use_list, jobs.row0[j], jobs.list);
+    else pack_body<false>(a, blk, four, jobs.n, jobs.use_list, jobs.row0[j], jobs.list);
 }
 
 template <bool BY_TABLE>
-__device__ __forceinline__ void pack_body(PackArgs a, uint32_t bid, uint32_t jobs, bool use_list, uint32_t row0, const int16_t* list) {
+__device__ __forceinline__ void pack_body(const PackArgs& a, uint32_t blk, uint32_t four, uint32_t jobs, bool use_list, uint32_t row0, const int16_t* list) {
     __shared__ __align__(16) uint8_t lds[4][1024];
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    // workgroup = four tokens of one block
-    const uint32_t blk = bid % a.bpr, t = (bid / a.bpr) * 4u + wave;
+    const uint32_t lane = threadIdx.x & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    // workgroup = four tokens (number `four`) of one block
+    const uint32_t t = four * 4u + wave;
     uint32_t src = 0xFFFFFFFFu;
     if ((int)t < a.M) src = jobs ? (use_list ? (uint32_t)list[row0 + t] : row0 + t) : a.tok ? (uint32_t)a.tok[t] : t;
     float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -219,7 +233,9 @@ __device__ __forceinline__ void pack_body(PackArgs a, uint32_t bid, uint32_t job
         const uint32_t at = place(p);
         mine[at] = (uint8_t)bytes; mine[256u + at] = (uint8_t)(bytes >> 8); mine[512u + at] = (uint8_t)(bytes >> 16); mine[768u + at] = (uint8_t)(bytes >> 24);
     });
-    const uint32_t tokens = kind_few(a.kind) ? 4u : 16u, tile = t / tokens, tt = t - tile * tokens;
+    // the token's tile: by digits (the first sixteen, or all), or of few
+    const bool few = kind_few(a.kind) || (t >= 16u && a.kind != kDigits32);
+    const uint32_t tokens = few ? 4u : 16u, tt = t & (tokens - 1u);
     if (lane == 0) reinterpret_cast<float*>(a.xp)[blk * (uint32_t)kMaxTokens + t] = undo;
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -228,8 +244,9 @@ __device__ __forceinline__ void pack_body(PackArgs a, uint32_t bid, uint32_t job
     const uint32_t d = lane >> 4, op = (lane >> 2) & 3u, kq = lane & 3u;
     const uint4 piece = *reinterpret_cast<const uint4*>(mine + 16u * lane);
     uint8_t* o = a.xp + undo_bytes(a.bpr) + (size_t)blk * kind_block_bytes(a.kind);
-    if (kind_few(a.kind)) *reinterpret_cast<uint4*>(o + tile * 4096u + op * 1024u + (kq * 16u + tt * 4u + d) * 16u) = piece;
-    else *reinterpret_cast<uint4*>(o + tile * 16384u + (d * 4u + op) * 1024u + (kq * 16u + tt) * 16u) = piece;
+    o += (t - tt) * 1024u;                                                 // the tiles before: 1 KB per token
+    if (few) *reinterpret_cast<uint4*>(o + op * 1024u + (kq * 16u + tt * 4u + d) * 16u) = piece;
+    else *reinterpret_cast<uint4*>(o + (d * 4u + op) * 1024u + (kq * 16u + tt) * 16u) = piece;
 }
 
 // ---- main kernel --------------------------------------------------------------------------------------------------
@@ -311,8 +328,7 @@ struct Split {
 template <int KIND, int G, int kMaxWaves, bool TABLE, bool SPLIT, bool FROM = SPLIT>
 __device__ __forceinline__ void
 multi_body(const BodyArgs& a, uint32_t g_begin, uint32_t g_end, float* lds, float* partial = nullptr, uint32_t ldp = 0) {
-    constexpr bool FEW = kind_few(KIND);
-    constexpr int NT = kind_tiles(KIND), PER = FEW ? 1 : 4, DIG = FEW ? 1 : 4;   // outputs of a lane per tile, operand pieces per half and parity
+    constexpr int NT = kind_tiles(KIND), PER = kind_few(KIND) ? 1 : 4, DIG = PER;   // at most: outputs of a lane per tile, operand pieces per half and parity
     constexpr int XD = x_slots(KIND, kMaxWaves);
     constexpr int WD = G < 3 ? XD : 1;                                     // weights in flight: the run's, for short runs of all blocks of the part
     const uint32_t lane = threadIdx.x & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), waves = blockDim.x >> 6;
@@ -325,11 +341,11 @@ multi_body(const BodyArgs& a, uint32_t g_begin, uint32_t g_end, float* lds, floa
     const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(base), (short)0, (int)0xFFFFFFFFu, 0x00020000);
     const float* undo = reinterpret_cast<const float*>(a.xp);
     const uint8_t* xblocks = a.xp + undo_bytes(bpr);
-    // five to eight tokens: rows of absent ones in the second tile repeat a present one, and nothing more is fetched (5 tokens, 4096 x 4096
+    // five to twelve tokens: rows of absent ones in the last tile repeat a present one, and nothing more is fetched (5 tokens, 4096 x 4096
     // 8.95 -> 8.40 us; for the other sizes level)
     uint32_t xlane[NT];
 #pragma unroll
-    for (int t = 0; t < NT; ++t) xlane[t] = KIND == kFew8 && t == 1 ? kq * 16u + min(li >> 2, (uint32_t)a.M - 5u) * 4u + (li & 3u) : lane;
+    for (int t = 0; t < NT; ++t) xlane[t] = kind_few(KIND) && t > 0 && t == NT - 1 ? kq * 16u + min(li >> 2, (uint32_t)a.M - 4u * t - 1u) * 4u + (li & 3u) : lane;
     const uint32_t scale_lane = li * 4u;                                   // ds_bpermute address of lane li: it holds the block's scale
     auto place = [&](uint32_t part, uint32_t i) { const uint32_t b = wave + i * waves; return b < a.part_blocks ? part * a.part_blocks + b : 0xFFFFFFFFu; };
     auto block_at = [&](uint32_t part, uint32_t i) { const uint32_t b = place(part, i); return b < bpr ? b : bpr - 1u; };
@@ -351,17 +367,19 @@ multi_body(const BodyArgs& a, uint32_t g_begin, uint32_t g_end, float* lds, floa
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
-            for (int d = 0; d < DIG; ++d) x[slot][t][d][o] = p[((t * DIG + d) * 4 + o) * 64 + (int)xlane[t]];
+            for (int d = 0; d < tile_outputs(KIND, t); ++d) x[slot][t][d][o] = p[(int)tokens_before(KIND, t) * 64 + (d * 4 + o) * 64 + (int)xlane[t]];
     };
     auto load_undo = [&](int slot, uint32_t blk) {
         const float* u = undo + blk * (uint32_t)kMaxTokens;
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
-            if constexpr (FEW) {
-                un[slot][t][0] = u[4 * t + kq];
+            if (tile_few(KIND, t)) {
+                un[slot][t][0] = u[tokens_before(KIND, t) + kq];
             } else {
-                const float4 f = *reinterpret_cast<const float4*>(u + 16 * t + 4 * kq);
-                un[slot][t][0] = f.x; un[slot][t][1] = f.y; un[slot][t][2] = f.z; un[slot][t][3] = f.w;
+                const float4 f = *reinterpret_cast<const float4*>(u + tokens_before(KIND, t) + 4 * kq);
+                const float all[4] = {f.x, f.y, f.z, f.w};
+#pragma unroll
+                for (int v = 0; v < PER; ++v) un[slot][t][v] = all[v];
             }
         }
     };
@@ -393,7 +411,7 @@ multi_body(const BodyArgs& a, uint32_t g_begin, uint32_t g_end, float* lds, floa
     }
     const uint32_t lane4 = 4u * lane;
     float* red = lds + (TABLE ? kDigitTab / 4u : 0u);
-    constexpr uint32_t OUT = (uint32_t)(G * NT * PER) * 64u;
+    constexpr uint32_t LANE = (uint32_t)lane_outputs(KIND), OUT = (uint32_t)G * LANE * 64u;
     const uint32_t held = kMaxWaves == 8 ? 8u : (waves + 3u) & ~3u, AREA = held * OUT;   // wavefronts that sums are held for
     float* keep = red + 2u * AREA;                                         // sums of the parts before, by run
     if (waves < held) {                                                  // the sums of absent wavefronts read as zero
@@ -444,10 +462,10 @@ multi_body(const BodyArgs& a, uint32_t g_begin, uint32_t g_end, float* lds, floa
                 }
 #pragma unroll
                 for (int t = 0; t < NT; ++t) {
-                    if constexpr (FEW) {
+                    if (tile_few(KIND, t)) {
                         sum[t].s[0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[XS][t][0][o], da, sum[t].s[0], 0, 0, 0);
                         sum[t].s[1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[XS][t][0][o], db, sum[t].s[1], 0, 0, 0);
-                    } else {                                               // digits of the activations: [0] low to [3] high
+                    } else if constexpr (!kind_few(KIND)) {                // digits of the activations: [0] low to [3] high
                         // (an order in which no instruction waits for the one before the last)
                         sum[t].s[1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[XS][t][3][o], db, sum[t].s[1], 0, 0, 0);     // 2^24
                         sum[t].s[2] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[XS][t][2][o], db, sum[t].s[2], 0, 0, 0);     // 2^16
@@ -462,12 +480,12 @@ multi_body(const BodyArgs& a, uint32_t g_begin, uint32_t g_end, float* lds, floa
             load_w(WS, g, npart, nrun, ni);
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
-                if constexpr (FEW) {                                       // element d is digit d of this lane's token
+                if (tile_few(KIND, t)) {                                   // element d is digit d of this lane's token
                     // below 252 (128 * 27178 + 128 * 106) < 2^30; the product of the two lowest digits is left out here as well
                     const float f = fmaf((float)(sum[t].s[0][3] * 256 + sum[t].s[1][3]), 65536.0f,
                                          fmaf((float)(sum[t].s[0][2] * 256 + sum[t].s[1][2]), 256.0f, (float)(sum[t].s[0][1] * 256 + (sum[t].s[1][1] + sum[t].s[0][0]))));
                     acc[g][t][0] = fmaf(f * scale, un[XS][t][0], acc[g][t][0]);
-                } else {
+                } else if constexpr (!kind_few(KIND)) {
 #pragma unroll
                     for (int v = 0; v < PER; ++v) {
                         // below 252 (128 * 128 + 128 * 106) (256 + 1) < 2^31
@@ -493,8 +511,9 @@ multi_body(const BodyArgs& a, uint32_t g_begin, uint32_t g_end, float* lds, floa
             float* k = keep + ((run % a.chunk) / G) * OUT + o;             // this thread's own from part to part
             if (part > part0) s += *k;
             if (part + 1u < a.parts) { *k = s; continue; }
-            const uint32_t l = o & 63u, e = o >> 6, v = e % PER, t = (e / PER) % NT, g = e / (PER * NT);
-            const uint32_t token = FEW ? 4u * t + (l >> 4) : 16u * t + 4u * (l >> 4) + v;
+            const uint32_t l = o & 63u, e = o >> 6, g = e / LANE, q = e % LANE;   // output q of the lane for group g
+            const bool few = kind_few(KIND) || (KIND != kDigits32 && q >= 4u);
+            const uint32_t token = few ? 4u * q + (l >> 4) : 16u * (q >> 2) + 4u * (l >> 4) + (q & 3u);
             const uint32_t r = (g_begin + run + g) * 16u + (l & 15u);
             if (run + g < ngroups && r < a.rows && (int)token < a.M) {
                 // (stores that are coherent across the device by themselves: a release fence would write a whole L2 back)
@@ -515,7 +534,7 @@ multi_body(const BodyArgs& a, uint32_t g_begin, uint32_t g_end, float* lds, floa
 #pragma unroll
                 for (int t = 0; t < NT; ++t)
 #pragma unroll
-                    for (int v = 0; v < PER; ++v) acc[g][t][v] = 0.0f;
+                    for (int v = 0; v < tile_outputs(KIND, t); ++v) acc[g][t][v] = 0.0f;
             step(std::integral_constant<int, 0>{}, part, run);
             if constexpr (XD > 1) if (iters > 1u) step(std::integral_constant<int, 1>{}, part, run);
             if constexpr (XD > 2) if (iters > 2u) step(std::integral_constant<int, 2>{}, part, run);
@@ -526,7 +545,7 @@ multi_body(const BodyArgs& a, uint32_t g_begin, uint32_t g_end, float* lds, floa
 #pragma unroll
                 for (int t = 0; t < NT; ++t)
 #pragma unroll
-                    for (int v = 0; v < PER; ++v) area[(uint32_t)((g * NT + t) * PER + v) * 64u + lane] = acc[g][t][v];
+                    for (int v = 0; v < tile_outputs(KIND, t); ++v) area[((uint32_t)g * LANE + (uint32_t)(outputs_before(KIND, t) + v)) * 64u + lane] = acc[g][t][v];
             lds_barrier();
             odd ^= 1u;
             done_part = part; done_run = run;
@@ -603,10 +622,13 @@ gemv_oil4_multi_jobs_kernel(const uint8_t* __restrict__ xp, uint32_t rows, uint3
         float* y = part ? jobs.sums[part - 1u] + (size_t)jobs.row0[j] * jobs.ld[part] : jobs.y[j];
         const BodyArgs a{jobs.W[j], xp + jobs.xp_off[j], y, rows, bpr, jobs.ld[part], parts.end[kind][part], parts.blocks[kind][part], parts.chunk[kind], jobs.M[j], parts.begin[kind][part]};
         switch (kind) {
-            case kFew4: multi_body<kFew4, longest_run(kFew4, 8), 8, TABLE, false, true>(a, g0, g1, lds); break;
-            case kFew8: multi_body<kFew8, longest_run(kFew8, 8), 8, TABLE, false, true>(a, g0, g1, lds); break;
-            case kDigits16: multi_body<kDigits16, longest_run(kDigits16, 8), 8, TABLE, false, true>(a, g0, g1, lds); break;
-            default: multi_body<kDigits32, longest_run(kDigits32, 8), 8, false, false, true>(a, g0, g1, lds); break;
+            case kFew4: multi_body<kFew4, jobs_run(kFew4), 8, TABLE, false, true>(a, g0, g1, lds); break;
+            case kFew8: multi_body<kFew8, jobs_run(kFew8), 8, TABLE, false, true>(a, g0, g1, lds); break;
+            case kFew12: multi_body<kFew12, jobs_run(kFew12), 8, TABLE, false, true>(a, g0, g1, lds); break;
+            case kDigits16: multi_body<kDigits16, jobs_run(kDigits16), 8, TABLE, false, true>(a, g0, g1, lds); break;
+            case kMixed20: multi_body<kMixed20, jobs_run(kMixed20), 8, false, false, true>(a, g0, g1, lds); break;
+            case kMixed24: multi_body<kMixed24, jobs_run(kMixed24), 8, false, false, true>(a, g0, g1, lds); break;
+            default: multi_body<kDigits32, jobs_run(kDigits32), 8, false, false, true>(a, g0, g1, lds); break;
         }
         __syncthreads();                                                   // the next job's sums go to the same places in LDS
     }
@@ -664,14 +686,17 @@ Cut whole_cut(int kind, uint32_t rows, uint32_t bpr) {
     return c;
 }
 // Where a workgroup has few row groups, what it takes in is mostly activations: K is cut between workgroups then.  The line is an estimate in
-// us that counts a workgroup's bytes of activations, its work and what the meeting of the sums costs; it was fitted to 1 to 8 parts on
-// 25 shapes (300 to 131072 rows, 1024 to 14336 columns), and on them its choice is 1.5 % slower than the best on average, 15 % at most, and never slower than no
-// cut by more than 3 %.  5 tokens, 1 / best: 600 x 14336 16.7 / 10.2 us, 5120 x 13824 25.3 / 18.3; 16 tokens 4096 x 11008 20.7 / 17.2;
-// 32 tokens 32.5 / 24.4; 4096 x 4096 stays whole up to 16 tokens (10.7 / 11.9 for 16).
+// us that counts a workgroup's bytes of activations, its work and what the meeting of the sums costs (with more than 16 tokens also their way through memory,
+// 0.35 us per 1000 rows and four parts); it was fitted to 1 to 8 parts on 25 shapes (300 to 131072 rows, 1024 to 14336 columns), `least` to 16 more
+// (600 to 20000 rows, 2048 to 14336 columns, 4 to 32 tokens): there its choice is 0.4 % slower than the better of cut and whole on average, 7 % at most, and never
+// slower than no cut by more than 3 %.  5 tokens, 1 / best: 600 x 14336 15.7 / 10.5 us, 5120 x 13824 23.1 / 18.5; 16 tokens 4096 x 11008 19.4 / 16.5;
+// 32 tokens 30.0 / 23.9; 24 tokens 25.2 / 21.2, 14336 x 5120 25.4 / 31.7: stays whole.
 Cut best_cut(int kind, uint32_t rows, uint32_t bpr) {
-    static const struct { double x, weights, unit, run, meet, meet_part, sums; } kCost[kPassKinds] = {
-        {1.59e-5, 0.0, 0.517, 0.131, 1.95, 0.19, 0.43}, {0.92e-5, 0.0, 0.574, 0.103, 2.01, 0.19, 0.0},
-        {0.99e-5, 7.0e-5, 0.0, 0.0, 2.65, 0.27, 0.0}, {0.96e-5, 11.3e-5, 0.0, 0.039, 1.91, 0.37, 0.0}};
+    static const struct { double x, weights, unit, run, meet, meet_part, sums, rows, least; } kCost[kPassKinds] = {
+        {1.59e-5, 0.0, 0.517, 0.131, 1.95, 0.19, 0.43, 0.0, 0.97}, {0.92e-5, 0.0, 0.574, 0.103, 2.01, 0.19, 0.0, 0.0, 0.97},
+        {0.92e-5, 0.0, 0.630, 0.103, 2.01, 0.19, 0.0, 0.0, 0.95}, {0.99e-5, 7.0e-5, 0.0, 0.0, 2.65, 0.27, 0.0, 0.0, 0.90},
+        {0.96e-5, 8.3e-5, 0.0, 0.039, 1.91, 0.37, 0.0, 0.0875e-3, 0.97}, {0.96e-5, 9.3e-5, 0.0, 0.039, 1.91, 0.37, 0.0, 0.0875e-3, 0.97},
+        {0.96e-5, 11.3e-5, 0.0, 0.039, 1.91, 0.37, 0.0, 0.0875e-3, 0.97}};
     const auto& k = kCost[kind];
     Cut best = whole_cut(kind, rows, bpr);
     const double x_block = (double)kind_block_bytes(kind);
@@ -681,11 +706,11 @@ Cut best_cut(int kind, uint32_t rows, uint32_t bpr) {
         const double turns = (double)((c.wgs * c.split + cus - 1u) / cus), side = std::max(1.0, w * turns / 4.0);
         const double units = (double)(c.most * c.each * ((c.part_blocks + w - 1u) / w)) * side;
         double t = turns * blocks * (k.x * x_block + k.weights * 2048.0 * c.most) + k.unit * units + k.run * (double)(c.each * (c.most / (uint32_t)c.run));
-        if (c.split > 1u) t += k.meet + k.meet_part * c.split + k.sums * c.split * c.most * kind_tokens(kind) / 256.0;
+        if (c.split > 1u) t += k.meet + (k.meet_part + k.rows * rows) * c.split + k.sums * c.split * c.most * kind_tokens(kind) / 256.0;
         return t;
     };
     // the estimate of the whole row is for the forms that it was fitted on; 4.6 us are in all of them
-    double least = (4.6 + cost(cut_for(kind, 8, false, rows, bpr, 1u))) * (kind == kDigits32 ? 0.92 : 0.97) - 4.6;
+    double least = (4.6 + cost(cut_for(kind, 8, false, rows, bpr, 1u))) * k.least - 4.6;
     for (uint32_t n : {2u, 3u, 4u, 5u, 6u, 8u}) {
         const Cut c = kind == kDigits16 ? cut_for(kind, 16, true, rows, bpr, n) : cut_for(kind, 8, false, rows, bpr, n);
         if (c.split != n) continue;
@@ -732,7 +757,7 @@ int launch_kind(BodyArgs a, const Cut& c, const Split& sp, hipStream_t s) {
         return c.table ? launch_run<KIND, 16, true, false>(a, c, sp, s) : launch_run<KIND, 8, false, false>(a, c, sp, s);
     } else {
         if (c.split > 1u) return launch_run<KIND, 8, false, true>(a, c, sp, s);
-        if constexpr (KIND != kDigits32)
+        if constexpr (KIND < kDigits16)
             if (c.table) return launch_run<KIND, 8, true, false>(a, c, sp, s);
         return launch_run<KIND, 8, false, false>(a, c, sp, s);
     }
@@ -742,7 +767,10 @@ int launch_main(int kind, const BodyArgs& a, const Cut& c, const Split& sp, hipS
     switch (kind) {
         case kFew4: return launch_kind<kFew4>(a, c, sp, s);
         case kFew8: return launch_kind<kFew8>(a, c, sp, s);
+        case kFew12: return launch_kind<kFew12>(a, c, sp, s);
         case kDigits16: return launch_kind<kDigits16>(a, c, sp, s);
+        case kMixed20: return launch_kind<kMixed20>(a, c, sp, s);
+        case kMixed24: return launch_kind<kMixed24>(a, c, sp, s);
         default: return launch_kind<kDigits32>(a, c, sp, s);
     }
 }
@@ -830,7 +858,7 @@ int launch_gemv_oil4_multi(const oilhip_weights& w, const float* d_x, const int*
             sp = sp2 = Split{};
         }
         const uint32_t counters = std::max(sp.n > 1u ? c.wgs : 0u, sp2.n > 1u ? c2.wgs : 0u);
-        hipLaunchKernelGGL(c.table ? pack_digits_kernel<true> : pack_digits_kernel<false>, dim3(bpr * kind_tokens(kind) / 4u), dim3(256), 0, s,
+        hipLaunchKernelGGL(c.table ? pack_digits_kernel<true> : pack_digits_kernel<false>, dim3(bpr, kind_tokens(kind) / 4u), dim3(256), 0, s,
                            PackArgs{act, d_tok ? d_tok + m0 : nullptr, xp, bpr, d_tok ? xrows : xrows - (uint32_t)m0, m, kind, reinterpret_cast<uint32_t*>(behind), counters});
         OILHIP_HIP(hipGetLastError());
         if (int rc = launch_main(kind, BodyArgs{w.d_payload, xp, d_y + (size_t)m0 * ldy, (uint32_t)w.rows, bpr, ldy, 0u, 0u, 0u, m}, c, sp, s)) return rc;
@@ -856,11 +884,12 @@ namespace {
 // Estimated us of a workgroup's piece of a job: a start per step (its activations, the table), then its runs of row groups at the pace of a
 // wavefront's blocks.  Fitted to the workgroups of seven steps of four to eight experts (1024 <-> 3584 to 4096 <-> 14336, 1 to 32 tokens
 // each) without and with the table, 2 us off on average in pieces of 5 to 170 us.
-struct PieceCost { double start, run; };                                   // run: of longest_run groups
+struct PieceCost { double start, run; };                                   // run: of jobs_run groups
 PieceCost piece_cost(int kind, bool table, uint32_t steps, uint32_t blocks, uint32_t waves) {
-    static const double kStart[2][kPassKinds] = {{3.6, 3.2, 3.9, 1.8}, {4.5, 4.3, 4.7, 1.8}}, kRun[2][kPassKinds] = {{0.083, 0.296, 0.533, 0.01}, {0.211, 0.419, 0.747, 0.01}},
-                        kGroupBlock[2][kPassKinds] = {{0.0936, 0.1081, 0.1267, 0.2225}, {0.0865, 0.0941, 0.1131, 0.2225}};
-    return {kStart[table][kind] * steps, steps * (kRun[table][kind] + 8.0 * ((blocks + waves - 1u) / waves) * kGroupBlock[table][kind] * longest_run(kind, 8))};
+    static const double kStart[2][kPassKinds] = {{3.6, 3.2, 3.5, 3.9, 2.0, 2.4, 1.9}, {4.5, 4.3, 4.4, 4.5, 2.0, 2.4, 1.9}},
+                        kRun[2][kPassKinds] = {{0.083, 0.296, 0.4, 0.533, 0.01, 0.01, 0.01}, {0.1, 0.36, 0.567, 0.79, 0.01, 0.01, 0.01}},
+                        kGroupBlock[2][kPassKinds] = {{0.0936, 0.1081, 0.119, 0.1267, 0.169, 0.190, 0.229}, {0.0880, 0.0955, 0.1091, 0.1130, 0.169, 0.190, 0.229}};
+    return {kStart[table][kind] * steps, steps * (kRun[table][kind] + 8.0 * ((blocks + waves - 1u) / waves) * kGroupBlock[table][kind] * jobs_run(kind))};
 }
 }  // namespace
 
@@ -925,7 +954,7 @@ int launch_gemv_oil4_multi_batches(int nb, const oilhip_weights* const* wa, floa
         double work = 0.0, start = 0.0, grain = 0.0;
         for (int k = 0; k < kPassKinds; ++k)
             for (uint32_t i = 0; of_kind[k] && i < split; ++i) {
-                const uint32_t run = (uint32_t)longest_run(k, 8);
+                const uint32_t run = (uint32_t)jobs_run(k);
                 const PieceCost c = p.cost[k][i] = piece_cost(k, table, p.parts.end[k][i] - p.parts.begin[k][i], p.parts.blocks[k][i], p.waves);
                 const double w = (double)of_kind[k] * ((groups + run - 1u) / run) * c.run;
                 work += w; start += w * c.start; grain += w * c.run;
@@ -950,7 +979,7 @@ int launch_gemv_oil4_multi_batches(int nb, const oilhip_weights* const* wa, floa
         double used = 0.0;
         for (uint32_t line = 0; line < mj.n * mj.split; ++line) {
             const int kind = mj.kind[line / mj.split];
-            const uint32_t run = (uint32_t)longest_run(kind, 8);
+            const uint32_t run = (uint32_t)jobs_run(kind);
             const PieceCost& c = plan.cost[kind][line % mj.split];
             auto fits = [&](double room) { return room > c.run + c.start ? (uint32_t)((room - c.start) / c.run) * run : 0u; };
             const uint32_t e = std::max(fits(most), run);
@@ -968,17 +997,16 @@ int launch_gemv_oil4_multi_batches(int nb, const oilhip_weights* const* wa, floa
         return true;
     };
     double most = plan.us;
-    while (!cut_line(most, mj)) most *= 1.01;
-    if (most == plan.us)
-        for (int i = 0; i < 16; ++i) {                                     // (pieces of one run each never stop fitting)
-            MultiJobs less = mj;
-            if (!cut_line(most *= 0.99, less)) break;
-            mj = less;
-        }
+    while (!cut_line(most, mj)) most *= 1.02;
+    for (double less : {0.92, 0.96, 0.98, 0.99}) {                         // (pieces of one run each get no shorter)
+        if (fullest <= 4u) break;
+        MultiJobs shorter = mj;
+        if (cut_line(most * less, shorter)) { mj = shorter; most *= less; }
+    }
     if ((fullest + 6ull) * 16u * (w0.cols / 2u) >= 0x80000000ull) return 1;
     size_t lds = 0;
     for (int k = 0; k < kPassKinds; ++k)
-        if (of_kind[k]) lds = std::max(lds, lds_of(k, 8, plan.waves, plan.table && jobs_table(k), longest_run(k, 8), plan.parts.chunk[k] != 0x7FFFFFFFu ? 2u : 1u, fullest));
+        if (of_kind[k]) lds = std::max(lds, lds_of(k, 8, plan.waves, plan.table && jobs_table(k), jobs_run(k), plan.parts.chunk[k] != 0x7FFFFFFFu ? 2u : 1u, fullest));
     mj.ld[0] = ldy;
     if (sums) {
         sums->n = (int)plan.split;

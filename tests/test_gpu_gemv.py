@@ -596,6 +596,22 @@ def test_oil4_several_rows_with_k_cut_between_workgroups(rows, cols, tokens):
     assert rel_l2(got.cpu().numpy(), want) <= 3e-7                # the digits' own error is 1e-7
 
 
+# passes of three tiles of few (9 to 12 tokens) and of a tile by digits with one or two of few (17 to 24): either end of each, alone and behind a
+# full pass; a single block, K whole and cut, several runs of row groups.  A sum has at most a rounding per block of 256 weights and per part of K.
+@pytest.mark.parametrize("rows,cols", [(16, 256), (1000, 1280), (600, 14336), (8209, 2816), (20000, 1024)])
+def test_oil4_several_rows_mixed_tiles(rows, cols):
+    w = gaussian_weights(rows * cols, rows + cols, outlier_every=13)
+    payload, blocks = ia.block_codec.quantize_tensor(w, ia.Format.OIL4)
+    X = torch.from_numpy(np.random.default_rng(cols).standard_normal((56, cols)).astype(np.float32)).cuda()
+    with ia.DeviceWeights.from_blocks(payload, blocks, rows, cols) as dw:
+        dense = dw.dequant().reshape(rows, cols).double()
+        for M in (9, 11, 12, 13, 16, 17, 18, 20, 21, 24, 25, 32 + 10, 32 + 19, 32 + 24):
+            got, want = dw.gemv(X[:M]), X[:M].double() @ dense.t().contiguous()
+            err = float((got.double() - want).norm() / want.norm())
+            assert err <= (cols / 256 + 16) * 2.0 ** -24, (M, err)
+            assert torch.equal(got, dw.gemv(X[:M])), M
+
+
 # Tall tensors, whose digits come from a table in LDS, against one row at a time through the FP32 kernel (its error is 1e-7 to 2e-7)
 @pytest.mark.parametrize("rows,cols,tokens", [(66001, 2048, 3), (66001, 2048, 8), (69633, 2048, 13), (20001, 8192, 5), (20001, 8192, 16), (8500, 2816, 11)])
 def test_oil4_several_rows_of_tall_tensors(rows, cols, tokens):
