@@ -67,7 +67,9 @@ struct PackArgs {
 
 __global__ void __launch_bounds__(256)
 pack_pieces_kernel(const PackArgs a) {
-    const uint32_t lane = threadIdx.x & 63u, blk = blockIdx.x % a.bpr, t = blockIdx.x / a.bpr * 4u + (threadIdx.x >> 6);
+    // (all arguments at once: read where they are needed, each adds a scalar load's latency)
+    asm volatile("" :: "s"(a.x), "s"(a.xp), "s"(a.ldx), "s"(a.bpr), "s"(a.tiles), "s"(a.grp), "s"(a.aligned), "s"(a.M));
+    const uint32_t lane = threadIdx.x & 63u, blk = blockIdx.x, t = blockIdx.y * 4u + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const uint32_t rows = 16u * a.tiles;
     if (3u * t >= rows) return;
     float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -80,7 +82,14 @@ pack_pieces_kernel(const PackArgs a) {
     uint32_t top = 0;
 #pragma unroll
     for (int e = 0; e < 4; ++e) top = max(top, __float_as_uint(v[e]) & 0x7FFFFFFFu);
-    for (int o = 32; o > 0; o >>= 1) top = max(top, (uint32_t)__shfl_xor((int)top, o, 64));
+    auto dpp = [&](auto ctrl) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)top, decltype(ctrl)::value, 0xF, 0xF, true); };
+    using std::integral_constant;
+    top = max(top, dpp(integral_constant<int, 0xB1>{}));                   // quad_perm [1,0,3,2]
+    top = max(top, dpp(integral_constant<int, 0x4E>{}));                   // [2,3,0,1]
+    top = max(top, dpp(integral_constant<int, 0x141>{}));                  // row_half_mirror
+    top = max(top, dpp(integral_constant<int, 0x140>{}));                  // row_mirror
+    top = max(max((uint32_t)__builtin_amdgcn_readlane((int)top, 0), (uint32_t)__builtin_amdgcn_readlane((int)top, 16)),
+              max((uint32_t)__builtin_amdgcn_readlane((int)top, 32), (uint32_t)__builtin_amdgcn_readlane((int)top, 48)));
     const bool bad = top >= 0x7F800000u;
     int ex = top == 0u || bad ? 0 : 14 - ((int)(top >> 23) - 127);         // to [2^14, 2^15)
     ex = ex > 140 ? 140 : ex;
@@ -707,7 +716,7 @@ int launch_gemv_any_multi(const oilhip_weights& w, const float* d_x, float* d_y,
         const float* x = d_x + (size_t)m0 * w.cols;
         const PackArgs p{x, xp, (uint32_t)w.cols, bpr, (uint32_t)tiles, grouped(src) ? 1u : 0u, (reinterpret_cast<uintptr_t>(x) & 15u) == 0 ? 1u : 0u, m};
         const uint32_t tokens = (16u * (uint32_t)tiles + 2u) / 3u;
-        hipLaunchKernelGGL(pack_pieces_kernel, dim3(bpr * ((tokens + 3u) / 4u)), dim3(256), 0, s, p);
+        hipLaunchKernelGGL(pack_pieces_kernel, dim3(bpr, (tokens + 3u) / 4u), dim3(256), 0, s, p);
         OILHIP_HIP(hipGetLastError());
         const BodyArgs a{w.d_payload + (by_descriptor(src) ? 0u : w.uniform_base), w.d_blocks, xp, d_y + (size_t)m0 * w.rows, (uint32_t)w.alloc_bytes,
                          (uint32_t)w.rows, bpr, (uint32_t)w.rows, 0u, 0u, 0u, 0u, 0u, m};

@@ -146,7 +146,7 @@ __device__ __forceinline__ void load_activations(const Activations& a, uint32_t 
             for (uint32_t i = 0; i < 8u; ++i)
                 s += b + i < bpr ? (f[i][0] * f[i][0] + f[i][1] * f[i][1]) + (f[i][2] * f[i][2] + f[i][3] * f[i][3]) : 0.0f;
         }
-        for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+        s = wave_sum(s);
         const float r = 1.0f / sqrtf(s / (float)(256u * bpr) + 1e-6f);
         for (int e = 0; e < 4; ++e) v[e] = v[e] * r * (1.0f + a.norm_w[256u * blk + 4u * lane + e]);
         if (a.xn) {

@@ -13,6 +13,7 @@
 // differ in format then diverge by 8-lane group).  Formats without a short routine go through the
 // general per-weight decoder.
 #include "common.h"
+#include "oil4_lds.h"
 #include "run_decode.h"
 
 namespace oilhip {
@@ -141,8 +142,7 @@ gemv_runs_kernel(const uint8_t* __restrict__ payload, const DevBlock* __restrict
 #pragma unroll
         for (int m = 0; m < MB; ++m) {
             float v = acc[m];
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+            v = oil4::wave_sum(v);
             if (lane == 0 && m0 + m < M) y[(size_t)(m0 + m) * rows + row] = v;
         }
     }

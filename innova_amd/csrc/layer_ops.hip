@@ -4,6 +4,7 @@
 #include <vector>
 
 #include "common.h"
+#include "oil4_lds.h"
 
 namespace oilhip {
 int launch_gemv_oil4_swiglu(const oilhip_weights& w, const float* d_h, float* d_y, hipStream_t s);
@@ -44,7 +45,7 @@ rmsnorm_kernel(const float* __restrict__ x, const float* __restrict__ w, int n, 
     } else {
         for (int i = tid; i < n; i += 1024) s = __fmaf_rn(xr[i], xr[i], s);
     }
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    s = oil4::wave_sum(s);
     if ((tid & 63) == 0) part[tid >> 6] = s;
     __syncthreads();
     float tot = 0.f;

@@ -34,6 +34,17 @@ __device__ __forceinline__ float dpp_row_bcast15(float v) {
 __device__ __forceinline__ float dpp_row_bcast31(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x143, 0xC, 0xF, false));
 }
+// The sum over the wavefront in every lane, halves first: the order of a __shfl_xor loop from 32 to 1 without its six LDS round trips.
+__device__ __forceinline__ float wave_sum(float v) {
+    const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(h[0]) + __uint_as_float(h[1]);
+    const auto q = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(q[0]) + __uint_as_float(q[1]);
+    v += dpp_row_ror8(v);
+    v += dpp_half_mirror(__int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x1B, 0xF, 0xF, true)));   // lane ^ 4: quads reversed, then the half row
+    v += dpp_quad_xor2(v);
+    return v + dpp_quad_xor1(v);
+}
 // value of the first lane of each group of 8 lanes, in all 8 lanes
 __device__ __forceinline__ uint32_t dpp_bcast8(uint32_t v) {
     const int q = __builtin_amdgcn_update_dpp(0, (int)v, 0x00, 0xF, 0xF, true);      // quad_perm [0,0,0,0]
