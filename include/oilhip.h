@@ -181,7 +181,7 @@ int oilhip_gemv_f32_ws(const oilhip_weights* w, const float* d_x, float* d_y, in
 
 /* The same product for uniform OIL4 tensors, for callers that cannot allocate device memory (code under HIP graph
  * capture, serving loops and harnesses that forbid hipMalloc).  No counterpart in the reference.  It calls no
- * hipMalloc/hipFree: the scratch its multi-row kernel needs (packed activations and their powers of two, 8 MB) is a fixed array in the
+ * hipMalloc/hipFree: the scratch its multi-row kernel needs (packed activations and their powers of two, sums of parts of wide rows where they fit, 8 MB) is a fixed array in the
  * library's code object, one per GPU.  Limits: uniform OIL4 in the plain block layout, cols <= 32768; and, for
  * wide rows (M >= 3 with cols > 8192, or M > 16 with cols > 4096), parts * tokens_per_pass * rows <= 1,043,456 (parts =
  * ceil(cols / 4096) for passes of up to 16 tokens, ceil(cols / 2048) for passes of 32; e.g. cols = 11008, M <= 16:
