@@ -153,7 +153,8 @@ int launch_gemv_oil4_multi_batches(int nb, const oilhip_weights* const* wa, floa
                                    const int* M, const int* row0, const int* list, int nlist, const float* d_x, const float* d_x2,
                                    uint32_t ldx, uint32_t xrows, uint32_t ldy, void* d_ws, size_t ws_bytes, hipStream_t s, BatchSums* sums = nullptr);
 // other formats, up to 16 rows per pass (FP16 MFMA, gemv_any_multi.hip)
-int launch_gemv_any_multi(const oilhip_weights& w, const float* d_x, float* d_y, int M, hipStream_t s, uint8_t* d_pack = nullptr);
+int launch_gemv_any_multi(const oilhip_weights& w, const float* d_x, float* d_y, int M, hipStream_t s, uint8_t* d_pack = nullptr,
+                          const MultiInput& in = {}, uint32_t ldx = 0);
 // bytes of d_pack that these two kernels need (0: they do not serve the tensor)
 size_t gemv_oil4_multi_bytes(const oilhip_weights& w, int M);
 size_t gemv_any_multi_bytes(const oilhip_weights& w, int M);

@@ -33,6 +33,7 @@
 #include "common.h"
 #include "level_digits.h"
 #include "oil4_lds.h"
+#include "pack_activations.h"
 
 namespace oilhip {
 namespace {
@@ -59,25 +60,21 @@ __host__ __device__ constexpr uint32_t tile_bytes(bool grp) { return (grp ? 9u :
 
 // ---- pre-pass --------------------------------------------------------------------------------------------------------
 struct PackArgs {
-    const float* x;
+    Activations in;
     uint8_t* xp;            // powers of two [block][16 NT] floats, one block of zeros, then the operands [block][tile][step][lane][8 halves]
-    uint32_t ldx, bpr, tiles, grp, aligned;
+    uint32_t bpr, tiles, grp;
     int M;
 };
 
 __global__ void __launch_bounds__(256)
 pack_pieces_kernel(const PackArgs a) {
     // (all arguments at once: read where they are needed, each adds a scalar load's latency)
-    asm volatile("" :: "s"(a.x), "s"(a.xp), "s"(a.ldx), "s"(a.bpr), "s"(a.tiles), "s"(a.grp), "s"(a.aligned), "s"(a.M));
+    asm volatile("" :: "s"(a.in.x), "s"(a.in.x2), "s"(a.in.norm_w), "s"(a.in.ldx), "s"(a.in.aligned), "s"(a.xp), "s"(a.bpr), "s"(a.tiles), "s"(a.grp), "s"(a.M));
     const uint32_t lane = threadIdx.x & 63u, blk = blockIdx.x, t = blockIdx.y * 4u + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const uint32_t rows = 16u * a.tiles;
     if (3u * t >= rows) return;
     float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    if ((int)t < a.M) {
-        const float* p = a.x + (size_t)t * a.ldx + 256u * blk + 4u * lane;
-        if (a.aligned) { const float4 f = *reinterpret_cast<const float4*>(p); v[0] = f.x; v[1] = f.y; v[2] = f.z; v[3] = f.w; }
-        else { for (int e = 0; e < 4; ++e) v[e] = p[e]; }
-    }
+    if ((int)t < a.M) load_activations(a.in, t, blk, a.bpr, lane, v);
     // the largest magnitude as a bit pattern: infinities and NaN are the largest of all
     uint32_t top = 0;
 #pragma unroll
@@ -703,7 +700,7 @@ size_t gemv_any_multi_bytes(const oilhip_weights& w, int M) {
 
 // Returns 1 where these kernels do not serve the call.  Without d_pack, a call that is being captured is left to the kernels that
 // use no scratch: two graphs captured on one stream would share the stream's, and they may be replayed side by side.
-int launch_gemv_any_multi(const oilhip_weights& w, const float* d_x, float* d_y, int M, hipStream_t s, uint8_t* d_pack) {
+int launch_gemv_any_multi(const oilhip_weights& w, const float* d_x, float* d_y, int M, hipStream_t s, uint8_t* d_pack, const MultiInput& in, uint32_t ldx) {
     const int src = source_for(w, M);
     if (src < 0 || (!d_pack && stream_capturing(s))) return 1;
     const uint32_t bpr = (uint32_t)(w.cols >> 8);
@@ -713,8 +710,11 @@ int launch_gemv_any_multi(const oilhip_weights& w, const float* d_x, float* d_y,
         if (int rc = stream_scratch(lock, kScratchGemvPack, kGemvPackBytes, reinterpret_cast<void**>(&xp))) return rc;
     for (int m0 = 0; m0 < M; m0 += kPassTokens) {
         const int m = std::min(M - m0, kPassTokens), tiles = tiles_for(m);
-        const float* x = d_x + (size_t)m0 * w.cols;
-        const PackArgs p{x, xp, (uint32_t)w.cols, bpr, (uint32_t)tiles, grouped(src) ? 1u : 0u, (reinterpret_cast<uintptr_t>(x) & 15u) == 0 ? 1u : 0u, m};
+        if (!ldx) ldx = (uint32_t)w.cols;
+        const size_t skip = (size_t)m0 * ldx;
+        const uint32_t aligned = ((reinterpret_cast<uintptr_t>(d_x) | reinterpret_cast<uintptr_t>(in.x2)) & 15u) == 0 && (ldx & 3u) == 0;
+        const PackArgs p{{d_x + skip, in.x2 ? in.x2 + skip : nullptr, in.norm_w, in.xn ? in.xn + skip : nullptr, ldx, aligned, in.inv_form ? 1u : 0u},
+                         xp, bpr, (uint32_t)tiles, grouped(src) ? 1u : 0u, m};
         const uint32_t tokens = (16u * (uint32_t)tiles + 2u) / 3u;
         hipLaunchKernelGGL(pack_pieces_kernel, dim3(bpr, (tokens + 3u) / 4u), dim3(256), 0, s, p);
         OILHIP_HIP(hipGetLastError());

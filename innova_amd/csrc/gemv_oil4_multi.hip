@@ -41,6 +41,7 @@
 #include "common.h"
 #include "level_digits.h"
 #include "oil4_lds.h"
+#include "pack_activations.h"
 
 namespace oilhip {
 namespace {
@@ -105,13 +106,6 @@ struct PackJobs {
 // where a batch's powers of two start (floats [block][kMaxTokens]) and its packed blocks after them
 __host__ __device__ constexpr uint32_t undo_bytes(uint32_t bpr) { return bpr * (uint32_t)kMaxTokens * 4u; }
 
-// What the rows are multiplied as: x, silu(x) * x2, or x * (1 + norm_w) / rms(x).
-struct Activations {
-    const float *x, *x2, *norm_w;
-    float* xn;                  // with norm_w: the normalised rows go here as well (optional, laid out like x)
-    uint32_t ldx, aligned, inv_form;
-};
-
 struct PackArgs {
     Activations in;
     const int* tok;
@@ -121,40 +115,6 @@ struct PackArgs {
     uint32_t* arrived;          // counters that the main launch wants zero
     uint32_t ncount;
 };
-
-// this lane's four columns of block `blk` of row `src`
-__device__ __forceinline__ void load_activations(const Activations& a, uint32_t src, uint32_t blk, uint32_t bpr, uint32_t lane, float (&v)[4]) {
-    const float* row = a.x + (size_t)src * a.ldx;
-    const float* p = row + 256u * blk + 4u * lane;
-    auto load = [&](const float* q, float (&o)[4]) {
-        if (a.aligned) { const float4 f = *reinterpret_cast<const float4*>(q); o[0] = f.x; o[1] = f.y; o[2] = f.z; o[3] = f.w; }
-        else { for (int e = 0; e < 4; ++e) o[e] = q[e]; }
-    };
-    load(p, v);
-    if (a.x2) {
-        float u[4];
-        load(a.x2 + (p - a.x), u);
-        // silu(g) * u as ExpertFFN::forward (src/moe_variants.cpp:77-91) or mlp_step (qwen35_engine.cpp:31,37,617) forms it
-        for (int e = 0; e < 4; ++e) v[e] = (a.inv_form ? v[e] * (1.0f / (1.0f + expf(-v[e]))) : v[e] / (1.0f + expf(-v[e]))) * u[e];
-    } else if (a.norm_w) {
-        float s = 0.0f;
-        for (uint32_t b = 0; b < bpr; b += 8u) {                           // eight loads in flight; past the end: the last block, counted as 0
-            float f[8][4];
-#pragma unroll
-            for (uint32_t i = 0; i < 8u; ++i) load(row + 256u * (b + i < bpr ? b + i : bpr - 1u) + 4u * lane, f[i]);
-#pragma unroll
-            for (uint32_t i = 0; i < 8u; ++i)
-                s += b + i < bpr ? (f[i][0] * f[i][0] + f[i][1] * f[i][1]) + (f[i][2] * f[i][2] + f[i][3] * f[i][3]) : 0.0f;
-        }
-        s = wave_sum(s);
-        const float r = 1.0f / sqrtf(s / (float)(256u * bpr) + 1e-6f);
-        for (int e = 0; e < 4; ++e) v[e] = v[e] * r * (1.0f + a.norm_w[256u * blk + 4u * lane + e]);
-        if (a.xn) {
-            float* o = a.xn + (size_t)src * a.ldx + 256u * blk + 4u * lane;
-            for (int e = 0; e < 4; ++e) o[e] = v[e];
-        }
-    }
-}
 
 // A block's 256 columns (four per lane) to digits: put(e, p, bytes) receives for column e of the lane its nibble p and the digits
 // as bytes 0 (low) to 3.  Returns what undoes the scaling.  Uniform over the wavefront.

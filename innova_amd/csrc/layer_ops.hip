@@ -108,6 +108,10 @@ int gemv_rmsnorm(const oilhip_weights& w, const float* d_x, const float* d_normw
                                               MultiInput{nullptr, d_normw, false, d_xn}, nullptr, nullptr, 0, d_pack);
         if (rc <= 0) return rc;
     }
+    if (M >= 2 && !plain_oil4(w) && w.cols <= kPackNormMaxCols && apart) { // likewise for the other formats
+        const int rc = launch_gemv_any_multi(w, d_x, d_y, M, s, d_pack, MultiInput{nullptr, d_normw, false, d_xn});
+        if (rc <= 0) return rc;
+    }
     if (int rc = oilhip_rmsnorm_f32(d_x, d_normw, (int)w.cols, M, d_xn, s)) return rc;
     return gemv_f32(w, d_xn, d_y, M, s, d_pack);
 }
@@ -134,6 +138,10 @@ int mlp_step(const oilhip_weights& gate_up, const oilhip_weights& down, const fl
     if (M > 2 && plain_oil4(down)) {                         // SwiGLU formed while the activations are packed
         const int rc = launch_gemv_oil4_multi(down, h2, nullptr, d_y, M, (uint32_t)(2 * F), (uint32_t)down.rows, (uint32_t)M, s,
                                               MultiInput{h2 + F, nullptr, true}, nullptr, nullptr, 0, d_pack);
+        if (rc <= 0) return rc;
+    }
+    if (M >= 2 && !plain_oil4(down)) {
+        const int rc = launch_gemv_any_multi(down, h2, d_y, M, s, d_pack, MultiInput{h2 + F, nullptr, true}, (uint32_t)(2 * F));
         if (rc <= 0) return rc;
     }
     const size_t n = (size_t)F * (size_t)M;

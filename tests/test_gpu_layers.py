@@ -205,3 +205,32 @@ def test_stack_rows_of_mixed_and_different_formats():
     assert np.array_equal(deq.view(np.uint32), np.concatenate(dq).view(np.uint32))
     for p in parts:
         p.close()
+
+
+# several rows of the other formats: norm and SwiGLU formed while the activations are packed; more rows than a pass holds, rows too wide for the
+# norm there, activations that are not aligned, and formats whose few rows keep the separate kernels
+@pytest.mark.parametrize("M,D,F,fmt,shift", [(3, 512, 768, (0, 1), 0), (17, 1024, 768, ia.Format.SPARK_Q0, 0), (6, 768, 512, (7, 9, 10, 11), 1),
+                                             (9, 512, 1024, ia.Format.OIL8, 0), (5, 8448, 512, ia.Format.OIL2, 0), (4, 512, 768, ia.Format.OIL8, 0),
+                                             (5, 512, 768, (0, 1, 3), 0)])
+def test_several_rows_of_other_formats_with_norm(M, D, F, fmt, shift):
+    rng = np.random.default_rng(D + F + M)
+    mats = {}
+    for name, (r, c) in (("gate", (F, D)), ("up", (F, D)), ("down", (D, F))):
+        w = gaussian_weights(r * c, seed=len(name) + D) * np.float32(50.0 / np.sqrt(c))
+        mats[name] = (r, c) + ia.block_codec.quantize_tensor(w, block_formats(fmt, r * c // 256, len(name)))
+    x = (rng.standard_normal((M, D)) * 2.0).astype(np.float32)
+    nw = (rng.standard_normal(D) * 0.2).astype(np.float32)
+    xd = torch.zeros(shift + M * D, device="cuda")[shift:].view(M, D)
+    xd.copy_(torch.from_numpy(x))
+    dev = {k: ia.DeviceWeights.from_blocks(v[2], v[3], v[0], v[1]) for k, v in mats.items()}
+    gu = ia.DeviceWeights.stack_rows([dev["gate"], dev["up"]])
+    got_gu = layers.gemv_rmsnorm(gu, xd, torch.from_numpy(nw).cuda()).cpu().numpy()
+    got = layers.mlp_step(gu, dev["down"], xd, norm_w=torch.from_numpy(nw).cuda()).cpu().numpy()
+    xn = O.rmsnorm(x, nw)
+    g = O.block_gemm(mats["gate"][2], to_orc_blocks(mats["gate"][3]), F, D, xn, wide=True)
+    u = O.block_gemm(mats["up"][2], to_orc_blocks(mats["up"][3]), F, D, xn, wide=True)
+    assert rel_l2(got_gu, np.concatenate([g, u], axis=1)) <= TOL
+    want = O.block_gemm(mats["down"][2], to_orc_blocks(mats["down"][3]), D, F, O.swiglu(g.astype(np.float32), u.astype(np.float32)), wide=True)
+    assert rel_l2(got, want) <= TOL
+    for d in list(dev.values()) + [gu]:
+        d.close()
