@@ -15,6 +15,7 @@
 #include <c10/hip/HIPStream.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "../../include/oilhip.h"
 
@@ -88,13 +89,17 @@ PyObject* raise(int rc) {
     Py_XDECREF(m);
     return nullptr;
 }
-template <class F>
-int without_gil(F&& f) {
-    int rc;
-    Py_BEGIN_ALLOW_THREADS
-    rc = f();
-    Py_END_ALLOW_THREADS
-    return rc;
+// The library's `f` without the interpreter's lock.  Its arguments are plain values, worked out while the lock is held: data_ptr() raises
+// for a tensor without storage (those of torch.func's transforms), and nothing may be thrown past a lock that is not taken again.
+struct Unlocked {
+    PyThreadState* state = PyEval_SaveThread();
+    ~Unlocked() { PyEval_RestoreThread(state); }
+};
+template <class... P, class... A>
+int without_gil(int (*f)(P...), A... a) {
+    static_assert((std::is_scalar_v<A> && ...), "pointers and numbers, not what they are read from");
+    const Unlocked unlocked;
+    return f(a...);
 }
 // `f` as a Python function: None for what it does not take, an OilHipError for a failed call
 template <class F>
@@ -123,7 +128,7 @@ PyObject* gemv(PyObject*, PyObject* const* a, Py_ssize_t n) {
         void* s = stream();
         if (M > 1) need_no_capture(s);
         const at::Tensor y = output(a[2], {M, size(a[3])}, x);
-        return result(without_gil([&] { return oilhip_gemv_f32(w, f32(x), f32(y), (int)M, s); }), a[2], y);
+        return result(without_gil(oilhip_gemv_f32, w, f32(x), f32(y), (int)M, s), a[2], y);
     });
 }
 // gemm(weights, x, out, rows, cols, bf16)
@@ -135,9 +140,8 @@ PyObject* gemm(PyObject*, PyObject* const* a, Py_ssize_t n) {
         const int64_t M = rows_of(x, size(a[4]));
         const at::Tensor y = output(a[2], {M, size(a[3])}, x);
         void* s = stream();
-        const int rc = without_gil([&] {
-            return bf16 ? oilhip_gemm_bf16(w, static_cast<const uint16_t*>(x.data_ptr()), f32(y), (int)M, s) : oilhip_gemm_f32(w, f32(x), f32(y), (int)M, s);
-        });
+        const int rc = bf16 ? without_gil(oilhip_gemm_bf16, w, static_cast<const uint16_t*>(x.data_ptr()), f32(y), (int)M, s)
+                            : without_gil(oilhip_gemm_f32, w, f32(x), f32(y), (int)M, s);
         return result(rc, a[2], y);
     });
 }
@@ -147,7 +151,7 @@ PyObject* dequant(PyObject*, PyObject* const* a, Py_ssize_t n) {
         const auto* w = handle<oilhip_weights>(a[0]);
         const at::Tensor y = at::empty({size(a[1]) * size(a[2])}, at::TensorOptions().dtype(at::kFloat).device(at::kCUDA, c10::hip::current_device()));
         void* s = stream();
-        return result(without_gil([&] { return oilhip_dequant_f32(w, f32(y), s); }), Py_None, y);
+        return result(without_gil(oilhip_dequant_f32, w, f32(y), s), Py_None, y);
     });
 }
 // embed_rows(weights, ids, cols) into a new tensor
@@ -158,7 +162,7 @@ PyObject* embed_rows(PyObject*, PyObject* const* a, Py_ssize_t n) {
         need(ids.numel() <= 0x7FFFFFFF);
         const at::Tensor y = empty({ids.numel(), size(a[2])}, ids);
         void* s = stream();
-        return result(without_gil([&] { return oilhip_embed_rows_f32(w, static_cast<const int*>(ids.data_ptr()), (int)ids.numel(), f32(y), s); }), Py_None, y);
+        return result(without_gil(oilhip_embed_rows_f32, w, static_cast<const int*>(ids.data_ptr()), (int)ids.numel(), f32(y), s), Py_None, y);
     });
 }
 // gemv_rmsnorm(weights, x, norm_w, out, rows, cols)
@@ -170,7 +174,7 @@ PyObject* gemv_rmsnorm(PyObject*, PyObject* const* a, Py_ssize_t n) {
         void* s = stream();
         if (M > 1) need_no_capture(s);
         const at::Tensor y = output(a[3], {M, size(a[4])}, x), xn = empty(x.sizes(), x);
-        return result(without_gil([&] { return oilhip_gemv_rmsnorm_f32(w, f32(x), f32(nw), f32(y), (int)M, f32(xn), s); }), a[3], y);
+        return result(without_gil(oilhip_gemv_rmsnorm_f32, w, f32(x), f32(nw), f32(y), (int)M, f32(xn), s), a[3], y);
     });
 }
 // mlp_step(gate_up, down, x, norm_w or None, out, rows of down, cols of gate_up, cols of down)
@@ -183,26 +187,22 @@ PyObject* mlp_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
         void* s = stream();
         if (M > 1) need_no_capture(s);
         const at::Tensor y = output(a[4], {M, size(a[5])}, x), scratch = empty({(3 * F + D) * M}, x);
-        return result(without_gil([&] { return oilhip_mlp_step_f32(gu, down, f32(x), nw, f32(y), (int)M, f32(scratch), s); }), a[4], y);
+        return result(without_gil(oilhip_mlp_step_f32, gu, down, f32(x), nw, f32(y), (int)M, f32(scratch), s), a[4], y);
     });
 }
 // oil8_gemm / oil4_gemm(codes, codebook, activations, M, N, K)
-template <class F>
-PyObject* flat_gemm(PyObject* const* a, Py_ssize_t n, F&& f) {
+template <class Book>
+PyObject* flat_gemm(PyObject* const* a, Py_ssize_t n, int (*f)(const uint8_t*, const Book*, const float*, float*, int, int, int, void*)) {
     return ordinary(n, 6, [&]() -> PyObject* {
         const at::Tensor &codes = tensor(a[0]), &cb = tensor(a[1]), &x = tensor(a[2]);
         const int M = (int)size(a[3]), N = (int)size(a[4]), K = (int)size(a[5]);
         const at::Tensor y = empty({M, N}, x);
         void* s = stream();
-        return result(without_gil([&] { return f(u8(codes), cb.data_ptr(), f32(x), f32(y), M, N, K, s); }), Py_None, y);
+        return result(without_gil(f, u8(codes), static_cast<const Book*>(cb.data_ptr()), f32(x), f32(y), M, N, K, s), Py_None, y);
     });
 }
-PyObject* oil8_gemm(PyObject*, PyObject* const* a, Py_ssize_t n) {
-    return flat_gemm(a, n, [](uint8_t* w, void* cb, float* x, float* y, int M, int N, int K, void* s) { return oilhip_flat_oil8_gemm(w, static_cast<float*>(cb), x, y, M, N, K, s); });
-}
-PyObject* oil4_gemm(PyObject*, PyObject* const* a, Py_ssize_t n) {
-    return flat_gemm(a, n, [](uint8_t* w, void* cb, float* x, float* y, int M, int N, int K, void* s) { return oilhip_flat_oil4_gemm(w, static_cast<uint16_t*>(cb), x, y, M, N, K, s); });
-}
+PyObject* oil8_gemm(PyObject*, PyObject* const* a, Py_ssize_t n) { return flat_gemm(a, n, oilhip_flat_oil8_gemm); }
+PyObject* oil4_gemm(PyObject*, PyObject* const* a, Py_ssize_t n) { return flat_gemm(a, n, oilhip_flat_oil4_gemm); }
 // prod(bits, codes, codebook or None, scale, activations, M, N, K): M weight rows, N activation rows
 PyObject* prod(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return ordinary(n, 8, [&]() -> PyObject* {
@@ -214,11 +214,9 @@ PyObject* prod(PyObject*, PyObject* const* a, Py_ssize_t n) {
         const int M = (int)size(a[5]), N = (int)size(a[6]), K = (int)size(a[7]);
         const at::Tensor y = empty({N, M}, x);
         void* s = stream();
-        const int rc = without_gil([&] {
-            return bits == 2 ? oilhip_prod_gemv_spark(u8(w), scale, f32(x), f32(y), M, K, N, s)
-                 : bits == 4 ? oilhip_prod_gemv_oil4(u8(w), static_cast<uint16_t*>(cb), scale, f32(x), f32(y), M, K, N, s)
-                             : oilhip_prod_gemv_oil8(u8(w), static_cast<float*>(cb), scale, f32(x), f32(y), M, K, N, s);
-        });
+        const int rc = bits == 2 ? without_gil(oilhip_prod_gemv_spark, u8(w), scale, f32(x), f32(y), M, K, N, s)
+                     : bits == 4 ? without_gil(oilhip_prod_gemv_oil4, u8(w), static_cast<uint16_t*>(cb), scale, f32(x), f32(y), M, K, N, s)
+                                 : without_gil(oilhip_prod_gemv_oil8, u8(w), static_cast<float*>(cb), scale, f32(x), f32(y), M, K, N, s);
         return result(rc, Py_None, y);
     });
 }
@@ -231,7 +229,7 @@ PyObject* engine_quant_gemm(PyObject*, PyObject* const* a, Py_ssize_t n) {
         const int64_t M = size(a[4]), N = size(a[5]), K = size(a[6]);
         const at::Tensor y = empty({M, N}, x);
         void* s = stream();
-        return result(without_gil([&] { return oilhip_engine_quant_gemm((int)bits, f32(x), u8(codes), f32(cb), f32(y), M, N, K, s); }), Py_None, y);
+        return result(without_gil(oilhip_engine_quant_gemm, (int)bits, f32(x), u8(codes), f32(cb), f32(y), M, N, K, s), Py_None, y);
     });
 }
 // kv_append(cache, layer, k, v, values of a token): True
@@ -244,7 +242,7 @@ PyObject* kv_append(PyObject*, PyObject* const* a, Py_ssize_t n) {
         const int64_t seq = k.size(2), token = size(a[4]);
         need(k.numel() == seq * token && v.numel() == k.numel());
         void* s = stream();
-        if (const int rc = without_gil([&] { return oilhip_kv_append(c, layer, f32(k), f32(v), seq, s); })) return raise(rc);
+        if (const int rc = without_gil(oilhip_kv_append, c, layer, f32(k), f32(v), seq, s)) return raise(rc);
         Py_RETURN_TRUE;
     });
 }
@@ -260,7 +258,7 @@ PyObject* kv_get_range(PyObject*, PyObject* const* a, Py_ssize_t n) {
         const at::Tensor k = at::empty({1, heads, len, dim}, options), v = at::empty({1, heads, len, dim}, options);
         int64_t got = 0;
         void* s = stream();
-        if (const int rc = without_gil([&] { return oilhip_kv_get_range(c, layer, start, end, f32(k), f32(v), &got, s); })) return raise(rc);
+        if (const int rc = without_gil(oilhip_kv_get_range, c, layer, start, end, f32(k), f32(v), &got, s)) return raise(rc);
         need(got == len);
         PyObject *pk = THPVariable_Wrap(k), *pv = THPVariable_Wrap(v), *pair = pk && pv ? PyTuple_Pack(2, pk, pv) : nullptr;
         Py_XDECREF(pk);
