@@ -40,15 +40,19 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 // Sign table of one activation row: for every four columns all sixteen sums +-x0 +-x1 +-x2 +-x3, entry n the one in which bit j of n makes x[j]
 // positive.  A SPARK_Q0 run is then eight reads instead of 32 products of unpacked signs: 30 vector instructions fewer per step, and
 // about 10 clocks of LDS for each read (16 for 16 bytes per lane of plain activations).  Where another format of the tensor works on few instructions per weight
-// beside it that pays: planner's mix, 12288 x 4096 7.53 -> 7.28 us, 22016 x 4096 12.3 -> 11.5, 30000 x 2048 10.4 -> 9.6.  SPARK_Q0 alone is bound by LDS
+// beside it that pays: planner's mix, 12288 x 4096 7.53 -> 7.38 us, 22016 x 4096 12.3 -> 11.4, 30000 x 2048 10.4 -> 9.5.  SPARK_Q0 alone is bound by LDS
 // then (11008 x 4096 10.2 -> 10.4), and with eight wavefronts building the table costs more than it saves (4096 x 4096 5.03 -> 5.22): both stay.  Error
-// against 64 bits (2-norm, planner's mix) 1.0e-7 -> 0.94e-7.
+// against 64 bits (2-norm, planner's mix) 1.0e-7 -> 0.94e-7.  The sums are of x / 32, so that those of a run's 32 activations stay below the largest float
+// where the activations do, and the block's scale is taken 32 times: both exact, but for activations below 2^-121, whose lowest bits go
+// (2^-150 at most: with weights below 1/32 that is less than the rounding of a subnormal product).  That costs 0.05 to 0.1 us at these sizes, which the figures
+include.
 constexpr uint32_t kSignRunBytes = 8u * 64u + 64u;        // a run's eight tables; the gap spreads runs over the LDS banks
 constexpr uint32_t kSignTab = kLevelTabBytes + 64;        // where the table starts in LDS
 typedef __attribute__((address_space(3))) f32x4_t lds_f4;
 
 // the entries of columns 4 * c4 .. 4 * c4 + 3
 __device__ __forceinline__ void put_signs(uint32_t c4, float4 t) {
+    t.x *= 0.03125f; t.y *= 0.03125f; t.z *= 0.03125f; t.w *= 0.03125f;
     // neighbouring lanes write their four 16-byte pieces in different orders, so that eight of them hit all banks: piece j ^ sw holds the
     // sums with the signs of j and those that sw flips
     const uint32_t g = c4 & 7u, sw = g >> 1, at = kSignTab + (c4 >> 3) * kSignRunBytes + g * 64u + sw * 16u;
@@ -61,7 +65,7 @@ __device__ __forceinline__ void put_signs(uint32_t c4, float4 t) {
     }
 }
 
-// sum of +-x over the run whose table is at `base`: bit k of u set -> +x[k], else -x[k]
+// a 32nd of the sum of +-x over the run whose table is at `base`: bit k of u set -> +x[k], else -x[k]
 __device__ __forceinline__ float signed_sum(uint32_t u, uint32_t base) {
     float v[8];
 #pragma unroll
@@ -147,7 +151,7 @@ __device__ __forceinline__ void run_entry(const uint8_t* data, const uint8_t* ta
         const uint32_t rowl = tag >> tshift, run = (tag & tmask) * 8u + r;
         float part[MB];
         if constexpr (FMT == 1 && SIGNS) {
-            part[0] = f16_bits(raw[0]) * signed_sum(raw[1], kSignTab + run * kSignRunBytes);
+            part[0] = (32.0f * f16_bits(raw[0])) * signed_sum(raw[1], kSignTab + run * kSignRunBytes);
         } else if constexpr (FMT == 1) {
             // weight k = bit k ? +scale : -scale; as FP16: |scale| with the sign bit from the (inverted) sign word.
             // Pair k holds weights k (low half) and k + 16 (high half).

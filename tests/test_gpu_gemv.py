@@ -123,6 +123,32 @@ def test_mixed_format_sign_table(rows, cols, fmt_ids):
         assert np.array_equal(np.isnan(inf), np.isnan(plain)) and np.array_equal(np.isinf(inf), np.isinf(plain))
 
 
+# The same table with activations whose signed sums over a run pass the largest float while every product with a weight, and the output, are far below
+# it, and with activations so small that their products are near the smallest normal float.  Signs alternate, so that OIL1's run sums stay finite.
+@pytest.mark.parametrize("fmt_ids", [(0, 1), (1, 13)])
+@pytest.mark.parametrize("rows,cols", [(8193, 512), (8200, 1280)])
+@pytest.mark.parametrize("size", [1e38, 1.0, 1e-34])
+def test_mixed_format_sign_table_range(rows, cols, fmt_ids, size):
+    rng = np.random.default_rng(rows + cols)
+    fmts = rng.choice(np.array(fmt_ids, dtype=np.uint8), size=rows * cols // 256)
+    payload, blocks = ia.block_codec.quantize_tensor(gaussian_weights(rows * cols, cols), fmts)
+    x = rng.uniform(0.3, 1.0, cols) * np.tile([1.0, -1.0], cols // 2)
+    xd = torch.from_numpy((x * size).astype(np.float32)).cuda()
+    one = torch.from_numpy(np.tile(np.float32([1.0, -1.0]), cols // 2)).cuda()
+    bound = (cols / 256 + 32 + 6) * 2.0 ** -24
+    with ia.DeviceWeights.from_blocks(payload, blocks, rows, cols) as dw:
+        W = dw.dequant().view(rows, cols).double()
+        got = dw.gemv(xd[None]).double() / size
+        want = W @ (xd.double() / size)
+        assert rel_l2(got.cpu().numpy(), want.cpu().numpy()) <= bound
+        assert rel_l2((dw.gemv(xd[None], general=True).double() / size).cpu().numpy(), want.cpu().numpy()) <= TOL
+        if size >= 1.0:                                   # behind the fused norm: its weights bring the size, the activations the alternating signs
+            nw = torch.from_numpy((np.abs(x) * size).astype(np.float32)).cuda()
+            got = layers.gemv_rmsnorm(dw, one[None], nw).double() / size
+            want = W @ (one.double() * ((1.0 + nw).double() / size)) / np.sqrt(1.0 + 1e-6)
+            assert rel_l2(got.cpu().numpy(), want.cpu().numpy()) <= bound + 2.0 ** -22      # the norm's own factor
+
+
 def test_mixed_format_skewed_tiles():
     """Tiles in which a format is absent, or holds a single block, or fills every block."""
     rows, cols = 24, 2048
