@@ -45,7 +45,7 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 // against 64 bits (2-norm, planner's mix) 1.0e-7 -> 0.94e-7.  The sums are of x / 32, so that those of a run's 32 activations stay below the largest float
 // where the activations do, and the block's scale is taken 32 times: both exact, but for activations below 2^-121, whose lowest bits go
 // (2^-150 at most: with weights below 1/32 that is less than the rounding of a subnormal product).  That costs 0.05 to 0.1 us at these sizes, which the figures
-include.
+// include.
 constexpr uint32_t kSignRunBytes = 8u * 64u + 64u;        // a run's eight tables; the gap spreads runs over the LDS banks
 constexpr uint32_t kSignTab = kLevelTabBytes + 64;        // where the table starts in LDS
 typedef __attribute__((address_space(3))) f32x4_t lds_f4;
