@@ -372,6 +372,8 @@ int oilhip_moe_forward(const oilhip_weights* const* gate, const oilhip_weights* 
  *                               written (end is clipped to the tokens held; 0 where the reference returns empty tensors).
  *                               get_all is get_range(layer, 0, context).  Tokens that were dropped are never returned
  *                               (the reference reads past its arrays there).
+ * oilhip_kv_held              : the tokens of a layer that get_range can return, for sizing its outputs (0 for a layer that the cache
+ *                               does not have)
  * oilhip_kv_info              : context_len() (layer 0), block_size(), size_bytes(), size_bytes_fp32_equivalent() (:364-392)
  * oilhip_kv_clear / _resize   : clear() (:394-402), resize(new_max_seq_len) (:404-416, every layer empty afterwards;
  *                               synchronises the device and reallocates)
@@ -388,6 +390,7 @@ int oilhip_kv_destroy(oilhip_kv* c);
 int oilhip_kv_append(oilhip_kv* c, int layer, const float* d_k, const float* d_v, int64_t seq_len, void* stream);
 int oilhip_kv_get_range(const oilhip_kv* c, int layer, int64_t start, int64_t end, float* d_k, float* d_v, int64_t* len_out,
                         void* stream);
+int oilhip_kv_held(const oilhip_kv* c, int layer, int64_t* tokens);
 int oilhip_kv_info(const oilhip_kv* c, int* context_len, int64_t* block_size, uint64_t* size_bytes, uint64_t* fp32_bytes);
 int oilhip_kv_clear(oilhip_kv* c, void* stream);
 int oilhip_kv_resize(oilhip_kv* c, int64_t new_max_seq_len);

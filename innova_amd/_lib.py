@@ -98,6 +98,7 @@ _SIGNATURES = {
     "oilhip_kv_destroy": (C.c_int, [vp]),
     "oilhip_kv_append": (C.c_int, [vp, C.c_int, vp, vp, C.c_int64, vp]),
     "oilhip_kv_get_range": (C.c_int, [vp, C.c_int, C.c_int64, C.c_int64, vp, vp, C.POINTER(C.c_int64), vp]),
+    "oilhip_kv_held": (C.c_int, [vp, C.c_int, C.POINTER(C.c_int64)]),
     "oilhip_kv_info": (C.c_int, [vp, C.POINTER(C.c_int), C.POINTER(C.c_int64), C.POINTER(C.c_uint64), C.POINTER(C.c_uint64)]),
     "oilhip_kv_clear": (C.c_int, [vp, vp]),
     "oilhip_kv_resize": (C.c_int, [vp, C.c_int64]),

@@ -692,18 +692,25 @@ int oilhip_kv_append(oilhip_kv* c, int layer, const float* d_k, const float* d_v
     return OILHIP_OK;
 }
 
+int oilhip_kv_held(const oilhip_kv* c, int layer, int64_t* tokens) {
+    if (!c || !tokens) return fail(OILHIP_E_ARG, "kv_held: null argument");
+    // the reference would read past its arrays where tokens were dropped; those are not returned
+    *tokens = layer < 0 || layer >= c->layers || c->per_token == 0 ? 0 : std::min(c->pos[(size_t)layer], c->max_seq);
+    return OILHIP_OK;
+}
+
 int oilhip_kv_get_range(const oilhip_kv* c, int layer, int64_t start, int64_t end, float* d_k, float* d_v, int64_t* len_out,
                         void* stream) {
     if (len_out) *len_out = 0;
     if (!c) return fail(OILHIP_E_ARG, "kv_get_range: cache is null");
     if (layer < 0 || start < 0) return fail(OILHIP_E_ARG, "kv_get_range: negative layer or start");
     if (layer >= c->layers) return OILHIP_OK;                                       // :295
-    int64_t held = c->pos[(size_t)layer];
-    if (held > c->max_seq) held = c->max_seq;          // the reference would read past its arrays here; tokens that were dropped are not returned
+    int64_t held = 0;
+    if (int rc = oilhip_kv_held(c, layer, &held)) return rc;
     int64_t len = end - start;
     if (len <= 0) return OILHIP_OK;
     if (start + len > held) len = held - start;
-    if (len <= 0 || c->per_token == 0) return OILHIP_OK;
+    if (len <= 0) return OILHIP_OK;
     if (!d_k || !d_v) return fail(OILHIP_E_ARG, "kv_get_range: null output");
     const uint64_t first = (uint64_t)start * (uint64_t)c->per_token, count = (uint64_t)len * (uint64_t)c->per_token;
     const uint32_t shift = c->block == 32 ? 5u : c->block == 64 ? 6u : 7u;

@@ -246,19 +246,22 @@ PyObject* kv_append(PyObject*, PyObject* const* a, Py_ssize_t n) {
         Py_RETURN_TRUE;
     });
 }
-// kv_get_range(cache, layer, start, end, max_seq, heads, dim): (k, v), when the layer holds all of the range
+// kv_get_range(cache, layer, start, end, max_seq, heads, dim): (k, v) of the tokens of the range that the layer holds
 PyObject* kv_get_range(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return ordinary(n, 7, [&]() -> PyObject* {
         auto* c = handle<oilhip_kv>(a[0]);
         const int layer = (int)size(a[1]);
-        const int64_t start = size(a[2]), end = size(a[3]), max_seq = size(a[4]), heads = size(a[5]), dim = size(a[6]);
-        const int64_t len = std::min(end, max_seq) - start;
+        const int64_t start = size(a[2]), end = std::min(size(a[3]), size(a[4])), heads = size(a[5]), dim = size(a[6]);
+        need(end > start);
+        int64_t held = 0;
+        need(oilhip_kv_held(c, layer, &held) == OILHIP_OK);
+        const int64_t len = std::min(end, held) - start;
         need(len > 0);
         const auto options = at::TensorOptions().dtype(at::kFloat).device(at::kCUDA, c10::hip::current_device());
         const at::Tensor k = at::empty({1, heads, len, dim}, options), v = at::empty({1, heads, len, dim}, options);
         int64_t got = 0;
         void* s = stream();
-        if (const int rc = without_gil(oilhip_kv_get_range, c, layer, start, end, f32(k), f32(v), &got, s)) return raise(rc);
+        if (const int rc = without_gil(oilhip_kv_get_range, c, layer, start, start + len, f32(k), f32(v), &got, s)) return raise(rc);
         need(got == len);
         PyObject *pk = THPVariable_Wrap(k), *pv = THPVariable_Wrap(v), *pair = pk && pv ? PyTuple_Pack(2, pk, pv) : nullptr;
         Py_XDECREF(pk);

@@ -65,13 +65,14 @@ class OIL4KVCache:
         if both is not None:
             return both
         import torch
-        n = max(0, min(end, self._max_seq) - start)
+        held, got = C.c_int64(), C.c_int64()    # an end past the tokens held: the reference returns the shorter tensors
+        _lib.check(_lib.lib().oilhip_kv_held(self._h, layer, C.byref(held)))
+        n = max(0, min(end, held.value) - start)
         k = torch.empty((1, self._heads, n, self._dim), dtype=torch.float32, device="cuda")
         v = torch.empty_like(k)
-        got = C.c_int64()
-        _lib.check(_lib.lib().oilhip_kv_get_range(self._h, layer, start, end, k.data_ptr(), v.data_ptr(), C.byref(got),
+        _lib.check(_lib.lib().oilhip_kv_get_range(self._h, layer, start, start + n, k.data_ptr(), v.data_ptr(), C.byref(got),
                                                   _lib.current_stream()))
-        if got.value != n:                      # end past the tokens held: the reference returns the shorter tensors
+        if got.value != n:                      # cleared in between
             k = k.reshape(-1)[: got.value * self._heads * self._dim].reshape(1, self._heads, got.value, self._dim)
             v = v.reshape(-1)[: got.value * self._heads * self._dim].reshape(1, self._heads, got.value, self._dim)
         return k, v

@@ -85,6 +85,45 @@ def test_cache_both_ways(monkeypatch, heads, dim, prompt):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("native", [True, False])
+@pytest.mark.parametrize("heads,dim", [(2, 80), (3, 27)])
+def test_cache_that_is_not_full(monkeypatch, native, heads, dim):
+    """get_all() and a range past the tokens held: one decode, and outputs of the tokens held alone."""
+    monkeypatch.setattr(_lib, "_native", None if native else _Python())
+    c, held = ia.OIL4KVCache(2, 4096, heads, dim, 64), 6
+    k, v = (torch.randn(1, heads, held, dim, device="cuda") for _ in range(2))
+    c.append(1, k, v)
+    wk, wv = c.get_range(1, 0, held)
+    calls, lib = [], _lib.lib()
+    if native:                                            # the whole call is the C function's
+        monkeypatch.setattr(_lib, "lib", lambda: pytest.fail("the way through Python was taken"))
+    else:
+        class Counting:
+            def __getattr__(self, name):
+                calls.append(name)
+                return getattr(lib, name)
+        monkeypatch.setattr(_lib, "lib", Counting)
+    for start, end in ((0, None), (2, 4096), (held - 1, held + 1)):
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        calls.clear()
+        gk, gv = c.get_all(1) if end is None else c.get_range(1, start, end)
+        n = held - start
+        assert torch.cuda.max_memory_allocated() - before <= 2 * (n * heads * dim * 4 + 512)
+        assert native or calls.count("oilhip_kv_get_range") == 1
+        assert gk.shape == gv.shape == (1, heads, n, dim)
+        flat = lambda t: t.reshape(-1, heads * dim)  # noqa: E731
+        assert torch.equal(flat(gk), flat(wk)[start:]) and torch.equal(flat(gv), flat(wv)[start:])
+    monkeypatch.setattr(_lib, "lib", lambda: lib)
+    for empty in (c.get_all(0), c.get_all(2), c.get_range(1, held, held + 3), c.get_range(1, held + 2, 4096)):
+        assert all(t.shape == (1, heads, 0, dim) for t in empty)
+    for bad in ((-1, 0, 3), (1, -1, 3)):
+        with pytest.raises(ia.OilHipError, match="negative layer or start"):
+            c.get_range(*bad)
+
+
+@pytest.mark.gpu
 def test_function_modes_and_subclasses_go_through_python(monkeypatch):
     """A torch function mode sees the calls that it saw before, and so does a tensor subclass."""
     from torch.overrides import TorchFunctionMode
