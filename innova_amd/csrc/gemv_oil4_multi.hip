@@ -768,12 +768,20 @@ int static_pack_buffer(uint8_t** out) {
 }  // namespace
 
 static size_t pack_bytes(uint32_t bpr, int kind) { return undo_bytes(bpr) + (size_t)bpr * kind_block_bytes(kind); }
+// What a pass may take of a stream's scratch: it comes in two sizes, one pass, and from rows of more than 4096 weights on the static scratch's.
+static size_t pass_room(uint32_t bpr) { return bpr > 16u ? kStaticScratchBytes : kGemvPackBytes; }
+// How a pass of m tokens is cut: K only as far as the sums fit behind the activations in a stream's scratch, whatever the scratch of the call is, so that
+// captured calls (a workspace) and those that allocate nothing add in the order of the eager one.
+static Cut pass_cut(int kind, uint32_t rows, uint32_t bpr, int m) {
+    const Cut c = best_cut(kind, rows, bpr);
+    return pack_bytes(bpr, kind) + split_bytes(c, rows, m) > pass_room(bpr) ? whole_cut(kind, rows, bpr) : c;
+}
 
 size_t gemv_oil4_multi_bytes(const oilhip_weights& w, int M) {
     if (!plain_oil4(w) || !shape_covered(w, 1, (uint32_t)w.cols)) return 0;
     const uint32_t bpr = (uint32_t)(w.cols >> 8);
-    const int m = std::min(M, kMaxTokens), kind = kind_of(m);
-    return pack_bytes(bpr, kind) + split_bytes(best_cut(kind, (uint32_t)w.rows, bpr), (uint32_t)w.rows, m);
+    auto pass = [&](int m) { return m < 1 ? 0u : pack_bytes(bpr, kind_of(m)) + split_bytes(pass_cut(kind_of(m), (uint32_t)w.rows, bpr, m), (uint32_t)w.rows, m); };
+    return M < kMaxTokens ? pass(M) : std::max(pass(kMaxTokens), pass(M % kMaxTokens));
 }
 
 // Y[m][r] for m < M: x row tok[m] (or m when tok is null) of an [xrows][ldx] activation matrix; with w2 the same activations
@@ -788,17 +796,16 @@ int launch_gemv_oil4_multi(const oilhip_weights& w, const float* d_x, const int*
     const uint32_t bpr = (uint32_t)(w.cols >> 8);
     const StreamLock lock(s);
     uint8_t* xp = d_pack;
-    // a stream's scratch comes in two sizes: one pass, and from rows of more than 4096 weights on the static scratch's
-    size_t room = bpr > 16u ? kStaticScratchBytes : kGemvPackBytes;
+    size_t room = pass_room(bpr);
     if (!xp) {
         if (int rc = stream_scratch(lock, kScratchGemvPack, room, reinterpret_cast<void**>(&xp))) return rc;
     } else {
         room = pack_room ? pack_room : gemv_oil4_multi_bytes(w, M);
     }
-    // how a tensor is cut; K only as far as the sums fit behind the activations
+    // (a second tensor's sums may need more room than a workspace that was made for the first has)
     auto cut = [&](const oilhip_weights& t, int kind, int m, uint8_t* behind, Split& sp) {
         const uint32_t rows = (uint32_t)t.rows;
-        Cut c = best_cut(kind, rows, bpr);
+        Cut c = pass_cut(kind, rows, bpr, m);
         if (c.split > 1u && pack_bytes(bpr, kind) + split_bytes(c, rows, m) > room) c = whole_cut(kind, rows, bpr);
         if (c.split > 1u) sp = {c.split, c.each, (rows + 15u) & ~15u, reinterpret_cast<float*>(behind + (((size_t)c.wgs * 4u + 255u) & ~(size_t)255u)), reinterpret_cast<uint32_t*>(behind)};
         return c;

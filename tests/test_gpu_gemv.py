@@ -621,6 +621,34 @@ def test_oil4_several_rows_with_k_cut_between_workgroups(rows, cols, tokens):
     assert rel_l2(got.cpu().numpy(), want) <= 3e-7                # the digits' own error is 1e-7
 
 
+# A captured call, whose workspace is made for it, adds in the order of the eager one: where the sums of a cut K just do not fit the scratch of a stream
+# (4096 x 32768, 32 tokens: 8.02 MB), where they do, and behind a full pass.
+@pytest.mark.parametrize("rows,cols,tokens", [(4096, 32768, 32), (4096, 32768, 33), (4000, 32768, 32), (600, 14336, 53), (3000, 8192, 24)])
+def test_oil4_several_rows_captured_and_eager(rows, cols, tokens):
+    bpr, pool = cols // 256, 4096
+    payload, blocks = ia.block_codec.quantize_tensor(gaussian_weights(pool * 256, 7, outlier_every=13), ia.Format.OIL4)
+    pick = np.random.default_rng(rows).integers(0, pool, rows * bpr)
+    desc = np.zeros(rows * bpr, dtype=blocks.dtype)
+    for name in ("nw", "fmt", "cb_bytes", "idx_bytes"):
+        desc[name] = blocks[name][0]
+    desc["cb_off"] = desc["idx_off"] = 128 * np.arange(rows * bpr, dtype=np.uint64)
+    with ia.DeviceWeights.from_blocks(payload.reshape(pool, 128)[pick].reshape(-1), desc, rows, cols) as dw:
+        x, y = torch.randn(tokens, cols, generator=torch.Generator().manual_seed(cols)).cuda(), torch.empty(tokens, rows, device="cuda")
+        side, g = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            want = dw.gemv(x)
+        torch.cuda.synchronize()
+        with torch.cuda.graph(g, stream=side):
+            dw.gemv(x, out=y)
+        for _ in range(3):
+            y.fill_(float("nan"))
+            g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(y, want)
+        del g
+
+
 # passes of three tiles of few (9 to 12 tokens) and of a tile by digits with one or two of few (17 to 24): either end of each, alone and behind a
 # full pass; a single block, K whole and cut, several runs of row groups.  A sum has at most a rounding per block of 256 weights and per part of K.
 @pytest.mark.parametrize("rows,cols", [(16, 256), (1000, 1280), (600, 14336), (8209, 2816), (20000, 1024)])
