@@ -189,8 +189,9 @@ int oilhip_gemv_f32_ws(const oilhip_weights* w, const float* d_x, float* d_y, in
  * threads) race on it and must be serialized by the caller. */
 int oilhip_gemv_oil4_f32_noalloc(const oilhip_weights* w, const float* d_x, float* d_y, int M, void* stream);
 
-/* The multi-row OIL4 kernel adds everything in a fixed order inside a workgroup, so a call returns the same bits every
- * time, like the reference's sequential loop (src/adapters/tools/qwen35_engine.cpp:71-78).  The call is accepted for
+/* The multi-row OIL4 kernel adds everything in a fixed order: a row's parts inside a workgroup, and where several workgroups
+ * share rows and take a part of K each, their sums part by part by the last one to arrive.  So a call returns the same bits every time, like the
+ * reference's sequential loop (src/adapters/tools/qwen35_engine.cpp:71-78), eager, captured or without allocation.  The call is accepted for
  * either argument and changes nothing. */
 int oilhip_set_ordered_sums(int ordered);
 

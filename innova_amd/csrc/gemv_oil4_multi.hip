@@ -26,11 +26,11 @@
 // 4.6 to 5 clocks each; 100 with the table) beside 8 to 56 matrix instructions (16 clocks each, 6.5 of which hold the issue back), and memory:
 // 131072 x 4096, 4 tokens 5.2 TB/s.
 // Before (FP16 halves of levels from a 64 KB LDS table, K cut between workgroups) -> now, pre-pass included, weights from memory:
-//   11008 x 4096, 4 / 8 / 16 / 32 tokens: 12.9 / 12.9 / 15.0 / 19.9 us -> 11.6 / 12.7 / 15.3 / 21.1 us
-//   4096 x 11008: 17.4 / 18.0 / 20.5 / 25.8 us -> 13.5 / 15.8 / 20.4 / 30.7 us
-//   131072 x 4096, 4 / 16 / 32 tokens: 81 / 86 / 127 us -> 72 / 90 / 133 us;  30000 x 14336: 77 / 81 / 120 us -> 68 / 83 / 130 us
-//   2838 x 512, 5 / 16 / 32 tokens: 7.5 / 8.7 / 9.3 -> 5.1 / 5.7 / 7.0 us
-// (slower with more than 16 tokens, where four digits cost more than the table did)
+//   11008 x 4096, 4 / 8 / 16 / 32 tokens: 12.9 / 12.9 / 15.0 / 19.9 us -> 11.7 / 13.2 / 15.3 / 21.0 us
+//   4096 x 11008: 17.4 / 18.0 / 20.5 / 25.8 us -> 13.9 / 16.1 / 18.0 / 24.5 us
+//   131072 x 4096, 4 / 16 / 32 tokens: 81 / 86 / 127 us -> 62 / 90 / 141 us;  30000 x 14336: 77 / 81 / 120 us -> 61 / 85 / 131 us
+//   2838 x 512, 5 / 16 / 32 tokens: 7.5 / 8.7 / 9.3 -> 5.4 / 5.7 / 7.1 us
+// (slower with more than 16 tokens of tall tensors, where four digits cost more than the table did)
 // Error against 64 bits (2-norm): 1.8e-7 -> 0.9e-7, whatever the distribution of the activations.
 #include <hip/hip_fp16.h>
 
@@ -1026,7 +1026,7 @@ extern "C" int oilhip_gemv_oil4_f32_noalloc(const oilhip_weights* w, const float
     return rc;
 }
 
-// The sums of the decode kernels have a fixed order whatever this says: nothing is added across workgroups any more.
+// The sums of the decode kernels have a fixed order whatever this says, also where workgroups take parts of K.
 extern "C" int oilhip_set_ordered_sums(int ordered) {
     (void)ordered;
     return OILHIP_OK;
