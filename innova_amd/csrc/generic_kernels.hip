@@ -8,6 +8,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "gemm_tiles.h"
 
 namespace oilhip {
 namespace {
@@ -181,6 +182,12 @@ struct PrepareArgs {
 };
 constexpr uint32_t kParkPitch = 256u + 8u;     // bf16 per parked row: 16-byte reads of 16 rows hit every bank once
 
+__host__ __device__ constexpr uint32_t largest_block(uint32_t formats) {
+    uint32_t n = 0;
+    for (int f = 0; f < 15; ++f) n = (formats >> f & 1u) && full_block_bytes(f) > n ? full_block_bytes(f) : n;
+    return n;
+}
+
 // FORMATS: the formats that may occur, as bits; several: each block's format from its descriptor
 // NW: wavefronts of a workgroup
 template <uint32_t FORMATS, uint32_t NW>
@@ -197,8 +204,11 @@ dense_prepare_kernel(const PrepareArgs a) {
     typedef u32x4 u32x4_2 __attribute__((aligned(2)));
     typedef f32x4 f32x4_4 __attribute__((aligned(4)));
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+    // Neighbouring blocks to one XCD: with every eighth block an XCD reads addresses that are a power of two apart and so lie in few of its L2's channels.
+    // The launch alone, 5000 x 2816 of the planner's mix 13.1 -> 9.3 us; whole calls: 11008 x 4096 SPARK_Q0, 512 tokens 78.4 -> 72.5, 900 x 1024
+    // planner's mix, 50 tokens 10.6 -> 9.3, 4096 x 4096 registry's mix, 64 tokens 28.7 -> 27.3, 11008 x 4096 OIL8, 256 tokens 58.7 -> 57.9.
     const bool of_x = blockIdx.x >= a.nw;
-    const uint32_t id = of_x ? blockIdx.x - a.nw : blockIdx.x, rb = id / a.bpr, blk = id % a.bpr;
+    const uint32_t id = of_x ? blockIdx.x - a.nw : xcd_chunk(blockIdx.x, a.nw), rb = id / a.bpr, blk = id % a.bpr;
     if (blockIdx.x == 0)
         for (uint32_t i = tid; i < a.ncount; i += 64u * NW) a.arrived[i] = 0u;
     if (of_x) {
@@ -230,8 +240,10 @@ dense_prepare_kernel(const PrepareArgs a) {
         float* tb = reinterpret_cast<float*>(lds);                          // decode tables, then the formats of the rows, then the raw blocks
         uint32_t* fmts = reinterpret_cast<uint32_t*>(tb + 256 * 3 + 20);
         uint8_t* raw = reinterpret_cast<uint8_t*>(fmts + 32);
-        // R rows of this wavefront (rows past the end repeat the last one)
-        const uint32_t row = min(rb * 32u + wave * R + lane % R, a.rows - 1u) + a.row0;
+        // R rows of this wavefront (rows past the end repeat the last one); blocks of up to 64 bytes: four lanes per row and one load for all rows, else
+        // one load per row.
+        constexpr uint32_t LANES = largest_block(FORMATS) <= 64u ? 4u : 1u;
+        const uint32_t mine_of = lane / LANES % R, row = min(rb * 32u + wave * R + mine_of, a.rows - 1u) + a.row0;
         uint64_t off;
         uint32_t fmt = ONLY >= 0 ? (uint32_t)ONLY : 0u;
         if (a.blocks) {
@@ -244,25 +256,36 @@ dense_prepare_kernel(const PrepareArgs a) {
         // 16-byte pieces of the row's block: one byte per format (full_block_bytes / 16), no table in memory
         constexpr auto sizes = [](int first) { uint64_t t = 0; for (int i = 0; i < 8; ++i) t |= (uint64_t)(full_block_bytes(first + i) / 16u) << (8 * i); return t; };
         const uint32_t pieces = (uint32_t)((fmt < 8u ? sizes(0) : sizes(8)) >> (8u * (fmt & 7u))) & 0xFFu;
-        u32x4 v[R];
-        uint32_t f[R];
+        constexpr uint32_t LOADS = LANES == 1u ? R : 1u;
+        u32x4 v[LOADS];
+        uint32_t f[LOADS];
+        const bool own_piece = lane < LANES * R && lane % LANES < pieces;
+        if constexpr (LANES > 1u) {
+            v[0] = u32x4{0, 0, 0, 0};
+            if (own_piece) v[0] = *reinterpret_cast<const u32x4_4*>(a.base + off + lane % LANES * 16u);
+        } else {
 #pragma unroll
-        for (int i = 0; i < (int)R; ++i) {
-            const uint64_t o = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)off, i) |
-                               (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(off >> 32), i) << 32;
-            f[i] = (uint32_t)__builtin_amdgcn_readlane((int)pieces, i);
-            v[i] = u32x4{0, 0, 0, 0};
-            if (lane < f[i]) v[i] = *reinterpret_cast<const u32x4_4*>(a.base + o + lane * 16u);
+            for (int i = 0; i < (int)R; ++i) {
+                const uint64_t o = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)off, i) |
+                                   (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(off >> 32), i) << 32;
+                f[i] = (uint32_t)__builtin_amdgcn_readlane((int)pieces, i);
+                v[i] = u32x4{0, 0, 0, 0};
+                if (lane < f[i]) v[i] = *reinterpret_cast<const u32x4_4*>(a.base + o + lane * 16u);
+            }
         }
         if (a.need_tables) {
             for (uint32_t i = tid; i < 256u; i += 64u * NW) { tb[i] = a.T->lv8[i]; tb[256 + i] = a.T->t255[i]; tb[512 + i] = a.T->q127[i]; }
         }
         if (tid < 16) tb[768 + tid] = kLv4[tid];
         if (tid < 4) tb[784 + tid] = kLv2[tid];
-        if (ONLY < 0 && lane < R) fmts[wave * R + lane] = fmt;
+        if (ONLY < 0 && lane < LANES * R && lane % LANES == 0u) fmts[wave * R + mine_of] = fmt;
+        if constexpr (LANES > 1u) {
+            if (own_piece) *reinterpret_cast<u32x4*>(raw + (wave * R + mine_of) * a.raw_pitch + lane % LANES * 16u) = v[0];
+        } else {
 #pragma unroll
-        for (int i = 0; i < (int)R; ++i)
-            if (lane < f[i]) *reinterpret_cast<u32x4*>(raw + (wave * R + (uint32_t)i) * a.raw_pitch + lane * 16u) = v[i];
+            for (int i = 0; i < (int)R; ++i)
+                if (lane < f[i]) *reinterpret_cast<u32x4*>(raw + (wave * R + (uint32_t)i) * a.raw_pitch + lane * 16u) = v[i];
+        }
         __syncthreads();
         const FullTables L{tb, tb + 256, tb + 512, tb + 768, tb + 784};
         const uint8_t* p = raw + (lane & 31u) * a.raw_pitch;
