@@ -159,6 +159,7 @@ int gemv_f32(const oilhip_weights& w, const float* d_x, float* d_y, int M, hipSt
         if (rc == 1 && M > 2 && M <= 4) rc = launch_gemv_oil4(w, d_x, d_y, M, s);
         if (rc <= 0) return rc;
     }
+    if (signs_fastest(w, M)) return launch_gemv_signs(w, d_x, d_y, M, s);
     if (M >= 2) {
         const int rc = launch_gemv_any_multi(w, d_x, d_y, M, s, d_pack);
         if (rc <= 0) return rc;
@@ -172,6 +173,7 @@ int gemv_f32(const oilhip_weights& w, const float* d_x, float* d_y, int M, hipSt
         }
         if (rc <= 0) return rc;
     }
+    if (w.seg.sign_tiles) return launch_gemv_signs(w, d_x, d_y, M, s);
     if (w.seg.nstreams) {
         const int rc = launch_gemv_seg(w, d_x, d_y, M, s);
         if (rc <= 0) return rc;
@@ -209,6 +211,54 @@ int oilhip_probe(int* gfx, uint64_t* hbm_bytes, int* compute_units, char* name, 
     return OILHIP_OK;
 }
 
+// Tensors of SPARK_Q0 and OIL1 blocks: rewrite `pay` as sign tiles (common.h) and point the descriptors at the blocks' new places.  Returns
+// false, and leaves everything as it is, where the tensor stays with window streams: other formats; scales or means that are not finite (sign tiles
+// are multiplied as signs times activations first, which would turn an infinity of either sign into one); payloads past 32-bit offsets; and
+//   few SPARK_Q0 blocks.  Sign tiles take the same time whatever the blocks are, window streams a few instructions for an OIL1 block; one row, us,
+//   window streams -> sign tiles with 0 / 5 / 10 / 20 / 40 % SPARK_Q0: 11008 x 4096 4.4 -> 5.1 / 5.6 -> 5.2 / 5.6 -> 5.1 / 6.3 -> 5.2 / 7.4 -> 5.2;
+//   4096 x 11008 4.6 -> 6.3 / - / 5.9 -> 6.3 / 6.6 -> 6.4;
+//   wide rows that are few.  Every workgroup packs all activations, a few tiles do not earn that, and more than 64 blocks a row take parts: planner's mix
+//   600 x 14336 6.8 -> 7.1, 2000 x 14336 7.2 -> 7.4, 4096 x 14336 8.7 -> 7.4, 700 x 20480 8.0 -> 10.9, 4096 x 20480 11.4 -> 11.1, 1000 x 11008 6.4 -> 6.1.
+static bool pack_sign_tiles(std::vector<uint8_t>& pay, std::vector<DevBlock>& db, uint64_t rows, uint64_t cols, SegLayout& g, uint32_t nf) {
+    const uint64_t bpr = cols / 256, ntiles = (rows + 15) / 16, cus = (uint64_t)device_cu_count();
+    if (bpr > 64 ? ntiles < cus : bpr > 48 && ntiles * 8 < cus * 5) return false;
+    uint64_t spark = 0;
+    for (const DevBlock& d : db) spark += d.fmt == OILHIP_SPARK_Q0;
+    if (spark * (bpr > 16 ? 6 : 20) < db.size()) return false;
+    uint64_t total = (8 * bpr * ntiles + 15) & ~15ull;
+    for (const DevBlock& d : db) {
+        if (d.fmt != OILHIP_SPARK_Q0 && d.fmt != OILHIP_OIL1) return false;
+        const uint32_t step = d.fmt == OILHIP_SPARK_Q0 ? 6u : 2u;       // a run: FP16 scale and 32 signs, or FP16 mean
+        for (uint32_t r = 0; r < 8; ++r) {
+            uint16_t h;
+            std::memcpy(&h, pay.data() + (size_t)d.off16 * 16 + step * r, 2);
+            if ((h & 0x7C00u) == 0x7C00u) return false;
+        }
+        total += 8 * step;
+    }
+    if (total + 64 >= 0x80000000ull) return false;
+    std::vector<uint8_t> out(total, 0);
+    uint64_t at = (8 * bpr * ntiles + 15) & ~15ull;
+    for (uint64_t t = 0; t < ntiles; ++t)
+        for (uint64_t c = 0; c < bpr; ++c) {
+            uint32_t head[2] = {(uint32_t)(at >> 4), 0u};
+            for (uint64_t r = 16 * t; r < std::min(rows, 16 * t + 16); ++r) {
+                DevBlock& d = db[r * bpr + c];
+                const uint32_t bytes = (uint32_t)d.cb_bytes + d.idx_bytes;
+                std::memcpy(out.data() + at, pay.data() + (size_t)d.off16 * 16, bytes);
+                d.off16 = (uint32_t)(at >> 4);
+                at += bytes;
+                if (d.fmt == OILHIP_SPARK_Q0) head[1] |= 1u << (r & 15);
+            }
+            std::memcpy(out.data() + 8 * (c * ntiles + t), head, 8);
+        }
+    pay.swap(out);
+    g.nf = nf;
+    g.sign_tiles = (uint32_t)ntiles;
+    g.waves = rows > cus * 32 ? 16u : 8u;            // (what gemv_any_multi's workspace rule goes by)
+    return true;
+}
+
 // Mixed-format tensors of full blocks: rewrite `pay` as the window streams the segmented GEMV reads (layout in
 // common.h, SegLayout) and point the descriptors at the blocks' new places.  Leaves everything as it is when the
 // tensor does not fit the scheme.
@@ -243,6 +293,7 @@ static void pack_window_streams(std::vector<uint8_t>& pay, std::vector<DevBlock>
             return;
         }
     }
+    if (pack_sign_tiles(pay, db, rows, cols, g, nf)) return;
     uint32_t widest = 0;
     for (uint32_t i = 0; i < nf; ++i) widest = std::max(widest, g.stride[i]);
     // Sixteen streams per CU for tensors of more than 32 rows per CU, else eight: a stream with fewer than two rows fills
@@ -412,7 +463,7 @@ static int upload(std::vector<uint8_t>& pay, std::vector<DevBlock>& db, std::vec
                             ((db[0].fmt == OILHIP_OIL4 && db[0].idx_bytes == 128) || (db[0].fmt == OILHIP_OIL8 && db[0].idx_bytes == 256)) &&
                             (nblocks == 1 || (db[1].off16 - db[0].off16) * 16u == db[0].idx_bytes);
     if (all_full && nblocks && !own_kernel) pack_window_streams(pay, db, rows, cols, w->seg);
-    if (w->seg.nstreams) regular = false;
+    if (w->seg.by_descriptor()) regular = false;
     // 64 spare bytes so vector loads that straddle the end of the last block stay in bounds
     w->alloc_bytes = pay.size() + 64;
     if ((e = hipMalloc(&w->d_payload, w->alloc_bytes)) != hipSuccess) return bail(e, "hipMalloc(payload)");

@@ -73,12 +73,16 @@ bool stream_capturing(hipStream_t s);
 // tags (per block: row of the tile and column block, in one byte (row << 6 | column) while a row has at most 64 blocks,
 // else two (row << 12 | column)); the blocks, 16-byte aligned, whole.  `blind16` = 16-byte pieces the fullest first
 // window fills.
+// Most tensors of SPARK_Q0 and OIL1 blocks alone (api.hip says which) are stored as `sign_tiles` tiles of 16 rows instead (gemv_signs.hip): at the start 8 bytes per (block of the row, tile), all tiles of the row's first block first: {byte offset / 16 in the buffer, a
+// bit per row that is SPARK_Q0 there}; then tile by tile, block of the row by block of the row, the up to 16 rows' blocks in the order of the rows, whole.
+// `nstreams` is 0 then.
 constexpr int kSegMaxFormats = 15;
 constexpr uint32_t kSegWindow = 4096;
 constexpr int kSegTileRows = 4;
 struct SegLayout {
-    uint32_t nf = 0, nstreams = 0, waves = 8, blind16 = 0, tag_bytes = 2;
+    uint32_t nf = 0, sign_tiles = 0, nstreams = 0, waves = 8, blind16 = 0, tag_bytes = 2;
     uint64_t stream_bytes = 0;
+    bool by_descriptor() const { return nstreams || sign_tiles; }      // blocks are found through their descriptors
     uint32_t fmt[kSegMaxFormats] = {}, cb_bytes[kSegMaxFormats] = {}, idx_bytes[kSegMaxFormats] = {}, stride[kSegMaxFormats] = {};
 };
 
@@ -167,6 +171,10 @@ constexpr uint32_t kGemvPackMaxCols = 32768;
 constexpr size_t kGemvPackBytes = (size_t)(kGemvPackMaxCols >> 8) * (192u + 32768u);
 // rows that mix formats, stored tile by tile and format by format
 int launch_gemv_seg(const oilhip_weights& w, const float* d_x, float* d_y, int M, hipStream_t s);
+// SPARK_Q0 and OIL1 blocks stored as sign tiles, kSignRows activation rows per launch
+constexpr int kSignRows = 4;
+bool signs_fastest(const oilhip_weights& w, int M);       // whether this kernel is faster than gemv_any_multi's
+int launch_gemv_signs(const oilhip_weights& w, const float* d_x, float* d_y, int M, hipStream_t s, const MultiInput& in = {}, uint32_t ldx = 0);
 // every format, a lane per run of 32 weights
 int launch_gemv_runs(const oilhip_weights& w, const float* d_x, float* d_y, int M, hipStream_t s);
 // prefill: x is bf16 bit patterns, or FP32 (rounded once to bf16) when x_is_f32; any tensor of full blocks (gemm_dense.hip) ...

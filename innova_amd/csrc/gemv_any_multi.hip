@@ -517,17 +517,20 @@ gemv_any_multi_kernel(const BodyArgs a) {
     float* keep = red + 2u * AREA;
     if (waves < (uint32_t)kMaxWaves)
         for (uint32_t o = waves * OUT + threadIdx.x; o < AREA; o += blockDim.x) { red[o] = 0.0f; red[AREA + o] = 0.0f; }
-    // outputs of a run: the eight wavefronts' sums of a token's three pieces
+    // outputs of a run: the eight wavefronts' sums of a token's three pieces (in 64 bits for the formats that gemv_signs serves one row of: its sums are of whole
+    // numbers, and several rows are to be no less accurate than one)
+    using Sum = std::conditional_t<S == kSpark || S == kPlanner, double, float>;
     auto finish = [&](uint32_t part, uint32_t run, const float* area) {
         for (uint32_t o = threadIdx.x; o < (uint32_t)(G * 16) * (uint32_t)a.M; o += blockDim.x) {
             const uint32_t l = o & 15u, g = (o >> 4) % G, token = (o >> 4) / G;
-            float s = 0.0f;
+            Sum sum = 0;
 #pragma unroll
             for (uint32_t d = 0; d < 3u; ++d) {
                 const uint32_t q = 3u * token + d;
                 const float* p = area + ((g * NT + (q >> 4)) * 4u + (q & 3u)) * 64u + ((q >> 2) & 3u) * 16u + l;
-                s += ((p[0] + p[OUT]) + (p[2u * OUT] + p[3u * OUT])) + ((p[4u * OUT] + p[5u * OUT]) + (p[6u * OUT] + p[7u * OUT]));
+                sum += (((Sum)p[0] + (Sum)p[OUT]) + ((Sum)p[2u * OUT] + (Sum)p[3u * OUT])) + (((Sum)p[4u * OUT] + (Sum)p[5u * OUT]) + ((Sum)p[6u * OUT] + (Sum)p[7u * OUT]));
             }
+            float s = (float)sum;
             float* k = keep + ((run % a.chunk) / G) * (uint32_t)(G * 16 * kPassTokens) + o;
             if (part) s += *k;
             if (part + 1u < a.parts) { *k = s; continue; }
@@ -631,7 +634,7 @@ int launch_tiles(int tiles, const BodyArgs& a, hipStream_t s) {
 }
 
 int source_of(const oilhip_weights& w) {
-    if (w.seg.nstreams && w.seg.nf > 0) {
+    if (w.seg.by_descriptor()) {
         uint32_t formats = 0;
         for (uint32_t i = 0; i < w.seg.nf; ++i) {
             if (w.seg.cb_bytes[i] != full_block_cb_bytes((int)w.seg.fmt[i]) || w.seg.cb_bytes[i] + w.seg.idx_bytes[i] != full_block_bytes((int)w.seg.fmt[i])) return -1;

@@ -1,6 +1,6 @@
-// gemv_seg.hip -- decode GEMV for tensors whose rows mix wire formats (the 1.50-bpw stacks
-// FormatPlanner::allocate produces, src/format_planner.cpp:133-315, and the SPARK mixes of
-// FormatRegistry::allocate_mix_blocks, src/format_registry.cpp:477-599): Qwen35Engine::gemm
+// gemv_seg.hip -- decode GEMV for tensors whose rows mix wire formats (the SPARK mixes of
+// FormatRegistry::allocate_mix_blocks, src/format_registry.cpp:477-599, and the stacks of FormatPlanner::allocate, src/format_planner.cpp:133-315,
+// that hold more than SPARK_Q0 and OIL1, whose mix gemv_signs.hip serves): Qwen35Engine::gemm
 // (src/adapters/tools/qwen35_engine.cpp:47-85) fused with dequantize_block_all (src/block_codec.cpp:576-720).
 //
 // Such a tensor is a few MB of small blocks (16 bytes for OIL1, 48 for SPARK_Q0), so the launch is bound by

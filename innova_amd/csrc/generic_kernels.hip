@@ -396,7 +396,7 @@ static int full_block_layout(const oilhip_weights& w) {
                            w.uniform_cb == full_block_cb_bytes(w.uniform_fmt) &&
                            w.uniform_cb + w.uniform_idx == w.uniform_stride;
     if (by_stride) return 1;
-    bool by_desc = w.seg.nstreams > 0;
+    bool by_desc = w.seg.by_descriptor();
     for (uint32_t i = 0; by_desc && i < w.seg.nf; ++i)
         by_desc = w.seg.cb_bytes[i] == full_block_cb_bytes((int)w.seg.fmt[i]) &&
                   w.seg.cb_bytes[i] + w.seg.idx_bytes[i] == full_block_bytes((int)w.seg.fmt[i]);

@@ -95,6 +95,7 @@ int gemv_rmsnorm(const oilhip_weights& w, const float* d_x, const float* d_normw
         const int rc = launch_gemv_oil4_rmsnorm(w, d_x, d_normw, d_y, s);  // the norm rides on the staging of x
         if (rc <= 0) return rc;
     }
+    if (M == 1 && w.seg.sign_tiles) return launch_gemv_signs(w, d_x, d_y, M, s, MultiInput{nullptr, d_normw});
     if (M == 1 && w.seg.nstreams) {
         const int rc = launch_gemv_seg_rmsnorm(w, d_x, d_normw, d_y, s);   // likewise for window-stream tensors
         if (rc <= 0) return rc;
@@ -108,6 +109,8 @@ int gemv_rmsnorm(const oilhip_weights& w, const float* d_x, const float* d_normw
                                               MultiInput{nullptr, d_normw, false, d_xn}, nullptr, nullptr, 0, d_pack);
         if (rc <= 0) return rc;
     }
+    if (signs_fastest(w, M) && apart)                                      // likewise, by each workgroup for itself
+        return launch_gemv_signs(w, d_x, d_y, M, s, MultiInput{nullptr, d_normw, false, d_xn});
     if (M >= 2 && !plain_oil4(w) && w.cols <= kPackNormMaxCols && apart) { // likewise for the other formats
         const int rc = launch_gemv_any_multi(w, d_x, d_y, M, s, d_pack, MultiInput{nullptr, d_normw, false, d_xn});
         if (rc <= 0) return rc;
@@ -131,6 +134,7 @@ int mlp_step(const oilhip_weights& gate_up, const oilhip_weights& down, const fl
         const int rc = launch_gemv_oil4_swiglu(down, h2, d_y, s);          // SwiGLU formed while the activations are staged
         if (rc <= 0) return rc;
     }
+    if (signs_fastest(down, M)) return launch_gemv_signs(down, h2, d_y, M, s, MultiInput{h2 + F, nullptr, true}, (uint32_t)(2 * F));
     if (M == 1 && down.seg.nstreams) {
         const int rc = launch_gemv_seg_swiglu(down, h2, d_y, s);
         if (rc <= 0) return rc;

@@ -1,0 +1,132 @@
+"""Tensors of SPARK_Q0 and OIL1 blocks stored as sign tiles (gemv_signs.hip): the edges of tiles of 16 rows, of the column blocks that a wavefront
+holds, of chunks of tiles and parts of K, and activations that the INT8 digits do not hold."""
+import numpy as np
+import pytest
+import torch
+
+import innova_amd as ia
+import oracle as O
+from gpu_util import gaussian_weights, rel_l2, to_orc_blocks
+from innova_amd import layers
+
+pytestmark = pytest.mark.gpu
+
+
+def tensor(rows, cols, share, seed):
+    """rows x cols with that share of SPARK_Q0 blocks, drawn from a pool of 512 blocks of each format."""
+    rng = np.random.default_rng(seed)
+    pool = [ia.block_codec.quantize_tensor(gaussian_weights(512 * 256, seed + f, outlier_every=13), ia.Format(f)) for f in (0, 1)]
+    n = rows * cols // 256
+    fm = (rng.random(n) < share).astype(np.uint8)
+    pick = rng.integers(0, 512, n)
+    desc = np.zeros(n, ia._lib.BLOCK_DTYPE)
+    for name in ("cb_off", "idx_off", "cb_bytes", "idx_bytes", "nw", "fmt"):
+        desc[name] = np.where(fm == 0, pool[0][1][name][pick], pool[1][1][name][pick])
+    spark = fm == 1
+    desc["cb_off"][spark] += pool[0][0].size
+    desc["idx_off"][spark] += pool[0][0].size
+    return ia.DeviceWeights.from_blocks(np.concatenate([pool[0][0], pool[1][0]]), desc, rows, cols)
+
+
+def reference(dw, x):
+    return x.double() @ dw.dequant().view(dw.rows, dw.cols).double().t().contiguous()
+
+
+# A run's sum is rounded to FP32 once, then meets a scale, its neighbour, up to four blocks, four lane groups and sixteen wavefronts (in four
+# sums), and a part of K each: at most 4 + blocks / 16 + 2 + 6 + parts roundings of partial sums that are no larger than the whole's norm.
+@pytest.mark.parametrize("share", [0.5, 1.0])
+@pytest.mark.parametrize("rows,cols", [(1, 256), (15, 512), (16, 4096), (17, 4352), (33, 8192), (40, 8448), (40, 12288), (2600, 12544), (4111, 16640),
+                                       (4096, 768), (66000, 256), (33500, 512), (50000, 4608)])
+@pytest.mark.parametrize("M", [1, 2, 3, 4])
+def test_sign_tiles(rows, cols, share, M):
+    if rows * cols > 50e6 and (share != 0.5 or M in (2, 3)):
+        pytest.skip("one mix and two batches of the largest tensors")
+    with tensor(rows, cols, share, rows + cols) as dw:
+        x = torch.randn(M, cols, generator=torch.Generator().manual_seed(M)).cuda()
+        got, want = dw.gemv(x), reference(dw, x)
+        assert float((got.double() - want).norm() / want.norm()) <= (12 + cols / 4096 + cols / 16384) * 2.0 ** -24
+        assert torch.equal(got, dw.gemv(x))
+
+
+@pytest.mark.parametrize("M", [1, 2, 4, 7])
+def test_captured_without_workspace(M):
+    """More rows than a pass, whichever kernel serves them eagerly, and rows past the part of K that a pass covers."""
+    with tensor(100, 4608, 0.5, 3) as dw:
+        x, y = torch.randn(M, 4608, device="cuda"), torch.empty(M, 100, device="cuda")
+        side, g, L = torch.cuda.Stream(), torch.cuda.CUDAGraph(), ia._lib.lib()
+        want = reference(dw, x)
+        torch.cuda.synchronize()
+        with torch.cuda.graph(g, stream=side):
+            ia._lib.check(L.oilhip_gemv_f32(dw.handle, x.data_ptr(), y.data_ptr(), M, ia._lib.current_stream()))
+        for _ in range(3):
+            y.fill_(float("nan"))
+            g.replay()
+            torch.cuda.synchronize()
+            assert rel_l2(y.cpu().numpy(), want.cpu().numpy()) <= 1e-6
+
+
+# infinities, NaN, a block of zeros, magnitudes whose power of two has no inverse among the floats, and the largest and smallest mantissas of a digit
+@pytest.mark.parametrize("M", [1, 2, 3, 4])
+def test_unusual_activations(M):
+    rows, cols, inf = 70, 1280, float("inf")
+    rng = np.random.default_rng(M)
+    with tensor(rows, cols, 0.5, 8) as dw:
+        W = dw.dequant().view(rows, cols).cpu().numpy().astype(np.float64)
+        for case in range(7):
+            x = rng.standard_normal((M, cols)).astype(np.float32)
+            m = M - 1
+            if case == 0: x[m, 5] = inf
+            if case == 1: x[m, [300, 1279]] = [inf, -inf]
+            if case == 2: x[m, 700] = float("nan")
+            if case == 3: x[:, 256:512] = 0.0
+            if case == 4: x[:, 512:768] *= np.float32(1e-36)
+            if case == 5: x *= np.float32(1e-41)
+            if case == 6: x[m, 256:260] = np.array([0x407F7F7F, 0xC07F7F80, 0x407FFFFF, 0xC0000001], np.uint32).view(np.float32)
+            got = dw.gemv(torch.from_numpy(x).cuda()).cpu().numpy()
+            with np.errstate(invalid="ignore"):
+                want = np.stack([(W * x[i].astype(np.float64)).sum(1) for i in range(M)])
+            assert np.array_equal(np.isnan(got), np.isnan(want)), case
+            assert np.array_equal(np.where(np.isinf(got), np.sign(got), 0), np.where(np.isinf(want), np.sign(want), 0)), case
+            ok = np.isfinite(want)
+            # (subnormal sums carry 2^-150 per addition)
+            assert rel_l2(np.where(ok, got, 0), np.where(ok, want, 0)) <= (1e-6 if case != 5 else 2e-3), case
+
+
+def test_scales_that_are_not_finite_keep_window_streams():
+    """+-inf times activations of both signs is NaN in FP32 sums: signs first would make it an infinity."""
+    payload, blocks = ia.block_codec.quantize_tensor(gaussian_weights(64 * 512, 5), ia.Format.SPARK_Q0)
+    payload = payload.copy()
+    payload[int(blocks["idx_off"][7]):][:2] = [0x00, 0x7C]
+    x = torch.randn(1, 512, generator=torch.Generator().manual_seed(1)).cuda()
+    with ia.DeviceWeights.from_blocks(payload, blocks, 64, 512) as dw:
+        got, plain = dw.gemv(x).cpu().numpy(), dw.gemv(x, general=True).cpu().numpy()
+        assert np.array_equal(np.isnan(got), np.isnan(plain)) and np.isnan(got).sum() == 1
+
+
+# one to four rows behind the norm and SwiGLU; blocks per wavefront 1 to 4, parts of K, activations at odd addresses, and the normalised rows
+@pytest.mark.parametrize("M,D,F,shift", [(1, 512, 4352, 1), (1, 4352, 8448, 0), (1, 8448, 12544, 0), (2, 1024, 4352, 3), (3, 512, 4096, 0), (4, 4096, 768, 1), (4, 4352, 512, 0)])
+def test_with_norm_and_swiglu(M, D, F, shift):
+    rng = np.random.default_rng(D + F + M)
+    gu, down = tensor(2 * F, D, 0.5, D), tensor(D, F, 0.5, F)
+    x = torch.zeros(shift + M * D, device="cuda")[shift:].view(M, D)
+    x.copy_(torch.from_numpy((rng.standard_normal((M, D)) * 2).astype(np.float32)))
+    nw = torch.from_numpy((rng.standard_normal(D) * 0.2).astype(np.float32)).cuda()
+    xn = x.double() / (x.double().pow(2).mean(1, keepdim=True) + 1e-6).sqrt() * (1.0 + nw.double())
+    want = reference(gu, xn)
+    got, out, L = layers.gemv_rmsnorm(gu, x, nw), torch.full((M, D), float("nan"), device="cuda"), ia._lib.lib()
+    assert rel_l2(got.cpu().numpy(), want.cpu().numpy()) <= 1e-6
+    if M > 1:
+        again = torch.empty_like(got)
+        ia._lib.check(L.oilhip_gemv_rmsnorm_f32(gu.handle, x.data_ptr(), nw.data_ptr(), again.data_ptr(), M, out.data_ptr(), ia._lib.current_stream()))
+        assert torch.equal(got, again) and rel_l2(out.cpu().numpy(), xn.cpu().numpy()) <= 3e-7
+    g, u = want[:, :F], want[:, F:]
+    want = reference(down, g / (1.0 + (-g).exp()) * u)
+    assert rel_l2(layers.mlp_step(gu, down, x, norm_w=nw).cpu().numpy(), want.cpu().numpy()) <= 3e-6
+    # a sum of squares past the largest float: the norm makes every x zero, an infinite one NaN
+    if M > 1:
+        x[0] = 3e38
+        x[1, 3] = float("inf")
+        y = layers.gemv_rmsnorm(gu, x, nw)
+        assert bool((y[0] == 0).all()) and bool(y[1].isnan().all()) and bool(torch.isfinite(y[2:]).all())
+    gu.close()
+    down.close()
