@@ -691,7 +691,8 @@ static int prefill(const oilhip_weights* w, const void* d_x, bool x_is_f32, floa
     const bool aligned = (reinterpret_cast<uintptr_t>(d_x) & 15u) == 0u;
     if (plain_oil4(*w) && (aligned || (uint64_t)M * w->cols * 2u >= 0x80000000ull || w->cols * 512u >= 0x80000000ull))
         return launch_gemm_oil4_frag(*w, d_x, x_is_f32, d_y, M, s);
-    const int rc = launch_gemm_any(*w, d_x, x_is_f32, d_y, M, s);
+    int rc = launch_gemm_signs(*w, d_x, x_is_f32, d_y, M, s);
+    if (rc == 1) rc = launch_gemm_any(*w, d_x, x_is_f32, d_y, M, s);
     if (rc == 1) return fail(OILHIP_E_ARG, "bf16 prefill GEMM needs full blocks with the channel sizes the quantizer writes");
     return rc;
 }

@@ -178,7 +178,10 @@ int launch_gemv_signs(const oilhip_weights& w, const float* d_x, float* d_y, int
 // every format, a lane per run of 32 weights
 int launch_gemv_runs(const oilhip_weights& w, const float* d_x, float* d_y, int M, hipStream_t s);
 // prefill: x is bf16 bit patterns, or FP32 (rounded once to bf16) when x_is_f32; any tensor of full blocks (gemm_dense.hip) ...
+double dense_estimate_us(uint32_t M, uint32_t N, uint32_t K);
 int launch_gemm_any(const oilhip_weights& w, const void* d_x, bool x_is_f32, float* d_y, int M, hipStream_t s);
+// ... sign tiles, decoded inside the kernel (gemm_signs.hip) ...
+int launch_gemm_signs(const oilhip_weights& w, const void* d_x, bool x_is_f32, float* d_y, int M, hipStream_t s);
 // ... and plain uniform OIL4, decoded inside the kernel (gemm_oil4_frag.hip)
 int launch_gemm_oil4_frag(const oilhip_weights& w, const void* d_x, bool x_is_f32, float* d_y, int M, hipStream_t s);
 }  // namespace oilhip

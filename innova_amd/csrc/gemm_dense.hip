@@ -199,20 +199,26 @@ int launch_tiles(const DenseArgs& a, hipStream_t s) {
 // than the best of f = 1, 2 and 1, 2, 4, 8 parts on average, 3.5 % at most; over 20 others that the numbers were not taken from (35 to
 // 3000 tokens) 1.4 %, 12 % at most.  719 x 3840, 81 tokens: f = 1 in 1 / 4 parts 23.5 / 17.1 us,
 // f = 2 in 1 / 4 39.1 / 24.6; 4096 x 11008, 700 tokens: f = 2 in 1 / 2 / 4 parts 114 / 111 / 134 us.
-struct DensePlan { uint32_t f, parts; };
+struct DensePlan { uint32_t f, parts; double clocks; };
 static DensePlan dense_plan(uint32_t M, uint32_t N, uint32_t K) {
     const double cus = (double)device_cu_count();
-    DensePlan best{2u, 1u};
-    double least = 1e30;
+    DensePlan best{2u, 1u, 1e30};
     for (uint32_t f = 1; f <= 2u; ++f)
         for (uint32_t parts = 1; parts <= 8u && parts * 4u <= K / 64u; parts *= 2u) {
             const uint32_t t = 64u * f;
             const double wgs = (double)((M + t - 1u) / t) * (double)((N + t - 1u) / t) * parts, each = std::max(wgs / cus, 1.0);
             const double stages = (double)K * f / 64.0 / parts * (f == 1u ? 480.0 : 540.0);
             const double clocks = (wgs <= cus ? 1.0 : each + 0.2) * stages + (parts > 1u ? (2500.0 * each + 1000.0 * parts) * f * f : 0.0);
-            if (clocks < least) { least = clocks; best = {f, parts}; }
+            if (clocks < best.clocks) best = {f, parts, clocks};
         }
     return best;
+}
+
+// The whole call, for the choice between this product and the one that decodes its weights itself: the launch that writes the operands at 5.3 TB/s behind
+// 5 us, the product at 1.9 GHz.  Planner's mix, estimate and time: 5000 x 2816, 437 tokens 36 / 33.8 us; 900 x 1024, 50 tokens 9.8 / 9.3; 2000 x 4096, 200 tokens
+// 18.8 / 19.9; 4096 x 11008, 64 tokens 36 / 37; 11008 x 4096, 512 / 2048 tokens 78 / 73, 224 / 200.
+double dense_estimate_us(uint32_t M, uint32_t N, uint32_t K) {
+    return dense_plan(M, N, K).clocks / 1900.0 + 5.0 + 2.0 * K * ((double)N + M) / 5.3e6;
 }
 
 // Prefill over a tensor of any format (full 256-weight blocks): slabs of weight rows are decoded to bf16 in a scratch

@@ -130,3 +130,15 @@ def test_with_norm_and_swiglu(M, D, F, shift):
         assert bool((y[0] == 0).all()) and bool(y[1].isnan().all()) and bool(torch.isfinite(y[2:]).all())
     gu.close()
     down.close()
+
+
+# prefill without a launch that decodes: K whole, in 2, 4 and 8 parts (uneven ones among them), and wavefronts of two row blocks; rows and tokens that end
+# inside a tile.  Each operand is rounded to bf16 once, the weights here only: 2^-9 at most, a third of it in the mean.
+@pytest.mark.parametrize("rows,cols,M", [(5001, 2816, 437), (11008, 4096, 40), (2600, 12544, 100), (4099, 11008, 64), (2600, 11008, 33), (11008, 4096, 2048)])
+def test_prefill(rows, cols, M):
+    with tensor(rows, cols, 0.5, rows + M) as dw:
+        x = torch.randn(M, cols, generator=torch.Generator().manual_seed(M)).cuda()
+        got = dw.gemm_f32(x)
+        want = reference(dw, x.to(torch.bfloat16))
+        assert float((got.double() - want).norm() / want.norm()) <= 2e-3
+        assert torch.equal(got, dw.gemm_bf16(x.to(torch.bfloat16))) and torch.equal(got, dw.gemm_f32(x))
