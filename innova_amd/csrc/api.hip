@@ -159,7 +159,7 @@ int gemv_f32(const oilhip_weights& w, const float* d_x, float* d_y, int M, hipSt
         if (rc == 1 && M > 2 && M <= 4) rc = launch_gemv_oil4(w, d_x, d_y, M, s);
         if (rc <= 0) return rc;
     }
-    if (signs_fastest(w, M)) return launch_gemv_signs(w, d_x, d_y, M, s);
+    if (signs_fastest(w, M) && (M == 1 || !rows_overlap(w, d_x, d_y, M))) return launch_gemv_signs(w, d_x, d_y, M, s);
     if (M >= 2) {
         const int rc = launch_gemv_any_multi(w, d_x, d_y, M, s, d_pack);
         if (rc <= 0) return rc;
@@ -297,7 +297,7 @@ static void pack_window_streams(std::vector<uint8_t>& pay, std::vector<DevBlock>
     uint32_t widest = 0;
     for (uint32_t i = 0; i < nf; ++i) widest = std::max(widest, g.stride[i]);
     // Sixteen streams per CU for tensors of more than 32 rows per CU, else eight: a stream with fewer than two rows fills
-    // too little of the decoding steps (4096 x 4096 of the planner's mix: 5.9 us with eight, 6.7 with sixteen).  With more, one row, eight -> sixteen:
+    // too little of the decoding steps (4096 x 4096 of the planner's mix, which sign tiles serve now: 5.9 us with eight, 6.7 with sixteen).  With more, one row, eight -> sixteen:
     // planner's mix 9000 x 2048 7.2 -> 6.5 us, 11008 x 4096 9.3 -> 9.0, 22016 x 4096 13.6 -> 13.6, 32768 x 4096 18.6 -> 16.5; SPARK_Q0, OIL2,
     // registry's mix 11008 x 4096 11.7 -> 11.2, 13.3 -> 12.5, 15.7 -> 13.4.  Of the stored floats' blocks (512 bytes and more) the smaller
     // windows would hold three at most.

@@ -37,6 +37,7 @@ constexpr int TR = kSegTileRows;           // accumulators per lane and activati
 typedef _Float16 h2v __attribute__((ext_vector_type(2)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
+// (Figures of the planner's mix and of SPARK_Q0 alone in this file are from before gemv_signs.hip served them.)
 // Sign table of one activation row: for every four columns all sixteen sums +-x0 +-x1 +-x2 +-x3, entry n the one in which bit j of n makes x[j]
 // positive.  A SPARK_Q0 run is then eight reads instead of 32 products of unpacked signs: 30 vector instructions fewer per step, and
 // about 10 clocks of LDS for each read (16 for 16 bytes per lane of plain activations).  Where another format of the tensor works on few instructions per weight

@@ -109,7 +109,7 @@ int gemv_rmsnorm(const oilhip_weights& w, const float* d_x, const float* d_normw
                                               MultiInput{nullptr, d_normw, false, d_xn}, nullptr, nullptr, 0, d_pack);
         if (rc <= 0) return rc;
     }
-    if (signs_fastest(w, M) && apart)                                      // likewise, by each workgroup for itself
+    if (signs_fastest(w, M) && apart && !rows_overlap(w, d_x, d_y, M))     // likewise, by each workgroup for itself
         return launch_gemv_signs(w, d_x, d_y, M, s, MultiInput{nullptr, d_normw, false, d_xn});
     if (M >= 2 && !plain_oil4(w) && w.cols <= kPackNormMaxCols && apart) { // likewise for the other formats
         const int rc = launch_gemv_any_multi(w, d_x, d_y, M, s, d_pack, MultiInput{nullptr, d_normw, false, d_xn});

@@ -65,6 +65,14 @@ def test_captured_without_workspace(M):
             assert rel_l2(y.cpu().numpy(), want.cpu().numpy()) <= 1e-6
 
 
+def test_outputs_over_the_activations():
+    """Several rows in place: a launch of its own packs the activations before any output is stored."""
+    with tensor(512, 512, 0.5, 4) as dw:
+        x = torch.randn(3, 512, generator=torch.Generator().manual_seed(1)).cuda()
+        want = reference(dw, x)
+        assert rel_l2(dw.gemv(x, out=x).cpu().numpy(), want.cpu().numpy()) <= 1e-6
+
+
 # infinities, NaN, a block of zeros, magnitudes whose power of two has no inverse among the floats, and the largest and smallest mantissas of a digit
 @pytest.mark.parametrize("M", [1, 2, 3, 4])
 def test_unusual_activations(M):
