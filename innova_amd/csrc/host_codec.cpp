@@ -320,7 +320,7 @@ bool encode_block(int fmt, std::span<const float> w, uint8_t* idx, size_t& il, u
 // that are bound by their instructions are written out: sums of runs whose floats are transposed eight by eight so that a lane is a chain, codes by a
 // search of four steps over thresholds that are in the weights' scale (no division per weight), halves and signs a register at a time, and
 // the next sixteen blocks fetched while these are encoded.  One thread, ns per weight without the output pages' first touch (Xeon 2.7 GHz), bit by bit -> plain
-// forms -> AVX-512: OIL4 54 -> 2.4 -> 0.8 to 1.0, OIL8 53 -> 1.5 -> 0.8 to 1.2, SPARK_Q0 11.9 -> 2.8 -> 0.4 to 0.6; whole calls of 4 M weights, ms:
+// forms -> AVX-512, weights in cache: OIL4 54 -> 1.6 to 2.3 -> 0.6 to 0.9, OIL8 53 -> 0.8 to 1.2 -> 0.6 to 0.9, SPARK_Q0 11.9 -> 1.7 to 2.5 -> 0.3 to 0.5; whole calls of 4 M weights, ms:
 // OIL4_GRP 18.1 -> 7.9, OIL8_GRP 12.9 -> 6.4, SPARK_Q0 and OIL1 mixed 10.7 -> 3.0, OIL2 7.6 -> 4.0.  16 M weights of OIL4 on eight threads 8.5 -> 5.0 ms, of
 // which the first touch of the output pages is a third.
 #define OIL_INLINE inline __attribute__((always_inline))
@@ -453,6 +453,19 @@ bool codes_avx512(const float* w, float scale, const std::array<float, N>& thres
     return true;
 }
 
+// level_code<8> of 256 weights over their scale, straight into the block: 254 bytes, the last of every 128 left out
+inline void codes8_avx512(const float* w, float scale, uint8_t* out) {
+    const __m512 sv = _mm512_set1_ps(scale);
+    for (int i = 0; i < 256; i += 16) {
+        const __m512 c = _mm512_max_ps(_mm512_min_ps(_mm512_div_ps(_mm512_loadu_ps(w + i), sv), _mm512_set1_ps(8.0f)), _mm512_set1_ps(-8.0f));
+        const __m512 r = _mm512_mul_ps(_mm512_mul_ps(_mm512_add_ps(c, _mm512_set1_ps(8.0f)), _mm512_set1_ps(255.0f)), _mm512_set1_ps(0.0625f));
+        const __m512i k = _mm512_cvttps_epi32(r);
+        const __mmask16 half = _mm512_cmp_ps_mask(_mm512_sub_ps(r, _mm512_cvtepi32_ps(k)), _mm512_set1_ps(0.5f), _CMP_GE_OQ);
+        const __m128i b = _mm512_cvtepi32_epi8(_mm512_mask_add_epi32(k, half, k, _mm512_set1_epi32(1)));
+        _mm_mask_storeu_epi8(out + i - i / 128, i % 128 == 112 ? 0x7FFF : 0xFFFF, b);
+    }
+}
+
 // 64 codes, one per byte -> 8 BITS bytes, first code in the low bits
 template <int BITS>
 OIL_INLINE auto pack64_avx512(__m512i c) {
@@ -579,6 +592,9 @@ OIL_INLINE void full_lattice(const float* w, double sum_sq, uint8_t* out) {
     const float scale = float(std::sqrt(sum_sq / 256.0));
     put16(out, to_half(scale));
     alignas(64) uint8_t code[256], dense[256];
+    if constexpr (WIDE && BITS == 8) {
+        if (scale > 1e-12f) { codes8_avx512(w, scale, out + 2); return; }
+    }
     if (scale <= 1e-12f) {
         const uint32_t q = level_code<BITS>(0.0f);
         for (int i = 0; i < 256; ++i) code[i] = uint8_t(q);
@@ -705,14 +721,20 @@ template <bool WIDE>
 OIL_INLINE void encode_range(const uint8_t* fmts, const float* w, uint64_t numel, const oilhip_block_t* blocks, uint8_t* payload,
                              uint32_t b0, uint32_t b1) {
     constexpr uint32_t SIDE = WIDE ? 16 : 8;                           // blocks whose sums run side by side
-    for (uint32_t b = b0; b < b1; b += SIDE) {
-        const uint32_t nb = std::min(SIDE, b1 - b);
-        const bool full = uint64_t(b + nb) * 256 <= numel;
+    auto encode_plain = [&](uint32_t b) {                              // one channel is empty in every format: both may point at the block's place
+        uint8_t* out = payload + blocks[b].cb_off;
+        size_t il = 0, cl = 0;
+        encode_block(fmts[b], {w + uint64_t(b) * 256, size_t(std::min<uint64_t>(256, numel - uint64_t(b) * 256))}, out, il, out, cl);
+    };
+    const uint32_t whole = uint32_t(std::min<uint64_t>(b1, numel / 256));
+    if (whole < b1) encode_plain(whole);                               // the tensor's last block, shorter than the others
+    for (uint32_t b = b0; b < whole; b += SIDE) {
+        const uint32_t nb = std::min(SIDE, whole - b);
         auto scaled_by_rms = [](uint8_t f) { return f == OILHIP_OIL2 || f == OILHIP_OIL4 || f == OILHIP_OIL8 || f == OILHIP_OIL1_GRP; };
         double s[SIDE] = {};
         bool scaled = false;
         for (uint32_t j = 0; j < nb; ++j) scaled |= scaled_by_rms(fmts[b + j]);
-        if (full && scaled) {
+        if (scaled) {
             if (nb < SIDE) for (uint32_t j = 0; j < nb; ++j) square_sums<1, 256>(w + uint64_t(b + j) * 256, s + j);
             else if constexpr (WIDE) run_sums_avx512<SIDE / 8, 256>(w + uint64_t(b) * 256, s);
             else square_sums<SIDE, 256>(w + uint64_t(b) * 256, s);
@@ -722,7 +744,7 @@ OIL_INLINE void encode_range(const uint8_t* fmts, const float* w, uint64_t numel
         if constexpr (WIDE) {
             const float* block[SIDE + 3];
             uint32_t n = 0;
-            for (uint32_t j = 0; j < nb && full; ++j)
+            for (uint32_t j = 0; j < nb; ++j)
                 if (fmts[b + j] == OILHIP_OIL2_GRP || fmts[b + j] == OILHIP_OIL4_GRP) block[n++] = w + uint64_t(b + j) * 256;
             for (uint32_t j = n; n && j < (n + 3) / 4 * 4; ++j) block[j] = block[n - 1];
             for (uint32_t j = 0; j < n; j += 4) {
@@ -739,7 +761,7 @@ OIL_INLINE void encode_range(const uint8_t* fmts, const float* w, uint64_t numel
             if (WIDE && at + (SIDE + 1) * 256 <= numel) for (int i = 0; i < 16; ++i) __builtin_prefetch(w + at + SIDE * 256 + 16 * i);
             const int fmt = fmts[b + j];
             if constexpr (WIDE) {
-                if (full && (fmt == OILHIP_OIL2_GRP || fmt == OILHIP_OIL4_GRP)) {
+                if (fmt == OILHIP_OIL2_GRP || fmt == OILHIP_OIL4_GRP) {
                     const uint32_t g = grouped++;
                     if (largest_bits(w + at) <= kLargestBits) {
                         if (fmt == OILHIP_OIL2_GRP) grouped_avx512<2>(w + at, zp[g], sc[g], out);
@@ -748,9 +770,7 @@ OIL_INLINE void encode_range(const uint8_t* fmts, const float* w, uint64_t numel
                     }
                 }
             }
-            if (full && encode_full<WIDE>(fmt, w + at, s[j], out)) continue;
-            size_t il = 0, cl = 0;                                     // one channel is empty in every format: both may point at `out`
-            encode_block(fmt, {w + at, size_t(std::min<uint64_t>(256, numel - at))}, out, il, out, cl);
+            if (!encode_full<WIDE>(fmt, w + at, s[j], out)) encode_plain(b + j);
         }
     }
 }
