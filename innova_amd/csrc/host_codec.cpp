@@ -462,7 +462,8 @@ inline void codes8_avx512(const float* w, float scale, uint8_t* out) {
         const __m512i k = _mm512_cvttps_epi32(r);
         const __mmask16 half = _mm512_cmp_ps_mask(_mm512_sub_ps(r, _mm512_cvtepi32_ps(k)), _mm512_set1_ps(0.5f), _CMP_GE_OQ);
         const __m128i b = _mm512_cvtepi32_epi8(_mm512_mask_add_epi32(k, half, k, _mm512_set1_epi32(1)));
-        _mm_mask_storeu_epi8(out + i - i / 128, i % 128 == 112 ? 0x7FFF : 0xFFFF, b);
+        if (i < 240) _mm_storeu_si128(reinterpret_cast<__m128i*>(out + i - i / 128), b);       // (code 127 lies under the next run's first)
+        else _mm_mask_storeu_epi8(out + 239, 0x7FFF, b);
     }
 }
 
@@ -488,8 +489,13 @@ void pack_lattice_avx512(const uint8_t* code, uint8_t* out) {
     }
     for (int i = 0; i < 4; ++i) {
         const auto b = pack64_avx512<BITS>(_mm512_load_si512(dense + 64 * i));
-        if constexpr (BITS == 4) _mm256_mask_storeu_epi8(out + 32 * i, i < 3 ? 0xFFFFFFFFu : 0x3FFFFFFFu, b);
-        else _mm_mask_storeu_epi8(out + 16 * i, i < 3 ? 0xFFFFu : 0x3FFFu, b);
+        if constexpr (BITS == 4) {
+            if (i < 3) _mm256_storeu_si256(reinterpret_cast<__m256i*>(out + 32 * i), b);
+            else _mm256_mask_storeu_epi8(out + 96, 0x3FFFFFFFu, b);
+        } else {
+            if (i < 3) _mm_storeu_si128(reinterpret_cast<__m128i*>(out + 16 * i), b);
+            else _mm_mask_storeu_epi8(out + 48, 0x3FFFu, b);
+        }
     }
 }
 
