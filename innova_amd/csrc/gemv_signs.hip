@@ -5,9 +5,11 @@
 // Both formats say the same thing: a run of 32 weights is an FP16 number times 32 signs, and an OIL1 run has the sign + everywhere.  So a
 // tile of 16 rows by one block is four INT8 matrix instructions (16x16x64) whatever its blocks are.  One operand are the signs as bytes of
 // +-64, two vector instructions per four weights (a shift, and one that masks and sets the magnitude).  The other are the activations as
-// four signed byte digits relative to the largest magnitude of their block (31 bits).  The digits of the run pair 2 q, 2 q + 1 are rows
+// four signed byte digits relative to the largest magnitude of their run (31 bits).  (Not of their block: where an outlier meets a scale of 0 or a small one,
+// the other runs would be left with few bits.  16 blocks, x N(0, 1), an outlier of 1e6 in each over a run of scale 0: 1.4e-4 with one power of two per
+// block, 0.8e-7 with one per run.)  The digits of the run pair 2 q, 2 q + 1 are rows
 // 4 q .. 4 q + 3 and are zero in the lane groups of other runs, so a lane gets the four digit sums of the two runs whose signs and scales it
-// holds: they become one float, exact but for its rounding, meet the two scales in FP32, and no lane ever holds another row's sum.
+// holds: they become one float, exact but for its rounding, meet the two scales in FP32 (a scale times its run's power of two is exact), and no lane ever holds another row's sum.
 //
 // A wavefront keeps the digits of its one to three column blocks in registers and walks down the workgroup's tiles; every workgroup packs
 // the activations itself (each wavefront its own blocks, without a barrier), so there is no second launch and no scratch.  The wavefronts'
@@ -16,16 +18,19 @@
 // What bounds it: vector issue (about 60 instructions per tile of one block, 30 of them making sign bytes; as many to pack a block of activations) and, below
 // ten tiles a workgroup, latency: the launch, the tiles' places, the blocks, each behind the other.  Before (window streams, gemv_seg.hip; several rows
 // gemv_any_multi.hip) -> now, us, planner's mix, launches of a graph over a ring of tensors in memory:
-//   one row   649 x 768 4.0 -> 2.6   4096 x 4096 5.4 -> 4.0   12288 x 4096 7.8 -> 5.1   22016 x 4096 12.0 -> 6.8   60000 x 4096 23.4 -> 12.1
-//             4096 x 11008 8.0 -> 6.2   SPARK_Q0 alone 11008 x 4096 10.6 -> 5.1
-//   two       4096 x 4096 6.7 -> 4.7   22016 x 4096 14.6 -> 8.2   4096 x 11008 15.2 -> 9.7
-//   three     1000 x 1280 5.6 -> 3.8   11008 x 4096 12.1 -> 8.1;   four   11008 x 4096 12.2 -> 9.0
+//   one row   649 x 768 4.0 -> 2.5   4096 x 4096 5.4 -> 3.9   12288 x 4096 7.8 -> 5.3   22016 x 4096 12.0 -> 7.1   60000 x 4096 23.4 -> 13.5
+//             4096 x 11008 8.0 -> 6.2   SPARK_Q0 alone 11008 x 4096 10.6 -> 5.3
+//   two       4096 x 4096 6.6 -> 4.7   22016 x 4096 14.7 -> 8.8   4096 x 11008 15.2 -> 10.0
+//   three     1000 x 1280 5.6 -> 3.8   11008 x 4096 12.1 -> 8.4;   four   11008 x 4096 12.2 -> 9.3
+// (One power of two per run instead of per block is an instruction more per tile of one block and row: long launches 1 to 4 % slower, short ones 1 to 3 % faster,
+// with eight instructions fewer in the packing.)
 // Error against 64 bits (2-norm, 4096 columns, one row) 1.1e-7 -> 0.8e-7.
 // Level or slower: an operand of 0 and 1 with the activations' sums as the matrix instruction's addend (24 registers per block instead of 16); sums over
 // the lane groups in front of LDS instead of behind it (22016 x 4096 8.5 us against 6.9, with the loop's waits then counting no loads).
 //
-// Blocks whose activations are not finite, or too small for the power of two that undoes the digits, add up their signed activations in FP32.
+// Runs whose activations are not finite, or too small for the power of two that undoes the digits, add up their signed activations in FP32.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 #include "oil4_lds.h"
@@ -79,14 +84,14 @@ gemv_signs_kernel(const SignArgs a) {
     float* sums = reinterpret_cast<float*>(smem) + waves * ((uint32_t)(CB * M) * 256u + 16u);      // [tile of the chunk][wavefront][row of y][lane]
     float* ssq_part = sums + (LOOP ? CHUNK : t_end - t_begin) * waves * (uint32_t)(64 * M);   // kNorm: [wavefront][row of y], then 1 where x is not finite
     const auto wrs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(a.W), (short)0, (int)a.wbytes, 0x00020000);
-    const uint2* heads = reinterpret_cast<const uint2*>(a.W);              // [block of the row][tile]: {place / 16, mask of SPARK_Q0 rows}
+    const uint32_t* heads = reinterpret_cast<const uint32_t*>(a.W);        // [block of the row][tile]: {place / 16, mask of SPARK_Q0 rows}
     const uint32_t row_bit = 1u << li, rows_before = row_bit - 1u, at_mean = 16u * li + 4u * q, at_sign = 16u * li + 12u * q;
     const uint32_t col = 32u * (lane >> 3) + (lane & 7u);                  // a lane packs columns col + 8 j of a block
     uint32_t tops = 0x80808080u, size = 0x40404040u;                       // in registers: one instruction masks and sets the magnitude
     asm volatile("" : "+s"(tops), "+v"(size));
 
-    // what a wavefront reads of the activations and the tiles' places for a chunk of tiles and a part of K
-    struct Input { uint2 head[CB]; float v[CB][M][4], u[CB][XF == kSwiglu ? M : 1][4]; };
+    // what a wavefront reads of the activations and the tiles' places for a chunk of tiles and a part of K (place of tile i in lane i, its mask in lane 16 + i)
+    struct Input { uint32_t head[CB]; float v[CB][M][4], u[CB][XF == kSwiglu ? M : 1][4]; };
     auto tiles_of = [&](uint32_t chunk) { return !LOOP || t_end - chunk < CHUNK ? t_end - chunk : CHUNK; };
     auto block_of = [&](uint32_t part, int s, bool& live) {
         const uint32_t first = LOOP ? part * a.per : 0u, last = LOOP && first + a.per < a.bpr ? first + a.per : a.bpr, b = first + (uint32_t)s * waves + wave;
@@ -97,7 +102,7 @@ gemv_signs_kernel(const SignArgs a) {
         const uint32_t n = tiles_of(chunk);
         bool live;
 #pragma unroll
-        for (int s = 0; s < CB; ++s) in.head[s] = heads[block_of(part, s, live) * a.ntiles + chunk + (lane < n ? lane : n - 1u)];
+        for (int s = 0; s < CB; ++s) in.head[s] = heads[2u * (block_of(part, s, live) * a.ntiles + chunk + (li < n ? li : n - 1u)) + (q & 1u)];
 #pragma unroll
         for (int s = 0; s < CB; ++s) {
             const uint32_t b = 256u * block_of(part, s, live);
@@ -113,9 +118,9 @@ gemv_signs_kernel(const SignArgs a) {
     };
 
     i32x4 dig[CB][M][4];
-    float undo[CB][M], ssq[M];
+    float undo[CB][M], ssq[M];                                             // undo: of the run that this lane packs, lane / 8; positive where it is held as floats
     uint32_t endless = 0;                                                  // kNorm, several rows: bit m: an x that is not finite
-    uint32_t slow = 0;                                                     // bit s * M + m: that block adds up in FP32
+    uint32_t slow = 0;                                                     // bit s * M + m: runs of that block add up in FP32
 #pragma unroll
     for (int m = 0; m < M; ++m) ssq[m] = 0.0f;
     // one block of one row to digits
@@ -140,38 +145,30 @@ gemv_signs_kernel(const SignArgs a) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) f[j] *= 1.0f + u[j];
         }
-        uint32_t top = 0;                                                  // the largest magnitude as a bit pattern
+        uint32_t top = 0;                                                  // the largest magnitude of this lane's run as a bit pattern
 #pragma unroll
         for (int j = 0; j < 4; ++j) top = max(top, __float_as_uint(f[j]) & 0x7FFFFFFFu);
         top = max(top, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)top, 0xB1, 0xF, 0xF, true));    // quad_perm [1,0,3,2]
         top = max(top, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)top, 0x4E, 0xF, 0xF, true));    // [2,3,0,1]
         top = max(top, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)top, 0x141, 0xF, 0xF, true));   // row_half_mirror
-        top = max(top, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)top, 0x140, 0xF, 0xF, true));   // row_mirror
-        top = max(max((uint32_t)__builtin_amdgcn_readlane((int)top, 0), (uint32_t)__builtin_amdgcn_readlane((int)top, 16)),
-                  max((uint32_t)__builtin_amdgcn_readlane((int)top, 32), (uint32_t)__builtin_amdgcn_readlane((int)top, 48)));
         // to [2^30, 2^31), one less where the top digit would pass 127
         int ex = 30 - ((int)(top >> 23) - 127) - ((top & 0x7FFFFFu) > 0x7EFEFEu ? 1 : 0);
         ex = top == 0u ? 0 : ex;
-        const bool odd = top >= 0x7F800000u || ex > 143;                   // 2^-143 / 64 is the smallest float
+        const bool odd = top >= 0x7F800000u || ex > 119;                   // (a half is a multiple of 2^-24: times 2^-119 / 64 it is still exact)
+        undo[s][m] = top >= 0x7F800000u ? 64.0f : odd ? 1.0f : -ldexpf(1.0f, -ex - 6);
+        slow = (slow & ~(1u << (s * M + m))) | (__ballot(odd) ? 1u << (s * M + m) : 0u);
+        uint32_t b[4];                                                     // signed digits: the bytes of X + 128 (1 + 2^8 + 2^16 + 2^24), less 128 each
+#pragma unroll
+        for (int j = 0; j < 4; ++j) b[j] = odd ? __float_as_uint(f[j]) : ((uint32_t)(int)rintf(ldexpf(f[j], ex)) + 0x80808080u) ^ 0x80808080u;
+        // digit d (of a run of floats: byte d) of the four columns in one dword: piece (q, d) of 64 bytes, run of the pair, dword lane % 8
+        const uint32_t l01 = __builtin_amdgcn_perm(b[1], b[0], 0x05010400u), h01 = __builtin_amdgcn_perm(b[1], b[0], 0x07030602u);
+        const uint32_t l23 = __builtin_amdgcn_perm(b[3], b[2], 0x05010400u), h23 = __builtin_amdgcn_perm(b[3], b[2], 0x07030602u);
         uint32_t* area = mine + (uint32_t)(s * M + m) * 256u;
-        undo[s][m] = __uint_as_float(scalar(__float_as_uint(odd ? 1.0f : -ldexpf(1.0f, -ex - 6))));
-        slow = (slow & ~(1u << (s * M + m))) | (odd ? 1u << (s * M + m) : 0u);
-        if (odd) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) area[col + 8u * j] = __float_as_uint(f[j]);
-        } else {
-            uint32_t b[4];                                                 // signed digits: the bytes of X + 128 (1 + 2^8 + 2^16 + 2^24), less 128 each
-#pragma unroll
-            for (int j = 0; j < 4; ++j) b[j] = ((uint32_t)(int)rintf(ldexpf(f[j], ex)) + 0x80808080u) ^ 0x80808080u;
-            // digit d of the four columns in one dword: piece (q, d) of 64 bytes, run of the pair, dword lane % 8
-            const uint32_t l01 = __builtin_amdgcn_perm(b[1], b[0], 0x05010400u), h01 = __builtin_amdgcn_perm(b[1], b[0], 0x07030602u);
-            const uint32_t l23 = __builtin_amdgcn_perm(b[3], b[2], 0x05010400u), h23 = __builtin_amdgcn_perm(b[3], b[2], 0x07030602u);
-            uint32_t* o = area + 64u * q + li;
-            o[0] = __builtin_amdgcn_perm(l23, l01, 0x05040100u);
-            o[16] = __builtin_amdgcn_perm(l23, l01, 0x07060302u);
-            o[32] = __builtin_amdgcn_perm(h23, h01, 0x05040100u);
-            o[48] = __builtin_amdgcn_perm(h23, h01, 0x07060302u);
-        }
+        uint32_t* o = area + 64u * q + li;
+        o[0] = __builtin_amdgcn_perm(l23, l01, 0x05040100u);
+        o[16] = __builtin_amdgcn_perm(l23, l01, 0x07060302u);
+        o[32] = __builtin_amdgcn_perm(h23, h01, 0x05040100u);
+        o[48] = __builtin_amdgcn_perm(h23, h01, 0x07060302u);
         // operand row 4 q + d: digit d of lane group q's runs, zero in the other lane groups
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -179,6 +176,10 @@ gemv_signs_kernel(const SignArgs a) {
 #pragma unroll
         for (int k = 0; k < 4; ++k) dig[s][m][k] = p[k];
         if constexpr (LOOP || M > 2 || CB > 3) __builtin_amdgcn_sched_barrier(0);    // one block's floats become digits at a time: registers
+    };
+    // of run 2 q + r: lane 8 r of the row of sixteen, which a multiplication takes as it reads its operand (row_newbcast)
+    auto undo_of = [&](int s, int m, auto r) {
+        return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(undo[s][m]), 0x150 + 8 * decltype(r)::value, 0xF, 0xF, true));
     };
     auto barrier = [] {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
@@ -196,7 +197,7 @@ gemv_signs_kernel(const SignArgs a) {
     for (uint32_t chunk = t_begin, part = 0;;) {
         const uint32_t n = tiles_of(chunk);
         const bool ends = !LOOP || part + 1u == a.parts, over = ends && (!LOOP || t_end - chunk <= CHUNK);
-        uint2 head[CB];
+        uint32_t head[CB];
         bool live[CB];
 #pragma unroll
         for (int s = 0; s < CB; ++s) { head[s] = in.head[s]; block_of(part, s, live[s]); }
@@ -205,7 +206,7 @@ gemv_signs_kernel(const SignArgs a) {
         u32x3 w[P][CB];
         auto load = [&](int p, int s, uint32_t i) {
             const uint32_t at = i < n ? i : n - 1u, off = i < n && live[s] ? 0u : 0x80000000u;     // past the end: out of range, zeros and no fetch
-            const uint32_t place = (uint32_t)__builtin_amdgcn_readlane((int)head[s].x, (int)at), mask = (uint32_t)__builtin_amdgcn_readlane((int)head[s].y, (int)at);
+            const uint32_t place = (uint32_t)__builtin_amdgcn_readlane((int)head[s], (int)at), mask = (uint32_t)__builtin_amdgcn_readlane((int)head[s], (int)(16u + at));
             const uint32_t before = 32u * (uint32_t)__builtin_popcount(mask & rows_before) + ((mask & row_bit) ? at_sign : at_mean);
             w[p][s] = __builtin_bit_cast(u32x3, __builtin_amdgcn_raw_buffer_load_b96(wrs, before + off, place * 16u, 0));
         };
@@ -220,9 +221,21 @@ gemv_signs_kernel(const SignArgs a) {
 #pragma unroll
                 for (int m = 0; m < M; ++m) pack(s, m, in.v[s][m], in.u[s][XF == kSwiglu ? m : 0], live[s], chunk == t_begin);
         }
+        if constexpr (XF == kNorm) {
+            if (ends && chunk == t_begin) {
+#pragma unroll
+                for (int m = 0; m < M; ++m) {
+                    const float t = oil4::wave_sum(ssq[m]);
+                    if (lane == 0) {
+                        ssq_part[wave * (uint32_t)M + (uint32_t)m] = t;
+                        if constexpr (M > 1) ssq_part[(waves + wave) * (uint32_t)M + (uint32_t)m] = (float)(endless >> m & 1u);
+                    }
+                }
+            }
+        }
         float acc[M];
         auto multiply = [&](int p, int s, uint32_t i) {
-            const uint32_t mask = (uint32_t)__builtin_amdgcn_readlane((int)head[s].y, (int)i);
+            const uint32_t mask = (uint32_t)__builtin_amdgcn_readlane((int)head[s], (int)(16u + i));
             const bool spark = (mask & row_bit) != 0u;
             const u32x3 o = w[p][s];
             const uint32_t s0 = spark ? __builtin_amdgcn_alignbit(o.y, o.x, 16) : 0xFFFFFFFFu, s1 = spark ? o.z : 0xFFFFFFFFu;
@@ -251,15 +264,25 @@ gemv_signs_kernel(const SignArgs a) {
                 auto one = [](const i32x4& d) { return fmaf((float)(d[3] * 256 + d[2]), 65536.0f, (float)(d[1] * 256 + d[0])); };
                 float f0 = one(d0[m]), f1 = one(d1[m]);
                 if (slow & (1u << (s * M + m))) {                          // uniform
-                    const float* x = reinterpret_cast<const float*>(mine + (uint32_t)(s * M + m) * 256u) + 64u * q;
-                    f0 = f1 = 0.0f;
+                    const uint8_t* x = reinterpret_cast<const uint8_t*>(mine + (uint32_t)(s * M + m) * 256u + 64u * q);
+                    auto floats = [&](float f, auto r, uint32_t signs, const uint8_t* run) {
+                        // (a 64th of each beside an infinity: finite ones must not add up to the other one)
+                        const bool infinite = undo_of(s, m, r) == 64.0f;
+                        float e = 0.0f;
 #pragma unroll 1
-                    for (uint32_t k = 0; k < 32u; ++k) {
-                        f0 += __uint_as_float(__float_as_uint(x[k]) ^ (~(s0 << (31u - k)) & 0x80000000u));
-                        f1 += __uint_as_float(__float_as_uint(x[32u + k]) ^ (~(s1 << (31u - k)) & 0x80000000u));
-                    }
+                        for (uint32_t k = 0; k < 32u; ++k) {
+                            const uint8_t* p = run + 4u * (k & 7u) + (k >> 3);                  // bytes 64 apart
+                            const uint32_t b = p[0] | p[64] << 8 | p[128] << 16 | (uint32_t)p[192] << 24;
+                            const float v = __uint_as_float(b ^ (~(signs << (31u - k)) & 0x80000000u));
+                            e += infinite ? v * 0.015625f : v;
+                        }
+                        return undo_of(s, m, r) > 0.0f ? e : f;
+                    };
+                    f0 = floats(f0, std::integral_constant<int, 0>{}, s0, x);
+                    f1 = floats(f1, std::integral_constant<int, 1>{}, s1, x + 32);
                 }
-                acc[m] = fmaf(fmaf(c1, f1, c0 * f0), undo[s][m], acc[m]);
+                acc[m] = fmaf(undo_of(s, m, std::integral_constant<int, 0>{}) * c0, f0, acc[m]);
+                acc[m] = fmaf(undo_of(s, m, std::integral_constant<int, 1>{}) * c1, f1, acc[m]);
             }
         };
         // the loop is left, never skipped within: so every wait for a load counts the loads behind it
@@ -279,18 +302,6 @@ gemv_signs_kernel(const SignArgs a) {
                 for (int m = 0; m < M; ++m) o[64 * m] = LOOP && part ? o[64 * m] + acc[m] : acc[m];
                 if (++i == n) { more = false; break; }
                 if (CB == 1) load(p, 0, i + (uint32_t)(P - 1));
-            }
-        }
-        if constexpr (XF == kNorm) {
-            if (ends && chunk == t_begin) {
-#pragma unroll
-                for (int m = 0; m < M; ++m) {
-                    const float t = oil4::wave_sum(ssq[m]);
-                    if (lane == 0) {
-                        ssq_part[wave * (uint32_t)M + (uint32_t)m] = t;
-                        if constexpr (M > 1) ssq_part[(waves + wave) * (uint32_t)M + (uint32_t)m] = (float)(endless >> m & 1u);
-                    }
-                }
             }
         }
         if (ends) {

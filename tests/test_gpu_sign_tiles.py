@@ -100,6 +100,51 @@ def test_unusual_activations(M):
             assert rel_l2(np.where(ok, got, 0), np.where(ok, want, 0)) <= (1e-6 if case != 5 else 2e-3), case
 
 
+# A run is held relative to its own largest magnitude: an outlier over a run of scale 0 (SPARK_Q0) or mean 0 (OIL1) must cost the others no bits.  The bound is
+# test_sign_tiles'.
+@pytest.mark.parametrize("M", [1, 2, 3, 4])
+@pytest.mark.parametrize("rows,cols", [(100, 4096), (8300, 1024), (40, 12288)])
+@pytest.mark.parametrize("outlier", [1e3, 1e6, 1e10, 1e30])
+def test_outliers_over_runs_of_scale_zero(rows, cols, outlier, M):
+    if M > 2 and cols > 4096:
+        pytest.skip("another kernel's call")
+    rng = np.random.default_rng(rows)
+    n = rows * cols // 256
+    fm = (rng.random(n) < 0.5).astype(np.uint8)
+    w = gaussian_weights(rows * cols, 3).reshape(n, 8, 32)
+    w[:, 2] = np.where(np.arange(32) % 2, 0.02, -0.02)     # run 2: OIL1 blocks of mean 0 ...
+    w[fm == 1, 2] = 0.0                                    # ... SPARK_Q0 blocks of scale 0
+    payload, blocks = ia.block_codec.quantize_tensor(w.reshape(-1), fm)
+    x = torch.randn(M, cols, generator=torch.Generator().manual_seed(M)).cuda()
+    x.view(M, -1, 256)[:, ::2, 69] = outlier
+    with ia.DeviceWeights.from_blocks(payload, blocks, rows, cols) as dw:
+        got, want = dw.gemv(x), reference(dw, x)
+    assert float((got.double() - want).norm() / want.norm()) <= (12 + cols / 4096) * 2.0 ** -24
+
+
+# runs held as floats beside runs held as digits: the sums of the former may pass the largest float where the products with their scale do not
+@pytest.mark.parametrize("M", [1, 2, 3, 4])
+def test_runs_that_are_not_finite_or_tiny(M):
+    rows, cols = 70, 1024
+    rng = np.random.default_rng(M)
+    with tensor(rows, cols, 0.5, 8) as dw:
+        W = dw.dequant().view(rows, cols).cpu().numpy().astype(np.float64)
+        for case in range(3):
+            x = rng.standard_normal((M, cols)).astype(np.float32)
+            m = M - 1
+            if case == 0: x[m, 64:96], x[m, 80] = 3e37, np.inf               # an infinity behind floats near the largest, in its run
+            if case == 1: x[m, 64:96], x[m, 400] = 3e37, -np.inf             # ... in another block
+            if case == 2: x[m, 32:64] *= np.float32(1e-30); x[m, 320:352] *= np.float32(1e-40); x[m, 352:384] = 1e37 * np.sign(x[m, 352:384])
+            got = dw.gemv(torch.from_numpy(x).cuda()).cpu().numpy()
+            with np.errstate(invalid="ignore"):
+                want = np.stack([(W * x[i].astype(np.float64)).sum(1) for i in range(M)])
+            assert np.array_equal(np.isnan(got), np.isnan(want)), case
+            assert np.array_equal(np.where(np.isinf(got), np.sign(got), 0), np.where(np.isinf(want), np.sign(want), 0)), case
+            for i in range(M):
+                ok = np.isfinite(want[i])
+                assert rel_l2(got[i][ok].astype(np.float64) * 1e-20, want[i][ok] * 1e-20) <= 1e-6, (case, i)
+
+
 def test_scales_that_are_not_finite_keep_window_streams():
     """+-inf times activations of both signs is NaN in FP32 sums: signs first would make it an infinity."""
     payload, blocks = ia.block_codec.quantize_tensor(gaussian_weights(64 * 512, 5), ia.Format.SPARK_Q0)
