@@ -187,6 +187,7 @@ int launch_gemv_runs(const oilhip_weights& w, const float* d_x, float* d_y, int 
 double dense_estimate_us(uint32_t M, uint32_t N, uint32_t K);
 int launch_gemm_any(const oilhip_weights& w, const void* d_x, bool x_is_f32, float* d_y, int M, hipStream_t s);
 // ... sign tiles, decoded inside the kernel (gemm_signs.hip) ...
+int check_sign_parts(uint32_t bpr, uint32_t parts);       // a plan's parts of K, checked before its launch
 int launch_gemm_signs(const oilhip_weights& w, const void* d_x, bool x_is_f32, float* d_y, int M, hipStream_t s);
 // ... and plain uniform OIL4, decoded inside the kernel (gemm_oil4_frag.hip)
 int launch_gemm_oil4_frag(const oilhip_weights& w, const void* d_x, bool x_is_f32, float* d_y, int M, hipStream_t s);

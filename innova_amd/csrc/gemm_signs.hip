@@ -17,6 +17,7 @@
 // Tried and slower: weights through LDS, each made once per workgroup of 128 x 128 (40 us for the first of these: LDS and issue), tiles in groups of four
 // token blocks (28.1), a stage more of activations in LDS (a workgroup less per compute unit: 512 tokens 55 -> 62), parts of K with 64 x 256 tiles (60).
 #include <algorithm>
+#include <string>
 
 #include "common.h"
 #include "gemm_tiles.h"
@@ -113,7 +114,8 @@ gemm_signs_kernel(const SignGemmArgs a) {
     }
     __syncthreads();
 
-    const u32x4 xrs = resource(a.Xf + (size_t)mt * FM * G * 512u + (size_t)bbeg * 8192u, 0xFFFFFFFFu), wrs = resource(a.W, a.wbytes);
+    // (to the end of the part's columns of the last row block: a stage past them reads zeros)
+    const u32x4 xrs = resource(a.Xf + (size_t)mt * FM * G * 512u + (size_t)bbeg * 8192u, ((uint32_t)(FM - 1) * G + 16u * nblk) * 1024u), wrs = resource(a.W, a.wbytes);
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
     uint32_t voff[FM];
 #pragma unroll
@@ -307,6 +309,11 @@ SignPlan sign_plan(uint32_t M, uint32_t N, uint32_t bpr) {
 
 }  // namespace
 
+// The kernel takes its loops' lengths from its part of K, and a part without blocks has none: the plan's parts are checked where they become a launch.
+int check_sign_parts(uint32_t bpr, uint32_t parts) {
+    return parts >= 1u && parts <= bpr ? OILHIP_OK : fail(OILHIP_E_ARG, "prefill plan of " + std::to_string(parts) + " parts for " + std::to_string(bpr) + " blocks");
+}
+
 // Returns 1 when the tensor is not stored as sign tiles, or decoding it first may be as fast (small products).  Both times are estimates, this one 11 % short at most and
 // the other 14 % long at most, so a fifth less is asked for.
 int launch_gemm_signs(const oilhip_weights& w, const void* d_x, bool x_is_f32, float* d_y, int M_, hipStream_t s) {
@@ -316,12 +323,13 @@ int launch_gemm_signs(const oilhip_weights& w, const void* d_x, bool x_is_f32, f
     const SignPlan pl = sign_plan(M, N, bpr);
     if (64ull * pl.fn * ((bpr + pl.parts - 1u) / pl.parts) > 49152u || (uint64_t)w.cols * 512u >= 0x80000000ull) return 1;
     if (pl.us > 0.8 * dense_estimate_us(M, N, (uint32_t)w.cols)) return 1;
+    if (int rc = check_sign_parts(bpr, pl.parts)) return rc;
     const StreamLock lock(s);
     uint16_t* xf = nullptr;
     const uint32_t mpad = (M + 255u) & ~255u;
     if (int rc = stream_scratch(lock, kScratchGemmX, (size_t)mpad * w.cols * 2, reinterpret_cast<void**>(&xf))) return rc;
     const uint32_t tm = 32u * FM, tn = 128u * pl.fn;
-    SignGemmArgs a{w.d_payload, xf, d_y, nullptr, nullptr, (uint32_t)w.alloc_bytes, M, N, bpr, w.seg.sign_tiles, (M + tm - 1u) / tm, (N + tn - 1u) / tn, pl.parts};   // (no more parts than blocks: none is empty)
+    SignGemmArgs a{w.d_payload, xf, d_y, nullptr, nullptr, (uint32_t)w.alloc_bytes, M, N, bpr, w.seg.sign_tiles, (M + tm - 1u) / tm, (N + tn - 1u) / tn, pl.parts};
     if (a.parts > 1u) {
         void* p = nullptr;
         const size_t counters = ((size_t)a.MT * a.NT * 4u + 255u) & ~(size_t)255u;
