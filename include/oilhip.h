@@ -317,6 +317,8 @@ int oilhip_dense_map_f32(int op, const float* d_a, const float* d_b, float s, fl
  *                             (:484-486 attention input, :611-614 MLP input).  With M = 1 and an OIL4 tensor or one
  *                             stored as window streams or sign tiles the norm is formed while the GEMV stages x (one launch, d_xn unused and may be NULL);
  *                             otherwise d_xn[M][cols] receives the normalised rows, whichever launch forms them.
+ *                             (x * r * (1 + w) in that order: where the sum of squares passes the largest float, r and every finite product are 0.  One row of
+ *                             OIL4 or window streams multiplies by r after the sums, which are NaN there if they pass the largest float themselves.)
  * oilhip_mlp_step_f32       : Qwen35Engine::mlp_step (:611-621): y[M][D] = down(siluf(gate x) * up x), gate_up = the
  *                             gate and up projections stacked (2F x D, gate rows first), down = D x F.  A non-NULL
  *                             d_normw applies rmsnorm(x; d_normw) first, as the caller of mlp_step does.

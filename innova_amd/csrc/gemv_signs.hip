@@ -82,7 +82,7 @@ gemv_signs_kernel(const SignArgs a) {
     uint32_t* mine = smem + wave * ((uint32_t)(CB * M) * 256u + 16u);      // digits (or floats) of this wavefront's blocks, 1 KB each, and 64 bytes of zeros
     mine[(uint32_t)(CB * M) * 256u + li] = 0u;
     float* sums = reinterpret_cast<float*>(smem) + waves * ((uint32_t)(CB * M) * 256u + 16u);      // [tile of the chunk][wavefront][row of y][lane]
-    float* ssq_part = sums + (LOOP ? CHUNK : t_end - t_begin) * waves * (uint32_t)(64 * M);   // kNorm: [wavefront][row of y], then 1 where x is not finite
+    float* ssq_part = sums + (LOOP ? CHUNK : t_end - t_begin) * waves * (uint32_t)(64 * M);   // kNorm: [wavefront][row of y], negative where x or its weight is not finite
     const auto wrs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(a.W), (short)0, (int)a.wbytes, 0x00020000);
     const uint32_t* heads = reinterpret_cast<const uint32_t*>(a.W);        // [block of the row][tile]: {place / 16, mask of SPARK_Q0 rows}
     const uint32_t row_bit = 1u << li, rows_before = row_bit - 1u, at_mean = 16u * li + 4u * q, at_sign = 16u * li + 12u * q;
@@ -118,11 +118,11 @@ gemv_signs_kernel(const SignArgs a) {
     };
 
     i32x4 dig[CB][M][4];
-    float undo[CB][M], ssq[M];                                             // undo: of the run that this lane packs, lane / 8; positive where it is held as floats
-    uint32_t endless = 0;                                                  // kNorm, several rows: bit m: an x that is not finite
+    float undo[CB][M], ssq[M], endless[M];                                             // undo: of the run that this lane packs, lane / 8; positive where it is held as floats; endless: kNorm: 0, or NaN where x or a
+                                                                           // weight of the norm is not finite
     uint32_t slow = 0;                                                     // bit s * M + m: runs of that block add up in FP32
 #pragma unroll
-    for (int m = 0; m < M; ++m) ssq[m] = 0.0f;
+    for (int m = 0; m < M; ++m) ssq[m] = endless[m] = 0.0f;
     // one block of one row to digits
     auto pack = [&](int s, int m, float (&f)[4], const float (&u)[4], bool on, bool counts) {
 #pragma unroll
@@ -135,12 +135,8 @@ gemv_signs_kernel(const SignArgs a) {
             }
         }
         if constexpr (XF == kNorm) {
-            if constexpr (M > 1) {
-                bool any = false;
 #pragma unroll
-                for (int j = 0; j < 4; ++j) any |= (__float_as_uint(f[j]) & 0x7F800000u) == 0x7F800000u;
-                endless |= __ballot(any) ? 1u << m : 0u;
-            }
+            for (int j = 0; j < 4; ++j) endless[m] = fmaf(f[j], 0.0f, fmaf(u[j], 0.0f, endless[m]));
             ssq[m] += counts ? (f[0] * f[0] + f[1] * f[1]) + (f[2] * f[2] + f[3] * f[3]) : 0.0f;
 #pragma unroll
             for (int j = 0; j < 4; ++j) f[j] *= 1.0f + u[j];
@@ -186,9 +182,16 @@ gemv_signs_kernel(const SignArgs a) {
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
     };
-    auto norm_of = [&](uint32_t m) {
-        float t = 0.0f;
-        for (uint32_t j = 0; j < waves; ++j) t += ssq_part[j * (uint32_t)M + m];
+    // (m is the same for a wavefront; a lane per wavefront's sum, then over the sixteen lanes: one read of LDS instead of one behind the other)
+    auto norm_of = [&](uint32_t m, bool& finite) {
+        const float p = li < waves ? ssq_part[li * (uint32_t)M + m] : 0.0f;
+        float t = fabsf(p);
+        auto add = [&](auto how) { t += __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(t), decltype(how)::value, 0xF, 0xF, true)); };
+        add(std::integral_constant<int, 0xB1>{});                          // quad_perm [1,0,3,2]
+        add(std::integral_constant<int, 0x4E>{});                          // [2,3,0,1]
+        add(std::integral_constant<int, 0x141>{});                         // row_half_mirror
+        add(std::integral_constant<int, 0x140>{});                         // row_mirror
+        finite = __ballot((int)__float_as_uint(p) < 0) == 0u;
         return 1.0f / sqrtf(t / (float)(256u * a.bpr) + 1e-6f);
     };
 
@@ -221,18 +224,16 @@ gemv_signs_kernel(const SignArgs a) {
 #pragma unroll
                 for (int m = 0; m < M; ++m) pack(s, m, in.v[s][m], in.u[s][XF == kSwiglu ? m : 0], live[s], chunk == t_begin);
         }
-        if constexpr (XF == kNorm) {
-            if (ends && chunk == t_begin) {
+        auto share_norm = [&] {
+            if (!ends || chunk != t_begin) return;
 #pragma unroll
-                for (int m = 0; m < M; ++m) {
-                    const float t = oil4::wave_sum(ssq[m]);
-                    if (lane == 0) {
-                        ssq_part[wave * (uint32_t)M + (uint32_t)m] = t;
-                        if constexpr (M > 1) ssq_part[(waves + wave) * (uint32_t)M + (uint32_t)m] = (float)(endless >> m & 1u);
-                    }
-                }
+            for (int m = 0; m < M; ++m) {
+                const float t = oil4::wave_sum(ssq[m]);
+                const bool any = __ballot(endless[m] != 0.0f) != 0u;
+                if (lane == 0) ssq_part[wave * (uint32_t)M + (uint32_t)m] = __uint_as_float((__float_as_uint(t) & 0x7FFFFFFFu) | (any ? 0x80000000u : 0u));
             }
-        }
+        };
+        if constexpr (XF == kNorm && M > 1) share_norm();                  // (one row: below, where the loads have arrived; several: registers)
         float acc[M];
         auto multiply = [&](int p, int s, uint32_t i) {
             const uint32_t mask = (uint32_t)__builtin_amdgcn_readlane((int)head[s], (int)(16u + i));
@@ -304,6 +305,7 @@ gemv_signs_kernel(const SignArgs a) {
                 if (CB == 1) load(p, 0, i + (uint32_t)(P - 1));
             }
         }
+        if constexpr (XF == kNorm && M == 1) share_norm();
         if (ends) {
             barrier();
             // a wavefront per tile and row of y: first over the wavefronts, four sums side by side, then over the lane groups
@@ -320,15 +322,10 @@ gemv_signs_kernel(const SignArgs a) {
                 const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(y), __float_as_uint(y), false, false);
                 y = __uint_as_float(r[0]) + __uint_as_float(r[1]);
                 if constexpr (XF == kNorm) {
-                    const float r = norm_of(m);
-                    if constexpr (M > 1) {
-                        // a sum of squares past the largest float makes every finite x zero, before it meets a weight
-                        float bad = 0.0f;
-                        for (uint32_t j = 0; j < waves; ++j) bad += ssq_part[(waves + j) * (uint32_t)M + m];
-                        y = r == 0.0f && bad == 0.0f ? 0.0f : y * r;
-                    } else {
-                        y *= r;
-                    }
+                    // a sum of squares past the largest float makes every finite x zero, before it meets a weight
+                    bool finite;
+                    const float r = norm_of(m, finite);
+                    y = r == 0.0f && finite ? 0.0f : y * r;
                 }
                 const uint32_t row = (chunk + t) * 16u + lane;
                 if (lane < 16u && row < a.rows) a.y[(size_t)m * a.rows + row] = y;
@@ -339,7 +336,8 @@ gemv_signs_kernel(const SignArgs a) {
                     for (uint32_t b = wg; b < a.bpr; b += gridDim.x)
                         for (uint32_t o = threadIdx.x; o < 256u * M; o += blockDim.x) {
                             const uint32_t m = o >> 8, c = 256u * b + (o & 255u);
-                            a.xn[(size_t)m * a.ldx + c] = a.x[(size_t)m * a.ldx + c] * norm_of(m) * (1.0f + a.norm_w[c]);
+                            bool finite;
+                            a.xn[(size_t)m * a.ldx + c] = a.x[(size_t)m * a.ldx + c] * norm_of(m, finite) * (1.0f + a.norm_w[c]);
                         }
             }
             if (over) break;
@@ -356,7 +354,7 @@ int launch_form(const SignArgs& a, uint32_t wgs, hipStream_t s) {
     static std::atomic<uint64_t> raised{0};
     auto kern = gemv_signs_kernel<M, CB, XF, LOOP>;
     if (int rc = ensure_max_lds(raised, reinterpret_cast<const void*>(kern), 160 * 1024)) return rc;
-    const size_t lds = (size_t)a.waves * (CB * M * 1024u + 64u + (LOOP ? chunk_for(M) : a.t_base + (a.t_rem ? 1u : 0u)) * 256u * M + 8u * M);
+    const size_t lds = (size_t)a.waves * (CB * M * 1024u + 64u + (LOOP ? chunk_for(M) : a.t_base + (a.t_rem ? 1u : 0u)) * 256u * M + 4u * M);
     hipLaunchKernelGGL(kern, dim3(wgs), dim3(64u * a.waves), lds, s, a);
     OILHIP_HIP(hipGetLastError());
     return OILHIP_OK;

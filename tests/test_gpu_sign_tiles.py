@@ -185,6 +185,23 @@ def test_with_norm_and_swiglu(M, D, F, shift):
     down.close()
 
 
+# x * r * (1 + w) in that order: a sum of squares past the largest float makes r and so every finite x zero, whatever x times a weight would be; an infinity
+# stays NaN, and so does zero times an infinite weight of the norm
+@pytest.mark.parametrize("M", [1, 2, 3, 4])
+@pytest.mark.parametrize("rows,cols", [(70, 768), (70, 4608), (9000, 512)])
+def test_norm_of_the_largest_activations(rows, cols, M):
+    with tensor(rows, cols, 0.5, rows + cols) as dw:
+        for case in range(4):
+            x = torch.randn(M, cols, generator=torch.Generator().manual_seed(M)).cuda()
+            nw = torch.zeros(cols, device="cuda")
+            x[M - 1] = 3e38 if case != 2 else 1e25
+            if case == 1: x[M - 1, cols - 1] = float("inf")
+            if case == 3: nw[5] = float("inf")
+            y = layers.gemv_rmsnorm(dw, x, nw)
+            assert bool((y[M - 1] == 0).all() if case in (0, 2) else y[M - 1].isnan().all()), case
+            assert case == 3 or bool(torch.isfinite(y[:M - 1]).all() and (M == 1 or y[:M - 1].abs().max() > 0)), case
+
+
 # prefill without a launch that decodes: K whole, in 2, 4 and 8 parts (uneven ones among them), and wavefronts of two row blocks; rows and tokens that end
 # inside a tile.  Each operand is rounded to bf16 once, the weights here only: 2^-9 at most, a third of it in the mean.
 @pytest.mark.parametrize("rows,cols,M", [(5001, 2816, 437), (11008, 4096, 40), (2600, 12544, 100), (4099, 11008, 64), (2600, 11008, 33), (11008, 4096, 2048)])
