@@ -167,7 +167,8 @@ int oilhip_dequant_f32(const oilhip_weights* w, float* d_out, void* stream);
 
 /* Qwen35Engine::gemm (src/adapters/tools/qwen35_engine.cpp:47-85):
  * d_y[b*rows + r] = sum_c W[r][c] * d_x[b*cols + c], FP32 in, FP32 out,
- * FP32 accumulation, 1 <= M (the reference caps a call at 512). */
+ * FP32 accumulation, 1 <= M (the reference caps a call at 512).  d_y must not share memory with d_x for M <= 2: workgroups read all activations while others
+ * store outputs.  (With more rows the activations are packed first wherever a kernel of several rows serves the tensor and finds its scratch.) */
 int oilhip_gemv_f32(const oilhip_weights* w, const float* d_x, float* d_y, int M, void* stream);
 
 /* The same product over a workspace of the caller's, where oilhip_gemv_f32 packs several activation rows in a scratch that

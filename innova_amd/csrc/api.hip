@@ -159,7 +159,7 @@ int gemv_f32(const oilhip_weights& w, const float* d_x, float* d_y, int M, hipSt
         if (rc == 1 && M > 2 && M <= 4) rc = launch_gemv_oil4(w, d_x, d_y, M, s);
         if (rc <= 0) return rc;
     }
-    if (signs_fastest(w, M) && (M == 1 || !rows_overlap(w, d_x, d_y, M))) return launch_gemv_signs(w, d_x, d_y, M, s);
+    if (signs_fastest(w, M) && (M == 1 || !overlap(d_x, M * w.cols, d_y, M * w.rows))) return launch_gemv_signs(w, d_x, d_y, M, s);
     if (M >= 2) {
         const int rc = launch_gemv_any_multi(w, d_x, d_y, M, s, d_pack);
         if (rc <= 0) return rc;

@@ -174,11 +174,11 @@ int launch_gemv_seg(const oilhip_weights& w, const float* d_x, float* d_y, int M
 // SPARK_Q0 and OIL1 blocks stored as sign tiles, kSignRows activation rows per launch
 constexpr int kSignRows = 4;
 bool signs_fastest(const oilhip_weights& w, int M);       // whether this kernel is faster than gemv_any_multi's
-// Whether y shares memory with x: then several rows go through a kernel whose activations are packed by a launch of their own, before any
-// output is stored, where there is one.
-inline bool rows_overlap(const oilhip_weights& w, const float* x, const float* y, int M) {
-    const uintptr_t x0 = reinterpret_cast<uintptr_t>(x), y0 = reinterpret_cast<uintptr_t>(y);
-    return x0 < y0 + 4u * (uintptr_t)M * w.rows && y0 < x0 + 4u * (uintptr_t)M * w.cols;
+// Whether arrays of na and nb floats share memory.  Several rows whose outputs lie over something that workgroups read, or store besides, go through a kernel
+// whose activations are packed by a launch of their own, before any output is stored, where there is one.
+inline bool overlap(const float* a, uint64_t na, const float* b, uint64_t nb) {
+    const uintptr_t a0 = reinterpret_cast<uintptr_t>(a), b0 = reinterpret_cast<uintptr_t>(b);
+    return a0 < b0 + 4u * nb && b0 < a0 + 4u * na;
 }
 int launch_gemv_signs(const oilhip_weights& w, const float* d_x, float* d_y, int M, hipStream_t s, const MultiInput& in = {}, uint32_t ldx = 0);
 // every format, a lane per run of 32 weights

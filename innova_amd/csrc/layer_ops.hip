@@ -109,7 +109,8 @@ int gemv_rmsnorm(const oilhip_weights& w, const float* d_x, const float* d_normw
                                               MultiInput{nullptr, d_normw, false, d_xn}, nullptr, nullptr, 0, d_pack);
         if (rc <= 0) return rc;
     }
-    if (signs_fastest(w, M) && apart && !rows_overlap(w, d_x, d_y, M))     // likewise, by each workgroup for itself
+    const bool y_apart = !overlap(d_y, M * w.rows, d_x, M * w.cols) && !overlap(d_y, M * w.rows, d_xn, M * w.cols) && !overlap(d_y, M * w.rows, d_normw, w.cols);
+    if (signs_fastest(w, M) && apart && y_apart)                           // likewise, by each workgroup for itself
         return launch_gemv_signs(w, d_x, d_y, M, s, MultiInput{nullptr, d_normw, false, d_xn});
     if (M >= 2 && !plain_oil4(w) && w.cols <= kPackNormMaxCols && apart) { // likewise for the other formats
         const int rc = launch_gemv_any_multi(w, d_x, d_y, M, s, d_pack, MultiInput{nullptr, d_normw, false, d_xn});
@@ -134,7 +135,8 @@ int mlp_step(const oilhip_weights& gate_up, const oilhip_weights& down, const fl
         const int rc = launch_gemv_oil4_swiglu(down, h2, d_y, s);          // SwiGLU formed while the activations are staged
         if (rc <= 0) return rc;
     }
-    if (signs_fastest(down, M)) return launch_gemv_signs(down, h2, d_y, M, s, MultiInput{h2 + F, nullptr, true}, (uint32_t)(2 * F));
+    if (signs_fastest(down, M) && (M == 1 || !overlap(d_y, M * down.rows, h2, M * 2 * F)))
+        return launch_gemv_signs(down, h2, d_y, M, s, MultiInput{h2 + F, nullptr, true}, (uint32_t)(2 * F));
     if (M == 1 && down.seg.nstreams) {
         const int rc = launch_gemv_seg_swiglu(down, h2, d_y, s);
         if (rc <= 0) return rc;

@@ -73,6 +73,62 @@ def test_outputs_over_the_activations():
         assert rel_l2(dw.gemv(x, out=x).cpu().numpy(), want.cpu().numpy()) <= 1e-6
 
 
+def test_two_rows_of_outputs_over_the_activations():
+    """More than 8192 rows, which are packed by a launch of their own (fewer never were: outputs may not lie over the activations there)."""
+    with tensor(8448, 8448, 0.5, 4) as dw:
+        x = torch.randn(2, 8448, generator=torch.Generator().manual_seed(1)).cuda()
+        want = reference(dw, x)
+        assert rel_l2(dw.gemv(x, out=x).cpu().numpy(), want.cpu().numpy()) <= 1e-6
+
+
+def test_captured_outputs_over_the_activations():
+    """The workspace that a captured call gets is what the activations are packed into; apart from them it stays unused."""
+    L = ia._lib.lib()
+    with tensor(512, 512, 0.5, 4) as dw:
+        assert [L.oilhip_gemv_workspace_bytes(dw.handle, M) > 0 for M in (1, 2, 3, 4, 5)] == [False, False, True, True, True]
+        x0 = torch.randn(3, 512, generator=torch.Generator().manual_seed(1)).cuda()
+        x, want = x0.clone(), reference(dw, x0)
+        dw.gemv(x.clone())
+        side, g = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+        torch.cuda.synchronize()
+        with torch.cuda.graph(g, stream=side):
+            dw.gemv(x, out=x)
+        for _ in range(3):
+            x.copy_(x0)
+            g.replay()
+            torch.cuda.synchronize()
+            assert rel_l2(x.cpu().numpy(), want.cpu().numpy()) <= 1e-6
+
+
+# outputs over the normalised rows (which are stored for the caller as well), over the norm's weights, over the step's scratch: calls of three and four rows,
+# whose activations were always packed before any output was stored
+@pytest.mark.parametrize("M", [3, 4])
+def test_outputs_over_other_arrays_of_the_call(M):
+    D, F, L, S = 1024, 2048, ia._lib.lib(), ia._lib.current_stream
+    sq, gu, down = tensor(D, D, 0.5, 1), tensor(2 * F, D, 0.5, 2), tensor(D, F, 0.5, 3)
+    x = torch.randn(M, D, generator=torch.Generator().manual_seed(M)).cuda()
+    nw = torch.randn(D, generator=torch.Generator().manual_seed(9)).cuda() * 0.2
+    xn = x.double() / (x.double().pow(2).mean(1, keepdim=True) + 1e-6).sqrt() * (1.0 + nw.double())
+    want = reference(sq, xn).cpu().numpy()
+    for _ in range(8):                                     # stores in any order: several tries
+        both = torch.empty(M, D, device="cuda")
+        ia._lib.check(L.oilhip_gemv_rmsnorm_f32(sq.handle, x.data_ptr(), nw.data_ptr(), both.data_ptr(), M, both.data_ptr(), S()))
+        assert rel_l2(both.cpu().numpy(), want) <= 1e-6
+        over = torch.empty(M, D, device="cuda")
+        over[M - 1] = nw
+        spare = torch.empty(M, D, device="cuda")
+        ia._lib.check(L.oilhip_gemv_rmsnorm_f32(sq.handle, x.data_ptr(), over[M - 1].data_ptr(), over.data_ptr(), M, spare.data_ptr(), S()))
+        assert rel_l2(over.cpu().numpy(), want) <= 1e-6
+    gate, up = reference(gu, xn)[:, :F], reference(gu, xn)[:, F:]
+    want = reference(down, gate / (1.0 + (-gate).exp()) * up).cpu().numpy()
+    for _ in range(8):
+        scratch = torch.empty(M * (3 * F + D), device="cuda")
+        ia._lib.check(L.oilhip_mlp_step_f32(gu.handle, down.handle, x.data_ptr(), nw.data_ptr(), scratch.data_ptr(), M, scratch.data_ptr(), S()))
+        assert rel_l2(scratch[:M * D].cpu().numpy(), want) <= 3e-6
+    for w in (sq, gu, down):
+        w.close()
+
+
 # infinities, NaN, a block of zeros, magnitudes whose power of two has no inverse among the floats, and the largest and smallest mantissas of a digit
 @pytest.mark.parametrize("M", [1, 2, 3, 4])
 def test_unusual_activations(M):
