@@ -620,9 +620,8 @@ OIL_INLINE void full_lattice(const float* w, double sum_sq, uint8_t* out) {
     pack_codes<BITS>(dense, 256 - 256 / RUN, out + 2);
 }
 
-template <int BITS, bool WIDE>
+template <int BITS>
 OIL_INLINE bool full_grouped(const float* w, uint8_t* out) {
-    if constexpr (WIDE && BITS == 8) return grouped8_avx512(w, out);
     float zp[4], sc[4];
     if constexpr (BITS == 8) {
         for (int g = 0; g < 4; ++g) {
@@ -686,9 +685,9 @@ OIL_INLINE bool encode_full(int fmt, const float* w, double sum_sq, uint8_t* out
         case OILHIP_OIL2: full_lattice<2, WIDE>(w, sum_sq, out); return true;
         case OILHIP_OIL4: full_lattice<4, WIDE>(w, sum_sq, out); return true;
         case OILHIP_OIL8: full_lattice<8, WIDE>(w, sum_sq, out); return true;
-        case OILHIP_OIL2_GRP: return full_grouped<2, WIDE>(w, out);
-        case OILHIP_OIL4_GRP: return full_grouped<4, WIDE>(w, out);
-        case OILHIP_OIL8_GRP: return full_grouped<8, WIDE>(w, out);
+        case OILHIP_OIL2_GRP: if constexpr (!WIDE) return full_grouped<2>(w, out); else return false;      // (WIDE: encode_range takes four blocks' groups side by side)
+        case OILHIP_OIL4_GRP: if constexpr (!WIDE) return full_grouped<4>(w, out); else return false;
+        case OILHIP_OIL8_GRP: if constexpr (!WIDE) return full_grouped<8>(w, out); else return grouped8_avx512(w, out);
         case OILHIP_OIL1: {
             if constexpr (WIDE) { means_avx512(w, out); return true; }
             double s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -769,11 +768,10 @@ OIL_INLINE void encode_range(const uint8_t* fmts, const float* w, uint64_t numel
             if constexpr (WIDE) {
                 if (fmt == OILHIP_OIL2_GRP || fmt == OILHIP_OIL4_GRP) {
                     const uint32_t g = grouped++;
-                    if (largest_bits(w + at) <= kLargestBits) {
-                        if (fmt == OILHIP_OIL2_GRP) grouped_avx512<2>(w + at, zp[g], sc[g], out);
-                        else grouped_avx512<4>(w + at, zp[g], sc[g], out);
-                        continue;
-                    }
+                    if (largest_bits(w + at) > kLargestBits) encode_plain(b + j);
+                    else if (fmt == OILHIP_OIL2_GRP) grouped_avx512<2>(w + at, zp[g], sc[g], out);
+                    else grouped_avx512<4>(w + at, zp[g], sc[g], out);
+                    continue;
                 }
             }
             if (!encode_full<WIDE>(fmt, w + at, s[j], out)) encode_plain(b + j);
