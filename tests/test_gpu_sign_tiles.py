@@ -268,3 +268,34 @@ def test_prefill(rows, cols, M):
         want = reference(dw, x.to(torch.bfloat16))
         assert float((got.double() - want).norm() / want.norm()) <= 2e-3
         assert torch.equal(got, dw.gemm_bf16(x.to(torch.bfloat16))) and torch.equal(got, dw.gemm_f32(x))
+
+
+# K whole and in parts; activations that start inside 16 bytes (packed by loads that ask for 4 and 2 bytes), tokens with infinities and NaN, outputs over the activations (which
+# are packed by a launch of their own)
+@pytest.mark.parametrize("rows,cols,M", [(5001, 2816, 437), (11008, 4096, 40), (2600, 12544, 100)])
+def test_prefill_of_unusual_activations(rows, cols, M):
+    L, S = ia._lib.lib(), ia._lib.current_stream
+    with tensor(rows, cols, 0.5, rows + M) as dw:
+        x = torch.randn(M, cols, generator=torch.Generator().manual_seed(M)).cuda()
+        x[3, 5], x[7, cols - 1], x[M - 1, 300] = float("inf"), float("-inf"), float("nan")
+        x[9, [8, 700]] = torch.tensor([float("inf"), float("inf")], device="cuda")
+        xb, plain = x.to(torch.bfloat16), dw.gemm_f32(x)
+        want = reference(dw, xb)
+        assert torch.equal(plain.isnan(), want.isnan()) and int(want.isnan().sum()) >= rows
+        assert torch.equal(torch.where(plain.isinf(), plain.sign(), 0.0).double(), torch.where(want.isinf(), want.sign(), 0.0)) and int(want.isinf().sum()) >= 2 * rows
+        ok = want.isfinite()
+        assert float((plain.double() - want)[ok].norm() / want[ok].norm()) <= 2e-3
+        bits = plain.view(torch.int32)
+        same = lambda y: torch.equal(torch.where(plain.isnan(), 0, bits), torch.where(y.isnan(), 0, y.view(torch.int32)))
+        for shift in (1, 2, 3):
+            f = torch.zeros(shift + M * cols, device="cuda")[shift:].view(M, cols)
+            f.copy_(x)
+            assert same(dw.gemm_f32(f)), shift
+        for shift in (1, 3, 7):
+            b = torch.zeros(shift + M * cols, device="cuda", dtype=torch.bfloat16)[shift:].view(M, cols)
+            b.copy_(xb)
+            assert same(dw.gemm_bf16(b)), shift
+        both = torch.zeros(M * max(rows, cols), device="cuda")
+        both[:M * cols] = x.view(-1)
+        ia._lib.check(L.oilhip_gemm_f32(dw.handle, both.data_ptr(), both.data_ptr(), M, S()))
+        assert same(both[:M * rows].view(M, rows))
