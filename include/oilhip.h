@@ -125,7 +125,7 @@ int oilhip_weights_info(const oilhip_weights* w, uint64_t* rows, uint64_t* cols,
                         uint32_t* nblocks, uint64_t* payload_bytes, int* uniform_fmt);
 
 /* Device memory the tensor occupies: block bytes as stored (padding, and for every tensor of full blocks except uniform
- * OIL4 / OIL8 the window headers and block tags of its streams), and the 16-byte per-block descriptors.  The difference between stored_bytes
+ * OIL4 / OIL8 the window headers and block tags of its streams, or 8 bytes per tile and block of the row where it is stored as sign tiles), and the 16-byte per-block descriptors.  The difference between stored_bytes
  * and payload_bytes is what a GEMV reads on top of the algorithmic bytes.  No counterpart in the reference, whose
  * tensors live in host memory (include/oil/qwen35_engine.h:29).  Either out pointer may be NULL. */
 int oilhip_weights_device_bytes(const oilhip_weights* w, uint64_t* stored_bytes, uint64_t* descriptor_bytes);
@@ -175,7 +175,8 @@ int oilhip_gemv_f32(const oilhip_weights* w, const float* d_x, float* d_y, int M
  * belongs to the stream.  For calls that are captured: a graph keeps the address of what it packs into, so two graphs captured
  * on one stream may be replayed side by side only if their calls had workspaces of their own (without one, calls on
  * uniform OIL4 tensors with M >= 3 share the stream's, and calls on other tensors take slower kernels that pack nothing).
- * d_ws: 16-byte aligned, at least oilhip_gemv_workspace_bytes(w, M), which may be 0; it has to live as long as the graph, and calls
+ * d_ws: 16-byte aligned, at least oilhip_gemv_workspace_bytes(w, M), which may be 0 (and which a call may leave unused: three and four rows of SPARK_Q0 and
+ * OIL1 blocks up to 4096 columns pack into it only where d_y lies over d_x); it has to live as long as the graph, and calls
  * that follow one another on the stream may share it.  No counterpart in the reference. */
 size_t oilhip_gemv_workspace_bytes(const oilhip_weights* w, int M);
 int oilhip_gemv_f32_ws(const oilhip_weights* w, const float* d_x, float* d_y, int M, void* d_ws, size_t ws_bytes, void* stream);

@@ -457,7 +457,7 @@ static int upload(std::vector<uint8_t>& pay, std::vector<DevBlock>& db, std::vec
     };
     hipError_t e;
     if ((e = hipGetDevice(&w->device)) != hipSuccess) return bail(e, "hipGetDevice");
-    // window streams for every tensor of full blocks but the uniform OIL4 and OIL8 ones, which have kernels of their own
+    // window streams or sign tiles for every tensor of full blocks but the uniform OIL4 and OIL8 ones, which have kernels of their own
     // that read the blocks back to back
     const bool own_kernel = uniform && regular && nblocks && db[0].cb_bytes == 0 && db[0].off16 == 0 &&
                             ((db[0].fmt == OILHIP_OIL4 && db[0].idx_bytes == 128) || (db[0].fmt == OILHIP_OIL8 && db[0].idx_bytes == 256)) &&
@@ -580,7 +580,7 @@ int oilhip_weights_stack_rows(const oilhip_weights* const* parts, int n, oilhip_
     }
     if (!regular) {
         // parts that mix formats (or differ in format): fetch their blocks back and upload the concatenation, which
-        // lays the rows out afresh (window streams for a mix)
+        // lays the rows out afresh (window streams or sign tiles)
         if (nblocks > 0xFFFFFFFFull) return fail(OILHIP_E_ARG, "stack_rows: too large");
         std::vector<uint8_t> pay;
         std::vector<DevBlock> db;

@@ -5,7 +5,9 @@
 //
 // The products run on v_mfma_f32_16x16x32_f16 and are exact: an activation is scaled by a power of two per (token, block) and cut
 // into three FP16 pieces (33 bits), which are three rows of the matrix instruction's A operand; a weight is an exact FP16 number
-// times a factor that its block, or its group of 64, shares:
+// times a factor that its block, or its group of 64, shares.  (A piece counts from the largest magnitude of its block: an outlier over a run whose scale is 0 costs
+// the other runs bits.  SPARK_Q0 and OIL1, five rows, an outlier over a run of scale 0 in every block, error against 64 bits: of 1e5 1.1e-7, 1e6 5.6e-7, 1e8 7e-5;
+// one to four rows, where gemv_signs serves them, 0.8e-7 throughout.)
 //   SPARK_Q0, OIL1, OIL1_GRP   the weight itself (+- an FP16 scale, an FP16 mean)
 //   OIL2, OIL2_GRP             10^4 times the level (15104, 4528)
 //   OIL4_GRP                   10^4 / 256 times the level as a sum of two (signed bytes a and b / 256 of 256 a + b)
@@ -14,7 +16,7 @@
 // one more matrix instruction (group sums of the activations, in three pieces, times the FP16 zero points).
 // A wavefront takes every n-th block of the row for a run of 16-row groups, keeps the activations of its block in registers, and
 // the wavefronts' sums meet in LDS once per run; every sum has a fixed order.  All but OIL8 are stored as
-// window streams; a block is found through its descriptor, two steps ahead.  The pieces lie in a workspace of the caller's or in scratch of the
+// window streams or sign tiles; a block is found through its descriptor, two steps ahead.  The pieces lie in a workspace of the caller's or in scratch of the
 // stream; a call that is being captured without a workspace is left to the kernels that pack nothing.
 //
 // What bounds it: latency at two wavefronts per SIMD and the two launches where rows are short or few (planner's mix, 11008 x 4096, five rows: vector
@@ -54,7 +56,7 @@ constexpr int kPassTokens = 16;
 // Operand columns: step s of a block, lane group kq, element e is column 64 kq + 8 s + e (A), or 64 (s / 2) + 16 kq + 8 (s % 2) + e (C).
 enum Source { kSpark = 0, kPlanner, kOil2, kOil8, kOil2Grp, kOil4Grp, kOil8Grp, kSparkMix };
 constexpr bool grouped(int S) { return S >= kOil2Grp; }
-constexpr bool by_descriptor(int S) { return S != kOil8; }                 // stored as window streams (common.h)
+constexpr bool by_descriptor(int S) { return S != kOil8; }                 // stored as window streams or sign tiles (common.h)
 constexpr int steps_of(int S) { return grouped(S) ? 9 : 8; }               // the ninth: group sums
 __host__ __device__ constexpr uint32_t tile_bytes(bool grp) { return (grp ? 9u : 8u) * 1024u; }
 
@@ -662,7 +664,8 @@ bool faster_than_row_kernels(int src, const oilhip_weights& w, int M) {
     const uint64_t weights = w.rows * w.cols;
     const bool light = src == kSpark || src == kPlanner;
     if (src == kOil8) return M <= 4 ? weights >= 12000000u : M > 2 && weights >= 2000000u;
-    // Two rows: tall tensors, which are packed for one row at a time, and of these the formats whose error is no larger here (11008 x 4096
+    // Two rows: tall tensors, which are packed for one row at a time, and of these the formats whose error is no larger here (as window streams; stored as
+    // sign tiles they come here only with outputs that lie over the activations: 11008 x 4096
     // SPARK_Q0 16.5 against 12.3 us, planner's mix 12.0 against 12.4; 22016 x 4096 24 against 13, 19 against 15).
     if (M == 2) return light && w.seg.waves == 16;
     // Three and four: SPARK_Q0 and the planner's mix always (1000 x 2048, 3 rows 7.2 against 6.1 us, 4096 x 11008, 4 rows 43 against 14).

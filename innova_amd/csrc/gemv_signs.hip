@@ -18,10 +18,10 @@
 // What bounds it: vector issue (about 60 instructions per tile of one block, 30 of them making sign bytes; as many to pack a block of activations) and, below
 // ten tiles a workgroup, latency: the launch, the tiles' places, the blocks, each behind the other.  Before (window streams, gemv_seg.hip; several rows
 // gemv_any_multi.hip) -> now, us, planner's mix, launches of a graph over a ring of tensors in memory:
-//   one row   649 x 768 4.0 -> 2.5   4096 x 4096 5.4 -> 3.9   12288 x 4096 7.8 -> 5.3   22016 x 4096 12.0 -> 7.1   60000 x 4096 23.4 -> 13.5
-//             4096 x 11008 8.0 -> 6.2   SPARK_Q0 alone 11008 x 4096 10.6 -> 5.3
-//   two       4096 x 4096 6.6 -> 4.7   22016 x 4096 14.7 -> 8.8   4096 x 11008 15.2 -> 10.0
-//   three     1000 x 1280 5.6 -> 3.8   11008 x 4096 12.1 -> 8.4;   four   11008 x 4096 12.2 -> 9.3
+//   one row   649 x 768 4.0 -> 2.5   4096 x 4096 5.3 -> 3.9   12288 x 4096 8.1 -> 5.3   22016 x 4096 12.3 -> 7.1   60000 x 4096 23.6 -> 13.6
+//             4096 x 11008 8.1 -> 6.2   SPARK_Q0 alone 11008 x 4096 10.8 -> 5.3   with the norm 12288 x 4096 8.7 -> 5.9
+//   two       4096 x 4096 6.7 -> 4.7   22016 x 4096 14.8 -> 8.7   4096 x 11008 15.3 -> 9.8   with the norm 12288 x 4096 13.2 -> 7.5
+//   three     1000 x 1280 5.6 -> 3.7   11008 x 4096 11.8 -> 8.3;   four   11008 x 4096 11.8 -> 9.3   with the norm 12288 x 4096 13.6 -> 11.1
 // (One power of two per run instead of per block is an instruction more per tile of one block and row: long launches 1 to 4 % slower, short ones 1 to 3 % faster,
 // with eight instructions fewer in the packing.)
 // Error against 64 bits (2-norm, 4096 columns, one row) 1.1e-7 -> 0.8e-7.
@@ -395,8 +395,9 @@ int launch_pass(const SignArgs& a, int M, hipStream_t s) {
 
 }  // namespace
 
-// One and two rows always.  Three and four while eight wavefronts hold the digits of the whole row (two blocks each): beyond, every workgroup packs part after
-// part, which costs more than the other kernel's pre-pass, us there -> here: 11008 x 4096 12.1 -> 8.1 (3 rows), 12.2 -> 9.0 (4); 60000 x 4096 38.4 -> 23.6, 38.4 -> 32.6;
+// One and two rows always, also of tensors that are tall and wide, where every chunk of tiles packs part after part (two rows, planner's mix, us before -> here: 12288 x 8192
+// 18.4 -> 10.8, 28672 x 8192 38.8 -> 18.6, 30000 x 16640 68.0 -> 44.3, 12000 x 20480 48.3 -> 22.4, 2048 x 8192 7.3 -> 7.3).  Three and four while eight wavefronts hold the digits of the whole row (two blocks each): beyond, every workgroup packs part after
+// part, which costs more than the other kernel's pre-pass, us there -> here: 11008 x 4096 11.8 -> 8.3 (3 rows), 11.8 -> 9.3 (4); 60000 x 4096 40.1 -> 25.2, 40.2 -> 35.2;
 // 8192 x 5120 10.5 -> 11.9, 10.5 -> 12.0; 4096 x 11008 13.5 -> 17.1 (4).  Five rows and more are two passes: 11008 x 4096, 8 rows 13.9 -> 18.
 bool signs_fastest(const oilhip_weights& w, int M) {
     return w.seg.sign_tiles && (M <= 2 || (M <= kSignRows && (w.cols >> 8) <= waves_for(M) * (uint32_t)most_blocks(M, kPlain, false)));

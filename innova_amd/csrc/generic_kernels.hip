@@ -34,7 +34,7 @@ dequant_kernel(const uint8_t* __restrict__ payload, const DevBlock* __restrict__
 // float4, so a block is one coalesced 1 KB store.  Every value is formed exactly as decode_weight forms it (level
 // from the literal / host-built tables times the FP16 scale widened by the integer rule, one fused multiply-add for
 // the grouped formats, scale == 0 -> zero point, slots 0).  Blocks sit back to back at a regular stride (`blocks`
-// null) or wherever their descriptors say (tensors stored as window streams).
+// null) or wherever their descriptors say (tensors stored as window streams or sign tiles).
 struct FullTables { const float* lv8; const float* t255; const float* q127; const float* lv4; const float* lv2; };   // LDS copies
 
 
@@ -387,7 +387,7 @@ int launch_block_mse(const oilhip_weights& w, const float* d_orig, const uint64_
     return OILHIP_OK;
 }
 
-// full blocks of nominal size: one format at a regular stride (1), or (window streams, one format or several) the place
+// full blocks of nominal size: one format at a regular stride (1), or (window streams and sign tiles) the place
 // and format of every block from its descriptor (2); 0: neither
 static int full_block_layout(const oilhip_weights& w) {
     if (!w.all_full || w.d_out_off) return 0;
