@@ -21,9 +21,9 @@
 //   one row   649 x 768 4.0 -> 2.5   4096 x 4096 5.3 -> 3.9   12288 x 4096 8.1 -> 5.3   22016 x 4096 12.3 -> 7.1   60000 x 4096 23.6 -> 13.6
 //             4096 x 11008 8.1 -> 6.2   SPARK_Q0 alone 11008 x 4096 10.8 -> 5.3   with the norm 12288 x 4096 8.7 -> 5.9
 //   two       4096 x 4096 6.7 -> 4.7   22016 x 4096 14.8 -> 8.7   4096 x 11008 15.3 -> 9.8   with the norm 12288 x 4096 13.2 -> 7.5
-//   three     1000 x 1280 5.6 -> 3.7   11008 x 4096 11.8 -> 8.3;   four   11008 x 4096 11.8 -> 9.3   with the norm 12288 x 4096 13.6 -> 11.1
-// (One power of two per run instead of per block is an instruction more per tile of one block and row: long launches 1 to 4 % slower, short ones 1 to 3 % faster,
-// with eight instructions fewer in the packing.)
+//   three     1000 x 1280 5.6 -> 3.7   11008 x 4096 11.8 -> 8.2;   four   11008 x 4096 11.8 -> 9.1   with the norm 12288 x 4096 13.6 -> 10.7
+// (One power of two per run instead of per block is an instruction more per tile of one block and row, and 82 vector instructions instead of 93 to pack a block; the
+// sums of runs held as floats stand behind the loop.  Launches of many tiles up to 2 % slower for it, the others 1 to 5 % faster.)
 // Error against 64 bits (2-norm, 4096 columns, one row) 1.1e-7 -> 0.8e-7.
 // Level or slower: an operand of 0 and 1 with the activations' sums as the matrix instruction's addend (24 registers per block instead of 16); sums over
 // the lane groups in front of LDS instead of behind it (22016 x 4096 8.5 us against 6.9, with the loop's waits then counting no loads).
@@ -264,7 +264,7 @@ gemv_signs_kernel(const SignArgs a) {
             for (int m = 0; m < M; ++m) {
                 auto one = [](const i32x4& d) { return fmaf((float)(d[3] * 256 + d[2]), 65536.0f, (float)(d[1] * 256 + d[0])); };
                 float f0 = one(d0[m]), f1 = one(d1[m]);
-                if (slow & (1u << (s * M + m))) {                          // uniform
+                if (__builtin_expect((slow & (1u << (s * M + m))) != 0u, 0)) {   // uniform; behind the loop: a branch that is not taken
                     const uint8_t* x = reinterpret_cast<const uint8_t*>(mine + (uint32_t)(s * M + m) * 256u + 64u * q);
                     auto floats = [&](float f, auto r, uint32_t signs, const uint8_t* run) {
                         // (a 64th of each beside an infinity: finite ones must not add up to the other one)
@@ -397,7 +397,7 @@ int launch_pass(const SignArgs& a, int M, hipStream_t s) {
 
 // One and two rows always, also of tensors that are tall and wide, where every chunk of tiles packs part after part (two rows, planner's mix, us before -> here: 12288 x 8192
 // 18.4 -> 10.8, 28672 x 8192 38.8 -> 18.6, 30000 x 16640 68.0 -> 44.3, 12000 x 20480 48.3 -> 22.4, 2048 x 8192 7.3 -> 7.3).  Three and four while eight wavefronts hold the digits of the whole row (two blocks each): beyond, every workgroup packs part after
-// part, which costs more than the other kernel's pre-pass, us there -> here: 11008 x 4096 11.8 -> 8.3 (3 rows), 11.8 -> 9.3 (4); 60000 x 4096 40.1 -> 25.2, 40.2 -> 35.2;
+// part, which costs more than the other kernel's pre-pass, us there -> here: 11008 x 4096 11.8 -> 8.2 (3 rows), 11.8 -> 9.1 (4); 60000 x 4096 40.1 -> 25.2, 40.2 -> 34.9;
 // 8192 x 5120 10.5 -> 11.9, 10.5 -> 12.0; 4096 x 11008 13.5 -> 17.1 (4).  Five rows and more are two passes: 11008 x 4096, 8 rows 13.9 -> 18.
 bool signs_fastest(const oilhip_weights& w, int M) {
     return w.seg.sign_tiles && (M <= 2 || (M <= kSignRows && (w.cols >> 8) <= waves_for(M) * (uint32_t)most_blocks(M, kPlain, false)));
