@@ -11,7 +11,7 @@
 // 4 q .. 4 q + 3 and are zero in the lane groups of other runs, so a lane gets the four digit sums of the two runs whose signs and scales it
 // holds: they become one float, exact but for its rounding, meet the two scales in FP32 (a scale times its run's power of two is exact), and no lane ever holds another row's sum.
 //
-// A wavefront keeps the digits of its one to three column blocks in registers and walks down the workgroup's tiles; every workgroup packs
+// A wavefront keeps the digits of its one to four column blocks in registers and walks down the workgroup's tiles; every workgroup packs
 // the activations itself (each wavefront its own blocks, without a barrier), so there is no second launch and no scratch.  The wavefronts'
 // sums meet in LDS once per 16 tiles, in a fixed order.
 //
